@@ -260,16 +260,120 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_bwd_kernel(
   }
 }
 
-// d_w[h] = (accumulate ? d_w[h] : 0) + sum_b partial[b, h], b ascending
+// The same for rows of at most 64 * V 16-byte vectors: one WAVE per row, so the row's dot product
+// needs no barrier (the block kernel above spends two per row, with every wave of the block waiting
+// on the slowest load).  Wave w of the grid walks rows w, w + waves, ...; its d_w sums stay in
+// registers, the four waves of a block add theirs in wave order through LDS and one partial row per
+// block goes to memory.  Bound by HBM (d_y and x in, d_x out).
+template <typename T, int V>
+__global__ __launch_bounds__(kRowThreads) void rmsnorm_bwd_wave_kernel(
+    const T* __restrict__ d_y, const T* __restrict__ x, const T* __restrict__ w,
+    const float* __restrict__ rstd, const T* __restrict__ addend, T* __restrict__ d_x,
+    float* __restrict__ partial, int64_t rows, int64_t H) {
+  using IO = RowIO<T, true>;
+  constexpr int N = PkVec16<T>::N, WAVES = kRowThreads / 64;
+  __shared__ float sums[64 * V * N];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nv = (int)(H / N);
+  float dw[V][N], wv[V][N];
+#pragma unroll
+  for (int c = 0; c < V; ++c) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) { dw[c][i] = 0.f; wv[c][i] = 0.f; }
+    if (lane + 64 * c < nv) IO::load(w, lane + 64 * c, wv[c]);
+  }
+  for (int64_t t = (int64_t)blockIdx.x * WAVES + wave; t < rows; t += (int64_t)gridDim.x * WAVES) {
+    const float rs = rstd[t];
+    PkVec16<T> vy[V], vx[V], va[V];
+#pragma unroll
+    for (int c = 0; c < V; ++c) {      // every load of the row first
+      const int v = lane + 64 * c;
+      if (v < nv) {
+        vy[c].v = reinterpret_cast<const decltype(vy[c].v)*>(d_y + t * H)[v];
+        vx[c].v = reinterpret_cast<const decltype(vx[c].v)*>(x + t * H)[v];
+        if (addend) va[c].v = reinterpret_cast<const decltype(va[c].v)*>(addend + t * H)[v];
+      } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) { vy[c].set(i, 0.f); vx[c].set(i, 0.f); va[c].set(i, 0.f); }
+      }
+    }
+    float dot = 0.f;
+#pragma unroll
+    for (int c = 0; c < V; ++c)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float xh = vx[c].get(i) * rs, dy = vy[c].get(i);
+        dw[c][i] = fmaf(dy, xh, dw[c][i]);
+        dot = fmaf(dy * wv[c][i], xh, dot);
+      }
+    dot = pk_wave_sum(dot) / (float)H;
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+      const int v = lane + 64 * c;
+      if (v < nv) {
+        float o[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          o[i] = rs * (vy[c].get(i) * wv[c][i] - (vx[c].get(i) * rs) * dot);
+          if (addend) o[i] = pk_to_float<T>(pk_from_float<T>(o[i])) + va[c].get(i);
+        }
+        IO::store(d_x + t * H, v, o);
+      }
+    }
+  }
+  if (!partial) return;
+  for (int k = 0; k < WAVES; ++k) {
+    if (wave == k) {
+#pragma unroll
+      for (int c = 0; c < V; ++c)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          float* const s = &sums[(i * V + c) * 64 + lane];      // lane-contiguous: no bank conflicts
+          *s = k == 0 ? dw[c][i] : *s + dw[c][i];
+        }
+    }
+    __syncthreads();
+  }
+  for (int h = threadIdx.x; h < (int)H; h += kRowThreads) {
+    const int v = h / N, i = h % N;
+    partial[(int64_t)blockIdx.x * H + h] = sums[(i * V + (v >> 6)) * 64 + (v & 63)];
+  }
+}
+
+// d_w[h] = (accumulate ? d_w[h] : 0) + sum_b partial[b, h].  A block takes 32 columns: its 32 row
+// groups each add up every 32nd partial row (at most 16 of them, loaded together), and the 32 group
+// sums are added in group order.  One thread per column walking all 512 partial rows was a chain of
+// 512 dependent round trips on 8 workgroups: 118 us at width 2048 whatever the token count, against
+// 5 us like this.
+constexpr int kDwCols = 32, kDwGroups = 32;
 template <typename T>
-__global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial, int nb,
-                                                                 T* __restrict__ d_w, int64_t H, int accumulate) {
-  const int64_t h = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (h >= H) return;
+__global__ __launch_bounds__(kDwCols * kDwGroups) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial, int nb,
+                                                                                 T* __restrict__ d_w, int64_t H, int accumulate) {
+  __shared__ float red[kDwGroups][kDwCols + 1];
+  constexpr int ROWS = 16;
+  const int c = threadIdx.x % kDwCols, g = threadIdx.x / kDwCols;
+  const int64_t h = (int64_t)blockIdx.x * kDwCols + c;
   float s = 0.f;
-  for (int b = 0; b < nb; ++b) s += partial[(int64_t)b * H + h];
-  if (accumulate) s += pk_to_float<T>(d_w[h]);
-  d_w[h] = pk_from_float<T>(s);
+  if (h < H)
+    for (int b0 = g; b0 < nb; b0 += kDwGroups * ROWS) {
+      float v[ROWS];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const int b = b0 + r * kDwGroups;
+        v[r] = b < nb ? partial[(int64_t)b * H + h] : 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) s += v[r];
+    }
+  red[g][c] = s;
+  __syncthreads();
+  if (g == 0 && h < H) {
+    float total = 0.f;
+#pragma unroll
+    for (int k = 0; k < kDwGroups; ++k) total += red[k][c];
+    if (accumulate) total += pk_to_float<T>(d_w[h]);
+    d_w[h] = pk_from_float<T>(total);
+  }
 }
 
 // Rows too long for the register-resident kernel (or not vectorisable): d_x with strided loops,
@@ -306,6 +410,7 @@ __global__ __launch_bounds__(256) void rmsnorm_dw_generic_kernel(const T* __rest
 
 constexpr int kNormBwdBlocks = 512;
 constexpr int kNormBwdMaxCpt = 4;   // column vectors per thread
+constexpr int kNormWaveVecs = 8;    // column vectors per lane of the wave-per-row kernel (4,096 bf16 or 2,048 fp32 columns)
 
 bool vec_ok(int dtype, int64_t H, std::initializer_list<const void*> ptrs) {
   const int n = dtype == PK_BF16 ? 8 : 4;
@@ -323,6 +428,20 @@ int rmsnorm_bwd_launch(const void* d_y, const void* x, const void* weight, const
   const int64_t nv = H / (VEC ? PkVec16<T>::N : 1);
   const int64_t cpt = pk_ceil_div(nv, kRowThreads);
   const dim3 grid((unsigned)nb);
+  if constexpr (VEC) {
+#define PK_NORM_BWD_WAVE(V)                                                                                       \
+  PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_bwd_wave_kernel<T, V>), grid, dim3(kRowThreads), 0, s, \
+                    (const T*)d_y, (const T*)x, (const T*)weight, rstd, (const T*)addend, (T*)d_x, partial, rows, H)
+    if (nv <= 64 * kNormWaveVecs) {
+      if (nv <= 64) { PK_NORM_BWD_WAVE(1); }
+      else if (nv <= 128) { PK_NORM_BWD_WAVE(2); }
+      else if (nv <= 256) { PK_NORM_BWD_WAVE(4); }
+      else { PK_NORM_BWD_WAVE(8); }
+      PK_RETURN_IF_LAUNCH_FAILED();
+      return PK_OK;
+    }
+#undef PK_NORM_BWD_WAVE
+  }
 #define PK_NORM_BWD(C)                                                                                       \
   PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_bwd_kernel<T, VEC, C>), grid, dim3(kRowThreads), 0, s, \
                     (const T*)d_y, (const T*)x, (const T*)weight, rstd, (const T*)addend, (T*)d_x, partial, rows, H)
@@ -482,13 +601,16 @@ int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight
   if (T == 0) return PK_OK;
   if (!d_y || !x || !weight || !rstd || !d_x) return PK_ERR_ARG;
   if (T > 0x7fffffffll) return PK_ERR_SHAPE;
-  const int nb = (int)(T < kNormBwdBlocks ? T : kNormBwdBlocks);
+  const bool vec = vec_ok(dtype, H, {d_y, x, weight, d_x, d_x_addend});
+  // rows that a wave holds in registers: four rows to a block (rmsnorm_bwd_wave_kernel), otherwise one
+  const bool by_wave = vec && H <= kNormWaveVecs * 64 * (dtype == PK_BF16 ? 8 : 4);
+  const int64_t row_blocks = by_wave ? pk_ceil_div(T, kRowThreads / 64) : T;
+  const int nb = (int)(row_blocks < kNormBwdBlocks ? row_blocks : kNormBwdBlocks);
   float* partial = nullptr;
   if (d_weight) {
     if (!workspace || workspace_bytes < pk_rmsnorm_bwd_workspace_bytes(T, H)) return PK_ERR_WORKSPACE;
     partial = reinterpret_cast<float*>(workspace);
   }
-  const bool vec = vec_ok(dtype, H, {d_y, x, weight, d_x, d_x_addend});
   hipStream_t s = (hipStream_t)stream;
   int rc;
   if (dtype == PK_BF16)
@@ -511,11 +633,11 @@ int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight
   }
   if (rc != PK_OK) return rc;
   if (d_weight) {
-    const dim3 grid((unsigned)pk_ceil_div(H, 256));
+    const dim3 grid((unsigned)pk_ceil_div(H, kDwCols));
     if (dtype == PK_BF16)
-      PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<bf16_t>), grid, dim3(256), 0, s, partial, nb, (bf16_t*)d_weight, H, accumulate ? 1 : 0);
+      PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<bf16_t>), grid, dim3(kDwCols * kDwGroups), 0, s, partial, nb, (bf16_t*)d_weight, H, accumulate ? 1 : 0);
     else
-      PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<float>), grid, dim3(256), 0, s, partial, nb, (float*)d_weight, H, accumulate ? 1 : 0);
+      PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<float>), grid, dim3(kDwCols * kDwGroups), 0, s, partial, nb, (float*)d_weight, H, accumulate ? 1 : 0);
     PK_RETURN_IF_LAUNCH_FAILED();
   }
   return PK_OK;

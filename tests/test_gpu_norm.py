@@ -98,3 +98,20 @@ def test_feed_forward_block_module(dev):
     assert got.shape == x.shape and torch.equal(got, want)
     assert sorted(n for n, _ in blk.named_parameters()) == [
         "ffn_norm.weight", "moe.experts.w1", "moe.experts.w2", "moe.experts.w3", "moe.router.gate.weight"]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,H", [(3, 264), (517, 1016), (1300, 2048), (2100, 2056), (9, 4096), (9, 4104)])
+def test_rmsnorm_bwd_on_both_sides_of_the_wave_kernel(dev, dtype, T, H):
+    """Rows that just fill or just exceed 1, 2, 4 and 8 vectors per lane, and row counts that leave
+    waves without a row, with one, and with several."""
+    print(f"[case] rmsnorm bwd {dtype} T={T} H={H}", flush=True)
+    g = torch.Generator().manual_seed(T + H)
+    x, dy, add = (torch.randn(T, H, generator=g).to(dtype) for _ in range(3))
+    w = (1.0 + 0.1 * torch.randn(H, generator=g)).to(dtype)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    O.rmsnorm(xr, wr, 1e-6).backward(dy.double())
+    tol = F32_TOL if dtype == torch.float32 else BF16_TOL
+    _, rstd = ops.rmsnorm_fwd(x.to(dev), w.to(dev), 1e-6)
+    dx, dw = ops.rmsnorm_bwd(dy.to(dev), x.to(dev), w.to(dev), rstd, d_x_addend=add.to(dev))
+    assert rel_err(dx, xr.grad + add.double()) <= tol and rel_err(dw, wr.grad) <= tol
