@@ -8,9 +8,13 @@
 //         operand from the transposed copies the scaled SwiGLU backward writes) for the fused
 //         region; wgrad_kernel (one workgroup per (expert, output tile), both operands through the
 //         transposing LDS read) for the piecewise entry points.
-//   f32 : tiled FMA kernel (simt_gemm.h) + elementwise SwiGLU kernels; exact fp32 arithmetic.
+//   f32, and bf16 widths that are no multiple of 128: 64x64 / 128x128 matrix-core tiles
+//         (tile_gemm.h; fp32 products and sums are exact) + elementwise SwiGLU backward kernels.
+//   rows that are no whole number of 16-byte pieces: tiled FMA kernel (simt_gemm.h).
 #include "pk_common.h"
 #include "simt_gemm.h"
+#include "tile_gemm.h"
+#include "unit_index.h"
 #include <functional>
 #include <initializer_list>
 #include <map>
@@ -33,10 +37,8 @@ constexpr int NXCD = 8;
 enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_SWIGLU_BWD = 2, EPI_SWIGLU_BWD_SCALED = 3 };
 
 typedef short shortx4_t __attribute__((ext_vector_type(4)));
-// Read-only tables (row offsets, row maps) addressed wave-uniformly: going through the constant
-// address space makes these scalar loads (lgkmcnt), which leaves vmcnt to the LDS ring.
-typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
-__device__ __forceinline__ const_i32_ptr as_const(const int32_t* p) { return (const_i32_ptr)(uintptr_t)p; }
+using pk_units::as_const;
+using pk_units::const_i32_ptr;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // 16 zero bytes: the source of operand rows past the end of a ragged reduction range.
@@ -321,54 +323,9 @@ __device__ __forceinline__ void wait_vm_le(int n) {
   }
 }
 
-// Per-lane slice of the prefix sum of work units over experts: lane l covers experts
-// [l*epl, (l+1)*epl).  Built once per wave with ordinary loads; locating a unit afterwards
-// takes a ballot plus a short scalar walk, so it can run in the middle of the k-loop without
-// touching the vector-memory counter that tracks the LDS ring.
-struct UnitIndex {
-  int excl, incl, total, epl;
-};
-template <int BM>
-__device__ __forceinline__ UnitIndex build_unit_index(const int32_t* __restrict__ starts, int E, int n_tiles) {
-  const int lane = threadIdx.x & 63;
-  UnitIndex ui;
-  ui.epl = (E + 63) >> 6;
-  const int e_lo = lane * ui.epl, e_hi = min(E, e_lo + ui.epl);
-  int mine = 0;
-  for (int e = e_lo; e < e_hi; ++e) mine += ((starts[e + 1] - starts[e] + BM - 1) / BM) * n_tiles;
-  int incl = mine;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(incl, off, PK_WAVE);
-    if (lane >= off) incl += v;
-  }
-  ui.incl = incl;
-  ui.excl = incl - mine;
-  ui.total = __builtin_amdgcn_readlane(incl, 63);
-  return ui;
-}
-// unit < ui.total.  Units of expert e are laid out [n-tile][m-tile], so neighbouring units share
-// the weight tile.  Everything returned is wave-uniform.
-template <int BM>
-__device__ __forceinline__ void locate_unit(const UnitIndex& ui, const_i32_ptr starts, int E, int n_tiles,
-                                            int unit, int& e_out, int& mt_out, int& nt_out) {
-  const unsigned long long bal = __ballot(unit >= ui.excl && unit < ui.incl);
-  const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)bal) - 1);
-  int u = unit - __builtin_amdgcn_readlane(ui.excl, src);
-  int e = src * ui.epl;
-  const int e_hi = min(E, e + ui.epl);
-  int tiles = 1;
-  for (; e < e_hi; ++e) {
-    tiles = (starts[e + 1] - starts[e] + BM - 1) / BM;
-    const int units = tiles * n_tiles;
-    if (u < units) break;
-    u -= units;
-  }
-  tiles = tiles > 0 ? tiles : 1;
-  e_out = e;
-  nt_out = u / tiles;
-  mt_out = u - nt_out * tiles;
-}
+using pk_units::UnitIndex;
+using pk_units::build_unit_index;
+using pk_units::locate_unit;
 
 // ---------------------------------------------------------------------------------------------
 // Work distribution of the persistent kernels.  Units are grouped in chunks of SCHED_CHUNK
@@ -2240,6 +2197,56 @@ int check_common(int64_t A, int64_t H, int64_t I, int64_t E, int dtype) {
   return PK_OK;
 }
 
+// Whether the tiles of tile_gemm.h can read and write the operands: rows of whole 16-byte pieces,
+// aligned bases.  They take every fp32 call and every bf16 call the 128-multiple kernels refuse as
+// long as this holds (forward + backward of a region, FMA tiles -> these: fp32, 4,000 rows of 16
+// experts, 512 x 256: 779 -> FIG_F32 us of GEMM time; bf16, 4,120 rows of 24 experts, 1000 x 360:
+// 1,369 -> FIG_BF us).
+bool tile_gemm_ok(int dtype, int64_t H, int64_t I, std::initializer_list<const void*> ptrs) {
+  const int64_t piece = 16 / (int64_t)pk_dtype_size(dtype);
+  return H % piece == 0 && I % piece == 0 && all_aligned16(ptrs);
+}
+
+template <typename T>
+int fwd_tile(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2, const void* w3,
+             const int32_t* starts, void* g, void* u, void* h, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
+  pk_tile::RaggedM p = {};
+  p.A0 = p.A1 = x; p.lda = H; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.B0 = w1; p.B1 = w3; p.ldb = H; p.strideB = I * H;
+  p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
+  p.O0 = g; p.O1 = u; p.O2 = h; p.ldc = I;
+  int rc = pk_tile::launch_ragged_m<T, true, true>(p, A, mf::persistent_grid(), pk_timing::K_SWIGLU_GATE_UP, s);
+  if (rc) return rc;
+  pk_tile::RaggedM q = {};
+  q.A0 = q.A1 = h; q.lda = I; q.map_div = 1;
+  q.B0 = q.B1 = w2; q.ldb = I; q.strideB = H * I;
+  q.starts = starts; q.E = (int32_t)E; q.K = (int32_t)I; q.nseg = 1; q.N = (int32_t)H;
+  q.O0 = y; q.ldc = H;
+  return pk_tile::launch_ragged_m<T, true, false>(q, A, mf::persistent_grid(), pk_timing::K_SWIGLU_DOWN, s);
+}
+// C [A, N] = sum over nseg weight matrices [K, N] (row-major) of A_seg . B_seg
+template <typename T>
+int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map, int64_t div, const void* B0, const void* B1,
+               void* C, int64_t N, int nseg, const int32_t* starts, int64_t A, int64_t E, int kernel_id, hipStream_t s) {
+  pk_tile::RaggedM p = {};
+  p.A0 = A0; p.A1 = nseg > 1 ? A1 : A0; p.lda = K; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.B0 = B0; p.B1 = nseg > 1 ? B1 : B0; p.ldb = N; p.strideB = K * N;
+  p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)K; p.nseg = nseg; p.N = (int32_t)N;
+  p.O0 = C; p.ldc = N;
+  return pk_tile::launch_ragged_m<T, false, false>(p, A, mf::persistent_grid(), kernel_id, s);
+}
+template <typename T>
+int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void* dg, const void* du, const void* x,
+               const int32_t* row_map, int64_t div, const int32_t* starts, void* dw1, void* dw2, void* dw3, int acc,
+               int64_t H, int64_t I, int64_t E, hipStream_t s) {
+  pk_tile::RaggedK p = {};
+  p.starts = starts; p.E = (int32_t)E; p.map_div = (int32_t)div; p.accumulate = acc ? 1 : 0;
+  if (dw2) p.prob[p.nprob++] = {dy, H, dy_map, h, I, nullptr, dw2, (int32_t)H, (int32_t)I};
+  if (dw1) p.prob[p.nprob++] = {dg, I, nullptr, x, H, row_map, dw1, (int32_t)I, (int32_t)H};
+  if (dw3) p.prob[p.nprob++] = {du, I, nullptr, x, H, row_map, dw3, (int32_t)I, (int32_t)H};
+  return pk_tile::launch_ragged_k<T>(p, mf::persistent_grid(), pk_timing::K_SWIGLU_WGRAD, s);
+}
+
 template <typename T>
 int fwd_simt(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2,
              const void* w3, const int32_t* starts, void* g, void* u, void* h, void* y, int64_t A,
@@ -2299,9 +2306,13 @@ int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t ro
   if (row_map && (row_map_div <= 0 || row_map_div > 0x7fffffffll)) return PK_ERR_ARG;
   if (!row_map) row_map_div = 1;
   hipStream_t s = (hipStream_t)stream;
+  const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({x_rows, w1, w2, w3, g, u, h, y});
+  if (!mfma && tile_gemm_ok(dtype, H, I, {x_rows, w1, w2, w3, g, u, h, y}))
+    return dtype == PK_F32 ? fwd_tile<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s)
+                           : fwd_tile<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
   if (dtype == PK_F32)
     return fwd_simt<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
-  if (!mfma_shape_ok(H, I) || !all_aligned16({x_rows, w1, w2, w3, g, u, h, y}))
+  if (!mfma)
     return fwd_simt<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
 
   mf::RaggedMParams p = {};
@@ -2333,13 +2344,16 @@ int pk_grouped_swiglu_dgrad_dh(const void* d_y, const void* w2, const void* g, c
   if (simt) {
     // d_h = d_y . w2[e]  (w2[e] is [H, I]: B(k=h, n=i) = w2[h*I + i]); staged in d_u's buffer
     const int64_t n = A * I;
+    const bool tile = tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u});
     if (dtype == PK_F32) {
-      rc = simt_ragged_m<float>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
+      rc = tile ? dgrad_tile<float>(d_y, nullptr, H, nullptr, 1, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s)
+                : simt_ragged_m<float>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
       if (rc) return rc;
       PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_ELEMENTWISE, s, (swiglu_bwd_kernel<float>), dim3((unsigned)pk_ceil_div(n, 256)), dim3(256), 0, s,
                         (const float*)d_u, (const float*)g, (const float*)u, (float*)d_g, (float*)d_u, n);
     } else {
-      rc = simt_ragged_m<bf16_t>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
+      rc = tile ? dgrad_tile<bf16_t>(d_y, nullptr, H, nullptr, 1, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s)
+                : simt_ragged_m<bf16_t>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
       if (rc) return rc;
       PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_ELEMENTWISE, s, (swiglu_bwd_kernel<bf16_t>), dim3((unsigned)pk_ceil_div(n, 256)), dim3(256), 0, s,
                         (const bf16_t*)d_u, (const bf16_t*)g, (const bf16_t*)u, (bf16_t*)d_g, (bf16_t*)d_u, n);
@@ -2397,7 +2411,12 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
   const bool simt = dtype == PK_F32 || !mfma_shape_ok(H, I) || !all_aligned16({d_out, w2, g, u, d_g, d_u, hs});
   if (simt) {
     // unscaled d_h = d_out[token] . w2[e], staged in d_u's buffer; then one wave per row
-    if (dtype == PK_F32) rc = simt_ragged_m<float>(d_out, H, row_map, row_map_div, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
+    const bool tile = tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs});
+    if (tile && dtype == PK_F32)
+      rc = dgrad_tile<float>(d_out, nullptr, H, row_map, row_map_div, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s);
+    else if (tile)
+      rc = dgrad_tile<bf16_t>(d_out, nullptr, H, row_map, row_map_div, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s);
+    else if (dtype == PK_F32) rc = simt_ragged_m<float>(d_out, H, row_map, row_map_div, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
     else rc = simt_ragged_m<bf16_t>(d_out, H, row_map, row_map_div, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
     if (rc) return rc;
     const dim3 grid((unsigned)pk_ceil_div(A, 4)), block(256);
@@ -2462,6 +2481,10 @@ int pk_grouped_swiglu_dgrad_dx(const void* d_g, const void* d_u, const void* w1,
   const bool simt = dtype == PK_F32 || !mfma_shape_ok(H, I) || !all_aligned16({d_g, d_u, w1, w3, d_x_sorted});
   if (simt) {
     // d_x = d_g . w1[e] + d_u . w3[e]   (w[e] is [I, H]: B(k=i, n=h) = w[i*H + h])
+    if (tile_gemm_ok(dtype, H, I, {d_g, d_u, w1, w3, d_x_sorted}))
+      return dtype == PK_F32
+                 ? dgrad_tile<float>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s)
+                 : dgrad_tile<bf16_t>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s);
     if (dtype == PK_F32) {
       rc = simt_ragged_m<float>(d_g, I, nullptr, 1, w1, H, 1, I * H, d_x_sorted, H, starts, A, H, I, E, 0, s);
       if (rc) return rc;
@@ -2535,9 +2558,14 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   if (!row_map) row_map_div = 1;
   const int32_t* dy_map = dy_gathered ? row_map : nullptr;
   hipStream_t s = (hipStream_t)stream;
+  const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3});
+  if (!mfma && tile_gemm_ok(dtype, H, I, {d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}))
+    return dtype == PK_F32
+               ? wgrad_tile<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s)
+               : wgrad_tile<bf16_t>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s);
   if (dtype == PK_F32)
     return wgrad_simt<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s);
-  if (!mfma_shape_ok(H, I) || !all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}))
+  if (!mfma)
     return wgrad_simt<bf16_t>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s);
 
   mf::WgradParams p = {};

@@ -493,3 +493,55 @@ def test_grouped_gemms_replay_in_a_hip_graph(dev):
         torch.cuda.synchronize()
         for got, ref, name in zip(outs, want, ("y", "dx", "dw1", "dw2", "dw3")):
             assert torch.equal(got, ref), f"replay {rep}: {name}"
+
+
+TILE_CASES = [
+    # (counts, H, I): rows on both sides of the 64-row tiles, empty experts, widths that leave a remainder in
+    # the 64-wide tiles and in the k-tiles (32 fp32 / 64 bf16), down to a single 16-byte piece
+    ([0, 1, 63, 64, 65, 127, 128, 129, 0], 72, 40),
+    ([3, 2], 8, 8),
+    ([70, 0, 33], 200, 1000),
+    # enough rows for the 128 x 128 tiles in every product
+    ([3000, 1, 4000, 200, 0, 2500], 1032, 520),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts,H,I", TILE_CASES)
+def test_widths_without_a_multiple_of_the_wide_tiles(dev, dtype, counts, H, I):
+    """tile_gemm.h (fp32, and bf16 widths that are no multiple of 128) against float64 matmuls of the same
+    inputs: x gathered through a row map, accumulation into existing gradients, exact zeros for an
+    expert without rows.  fp32 sums of n products are within n * 2^-24 of the sum of magnitudes, far
+    below F32_TOL of the largest result; bf16 as everywhere (BF16_TOL)."""
+    print(f"[case] tile gemm {dtype} E={len(counts)} A={sum(counts)} H={H} I={I}", flush=True)
+    x, w1, w2, w3, dy, cnt = (t.to(dev) for t in _make(31, counts, H, I, dtype))
+    E, A = len(counts), x.shape[0]
+    tol = BF16_TOL if dtype == torch.bfloat16 else F32_TOL
+    order = torch.randperm(A, generator=torch.Generator().manual_seed(1)).to(dev)
+    x_at = torch.empty_like(x)
+    x_at[order] = x                      # row p of the sorted operand is x_at[order[p]]
+    rows = order.to(torch.int32)
+    starts = ops.counts_to_starts(cnt)
+    y, g, u, h = ops.grouped_swiglu_fwd(x_at, w1, w2, w3, starts, row_map=rows, row_map_div=1)
+    dx, dg, du = ops.grouped_swiglu_dgrad(dy, w1, w2, w3, g, u, starts)
+    dw1, dw2, dw3 = ops.grouped_swiglu_wgrad(dy, h, dg, du, x_at, starts, E, row_map=rows, row_map_div=1)
+    acc = [t.clone() for t in (dw1, dw2, dw3)]
+    ops.grouped_swiglu_wgrad(dy, h, dg, du, x_at, starts, E, row_map=rows, row_map_div=1, d_w1=acc[0], d_w2=acc[1], d_w3=acc[2],
+                             accumulate=True)
+    torch.cuda.synchronize()
+    s = 0
+    for e, c in enumerate(counts):
+        if c == 0:
+            assert all(float(t[e].abs().max()) == 0.0 for t in (dw1, dw2, dw3, *acc))
+            continue
+        leaves = [t.double().requires_grad_(True) for t in (x[s:s + c], w1[e], w2[e], w3[e])]
+        xe, a1, a2, a3 = leaves
+        ge, ue = xe @ a1.t(), xe @ a3.t()
+        he = torch.nn.functional.silu(ge) * ue
+        ye = he @ a2.t()
+        dxe, d1, d2, d3 = torch.autograd.grad(ye, leaves, dy[s:s + c].double())
+        for name, got, ref in (("g", g[s:s + c], ge), ("u", u[s:s + c], ue), ("h", h[s:s + c], he), ("y", y[s:s + c], ye),
+                               ("dx", dx[s:s + c], dxe), ("dw1", dw1[e], d1), ("dw2", dw2[e], d2), ("dw3", dw3[e], d3),
+                               ("dw1 added", acc[0][e], 2 * d1), ("dw2 added", acc[1][e], 2 * d2), ("dw3 added", acc[2][e], 2 * d3)):
+            assert rel_err(got, ref) <= tol, (name, e, c, rel_err(got, ref))
+        s += c
