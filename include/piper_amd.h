@@ -192,8 +192,8 @@ PK_API int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void*
  * Together these replace _run_bmm_experts (qwen3_bmm_experts_patch.py:11-50) and the
  * autograd graph torch builds for it (src/executors.py:257-296).
  * bf16 runs on MFMA tiles when H % 128 == 0, I % 128 == 0 and every operand is 16-byte aligned,
- * and on a shape-unrestricted FMA kernel (still HIP, same results to rounding) otherwise; f32 runs on a
- * tiled FMA kernel with no shape restriction.
+ * f32, and bf16 with other widths, runs on smaller matrix-core tiles when rows are whole 16-byte pieces
+ * (fp32 products and sums are exact), and on a shape-unrestricted FMA kernel otherwise.
  * On the MFMA path an operand whose rows are gathered through a row map (x_rows, d_out) is addressed with
  * 32-bit byte offsets from its first row: the rows that the map can name (ceil(A / row_map_div) of them)
  * must span less than 4 GiB, otherwise the call returns PK_ERR_SHAPE and launches nothing.
@@ -202,7 +202,9 @@ PK_API int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void*
 /* Forward.  x_rows[A_x,H]: when row_map is NULL, row p of the A operand is x_rows[p]
  * (x already expert-sorted, the reference boundary); otherwise it is
  * x_rows[row_map[p] / row_map_div] (permute fused into the operand load; pass perm and K).
- *   g[A,I] = x . w1[e]^T,  u[A,I] = x . w3[e]^T   (saved for backward)
+ *   g[A,I] = x . w1[e]^T,  u[A,I] = x . w3[e]^T   (saved for backward; both may be NULL when there is
+ *                                                  none, if rows are whole 16-byte pieces and every
+ *                                                  operand is 16-byte aligned, else PK_ERR_ARG)
  *   h[A,I] = silu(g) * u
  *   y[A,H] = h . w2[e]^T */
 PK_API int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t row_map_div,

@@ -13,6 +13,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libpiper_amd.so"
+HOST_PATH = Path(__file__).resolve().parent / "_pk_host.so"
 
 PK_F32 = 0
 PK_BF16 = 1
@@ -103,8 +104,24 @@ def load() -> C.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native host path of the operators (csrc/host.cpp), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        if not HOST_PATH.exists():
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m piper_amd.build` "
+                               "(there is no fallback implementation)")
+        from . import _pk_host
+        _host = _pk_host
+    return _host
+
+
 def is_built() -> bool:
-    return LIB_PATH.exists()
+    return LIB_PATH.exists() and HOST_PATH.exists()
 
 
 def status_string(status: int) -> str:

@@ -19,6 +19,7 @@ import logging
 import torch
 
 from . import ops
+from ._lib import host
 from .optim import FusedAdamW
 
 BUCKET_ALIGN_BYTES = 256
@@ -114,6 +115,11 @@ def flatten_params(bucket: BucketState, params: Sequence[torch.nn.Parameter], *,
     bucket.full_params_fresh = True
     bucket.optimizer = None
     return bucket
+
+
+def _stream_key(stream):
+    """A torch stream as the native host path takes it (None: the caller's current stream)."""
+    return None if stream is None else (stream.stream_id, stream.device_index, stream.device_type)
 
 
 @dataclass
@@ -227,8 +233,7 @@ class ParamStorage:
 
     def clear_param_grads(self) -> None:
         for bucket in self._all_states():
-            for p, *_ in bucket.param_view_specs:
-                p.grad = None
+            host().clear_param_grads(bucket.param_view_specs)
 
     def zero_grad_buffers(self, stream: torch.cuda.Stream | None = None) -> None:
         """src/runtime.py:223-229."""
@@ -259,21 +264,7 @@ class ParamStorage:
                 bucket.flat_grads = torch.zeros(bucket.param_shard_info[1], dtype=self.grad_buffer_dtype,
                                                 device=bucket.flat_params.device)
                 bucket.reduce_scatter_grads = bucket.flat_grads
-            by_dtype: dict = {}
-            for param, offset, numel, _shape in specs:
-                grad = param.grad
-                if grad is None:
-                    continue
-                g = grad.detach()
-                if stream is not None:
-                    g.record_stream(stream)
-                by_dtype.setdefault(g.dtype, ([], []))
-                by_dtype[g.dtype][0].append(g.reshape(-1))
-                by_dtype[g.dtype][1].append(offset)
-            for grads, offs in by_dtype.values():
-                ops.bucket_pack(grads, offs, bucket.flat_grads, accumulate=True)
-            for param, *_ in specs:
-                param.grad = None
+            host().pack_param_grads(specs, bucket.flat_grads, _stream_key(stream))
 
     def hold_param_grads(self, ubid, stream: torch.cuda.Stream | None = None) -> None:
         """In place of the LAST accumulate_zero_param_grads_to_flat of an iteration: keep the
@@ -284,16 +275,7 @@ class ParamStorage:
         if ubid is None or ubid not in self.stages.zero_managed_ubids:
             return
         for bucket in self.stages.bucket(ubid).with_companions():
-            held = []
-            for param, *_ in bucket.param_view_specs:
-                g = param.grad
-                if g is not None:
-                    g = g.detach()
-                    if stream is not None:
-                        g.record_stream(stream)
-                held.append(g)
-                param.grad = None
-            bucket.pending_grads = held
+            bucket.pending_grads = host().hold_param_grads(bucket.param_view_specs, _stream_key(stream))
 
     def alloc_full_params(self, ubid) -> None:
         """Unflatten (src/runtime.py:312-352): make every parameter a view of the flat bucket."""
@@ -325,8 +307,7 @@ class ParamStorage:
 
     def free_full_grads(self, ubid) -> None:
         for bucket in self.stages.bucket(ubid).with_companions():
-            for param, *_ in bucket.param_view_specs:
-                param.grad = None
+            host().clear_param_grads(bucket.param_view_specs)
 
     def all_gather_full_params(self, ubid, stream: torch.cuda.Stream | None = None) -> int:
         """dp_degree == 1: the shard is the whole bucket, so the gather moves no bytes."""
@@ -361,5 +342,4 @@ class ParamStorage:
                     bucket.shard_param.grad = bucket.reduce_scatter_grads
                     opt.step()
             bucket.shard_param.grad = None
-            for param, *_ in bucket.param_view_specs:
-                param.grad = None
+            host().clear_param_grads(bucket.param_view_specs)

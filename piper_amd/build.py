@@ -1,7 +1,8 @@
-"""Build libpiper_amd.so (gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Build libpiper_amd.so (gfx950 HIP kernels + C ABI) with hipcc and _pk_host.so (the native host path
+of the torch operators, linked against it) with g++, both in-tree.
 
 Usage: ``python -m piper_amd.build`` or ``piper_amd.build.build_library()``.
-The library is written next to this file so that it travels with the source tree.
+The libraries are written next to this file so that they travel with the source tree.
 """
 from __future__ import annotations
 
@@ -9,12 +10,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libpiper_amd.so"
+HOST_PATH = PKG_DIR / "_pk_host.so"
 SOURCES = ["bucket.hip", "route.hip", "permute.hip", "grouped_gemm.hip", "timing.hip"]
 
 HIPCC_FLAGS = [
@@ -45,8 +48,25 @@ def _run(cmd: list[str]) -> None:
         print(out, file=sys.stderr)
 
 
+def _host_commands(obj: Path, out: Path) -> tuple[list[str], list[str]]:
+    """Compile and link commands of the torch extension module (no device code in it)."""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    inc = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include", Path("/opt/rocm/include"),
+           Path(sysconfig.get_paths()["include"])]
+    cxx = shutil.which("g++") or "g++"
+    compile_cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wno-unused-function", "-D__HIP_PLATFORM_AMD__=1",
+                   "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_pk_host", "-DTORCH_API_INCLUDE_EXTENSION_H",
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-isystem{i}" for i in inc],
+                   "-c", str(CSRC / "host.cpp"), "-o", str(obj)]
+    link_cmd = [cxx, "-shared", "-o", str(out), str(obj), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
+                "-ltorch_python", f"-L{PKG_DIR}", "-l:libpiper_amd.so", "-Wl,-rpath,$ORIGIN"]
+    return compile_cmd, link_cmd
+
+
 def build_library(verbose: bool = False) -> Path:
-    """Compile every .hip source for gfx950 and link the shared library.  Always rebuilds."""
+    """Compile every source and link both shared libraries.  Always rebuilds."""
     hipcc = _hipcc()
     obj_dir = PKG_DIR / "build"
     obj_dir.mkdir(exist_ok=True)
@@ -56,14 +76,19 @@ def build_library(verbose: bool = False) -> Path:
         obj = obj_dir / (src.replace(".hip", ".o"))
         objs.append(str(obj))
         cmds.append([hipcc, *HIPCC_FLAGS, "-c", str(CSRC / src), "-o", str(obj)])
+    host_obj, host_tmp = obj_dir / "host.o", HOST_PATH.with_suffix(".so.tmp")
+    host_compile, host_link = _host_commands(host_obj, host_tmp)
+    cmds.append(host_compile)
     if verbose:
         for c in cmds:
             print(" ".join(c))
-    with ThreadPoolExecutor(max_workers=min(5, len(cmds))) as pool:
+    with ThreadPoolExecutor(max_workers=min(6, len(cmds))) as pool:
         list(pool.map(_run, cmds))
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *objs])
     os.replace(tmp, LIB_PATH)
+    _run(host_link)
+    os.replace(host_tmp, HOST_PATH)
     return LIB_PATH
 
 

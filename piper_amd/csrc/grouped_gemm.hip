@@ -1075,7 +1075,9 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
       if (EPI == EPI_SWIGLU) {
 #pragma unroll
         for (int which = 0; which < 3; ++which) {
-          if (crows > 0) {
+          // (a call without a backward does not ask for g and u)
+          bf16_t* const out = which == 0 ? p.O0 : which == 1 ? p.O1 : p.O2;
+          if (crows > 0 && out) {
 #pragma unroll
             for (int j = 0; j < TN; j += 2)
 #pragma unroll
@@ -1093,7 +1095,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
                 St::put(sbuf, lrow, 16 * j + 8 * q + lq, v);
               }
             wave_lds_fence();
-            st_after += St::template flush<false>(sbuf, (which == 0 ? p.O0 : which == 1 ? p.O1 : p.O2) + goff, p.ldc, crows);
+            st_after += St::template flush<false>(sbuf, out + goff, p.ldc, crows);
             wave_lds_fence();
           }
         }
@@ -2200,8 +2202,8 @@ int check_common(int64_t A, int64_t H, int64_t I, int64_t E, int dtype) {
 // Whether the tiles of tile_gemm.h can read and write the operands: rows of whole 16-byte pieces,
 // aligned bases.  They take every fp32 call and every bf16 call the 128-multiple kernels refuse as
 // long as this holds (forward + backward of a region, FMA tiles -> these: fp32, 4,000 rows of 16
-// experts, 512 x 256: 779 -> FIG_F32 us of GEMM time; bf16, 4,120 rows of 24 experts, 1000 x 360:
-// 1,369 -> FIG_BF us).
+// experts, 512 x 256: 779 -> 193 us of GEMM time; bf16, 4,120 rows of 24 experts, 1000 x 360:
+// 1,369 -> 143 us).
 bool tile_gemm_ok(int dtype, int64_t H, int64_t I, std::initializer_list<const void*> ptrs) {
   const int64_t piece = 16 / (int64_t)pk_dtype_size(dtype);
   return H % piece == 0 && I % piece == 0 && all_aligned16(ptrs);
@@ -2302,7 +2304,7 @@ int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t ro
   int rc = check_common(A, H, I, E, dtype);
   if (rc) return rc;
   if (A == 0) return PK_OK;
-  if (!x_rows || !w1 || !w2 || !w3 || !starts || !g || !u || !h || !y) return PK_ERR_ARG;
+  if (!x_rows || !w1 || !w2 || !w3 || !starts || !h || !y || (g == nullptr) != (u == nullptr)) return PK_ERR_ARG;
   if (row_map && (row_map_div <= 0 || row_map_div > 0x7fffffffll)) return PK_ERR_ARG;
   if (!row_map) row_map_div = 1;
   hipStream_t s = (hipStream_t)stream;
@@ -2310,6 +2312,7 @@ int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t ro
   if (!mfma && tile_gemm_ok(dtype, H, I, {x_rows, w1, w2, w3, g, u, h, y}))
     return dtype == PK_F32 ? fwd_tile<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s)
                            : fwd_tile<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
+  if (!mfma && !g) return PK_ERR_ARG;      // the FMA kernels form h from g and u in memory
   if (dtype == PK_F32)
     return fwd_simt<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
   if (!mfma)

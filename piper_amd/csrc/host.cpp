@@ -1,0 +1,890 @@
+// The host path of the operators in native code: argument checks, allocation, the launch sequences of
+// the C ABI and the autograd nodes.  One forward and backward of the expert region is about thirty
+// launches of 2 us each on the host; with a Python call, a ctypes call and one to three tensor
+// allocations in front of every one of them it was 370 us, more than the GPU needs below about a
+// thousand tokens.  Here a node allocates one block of memory for what it saves and one for what it
+// does not, and issues its launches back to back.
+//
+// Python keeps what it is the better place for: the torch.library definitions (functional.py), the
+// modules, and every decision that depends on Python state.  Functions that may meet something else
+// than ordinary GPU tensors (fake tensors, tracing modes) return None and leave the call to the
+// dispatcher.
+#include <c10/hip/HIPStream.h>
+#include <c10/hip/HIPGuard.h>
+#include <hip/hip_runtime.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/extension.h>
+
+#include <array>
+#include <atomic>
+#include <functional>
+#include <mutex>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "../../include/piper_amd.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+namespace {
+
+// ------------------------------------------------------------------------------ small helpers
+void ok(int rc, const char* name) {
+  TORCH_CHECK(rc == 0, name, " failed with status ", rc, ": ", pk_status_string(rc));
+}
+#define PK_CALL(fn, ...) ok(fn(__VA_ARGS__), #fn)
+
+int dtype_code(const Tensor& t) {
+  if (t.scalar_type() == at::kFloat) return PK_F32;
+  if (t.scalar_type() == at::kBFloat16) return PK_BF16;
+  TORCH_CHECK_TYPE(false, "piper_amd kernels support float32 and bfloat16, got ", t.scalar_type());
+}
+
+void require_gpu(const Tensor& t) {
+  TORCH_CHECK(t.is_cuda(), "piper_amd kernels run on the GPU only; got a tensor on ", t.device(), " (there is no CPU fallback)");
+}
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+const float* fptr(const Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
+Tensor contig(const Tensor& t) { return t.defined() && !t.is_contiguous() ? t.contiguous() : t; }
+Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0; }
+
+// The stream of the current context on t's device; pk_init runs once per device before its first
+// launch, so that the launch may already sit inside a HIP graph capture.
+pk_stream_t stream_of(const Tensor& t) {
+  static std::atomic<uint64_t> ready{0};
+  const int dev = t.get_device();
+  const uint64_t bit = 1ull << (dev & 63);
+  if (!(ready.load(std::memory_order_acquire) & bit)) {
+    PK_CALL(pk_init);
+    ready.fetch_or(bit, std::memory_order_release);
+  }
+  return reinterpret_cast<pk_stream_t>(c10::hip::getCurrentHIPStream(dev).stream());
+}
+
+// Ordinary tensors outside every tracing or dispatch mode: the kernels may be launched directly.
+bool plain(std::initializer_list<const Tensor*> ts) {
+  if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python) ||
+      c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return false;
+  for (const Tensor* t : ts) {
+    if (!t->defined()) continue;
+    if (!t->is_cuda() || t->key_set().has(c10::DispatchKey::Python)) return false;
+  }
+  return true;
+}
+bool wants_grad(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
+// Several buffers in one allocation, each on a 256-byte boundary.
+class Block {
+ public:
+  // returns the position of a buffer of `bytes`
+  size_t add(int64_t bytes) {
+    const size_t at = size_;
+    size_ += ((size_t)(bytes > 0 ? bytes : 0) + 255) / 256 * 256;
+    return at;
+  }
+  void allocate(const Tensor& like) {
+    mem_ = at::empty({(int64_t)(size_ ? size_ : 256)}, like.options().dtype(at::kByte));
+    base_ = static_cast<char*>(mem_.data_ptr());
+  }
+  void adopt(Tensor mem) {
+    mem_ = std::move(mem);
+    base_ = static_cast<char*>(mem_.data_ptr());
+  }
+  void* at_(size_t pos) const { return base_ + pos; }
+  int32_t* i32(size_t pos) const { return reinterpret_cast<int32_t*>(base_ + pos); }
+  float* f32(size_t pos) const { return reinterpret_cast<float*>(base_ + pos); }
+  const Tensor& memory() const { return mem_; }
+
+ private:
+  size_t size_ = 0;
+  Tensor mem_;
+  char* base_ = nullptr;
+};
+
+// ------------------------------------------------------------------------------ Python-side switches
+std::atomic<bool> g_accumulate{false};       // functional.accumulate_weight_grads
+std::atomic<bool> g_overlap{false};          // functional.set_overlap_wgrad
+PyObject* g_queue = nullptr;                 // functional.defer_weight_grads: a WeightGradQueue or null
+std::atomic<bool> g_deferring{false};
+
+void push_deferred(std::function<void()> fn) {
+  py::gil_scoped_acquire gil;
+  py::handle(g_queue).attr("push")(py::cpp_function(std::move(fn)));
+}
+bool leaf(const Tensor& p) { return p.is_leaf() && p.requires_grad(); }
+// A leaf whose existing .grad the kernels can add to directly.
+bool accumulates_in_place(const Tensor& p) {
+  if (!p.defined() || !leaf(p)) return false;
+  const Tensor& g = p.grad();
+  return g.defined() && g.scalar_type() == p.scalar_type() && g.sizes() == p.sizes() && g.is_contiguous() && g.device() == p.device();
+}
+void add_or_set_grad(const Tensor& p, const Tensor& g) {
+  Tensor& slot = const_cast<Tensor&>(p).mutable_grad();
+  if (slot.defined()) {
+    at::NoGradGuard no_grad;
+    slot.add_(g);
+  } else {
+    slot = g;
+  }
+}
+
+// ------------------------------------------------------------------------------ router gate backward
+// d_x (fp32, may be null) and the gate weight / bias gradients of d_logits.
+void gate_bwd(const float* d_logits, const void* x, int x_dtype, const Tensor& w_gate, float* d_x32, const Tensor& d_w, const Tensor& d_b,
+              bool accumulate, int64_t T, int64_t H, int64_t E) {
+  Tensor ws;
+  if (d_w.defined()) {
+    const int64_t bytes = pk_gate_bwd_workspace_bytes(T, H, E);
+    if (bytes > 0) ws = at::empty({bytes}, w_gate.options().dtype(at::kByte));
+  }
+  PK_CALL(pk_gate_logits_bwd, d_logits, x, x_dtype, fptr(w_gate), d_x32, static_cast<float*>(ptr(d_w)),
+          static_cast<float*>(ptr(d_b)), accumulate ? 1 : 0, T, H, E, ptr(ws), ws.defined() ? ws.numel() : 0, stream_of(w_gate));
+}
+// d_w_gate (and d_gate_bias) added to / stored as the parameters' .grad.  The two may be at different
+// points of their accumulation (one of them cleared); the kernel has one flag for both.
+void router_weight_grads(const Tensor& p_gate, const Tensor& p_bias, const float* d_logits, const void* x, int x_dtype, const Tensor& w_gate,
+                         int64_t T, int64_t H, int64_t E) {
+  const bool have_w = p_gate.grad().defined(), have_b = p_bias.defined() && p_bias.grad().defined();
+  const auto f32 = w_gate.options();
+  if (!p_bias.defined() || have_w == have_b) {
+    Tensor gw = have_w ? p_gate.grad() : at::empty_like(p_gate);
+    Tensor gb = !p_bias.defined() ? Tensor() : have_b ? p_bias.grad() : at::empty({E}, f32);
+    gate_bwd(d_logits, x, x_dtype, w_gate, nullptr, gw, gb, have_w, T, H, E);
+    const_cast<Tensor&>(p_gate).mutable_grad() = gw;
+    if (p_bias.defined()) const_cast<Tensor&>(p_bias).mutable_grad() = gb;
+    return;
+  }
+  Tensor gw = at::empty_like(p_gate), gb = at::empty({E}, f32);
+  gate_bwd(d_logits, x, x_dtype, w_gate, nullptr, gw, gb, false, T, H, E);
+  add_or_set_grad(p_gate, gw);
+  add_or_set_grad(p_bias, gb);
+}
+
+// ------------------------------------------------------------------------------ the fused region
+struct Shape {
+  int64_t T, H, E, I, K, A;
+  int dtype;
+  int64_t es;
+  double route_scale, eps;
+  bool route_norm;
+};
+
+Shape region_shape(const Tensor& x, const Tensor& w_gate, const Tensor& bias, const Tensor& w1, const Tensor& w2, const Tensor& w3,
+                   int64_t top_k, bool route_norm, double route_scale, double eps, const Tensor& residual, const Tensor& norm_w) {
+  require_gpu(x);
+  TORCH_CHECK_VALUE(x.dim() == 2 && w_gate.dim() == 2 && x.size(1) == w_gate.size(1), "gate_logits: x [T,H], w_gate [E,H]");
+  TORCH_CHECK_VALUE(w_gate.scalar_type() == at::kFloat, "gate_logits: the router gate is kept in float32");
+  TORCH_CHECK_VALUE(w1.dim() == 3 && w2.dim() == 3 && w3.dim() == 3, "expert weights must be [E,I,H], [E,H,I], [E,I,H]");
+  Shape s;
+  s.T = x.size(0); s.H = x.size(1); s.E = w1.size(0); s.I = w1.size(1); s.K = top_k; s.A = s.T * top_k;
+  TORCH_CHECK_VALUE(w_gate.size(0) == s.E && w1.size(2) == s.H && w3.sizes() == w1.sizes() && w2.size(0) == s.E && w2.size(1) == s.H &&
+                        w2.size(2) == s.I, "expert weight shapes disagree");
+  TORCH_CHECK_VALUE(w1.scalar_type() == x.scalar_type() && w2.scalar_type() == x.scalar_type() && w3.scalar_type() == x.scalar_type(),
+                    "expert weights and activations must share a dtype");
+  TORCH_CHECK_VALUE(!bias.defined() || (bias.scalar_type() == at::kFloat && bias.dim() == 1 && bias.size(0) == s.E),
+                    "gate_logits: bias must be float32 [E]");
+  TORCH_CHECK_VALUE(!residual.defined() || (residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type()),
+                    "combine_fwd: residual must be [T,H] in the dtype of y");
+  TORCH_CHECK_VALUE(!norm_w.defined() || (norm_w.dim() == 1 && norm_w.size(0) == s.H && norm_w.scalar_type() == x.scalar_type()),
+                    "rmsnorm_fwd: x [T,H], weight [H] in the dtype of x");
+  for (const Tensor* t : {&w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w})
+    TORCH_CHECK_VALUE(!t->defined() || t->device() == x.device(), "all tensors of a call must be on one device");
+  s.dtype = dtype_code(x);
+  s.es = s.dtype == PK_BF16 ? 2 : 4;
+  s.route_norm = route_norm; s.route_scale = route_scale; s.eps = eps;
+  return s;
+}
+
+// What a forward leaves for its backward, in one allocation.
+struct Saved {
+  Block mem;
+  size_t logits, scores, idx, starts, perm, inv, order, g, u, xn, rstd;
+  // grads: g and u are kept, and with a norm its output and 1/rms
+  Saved(const Shape& s, bool grads, bool norm) {
+    const int64_t es = s.es;
+    logits = mem.add(s.T * s.E * 4);
+    scores = mem.add(s.A * 4);
+    idx = mem.add(s.A * 4);
+    starts = mem.add((s.E + 1) * 4);
+    perm = mem.add(s.A * 4);
+    inv = mem.add(s.A * 4);
+    order = mem.add(s.E * 4);
+    xn = mem.add(norm ? s.T * s.H * es : 0);
+    rstd = mem.add(norm ? s.T * 4 : 0);
+    g = mem.add(grads ? s.A * s.I * es : 0);
+    u = mem.add(grads ? s.A * s.I * es : 0);
+  }
+};
+
+// The routing step through a Python callable (a replaced ops.route_topk: somebody records or forces the
+// choice): logits -> (scores, expert indices), copied to where the kernels expect them.
+void route_in_python(PyObject* route, const Shape& s, const Saved& sv, const Tensor& like) {
+  py::gil_scoped_acquire gil;
+  const auto keep = [mem = sv.mem.memory()](void*) {};
+  const auto f32 = like.options().dtype(at::kFloat);
+  Tensor logits = at::from_blob(sv.mem.at_(sv.logits), {s.T, s.E}, keep, f32);
+  py::tuple r = py::handle(route)(logits, s.K, s.route_norm, s.route_scale);
+  at::from_blob(sv.mem.at_(sv.scores), {s.T, s.K}, keep, f32).copy_(r[0].cast<Tensor>());
+  at::from_blob(sv.mem.at_(sv.idx), {s.T, s.K}, keep, f32.dtype(at::kInt)).copy_(r[1].cast<Tensor>());
+}
+
+// out = [residual +] region([norm](x)); every input contiguous
+Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, const Tensor& x, const Tensor& w_gate, const Tensor& bias, const Tensor& w1,
+                      const Tensor& w2, const Tensor& w3, const Tensor& residual, const Tensor& norm_w) {
+  Tensor out = at::empty({s.T, s.H}, x.options());
+  sv.mem.allocate(x);
+  Block tmp;
+  const int64_t gate_ws = pk_gate_workspace_bytes(s.T, s.H, s.E), sort_ws = pk_sort_workspace_bytes(s.A, s.E);
+  const size_t ws = tmp.add(std::max(gate_ws, sort_ws));
+  const size_t counts = tmp.add(s.E * 4);
+  const size_t h = tmp.add(s.A * s.I * s.es), y = tmp.add(s.A * s.H * s.es);
+  tmp.allocate(x);
+  const pk_stream_t st = stream_of(x);
+  const Block& m = sv.mem;
+  const void* xin = x.data_ptr();
+  if (norm_w.defined()) {
+    PK_CALL(pk_rmsnorm_fwd, xin, s.dtype, ptr(norm_w), (float)s.eps, m.at_(sv.xn), m.f32(sv.rstd), s.T, s.H, st);
+    xin = m.at_(sv.xn);
+  }
+  PK_CALL(pk_gate_logits, xin, s.dtype, fptr(w_gate), fptr(bias), m.f32(sv.logits), s.T, s.H, s.E, tmp.at_(ws), std::max<int64_t>(gate_ws, 0), st);
+  if (route) route_in_python(route, s, sv, x);
+  else PK_CALL(pk_route_topk, m.f32(sv.logits), s.T, s.E, s.K, s.route_norm, (float)s.route_scale, m.f32(sv.scores), m.i32(sv.idx), st);
+  PK_CALL(pk_sort_by_expert, m.i32(sv.idx), s.A, s.E, tmp.i32(counts), m.i32(sv.starts), m.i32(sv.perm), m.i32(sv.inv), m.i32(sv.order),
+          tmp.at_(ws), sort_ws, st);
+  PK_CALL(pk_grouped_swiglu_fwd, xin, m.i32(sv.perm), s.K, ptr(w1), ptr(w2), ptr(w3), m.i32(sv.starts), keep_gu ? m.at_(sv.g) : nullptr,
+          keep_gu ? m.at_(sv.u) : nullptr, tmp.at_(h), tmp.at_(y), s.A, s.H, s.I, s.E, s.dtype, st);
+  PK_CALL(pk_combine_fwd, tmp.at_(y), s.dtype, m.i32(sv.inv), m.f32(sv.scores), ptr(residual), ptr(out), s.T, s.H, s.K, st);
+  return out;
+}
+
+// Weight-gradient kernels of the fused region with everything they read.
+struct RegionWgrad {
+  Shape s;
+  Tensor d_out, x, saved, tmp;            // owners of the memory below
+  const void *x_rows, *d_g, *d_u, *hs;    // row-major, or
+  const void *d_gT, *d_uT, *hsT;          // the transposed copies
+  int64_t ldt;
+  const int32_t *perm, *starts, *order;
+  void operator()(const Tensor& dw1, const Tensor& dw2, const Tensor& dw3, bool accumulate) const {
+    const pk_stream_t st = stream_of(d_out);
+    if (ldt > 0)
+      PK_CALL(pk_grouped_swiglu_wgrad_scaled_t, ptr(d_out), hsT, d_gT, d_uT, ldt, x_rows, perm, s.K, starts, order, ptr(dw1), ptr(dw2),
+              ptr(dw3), accumulate, s.A, s.H, s.I, s.E, s.dtype, st);
+    else
+      PK_CALL(pk_grouped_swiglu_wgrad_scaled, ptr(d_out), hs, d_g, d_u, x_rows, perm, s.K, starts, order, ptr(dw1), ptr(dw2), ptr(dw3),
+              accumulate, s.A, s.H, s.I, s.E, s.dtype, st);
+  }
+};
+// `wgrad` into the three parameters' .grad: inside the kernels where all three exist
+template <typename F>
+void weight_grads_into_params(const Tensor& p1, const Tensor& p2, const Tensor& p3, const F& wgrad) {
+  if (p1.grad().defined() && p2.grad().defined() && p3.grad().defined()) {
+    wgrad(p1.grad(), p2.grad(), p3.grad(), true);
+    return;
+  }
+  Tensor g1 = at::empty_like(p1, at::MemoryFormat::Contiguous), g2 = at::empty_like(p2, at::MemoryFormat::Contiguous),
+         g3 = at::empty_like(p3, at::MemoryFormat::Contiguous);
+  wgrad(g1, g2, g3, false);
+  add_or_set_grad(p1, g1);
+  add_or_set_grad(p2, g2);
+  add_or_set_grad(p3, g3);
+}
+
+c10::hip::HIPStream side_stream(int dev) {
+  static std::mutex mu;
+  static std::vector<std::optional<c10::hip::HIPStream>> streams(64);
+  std::lock_guard<std::mutex> lock(mu);
+  if (!streams[dev]) streams[dev] = c10::hip::getStreamFromPool(false, dev);
+  return *streams[dev];
+}
+// ROCm tensors call their device type CUDA, and record_stream wants a stream of that type
+c10::Stream as_cuda(const c10::hip::HIPStream& s) {
+  return c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::CUDA, s.device_index()), s.id());
+}
+// `waiter` waits for everything queued on `other` so far
+void wait_stream(hipStream_t waiter, hipStream_t other) {
+  hipEvent_t e;
+  TORCH_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
+  const bool fine = hipEventRecord(e, other) == hipSuccess && hipStreamWaitEvent(waiter, e, 0) == hipSuccess;
+  (void)hipEventDestroy(e);
+  TORCH_CHECK(fine, "event between two streams failed");
+}
+
+// x [T,H] -> out [T,H]; with norm_w the norm in front of the region belongs to the node and x is its
+// own residual (h + moe(ffn_norm(h))): the backward then adds the residual branch's gradient inside the
+// norm's backward kernel.
+struct RegionFn : public torch::autograd::Function<RegionFn> {
+  enum { X, W_GATE, BIAS, W1, W2, W3, RESIDUAL, NORM_W, N_TENSORS };
+
+  // (tensors that are absent are passed as empty optionals: autograd gives them no edge)
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w_gate, const OptTensor& bias_, const Tensor& w1, const Tensor& w2,
+                        const Tensor& w3, const OptTensor& residual_, const OptTensor& norm_w_, int64_t top_k, bool route_norm,
+                        double route_scale, double eps, PyObject* route) {
+    const Tensor bias = opt(bias_), residual = opt(residual_), norm_w = opt(norm_w_);
+    const Shape s = region_shape(x, w_gate, bias, w1, w2, w3, top_k, route_norm, route_scale, eps, residual, norm_w);
+    const bool norm = norm_w.defined();
+    Saved sv(s, true, norm);
+    const Tensor xc = contig(x);
+    Tensor out = region_forward(s, route, sv, true, xc, contig(w_gate), contig(bias), contig(w1), contig(w2), contig(w3),
+                                norm ? xc : contig(residual), contig(norm_w));
+    ctx->save_for_backward({x, w_gate, bias, w1, w2, w3, norm_w, sv.mem.memory()});
+    ctx->saved_data["k"] = top_k;
+    ctx->saved_data["norm"] = route_norm;
+    ctx->saved_data["scale"] = route_scale;
+    ctx->saved_data["eps"] = eps;
+    ctx->saved_data["residual"] = residual.defined();
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &p_gate = saved[1], &p_bias = saved[2], &p1 = saved[3], &p2 = saved[4], &p3 = saved[5], &norm_w = saved[6];
+    const bool norm = norm_w.defined();
+    const Shape s = region_shape(x, p_gate, p_bias, p1, p2, p3, ctx->saved_data["k"].toInt(), ctx->saved_data["norm"].toBool(),
+                                 ctx->saved_data["scale"].toDouble(), ctx->saved_data["eps"].toDouble(), Tensor(), norm_w);
+    Saved sv(s, true, norm);
+    sv.mem.adopt(saved[7]);
+    const Block& m = sv.mem;
+    bool need[N_TENSORS];
+    const bool present[N_TENSORS] = {true, true, p_bias.defined(), true, true, true, ctx->saved_data["residual"].toBool(), norm};
+    for (int i = 0, edge = 0; i < N_TENSORS; ++i) need[i] = present[i] && ctx->needs_input_grad(edge++);
+    const bool need_xn = need[X] || (norm && need[NORM_W]);      // the gradient of what the router and the experts read
+    const Tensor d_out = contig(grads[0]);
+    const Tensor xc = contig(x), w_gate = contig(p_gate), w1 = contig(p1), w2 = contig(p2), w3 = contig(p3);
+    const void* x_rows = norm ? m.at_(sv.xn) : xc.data_ptr();
+    const int32_t *perm = m.i32(sv.perm), *starts = m.i32(sv.starts);
+
+    // Shapes with a K-contiguous weight-gradient path get d_g, d_u and score*h transposed; with long
+    // experts the d_x GEMM reads its A operand from the same blocks and the row-major pair is left out.
+    const int64_t ldt = s.dtype == PK_BF16 ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
+    const bool blocks_only = ldt > 0 && pk_grouped_swiglu_dx_from_transposed_pays(s.A, s.H, s.I, s.E, s.dtype);
+    Block t;
+    const int64_t ai = s.A * s.I * s.es, ait = ldt * s.I * s.es;
+    const int64_t ds_ws = std::max<int64_t>(pk_grouped_swiglu_dgrad_dh_scaled_workspace_bytes(s.A, s.I), 4);
+    const size_t d_g = t.add(blocks_only ? 0 : ai), d_u = t.add(blocks_only ? 0 : ai), hs = t.add(ldt > 0 ? 0 : ai);
+    const size_t d_gT = t.add(ait), d_uT = t.add(ait), hsT = t.add(ait);
+    const size_t d_scores = t.add(s.A * 4), part = t.add(ds_ws), d_logits = t.add(s.T * s.E * 4);
+    const size_t d_xs = t.add(need_xn ? s.A * s.H * s.es : 0), d_x32 = t.add(need_xn ? s.T * s.H * 4 : 0);
+    const size_t d_xn = t.add(norm && need_xn ? s.T * s.H * s.es : 0);
+    t.allocate(x);
+    const pk_stream_t st = stream_of(x);
+    void *dg = blocks_only ? nullptr : t.at_(d_g), *du = blocks_only ? nullptr : t.at_(d_u);
+    // the combine backward is folded into the d_h GEMM: d_out rows are gathered per routed row, the score
+    // is applied in the epilogue
+    if (ldt > 0)
+      PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled_t, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
+              t.at_(d_gT), t.at_(d_uT), t.at_(hsT), ldt, t.f32(d_scores), t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
+    else
+      PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
+              t.at_(hs), t.f32(d_scores), t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
+
+    const RegionWgrad wgrad{s, d_out, xc, sv.mem.memory(), t.memory(), x_rows, dg, du, t.at_(hs), t.at_(d_gT), t.at_(d_uT), t.at_(hsT),
+                            ldt, perm, starts, m.i32(sv.order)};
+    const bool any_w = need[W1] || need[W2] || need[W3], all_w = need[W1] && need[W2] && need[W3];
+    const auto input_grad = [&] {
+      if (!need_xn) return;
+      if (blocks_only)
+        PK_CALL(pk_grouped_swiglu_dgrad_dx_t, t.at_(d_gT), t.at_(d_uT), ldt, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
+      else
+        PK_CALL(pk_grouped_swiglu_dgrad_dx, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
+    };
+    const auto route_bwd = [&] {
+      PK_CALL(pk_route_topk_bwd, m.f32(sv.logits), m.i32(sv.idx), t.f32(d_scores), s.T, s.E, s.K, s.route_norm, (float)s.route_scale,
+              t.f32(d_logits), st);
+    };
+    Tensor d_x, d_norm_w;
+    const auto finish_input = [&] {
+      if (!need_xn) return;
+      Tensor dest = need[X] && !norm ? at::empty({s.T, s.H}, x.options()) : Tensor();
+      void* const to = norm ? t.at_(d_xn) : ptr(dest);
+      PK_CALL(pk_permute_bwd, t.at_(d_xs), s.dtype, m.i32(sv.inv), t.f32(d_x32), to, s.T, s.H, s.K, st);
+      if (!norm) { d_x = dest; return; }
+      d_x = at::empty({s.T, s.H}, x.options());
+      Tensor ws;
+      if (need[NORM_W]) {
+        d_norm_w = at::empty({s.H}, norm_w.options());
+        ws = at::empty({pk_rmsnorm_bwd_workspace_bytes(s.T, s.H)}, x.options().dtype(at::kByte));
+      }
+      PK_CALL(pk_rmsnorm_bwd, to, ptr(xc), s.dtype, ptr(contig(norm_w)), m.f32(sv.rstd), ptr(d_out), ptr(d_x), ptr(d_norm_w), 0, s.T, s.H,
+              ptr(ws), ws.defined() ? ws.numel() : 0, st);
+      if (!need[X]) d_x = Tensor();
+    };
+    Tensor d_w1, d_w2, d_w3, d_wg, d_b;
+    const Tensor d_res = !norm && need[RESIDUAL] ? d_out : Tensor();
+
+    if (g_deferring.load() && all_w && need[W_GATE] && leaf(p_gate) && (!p_bias.defined() || leaf(p_bias)) && leaf(p1) && leaf(p2) && leaf(p3)) {
+      // backward-input pass: the weight gradients of the experts and of the router gate are queued with
+      // the tensors they need and computed by the weight pass
+      push_deferred([wgrad, p1, p2, p3] { weight_grads_into_params(p1, p2, p3, wgrad); });
+      input_grad();
+      route_bwd();
+      if (need_xn) gate_bwd(t.f32(d_logits), x_rows, s.dtype, w_gate, t.f32(d_x32), Tensor(), Tensor(), false, s.T, s.H, s.E);
+      finish_input();
+      push_deferred([s, p_gate, p_bias, w_gate, x_rows, dl = t.f32(d_logits), keep = std::array<Tensor, 3>{t.memory(), sv.mem.memory(), xc}] {
+        router_weight_grads(p_gate, p_bias, dl, x_rows, s.dtype, w_gate, s.T, s.H, s.E);
+      });
+      return {d_x, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), d_res, d_norm_w, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+    // backward into .grad with gradients already there (a later microbatch of an iteration): the
+    // weight-gradient kernels add to them in their epilogues and autograd gets nothing to add
+    const bool acc = g_accumulate.load();
+    const bool experts_in_place = acc && all_w && accumulates_in_place(p1) && accumulates_in_place(p2) && accumulates_in_place(p3);
+    const bool gate_in_place = acc && need[W_GATE] && accumulates_in_place(p_gate) && (!p_bias.defined() || (need[BIAS] && leaf(p_bias)));
+    const bool overlap = any_w && g_overlap.load() && !experts_in_place;
+    const auto cur = c10::hip::getCurrentHIPStream(x.get_device());
+    if (experts_in_place) {
+      wgrad(p1.grad(), p2.grad(), p3.grad(), true);
+    } else if (any_w) {
+      const auto fresh = [&] {
+        d_w1 = at::empty({s.E, s.I, s.H}, x.options());
+        d_w2 = at::empty({s.E, s.H, s.I}, x.options());
+        d_w3 = at::empty({s.E, s.I, s.H}, x.options());
+        wgrad(d_w1, d_w2, d_w3, false);
+      };
+      if (overlap) {
+        const auto side = side_stream(x.get_device());
+        wait_stream(side.stream(), cur.stream());
+        c10::hip::HIPStreamGuard guard(side);
+        fresh();
+      } else {
+        fresh();
+      }
+    }
+    input_grad();
+    route_bwd();
+    if (gate_in_place) {
+      if (need_xn) gate_bwd(t.f32(d_logits), x_rows, s.dtype, w_gate, t.f32(d_x32), Tensor(), Tensor(), false, s.T, s.H, s.E);
+      router_weight_grads(p_gate, p_bias, t.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
+    } else {
+      if (need[W_GATE]) d_wg = at::empty({s.E, s.H}, w_gate.options());
+      if (p_bias.defined() && need[BIAS]) d_b = at::empty({s.E}, w_gate.options());
+      if (need_xn || d_wg.defined() || d_b.defined())
+        gate_bwd(t.f32(d_logits), x_rows, s.dtype, w_gate, need_xn ? t.f32(d_x32) : nullptr, d_wg, d_b, false, s.T, s.H, s.E);
+    }
+    finish_input();
+    if (overlap) {
+      const auto side = side_stream(x.get_device());
+      wait_stream(cur.stream(), side.stream());
+      for (const Tensor* b : {&d_out, &xc, &sv.mem.memory(), &t.memory()}) b->record_stream(as_cuda(side));
+      for (const Tensor* b : {&d_w1, &d_w2, &d_w3}) b->record_stream(as_cuda(cur));
+    }
+    return {d_x, d_wg, d_b, d_w1, d_w2, d_w3, d_res, d_norm_w, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+// None (with `direct`): not ordinary GPU tensors, or a tracing mode is on
+std::optional<Tensor> expert_region(const Tensor& x, const Tensor& w_gate, const OptTensor& bias_, const Tensor& w1, const Tensor& w2,
+                                    const Tensor& w3, int64_t top_k, bool route_norm, double route_scale, const OptTensor& residual_,
+                                    const OptTensor& norm_w_, double eps, const py::object& route_, bool direct) {
+  PyObject* const route = route_.ptr() == Py_None ? nullptr : route_.ptr();
+  const Tensor bias = opt(bias_), residual = opt(residual_), norm_w = opt(norm_w_);
+  if (direct && !plain({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w})) return std::nullopt;
+  require_gpu(x);
+  c10::hip::HIPGuard device(x.device().index());
+  if (wants_grad({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w}))
+    return RegionFn::apply(x, w_gate, bias_, w1, w2, w3, residual_, norm_w_, top_k, route_norm, route_scale, eps, route);
+  const Shape s = region_shape(x, w_gate, bias, w1, w2, w3, top_k, route_norm, route_scale, eps, residual, norm_w);
+  const Tensor xc = contig(x), w1c = contig(w1), w2c = contig(w2), w3c = contig(w3);
+  // without a backward the pre-activations need not be written, except by the any-width kernels
+  const int64_t piece = 16 / s.es;
+  const bool keep_gu = s.H % piece != 0 || s.I % piece != 0 || !aligned16(xc) || !aligned16(w1c) || !aligned16(w2c) || !aligned16(w3c);
+  Saved sv(s, keep_gu, norm_w.defined());
+  return region_forward(s, route, sv, keep_gu, xc, contig(w_gate), contig(bias), w1c, w2c, w3c, norm_w.defined() ? xc : contig(residual), contig(norm_w));
+}
+
+// ------------------------------------------------------------------------------ RMSNorm
+struct NormFn : public torch::autograd::Function<NormFn> {
+  static Tensor run(const Tensor& x, const Tensor& w, double eps, const Tensor& rstd) {
+    TORCH_CHECK_VALUE(x.dim() == 2 && w.dim() == 1 && w.size(0) == x.size(1) && w.scalar_type() == x.scalar_type(),
+                      "rmsnorm_fwd: x [T,H], weight [H] in the dtype of x");
+    const Tensor xc = contig(x);
+    Tensor y = at::empty({x.size(0), x.size(1)}, x.options());
+    PK_CALL(pk_rmsnorm_fwd, ptr(xc), dtype_code(x), ptr(contig(w)), (float)eps, ptr(y), static_cast<float*>(ptr(rstd)), x.size(0), x.size(1),
+            stream_of(x));
+    return y;
+  }
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
+    require_gpu(x);
+    Tensor rstd = at::empty({x.size(0)}, x.options().dtype(at::kFloat));
+    Tensor y = run(x, w, eps, rstd);
+    ctx->save_for_backward({x, w, rstd});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor x = contig(sv[0]), w = contig(sv[1]), d_y = contig(grads[0]);
+    const int64_t T = x.size(0), H = x.size(1);
+    Tensor d_x = at::empty_like(x), d_w, ws;
+    if (ctx->needs_input_grad(1)) {
+      d_w = at::empty_like(w);
+      ws = at::empty({pk_rmsnorm_bwd_workspace_bytes(T, H)}, x.options().dtype(at::kByte));
+    }
+    PK_CALL(pk_rmsnorm_bwd, ptr(d_y), ptr(x), dtype_code(x), ptr(w), fptr(sv[2]), nullptr, ptr(d_x), ptr(d_w), 0, T, H, ptr(ws),
+            ws.defined() ? ws.numel() : 0, stream_of(x));
+    if (!ctx->needs_input_grad(0)) d_x = Tensor();
+    return {d_x, d_w, Tensor()};
+  }
+};
+std::optional<Tensor> rmsnorm(const Tensor& x, const Tensor& w, double eps, bool direct) {
+  if (direct && !plain({&x, &w})) return std::nullopt;
+  require_gpu(x);
+  c10::hip::HIPGuard device(x.device().index());
+  return wants_grad({&x, &w}) ? NormFn::apply(x, w, eps) : NormFn::run(x, w, eps, Tensor());
+}
+
+// ------------------------------------------------------------------------------ piecewise operators
+// (counts [E], starts [E+1], perm [A], inv_perm [A]) of the stable counting sort of top_idx
+std::vector<Tensor> sort_by_expert(const Tensor& top_idx, int64_t E) {
+  require_gpu(top_idx);
+  TORCH_CHECK_VALUE(top_idx.scalar_type() == at::kInt, "sort_by_expert: top_idx must be int32");
+  const Tensor flat = contig(top_idx);
+  const int64_t A = flat.numel(), ws_bytes = pk_sort_workspace_bytes(A, E);
+  TORCH_CHECK(ws_bytes >= 0, "pk_sort_workspace_bytes failed: ", pk_status_string((int)ws_bytes));
+  const auto i32 = flat.options();
+  Tensor counts = at::empty({E}, i32), starts = at::empty({E + 1}, i32), perm = at::empty({A}, i32), inv = at::empty({A}, i32);
+  Tensor ws = at::empty({std::max<int64_t>(ws_bytes, 4)}, i32.dtype(at::kByte));
+  PK_CALL(pk_sort_by_expert, flat.data_ptr<int32_t>(), A, E, counts.data_ptr<int32_t>(), starts.data_ptr<int32_t>(), perm.data_ptr<int32_t>(),
+          inv.data_ptr<int32_t>(), nullptr, ptr(ws), ws.numel(), stream_of(flat));
+  return {counts, starts, perm, inv};
+}
+
+struct RouterFn : public torch::autograd::Function<RouterFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w_gate, const OptTensor& bias_, int64_t top_k, bool route_norm,
+                               double route_scale, PyObject* route) {
+    require_gpu(x);
+    const Tensor bias = opt(bias_);
+    TORCH_CHECK_VALUE(x.dim() == 2 && w_gate.dim() == 2 && x.size(1) == w_gate.size(1), "gate_logits: x [T,H], w_gate [E,H]");
+    TORCH_CHECK_VALUE(w_gate.scalar_type() == at::kFloat, "gate_logits: the router gate is kept in float32");
+    const int64_t T = x.size(0), H = x.size(1), E = w_gate.size(0);
+    TORCH_CHECK_VALUE(!bias.defined() || (bias.scalar_type() == at::kFloat && bias.dim() == 1 && bias.size(0) == E),
+                      "gate_logits: bias must be float32 [E]");
+    const auto f32 = x.options().dtype(at::kFloat);
+    Tensor logits = at::empty({T, E}, f32), scores = at::empty({T, top_k}, f32), idx = at::empty({T, top_k}, f32.dtype(at::kInt));
+    const int64_t ws_bytes = pk_gate_workspace_bytes(T, H, E);
+    Tensor ws = ws_bytes > 0 ? at::empty({ws_bytes}, f32.dtype(at::kByte)) : Tensor();
+    const pk_stream_t st = stream_of(x);
+    PK_CALL(pk_gate_logits, ptr(contig(x)), dtype_code(x), fptr(contig(w_gate)), fptr(contig(bias)), logits.data_ptr<float>(), T, H, E, ptr(ws),
+            ws.defined() ? ws_bytes : 0, st);
+    if (route) {
+      py::gil_scoped_acquire gil;
+      py::tuple r = py::handle(route)(logits, top_k, route_norm, route_scale);
+      scores.copy_(r[0].cast<Tensor>());
+      idx.copy_(r[1].cast<Tensor>());
+    } else {
+      PK_CALL(pk_route_topk, logits.data_ptr<float>(), T, E, top_k, route_norm, (float)route_scale, scores.data_ptr<float>(),
+              idx.data_ptr<int32_t>(), st);
+    }
+    ctx->save_for_backward({x, w_gate, bias, logits, idx});
+    ctx->saved_data["norm"] = route_norm;
+    ctx->saved_data["scale"] = route_scale;
+    ctx->mark_non_differentiable({idx});
+    return {scores, idx};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor x = contig(sv[0]), w_gate = contig(sv[1]), logits = sv[3], idx = sv[4];
+    const int64_t T = x.size(0), H = x.size(1), E = w_gate.size(0), K = idx.size(1);
+    Tensor d_s = grads[0].defined() ? contig(grads[0]).to(at::kFloat) : at::zeros({T, K}, logits.options());
+    Tensor d_logits = at::empty_like(logits);
+    PK_CALL(pk_route_topk_bwd, fptr(logits), idx.data_ptr<int32_t>(), fptr(d_s), T, E, K, ctx->saved_data["norm"].toBool(),
+            (float)ctx->saved_data["scale"].toDouble(), d_logits.data_ptr<float>(), stream_of(x));
+    Tensor d_x32, d_w, d_b;
+    if (ctx->needs_input_grad(0)) d_x32 = at::empty({T, H}, logits.options());
+    if (ctx->needs_input_grad(1)) d_w = at::empty({E, H}, logits.options());
+    if (sv[2].defined() && ctx->needs_input_grad(2)) d_b = at::empty({E}, logits.options());
+    gate_bwd(fptr(d_logits), ptr(x), dtype_code(x), w_gate, static_cast<float*>(ptr(d_x32)), d_w, d_b, false, T, H, E);
+    return {d_x32.defined() ? d_x32.to(x.scalar_type()) : Tensor(), d_w, d_b, Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+std::pair<Tensor, Tensor> router(const Tensor& x, const Tensor& w_gate, const OptTensor& bias, int64_t top_k, bool route_norm, double route_scale,
+                                 const py::object& route) {
+  require_gpu(x);
+  c10::hip::HIPGuard device(x.device().index());
+  auto r = RouterFn::apply(x, w_gate, bias, top_k, route_norm, route_scale, route.ptr() == Py_None ? nullptr : route.ptr());
+  return {r[0], r[1]};
+}
+
+struct PermuteFn : public torch::autograd::Function<PermuteFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& perm, const Tensor& inv, int64_t top_k) {
+    require_gpu(x);
+    const int64_t H = x.size(1), A = perm.numel();
+    Tensor routed = at::empty({A, H}, x.options());
+    PK_CALL(pk_permute_fwd, ptr(contig(x)), dtype_code(x), contig(perm).data_ptr<int32_t>(), ptr(routed), A, H, top_k, stream_of(x));
+    ctx->save_for_backward({inv});
+    ctx->saved_data["k"] = top_k;
+    return routed;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const Tensor d = contig(grads[0]), inv = ctx->get_saved_variables()[0];
+    const int64_t K = ctx->saved_data["k"].toInt(), T = d.size(0) / K, H = d.size(1);
+    Tensor d_x = at::empty({T, H}, d.options());
+    PK_CALL(pk_permute_bwd, ptr(d), dtype_code(d), inv.data_ptr<int32_t>(), nullptr, ptr(d_x), T, H, K, stream_of(d));
+    return {d_x, Tensor(), Tensor(), Tensor()};
+  }
+};
+Tensor permute(const Tensor& x, const Tensor& perm, const Tensor& inv, int64_t top_k) {
+  require_gpu(x);
+  c10::hip::HIPGuard device(x.device().index());
+  return PermuteFn::apply(x, perm, inv, top_k);
+}
+
+struct CombineFn : public torch::autograd::Function<CombineFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& y, const Tensor& perm, const Tensor& inv, const Tensor& scores) {
+    require_gpu(y);
+    const int64_t A = y.size(0), H = y.size(1), T = scores.size(0), K = scores.size(1);
+    TORCH_CHECK_VALUE(A == T * K, "combine_fwd: y_sorted rows must equal T*K");
+    Tensor out = at::empty({T, H}, y.options());
+    PK_CALL(pk_combine_fwd, ptr(contig(y)), dtype_code(y), contig(inv).data_ptr<int32_t>(), fptr(contig(scores)), nullptr, ptr(out), T, H, K, stream_of(y));
+    ctx->save_for_backward({y, perm, scores});
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor y = contig(sv[0]), perm = contig(sv[1]), scores = contig(sv[2]), d_out = contig(grads[0]);
+    const int64_t A = y.size(0), H = y.size(1), K = scores.size(1);
+    Tensor d_y = at::empty({A, H}, y.options()), d_s = at::empty({scores.size(0), K}, scores.options());
+    PK_CALL(pk_combine_bwd, ptr(d_out), ptr(y), dtype_code(y), perm.data_ptr<int32_t>(), fptr(scores), ptr(d_y), d_s.data_ptr<float>(), A, H, K, stream_of(y));
+    return {d_y, Tensor(), Tensor(), d_s};
+  }
+};
+Tensor combine(const Tensor& y, const Tensor& perm, const Tensor& inv, const Tensor& scores) {
+  require_gpu(y);
+  c10::hip::HIPGuard device(y.device().index());
+  return CombineFn::apply(y, perm, inv, scores);
+}
+
+// ------------------------------------------------------------------------------ bmm_experts
+struct ExpertsFn : public torch::autograd::Function<ExpertsFn> {
+  static Tensor counts_to_starts(const Tensor& counts) {
+    TORCH_CHECK_VALUE(counts.scalar_type() == at::kInt || counts.scalar_type() == at::kLong, "counts must be int32 or int64");
+    Tensor starts = at::empty({counts.numel() + 1}, counts.options().dtype(at::kInt));
+    PK_CALL(pk_counts_to_starts, ptr(contig(counts)), counts.scalar_type() == at::kLong, counts.numel(), starts.data_ptr<int32_t>(), stream_of(counts));
+    return starts;
+  }
+  // rows past sum(num_tokens_per_expert) belong to no expert: zeros, as in the reference
+  // (qwen3_bmm_experts_patch.py:43); the kernels only write rows below starts[E]
+  static void zero_tail(const Tensor& buf, const Tensor& starts) {
+    PK_CALL(pk_zero_rows_from, ptr(buf), dtype_code(buf), starts.data_ptr<int32_t>() + starts.numel() - 1, buf.size(0), buf.size(1), stream_of(buf));
+  }
+  // y [A,H]; the pre-activations and h are left in one tensor [3,A,I]
+  static Tensor run(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& starts, Tensor& guh) {
+    TORCH_CHECK_VALUE(w1.dim() == 3 && w2.dim() == 3 && w3.dim() == 3, "expert weights must be [E,I,H], [E,H,I], [E,I,H]");
+    const int64_t E = w1.size(0), I = w1.size(1), H = w1.size(2), A = x.size(0);
+    TORCH_CHECK_VALUE(w3.sizes() == w1.sizes() && w2.size(0) == E && w2.size(1) == H && w2.size(2) == I, "expert weight shapes disagree");
+    TORCH_CHECK_VALUE(w1.scalar_type() == x.scalar_type() && w2.scalar_type() == x.scalar_type() && w3.scalar_type() == x.scalar_type(),
+                      "expert weights and activations must share a dtype");
+    guh = at::empty({3, A, I}, x.options());
+    Tensor y = at::empty({A, H}, x.options());
+    char* const g = static_cast<char*>(guh.data_ptr());
+    const int64_t step = A * I * x.element_size();
+    PK_CALL(pk_grouped_swiglu_fwd, ptr(contig(x)), nullptr, 1, ptr(contig(w1)), ptr(contig(w2)), ptr(contig(w3)), starts.data_ptr<int32_t>(), g,
+            g + step, g + 2 * step, ptr(y), A, H, I, E, dtype_code(x), stream_of(x));
+    zero_tail(y, starts);
+    return y;
+  }
+  static Tensor forward(AutogradContext* ctx, const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& counts) {
+    require_gpu(x);
+    Tensor starts = counts_to_starts(counts), guh;
+    Tensor y = run(w1, w2, w3, x, starts, guh);
+    ctx->save_for_backward({w1, w2, w3, x, starts, guh});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor &p1 = sv[0], &p2 = sv[1], &p3 = sv[2], starts = sv[4], guh = sv[5];
+    const Tensor w1 = contig(p1), w2 = contig(p2), w3 = contig(p3), x = contig(sv[3]), d_y = contig(grads[0]);
+    const int64_t E = w1.size(0), I = w1.size(1), H = w1.size(2), A = x.size(0);
+    const int code = dtype_code(x);
+    const pk_stream_t st = stream_of(x);
+    const int64_t step = A * I * x.element_size();
+    char* const g = static_cast<char*>(guh.data_ptr());
+    Tensor dgu = at::empty({2, A, I}, x.options()), d_x = at::empty({A, H}, x.options());
+    char* const dg = static_cast<char*>(dgu.data_ptr());
+    PK_CALL(pk_grouped_swiglu_dgrad, ptr(d_y), ptr(w1), ptr(w2), ptr(w3), g, g + step, starts.data_ptr<int32_t>(), dg, dg + step, ptr(d_x), A, H, I, E, code, st);
+    zero_tail(d_x, starts);
+    const auto wgrad = [=](const Tensor& d1, const Tensor& d2, const Tensor& d3, bool accumulate) {
+      char* const gs = static_cast<char*>(guh.data_ptr());
+      char* const ds = static_cast<char*>(dgu.data_ptr());
+      PK_CALL(pk_grouped_swiglu_wgrad, ptr(d_y), gs + 2 * step, ds, ds + step, ptr(x), nullptr, 1, starts.data_ptr<int32_t>(), nullptr, ptr(d1),
+              ptr(d2), ptr(d3), accumulate, A, H, I, E, code, stream_of(x));
+    };
+    Tensor d1, d2, d3;
+    const bool n1 = ctx->needs_input_grad(0), n2 = ctx->needs_input_grad(1), n3 = ctx->needs_input_grad(2);
+    if (n1 && n2 && n3 && g_deferring.load() && leaf(p1) && leaf(p2) && leaf(p3)) {
+      push_deferred([wgrad, p1, p2, p3] { weight_grads_into_params(p1, p2, p3, wgrad); });
+    } else if (n1 && n2 && n3 && g_accumulate.load() && accumulates_in_place(p1) && accumulates_in_place(p2) && accumulates_in_place(p3)) {
+      wgrad(p1.grad(), p2.grad(), p3.grad(), true);
+    } else if (n1 || n2 || n3) {
+      d1 = at::empty({E, I, H}, x.options());
+      d2 = at::empty({E, H, I}, x.options());
+      d3 = at::empty({E, I, H}, x.options());
+      wgrad(d1, d2, d3, false);
+    }
+    return {d1, d2, d3, d_x, Tensor()};
+  }
+};
+std::optional<Tensor> bmm_experts(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& counts, bool direct) {
+  require_gpu(x);
+  if (direct && !plain({&w1, &w2, &w3, &x, &counts})) return std::nullopt;
+  c10::hip::HIPGuard device(x.device().index());
+  if (wants_grad({&w1, &w2, &w3, &x})) return ExpertsFn::apply(w1, w2, w3, x, counts);
+  Tensor guh;
+  return ExpertsFn::run(w1, w2, w3, x, ExpertsFn::counts_to_starts(counts), guh);
+}
+
+// ------------------------------------------------------------------------------ bucket path
+// A bucket's tensors with their places, as BucketState.param_view_specs lists them:
+// (parameter, element offset, element count, shape).
+PyObject* spec_item(PyObject* spec, int i) {
+  TORCH_CHECK_TYPE(PyTuple_Check(spec) && PyTuple_GET_SIZE(spec) > i, "param_view_specs: tuples (param, offset, numel, shape)");
+  return PyTuple_GET_ITEM(spec, i);
+}
+Tensor spec_param(PyObject* spec) {
+  PyObject* const p = spec_item(spec, 0);
+  TORCH_CHECK_TYPE(THPVariable_Check(p), "param_view_specs: tuples (param, offset, numel, shape)");
+  return THPVariable_Unpack(p);
+}
+int64_t spec_int(PyObject* spec, int i) { return PyLong_AsLongLong(spec_item(spec, i)); }
+
+std::optional<c10::Stream> unpack_stream(const std::optional<std::tuple<int64_t, int64_t, int64_t>>& s) {
+  if (!s) return std::nullopt;
+  return c10::Stream::unpack3(std::get<0>(*s), (c10::DeviceIndex)std::get<1>(*s), (c10::DeviceType)std::get<2>(*s));
+}
+
+// Takes the gradients off the parameters (p.grad = None); undefined where there was none.  With a
+// stream the memory is marked as used on it.
+std::vector<Tensor> take_grads(const py::list& specs, const std::optional<c10::Stream>& stream) {
+  std::vector<Tensor> grads;
+  grads.reserve(specs.size());
+  for (const py::handle spec : specs) {
+    Tensor p = spec_param(spec.ptr());
+    Tensor g = p.grad();
+    if (g.defined()) {
+      if (g.requires_grad()) g = g.detach();
+      if (stream) g.record_stream(*stream);
+      p.mutable_grad().reset();
+    }
+    grads.push_back(std::move(g));
+  }
+  return grads;
+}
+// flat[off : off + n] += grad.to(flat.dtype) for the bucket's gradients, one launch per gradient dtype;
+// the parameters end without gradients.
+void pack_param_grads(const py::list& specs, const Tensor& flat, const std::optional<std::tuple<int64_t, int64_t, int64_t>>& stream) {
+  require_gpu(flat);
+  const std::vector<Tensor> grads = take_grads(specs, unpack_stream(stream));
+  const size_t n = grads.size();
+  std::vector<const void*> ptrs(n);
+  std::vector<int64_t> offs(n), nums(n);
+  std::vector<Tensor> keep;
+  for (const at::ScalarType want : {at::kBFloat16, at::kFloat}) {
+    size_t m = 0;
+    for (size_t i = 0; i < n; ++i) {
+      if (!grads[i].defined()) continue;
+      dtype_code(grads[i]);
+      if (grads[i].scalar_type() != want) continue;
+      Tensor g = contig(grads[i]);
+      ptrs[m] = g.data_ptr();
+      if (!g.is_same(grads[i])) keep.push_back(g);
+      PyObject* const spec = PyList_GET_ITEM(specs.ptr(), i);
+      offs[m] = spec_int(spec, 1);
+      nums[m] = g.numel();
+      TORCH_CHECK_VALUE(offs[m] >= 0 && offs[m] + nums[m] <= flat.numel(), "bucket_pack: tensor outside the bucket");
+      ++m;
+    }
+    if (m)
+      PK_CALL(pk_bucket_pack, ptrs.data(), offs.data(), nums.data(), (int64_t)m, want == at::kBFloat16 ? PK_BF16 : PK_F32, flat.data_ptr(),
+              dtype_code(flat), 1, stream_of(flat));
+  }
+}
+std::vector<Tensor> hold_param_grads(const py::list& specs, const std::optional<std::tuple<int64_t, int64_t, int64_t>>& stream) {
+  return take_grads(specs, unpack_stream(stream));
+}
+void clear_param_grads(const py::list& specs) {
+  for (const py::handle spec : specs) {
+    Tensor p = spec_param(spec.ptr());
+    p.mutable_grad().reset();
+  }
+}
+
+void adamw_packed(const Tensor& master, const Tensor& exp_avg, const Tensor& exp_avg_sq, const Tensor& flat_grad, const std::vector<OptTensor>& grads,
+                  const std::vector<int64_t>& offsets, const std::vector<int64_t>& numels, int64_t step, double lr, double beta1, double beta2,
+                  double eps, double weight_decay, const Tensor& shadow, double grad_scale, bool zero_grad) {
+  require_gpu(master);
+  const size_t n = grads.size();
+  TORCH_CHECK_VALUE(offsets.size() == n && numels.size() == n, "adamw_fused_packed: one offset and element count per tensor");
+  const int64_t total = master.numel();
+  for (const Tensor* t : {&master, &exp_avg, &exp_avg_sq})
+    TORCH_CHECK_VALUE(t->scalar_type() == at::kFloat && t->numel() == total && t->is_contiguous(), "adamw_fused_packed: fp32 contiguous buffers of equal size");
+  TORCH_CHECK_VALUE(!flat_grad.defined() || (flat_grad.scalar_type() == at::kFloat && flat_grad.numel() == total && flat_grad.is_contiguous()),
+                    "adamw_fused_packed: flat_grad must match the bucket");
+  TORCH_CHECK_VALUE(!shadow.defined() || (shadow.scalar_type() == at::kBFloat16 && shadow.numel() == total && shadow.is_contiguous()),
+                    "adamw_fused_packed: bf16 shadow of the bucket's size");
+  std::vector<const void*> ptrs(std::max<size_t>(n, 1), nullptr);
+  std::vector<Tensor> keep;
+  std::optional<at::ScalarType> dtype;
+  for (size_t i = 0; i < n; ++i) {
+    TORCH_CHECK_VALUE(offsets[i] >= 0 && offsets[i] + numels[i] <= total, "adamw_fused_packed: tensor outside the bucket");
+    if (!grads[i].has_value() || !grads[i]->defined()) continue;
+    const Tensor& g = *grads[i];
+    TORCH_CHECK_VALUE(g.numel() == numels[i], "adamw_fused_packed: gradient size differs from the tensor's");
+    TORCH_CHECK_VALUE(!dtype || *dtype == g.scalar_type(), "adamw_fused_packed: gradients of one call must share a dtype");
+    dtype = g.scalar_type();
+    if (g.is_contiguous()) {
+      ptrs[i] = g.data_ptr();
+    } else {
+      keep.push_back(g.contiguous());
+      ptrs[i] = keep.back().data_ptr();
+    }
+  }
+  int code = PK_BF16;
+  if (dtype) { code = *dtype == at::kBFloat16 ? PK_BF16 : PK_F32; TORCH_CHECK_TYPE(*dtype == at::kBFloat16 || *dtype == at::kFloat, "piper_amd kernels support float32 and bfloat16"); }
+  PK_CALL(pk_adamw_fused_packed, master.data_ptr<float>(), exp_avg.data_ptr<float>(), exp_avg_sq.data_ptr<float>(), static_cast<float*>(ptr(flat_grad)),
+          ptrs.data(), offsets.data(), numels.data(), (int64_t)n, code, ptr(shadow), PK_BF16, (float)lr, (float)beta1, (float)beta2, (float)eps,
+          (float)weight_decay, step, (float)grad_scale, zero_grad, stream_of(master));
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  const auto nogil = py::call_guard<py::gil_scoped_release>();
+  m.def("expert_region", &expert_region, nogil);
+  m.def("rmsnorm", &rmsnorm, nogil);
+  m.def("sort_by_expert", &sort_by_expert, nogil);
+  m.def("router", &router, nogil);
+  m.def("permute", &permute, nogil);
+  m.def("combine", &combine, nogil);
+  m.def("bmm_experts", &bmm_experts, nogil);
+  m.def("pack_param_grads", &pack_param_grads);
+  m.def("hold_param_grads", &hold_param_grads);
+  m.def("clear_param_grads", &clear_param_grads);
+  m.def("adamw_packed", [](const Tensor& master, const Tensor& exp_avg, const Tensor& exp_avg_sq, const OptTensor& flat_grad,
+                           const std::vector<OptTensor>& grads, const std::vector<int64_t>& offsets, const std::vector<int64_t>& numels, int64_t step,
+                           double lr, double beta1, double beta2, double eps, double weight_decay, const OptTensor& shadow, double grad_scale,
+                           bool zero_grad) {
+    adamw_packed(master, exp_avg, exp_avg_sq, opt(flat_grad), grads, offsets, numels, step, lr, beta1, beta2, eps, weight_decay, opt(shadow),
+                 grad_scale, zero_grad);
+  });
+  m.def("set_accumulate", [](bool on) { return g_accumulate.exchange(on); });
+  m.def("set_overlap", [](bool on) { return g_overlap.exchange(on); });
+  // the WeightGradQueue that backward passes hand their weight gradients to (None: they run them)
+  m.def("set_queue", [](py::object q) {
+    PyObject* const old = g_queue;
+    g_queue = q.is_none() ? nullptr : q.inc_ref().ptr();
+    g_deferring.store(g_queue != nullptr);
+    Py_XDECREF(old);
+  });
+}

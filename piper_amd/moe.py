@@ -152,5 +152,22 @@ class MoEFeedForwardBlock(nn.Module):
         self.ffn_norm = RMSNorm(dim, norm_eps, dtype=dtype)
         self.moe = AnnotatedMoE(moe_args, dim, hidden_dim, dtype=dtype, fused=True)
 
+    def _one_node(self) -> bool:
+        """Whether nobody can tell the submodules' own calls from one fused call: no hooks on them, no
+        replaced or subclassed parts."""
+        norm, moe = self.ffn_norm, self.moe
+        return (type(norm) is RMSNorm and type(moe) is AnnotatedMoE and moe.fused and not torch.compiler.is_compiling()
+                and not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                            for m in (norm, moe)))
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.moe(self.ffn_norm(x), residual=x)
+        if not self._one_node():
+            return self.moe(self.ffn_norm(x), residual=x)
+        norm, moe = self.ffn_norm, self.moe
+        router, experts = moe.router, moe.experts
+        shape = x.shape
+        with annotate(EP_TAG):
+            out = F_.moe_block(x.reshape(-1, shape[-1]), norm.weight, router.gate.weight, router.gate.bias, experts.w1, experts.w2,
+                               experts.w3, top_k=router.top_k, route_norm=router.route_norm, route_scale=router.route_scale,
+                               norm_eps=norm.eps)
+        return out.reshape(shape)
