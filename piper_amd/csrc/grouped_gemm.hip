@@ -14,6 +14,7 @@
 #include "pk_common.h"
 #include "simt_gemm.h"
 #include "tile_gemm.h"
+#include "skinny_gemm.h"
 #include "unit_index.h"
 #include <functional>
 #include <initializer_list>
@@ -2209,6 +2210,36 @@ bool tile_gemm_ok(int dtype, int64_t H, int64_t I, std::initializer_list<const v
   return H % piece == 0 && I % piece == 0 && all_aligned16(ptrs);
 }
 
+// Expected rows of an expert that has any, if they are few enough for the weight-streaming forward
+// kernels of skinny_gemm.h; 0 otherwise.  Measured (gate/up + down, us, wide tiles -> streaming):
+//   128 experts 2048 x 768:  1 token 62 -> 20, 24 tokens 211 -> 172, 8 rows each 262 -> 257, 12 rows 266 -> 281
+//   32 experts 1024 x 512:   1 row each 48 -> 14, 16 rows 53 -> 28, 48 rows 61 -> 55, 64 rows 65 -> 69
+//   8 experts 4096 x 1536:   1 row each 137 -> 43, 48 rows 167 -> 142, 64 rows 176 -> 184
+//   24 experts 1000 x 360 (against the tiles of tile_gemm.h): 21 rows each 29 -> 21, 32 rows 29 -> 31
+// Where the wide tiles have a unit for every CU they hold their own from about 8 rows per expert on;
+// where they leave CUs idle, only from about 50, and the smaller tiles of tile_gemm.h from about 24.
+int64_t skinny_rows(int64_t A, int64_t I, int64_t E, bool wide) {
+  const int64_t touched = A < E ? A : E, rows = pk_ceil_div(A, touched);
+  const bool fills = touched * pk_ceil_div(I, 128) >= mf::persistent_grid();
+  return rows <= (fills ? 8 : wide ? 48 : 24) ? rows : 0;
+}
+int fwd_skinny(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2, const void* w3, const int32_t* starts,
+               void* g, void* u, void* h, void* y, int64_t A, int64_t H, int64_t I, int64_t E, int64_t rows, hipStream_t s) {
+  pk_skinny::Params p = {};
+  p.A = (const bf16_t*)x; p.lda = H; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.B0 = (const bf16_t*)w1; p.B1 = (const bf16_t*)w3; p.ldb = H; p.strideB = I * H;
+  p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.N = (int32_t)I;
+  p.O0 = (bf16_t*)g; p.O1 = (bf16_t*)u; p.O2 = (bf16_t*)h; p.ldc = I;
+  const int rc = pk_skinny::launch_for_rows<true>(p, A, rows, pk_timing::K_SWIGLU_GATE_UP, s);
+  if (rc) return rc;
+  pk_skinny::Params q = {};
+  q.A = (const bf16_t*)h; q.lda = I; q.map_div = 1;
+  q.B0 = (const bf16_t*)w2; q.ldb = I; q.strideB = H * I;
+  q.starts = starts; q.E = (int32_t)E; q.K = (int32_t)I; q.N = (int32_t)H;
+  q.O0 = (bf16_t*)y; q.ldc = H;
+  return pk_skinny::launch_for_rows<false>(q, A, rows, pk_timing::K_SWIGLU_DOWN, s);
+}
+
 template <typename T>
 int fwd_tile(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2, const void* w3,
              const int32_t* starts, void* g, void* u, void* h, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
@@ -2309,7 +2340,11 @@ int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t ro
   if (!row_map) row_map_div = 1;
   hipStream_t s = (hipStream_t)stream;
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({x_rows, w1, w2, w3, g, u, h, y});
-  if (!mfma && tile_gemm_ok(dtype, H, I, {x_rows, w1, w2, w3, g, u, h, y}))
+  const bool pieces = tile_gemm_ok(dtype, H, I, {x_rows, w1, w2, w3, g, u, h, y});
+  const int64_t few = skinny_rows(A, I, E, mfma);
+  if (dtype == PK_BF16 && pieces && few > 0)
+    return fwd_skinny(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, few, s);
+  if (!mfma && pieces)
     return dtype == PK_F32 ? fwd_tile<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s)
                            : fwd_tile<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
   if (!mfma && !g) return PK_ERR_ARG;      // the FMA kernels form h from g and u in memory

@@ -545,3 +545,44 @@ def test_widths_without_a_multiple_of_the_wide_tiles(dev, dtype, counts, H, I):
                                ("dw1 added", acc[0][e], 2 * d1), ("dw2 added", acc[1][e], 2 * d2), ("dw3 added", acc[2][e], 2 * d3)):
             assert rel_err(got, ref) <= tol, (name, e, c, rel_err(got, ref))
         s += c
+
+
+SKINNY_CASES = [
+    # (counts, H, I): below, at and above the 16- and 32-row units, reductions of less than one step (64)
+    # per wave and with a remainder, widths with a partly filled column tile, empty experts
+    ([1], 64, 16),
+    ([0, 1, 0, 2, 15, 16, 17, 0, 3], 200, 72),
+    ([33, 1, 31, 32, 40, 0], 520, 264),
+    ([9] * 12, 2048, 768),
+]
+
+
+@pytest.mark.parametrize("counts,H,I", SKINNY_CASES)
+def test_experts_with_few_rows(dev, counts, H, I):
+    """The weight-streaming forward (skinny_gemm.h) against float64 matmuls of the same bf16 inputs, with
+    and without a row map and with g and u left out: the same bits every time."""
+    from piper_amd import _lib
+    print(f"[case] skinny counts={counts[:9]} H={H} I={I}", flush=True)
+    x, w1, w2, w3, _, cnt = (t.to(dev) for t in _make(37, counts, H, I, torch.bfloat16))
+    A = x.shape[0]
+    starts = ops.counts_to_starts(cnt)
+    y, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts)
+    order = torch.randperm(A, generator=torch.Generator().manual_seed(2)).to(dev)
+    x_at = torch.empty_like(x)
+    x_at[order] = x
+    y2, g2, u2, h2 = ops.grouped_swiglu_fwd(x_at, w1, w2, w3, starts, row_map=order.to(torch.int32), row_map_div=1)
+    assert torch.equal(y, y2) and torch.equal(g, g2) and torch.equal(u, u2) and torch.equal(h, h2)
+    h3, y3 = torch.empty_like(h), torch.empty_like(y)
+    rc = _lib.load().pk_grouped_swiglu_fwd(x.data_ptr(), None, 1, w1.data_ptr(), w2.data_ptr(), w3.data_ptr(), starts.data_ptr(), None, None,
+                                           h3.data_ptr(), y3.data_ptr(), A, H, I, len(counts), _lib.PK_BF16, _lib.current_stream(dev))
+    assert rc == 0 and torch.equal(h, h3) and torch.equal(y, y3)
+    s = 0
+    for e, c in enumerate(counts):
+        if c == 0:
+            continue
+        xe = x[s:s + c].double()
+        ge, ue = xe @ w1[e].double().t(), xe @ w3[e].double().t()
+        he = torch.nn.functional.silu(ge) * ue
+        for name, got, ref in (("g", g, ge), ("u", u, ue), ("h", h, he), ("y", y, he @ w2[e].double().t())):
+            assert rel_err(got[s:s + c], ref) <= BF16_TOL, (name, e, c)
+        s += c
