@@ -81,6 +81,14 @@ PK_API int pk_gate_logits(const void* x, int x_dtype, const float* w_gate, const
 PK_API int pk_route_topk(const float* logits, int64_t T, int64_t E, int64_t K, int route_norm,
                   float route_scale, float* top_scores, int32_t* top_idx, pk_stream_t stream);
 
+/* pk_gate_logits and pk_route_topk in one call, with the same results bit for bit: where the gate GEMM
+ * splits its reduction, the top-k kernel sums the partial results on its way (one launch and one pass
+ * over [T, E] less).  workspace as for pk_gate_logits. */
+PK_API int pk_gate_route(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, int64_t T,
+                  int64_t H, int64_t E, int64_t K, int route_norm, float route_scale, float* logits,
+                  float* top_scores, int32_t* top_idx, void* workspace, int64_t workspace_bytes,
+                  pk_stream_t stream);
+
 /* Backward of pk_route_topk: d_logits[T,E] (f32, fully written) from d_top_scores[T,K]. */
 PK_API int pk_route_topk_bwd(const float* logits, const int32_t* top_idx, const float* d_top_scores,
                       int64_t T, int64_t E, int64_t K, int route_norm, float route_scale,
@@ -112,6 +120,33 @@ PK_API int64_t pk_sort_workspace_bytes(int64_t A, int64_t E);
 PK_API int pk_sort_by_expert(const int32_t* top_idx, int64_t A, int64_t E, int32_t* counts,
                       int32_t* starts, int32_t* perm, int32_t* inv_perm, int32_t* order,
                       void* workspace, int64_t workspace_bytes, pk_stream_t stream);
+
+/* Backward of the router together with the gradient of the region's input, for the fused region:
+ *   d_logits = pk_route_topk_bwd(logits, top_idx, d_top_scores)
+ *   d_w_gate, d_gate_bias (each may be NULL) as pk_gate_logits_bwd
+ *   d_x[t] = sum_k d_rows[inv_perm[t*K + k]] + d_logits[t] . w_gate      (d_x may be NULL)
+ * i.e. pk_route_topk_bwd, pk_gate_logits_bwd and pk_permute_bwd with the same results, but the gate's
+ * share of d_x is added where the routed rows are gathered (no fp32 [T, H] tensor in between) and the
+ * score gradients may come as the partial sums that pk_grouped_swiglu_dgrad_dh_scaled_t leaves
+ * (d_top_scores NULL; ds_partial [n_partial][T*K] in sorted row order).  d_rows and d_x have x's dtype;
+ * w_gate, d_rows, d_x and d_logits must be 16-byte aligned. */
+PK_API int64_t pk_region_router_bwd_workspace_bytes(int64_t T, int64_t H, int64_t E, int x_dtype);
+PK_API int pk_region_router_bwd(const float* logits, const int32_t* top_idx, const float* d_top_scores,
+                         const float* ds_partial, int64_t n_partial, const int32_t* inv_perm, int route_norm,
+                         float route_scale, const void* x, int x_dtype, const float* w_gate, const void* d_rows,
+                         void* d_x, float* d_w_gate, float* d_gate_bias, int accumulate, float* d_logits,
+                         int64_t T, int64_t H, int64_t E, int64_t K, void* workspace, int64_t workspace_bytes,
+                         pk_stream_t stream);
+
+/* pk_gate_route and pk_sort_by_expert in one call (same results): for a decode step the top-k and the
+ * sort share one launch.  counts, inv_perm and order may be NULL.  workspace:
+ * pk_gate_route_sort_workspace_bytes. */
+PK_API int64_t pk_gate_route_sort_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K);
+PK_API int pk_gate_route_sort(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, int64_t T,
+                       int64_t H, int64_t E, int64_t K, int route_norm, float route_scale, float* logits,
+                       float* top_scores, int32_t* top_idx, int32_t* counts, int32_t* starts, int32_t* perm,
+                       int32_t* inv_perm, int32_t* order, void* workspace, int64_t workspace_bytes,
+                       pk_stream_t stream);
 
 /* pk_sort_by_expert for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same
@@ -301,7 +336,9 @@ PK_API int pk_grouped_swiglu_wgrad_scaled(const void* d_out, const void* hs, con
  * expert's last row (rows of the next expert's tokens).  Zero times a finite value is zero; zero
  * times Inf or NaN is NaN.  A non-finite row of x or d_out can therefore reach the weight gradients
  * of the expert in front of the one it was routed to, which pk_grouped_swiglu_wgrad_scaled (rows
- * past an expert's end read as zeros) confines to its own experts. */
+ * past an expert's end read as zeros) confines to its own experts. 
+ * d_scores may be NULL: the score gradients then stay in the workspace as ceil(I / 64) partial sums per
+ * sorted row, [ceil(I / 64)][A] fp32, for pk_region_router_bwd. */
 PK_API int64_t pk_grouped_swiglu_transposed_ld(int64_t A, int64_t H, int64_t I, int64_t E, int dtype);
 PK_API int pk_grouped_swiglu_dgrad_dh_scaled_t(const void* d_out, const int32_t* row_map, int64_t row_map_div,
                                         const float* scores, const void* w2, const void* g,

@@ -32,6 +32,14 @@ SIGNATURES = {
     "pk_gate_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "pk_gate_logits": (_c_int, [_p, _c_int, _p, _p, _p, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),
     "pk_route_topk": (_c_int, [_p, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p]),
+    "pk_gate_route": (_c_int, [_p, _c_int, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p, _p, _c_i64, _p]),
+    "pk_region_router_bwd_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int]),
+    # logits idx d_scores part n_part inv_perm norm scale x x_dtype w_gate d_rows d_x d_w d_b accumulate d_logits T H E K ws ws_bytes stream
+    "pk_region_router_bwd": (_c_int, [_p, _p, _p, _p, _c_i64, _p, _c_int, _c_f32, _p, _c_int, _p, _p, _p, _p, _p, _c_int, _p,
+                                      _c_i64, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),
+    "pk_gate_route_sort_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
+    "pk_gate_route_sort": (_c_int, [_p, _c_int, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p, _p, _p, _p, _p, _p,
+                                    _p, _c_i64, _p]),
     "pk_route_topk_bwd": (_c_int, [_p, _p, _p, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p]),
     "pk_gate_bwd_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "pk_gate_logits_bwd": (_c_int, [_p, _p, _c_int, _p, _p, _p, _p, _c_int, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),

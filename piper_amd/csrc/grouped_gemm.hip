@@ -2435,7 +2435,8 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
   if (rc) return rc;
   if (A == 0) return PK_OK;
   const bool transposed = d_gT != nullptr;
-  if (!d_out || !row_map || row_map_div <= 0 || row_map_div > 0x7fffffffll || !scores || !w2 || !g || !u || !starts || !d_scores)
+  if (!d_out || !row_map || row_map_div <= 0 || row_map_div > 0x7fffffffll || !scores || !w2 || !g || !u || !starts ||
+      (!d_scores && !transposed))
     return PK_ERR_ARG;
   if ((!hs || !d_g || !d_u) && !transposed) return PK_ERR_ARG;      // the row-major outputs are optional beside the transposed ones
   if ((d_g == nullptr) != (d_u == nullptr)) return PK_ERR_ARG;
@@ -2479,7 +2480,7 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
   p.T0 = (bf16_t*)d_gT; p.T1 = (bf16_t*)d_uT; p.T2 = (bf16_t*)hsT; p.ldt = ldt;
   p.scores = scores; p.ds_partial = (float*)workspace; p.total_rows = A;
   rc = launch_rm<false, mf::EPI_SWIGLU_BWD_SCALED>(p, A, I, pk_timing::K_SWIGLU_DGRAD_DH, s);
-  if (rc) return rc;
+  if (rc || !d_scores) return rc;      // without d_scores the partial sums stay in the workspace
   PK_LAUNCH_NOCHECK(pk_timing::K_COMBINE_BWD, s, dscore_reduce_kernel, dim3((unsigned)pk_ceil_div(A, 256)), dim3(256), 0, s,
                     (const float*)workspace, (int)(I / 64), A, row_map, d_scores);
   PK_RETURN_IF_LAUNCH_FAILED();

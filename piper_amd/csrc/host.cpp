@@ -242,28 +242,32 @@ void route_in_python(PyObject* route, const Shape& s, const Saved& sv, const Ten
 }
 
 // out = [residual +] region([norm](x)); every input contiguous
-Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, const Tensor& x, const Tensor& w_gate, const Tensor& bias, const Tensor& w1,
+Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, bool keep_order, const Tensor& x, const Tensor& w_gate, const Tensor& bias, const Tensor& w1,
                       const Tensor& w2, const Tensor& w3, const Tensor& residual, const Tensor& norm_w) {
   Tensor out = at::empty({s.T, s.H}, x.options());
   sv.mem.allocate(x);
   Block tmp;
-  const int64_t gate_ws = pk_gate_workspace_bytes(s.T, s.H, s.E), sort_ws = pk_sort_workspace_bytes(s.A, s.E);
-  const size_t ws = tmp.add(std::max(gate_ws, sort_ws));
-  const size_t counts = tmp.add(s.E * 4);
+  const int64_t ws_bytes = pk_gate_route_sort_workspace_bytes(s.T, s.H, s.E, s.K);
+  TORCH_CHECK(ws_bytes >= 0, "pk_gate_route_sort_workspace_bytes failed: ", pk_status_string((int)ws_bytes));
+  const size_t ws = tmp.add(ws_bytes);
   const size_t h = tmp.add(s.A * s.I * s.es), y = tmp.add(s.A * s.H * s.es);
   tmp.allocate(x);
   const pk_stream_t st = stream_of(x);
   const Block& m = sv.mem;
+  int32_t* const order = keep_order ? m.i32(sv.order) : nullptr;      // only the weight gradient asks for it
   const void* xin = x.data_ptr();
   if (norm_w.defined()) {
     PK_CALL(pk_rmsnorm_fwd, xin, s.dtype, ptr(norm_w), (float)s.eps, m.at_(sv.xn), m.f32(sv.rstd), s.T, s.H, st);
     xin = m.at_(sv.xn);
   }
-  PK_CALL(pk_gate_logits, xin, s.dtype, fptr(w_gate), fptr(bias), m.f32(sv.logits), s.T, s.H, s.E, tmp.at_(ws), std::max<int64_t>(gate_ws, 0), st);
-  if (route) route_in_python(route, s, sv, x);
-  else PK_CALL(pk_route_topk, m.f32(sv.logits), s.T, s.E, s.K, s.route_norm, (float)s.route_scale, m.f32(sv.scores), m.i32(sv.idx), st);
-  PK_CALL(pk_sort_by_expert, m.i32(sv.idx), s.A, s.E, tmp.i32(counts), m.i32(sv.starts), m.i32(sv.perm), m.i32(sv.inv), m.i32(sv.order),
-          tmp.at_(ws), sort_ws, st);
+  if (route) {
+    PK_CALL(pk_gate_logits, xin, s.dtype, fptr(w_gate), fptr(bias), m.f32(sv.logits), s.T, s.H, s.E, tmp.at_(ws), ws_bytes, st);
+    route_in_python(route, s, sv, x);
+    PK_CALL(pk_sort_by_expert, m.i32(sv.idx), s.A, s.E, nullptr, m.i32(sv.starts), m.i32(sv.perm), m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
+  } else {
+    PK_CALL(pk_gate_route_sort, xin, s.dtype, fptr(w_gate), fptr(bias), s.T, s.H, s.E, s.K, s.route_norm, (float)s.route_scale, m.f32(sv.logits),
+            m.f32(sv.scores), m.i32(sv.idx), nullptr, m.i32(sv.starts), m.i32(sv.perm), m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
+  }
   PK_CALL(pk_grouped_swiglu_fwd, xin, m.i32(sv.perm), s.K, ptr(w1), ptr(w2), ptr(w3), m.i32(sv.starts), keep_gu ? m.at_(sv.g) : nullptr,
           keep_gu ? m.at_(sv.u) : nullptr, tmp.at_(h), tmp.at_(y), s.A, s.H, s.I, s.E, s.dtype, st);
   PK_CALL(pk_combine_fwd, tmp.at_(y), s.dtype, m.i32(sv.inv), m.f32(sv.scores), ptr(residual), ptr(out), s.T, s.H, s.K, st);
@@ -338,7 +342,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const bool norm = norm_w.defined();
     Saved sv(s, true, norm);
     const Tensor xc = contig(x);
-    Tensor out = region_forward(s, route, sv, true, xc, contig(w_gate), contig(bias), contig(w1), contig(w2), contig(w3),
+    Tensor out = region_forward(s, route, sv, true, true, xc, contig(w_gate), contig(bias), contig(w1), contig(w2), contig(w3),
                                 norm ? xc : contig(residual), contig(norm_w));
     ctx->save_for_backward({x, w_gate, bias, w1, w2, w3, norm_w, sv.mem.memory()});
     ctx->saved_data["k"] = top_k;
@@ -363,7 +367,9 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     for (int i = 0, edge = 0; i < N_TENSORS; ++i) need[i] = present[i] && ctx->needs_input_grad(edge++);
     const bool need_xn = need[X] || (norm && need[NORM_W]);      // the gradient of what the router and the experts read
     const Tensor d_out = contig(grads[0]);
-    const Tensor xc = contig(x), w_gate = contig(p_gate), w1 = contig(p1), w2 = contig(p2), w3 = contig(p3);
+    const Tensor xc = contig(x), w1 = contig(p1), w2 = contig(p2), w3 = contig(p3);
+    Tensor w_gate = contig(p_gate);
+    if (!aligned16(w_gate)) w_gate = w_gate.clone();
     const void* x_rows = norm ? m.at_(sv.xn) : xc.data_ptr();
     const int32_t *perm = m.i32(sv.perm), *starts = m.i32(sv.starts);
 
@@ -376,8 +382,10 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const int64_t ds_ws = std::max<int64_t>(pk_grouped_swiglu_dgrad_dh_scaled_workspace_bytes(s.A, s.I), 4);
     const size_t d_g = t.add(blocks_only ? 0 : ai), d_u = t.add(blocks_only ? 0 : ai), hs = t.add(ldt > 0 ? 0 : ai);
     const size_t d_gT = t.add(ait), d_uT = t.add(ait), hsT = t.add(ait);
-    const size_t d_scores = t.add(s.A * 4), part = t.add(ds_ws), d_logits = t.add(s.T * s.E * 4);
-    const size_t d_xs = t.add(need_xn ? s.A * s.H * s.es : 0), d_x32 = t.add(need_xn ? s.T * s.H * 4 : 0);
+    const size_t d_scores = t.add(ldt > 0 ? 0 : s.A * 4), part = t.add(ds_ws), d_logits = t.add(s.T * s.E * 4);
+    const size_t d_xs = t.add(need_xn ? s.A * s.H * s.es : 0);
+    const int64_t router_ws_bytes = pk_region_router_bwd_workspace_bytes(s.T, s.H, s.E, s.dtype);
+    const size_t router_ws = t.add(router_ws_bytes);
     const size_t d_xn = t.add(norm && need_xn ? s.T * s.H * s.es : 0);
     t.allocate(x);
     const pk_stream_t st = stream_of(x);
@@ -386,7 +394,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     // is applied in the epilogue
     if (ldt > 0)
       PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled_t, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
-              t.at_(d_gT), t.at_(d_uT), t.at_(hsT), ldt, t.f32(d_scores), t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
+              t.at_(d_gT), t.at_(d_uT), t.at_(hsT), ldt, nullptr, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
     else
       PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
               t.at_(hs), t.f32(d_scores), t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
@@ -401,24 +409,22 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       else
         PK_CALL(pk_grouped_swiglu_dgrad_dx, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
     };
-    const auto route_bwd = [&] {
-      PK_CALL(pk_route_topk_bwd, m.f32(sv.logits), m.i32(sv.idx), t.f32(d_scores), s.T, s.E, s.K, s.route_norm, (float)s.route_scale,
-              t.f32(d_logits), st);
-    };
+    // The router's backward and the gradient of the region's input; with a norm in front its backward
+    // follows and adds the residual branch's gradient.
     Tensor d_x, d_norm_w;
-    const auto finish_input = [&] {
-      if (!need_xn) return;
-      Tensor dest = need[X] && !norm ? at::empty({s.T, s.H}, x.options()) : Tensor();
-      void* const to = norm ? t.at_(d_xn) : ptr(dest);
-      PK_CALL(pk_permute_bwd, t.at_(d_xs), s.dtype, m.i32(sv.inv), t.f32(d_x32), to, s.T, s.H, s.K, st);
-      if (!norm) { d_x = dest; return; }
-      d_x = at::empty({s.T, s.H}, x.options());
+    const auto router_and_input = [&](const Tensor& d_wg, const Tensor& d_b) {
+      if (need_xn) d_x = at::empty({s.T, s.H}, x.options());
+      PK_CALL(pk_region_router_bwd, m.f32(sv.logits), m.i32(sv.idx), ldt > 0 ? nullptr : t.f32(d_scores), t.f32(part), (s.I + 63) / 64, m.i32(sv.inv),
+              s.route_norm, (float)s.route_scale, x_rows, s.dtype, fptr(w_gate), t.at_(d_xs), !need_xn ? nullptr : norm ? t.at_(d_xn) : ptr(d_x),
+              static_cast<float*>(ptr(d_wg)), static_cast<float*>(ptr(d_b)), 0, t.f32(d_logits), s.T, s.H, s.E, s.K, t.at_(router_ws),
+              router_ws_bytes, st);
+      if (!norm || !need_xn) return;
       Tensor ws;
       if (need[NORM_W]) {
         d_norm_w = at::empty({s.H}, norm_w.options());
         ws = at::empty({pk_rmsnorm_bwd_workspace_bytes(s.T, s.H)}, x.options().dtype(at::kByte));
       }
-      PK_CALL(pk_rmsnorm_bwd, to, ptr(xc), s.dtype, ptr(contig(norm_w)), m.f32(sv.rstd), ptr(d_out), ptr(d_x), ptr(d_norm_w), 0, s.T, s.H,
+      PK_CALL(pk_rmsnorm_bwd, t.at_(d_xn), ptr(xc), s.dtype, ptr(contig(norm_w)), m.f32(sv.rstd), ptr(d_out), ptr(d_x), ptr(d_norm_w), 0, s.T, s.H,
               ptr(ws), ws.defined() ? ws.numel() : 0, st);
       if (!need[X]) d_x = Tensor();
     };
@@ -430,9 +436,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       // the tensors they need and computed by the weight pass
       push_deferred([wgrad, p1, p2, p3] { weight_grads_into_params(p1, p2, p3, wgrad); });
       input_grad();
-      route_bwd();
-      if (need_xn) gate_bwd(t.f32(d_logits), x_rows, s.dtype, w_gate, t.f32(d_x32), Tensor(), Tensor(), false, s.T, s.H, s.E);
-      finish_input();
+      router_and_input(Tensor(), Tensor());
       push_deferred([s, p_gate, p_bias, w_gate, x_rows, dl = t.f32(d_logits), keep = std::array<Tensor, 3>{t.memory(), sv.mem.memory(), xc}] {
         router_weight_grads(p_gate, p_bias, dl, x_rows, s.dtype, w_gate, s.T, s.H, s.E);
       });
@@ -464,17 +468,12 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       }
     }
     input_grad();
-    route_bwd();
-    if (gate_in_place) {
-      if (need_xn) gate_bwd(t.f32(d_logits), x_rows, s.dtype, w_gate, t.f32(d_x32), Tensor(), Tensor(), false, s.T, s.H, s.E);
-      router_weight_grads(p_gate, p_bias, t.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
-    } else {
+    if (!gate_in_place) {
       if (need[W_GATE]) d_wg = at::empty({s.E, s.H}, w_gate.options());
       if (p_bias.defined() && need[BIAS]) d_b = at::empty({s.E}, w_gate.options());
-      if (need_xn || d_wg.defined() || d_b.defined())
-        gate_bwd(t.f32(d_logits), x_rows, s.dtype, w_gate, need_xn ? t.f32(d_x32) : nullptr, d_wg, d_b, false, s.T, s.H, s.E);
     }
-    finish_input();
+    router_and_input(d_wg, d_b);
+    if (gate_in_place) router_weight_grads(p_gate, p_bias, t.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
     if (overlap) {
       const auto side = side_stream(x.get_device());
       wait_stream(cur.stream(), side.stream());
@@ -502,7 +501,7 @@ std::optional<Tensor> expert_region(const Tensor& x, const Tensor& w_gate, const
   const int64_t piece = 16 / s.es;
   const bool keep_gu = s.H % piece != 0 || s.I % piece != 0 || !aligned16(xc) || !aligned16(w1c) || !aligned16(w2c) || !aligned16(w3c);
   Saved sv(s, keep_gu, norm_w.defined());
-  return region_forward(s, route, sv, keep_gu, xc, contig(w_gate), contig(bias), w1c, w2c, w3c, norm_w.defined() ? xc : contig(residual), contig(norm_w));
+  return region_forward(s, route, sv, keep_gu, false, xc, contig(w_gate), contig(bias), w1c, w2c, w3c, norm_w.defined() ? xc : contig(residual), contig(norm_w));
 }
 
 // ------------------------------------------------------------------------------ RMSNorm
@@ -576,16 +575,17 @@ struct RouterFn : public torch::autograd::Function<RouterFn> {
     const int64_t ws_bytes = pk_gate_workspace_bytes(T, H, E);
     Tensor ws = ws_bytes > 0 ? at::empty({ws_bytes}, f32.dtype(at::kByte)) : Tensor();
     const pk_stream_t st = stream_of(x);
-    PK_CALL(pk_gate_logits, ptr(contig(x)), dtype_code(x), fptr(contig(w_gate)), fptr(contig(bias)), logits.data_ptr<float>(), T, H, E, ptr(ws),
-            ws.defined() ? ws_bytes : 0, st);
+    const Tensor xc = contig(x), wc = contig(w_gate), bc = contig(bias);
+    const int64_t bytes = ws.defined() ? ws_bytes : 0;
     if (route) {
+      PK_CALL(pk_gate_logits, ptr(xc), dtype_code(x), fptr(wc), fptr(bc), logits.data_ptr<float>(), T, H, E, ptr(ws), bytes, st);
       py::gil_scoped_acquire gil;
       py::tuple r = py::handle(route)(logits, top_k, route_norm, route_scale);
       scores.copy_(r[0].cast<Tensor>());
       idx.copy_(r[1].cast<Tensor>());
     } else {
-      PK_CALL(pk_route_topk, logits.data_ptr<float>(), T, E, top_k, route_norm, (float)route_scale, scores.data_ptr<float>(),
-              idx.data_ptr<int32_t>(), st);
+      PK_CALL(pk_gate_route, ptr(xc), dtype_code(x), fptr(wc), fptr(bc), T, H, E, top_k, route_norm, (float)route_scale, logits.data_ptr<float>(),
+              scores.data_ptr<float>(), idx.data_ptr<int32_t>(), ptr(ws), bytes, st);
     }
     ctx->save_for_backward({x, w_gate, bias, logits, idx});
     ctx->saved_data["norm"] = route_norm;

@@ -95,56 +95,76 @@ __device__ __forceinline__ void zero_planes(bf16x4_t (&out)[P]) {
 #pragma unroll
   for (int q = 0; q < P; ++q) out[q] = zero;
 }
-// four consecutive elements of an operand as planes of four bf16
+// Four consecutive elements of an operand as they come from memory (Raw: fp32 values, or the planes),
+// and as planes of four bf16.  They are split when they go to LDS: a split at the fetch waits for the
+// load there and then (forward 61 -> 50 us, d_x 103 -> 84 us at 16,384 tokens, 128 experts, 2048 wide).
+template <typename T> struct Raw { bf16x4_t v[Planes<T>::N]; };
+template <> struct Raw<float> { floatx4_t v; };
 template <typename T>
-__device__ __forceinline__ void fetch4(const typename Mem<T>::type* src, int64_t plane_stride, bf16x4_t (&out)[Planes<T>::N]) {
+__device__ __forceinline__ void zero_raw(Raw<T>& r) {
+  if constexpr (std::is_same<T, float>::value) r.v = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  else zero_planes<Planes<T>::N>(r.v);
+}
+template <typename T>
+__device__ __forceinline__ void fetch4(const typename Mem<T>::type* src, int64_t plane_stride, Raw<T>& out) {
+  if constexpr (std::is_same<T, float>::value) {
+    out.v = *reinterpret_cast<const floatx4_t*>(src);
+  } else {
+#pragma unroll
+    for (int q = 0; q < Planes<T>::N; ++q) out.v[q] = *reinterpret_cast<const bf16x4_t*>(src + q * plane_stride);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void to_planes(const Raw<T>& r, bf16x4_t (&out)[Planes<T>::N]) {
   constexpr int P = Planes<T>::N;
   if constexpr (std::is_same<T, float>::value) {
-    float v[4];
-    pk_f32mm::load4<float>(src, v);
     bf16_t pl[4][P];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) split<P>(v[j], pl[j]);
+    for (int j = 0; j < 4; ++j) split<P>(r.v[j], pl[j]);
 #pragma unroll
     for (int q = 0; q < P; ++q)
 #pragma unroll
       for (int j = 0; j < 4; ++j) out[q][j] = pl[j][q];
   } else {
 #pragma unroll
-    for (int q = 0; q < P; ++q) out[q] = *reinterpret_cast<const bf16x4_t*>(src + q * plane_stride);
+    for (int q = 0; q < P; ++q) out[q] = r.v[q];
   }
 }
 
 template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
-__global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
+struct Lds {
+  static constexpr int BM = 32 * WM, BN = 32 * WN;
+  static constexpr int LDA = BM + MN_PAD, LDB = BN + MN_PAD;     // [k][row] layouts
+  __attribute__((aligned(16))) bf16_t As[Planes<TA>::N][A_KC ? BM * LDK : BK * LDA];
+  __attribute__((aligned(16))) bf16_t Bs[Planes<TB>::N][B_KC ? BN * LDK : BK * LDB];
+};
+
+// acc of one wave: rows m0 + 32 wm .., columns n0 + 32 wn .. of the product over k in [kbeg, kend)
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+__device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
+                                        int64_t kend, floatx16_t& acc) {
   constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
   constexpr int PA = Planes<TA>::N, PB = Planes<TB>::N;
-  constexpr int LDA = BM + MN_PAD, LDB = BN + MN_PAD;     // [k][row] layouts
-  __shared__ __attribute__((aligned(16))) bf16_t As[PA][A_KC ? BM * LDK : BK * LDA];
-  __shared__ __attribute__((aligned(16))) bf16_t Bs[PB][B_KC ? BN * LDK : BK * LDB];
-
+  constexpr int LDA = BM + MN_PAD, LDB = BN + MN_PAD;
+  auto& As = lds.As;
+  auto& Bs = lds.Bs;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;
-  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
-  const int64_t kchunk = ((p.K + p.splits - 1) / p.splits + BK - 1) / BK * BK;
-  const int64_t kbeg = (int64_t)blockIdx.z * kchunk;
-  const int64_t kend = kbeg + kchunk < p.K ? kbeg + kchunk : p.K;
-
   typedef typename Mem<TA>::type MA;
   typedef typename Mem<TB>::type MB;
   const MA* A = reinterpret_cast<const MA*>(p.A);
   const MB* B = reinterpret_cast<const MB*>(p.B);
 
-  floatx16_t acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
 
   // every thread fetches 4 consecutive elements of the contiguous index per load (every plane of
   // them for a pre-split operand); the loads of tile k+1 are in flight while tile k is multiplied
+  // (two, four and eight tiles in flight: no gain at 509 tokens, 2 to 20 % slower at 16,384)
   constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
   static_assert(NA >= 1 && NB >= 1, "tile too small for the thread count");
-  // four fetched elements as planes of four bf16 (an fp32 operand is split here, once per load)
-  bf16x4_t ra[NA][PA], rb[NB][PB];
+  Raw<TA> ra[NA];
+  Raw<TB> rb[NB];
   auto slot = [](int idx, bool kc, int R, int& row, int& k) {
     if (kc) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); }
     else { row = (idx % (R / 4)) * 4; k = idx / (R / 4); }
@@ -154,14 +174,14 @@ __global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
     for (int i = 0; i < NA; ++i) {
       int m, k;
       slot(tid + i * THREADS, A_KC, BM, m, k);
-      zero_planes<PA>(ra[i]);
+      zero_raw<TA>(ra[i]);
       if (m0 + m < p.M && k0 + k < kend) fetch4<TA>(A + (m0 + m) * p.sam + (k0 + k) * p.sak, p.plane_a, ra[i]);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       int n, k;
       slot(tid + i * THREADS, B_KC, BN, n, k);
-      zero_planes<PB>(rb[i]);
+      zero_raw<TB>(rb[i]);
       if (n0 + n < p.N && k0 + k < kend) fetch4<TB>(B + (k0 + k) * p.sbk + (n0 + n) * p.sbn, p.plane_b, rb[i]);
     }
   };
@@ -178,13 +198,17 @@ __global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
     for (int i = 0; i < NA; ++i) {
       int m, k;
       slot(tid + i * THREADS, A_KC, BM, m, k);
-      store4(As, std::integral_constant<int, PA>{}, A_KC, LDA, m, k, ra[i]);
+      bf16x4_t v[PA];
+      to_planes<TA>(ra[i], v);
+      store4(As, std::integral_constant<int, PA>{}, A_KC, LDA, m, k, v);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       int n, k;
       slot(tid + i * THREADS, B_KC, BN, n, k);
-      store4(Bs, std::integral_constant<int, PB>{}, B_KC, LDB, n, k, rb[i]);
+      bf16x4_t v[PB];
+      to_planes<TB>(rb[i], v);
+      store4(Bs, std::integral_constant<int, PB>{}, B_KC, LDB, n, k, v);
     }
     __syncthreads();
     if (k0 + BK < kend) load_tile(k0 + BK);
@@ -207,6 +231,21 @@ __global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
     __syncthreads();
   }
 
+}
+
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+__global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
+  constexpr int BM = 32 * WM, BN = 32 * WN;
+  __shared__ Lds<WM, WN, A_KC, B_KC, TA, TB> lds;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+  const int64_t kchunk = ((p.K + p.splits - 1) / p.splits + BK - 1) / BK * BK;
+  const int64_t kbeg = (int64_t)blockIdx.z * kchunk;
+  const int64_t kend = kbeg + kchunk < p.K ? kbeg + kchunk : p.K;
+  floatx16_t acc;
+  product<WM, WN, A_KC, B_KC, TA, TB>(p, lds, m0, n0, kbeg, kend, acc);
+
   float* C = p.C + (p.splits > 1 ? (int64_t)blockIdx.z * p.M * p.N : 0);
   const int64_t n = n0 + wn * 32 + (lane & 31);
   if (n < p.N) {
@@ -220,6 +259,68 @@ __global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
         C[m * p.N + n] = r;
       }
     }
+  }
+}
+
+// The gradient of the region's input in one pass: out[t] = sum_k rows[inv_perm[t*K + k]] + d_logits[t] .
+// w_gate, the second term being this GEMM.  Its tile goes through LDS, and every thread then adds the K
+// gathered rows for 16 bytes of a token (the sum over k first, the GEMM's value last, rounded once: what
+// the GEMM into an fp32 [T, H] tensor and gather_reduce_kernel behind it compute), so that tensor is
+// neither written nor read.  STREAM: the gathered rows are too many to stay in a cache.
+struct GatherAdd {
+  const void* rows;           // [T * K, H], element type TG
+  const int32_t* inv_perm;    // [T * K]
+  void* out;                  // [T, H]
+  int32_t K;
+};
+template <int WM, int WN, typename TG, bool STREAM>
+__global__ __launch_bounds__(64 * WM * WN) void gather_kernel(const Params p, const GatherAdd ga) {
+  constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
+  typedef Lds<WM, WN, true, false, float, float> Tiles;
+  constexpr int LDO = BN + 4;
+  constexpr int BYTES = sizeof(Tiles) > BM * LDO * 4 ? (int)sizeof(Tiles) : BM * LDO * 4;
+  __shared__ __attribute__((aligned(16))) char smem[BYTES];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+  floatx16_t acc;
+  product<WM, WN, true, false, float, float>(p, *reinterpret_cast<Tiles*>(smem), m0, n0, 0, p.K, acc);
+  float* const tile = reinterpret_cast<float*>(smem);       // (product ends with a barrier)
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    tile[(wm * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * LDO + wn * 32 + (lane & 31)] = acc[v];
+  __syncthreads();
+  constexpr int N = PkVec16<TG>::N, PIECES = BN / N;        // 16-byte pieces of a token's columns
+  constexpr int KB = 8;
+  const int H = (int)p.N;
+  for (int i = tid; i < BM * PIECES; i += THREADS) {
+    const int r = i / PIECES, c = (i % PIECES) * N;
+    const int64_t t = m0 + r;
+    if (t >= p.M || n0 + c >= H) continue;
+    float sum[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) sum[j] = 0.f;
+    const int32_t* inv = ga.inv_perm + t * ga.K;
+    for (int k0 = 0; k0 < ga.K; k0 += KB) {
+      PkVec16<TG> v[KB];
+#pragma unroll
+      for (int j = 0; j < KB; ++j) {
+        const int64_t row = inv[k0 + j < ga.K ? k0 + j : ga.K - 1];
+        const auto* src = reinterpret_cast<const decltype(v[j].v)*>(reinterpret_cast<const TG*>(ga.rows) + row * H + n0 + c);
+        if (STREAM) v[j].v = __builtin_nontemporal_load(src);
+        else v[j].v = *src;
+      }
+#pragma unroll
+      for (int j = 0; j < KB; ++j)
+        if (k0 + j < ga.K) {
+#pragma unroll
+          for (int e = 0; e < N; ++e) sum[e] += v[j].get(e);
+        }
+    }
+    PkVec16<TG> o;
+#pragma unroll
+    for (int e = 0; e < N; ++e) o.set(e, sum[e] + tile[r * LDO + c + e]);
+    *reinterpret_cast<decltype(o.v)*>(reinterpret_cast<TG*>(ga.out) + t * H + n0 + c) = o.v;
   }
 }
 
@@ -246,6 +347,24 @@ inline int launch(const Params& p, int kernel_id, hipStream_t s) {
   dim3 grid((unsigned)pk_ceil_div(p.N, 32 * WN), (unsigned)pk_ceil_div(p.M, 32 * WM), (unsigned)p.splits);
   if (grid.y > 65535u || grid.z > 65535u) return PK_ERR_SHAPE;
   PK_LAUNCH_NOCHECK(kernel_id, s, (kernel<WM, WN, A_KC, B_KC, TA, TB>), grid, dim3(64 * WM * WN), 0, s, p);
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+
+// d_logits: p.A [T, E], w_gate: p.B [E, H] (p.M = T, p.N = H, p.K = E).  PK_ERR_ALIGN: the operands cannot
+// be read in 16-byte pieces; the caller takes the two kernels instead.
+template <typename TG>
+inline int launch_gather(const Params& p, const GatherAdd& ga, int kernel_id, hipStream_t s) {
+  // 32 tokens x 128 columns (16,384 tokens, the router backward as a whole: 212 us; 64 x 128: 214, 64 x 64: 222;
+  // with the GEMM and the gather apart 270)
+  constexpr int WM = 1, WN = 4;
+  if (!usable<WM, WN, true, false, float, float>(p) || p.N % PkVec16<TG>::N != 0 || !pk_aligned16(ga.rows) || !pk_aligned16(ga.out))
+    return PK_ERR_ALIGN;
+  dim3 grid((unsigned)pk_ceil_div(p.N, 32 * WN), (unsigned)pk_ceil_div(p.M, 32 * WM));
+  if (grid.y > 65535u) return PK_ERR_SHAPE;
+  const bool stream_rows = p.M * ga.K * p.N * (int64_t)sizeof(TG) > (int64_t)192 * 1024 * 1024;
+  if (stream_rows) PK_LAUNCH_NOCHECK(kernel_id, s, (gather_kernel<WM, WN, TG, true>), grid, dim3(64 * WM * WN), 0, s, p, ga);
+  else PK_LAUNCH_NOCHECK(kernel_id, s, (gather_kernel<WM, WN, TG, false>), grid, dim3(64 * WM * WN), 0, s, p, ga);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }

@@ -22,27 +22,81 @@ __device__ __forceinline__ float from_orderable(uint32_t o) {
 
 constexpr int kRouteThreads = 256;  // 4 waves, one token per wave
 
-// One wave per token.  Lane l owns experts l, l+64, ... (EPL of them).
-template <int EPL>
-__global__ __launch_bounds__(kRouteThreads) void route_topk_kernel(
-    const float* __restrict__ logits, int T, int E, int K, int route_norm, float route_scale,
-    float* __restrict__ top_scores, int32_t* __restrict__ top_idx) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * (kRouteThreads / 64) + wave;
-  if (t >= T) return;
-  const float* row = logits + (int64_t)t * E;
+// Wave-wide reductions on the vector ALU: lanes are combined within rows of 16 and then across rows with
+// data-parallel-primitive operands, and lane 63 ends with the result, read back into a scalar.  Six
+// dependent instructions, where a butterfly of LDS-permute shuffles waits for the LDS six times (twelve
+// for a 64-bit value): top-8 of 128 spent most of its time in them.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+#define PK_DPP_STEPS(OP)                    \
+  OP(0x111, 0xf) /* row_shr 1 */            \
+  OP(0x112, 0xf) /* row_shr 2 */            \
+  OP(0x114, 0xf) /* row_shr 4 */            \
+  OP(0x118, 0xf) /* row_shr 8 */            \
+  OP(0x142, 0xa) /* row_bcast 15 */         \
+  OP(0x143, 0xc) /* row_bcast 31 */
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {      // identity 0
+#define PK_STEP(C, R) { const uint32_t o = dpp_or_zero<C, R>(v); v = o > v ? o : v; }
+  PK_DPP_STEPS(PK_STEP)
+#undef PK_STEP
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ float wave_sum_f32(float f) {
+#define PK_STEP(C, R) f += __uint_as_float(dpp_or_zero<C, R>(__float_as_uint(f)));
+  PK_DPP_STEPS(PK_STEP)
+#undef PK_STEP
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(f), 63));
+}
+#undef PK_DPP_STEPS
 
+// Split-K partial results of the gate GEMM, summed by whoever reads the logits first.
+struct GatePartials {
+  const float* part;    // [splits][T][E], or nullptr: the logits are complete
+  const float* bias;    // [E] or nullptr
+  int splits;
+};
+
+// One wave per token.  Lane l owns experts l, l+64, ... (EPL of them).
+// PARTIALS: the logits are still split-K partial results; they are summed here (in split order, then
+// the bias: what reduce_partials_kernel would store) and written out on the way, which saves a launch
+// and a pass over [T, E].
+template <int EPL, bool PARTIALS>
+__device__ __forceinline__ void route_topk_token(int t, int lane, const GatePartials gp, float* __restrict__ logits, int T, int E, int K,
+                                                 int route_norm, float route_scale, float& out_s, int& out_e) {
+  float* row = logits + (int64_t)t * E;
   float val[EPL];
-  unsigned long long key[EPL];
+  uint32_t key[EPL];
+  if (PARTIALS) {
+    const int64_t n = (int64_t)T * E;
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      const int e = lane + 64 * j;
+      float s = 0.f;
+      if (e < E) {
+        const float* src = gp.part + (int64_t)t * E + e;
+        float v[8];
+#pragma unroll
+        for (int z = 0; z < 8; ++z) v[z] = z < gp.splits ? src[z * n] : 0.f;
+#pragma unroll
+        for (int z = 0; z < 8; ++z)
+          if (z < gp.splits) s += v[z];
+        if (gp.bias) s += gp.bias[e];
+        row[e] = s;
+      }
+      val[j] = s;
+    }
+  }
 #pragma unroll
   for (int j = 0; j < EPL; ++j) {
     const int e = lane + 64 * j;
     if (e < E) {
-      val[j] = row[e];
-      key[j] = ((unsigned long long)orderable(val[j]) << 32) | (unsigned long long)(0xffffffffu - (uint32_t)e);
+      if (!PARTIALS) val[j] = row[e];
+      key[j] = orderable(val[j]);
     } else {
       val[j] = 0.f;
-      key[j] = 0ull;  // never wins: every real key has a non-zero high word
+      key[j] = 0u;  // never wins: no value maps to 0 (the smallest, -inf, maps to 0x007fffff)
     }
   }
 
@@ -50,41 +104,72 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_kernel(
   float my_v = 0.f;
   int my_e = 0;
   for (int k = 0; k < K; ++k) {
-    unsigned long long best = 0ull;
+    uint32_t best = 0u;
 #pragma unroll
     for (int j = 0; j < EPL; ++j) best = key[j] > best ? key[j] : best;
-    best = pk_wave_max_u64(best);
-    const uint32_t e_win = 0xffffffffu - (uint32_t)(best & 0xffffffffull);
-    const float v_win = from_orderable((uint32_t)(best >> 32));
+    best = wave_max_u32(best);
+    // the lowest expert id among those that hold the maximum: ids are lane + 64 j
+    int e_win = 0;
+    bool found = false;
 #pragma unroll
-    for (int j = 0; j < EPL; ++j)
-      if ((int)e_win == lane + 64 * j) key[j] = 0ull;
+    for (int j = 0; j < EPL; ++j) {
+      const unsigned long long at = __ballot(key[j] == best);
+      if (!found && at != 0ull) {
+        found = true;
+        const int l = (int)__ffsll((long long)at) - 1;
+        e_win = l + 64 * j;
+        if (lane == l) key[j] = 0u;
+      }
+    }
+    const float v_win = from_orderable(best);
     if (k == 0) vmax = v_win;
-    if (lane == k) { my_v = v_win; my_e = (int)e_win; }
+    if (lane == k) { my_v = v_win; my_e = e_win; }
   }
 
   float part = 0.f;
 #pragma unroll
   for (int j = 0; j < EPL; ++j)
     if (lane + 64 * j < E) part += expf(val[j] - vmax);
-  const float denom = pk_wave_sum(part);
+  const float denom = wave_sum_f32(part);
 
   float s = (lane < K) ? expf(my_v - vmax) / denom : 0.f;
   if (route_norm) {
-    const float S = pk_wave_sum(s);
+    const float S = wave_sum_f32(s);
     s = s / (S + 1e-20f);
   }
-  s *= route_scale;
+  out_s = s * route_scale;
+  out_e = my_e;
+}
+
+template <int EPL, bool PARTIALS>
+__global__ __launch_bounds__(kRouteThreads) void route_topk_kernel(
+    const GatePartials gp, float* __restrict__ logits, int T, int E, int K, int route_norm, float route_scale,
+    float* __restrict__ top_scores, int32_t* __restrict__ top_idx) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = blockIdx.x * (kRouteThreads / 64) + wave;
+  if (t >= T) return;
+  float s;
+  int e;
+  route_topk_token<EPL, PARTIALS>(t, lane, gp, logits, T, E, K, route_norm, route_scale, s, e);
   if (lane < K) {
     top_scores[(int64_t)t * K + lane] = s;
-    top_idx[(int64_t)t * K + lane] = my_e;
+    top_idx[(int64_t)t * K + lane] = e;
   }
 }
 
+// Where the score gradients come from and where d_logits goes besides its own tensor.
+struct RouteBwdIo {
+  const float* d_top_scores;    // [T, K], or nullptr:
+  const float* part;            //   the d_h GEMM's partial sums [n_part][A], in sorted row order
+  const int32_t* inv_perm;      //   flat slot -> sorted row
+  int64_t A;
+  int32_t n_part;
+  bf16_t* planes;               // optional: d_logits as three bf16 planes [3][T * E] for the gate weight gradient
+};
 template <int EPL>
 __global__ __launch_bounds__(kRouteThreads) void route_topk_bwd_kernel(
     const float* __restrict__ logits, const int32_t* __restrict__ top_idx,
-    const float* __restrict__ d_top_scores, int T, int E, int K, int route_norm,
+    const RouteBwdIo io, int T, int E, int K, int route_norm,
     float route_scale, float* __restrict__ d_logits) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int t = blockIdx.x * (kRouteThreads / 64) + wave;
@@ -99,7 +184,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_bwd_kernel(
     val[j] = (e < E) ? row[e] : -INFINITY;
     mx = fmaxf(mx, val[j]);
   }
-  mx = pk_wave_max(mx);
+  mx = from_orderable(wave_max_u32(orderable(mx)));
   float p[EPL];
   float part = 0.f;
 #pragma unroll
@@ -107,7 +192,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_bwd_kernel(
     p[j] = (lane + 64 * j < E) ? expf(val[j] - mx) : 0.f;
     part += p[j];
   }
-  const float denom = pk_wave_sum(part);
+  const float denom = wave_sum_f32(part);
 #pragma unroll
   for (int j = 0; j < EPL; ++j) p[j] = p[j] / denom;
 
@@ -117,25 +202,37 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_bwd_kernel(
   if (lane < K) {
     my_e = top_idx[(int64_t)t * K + lane];
     s = expf(row[my_e] - mx) / denom;
-    dw = d_top_scores[(int64_t)t * K + lane];
+    if (io.d_top_scores) {
+      dw = io.d_top_scores[(int64_t)t * K + lane];
+    } else {      // summed in partial order, like dscore_reduce_kernel
+      const int64_t r = io.inv_perm[(int64_t)t * K + lane];
+      for (int q0 = 0; q0 < io.n_part; q0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = q0 + q < io.n_part ? io.part[(q0 + q) * io.A + r] : 0.f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          if (q0 + q < io.n_part) dw += v[q];
+      }
+    }
   }
   float ds;
   if (route_norm) {
-    const float S = pk_wave_sum(s) + 1e-20f;
-    const float dot = pk_wave_sum(dw * s);
+    const float S = wave_sum_f32(s) + 1e-20f;
+    const float dot = wave_sum_f32(dw * s);
     ds = route_scale * (dw / S - dot / (S * S));
   } else {
     ds = route_scale * dw;
   }
   if (lane >= K) ds = 0.f;
-  const float D = pk_wave_sum(ds * s);  // sum_j dp_j p_j
+  const float D = wave_sum_f32(ds * s);  // sum_j dp_j p_j
 
   float dp[EPL];
 #pragma unroll
   for (int j = 0; j < EPL; ++j) dp[j] = 0.f;
   for (int k = 0; k < K; ++k) {
-    const int ek = __shfl(my_e, k, PK_WAVE);
-    const float dsk = __shfl(ds, k, PK_WAVE);
+    const int ek = __builtin_amdgcn_readlane(my_e, k);
+    const float dsk = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ds), k));
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
       if (lane + 64 * j == ek) dp[j] = dsk;
@@ -143,7 +240,17 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_bwd_kernel(
 #pragma unroll
   for (int j = 0; j < EPL; ++j) {
     const int e = lane + 64 * j;
-    if (e < E) d_logits[(int64_t)t * E + e] = p[j] * (dp[j] - D);
+    if (e < E) {
+      const float d = p[j] * (dp[j] - D);
+      const int64_t at = (int64_t)t * E + e;
+      d_logits[at] = d;
+      if (io.planes) {
+        const int64_t n = (int64_t)T * E;
+        bf16_t pl[3];
+        pk_x3mm::split<3>(d, pl);
+        io.planes[at] = pl[0]; io.planes[n + at] = pl[1]; io.planes[2 * n + at] = pl[2];
+      }
+    }
   }
 }
 
@@ -167,124 +274,231 @@ __global__ __launch_bounds__(64) void sort_hist_kernel(const int32_t* __restrict
   for (int e = threadIdx.x; e < E; e += 64) chunk_hist[(int64_t)blockIdx.x * E + e] = hist[e];
 }
 
-// Single block.  counts[e] = sum over chunks; starts = exclusive scan; chunk_hist[c][e] is
-// replaced by the first output position of expert e's rows coming from chunk c.
-__global__ __launch_bounds__(1024) void sort_scan_kernel(int32_t* __restrict__ chunk_hist,
-                                                         int nchunks, int E,
-                                                         int32_t* __restrict__ counts,
-                                                         int32_t* __restrict__ starts,
-                                                         int32_t* __restrict__ order) {
-  // One block.  The 1024 threads form G = 1024 / Epad groups (Epad = E rounded up to a power of
-  // two); group g of expert e walks chunks [g*cpg, (g+1)*cpg), so the two passes over the
-  // chunk histograms are G times shorter than with one thread per expert.
-  __shared__ int32_t part[1024];     // [g][e]: rows of expert e in the chunks of group g
-  __shared__ int32_t scan[PK_MAX_EXPERTS];
-  __shared__ int32_t cnts[PK_MAX_EXPERTS];
-  int epad = 1;
-  while (epad < E) epad <<= 1;
-  const int G = 1024 / epad;
-  const int e = threadIdx.x % epad, g = threadIdx.x / epad;
-  const int cpg = (nchunks + G - 1) / G;
-  const int c0 = g * cpg, c1 = min(nchunks, c0 + cpg);
-  // (both walks over the chunks fetch eight values at a time: one round trip per eight chunks)
-  constexpr int WALK = 8;
-  int mine = 0;
-  if (e < E)
-    for (int c = c0; c < c1; c += WALK) {
-      int v[WALK];
-#pragma unroll
-      for (int i = 0; i < WALK; ++i) v[i] = c + i < c1 ? chunk_hist[(int64_t)(c + i) * E + e] : 0;
-#pragma unroll
-      for (int i = 0; i < WALK; ++i) mine += v[i];
-    }
-  part[threadIdx.x] = mine;
-  __syncthreads();
-  int total = 0, before = 0;      // rows of expert e in all chunks / in the chunks of earlier groups
-  for (int k = 0; k < G; ++k) {
-    const int v = part[k * epad + e];
-    total += v;
-    before += k < g ? v : 0;
+// Lanes of the wave that hold the same expert id as this one (ids below 1,024; inactive lanes: none).
+__device__ __forceinline__ unsigned long long same_expert_lanes(int e, bool active, int id_bits) {
+  unsigned long long same = __ballot(active);
+  for (int b = 0; b < id_bits; ++b) {
+    const unsigned long long bal = __ballot((e >> b) & 1);
+    same &= ((e >> b) & 1) ? bal : ~bal;
   }
-  if (threadIdx.x < 1024 && g == 0) {
-    if (e < E && counts) counts[e] = total;
-    scan[e] = (e < E) ? total : 0;
-    cnts[e] = (e < E) ? total : -1;
-  }
-  __syncthreads();
-  if (order && g == 0 && e < E) {
-    // experts by descending row count, ties by index: order[rank] = e
-    int rank = 0;
-    for (int o = 0; o < E; ++o) {
-      const int oc = cnts[o];
-      rank += (oc > total || (oc == total && o < e)) ? 1 : 0;
-    }
-    order[rank] = e;
-  }
-  // Hillis-Steele inclusive scan over the Epad expert totals
-  for (int off = 1; off < epad; off <<= 1) {
-    int v = 0;
-    if (g == 0 && e >= off) v = scan[e - off];
-    __syncthreads();
-    if (g == 0) scan[e] += v;
-    __syncthreads();
-  }
-  const int start = scan[e] - total;  // exclusive
-  if (e < E) {
-    if (g == 0) {
-      starts[e] = start;
-      if (e == E - 1) starts[E] = scan[e];
-    }
-    int run = start + before;
-    for (int c = c0; c < c1; c += WALK) {
-      int v[WALK];
-#pragma unroll
-      for (int i = 0; i < WALK; ++i) v[i] = c + i < c1 ? chunk_hist[(int64_t)(c + i) * E + e] : 0;
-#pragma unroll
-      for (int i = 0; i < WALK; ++i)
-        if (c + i < c1) {
-          chunk_hist[(int64_t)(c + i) * E + e] = run;
-          run += v[i];
-        }
-    }
-  }
+  return same;
 }
-
-__global__ __launch_bounds__(64) void sort_scatter_kernel(const int32_t* __restrict__ idx, int A,
-                                                          int E, const int32_t* __restrict__ chunk_base,
-                                                          int32_t* __restrict__ perm,
-                                                          int32_t* __restrict__ inv_perm) {
-  extern __shared__ int32_t base[];  // [E] next free position per expert
-  const int lane = threadIdx.x;
-  for (int e = lane; e < E; e += 64) base[e] = chunk_base[(int64_t)blockIdx.x * E + e];
-  __syncthreads();
-  const int s0 = blockIdx.x * kSortChunk;
+// One wave places slots [s0, s0 + n), in order: `cursor` (LDS, private to the wave) holds the next free
+// position per expert.  The rank of a slot among the 64 of a step is a population count, so equal
+// experts keep their slot order.
+__device__ __forceinline__ void place_slots(const int32_t* __restrict__ idx, int s0, int n, int A, int E, int id_bits, int32_t* cursor,
+                                            int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm) {
+  const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int i = 0; i < kSortChunk; i += 64) {
+  for (int i = 0; i < n; i += 64) {
     const int s = s0 + i + lane;
-    int e = (s < A) ? idx[s] : -1;
-    if ((unsigned)e >= (unsigned)E) e = -1;
-    const bool active = e >= 0;
-    // lanes holding the same expert id
-    unsigned long long same = __ballot(active);
-    for (int b = 0; b < 10; ++b) {
-      const unsigned long long bal = __ballot((e >> b) & 1);
-      same &= ((e >> b) & 1) ? bal : ~bal;
-    }
+    int e = (i + lane < n && s < A) ? idx[s] : -1;
+    const bool active = (unsigned)e < (unsigned)E;      // out-of-range ids are dropped
+    const unsigned long long same = same_expert_lanes(e, active, id_bits);
     int pos = 0;
+    if (active) pos = cursor[e] + __popcll(same & lt_mask);
+    __builtin_amdgcn_wave_barrier();
     if (active) {
-      const int rank = __popcll(same & lt_mask);
-      pos = base[e] + rank;
-    }
-    __syncthreads();
-    if (active) {
-      // the last lane of each group advances the expert's cursor
-      const int top = 63 - __clzll(same);
-      if (lane == top) base[e] += __popcll(same);
+      if (lane == 63 - __clzll(same)) cursor[e] += __popcll(same);     // the last lane of a group advances the cursor
       perm[pos] = s;
       if (inv_perm) inv_perm[s] = pos;
     }
-    __syncthreads();
+    __builtin_amdgcn_wave_barrier();
   }
+}
+__host__ __device__ inline int id_bits_for(int E) {
+  int b = 0;
+  while ((1 << b) < E) ++b;
+  return b;
+}
+// Exclusive prefix sum over v[0, n) in LDS by the whole block (n <= blockDim.x rounded up to a power of
+// two); every thread passes its own element and gets its exclusive sum.
+__device__ __forceinline__ int block_exclusive_scan(int mine, int32_t* wave_sums) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int incl = mine;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(incl, off, PK_WAVE);
+    if (lane >= off) incl += v;
+  }
+  if (lane == 63) wave_sums[wave] = incl;
+  __syncthreads();
+  int before = 0;
+  for (int w = 0; w < nw; ++w) before += w < wave ? wave_sums[w] : 0;
+  __syncthreads();
+  return before + incl - mine;
+}
+// order[rank] = e: experts by descending row count, ties by index.  cnt: LDS, rank: LDS scratch [E].
+__device__ __forceinline__ void write_order(const int32_t* cnt, int32_t* rank, int E, int32_t* __restrict__ order) {
+  for (int e = threadIdx.x; e < E; e += blockDim.x) rank[e] = 0;
+  __syncthreads();
+  int parts = blockDim.x / E;                    // threads that share an expert's comparisons
+  if (parts < 1) parts = 1;
+  for (int i = threadIdx.x; i < E * parts; i += blockDim.x) {
+    const int e = i % E, part = i / E, c = cnt[e];
+    int r = 0;
+    for (int o = part; o < E; o += parts) {
+      const int oc = cnt[o];
+      r += (oc > c || (oc == c && o < e)) ? 1 : 0;
+    }
+    if (r) atomicAdd(&rank[e], r);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += blockDim.x) order[rank[e]] = e;
+}
+
+// The whole sort in one workgroup of 16 waves, for inputs short enough that one CU's scattered stores
+// (about one lane per cycle) do not matter: wave w owns the w-th sixteenth of the slots, counts its
+// experts in LDS, the counts become first positions, and it places its slots.  Three launches took
+// 16 us at 192 slots and 19 us at 4,072 (mostly gaps and latency), this one 5 and 11 us; at 8,192 the
+// two kernels below are as quick.
+constexpr int kSmallSortWaves = 16, kSmallSortSlots = 4096, kSmallSortExperts = 512;
+struct SortOut {
+  int32_t *counts, *starts, *perm, *inv_perm, *order;     // counts, inv_perm, order may be null
+};
+struct SmallSortLds {
+  int32_t hist[kSmallSortWaves * kSmallSortExperts];      // [wave][E]
+  int32_t cnt[kSmallSortExperts], rank[kSmallSortExperts], wave_sums[kSmallSortWaves];
+};
+__device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, const SortOut& out, SmallSortLds& l) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int per = ((A + kSmallSortWaves - 1) / kSmallSortWaves + 63) & ~63;      // slots per wave
+  const int s0 = wave * per;
+  for (int i = threadIdx.x; i < kSmallSortWaves * E; i += blockDim.x) l.hist[i] = 0;
+  __syncthreads();
+  for (int i = lane; i < per; i += 64) {
+    const int s = s0 + i;
+    if (s < A) {
+      const int e = idx[s];
+      if ((unsigned)e < (unsigned)E) atomicAdd(&l.hist[wave * E + e], 1);
+    }
+  }
+  __syncthreads();
+  const int e = threadIdx.x;
+  int total = 0;
+  if (e < E) {
+#pragma unroll
+    for (int w = 0; w < kSmallSortWaves; ++w) total += l.hist[w * E + e];
+  }
+  const int start = block_exclusive_scan(total, l.wave_sums);
+  if (e < E) {
+    int run = start;
+    for (int w = 0; w < kSmallSortWaves; ++w) {
+      const int n = l.hist[w * E + e];
+      l.hist[w * E + e] = run;
+      run += n;
+    }
+    l.cnt[e] = total;
+    if (out.counts) out.counts[e] = total;
+    out.starts[e] = start;
+    if (e == E - 1) out.starts[E] = run;
+  }
+  __syncthreads();
+  place_slots(idx, s0, per, A, E, id_bits_for(E), &l.hist[wave * E], out.perm, out.inv_perm);
+  if (out.order) write_order(l.cnt, l.rank, E, out.order);
+}
+__global__ __launch_bounds__(64 * kSmallSortWaves) void sort_small_kernel(const int32_t* __restrict__ idx, int A, int E, const SortOut out) {
+  __shared__ SmallSortLds l;
+  sort_small(idx, A, E, out, l);
+}
+// Top-k and sort in one launch for a decode step: the 16 waves take the tokens in turn and hand the
+// chosen experts over in LDS.
+constexpr int kRouteSortTokens = 32, kRouteSortSlots = 1024;
+template <int EPL, bool PARTIALS>
+__global__ __launch_bounds__(64 * kSmallSortWaves) void route_sort_small_kernel(const GatePartials gp, float* __restrict__ logits, int T, int E, int K,
+                                                                                int route_norm, float route_scale, float* __restrict__ top_scores,
+                                                                                int32_t* __restrict__ top_idx, const SortOut out) {
+  __shared__ SmallSortLds l;
+  __shared__ int32_t chosen[kRouteSortSlots];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int t = wave; t < T; t += kSmallSortWaves) {
+    float s;
+    int e;
+    route_topk_token<EPL, PARTIALS>(t, lane, gp, logits, T, E, K, route_norm, route_scale, s, e);
+    if (lane < K) {
+      top_scores[t * K + lane] = s;
+      top_idx[t * K + lane] = e;
+      chosen[t * K + lane] = e;
+    }
+  }
+  __syncthreads();
+  sort_small(chosen, T * K, E, out, l);
+}
+
+// Longer inputs: after sort_hist_kernel one workgroup per chunk works out for itself where every expert
+// starts and how many of its rows come from earlier chunks -- all of them read all the chunk
+// histograms, a few tens of kB out of the L2, which is quicker than a launch of one workgroup in
+// between that everybody waits for (10 us at 64 chunks, 16 us at 256) -- and then places its chunk with
+// four waves.  Workgroup 0 also writes counts, starts and order.
+constexpr int kScatterThreads = 1024, kScatterWaves = kSortChunk / 128;
+__global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int32_t* __restrict__ idx, int A, int E,
+                                                                       const int32_t* __restrict__ chunk_hist, int nchunks,
+                                                                       int32_t* __restrict__ counts, int32_t* __restrict__ starts,
+                                                                       int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm,
+                                                                       int32_t* __restrict__ order) {
+  extern __shared__ int32_t lds[];                   // cnt [E], before [E], cursor [kScatterWaves][E]
+  __shared__ int32_t wave_sums[kScatterThreads / 64];
+  int32_t* const cnt = lds;
+  int32_t* const before = lds + E;
+  int32_t* const cursor = lds + 2 * E;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int chunk = blockIdx.x;
+  for (int i = threadIdx.x; i < (2 + kScatterWaves) * E; i += blockDim.x) lds[i] = 0;
+  __syncthreads();
+  {
+    // 1024 threads = G groups of E columns; group g adds up chunks g, g + G, ..., eight loads at a time
+    int cols = 1;
+    while (cols < E) cols <<= 1;
+    const int e = threadIdx.x % cols, g = threadIdx.x / cols, G = blockDim.x / cols;
+    constexpr int WALK = 8;
+    int total = 0, early = 0;
+    if (e < E)
+      for (int c = g; c < nchunks; c += G * WALK) {
+        int v[WALK];
+#pragma unroll
+        for (int i = 0; i < WALK; ++i) v[i] = c + i * G < nchunks ? chunk_hist[(int64_t)(c + i * G) * E + e] : 0;
+#pragma unroll
+        for (int i = 0; i < WALK; ++i) {
+          total += v[i];
+          early += c + i * G < chunk ? v[i] : 0;
+        }
+      }
+    if (e < E) {
+      atomicAdd(&cnt[e], total);
+      atomicAdd(&before[e], early);
+    }
+  }
+  // the wave's own share of the chunk, counted before anything is placed
+  const int s0 = chunk * kSortChunk + wave * 128;
+  if (wave < kScatterWaves)
+    for (int i = lane; i < 128; i += 64) {
+      const int s = s0 + i;
+      if (s < A) {
+        const int e = idx[s];
+        if ((unsigned)e < (unsigned)E) atomicAdd(&cursor[wave * E + e], 1);
+      }
+    }
+  __syncthreads();
+  const int e = threadIdx.x;
+  const int total = e < E ? cnt[e] : 0;
+  const int start = block_exclusive_scan(total, wave_sums);
+  if (e < E) {
+    int run = start + before[e];
+#pragma unroll
+    for (int w = 0; w < kScatterWaves; ++w) {
+      const int n = cursor[w * E + e];
+      cursor[w * E + e] = run;
+      run += n;
+    }
+    if (chunk == 0) {
+      if (counts) counts[e] = total;
+      starts[e] = start;
+      if (e == E - 1) starts[E] = start + total;
+    }
+  }
+  __syncthreads();
+  if (wave < kScatterWaves) place_slots(idx, s0, 128, A, E, id_bits_for(E), cursor + wave * E, perm, inv_perm);
+  if (chunk == 0 && order) write_order(cnt, before, E, order);
 }
 
 __global__ __launch_bounds__(1024) void counts_to_starts_kernel(const void* __restrict__ counts,
@@ -441,13 +655,73 @@ int64_t pk_gate_workspace_bytes(int64_t T, int64_t H, int64_t E) {
   return gate_fwd_partial_bytes(T, H, E);
 }
 
-int pk_gate_logits(const void* x, int x_dtype, const float* w_gate, const float* gate_bias,
-                   float* logits, int64_t T, int64_t H, int64_t E, void* workspace,
-                   int64_t workspace_bytes, pk_stream_t stream) {
+}  // extern "C"
+
+// The gate for a few tokens: one wave per expert and TOKENS tokens, lanes along the reduction, fp32 FMAs.
+// The GEMM pads the tokens to 64 and walks the reduction in latency-bound k-tiles: 14 us at one token,
+// 18 us at 24 (width 2048, 128 experts); here the loads of eight steps are in flight at once.
+constexpr int kGateTokens = 4, kGateSmallMax = 64;
+template <typename T, int TOKENS>
+__global__ __launch_bounds__(256) void gate_small_kernel(const T* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+                                                         float* __restrict__ logits, int tokens, int H, int E) {
+  constexpr int STEPS = TOKENS == 1 ? 8 : 4;
+  const int lane = threadIdx.x & 63;
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int t0 = blockIdx.y * TOKENS;
+  if (e >= E) return;
+  float acc[TOKENS];
+  const T* xr[TOKENS];
+#pragma unroll
+  for (int j = 0; j < TOKENS; ++j) {
+    acc[j] = 0.f;
+    xr[j] = x + (int64_t)min(t0 + j, tokens - 1) * H;      // past the end: the last token again, not stored
+  }
+  const float* wr = w + (int64_t)e * H;
+  for (int k0 = 4 * lane; k0 < H; k0 += 256 * STEPS) {
+    float wv[STEPS][4], xv[STEPS][TOKENS][4];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const int k = k0 + 256 * s;
+      const int kk = k < H ? k : 0;
+      pk_f32mm::load4<float>(wr + kk, wv[s]);
+#pragma unroll
+      for (int j = 0; j < TOKENS; ++j) pk_f32mm::load4<T>(xr[j] + kk, xv[s][j]);
+    }
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+      if (k0 + 256 * s < H) {
+#pragma unroll
+        for (int j = 0; j < TOKENS; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[j] = fmaf(xv[s][j][i], wv[s][i], acc[j]);
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < TOKENS; ++j) {
+    const float s = wave_sum_f32(acc[j]);
+    if (lane == 0 && t0 + j < tokens) logits[(int64_t)(t0 + j) * E + e] = s + (bias ? bias[e] : 0.f);
+  }
+}
+
+// The gate GEMM.  *splits > 1: `workspace` holds that many partial results [T, E] and logits is not
+// written yet (no bias either); otherwise the logits are complete.
+static int gate_gemm(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, float* logits, int64_t T, int64_t H,
+                     int64_t E, void* workspace, int64_t workspace_bytes, hipStream_t s, int* splits) {
   if (T < 0 || H <= 0 || E <= 0 || !pk_dtype_ok(x_dtype)) return PK_ERR_ARG;
+  *splits = 1;
   if (T == 0) return PK_OK;
   if (!x || !w_gate || !logits) return PK_ERR_ARG;
-  hipStream_t s = (hipStream_t)stream;
+  if (T <= kGateSmallMax && H % 4 == 0 && pk_aligned16(x) && pk_aligned16(w_gate)) {
+    const dim3 grid((unsigned)pk_ceil_div(E, 4), (unsigned)pk_ceil_div(T, T == 1 ? 1 : kGateTokens)), block(256);
+#define PK_GATE_SMALL(TYPE, N)                                                                                                  \
+  PK_LAUNCH_NOCHECK(pk_timing::K_GATE_LOGITS, s, (gate_small_kernel<TYPE, N>), grid, block, 0, s, (const TYPE*)x, w_gate, gate_bias, \
+                    logits, (int)T, (int)H, (int)E)
+    if (x_dtype == PK_BF16) { if (T == 1) PK_GATE_SMALL(bf16_t, 1); else PK_GATE_SMALL(bf16_t, kGateTokens); }
+    else { if (T == 1) PK_GATE_SMALL(float, 1); else PK_GATE_SMALL(float, kGateTokens); }
+#undef PK_GATE_SMALL
+    PK_RETURN_IF_LAUNCH_FAILED();
+    return PK_OK;
+  }
   int sp = gate_fwd_splits(H);
   // the reduction is split only as far as it takes to give every CU two workgroups: each split
   // writes and re-reads a [T, E] fp32 partial result, which soon outweighs reading x
@@ -463,34 +737,47 @@ int pk_gate_logits(const void* x, int x_dtype, const float* w_gate, const float*
   p.M = T; p.N = E; p.K = H;
   p.sam = H; p.sak = 1; p.sbk = 1; p.sbn = H;
   p.splits = sp; p.accumulate = 0;
-  int rc;
+  *splits = sp;
   const bool xb = x_dtype == PK_BF16;
   if (E > 64)  // 64-token x 128-expert tiles, 8 waves
-    rc = xb ? pk_x3mm::launch<2, 4, true, true, bf16_t, float>(p, pk_timing::K_GATE_LOGITS, s)
-            : pk_x3mm::launch<2, 4, true, true, float, float>(p, pk_timing::K_GATE_LOGITS, s);
-  else         // 64-token x 64-expert tiles, 4 waves
-    rc = xb ? pk_x3mm::launch<2, 2, true, true, bf16_t, float>(p, pk_timing::K_GATE_LOGITS, s)
+    return xb ? pk_x3mm::launch<2, 4, true, true, bf16_t, float>(p, pk_timing::K_GATE_LOGITS, s)
+              : pk_x3mm::launch<2, 4, true, true, float, float>(p, pk_timing::K_GATE_LOGITS, s);
+  // 64-token x 64-expert tiles, 4 waves
+  return xb ? pk_x3mm::launch<2, 2, true, true, bf16_t, float>(p, pk_timing::K_GATE_LOGITS, s)
             : pk_x3mm::launch<2, 2, true, true, float, float>(p, pk_timing::K_GATE_LOGITS, s);
-  if (rc != PK_OK) return rc;
-  if (sp > 1) {
-    const int64_t n = T * E;
-    PK_LAUNCH_NOCHECK(pk_timing::K_GATE_LOGITS, s, pk_f32mm::reduce_partials_kernel,
-                      dim3((unsigned)pk_ceil_div(n, 256)), dim3(256), 0, s,
-                      reinterpret_cast<const float*>(workspace), logits, n, sp, 0, gate_bias, (int)E);
-    PK_RETURN_IF_LAUNCH_FAILED();
-  }
+}
+
+extern "C" {
+
+int pk_gate_logits(const void* x, int x_dtype, const float* w_gate, const float* gate_bias,
+                   float* logits, int64_t T, int64_t H, int64_t E, void* workspace,
+                   int64_t workspace_bytes, pk_stream_t stream) {
+  hipStream_t s = (hipStream_t)stream;
+  int splits = 1;
+  const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, s, &splits);
+  if (rc != PK_OK || splits == 1) return rc;
+  const int64_t n = T * E;
+  PK_LAUNCH_NOCHECK(pk_timing::K_GATE_LOGITS, s, pk_f32mm::reduce_partials_kernel,
+                    dim3((unsigned)pk_ceil_div(n, 256)), dim3(256), 0, s,
+                    reinterpret_cast<const float*>(workspace), logits, n, splits, 0, gate_bias, (int)E);
+  PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
 
-static int gate_bwd_splits(int64_t T) {
-  int64_t sp = T / 256;
+// Workgroups that share the reduction over the tokens in the weight-gradient GEMM: one per 256 tokens,
+// and with few output tiles (H/64 x E/64) more, down to 64 tokens each, until there are two for a CU
+// (509 tokens, 512 x 16, fp32: 26 us on 8 workgroups, 9 us on 64).
+static int gate_bwd_splits(int64_t T, int64_t H, int64_t E) {
+  const int64_t tiles = pk_ceil_div(H, 64) * pk_ceil_div(E, 64);
+  int64_t sp = T / 256, fill = 512 / tiles < T / 64 ? 512 / tiles : T / 64;
+  if (fill > sp) sp = fill;
   return (int)(sp < 1 ? 1 : (sp > 16 ? 16 : sp));
 }
 
 // workspace of the backward: [split-K partials of d_w_gate, reused for the bias partial sums]
 // [d_logits as three bf16 planes, for the weight gradient]
 static int64_t gate_bwd_partial_bytes(int64_t T, int64_t H, int64_t E) {
-  const int sp = gate_bwd_splits(T);
+  const int sp = gate_bwd_splits(T, H, E);
   const int64_t part = sp > 1 ? (int64_t)sp * E * H * (int64_t)sizeof(float) : 0;
   const int64_t colsum = (int64_t)kColsumBlocks * E * (int64_t)sizeof(float);
   return align256(part > colsum ? part : colsum);
@@ -501,10 +788,13 @@ int64_t pk_gate_bwd_workspace_bytes(int64_t T, int64_t H, int64_t E) {
   return gate_bwd_partial_bytes(T, H, E) + plane_bytes(T * E);
 }
 
-int pk_gate_logits_bwd(const float* d_logits, const void* x, int x_dtype, const float* w_gate,
-                       float* d_x_f32, float* d_w_gate, float* d_gate_bias, int accumulate,
-                       int64_t T, int64_t H, int64_t E, void* workspace, int64_t workspace_bytes,
-                       pk_stream_t stream) {
+}  // extern "C"
+
+// planes_ready: d_logits already lies split in the workspace, where this function would put it
+static int gate_bwd(const float* d_logits, const void* x, int x_dtype, const float* w_gate,
+                    float* d_x_f32, float* d_w_gate, float* d_gate_bias, int accumulate,
+                    int64_t T, int64_t H, int64_t E, void* workspace, int64_t workspace_bytes, bool planes_ready,
+                    pk_stream_t stream) {
   if (T < 0 || H <= 0 || E <= 0 || !pk_dtype_ok(x_dtype)) return PK_ERR_ARG;
   if (!d_logits && T > 0) return PK_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
@@ -524,7 +814,7 @@ int pk_gate_logits_bwd(const float* d_logits, const void* x, int x_dtype, const 
   }
   if (d_w_gate) {
     if (!x && T > 0) return PK_ERR_ARG;
-    int sp = gate_bwd_splits(T);
+    int sp = gate_bwd_splits(T, H, E);
     if (sp > 1 && !have_part) sp = 1;
     pk_f32mm::Params p = {};
     p.B = x;
@@ -541,8 +831,10 @@ int pk_gate_logits_bwd(const float* d_logits, const void* x, int x_dtype, const 
     int rc = PK_ERR_ALIGN;
     if (presplit) {
       bf16_t* planes = reinterpret_cast<bf16_t*>(reinterpret_cast<char*>(workspace) + part_bytes);
-      rc = split_planes(d_logits, planes, T * E, pk_timing::K_GATE_LOGITS_BWD, s);
-      if (rc != PK_OK) return rc;
+      if (!planes_ready) {
+        rc = split_planes(d_logits, planes, T * E, pk_timing::K_GATE_LOGITS_BWD, s);
+        if (rc != PK_OK) return rc;
+      }
       p.A = planes; p.plane_a = T * E;
       rc = x_dtype == PK_BF16 ? pk_x3mm::launch<2, 2, false, false, split3_t, bf16_t>(p, pk_timing::K_GATE_LOGITS_BWD, s)
                               : pk_x3mm::launch<2, 2, false, false, split3_t, float>(p, pk_timing::K_GATE_LOGITS_BWD, s);
@@ -583,6 +875,15 @@ int pk_gate_logits_bwd(const float* d_logits, const void* x, int x_dtype, const 
   return PK_OK;
 }
 
+extern "C" {
+
+int pk_gate_logits_bwd(const float* d_logits, const void* x, int x_dtype, const float* w_gate,
+                       float* d_x_f32, float* d_w_gate, float* d_gate_bias, int accumulate,
+                       int64_t T, int64_t H, int64_t E, void* workspace, int64_t workspace_bytes,
+                       pk_stream_t stream) {
+  return gate_bwd(d_logits, x, x_dtype, w_gate, d_x_f32, d_w_gate, d_gate_bias, accumulate, T, H, E, workspace, workspace_bytes, false, stream);
+}
+
 #define PK_DISPATCH_EPL(E, LAUNCH)                 \
   do {                                             \
     if ((E) <= 64) { LAUNCH(1); }                  \
@@ -601,10 +902,44 @@ int pk_route_topk(const float* logits, int64_t T, int64_t E, int64_t K, int rout
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)pk_ceil_div(T, kRouteThreads / 64)), block(kRouteThreads);
 #define PK_LAUNCH_TOPK(EPL)                                                                 \
-  PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK, s, (route_topk_kernel<EPL>), grid, block, 0, s, logits, (int)T, (int)E,   \
-                     (int)K, route_norm, route_scale, top_scores, top_idx)
+  PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK, s, (route_topk_kernel<EPL, false>), grid, block, 0, s, GatePartials{}, const_cast<float*>(logits), \
+                     (int)T, (int)E, (int)K, route_norm, route_scale, top_scores, top_idx)
   PK_DISPATCH_EPL(E, PK_LAUNCH_TOPK);
 #undef PK_LAUNCH_TOPK
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+
+int pk_gate_route(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, int64_t T, int64_t H, int64_t E, int64_t K,
+                  int route_norm, float route_scale, float* logits, float* top_scores, int32_t* top_idx, void* workspace,
+                  int64_t workspace_bytes, pk_stream_t stream) {
+  if (K <= 0) return PK_ERR_ARG;
+  if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E) return PK_ERR_SHAPE;
+  if (T > 0 && (!top_scores || !top_idx)) return PK_ERR_ARG;
+  int splits = 1;
+  const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, (hipStream_t)stream, &splits);
+  if (rc != PK_OK || T == 0) return rc;
+  if (splits == 1) return pk_route_topk(logits, T, E, K, route_norm, route_scale, top_scores, top_idx, stream);
+  hipStream_t s = (hipStream_t)stream;
+  const dim3 grid((unsigned)pk_ceil_div(T, kRouteThreads / 64)), block(kRouteThreads);
+  const GatePartials gp{reinterpret_cast<const float*>(workspace), gate_bias, splits};
+#define PK_LAUNCH_TOPK(EPL)                                                                                              \
+  PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK, s, (route_topk_kernel<EPL, true>), grid, block, 0, s, gp, logits, (int)T, (int)E, \
+                    (int)K, route_norm, route_scale, top_scores, top_idx)
+  PK_DISPATCH_EPL(E, PK_LAUNCH_TOPK);
+#undef PK_LAUNCH_TOPK
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+
+static int route_topk_bwd(const float* logits, const int32_t* top_idx, const RouteBwdIo& io, int64_t T, int64_t E, int64_t K, int route_norm,
+                          float route_scale, float* d_logits, hipStream_t s) {
+  const dim3 grid((unsigned)pk_ceil_div(T, kRouteThreads / 64)), block(kRouteThreads);
+#define PK_LAUNCH_TOPK_BWD(EPL)                                                                                          \
+  PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK_BWD, s, (route_topk_bwd_kernel<EPL>), grid, block, 0, s, logits, top_idx, io, \
+                    (int)T, (int)E, (int)K, route_norm, route_scale, d_logits)
+  PK_DISPATCH_EPL(E, PK_LAUNCH_TOPK_BWD);
+#undef PK_LAUNCH_TOPK_BWD
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
@@ -616,15 +951,65 @@ int pk_route_topk_bwd(const float* logits, const int32_t* top_idx, const float* 
   if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E) return PK_ERR_SHAPE;
   if (T == 0) return PK_OK;
   if (!logits || !top_idx || !d_top_scores || !d_logits) return PK_ERR_ARG;
+  RouteBwdIo io = {};
+  io.d_top_scores = d_top_scores;
+  return route_topk_bwd(logits, top_idx, io, T, E, K, route_norm, route_scale, d_logits, (hipStream_t)stream);
+}
+
+// workspace of pk_region_router_bwd: [what pk_gate_logits_bwd takes][fp32 d_x for operands that the fused
+// kernel cannot read in 16-byte pieces]
+static bool region_bwd_fused(int x_dtype, int64_t H, int64_t E) { return H % (x_dtype == PK_BF16 ? 8 : 4) == 0 && E % 4 == 0; }
+int64_t pk_region_router_bwd_workspace_bytes(int64_t T, int64_t H, int64_t E, int x_dtype) {
+  if (T < 0 || H <= 0 || E <= 0 || !pk_dtype_ok(x_dtype)) return PK_ERR_ARG;
+  return align256(pk_gate_bwd_workspace_bytes(T, H, E)) + (region_bwd_fused(x_dtype, H, E) ? 0 : T * H * (int64_t)sizeof(float));
+}
+
+int pk_region_router_bwd(const float* logits, const int32_t* top_idx, const float* d_top_scores, const float* ds_partial,
+                         int64_t n_partial, const int32_t* inv_perm, int route_norm, float route_scale, const void* x, int x_dtype,
+                         const float* w_gate, const void* d_rows, void* d_x, float* d_w_gate, float* d_gate_bias, int accumulate,
+                         float* d_logits, int64_t T, int64_t H, int64_t E, int64_t K, void* workspace, int64_t workspace_bytes,
+                         pk_stream_t stream) {
+  if (T < 0 || H <= 0 || E <= 0 || K <= 0 || !pk_dtype_ok(x_dtype)) return PK_ERR_ARG;
+  if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E || T > 0x7fffffffll / K) return PK_ERR_SHAPE;
+  if (T > 0 && (!logits || !top_idx || !d_logits || !inv_perm || (!d_top_scores && (!ds_partial || n_partial <= 0)))) return PK_ERR_ARG;
+  if (T > 0 && d_x && (!d_rows || !w_gate)) return PK_ERR_ARG;
+  const int64_t gate_bytes = align256(pk_gate_bwd_workspace_bytes(T, H, E));
+  if (!workspace || workspace_bytes < pk_region_router_bwd_workspace_bytes(T, H, E, x_dtype) || !pk_aligned16(workspace)) return PK_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)pk_ceil_div(T, kRouteThreads / 64)), block(kRouteThreads);
-#define PK_LAUNCH_TOPK_BWD(EPL)                                                              \
-  PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK_BWD, s, (route_topk_bwd_kernel<EPL>), grid, block, 0, s, logits, top_idx,       \
-                     d_top_scores, (int)T, (int)E, (int)K, route_norm, route_scale, d_logits)
-  PK_DISPATCH_EPL(E, PK_LAUNCH_TOPK_BWD);
-#undef PK_LAUNCH_TOPK_BWD
-  PK_RETURN_IF_LAUNCH_FAILED();
-  return PK_OK;
+  int rc;
+  bool planes_ready = false;
+  if (T > 0) {
+    RouteBwdIo io = {};
+    io.d_top_scores = d_top_scores;
+    io.part = ds_partial; io.n_part = (int32_t)n_partial; io.inv_perm = inv_perm; io.A = T * K;
+    if (d_w_gate && plane_bytes(T * E) > 0 && E % 4 == 0) {
+      io.planes = reinterpret_cast<bf16_t*>(reinterpret_cast<char*>(workspace) + gate_bwd_partial_bytes(T, H, E));
+      planes_ready = true;
+    }
+    rc = route_topk_bwd(logits, top_idx, io, T, E, K, route_norm, route_scale, d_logits, s);
+    if (rc != PK_OK) return rc;
+  }
+  if (d_w_gate || d_gate_bias) {
+    rc = gate_bwd(d_logits, x, x_dtype, w_gate, nullptr, d_w_gate, d_gate_bias, accumulate, T, H, E, workspace, gate_bytes, planes_ready, stream);
+    if (rc != PK_OK) return rc;
+  }
+  if (!d_x || T == 0) return PK_OK;
+  pk_f32mm::Params p = {};
+  p.A = d_logits; p.B = w_gate;
+  p.M = T; p.N = H; p.K = E;
+  p.sam = E; p.sak = 1; p.sbk = H; p.sbn = 1;
+  p.splits = 1;
+  const pk_x3mm::GatherAdd ga{d_rows, inv_perm, d_x, (int32_t)K};
+  if (region_bwd_fused(x_dtype, H, E)) {
+    rc = x_dtype == PK_BF16 ? pk_x3mm::launch_gather<bf16_t>(p, ga, pk_timing::K_GATHER_REDUCE, s)
+                            : pk_x3mm::launch_gather<float>(p, ga, pk_timing::K_GATHER_REDUCE, s);
+    return rc;
+  }
+  float* const d_x32 = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + gate_bytes);
+  p.C = d_x32;
+  rc = pk_x3mm::launch<2, 2, true, false, float, float>(p, pk_timing::K_GATE_LOGITS_BWD, s);
+  if (rc != PK_OK) return rc;
+  return pk_permute_bwd(d_rows, x_dtype, inv_perm, d_x32, d_x, T, H, K, stream);
 }
 
 int64_t pk_sort_workspace_bytes(int64_t A, int64_t E) {
@@ -641,20 +1026,62 @@ int pk_sort_by_expert(const int32_t* top_idx, int64_t A, int64_t E, int32_t* cou
   if (!starts || !workspace || (A > 0 && (!top_idx || !perm))) return PK_ERR_ARG;
   if (workspace_bytes < pk_sort_workspace_bytes(A, E)) return PK_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
+  if (A <= kSmallSortSlots && E <= kSmallSortExperts) {
+    PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_small_kernel, dim3(1), dim3(64 * kSmallSortWaves), 0, s, top_idx, (int)A, (int)E,
+                      SortOut{counts, starts, perm, inv_perm, order});
+    PK_RETURN_IF_LAUNCH_FAILED();
+    return PK_OK;
+  }
   const int nchunks = (int)pk_ceil_div(A > 0 ? A : 1, kSortChunk);
   int32_t* chunk_hist = reinterpret_cast<int32_t*>(workspace);
-  const size_t lds = (size_t)E * sizeof(int32_t);
-  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_HIST, s, sort_hist_kernel, dim3(nchunks), dim3(64), lds, s, top_idx, (int)A, (int)E,
+  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_HIST, s, sort_hist_kernel, dim3(nchunks), dim3(64), (size_t)E * sizeof(int32_t), s, top_idx, (int)A, (int)E,
                      chunk_hist);
   PK_RETURN_IF_LAUNCH_FAILED();
-  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCAN, s, sort_scan_kernel, dim3(1), dim3(1024), 0, s, chunk_hist, nchunks, (int)E,
-                     counts, starts, order);
+  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel, dim3(nchunks), dim3(kScatterThreads),
+                    (size_t)(2 + kScatterWaves) * E * sizeof(int32_t), s, top_idx, (int)A, (int)E, chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
   PK_RETURN_IF_LAUNCH_FAILED();
-  if (A > 0) {
-    PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel, dim3(nchunks), dim3(64), lds, s, top_idx, (int)A,
-                       (int)E, chunk_hist, perm, inv_perm);
-    PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+
+int64_t pk_gate_route_sort_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K) {
+  if (T < 0 || H <= 0 || E <= 0 || K <= 0) return PK_ERR_ARG;
+  const int64_t gate = pk_gate_workspace_bytes(T, H, E), sort = pk_sort_workspace_bytes(T * K, E);
+  return gate > sort ? gate : sort;
+}
+
+int pk_gate_route_sort(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, int64_t T, int64_t H, int64_t E,
+                       int64_t K, int route_norm, float route_scale, float* logits, float* top_scores, int32_t* top_idx,
+                       int32_t* counts, int32_t* starts, int32_t* perm, int32_t* inv_perm, int32_t* order, void* workspace,
+                       int64_t workspace_bytes, pk_stream_t stream) {
+  if (T < 0 || K <= 0 || E <= 0) return PK_ERR_ARG;
+  if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E || T > 0x7fffffffll / K) return PK_ERR_SHAPE;
+  if (!starts || !workspace || (T > 0 && (!top_scores || !top_idx || !perm))) return PK_ERR_ARG;
+  if (workspace_bytes < pk_gate_route_sort_workspace_bytes(T, H, E, K)) return PK_ERR_WORKSPACE;
+  if (T == 0 || T > kRouteSortTokens || T * K > kRouteSortSlots || E > kSmallSortExperts) {
+    const int rc = pk_gate_route(x, x_dtype, w_gate, gate_bias, T, H, E, K, route_norm, route_scale, logits, top_scores, top_idx, workspace,
+                                 workspace_bytes, stream);
+    if (rc != PK_OK) return rc;
+    return pk_sort_by_expert(top_idx, T * K, E, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
   }
+  hipStream_t s = (hipStream_t)stream;
+  int splits = 1;
+  const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, s, &splits);
+  if (rc != PK_OK) return rc;
+  const GatePartials gp{splits > 1 ? reinterpret_cast<const float*>(workspace) : nullptr, gate_bias, splits};
+  const SortOut out{counts, starts, perm, inv_perm, order};
+  const dim3 grid(1), block(64 * kSmallSortWaves);
+#define PK_LAUNCH_ROUTE_SORT(EPL)                                                                                                   \
+  do {                                                                                                                              \
+    if (splits > 1)                                                                                                                 \
+      PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK, s, (route_sort_small_kernel<EPL, true>), grid, block, 0, s, gp, logits, (int)T, (int)E, (int)K,  \
+                        route_norm, route_scale, top_scores, top_idx, out);                                                         \
+    else                                                                                                                            \
+      PK_LAUNCH_NOCHECK(pk_timing::K_ROUTE_TOPK, s, (route_sort_small_kernel<EPL, false>), grid, block, 0, s, gp, logits, (int)T, (int)E, (int)K, \
+                        route_norm, route_scale, top_scores, top_idx, out);                                                         \
+  } while (0)
+  PK_DISPATCH_EPL(E, PK_LAUNCH_ROUTE_SORT);
+#undef PK_LAUNCH_ROUTE_SORT
+  PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
 

@@ -183,3 +183,66 @@ def test_sort_expert_order_hint(dev):
     c = counts.cpu().tolist()
     expect = sorted(range(24), key=lambda e: (-c[e], e))
     assert order.cpu().tolist() == expect and c[7] == 0 and expect[0] == 3
+
+
+@pytest.mark.parametrize("A,E", [(1, 1), (63, 512), (1024, 128), (4096, 100), (4096, 513), (4097, 128), (8704, 7), (20000, 1000)])
+def test_counting_sort_on_both_sides_of_its_dispatch(dev, A, E):
+    """One workgroup (up to 4,096 slots and 512 experts) and histogram + scatter beyond: every table
+    bit for bit."""
+    print(f"[case] sort A={A} E={E}", flush=True)
+    g = torch.Generator().manual_seed(A + E)
+    ids = torch.randint(0, E, (A, 1), generator=g, dtype=torch.int32)
+    counts, starts, perm, inv, order = ops.sort_by_expert(ids.to(dev), E, with_order=True)
+    flat = ids.reshape(-1).long()
+    want = torch.argsort(flat, stable=True)
+    ref_counts = torch.bincount(flat, minlength=E)
+    assert torch.equal(perm.cpu().long(), want)
+    assert torch.equal(inv.cpu().long()[want], torch.arange(A))
+    assert torch.equal(counts.cpu().long(), ref_counts)
+    assert torch.equal(starts.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), ref_counts.cumsum(0)]))
+    assert torch.equal(order.cpu().long(), torch.argsort(-ref_counts, stable=True))
+
+
+@pytest.mark.parametrize("T,H,E,K,bias", [(1, 256, 8, 2, True), (65, 2048, 128, 8, False), (70, 520, 130, 5, True), (5000, 2048, 128, 8, True)])
+def test_gate_and_topk_in_one_call_match_the_two_calls(dev, T, H, E, K, bias):
+    """pk_gate_route sums the gate GEMM's split-K partial results inside the top-k kernel: logits,
+    scores and indices bit for bit those of pk_gate_logits followed by pk_route_topk."""
+    from piper_amd._lib import host
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).bfloat16().to(dev)
+    w = (torch.randn(E, H, generator=g) * 0.02).to(dev)
+    b = torch.randn(E, generator=g).to(dev) if bias else None
+    want_s, want_i = ops.route_topk(ops.gate_logits(x, w, b), K, True, 1.5)
+    got_s, got_i = host().router(x, w, b, K, True, 1.5, None)
+    assert torch.equal(got_i, want_i) and torch.equal(got_s, want_s)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,H,E,K", [(1, 8, 4, 2), (33, 136, 8, 3), (300, 2048, 128, 8), (65, 72, 6, 2), (40, 70, 12, 9)])
+def test_router_backward_in_one_call_matches_the_three_calls(dev, dtype, T, H, E, K):
+    """pk_region_router_bwd adds the gate's share of d_x where the routed rows are gathered: d_logits, d_x
+    and the gate's gradients bit for bit those of route_topk_bwd, gate_logits_bwd and permute_bwd, with
+    the score gradients given directly and as partial sums; widths that cannot be read in 16-byte
+    pieces take the separate kernels inside."""
+    from piper_amd import _lib
+    from piper_amd._lib import call, current_stream, dtype_code, ptr
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T, H, generator=g).to(dtype).to(dev)
+    w = (torch.randn(E, H, generator=g) * 0.02).to(dev)
+    logits = torch.randn(T, E, generator=g).to(dev)
+    rows = torch.randn(T * K, H, generator=g).to(dtype).to(dev)
+    part = torch.randn(3, T * K, generator=g).to(dev)
+    _, idx = ops.route_topk(logits, K, True)
+    _, _, perm, inv = ops.sort_by_expert(idx, E)
+    d_s = ((part[0] + part[1]) + part[2])[inv.long()].reshape(T, K)
+    d_logits = ops.route_topk_bwd(logits, idx, d_s, True, 1.5)
+    want_w, want_b = torch.empty_like(w), torch.empty(E, device=dev)
+    d_x32 = ops.gate_logits_bwd(d_logits, x, w, d_w_gate=want_w, d_gate_bias=want_b)
+    want_x = ops.permute_bwd(rows, inv, K, addend_f32=d_x32)
+    ws = torch.empty(int(_lib.load().pk_region_router_bwd_workspace_bytes(T, H, E, dtype_code(dtype))), dtype=torch.uint8, device=dev)
+    for partial in (False, True):
+        got_l, got_x, got_w, got_b = torch.empty_like(logits), torch.empty_like(x), torch.empty_like(w), torch.empty(E, device=dev)
+        call("pk_region_router_bwd", ptr(logits), ptr(idx), None if partial else ptr(d_s), ptr(part), 3, ptr(inv), 1, 1.5, ptr(x),
+             dtype_code(dtype), ptr(w), ptr(rows), ptr(got_x), ptr(got_w), ptr(got_b), 0, ptr(got_l), T, H, E, K, ptr(ws), ws.numel(),
+             current_stream(dev))
+        assert torch.equal(got_l, d_logits) and torch.equal(got_x, want_x) and torch.equal(got_w, want_w) and torch.equal(got_b, want_b)
