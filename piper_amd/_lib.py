@@ -7,6 +7,7 @@ driver (e.g. the assertions in src/runtime.py:313-328).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 from pathlib import Path
 
@@ -212,6 +213,15 @@ def current_stream(device: torch.device | None = None):
     exactly like the ATen ops they replace (src/executors.py:231-232)."""
     init_device()
     return torch.cuda.current_stream(device).cuda_stream
+
+
+_NO_STREAM = contextlib.nullcontext()
+
+
+def on_stream(stream):
+    """Context manager: `stream` is the current one inside (None: nothing changes), as
+    `torch.cuda.stream(stream)` without the Python in it."""
+    return _NO_STREAM if stream is None else host().StreamScope(stream.stream_id, stream.device_index, stream.device_type)
 
 
 def require_gpu(t: torch.Tensor) -> None:

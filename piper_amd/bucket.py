@@ -19,7 +19,7 @@ import logging
 import torch
 
 from . import ops
-from ._lib import host
+from ._lib import host, on_stream
 from .optim import FusedAdamW
 
 BUCKET_ALIGN_BYTES = 256
@@ -237,7 +237,7 @@ class ParamStorage:
 
     def zero_grad_buffers(self, stream: torch.cuda.Stream | None = None) -> None:
         """src/runtime.py:223-229."""
-        with torch.cuda.stream(stream):
+        with on_stream(stream):
             for bucket in self._all_states():
                 if bucket.flat_grads is not None:
                     ops.bucket_zero(bucket.flat_grads)
@@ -259,7 +259,7 @@ class ParamStorage:
         specs = bucket.param_view_specs
         if not specs:
             return
-        with torch.cuda.stream(stream):
+        with on_stream(stream):
             if bucket.flat_grads is None:
                 bucket.flat_grads = torch.zeros(bucket.param_shard_info[1], dtype=self.grad_buffer_dtype,
                                                 device=bucket.flat_params.device)
@@ -299,7 +299,7 @@ class ParamStorage:
     def alloc_full_grads(self, ubid, stream: torch.cuda.Stream | None = None) -> None:
         bucket = self.stages.bucket(ubid)
         self.wait_pending_free(self.pending_grad_frees, ubid)
-        with torch.cuda.stream(stream):
+        with on_stream(stream):
             if bucket.flat_grads is None:
                 bucket.flat_grads = torch.zeros(bucket.param_shard_info[1], dtype=self.grad_buffer_dtype,
                                                 device=bucket.flat_params.device)
@@ -329,7 +329,7 @@ class ParamStorage:
             if opt is None or bucket.reduce_scatter_grads is None:
                 continue
             held, bucket.pending_grads = bucket.pending_grads, None
-            with torch.cuda.stream(stream):
+            with on_stream(stream):
                 if held is not None and hasattr(opt, "step_packed") and len({g.dtype for g in held if g is not None}) <= 1:
                     specs = bucket.param_view_specs
                     opt.step_packed(bucket.shard_param, held, [s[1] for s in specs], [s[2] for s in specs],

@@ -2271,13 +2271,13 @@ int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map
 template <typename T>
 int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void* dg, const void* du, const void* x,
                const int32_t* row_map, int64_t div, const int32_t* starts, void* dw1, void* dw2, void* dw3, int acc,
-               int64_t H, int64_t I, int64_t E, hipStream_t s) {
+               int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedK p = {};
   p.starts = starts; p.E = (int32_t)E; p.map_div = (int32_t)div; p.accumulate = acc ? 1 : 0;
   if (dw2) p.prob[p.nprob++] = {dy, H, dy_map, h, I, nullptr, dw2, (int32_t)H, (int32_t)I};
   if (dw1) p.prob[p.nprob++] = {dg, I, nullptr, x, H, row_map, dw1, (int32_t)I, (int32_t)H};
   if (dw3) p.prob[p.nprob++] = {du, I, nullptr, x, H, row_map, dw3, (int32_t)I, (int32_t)H};
-  return pk_tile::launch_ragged_k<T>(p, mf::persistent_grid(), pk_timing::K_SWIGLU_WGRAD, s);
+  return pk_tile::launch_ragged_k<T>(p, A, mf::persistent_grid(), pk_timing::K_SWIGLU_WGRAD, s);
 }
 
 template <typename T>
@@ -2600,8 +2600,8 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3});
   if (!mfma && tile_gemm_ok(dtype, H, I, {d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}))
     return dtype == PK_F32
-               ? wgrad_tile<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s)
-               : wgrad_tile<bf16_t>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s);
+               ? wgrad_tile<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, A, H, I, E, s)
+               : wgrad_tile<bf16_t>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, A, H, I, E, s);
   if (dtype == PK_F32)
     return wgrad_simt<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, H, I, E, s);
   if (!mfma)

@@ -318,6 +318,28 @@ c10::hip::HIPStream side_stream(int dev) {
 c10::Stream as_cuda(const c10::hip::HIPStream& s) {
   return c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::CUDA, s.device_index()), s.id());
 }
+// `with torch.cuda.stream(s)` without its Python (about ten calls on the way in and out): makes a stream,
+// and its device, the current one.
+class StreamScope {
+ public:
+  StreamScope(int64_t id, int64_t device, int64_t) : stream_(c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::HIP, (c10::DeviceIndex)device), id)) {}
+  void enter() {
+    device_ = c10::hip::current_device();
+    if (device_ != stream_.device_index()) c10::hip::set_device(stream_.device_index());
+    before_ = c10::hip::getCurrentHIPStream(stream_.device_index());
+    c10::hip::setCurrentHIPStream(c10::hip::HIPStream(stream_));
+  }
+  void exit() {
+    c10::hip::setCurrentHIPStream(*before_);
+    if (device_ != stream_.device_index()) c10::hip::set_device(device_);
+  }
+
+ private:
+  c10::Stream stream_;
+  std::optional<c10::hip::HIPStream> before_;
+  c10::DeviceIndex device_ = 0;
+};
+
 // `waiter` waits for everything queued on `other` so far
 void wait_stream(hipStream_t waiter, hipStream_t other) {
   hipEvent_t e;
@@ -878,6 +900,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     adamw_packed(master, exp_avg, exp_avg_sq, opt(flat_grad), grads, offsets, numels, step, lr, beta1, beta2, eps, weight_decay, opt(shadow),
                  grad_scale, zero_grad);
   });
+  py::class_<StreamScope>(m, "StreamScope")
+      .def(py::init<int64_t, int64_t, int64_t>())
+      .def("__enter__", &StreamScope::enter)
+      .def("__exit__", [](StreamScope& s, const py::args&) { s.exit(); });
+  // everything queued on `other` (a hipStream_t) so far happens before what `waiter` gets from now on
+  m.def("wait_stream", [](uintptr_t waiter, uintptr_t other) { wait_stream(reinterpret_cast<hipStream_t>(waiter), reinterpret_cast<hipStream_t>(other)); }, nogil);
   m.def("set_accumulate", [](bool on) { return g_accumulate.exchange(on); });
   m.def("set_overlap", [](bool on) { return g_overlap.exchange(on); });
   // the WeightGradQueue that backward passes hand their weight gradients to (None: they run them)

@@ -7,17 +7,17 @@
 //   ragged K: C[e][M, N] (+)= A[rows_e, M]^T . B[rows_e, N]           (weight gradient)
 //
 // One workgroup of four waves (2 x 2) per output tile of 64 x 64 or 128 x 128.  A k-tile is 128 bytes
-// of the reduction index of every operand row (32 fp32 or 64 bf16); the pieces of tile k+1 are fetched
-// into registers while tile k is multiplied out of LDS and then stored to the other LDS buffer: one
-// barrier per k-tile.  The operands pass through registers rather than straight into LDS because the
-// masking then costs one select per piece and nothing has to be counted by hand; at fp32, where a
-// k-tile of a 64 x 64 wave tile is 64 MFMAs of 64 cycles, the round trip to memory is covered entirely,
-// and with bf16 two (128 x 128) or five (64 x 64) workgroups share a CU.
+// of the reduction index of every operand row (32 fp32 or 64 bf16); two or three k-tiles are in flight in
+// registers (against one: -7 %) while another is multiplied out of LDS; two LDS buffers, one barrier per
+// k-tile.  The operands pass through registers rather than straight into LDS because the masking then
+// costs one select per piece and nothing has to be counted by hand.  Where the tiles are too few for
+// the chip, several groups of four waves share a tile's reduction.
 // Against one 64 x 64 FMA tile per workgroup (simt_gemm.h, which keeps the widths that are no multiple
 // of 16 bytes): see the figures at tile_gemm_ok in grouped_gemm.hip.
 #pragma once
 #include "pk_common.h"
 #include "unit_index.h"
+#include <type_traits>
 
 namespace pk_tile {
 
@@ -82,12 +82,22 @@ __device__ __forceinline__ Frag<T> frag_mn(const char* tile, int col0, int step,
 }
 // acc += b . a, operands swapped so that a lane holds 4 consecutive columns of one output row:
 //   acc[v] = C[row = lane % 32][col = 8 * (v / 4) + 4 * (lane / 32) + v % 4]
-__device__ __forceinline__ void mma(floatx16_t& acc, const Frag<bf16_t>& a, const Frag<bf16_t>& b) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.v, a.v, acc, 0, 0, 0);
-}
-__device__ __forceinline__ void mma(floatx16_t& acc, const Frag<float>& a, const Frag<float>& b) {
+// (fp32: the four MFMAs of a piece go round the tiles, so that neighbours do not share an accumulator)
+template <int TM, int TN>
+__device__ __forceinline__ void mma_tiles(floatx16_t (&acc)[TM][TN], const Frag<bf16_t> (&a)[TM], const Frag<bf16_t> (&b)[TN]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(b.v[j], a.v[j], acc, 0, 0, 0);
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j].v, a[i].v, acc[i][j], 0, 0, 0);
+}
+template <int TM, int TN>
+__device__ __forceinline__ void mma_tiles(floatx16_t (&acc)[TM][TN], const Frag<float> (&a)[TM], const Frag<float> (&b)[TN]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j].v[q], a[i].v[q], acc[i][j], 0, 0, 0);
 }
 
 template <typename T>
@@ -118,6 +128,43 @@ __device__ __forceinline__ void load4<bf16_t>(const bf16_t* p, float (&f)[4]) {
   for (int i = 0; i < 4; ++i) f[i] = (float)v[i];
 }
 
+// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
+// acc of group 0 += acc of the other groups, in group order (every thread of the workgroup calls it).
+template <int KS, int TILES>
+__device__ __forceinline__ void add_groups(floatx16_t* acc, float* lds, int group, int tid) {
+  __syncthreads();                         // the last k-tiles have been read
+  if (group > 0) {
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) lds[(((group - 1) * TILES + t) * 16 + v) * THREADS + tid] = acc[t][v];
+  }
+  __syncthreads();
+  if (group == 0) {
+#pragma unroll
+    for (int g = 1; g < KS; ++g)
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[t][v] += lds[(((g - 1) * TILES + t) * 16 + v) * THREADS + tid];
+  }
+}
+// Groups of four waves per output tile: few tiles leave most CUs idle and a long reduction on the
+// others, so it is split inside the workgroup (up to four ways, at least four k-tiles each).
+inline int reduction_groups(int64_t tiles, int64_t k_tiles, int cus) {
+  int ks = 1;
+  while (ks < 4 && tiles * ks * 2 <= 2 * (int64_t)cus && k_tiles >= ks * 2 * 2) ks *= 2;
+  return ks;
+}
+
 // ---------------------------------------------------------------------------------- ragged M
 struct RaggedM {
   const void* A0;           // A of k-segment 0, row-major [rows, lda]
@@ -137,26 +184,32 @@ struct RaggedM {
   int64_t ldc;
 };
 
-// Tile b of a launch.  Blocks b, b + 8, ... run on one XCD: four neighbouring tiles (which share
-// weights or rows) stay on it, the next four go to the next XCD.
+// Tile b of a launch.  Blocks b, b + 8, ... run on one XCD: CHUNK neighbouring tiles (which share
+// weights or rows) stay on it, the next ones go to the next XCD (16 against 4: -3 to -12 % where the
+// operands do not fit the L2 of an XCD; 32 leaves XCDs without work at small sizes).
+constexpr int CHUNK = 16;
 __device__ __forceinline__ int unit_of_block(int b) {
   const int x = b % NXCD, q = b / NXCD;
-  return ((q >> 2) * NXCD + x) * 4 + (q & 3);
+  return ((q / CHUNK) * NXCD + x) * CHUNK + (q % CHUNK);
 }
 
 // DUAL: two weight matrices (gate and up) against the same A rows, SiLU(g) * u in the epilogue.
-template <typename T, int TM, int TN, bool B_KC, bool DUAL>
-__global__ __launch_bounds__(THREADS) void ragged_m_kernel(const RaggedM p) {
+template <typename T, int TM, int TN, int DEPTH, int KS, bool B_KC, bool DUAL>
+__global__ __launch_bounds__(THREADS * KS) void ragged_m_kernel(const RaggedM p) {
   constexpr int BM = 64 * TM, BN = 64 * TN, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr int NB = DUAL ? 2 : 1;
   constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, STAGE = A_BYTES + NB * B_BYTES;
   static_assert(!DUAL || B_KC, "gate and up weights are K-contiguous");
-  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  static_assert((KS - 1) * NB * BM * BN * 4 <= KS * 2 * STAGE, "the partial sums reuse the k-tiles' LDS");
+  __shared__ __attribute__((aligned(16))) char smem_[KS * 2 * STAGE];
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  // KS groups of four waves take every KS-th k-tile each, in LDS of their own
+  const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / THREADS);
+  const int tid = threadIdx.x % THREADS, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
+  char* const smem = smem_ + group * 2 * STAGE;
   const pk_units::UnitIndex ui = pk_units::build_unit_index<BM>(p.starts, p.E, p.n_tiles);
   const int unit = unit_of_block(blockIdx.x);
   if (unit >= ui.total) return;
@@ -200,15 +253,17 @@ __global__ __launch_bounds__(THREADS) void ragged_m_kernel(const RaggedM p) {
   const int64_t seg_b = reinterpret_cast<const T*>(p.B1) - reinterpret_cast<const T*>(p.B0);
   const int kt_per_seg = (p.K + BK - 1) / BK, nkt = kt_per_seg * p.nseg;
 
-  u32x4_t ra[LA], rb[NB][LB];
-  auto fetch = [&](int kt) {
+  u32x4_t ra_[DEPTH][LA], rb_[DEPTH][NB][LB];
+  auto fetch = [&](auto d_c, int kt) {
+    auto& ra = ra_[decltype(d_c)::value];
+    auto& rb = rb_[decltype(d_c)::value];
     const bool second = kt >= kt_per_seg;
     const int k0 = (second ? kt - kt_per_seg : kt) * BK;
     const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
       ra[i] = zero;
-      if (a_ok[i] && k0 + a_kofs < p.K) ra[i] = *reinterpret_cast<const u32x4_t*>(a_ptr[i] + k0 + (second ? seg_a : 0));
+      if (a_ok[i] && kt < nkt && k0 + a_kofs < p.K) ra[i] = *reinterpret_cast<const u32x4_t*>(a_ptr[i] + k0 + (second ? seg_a : 0));
     }
 #pragma unroll
     for (int q = 0; q < NB; ++q)
@@ -216,11 +271,13 @@ __global__ __launch_bounds__(THREADS) void ragged_m_kernel(const RaggedM p) {
       for (int i = 0; i < LB; ++i) {
         rb[q][i] = zero;
         const int64_t k_at = B_KC ? (int64_t)k0 : (int64_t)k0 * p.ldb;
-        if (b_ok[i] && k0 + b_k[i] < p.K)
+        if (b_ok[i] && kt < nkt && k0 + b_k[i] < p.K)
           rb[q][i] = *reinterpret_cast<const u32x4_t*>(b_ptr[i] + k_at + (DUAL ? (q ? seg_b : 0) : (second ? seg_b : 0)));
       }
   };
-  auto deposit = [&](char* st) {
+  auto deposit = [&](auto d_c, char* st) {
+    auto& ra = ra_[decltype(d_c)::value];
+    auto& rb = rb_[decltype(d_c)::value];
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
       const int s = tid + i * THREADS, r = s >> 3, c = s & 7;
@@ -254,13 +311,14 @@ __global__ __launch_bounds__(THREADS) void ragged_m_kernel(const RaggedM p) {
         for (int v = 0; v < 16; ++v) acc[q][i][j][v] = 0.f;
 
   const bool wave_has_rows = wm * 32 * TM < rows;
-  fetch(0);
-  deposit(smem);
-  __syncthreads();
-  for (int kt = 0; kt < nkt; ++kt) {
-    const char* const st = smem + (kt & 1) * STAGE;
-    const bool more = kt + 1 < nkt;
-    if (more) fetch(kt + 1);
+  const int mine = (nkt + KS - 1) / KS;      // k-tiles of a group (past the last one: zeros)
+  // DEPTH of the group's k-tiles are in flight, each in a register set of its own
+  auto step = [&](auto d_c, int kt) {
+    constexpr int d = decltype(d_c)::value;
+    char* const st = smem + (kt & 1) * STAGE;
+    deposit(d_c, st);
+    __syncthreads();
+    if (kt + DEPTH < mine) fetch(std::integral_constant<int, d>{}, (kt + DEPTH) * KS + group);
     if (wave_has_rows) {
 #pragma unroll
       for (int step = 0; step < 4; ++step) {
@@ -276,17 +334,16 @@ __global__ __launch_bounds__(THREADS) void ragged_m_kernel(const RaggedM p) {
             else b[q][j] = frag_mn<T, BN>(t, (wn * TN + j) * 32, step, lane);
           }
 #pragma unroll
-        for (int q = 0; q < NB; ++q)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) mma(acc[q][i][j], a[i], b[q][j]);
+        for (int q = 0; q < NB; ++q) mma_tiles<TM, TN>(acc[q], a, b[q]);
       }
     }
-    if (more) {
-      deposit(smem + ((kt + 1) & 1) * STAGE);
-      __syncthreads();
-    }
+  };
+  static_for<DEPTH>([&](auto d) { if (d < mine) fetch(d, d * KS + group); });
+  for (int kt = 0; kt < mine; kt += DEPTH)
+    static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
+  if constexpr (KS > 1) {
+    add_groups<KS, NB * TM * TN>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
+    if (group > 0) return;
   }
 
 #pragma unroll
@@ -331,9 +388,14 @@ inline int launch_ragged_m(RaggedM p, int64_t A_rows, int cus, int kernel_id, hi
   p.n_tiles = (int32_t)pk_ceil_div(p.N, bm);
   const int64_t units = (pk_ceil_div(A_rows, bm) + p.E) * p.n_tiles;
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
-  const dim3 grid((unsigned)(pk_ceil_div(units, 4 * NXCD) * 4 * NXCD)), block(THREADS);
-  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 2, 2, B_KC, DUAL>), grid, block, 0, s, p);
-  else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, B_KC, DUAL>), grid, block, 0, s, p);
+  const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(THREADS);
+  // row tiles that hold rows, about: every expert's last one is half full
+  const int64_t tiles = (A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2) * p.n_tiles;
+  const int ks = large ? 1 : reduction_groups(tiles, pk_ceil_div(p.K, kBK<T>) * p.nseg, cus);
+  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 2, 2, 2, 1, B_KC, DUAL>), grid, block, 0, s, p);
+  else if (ks == 4) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, 2, DUAL ? 2 : 4, B_KC, DUAL>), grid, dim3(THREADS * (DUAL ? 2 : 4)), 0, s, p);
+  else if (ks == 2) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, 2, 2, B_KC, DUAL>), grid, dim3(THREADS * 2), 0, s, p);
+  else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, 3, 1, B_KC, DUAL>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
@@ -353,18 +415,20 @@ struct RaggedK {
   int32_t E, map_div, accumulate;
 };
 
-template <typename T, int TM, int TN>
-__global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
+template <typename T, int TM, int TN, int DEPTH, int KS>
+__global__ __launch_bounds__(THREADS * KS) void ragged_k_kernel(const RaggedK p) {
   constexpr int BM = 64 * TM, BN = 64 * TN, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
   constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
   using MA = Mn<T, BM>;
   using MB = Mn<T, BN>;
-  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) char smem_[KS * 2 * STAGE];
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / THREADS);      // as in ragged_m_kernel
+  const int tid = threadIdx.x % THREADS, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
+  char* const smem = smem_ + group * 2 * STAGE;
   const int per_expert = p.first[p.nprob];
   const int unit = unit_of_block(blockIdx.x);
   if (unit >= p.E * per_expert) return;
@@ -376,7 +440,7 @@ __global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
   const int n_tiles = (q.N + BN - 1) / BN;
   const int m0 = t / n_tiles * BM, n0 = t % n_tiles * BN;
   const int row0 = p.starts[e], rows = p.starts[e + 1] - row0;
-  const int nkt = (rows + BK - 1) / BK;
+  const int nkt = (rows + BK - 1) / BK, mine = (nkt + KS - 1) / KS;
 
   int a_k[LA], b_k[LB], a_col[LA], b_col[LB];
 #pragma unroll
@@ -408,8 +472,10 @@ __global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
       if (k < rows && b_col[i] < q.N) b_row[i] = q.b_map ? q.b_map[row0 + k] / p.map_div : row0 + k;
     }
   };
-  u32x4_t ra[LA], rb[LB];
-  auto fetch = [&]() {
+  u32x4_t ra_[DEPTH][LA], rb_[DEPTH][LB];
+  auto fetch = [&](auto d_c) {
+    auto& ra = ra_[decltype(d_c)::value];
+    auto& rb = rb_[decltype(d_c)::value];
     const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
@@ -422,7 +488,9 @@ __global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
       if (b_row[i] >= 0) rb[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const T*>(q.B) + (int64_t)b_row[i] * q.ldb + b_col[i]);
     }
   };
-  auto deposit = [&](char* st) {
+  auto deposit = [&](auto d_c, char* st) {
+    auto& ra = ra_[decltype(d_c)::value];
+    auto& rb = rb_[decltype(d_c)::value];
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
       const int s = tid + i * THREADS, c = s % MA::CPR;
@@ -444,17 +512,20 @@ __global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
   if (nkt > 0) {
-    lookup(0);
-    fetch();
-    lookup(1);
-    deposit(smem);
-    __syncthreads();
-    for (int kt = 0; kt < nkt; ++kt) {
-      const char* const st = smem + (kt & 1) * STAGE;
-      const bool more = kt + 1 < nkt;
-      if (more) {
-        fetch();
-        lookup(kt + 2);
+    lookup(group);
+    static_for<DEPTH>([&](auto d) {
+      if (d < mine) {
+        fetch(d);
+        lookup((d + 1) * KS + group);
+      }
+    });
+    auto step = [&](auto d_c, int kt) {
+      char* const st = smem + (kt & 1) * STAGE;
+      deposit(d_c, st);
+      __syncthreads();
+      if (kt + DEPTH < mine) {
+        fetch(d_c);
+        lookup((kt + DEPTH + 1) * KS + group);
       }
 #pragma unroll
       for (int step = 0; step < 4; ++step) {
@@ -463,17 +534,16 @@ __global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
         for (int i = 0; i < TM; ++i) a[i] = frag_mn<T, BM>(st, (wm * TM + i) * 32, step, lane);
 #pragma unroll
         for (int j = 0; j < TN; ++j) b[j] = frag_mn<T, BN>(st + A_BYTES, (wn * TN + j) * 32, step, lane);
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) mma(acc[i][j], a[i], b[j]);
+        mma_tiles<TM, TN>(acc, a, b);
       }
-      if (more) {
-        deposit(smem + ((kt + 1) & 1) * STAGE);
-        __syncthreads();
-      }
+    };
+    for (int kt = 0; kt < mine; kt += DEPTH)
+      static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
+    if constexpr (KS > 1) {
+      add_groups<KS, TM * TN>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
+      if (group > 0) return;
     }
-  } else if (p.accumulate) {
+  } else if (p.accumulate || group > 0) {
     return;                       // an expert without rows adds nothing
   }
 
@@ -504,7 +574,7 @@ __global__ __launch_bounds__(THREADS) void ragged_k_kernel(const RaggedK p) {
 }
 
 template <typename T>
-inline int launch_ragged_k(RaggedK p, int cus, int kernel_id, hipStream_t s) {
+inline int launch_ragged_k(RaggedK p, int64_t A_rows, int cus, int kernel_id, hipStream_t s) {
   auto plan = [&](int bm) {
     int64_t tiles = 0;
     for (int q = 0; q < p.nprob; ++q) {
@@ -519,9 +589,12 @@ inline int launch_ragged_k(RaggedK p, int cus, int kernel_id, hipStream_t s) {
   if (!large) units = plan(64);
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
   if (units == 0) return PK_OK;
-  const dim3 grid((unsigned)(pk_ceil_div(units, 4 * NXCD) * 4 * NXCD)), block(THREADS);
-  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 2, 2>), grid, block, 0, s, p);
-  else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1>), grid, block, 0, s, p);
+  const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(THREADS);
+  const int ks = large ? 1 : reduction_groups(units, pk_ceil_div(pk_ceil_div(A_rows, p.E), kBK<T>), cus);
+  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 2, 2, 1, 1>), grid, block, 0, s, p);
+  else if (ks == 4) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 4>), grid, dim3(THREADS * 4), 0, s, p);
+  else if (ks == 2) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 2>), grid, dim3(THREADS * 2), 0, s, p);
+  else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 3, 1>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }

@@ -16,6 +16,7 @@ from typing import Any, Sequence
 import torch
 
 from . import functional as F_
+from ._lib import host, on_stream
 from .bucket import ParamStorage, StageStore
 from .planner import plan_zero_lifetimes
 from .tasks import COMM_TASKS, TaskType
@@ -60,7 +61,7 @@ class ComputeExecutor:
             args[slot] = leaf
         fwd_inputs = [args[slot] for slot in slots]
         try:
-            with torch.cuda.stream(compute_stream):
+            with on_stream(compute_stream):
                 result = bucket.forward_fn(args)
         finally:
             for slot in slots:            # activations must not stay alive inside the argument list
@@ -96,7 +97,7 @@ class ComputeExecutor:
                                      "bucket received a gradient from its consumer")
         # the backward accumulates into .grad; the HIP operators add to gradients that exist
         # already (later microbatches of an iteration) inside their kernels
-        with torch.cuda.stream(compute_stream), F_.accumulate_weight_grads():
+        with on_stream(compute_stream), F_.accumulate_weight_grads():
             torch.autograd.backward(roots, grads)
         received = [t.grad for t in (inp_with_grad or ()) if t.grad is not None]
         return {"send_output": received} if received else None
@@ -151,9 +152,9 @@ class StageExecutor:
         ps = self.pack_stream or cs
         # the microbatches (and whatever else the caller queued) were produced on the caller's stream
         if cs != caller:
-            cs.wait_stream(caller)
+            host().wait_stream(cs.cuda_stream, caller.cuda_stream)
         if ps != caller and ps is not cs:
-            ps.wait_stream(caller)
+            host().wait_stream(ps.cuda_stream, caller.cuda_stream)
         self.params.drain_pending_frees()        # src/executors.py:584
         self._fwd.clear()
         self._inp_grads.clear()
@@ -163,7 +164,7 @@ class StageExecutor:
         self.params.clear_param_grads()
         self.params.zero_grad_buffers(ps)
         if ps is not cs:
-            cs.wait_stream(ps)
+            host().wait_stream(cs.cuda_stream, ps.cuda_stream)
         ubids = list(self.stages.buckets.keys())
         # which task gathers / frees a bucket's parameters and which one packs its gradients
         lifetimes = plan_zero_lifetimes(tasks)
@@ -200,7 +201,7 @@ class StageExecutor:
                 queue = ctx.__enter__() if split else None
                 try:
                     if pos == len(ubids) - 1:
-                        with torch.cuda.stream(cs):
+                        with on_stream(cs):
                             out = rec["pre_detach_outs"][0]
                             if self.loss_fn is not None:
                                 loss = self.loss_fn(out, None if targets is None else targets[task.mb])
@@ -231,7 +232,7 @@ class StageExecutor:
                     self._free_params_after(task.ubid, cs)
             elif tt is TaskType.BWD_W:
                 queue = self._wgrad_queues.pop((task.ubid, task.mb))
-                with torch.cuda.stream(cs):
+                with on_stream(cs):
                     queue.run()
                 if life.reduce_grads_after:
                     self._pack_after_backward(task.ubid, cs, ps, pack_events, hold=last_pack.get(task.ubid) == ti)
@@ -260,9 +261,7 @@ class StageExecutor:
             self.params.hold_param_grads(ubid, cs)
             return
         if ps is not cs:
-            evt = torch.cuda.Event()
-            evt.record(cs)
-            ps.wait_event(evt)
+            host().wait_stream(ps.cuda_stream, cs.cuda_stream)
         self.params.accumulate_zero_param_grads_to_flat(ubid, ps)
         if ps is not cs:
             done = torch.cuda.Event()
@@ -278,6 +277,6 @@ class StageExecutor:
             self.params.step_zero_shard_optimizers(stream, pack_events)
         for bucket in self.stages.buckets.values():
             if bucket.optimizer is not None:
-                with torch.cuda.stream(stream):
+                with on_stream(stream):
                     bucket.optimizer.step()
         torch.cuda.synchronize()
