@@ -21,7 +21,6 @@
 
 namespace pk_tile {
 
-constexpr int THREADS = 256;
 constexpr int NXCD = 8;
 
 typedef short shortx4_t __attribute__((ext_vector_type(4)));
@@ -39,7 +38,7 @@ struct Mn {
   __device__ static __forceinline__ int swz(int k) {
     // the transposing read of bf16 takes four k-rows at once: spread them over the banks
     if (sizeof(T) == 4) return 0;
-    return CPR >= 16 ? (k & 3) << 2 : (k & 1) << 2;
+    return CPR >= 16 ? (k & 3) << 2 : CPR >= 8 ? (k & 1) << 2 : 0;
   }
 };
 __device__ __forceinline__ int kc_swz(int r) { return (r >> 1) & 7; }
@@ -138,7 +137,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // acc of group 0 += acc of the other groups, in group order (every thread of the workgroup calls it).
-template <int KS, int TILES>
+template <int KS, int TILES, int THREADS>
 __device__ __forceinline__ void add_groups(floatx16_t* acc, float* lds, int group, int tid) {
   __syncthreads();                         // the last k-tiles have been read
   if (group > 0) {
@@ -194,9 +193,10 @@ __device__ __forceinline__ int unit_of_block(int b) {
 }
 
 // DUAL: two weight matrices (gate and up) against the same A rows, SiLU(g) * u in the epilogue.
-template <typename T, int TM, int TN, int DEPTH, int KS, bool B_KC, bool DUAL>
-__global__ __launch_bounds__(THREADS * KS) void ragged_m_kernel(const RaggedM p) {
-  constexpr int BM = 64 * TM, BN = 64 * TN, BK = kBK<T>, PIECE = kPiece<T>;
+template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, bool DUAL>
+__global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const RaggedM p) {
+  constexpr int THREADS = 64 * WM * WN;       // of a group: WM x WN waves of TM x TN MFMA tiles
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr int NB = DUAL ? 2 : 1;
   constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, STAGE = A_BYTES + NB * B_BYTES;
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(THREADS * KS) void ragged_m_kernel(const RaggedM p)
   const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / THREADS);
   const int tid = threadIdx.x % THREADS, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
   char* const smem = smem_ + group * 2 * STAGE;
   const pk_units::UnitIndex ui = pk_units::build_unit_index<BM>(p.starts, p.E, p.n_tiles);
   const int unit = unit_of_block(blockIdx.x);
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(THREADS * KS) void ragged_m_kernel(const RaggedM p)
   for (int kt = 0; kt < mine; kt += DEPTH)
     static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
   if constexpr (KS > 1) {
-    add_groups<KS, NB * TM * TN>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
+    add_groups<KS, NB * TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
     if (group > 0) return;
   }
 
@@ -378,26 +378,36 @@ __global__ __launch_bounds__(THREADS * KS) void ragged_m_kernel(const RaggedM p)
   }
 }
 
+template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, bool DUAL>
+inline int launch_tiles(RaggedM p, int64_t A_rows, int kernel_id, hipStream_t s) {
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
+  p.n_tiles = (int32_t)pk_ceil_div(p.N, BN);
+  const int64_t units = (pk_ceil_div(A_rows, BM) + p.E) * p.n_tiles;
+  if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
+  const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(64 * WM * WN * KS);
+  PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, DEPTH, KS, B_KC, DUAL>), grid, block, 0, s, p);
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
 template <typename T, bool B_KC, bool DUAL>
-inline int launch_ragged_m(RaggedM p, int64_t A_rows, int cus, int kernel_id, hipStream_t s) {
+inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int kernel_id, hipStream_t s) {
   // 128 x 128 tiles once they give every CU work for two rounds; below that the chip is filled by
   // four times as many 64 x 64 tiles
   const int64_t big = (A_rows / 128 + (p.E + 1) / 2) * pk_ceil_div(p.N, 128);
-  const bool large = big >= 2 * (int64_t)cus;
-  const int64_t bm = large ? 128 : 64;
-  p.n_tiles = (int32_t)pk_ceil_div(p.N, bm);
-  const int64_t units = (pk_ceil_div(A_rows, bm) + p.E) * p.n_tiles;
-  if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
-  const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(THREADS);
+  if (big >= 2 * (int64_t)cus) return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, DUAL>(p, A_rows, kernel_id, s);
   // row tiles that hold rows, about: every expert's last one is half full
-  const int64_t tiles = (A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2) * p.n_tiles;
-  const int ks = large ? 1 : reduction_groups(tiles, pk_ceil_div(p.K, kBK<T>) * p.nseg, cus);
-  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 2, 2, 2, 1, B_KC, DUAL>), grid, block, 0, s, p);
-  else if (ks == 4) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, 2, DUAL ? 2 : 4, B_KC, DUAL>), grid, dim3(THREADS * (DUAL ? 2 : 4)), 0, s, p);
-  else if (ks == 2) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, 2, 2, B_KC, DUAL>), grid, dim3(THREADS * 2), 0, s, p);
-  else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, 1, 1, 3, 1, B_KC, DUAL>), grid, block, 0, s, p);
-  PK_RETURN_IF_LAUNCH_FAILED();
-  return PK_OK;
+  const int64_t row_tiles = A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2;
+  const int64_t tiles = row_tiles * pk_ceil_div(p.N, 64), k_tiles = pk_ceil_div(p.K, kBK<T>) * p.nseg;
+  // an fp32 tile is 1,024 cycles of the matrix cores per k-tile, whoever shares it: 64 x 32 tiles while
+  // even those do not outnumber the CUs (200 to 512 rows, 256 x 512: -20 %)
+  if (sizeof(T) == 4 && 2 * tiles <= cus) {
+    if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, DUAL>(p, A_rows, kernel_id, s);
+    return launch_tiles<T, 2, 1, 1, 1, 2, 1, B_KC, DUAL>(p, A_rows, kernel_id, s);
+  }
+  const int ks = reduction_groups(tiles, k_tiles, cus);
+  if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, DUAL ? 2 : 4, B_KC, DUAL>(p, A_rows, kernel_id, s);
+  if (ks == 2) return launch_tiles<T, 2, 2, 1, 1, 2, 2, B_KC, DUAL>(p, A_rows, kernel_id, s);
+  return launch_tiles<T, 2, 2, 1, 1, 3, 1, B_KC, DUAL>(p, A_rows, kernel_id, s);
 }
 
 // ---------------------------------------------------------------------------------- ragged K
@@ -416,7 +426,8 @@ struct RaggedK {
 };
 
 template <typename T, int TM, int TN, int DEPTH, int KS>
-__global__ __launch_bounds__(THREADS * KS) void ragged_k_kernel(const RaggedK p) {
+__global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
+  constexpr int THREADS = 256;
   constexpr int BM = 64 * TM, BN = 64 * TN, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
   constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
@@ -540,7 +551,7 @@ __global__ __launch_bounds__(THREADS * KS) void ragged_k_kernel(const RaggedK p)
     for (int kt = 0; kt < mine; kt += DEPTH)
       static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
     if constexpr (KS > 1) {
-      add_groups<KS, TM * TN>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
+      add_groups<KS, TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
       if (group > 0) return;
     }
   } else if (p.accumulate || group > 0) {
@@ -589,11 +600,11 @@ inline int launch_ragged_k(RaggedK p, int64_t A_rows, int cus, int kernel_id, hi
   if (!large) units = plan(64);
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
   if (units == 0) return PK_OK;
-  const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(THREADS);
+  const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(256);
   const int ks = large ? 1 : reduction_groups(units, pk_ceil_div(pk_ceil_div(A_rows, p.E), kBK<T>), cus);
   if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 2, 2, 1, 1>), grid, block, 0, s, p);
-  else if (ks == 4) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 4>), grid, dim3(THREADS * 4), 0, s, p);
-  else if (ks == 2) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 2>), grid, dim3(THREADS * 2), 0, s, p);
+  else if (ks == 4) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 4>), grid, dim3(256 * 4), 0, s, p);
+  else if (ks == 2) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 2>), grid, dim3(256 * 2), 0, s, p);
   else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 3, 1>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
