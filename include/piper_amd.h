@@ -346,6 +346,21 @@ PK_API int pk_grouped_swiglu_dgrad_dh_scaled_t(const void* d_out, const int32_t*
                                         void* d_gT, void* d_uT, void* hsT, int64_t ldt, float* d_scores,
                                         void* workspace, int64_t workspace_bytes, int64_t A, int64_t H,
                                         int64_t I, int64_t E, int dtype, pk_stream_t stream);
+/* pk_grouped_swiglu_dgrad_dh_scaled as a region's backward calls it: tiles by size, and the score gradient
+ * either in d_scores (*n_partial = 0) or left in the workspace as *n_partial rows of A partial sums, for
+ * pk_region_router_bwd.  n_partial is written before the call returns. */
+PK_API int64_t pk_region_dgrad_dh_workspace_bytes(int64_t A, int64_t I);
+PK_API int pk_region_dgrad_dh(const void* d_out, const int32_t* row_map, int64_t row_map_div, const float* scores,
+                       const void* w2, const void* g, const void* u, const int32_t* starts, void* d_g, void* d_u,
+                       void* hs, float* d_scores, int64_t* n_partial, void* workspace, int64_t workspace_bytes,
+                       int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream);
+/* pk_grouped_swiglu_dgrad_dx with the tiles chosen by size. */
+PK_API int pk_region_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3,
+                       const int32_t* starts, void* d_x_sorted, int64_t A, int64_t H, int64_t I, int64_t E,
+                       int dtype, pk_stream_t stream);
+/* HOST, tuning hint: 1 when the backward of a region is faster through the transposed copies (0 also where
+ * pk_grouped_swiglu_transposed_ld says there are none). */
+PK_API int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dtype);
 /* HOST, tuning hint: 1 when leaving out the row-major d_g / d_u and running
  * pk_grouped_swiglu_dgrad_dx_t is the faster pair for this shape (long experts), 0 when the
  * row-major pair is (or the shape has no transposed path). */

@@ -2147,8 +2147,6 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_RM_SHORT 128, 256, 64, 2, 4, 3
 #define PK_RM_LOWM_UNITS 3
 #define PK_RM_SHORT_ROWS 512
-// Output widths that are a multiple of 128 but not of 256.
-#define PK_RM_ALT 128, 128, 64, 2, 2, 4
 // Weight gradient of the piecewise entry points (wgrad_kernel; the fused region runs
 // wgrad_pp_kernel, whose tile is fixed): 256x256x64 in a 2-stage ring; with fewer than
 // PK_WG_SHORTK_ROWS rows per expert on average 32-deep tiles in a 4-stage ring with the loads spread
@@ -2157,35 +2155,64 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_WG_BIG_THREADS 512
 #define PK_WG_BIG_SHORTK 256, 256, 32, 2, 4, 4
 #define PK_WG_SHORTK_ROWS 512
-#define PK_WG_SMALL 128, 128, 64, 2, 2, 4
-#define PK_WG_SMALL_THREADS 256
 
 bool mfma_shape_ok(int64_t H, int64_t I) { return H % 128 == 0 && I % 128 == 0; }
 
-// Pick the tile width by the output width N of the GEMM (for the gate/up kernel a tile holds
-// BN/2 gate and BN/2 up columns).
+// SwiGLU backward of intermediate sizes that are a multiple of 128 but not of 256.  The other products of
+// such widths run on the tiles of tile_gemm.h (24,000 rows of 24 experts, 640 x 896, us, these tiles -> those:
+// down 63 -> 55, weight gradients 375 -> 197, d_x equal, but d_h 97 -> 107: its epilogue moves six arrays in rows of a
+// tile, which this kernel stages through LDS).
+#define PK_RM_ALT 128, 128, 64, 2, 2, 4
+
+// 256 output columns per unit (for the gate/up kernel 128 gate and 128 up columns).
 template <bool B_KC, int EPI, bool A_T = false>
 int launch_rm(mf::RaggedMParams& p, int64_t A, int64_t N, int kernel_id, hipStream_t s) {
-  const int64_t per_tile_big = (EPI == mf::EPI_SWIGLU) ? PK_RM_BN / 2 : PK_RM_BN;
-  if (N % per_tile_big == 0) {
-    p.n_tiles = (int32_t)(N / per_tile_big);
-    // 256-row tiles unless they would leave the persistent grid with only a few units per
-    // workgroup (then the last round of units runs on a half-empty chip)
-    const int64_t big_units = (A / 256 + p.E / 2) * p.n_tiles;
-    const bool lowm = big_units < (int64_t)PK_RM_LOWM_UNITS * mf::persistent_grid();
-    // the scaled SwiGLU backward stays on 128-row units: its time goes into the epilogue (loads of g
-    // and u, the arithmetic, six stores per value), which 256-row units do not shorten, and with
-    // 128 accumulator registers that epilogue spills (measured 14 % slower at 16,384 tokens even
-    // with the packed outputs staged 32 columns at a time)
-    if (EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)PK_RM_SHORT_ROWS * p.E)
-      return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
-    if constexpr (EPI != mf::EPI_SWIGLU_BWD_SCALED) return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  const int64_t per_tile = (EPI == mf::EPI_SWIGLU) ? PK_RM_BN / 2 : PK_RM_BN;
+  if constexpr (EPI == mf::EPI_SWIGLU_BWD || EPI == mf::EPI_SWIGLU_BWD_SCALED) {
+    if (N % 256 != 0) {
+      p.n_tiles = (int32_t)(N / 128);
+      return mf::launch_ragged_m<PK_RM_ALT, B_KC, EPI>(p, A, kernel_id, s);
+    }
   }
-  if constexpr (A_T) return PK_ERR_SHAPE;      // the transposed copies exist for widths that are multiples of 256 only
-  const int64_t per_tile_alt = (EPI == mf::EPI_SWIGLU) ? 64 : 128;
-  p.n_tiles = (int32_t)(N / per_tile_alt);
-  return mf::launch_ragged_m<PK_RM_ALT, B_KC, EPI>(p, A, kernel_id, s);
+  if (N % per_tile != 0) return PK_ERR_SHAPE;
+  p.n_tiles = (int32_t)(N / per_tile);
+  // 256-row tiles unless they would leave the persistent grid with only a few units per
+  // workgroup (then the last round of units runs on a half-empty chip)
+  const int64_t big_units = (A / 256 + p.E / 2) * p.n_tiles;
+  const bool lowm = big_units < (int64_t)PK_RM_LOWM_UNITS * mf::persistent_grid();
+  // the scaled SwiGLU backward stays on 128-row units: its time goes into the epilogue (loads of g
+  // and u, the arithmetic, six stores per value), which 256-row units do not shorten, and with
+  // 128 accumulator registers that epilogue spills (measured 14 % slower at 16,384 tokens even
+  // with the packed outputs staged 32 columns at a time)
+  if (EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)PK_RM_SHORT_ROWS * p.E)
+    return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  if constexpr (EPI != mf::EPI_SWIGLU_BWD_SCALED) return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  return PK_ERR_SHAPE;
 }
+
+// Whether a bf16 product with N output columns (gate and up: 2 I) goes to the persistent kernels: their
+// 128 x 256 units have to outnumber the CUs, by a quarter where the epilogue is short.  Below, a CU
+// has one unit and its whole reduction to itself and the tiles of tile_gemm.h, four to eight times as
+// many and with a split reduction, are done first.  Forward and backward of a region, all its grouped products,
+// us, these kernels -> those (rows an expert, widths, experts; units of d_h against 256 CUs):
+//     32 rows, 1024 x 512, 32 experts ( 48 units)  161 ->  94      128 rows (96 units)   204 -> 147
+//    256 rows                         (160 units)  256 -> 223      512 rows (288 units)  both at 353
+//   1024 rows, 1024 x 512,  8 experts (136 units)  315 -> 218     2048 rows, 2048 x 1024, 4 experts (264 units): d_h 86 -> 107
+bool wide_fills(int64_t A, int64_t N, int64_t E, int quarters) {
+  return (A / 128 + (A < E ? A : E) / 2) * pk_ceil_div(N, 256) * 4 > quarters * (int64_t)mf::persistent_grid();
+}
+bool wide_gate_up(int64_t A, int64_t I, int64_t E) { return wide_fills(A, 2 * I, E, 5); }
+bool wide_dh(int64_t A, int64_t I, int64_t E) { return wide_fills(A, I, E, 4); }
+// With few rows an expert the last 128-row unit of an expert is mostly padding as often as not, and 64-row tiles
+// are the faster ones at several units per CU: up to 512 rows with a short reduction (512 rows, 1024 x 512,
+// 32 experts: 53 -> 49; 256 rows, 512 x 256, 128 experts: 46 -> 36; 1,024 rows: 70 -> 77), up to 64 with any
+// (128 experts, 2048 x 768: 19 rows 101 -> 86, 32 rows 105 -> 90, 64 rows 111 -> 102, 111 rows 122 -> 122).
+bool wide_down(int64_t A, int64_t H, int64_t I, int64_t E) {
+  const bool short_rows = A <= (I <= 512 ? 512 : 64) * E;
+  return H % 256 == 0 && wide_fills(A, H, E, short_rows ? 16 : 5);
+}
+// the same for a reduction of a few k-tiles (256 rows, 512 x 256, 128 experts: 58 -> 50)
+bool wide_dx(int64_t A, int64_t H, int64_t I, int64_t E) { return H % 256 == 0 && wide_fills(A, H, E, I < 512 ? 12 : 4); }
 
 bool all_aligned16(std::initializer_list<const void*> ptrs) {
   for (const void* p : ptrs)
@@ -2213,15 +2240,14 @@ bool tile_gemm_ok(int dtype, int64_t H, int64_t I, std::initializer_list<const v
 // Expected rows of an expert that has any, if they are few enough for the weight-streaming forward
 // kernels of skinny_gemm.h; 0 otherwise.  Measured (gate/up + down, us, wide tiles -> streaming):
 //   128 experts 2048 x 768:  1 token 62 -> 20, 24 tokens 211 -> 172, 8 rows each 262 -> 257, 12 rows 266 -> 281
-//   32 experts 1024 x 512:   1 row each 48 -> 14, 16 rows 53 -> 28, 48 rows 61 -> 55, 64 rows 65 -> 69
-//   8 experts 4096 x 1536:   1 row each 137 -> 43, 48 rows 167 -> 142, 64 rows 176 -> 184
+//   32 experts 1024 x 512 (tiles of tile_gemm.h -> streaming): 32 rows 30 -> 52;  64 experts 1536 x 384, 48 rows 79 -> 117
 //   24 experts 1000 x 360 (against the tiles of tile_gemm.h): 21 rows each 29 -> 21, 32 rows 29 -> 31
-// Where the wide tiles have a unit for every CU they hold their own from about 8 rows per expert on;
-// where they leave CUs idle, only from about 50, and the smaller tiles of tile_gemm.h from about 24.
-int64_t skinny_rows(int64_t A, int64_t I, int64_t E, bool wide) {
+// Where the wide tiles have a unit for every CU they hold their own from about 8 rows per expert on, the
+// smaller tiles of tile_gemm.h elsewhere from about 24.
+int64_t skinny_rows(int64_t A, int64_t I, int64_t E) {
   const int64_t touched = A < E ? A : E, rows = pk_ceil_div(A, touched);
   const bool fills = touched * pk_ceil_div(I, 128) >= mf::persistent_grid();
-  return rows <= (fills ? 8 : wide ? 48 : 24) ? rows : 0;
+  return rows <= (fills ? 8 : 24) ? rows : 0;
 }
 int fwd_skinny(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2, const void* w3, const int32_t* starts,
                void* g, void* u, void* h, void* y, int64_t A, int64_t H, int64_t I, int64_t E, int64_t rows, hipStream_t s) {
@@ -2241,21 +2267,23 @@ int fwd_skinny(const void* x, const int32_t* row_map, int64_t div, const void* w
 }
 
 template <typename T>
-int fwd_tile(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2, const void* w3,
-             const int32_t* starts, void* g, void* u, void* h, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
+int gate_up_tile(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w3, const int32_t* starts,
+                 void* g, void* u, void* h, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedM p = {};
   p.A0 = p.A1 = x; p.lda = H; p.row_map = row_map; p.map_div = (int32_t)div;
   p.B0 = w1; p.B1 = w3; p.ldb = H; p.strideB = I * H;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
   p.O0 = g; p.O1 = u; p.O2 = h; p.ldc = I;
-  int rc = pk_tile::launch_ragged_m<T, true, true>(p, A, mf::persistent_grid(), pk_timing::K_SWIGLU_GATE_UP, s);
-  if (rc) return rc;
+  return pk_tile::launch_ragged_m<T, true, pk_tile::GATE_UP>(p, A, mf::persistent_grid(), nullptr, pk_timing::K_SWIGLU_GATE_UP, s);
+}
+template <typename T>
+int down_tile(const void* h, const void* w2, const int32_t* starts, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedM q = {};
   q.A0 = q.A1 = h; q.lda = I; q.map_div = 1;
   q.B0 = q.B1 = w2; q.ldb = I; q.strideB = H * I;
   q.starts = starts; q.E = (int32_t)E; q.K = (int32_t)I; q.nseg = 1; q.N = (int32_t)H;
   q.O0 = y; q.ldc = H;
-  return pk_tile::launch_ragged_m<T, true, false>(q, A, mf::persistent_grid(), pk_timing::K_SWIGLU_DOWN, s);
+  return pk_tile::launch_ragged_m<T, true, pk_tile::PLAIN>(q, A, mf::persistent_grid(), nullptr, pk_timing::K_SWIGLU_DOWN, s);
 }
 // C [A, N] = sum over nseg weight matrices [K, N] (row-major) of A_seg . B_seg
 template <typename T>
@@ -2266,7 +2294,23 @@ int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map
   p.B0 = B0; p.B1 = nseg > 1 ? B1 : B0; p.ldb = N; p.strideB = K * N;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)K; p.nseg = nseg; p.N = (int32_t)N;
   p.O0 = C; p.ldc = N;
-  return pk_tile::launch_ragged_m<T, false, false>(p, A, mf::persistent_grid(), kernel_id, s);
+  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), nullptr, kernel_id, s);
+}
+// d_h = d_y . w2[e] with the SwiGLU backward in the epilogue.  With scores: d_y is d_out, gathered through
+// row_map, and the score gradient is left as partial sums over *part_cols columns each.
+template <typename T>
+int dh_tile(const void* dy, const int32_t* row_map, int64_t div, const float* scores, const void* w2, const void* g, const void* u,
+            const int32_t* starts, void* d_g, void* d_u, void* hs, float* parts, int* part_cols, int64_t A, int64_t H,
+            int64_t I, int64_t E, hipStream_t s) {
+  pk_tile::RaggedM p = {};
+  p.A0 = p.A1 = dy; p.lda = H; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.B0 = p.B1 = w2; p.ldb = I; p.strideB = H * I;
+  p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
+  p.O0 = d_g; p.O1 = d_u; p.O2 = hs; p.ldc = I;
+  p.Gin = g; p.Uin = u; p.scores = scores; p.ds_part = parts; p.total_rows = A;
+  const int id = pk_timing::K_SWIGLU_DGRAD_DH;
+  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), nullptr, id, s);
+  return pk_tile::launch_ragged_m<T, false, pk_tile::BWD_SCALED>(p, A, mf::persistent_grid(), part_cols, id, s);
 }
 template <typename T>
 int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void* dg, const void* du, const void* x,
@@ -2341,26 +2385,32 @@ int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t ro
   hipStream_t s = (hipStream_t)stream;
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({x_rows, w1, w2, w3, g, u, h, y});
   const bool pieces = tile_gemm_ok(dtype, H, I, {x_rows, w1, w2, w3, g, u, h, y});
-  const int64_t few = skinny_rows(A, I, E, mfma);
+  const int64_t few = skinny_rows(A, I, E);
   if (dtype == PK_BF16 && pieces && few > 0)
     return fwd_skinny(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, few, s);
-  if (!mfma && pieces)
-    return dtype == PK_F32 ? fwd_tile<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s)
-                           : fwd_tile<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
-  if (!mfma && !g) return PK_ERR_ARG;      // the FMA kernels form h from g and u in memory
+  if (!mfma && pieces && dtype == PK_F32) {
+    rc = gate_up_tile<float>(x_rows, row_map, row_map_div, w1, w3, starts, g, u, h, A, H, I, E, s);
+    return rc ? rc : down_tile<float>(h, w2, starts, y, A, H, I, E, s);
+  }
+  if (!pieces && !g) return PK_ERR_ARG;      // the FMA kernels form h from g and u in memory
   if (dtype == PK_F32)
     return fwd_simt<float>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
-  if (!mfma)
+  if (!pieces)
     return fwd_simt<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
 
-  mf::RaggedMParams p = {};
-  p.A0 = (const bf16_t*)x_rows; p.A1 = nullptr; p.lda = H;
-  p.row_map = row_map; p.map_div = mf::make_fastdiv(row_map_div);
-  p.B0 = (const bf16_t*)w1; p.B1 = (const bf16_t*)w3; p.ldb = H; p.strideB = I * H;
-  p.starts = starts; p.E = (int32_t)E; p.Kseg = (int32_t)H; p.nseg = 1;
-  p.O0 = (bf16_t*)g; p.O1 = (bf16_t*)u; p.O2 = (bf16_t*)h; p.ldc = I;
-  rc = launch_rm<true, mf::EPI_SWIGLU>(p, A, I, pk_timing::K_SWIGLU_GATE_UP, s);
+  if (mfma && wide_gate_up(A, I, E)) {
+    mf::RaggedMParams p = {};
+    p.A0 = (const bf16_t*)x_rows; p.A1 = nullptr; p.lda = H;
+    p.row_map = row_map; p.map_div = mf::make_fastdiv(row_map_div);
+    p.B0 = (const bf16_t*)w1; p.B1 = (const bf16_t*)w3; p.ldb = H; p.strideB = I * H;
+    p.starts = starts; p.E = (int32_t)E; p.Kseg = (int32_t)H; p.nseg = 1;
+    p.O0 = (bf16_t*)g; p.O1 = (bf16_t*)u; p.O2 = (bf16_t*)h; p.ldc = I;
+    rc = launch_rm<true, mf::EPI_SWIGLU>(p, A, I, pk_timing::K_SWIGLU_GATE_UP, s);
+  } else {
+    rc = gate_up_tile<bf16_t>(x_rows, row_map, row_map_div, w1, w3, starts, g, u, h, A, H, I, E, s);
+  }
   if (rc) return rc;
+  if (!mfma || !wide_down(A, H, I, E)) return down_tile<bf16_t>(h, w2, starts, y, A, H, I, E, s);
 
   mf::RaggedMParams q = {};
   q.A0 = (const bf16_t*)h; q.lda = I;
@@ -2378,20 +2428,20 @@ int pk_grouped_swiglu_dgrad_dh(const void* d_y, const void* w2, const void* g, c
   if (A == 0) return PK_OK;
   if (!d_y || !w2 || !g || !u || !starts || !d_g || !d_u) return PK_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const bool simt = dtype == PK_F32 || !mfma_shape_ok(H, I) || !all_aligned16({d_y, w2, g, u, d_g, d_u});
-  if (simt) {
+  const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_y, w2, g, u, d_g, d_u});
+  if (!(mfma && wide_dh(A, I, E)) && tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u}))
+    return dtype == PK_F32 ? dh_tile<float>(d_y, nullptr, 1, nullptr, w2, g, u, starts, d_g, d_u, nullptr, nullptr, nullptr, A, H, I, E, s)
+                           : dh_tile<bf16_t>(d_y, nullptr, 1, nullptr, w2, g, u, starts, d_g, d_u, nullptr, nullptr, nullptr, A, H, I, E, s);
+  if (!mfma) {
     // d_h = d_y . w2[e]  (w2[e] is [H, I]: B(k=h, n=i) = w2[h*I + i]); staged in d_u's buffer
     const int64_t n = A * I;
-    const bool tile = tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u});
     if (dtype == PK_F32) {
-      rc = tile ? dgrad_tile<float>(d_y, nullptr, H, nullptr, 1, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s)
-                : simt_ragged_m<float>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
+      rc = simt_ragged_m<float>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
       if (rc) return rc;
       PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_ELEMENTWISE, s, (swiglu_bwd_kernel<float>), dim3((unsigned)pk_ceil_div(n, 256)), dim3(256), 0, s,
                         (const float*)d_u, (const float*)g, (const float*)u, (float*)d_g, (float*)d_u, n);
     } else {
-      rc = tile ? dgrad_tile<bf16_t>(d_y, nullptr, H, nullptr, 1, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s)
-                : simt_ragged_m<bf16_t>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
+      rc = simt_ragged_m<bf16_t>(d_y, H, nullptr, 1, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
       if (rc) return rc;
       PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_ELEMENTWISE, s, (swiglu_bwd_kernel<bf16_t>), dim3((unsigned)pk_ceil_div(n, 256)), dim3(256), 0, s,
                         (const bf16_t*)d_u, (const bf16_t*)g, (const bf16_t*)u, (bf16_t*)d_g, (bf16_t*)d_u, n);
@@ -2429,10 +2479,11 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
                                 const float* scores, const void* w2, const void* g,
                                 const void* u, const int32_t* starts, void* d_g, void* d_u,
                                 void* hs, void* d_gT, void* d_uT, void* hsT, int64_t ldt, float* d_scores,
-                                void* workspace, int64_t workspace_bytes, int64_t A, int64_t H, int64_t I,
-                                int64_t E, int dtype, pk_stream_t stream) {
+                                void* workspace, int64_t workspace_bytes, int64_t* n_partial, int64_t A, int64_t H,
+                                int64_t I, int64_t E, int dtype, pk_stream_t stream) {
   int rc = check_common(A, H, I, E, dtype);
   if (rc) return rc;
+  if (n_partial) *n_partial = 0;
   if (A == 0) return PK_OK;
   const bool transposed = d_gT != nullptr;
   if (!d_out || !row_map || row_map_div <= 0 || row_map_div > 0x7fffffffll || !scores || !w2 || !g || !u || !starts ||
@@ -2447,8 +2498,18 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
     if (!all_aligned16({d_out, w2, g, u, d_g, d_u, hs, d_gT, d_uT, hsT})) return PK_ERR_ALIGN;
   }
   hipStream_t s = (hipStream_t)stream;
-  const bool simt = dtype == PK_F32 || !mfma_shape_ok(H, I) || !all_aligned16({d_out, w2, g, u, d_g, d_u, hs});
-  if (simt) {
+  const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_out, w2, g, u, d_g, d_u, hs});
+  if (n_partial && !(mfma && wide_dh(A, I, E)) && tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs})) {
+    if (!workspace || workspace_bytes < pk_region_dgrad_dh_workspace_bytes(A, I)) return PK_ERR_WORKSPACE;
+    int part_cols = 0;
+    rc = dtype == PK_F32 ? dh_tile<float>(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, hs, (float*)workspace, &part_cols,
+                                          A, H, I, E, s)
+                         : dh_tile<bf16_t>(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, hs, (float*)workspace, &part_cols,
+                                           A, H, I, E, s);
+    if (!rc) *n_partial = pk_ceil_div(I, part_cols);
+    return rc;
+  }
+  if (!mfma) {
     // unscaled d_h = d_out[token] . w2[e], staged in d_u's buffer; then one wave per row
     const bool tile = tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs});
     if (tile && dtype == PK_F32)
@@ -2470,6 +2531,10 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
   }
   const int64_t need = pk_grouped_swiglu_dgrad_dh_scaled_workspace_bytes(A, I);
   if (!workspace || workspace_bytes < need) return PK_ERR_WORKSPACE;
+  if (n_partial) {
+    *n_partial = I / 64;
+    d_scores = nullptr;
+  }
   mf::RaggedMParams p = {};
   p.A0 = (const bf16_t*)d_out; p.lda = H;
   p.row_map = row_map; p.map_div = mf::make_fastdiv(row_map_div);
@@ -2495,7 +2560,20 @@ int pk_grouped_swiglu_dgrad_dh_scaled(const void* d_out, const int32_t* row_map,
                                       int64_t E, int dtype, pk_stream_t stream) {
   if (A > 0 && !hs) return PK_ERR_ARG;
   return dgrad_dh_scaled_impl(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, hs, nullptr, nullptr,
-                              nullptr, 0, d_scores, workspace, workspace_bytes, A, H, I, E, dtype, stream);
+                              nullptr, 0, d_scores, workspace, workspace_bytes, nullptr, A, H, I, E, dtype, stream);
+}
+
+int64_t pk_region_dgrad_dh_workspace_bytes(int64_t A, int64_t I) {
+  if (A < 0 || I <= 0) return PK_ERR_ARG;
+  return pk_ceil_div(I, 32) * A * (int64_t)sizeof(float);
+}
+int pk_region_dgrad_dh(const void* d_out, const int32_t* row_map, int64_t row_map_div, const float* scores, const void* w2, const void* g,
+                       const void* u, const int32_t* starts, void* d_g, void* d_u, void* hs, float* d_scores, int64_t* n_partial,
+                       void* workspace, int64_t workspace_bytes, int64_t A, int64_t H, int64_t I, int64_t E, int dtype,
+                       pk_stream_t stream) {
+  if (!n_partial || (A > 0 && !hs)) return PK_ERR_ARG;
+  return dgrad_dh_scaled_impl(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, hs, nullptr, nullptr, nullptr, 0, d_scores,
+                              workspace, workspace_bytes, n_partial, A, H, I, E, dtype, stream);
 }
 
 int pk_grouped_swiglu_dgrad_dh_scaled_t(const void* d_out, const int32_t* row_map, int64_t row_map_div,
@@ -2506,19 +2584,21 @@ int pk_grouped_swiglu_dgrad_dh_scaled_t(const void* d_out, const int32_t* row_ma
                                         int64_t I, int64_t E, int dtype, pk_stream_t stream) {
   if (A > 0 && (!d_gT || !d_uT || !hsT)) return PK_ERR_ARG;
   return dgrad_dh_scaled_impl(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, nullptr, d_gT, d_uT, hsT,
-                              ldt, d_scores, workspace, workspace_bytes, A, H, I, E, dtype, stream);
+                              ldt, d_scores, workspace, workspace_bytes, nullptr, A, H, I, E, dtype, stream);
 }
 
-int pk_grouped_swiglu_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3,
-                               const int32_t* starts, void* d_x_sorted, int64_t A, int64_t H,
-                               int64_t I, int64_t E, int dtype, pk_stream_t stream) {
+// by_size: small products may go to the tiles of tile_gemm.h.  Without it a shape that has a transposed path
+// stays on the kernels of that path, whose result is then the same bit for bit.
+static int dgrad_dx_impl(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
+                         bool by_size, int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
   int rc = check_common(A, H, I, E, dtype);
   if (rc) return rc;
   if (A == 0) return PK_OK;
   if (!d_g || !d_u || !w1 || !w3 || !starts || !d_x_sorted) return PK_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const bool simt = dtype == PK_F32 || !mfma_shape_ok(H, I) || !all_aligned16({d_g, d_u, w1, w3, d_x_sorted});
-  if (simt) {
+  const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_g, d_u, w1, w3, d_x_sorted}) &&
+                    (wide_dx(A, H, I, E) || (!by_size && H % 256 == 0 && I % 256 == 0));
+  if (!mfma) {
     // d_x = d_g . w1[e] + d_u . w3[e]   (w[e] is [I, H]: B(k=i, n=h) = w[i*H + h])
     if (tile_gemm_ok(dtype, H, I, {d_g, d_u, w1, w3, d_x_sorted}))
       return dtype == PK_F32
@@ -2542,6 +2622,15 @@ int pk_grouped_swiglu_dgrad_dx(const void* d_g, const void* d_u, const void* w1,
   return launch_rm<false, mf::EPI_PLAIN>(q, A, H, pk_timing::K_SWIGLU_DGRAD_DX, s);
 }
 
+int pk_grouped_swiglu_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
+                               int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
+  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, false, A, H, I, E, dtype, stream);
+}
+int pk_region_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
+                       int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
+  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, true, A, H, I, E, dtype, stream);
+}
+
 int pk_grouped_swiglu_dx_from_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dtype) {
   if (pk_grouped_swiglu_transposed_ld(A, H, I, E, dtype) <= 0) return 0;
   // measured on MI355X (H 2048, I 768, 128 experts): with 1,024 rows per expert the SwiGLU backward is
@@ -2549,6 +2638,20 @@ int pk_grouped_swiglu_dx_from_transposed_pays(int64_t A, int64_t H, int64_t I, i
   // as runs of 4 KB); with 256 rows per expert the d_x GEMM on 128-row units loses 6 %, more than
   // the SwiGLU backward gains
   return A >= (int64_t)PK_RM_SHORT_ROWS * E ? 1 : 0;
+}
+
+int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dtype) {
+  if (pk_grouped_swiglu_transposed_ld(A, H, I, E, dtype) <= 0) return 0;
+  // The transposed pair runs the weight gradients as two launches of 256 x 256 tiles; wgrad_kernel takes all three
+  // in one, and d_h may then use smaller tiles.  Two launches that each leave half of the CUs idle lose to it
+  // (d_h + weight gradients, us, transposed -> plain: 8 experts 1024 x 512, 64 tiles each, 4,096 rows an expert
+  // 440 -> 270; 16 experts 512 x 256, 32 tiles, 4,096 rows 419 -> 304), and with 256 tiles it depends on whether
+  // d_h fills the chip (32 experts 1024 x 512: 128 rows 100 -> 66, 512 rows 168 -> 158, 1,024 rows 246 -> 241).  Above,
+  // the transposed pair is ahead (16 experts 2048 x 1024, 1,024 rows 369 -> 410); wgrad_kernel deals experts out
+  // over the XCDs and leaves some idle below eight (4 experts 2048 x 1024, 2,048 rows 275 -> 349).
+  const int64_t w2_units = E * (H / 256) * (I / 256);
+  if (w2_units < mf::persistent_grid() / 2) return 0;
+  return E < mf::NXCD || w2_units > mf::persistent_grid() || wide_fills(A, I, E, 8);
 }
 
 int pk_grouped_swiglu_dgrad_dx_t(const void* d_gT, const void* d_uT, int64_t ldt, const void* w1, const void* w3,
@@ -2576,7 +2679,7 @@ int pk_grouped_swiglu_dgrad(const void* d_y, const void* w1, const void* w2, con
                             int64_t E, int dtype, pk_stream_t stream) {
   int rc = pk_grouped_swiglu_dgrad_dh(d_y, w2, g, u, starts, d_g, d_u, A, H, I, E, dtype, stream);
   if (rc) return rc;
-  return pk_grouped_swiglu_dgrad_dx(d_g, d_u, w1, w3, starts, d_x_sorted, A, H, I, E, dtype, stream);
+  return pk_region_dgrad_dx(d_g, d_u, w1, w3, starts, d_x_sorted, A, H, I, E, dtype, stream);
 }
 
 // d_y rows are addressed directly (dy_gathered == 0) or through the row map like x
@@ -2597,7 +2700,13 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   if (!row_map) row_map_div = 1;
   const int32_t* dy_map = dy_gathered ? row_map : nullptr;
   hipStream_t s = (hipStream_t)stream;
-  const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3});
+  // wgrad_kernel's 256 x 256 tiles where they give at least half of the CUs work and every XCD an expert; otherwise
+  // the 64- or 128-wide tiles of tile_gemm.h (us, 256 x 256 or, at widths that are not multiples of 256, its former
+  // 128 x 128 tiles -> those: 4 experts 2048 x 1024, 2,048 rows 260 -> 219; 24 experts 640 x 896, 1,000 rows 379 -> 196;
+  // 64 experts 384 x 640, 1,536 rows 614 -> 338; but 8 experts 1024 x 512, 1,024 rows, 192 tiles 50 against 79)
+  const int n_weights = (d_w1 ? 1 : 0) + (d_w2 ? 1 : 0) + (d_w3 ? 1 : 0);
+  const bool mfma = dtype == PK_BF16 && H % 256 == 0 && I % 256 == 0 && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}) &&
+                    E >= mf::NXCD && E * (H / 256) * (I / 256) * n_weights >= mf::persistent_grid() / 2;
   if (!mfma && tile_gemm_ok(dtype, H, I, {d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}))
     return dtype == PK_F32
                ? wgrad_tile<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, A, H, I, E, s)
@@ -2630,19 +2739,15 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   if (n == 0) return PK_OK;
   p.starts = starts; p.order = expert_order; p.E = (int32_t)E; p.map_div = mf::make_fastdiv(row_map_div);
   p.accumulate = accumulate ? 1 : 0;
-  const bool big = (H % 256 == 0) && (I % 256 == 0);
-  const int tile = big ? 256 : 128;
-  p.tiles_per_expert = (int32_t)((H / tile) * (I / tile));
+  p.tiles_per_expert = (int32_t)((H / 256) * (I / 256));
   p.nprob = n;
   const int64_t blocks = (int64_t)p.tiles_per_expert * n * pk_ceil_div(E, mf::NXCD) * mf::NXCD;
   const int gy = 1;
   if (blocks > 0x7ffffff0ll) return PK_ERR_SHAPE;
-  if (big && A < (int64_t)PK_WG_SHORTK_ROWS * E)
+  if (A < (int64_t)PK_WG_SHORTK_ROWS * E)
     PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG_SHORTK>), dim3((unsigned)blocks, gy), dim3(PK_WG_BIG_THREADS), 0, s, p);
-  else if (big)
-    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), dim3((unsigned)blocks, gy), dim3(PK_WG_BIG_THREADS), 0, s, p);
   else
-    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_SMALL>), dim3((unsigned)blocks, gy), dim3(PK_WG_SMALL_THREADS), 0, s, p);
+    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), dim3((unsigned)blocks, gy), dim3(PK_WG_BIG_THREADS), 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }

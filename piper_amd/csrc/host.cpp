@@ -395,13 +395,14 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const void* x_rows = norm ? m.at_(sv.xn) : xc.data_ptr();
     const int32_t *perm = m.i32(sv.perm), *starts = m.i32(sv.starts);
 
-    // Shapes with a K-contiguous weight-gradient path get d_g, d_u and score*h transposed; with long
+    // Shapes where the K-contiguous weight-gradient path pays get d_g, d_u and score*h transposed; with long
     // experts the d_x GEMM reads its A operand from the same blocks and the row-major pair is left out.
-    const int64_t ldt = s.dtype == PK_BF16 ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
+    const int64_t ldt = pk_region_transposed_pays(s.A, s.H, s.I, s.E, s.dtype) ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
     const bool blocks_only = ldt > 0 && pk_grouped_swiglu_dx_from_transposed_pays(s.A, s.H, s.I, s.E, s.dtype);
     Block t;
     const int64_t ai = s.A * s.I * s.es, ait = ldt * s.I * s.es;
-    const int64_t ds_ws = std::max<int64_t>(pk_grouped_swiglu_dgrad_dh_scaled_workspace_bytes(s.A, s.I), 4);
+    const int64_t ds_ws = std::max<int64_t>(pk_region_dgrad_dh_workspace_bytes(s.A, s.I), 4);
+    int64_t n_part = (s.I + 63) / 64;      // rows of partial score gradients; 0: d_scores is written
     const size_t d_g = t.add(blocks_only ? 0 : ai), d_u = t.add(blocks_only ? 0 : ai), hs = t.add(ldt > 0 ? 0 : ai);
     const size_t d_gT = t.add(ait), d_uT = t.add(ait), hsT = t.add(ait);
     const size_t d_scores = t.add(ldt > 0 ? 0 : s.A * 4), part = t.add(ds_ws), d_logits = t.add(s.T * s.E * 4);
@@ -418,8 +419,8 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled_t, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
               t.at_(d_gT), t.at_(d_uT), t.at_(hsT), ldt, nullptr, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
     else
-      PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
-              t.at_(hs), t.f32(d_scores), t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
+      PK_CALL(pk_region_dgrad_dh, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
+              t.at_(hs), t.f32(d_scores), &n_part, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
 
     const RegionWgrad wgrad{s, d_out, xc, sv.mem.memory(), t.memory(), x_rows, dg, du, t.at_(hs), t.at_(d_gT), t.at_(d_uT), t.at_(hsT),
                             ldt, perm, starts, m.i32(sv.order)};
@@ -429,14 +430,14 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       if (blocks_only)
         PK_CALL(pk_grouped_swiglu_dgrad_dx_t, t.at_(d_gT), t.at_(d_uT), ldt, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
       else
-        PK_CALL(pk_grouped_swiglu_dgrad_dx, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
+        PK_CALL(pk_region_dgrad_dx, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
     };
     // The router's backward and the gradient of the region's input; with a norm in front its backward
     // follows and adds the residual branch's gradient.
     Tensor d_x, d_norm_w;
     const auto router_and_input = [&](const Tensor& d_wg, const Tensor& d_b) {
       if (need_xn) d_x = at::empty({s.T, s.H}, x.options());
-      PK_CALL(pk_region_router_bwd, m.f32(sv.logits), m.i32(sv.idx), ldt > 0 ? nullptr : t.f32(d_scores), t.f32(part), (s.I + 63) / 64, m.i32(sv.inv),
+      PK_CALL(pk_region_router_bwd, m.f32(sv.logits), m.i32(sv.idx), n_part > 0 ? nullptr : t.f32(d_scores), t.f32(part), n_part, m.i32(sv.inv),
               s.route_norm, (float)s.route_scale, x_rows, s.dtype, fptr(w_gate), t.at_(d_xs), !need_xn ? nullptr : norm ? t.at_(d_xn) : ptr(d_x),
               static_cast<float*>(ptr(d_wg)), static_cast<float*>(ptr(d_b)), 0, t.f32(d_logits), s.T, s.H, s.E, s.K, t.at_(router_ws),
               router_ws_bytes, st);

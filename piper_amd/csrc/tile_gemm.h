@@ -177,10 +177,15 @@ struct RaggedM {
   const int32_t* starts;
   int32_t E, K, nseg, N;
   int32_t n_tiles;
-  void* O0;                 // C;  DUAL: g (optional)
-  void* O1;                 //     DUAL: u (optional)
-  void* O2;                 //     DUAL: h = silu(g) * u
+  void* O0;                 // C;  GATE_UP: g (optional);  BWD, BWD_SCALED: d_g
+  void* O1;                 //     GATE_UP: u (optional);  BWD, BWD_SCALED: d_u
+  void* O2;                 //     GATE_UP: h = silu(g) * u;  BWD_SCALED: score * h
   int64_t ldc;
+  const void* Gin;          // BWD, BWD_SCALED: g and u of the forward [rows, ldc]
+  const void* Uin;
+  const float* scores;      // BWD_SCALED: score of every routed slot (row_map names the slot of a sorted row)
+  float* ds_part;           // BWD_SCALED: [ceil(N / columns of a wave)][total_rows]: the score gradient in parts
+  int64_t total_rows;
 };
 
 // Tile b of a launch.  Blocks b, b + 8, ... run on one XCD: CHUNK neighbouring tiles (which share
@@ -192,11 +197,18 @@ __device__ __forceinline__ int unit_of_block(int b) {
   return ((q / CHUNK) * NXCD + x) * CHUNK + (q % CHUNK);
 }
 
-// DUAL: two weight matrices (gate and up) against the same A rows, SiLU(g) * u in the epilogue.
-template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, bool DUAL>
+// What happens to the product.
+// GATE_UP: two weight matrices (gate and up) against the same A rows, SiLU(g) * u.
+// BWD: the product is d_h; d_g = d_h * u * silu'(g), d_u = d_h * silu(g).
+// BWD_SCALED: the A rows are rows of d_out (gathered), the product is d_h before the routed row's score:
+// d_g and d_u from score * d_h, score * h for the weight gradient, and the row sums of d_h * h over a
+// wave's columns, whose total is the score's gradient.  d_h never leaves the registers.
+enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
+template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, int EPI>
 __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const RaggedM p) {
   constexpr int THREADS = 64 * WM * WN;       // of a group: WM x WN waves of TM x TN MFMA tiles
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, BK = kBK<T>, PIECE = kPiece<T>;
+  constexpr bool DUAL = EPI == GATE_UP;
   constexpr int NB = DUAL ? 2 : 1;
   constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, STAGE = A_BYTES + NB * B_BYTES;
@@ -346,6 +358,57 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
     if (group > 0) return;
   }
 
+  if constexpr (EPI == BWD || EPI == BWD_SCALED) {
+    constexpr int PART = 32 * TN;
+    const int col0 = n0 + wn * PART;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int r = (wm * TM + i) * 32 + (lane & 31);
+      const bool live = r < rows;
+      const int64_t o0 = (int64_t)(row0 + r) * p.ldc + col0 + 4 * (lane >> 5);
+      float g[TN][4][4], u[TN][4][4];       // all loads of a 32-row group are in flight together
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) g[j][q][t] = u[j][q][t] = 0.f;
+          if (live && col0 + 32 * j + 8 * q + 4 * (lane >> 5) < p.N) {
+            load4<T>(reinterpret_cast<const T*>(p.Gin) + o0 + 32 * j + 8 * q, g[j][q]);
+            load4<T>(reinterpret_cast<const T*>(p.Uin) + o0 + 32 * j + 8 * q, u[j][q]);
+          }
+        }
+      float sc = 1.f, ds = 0.f;
+      if (EPI == BWD_SCALED && live) sc = p.scores[p.row_map[row0 + r]];
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float og[4], ou[4], oh[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const float a = acc[0][i][j][4 * q + t], gv = g[j][q][t], uv = u[j][q][t];
+            const float sg = 1.f / (1.f + expf(-gv));
+            const float d = pk_to_float<T>(pk_from_float<T>(sc * a));      // d_h is a tensor of T
+            og[t] = d * uv * (sg * (1.f + gv * (1.f - sg)));
+            ou[t] = d * (gv * sg);
+            const float hv = (gv * sg) * uv;
+            ds += a * hv;
+            oh[t] = sc * hv;
+          }
+          if (live && col0 + 32 * j + 8 * q + 4 * (lane >> 5) < p.N) {
+            store4<T>(reinterpret_cast<T*>(p.O0) + o0 + 32 * j + 8 * q, og);
+            store4<T>(reinterpret_cast<T*>(p.O1) + o0 + 32 * j + 8 * q, ou);
+            if (EPI == BWD_SCALED) store4<T>(reinterpret_cast<T*>(p.O2) + o0 + 32 * j + 8 * q, oh);
+          }
+        }
+      if constexpr (EPI == BWD_SCALED) {
+        ds += __shfl_xor(ds, 32);             // lanes l and l + 32 hold the two column halves of a row
+        if (live && lane < 32 && col0 < p.N) p.ds_part[(int64_t)(col0 / PART) * p.total_rows + row0 + r] = ds;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int r = (wm * TM + i) * 32 + (lane & 31);
@@ -378,36 +441,38 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
   }
 }
 
-template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, bool DUAL>
-inline int launch_tiles(RaggedM p, int64_t A_rows, int kernel_id, hipStream_t s) {
+// *part_cols: columns per part of the score gradient
+template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, int EPI>
+inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id, hipStream_t s) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   p.n_tiles = (int32_t)pk_ceil_div(p.N, BN);
   const int64_t units = (pk_ceil_div(A_rows, BM) + p.E) * p.n_tiles;
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
+  if (part_cols) *part_cols = 32 * TN;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(64 * WM * WN * KS);
-  PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, DEPTH, KS, B_KC, DUAL>), grid, block, 0, s, p);
+  PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, DEPTH, KS, B_KC, EPI>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
-template <typename T, bool B_KC, bool DUAL>
-inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int kernel_id, hipStream_t s) {
+template <typename T, bool B_KC, int EPI>
+inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int* part_cols, int kernel_id, hipStream_t s) {
   // 128 x 128 tiles once they give every CU work for two rounds; below that the chip is filled by
   // four times as many 64 x 64 tiles
   const int64_t big = (A_rows / 128 + (p.E + 1) / 2) * pk_ceil_div(p.N, 128);
-  if (big >= 2 * (int64_t)cus) return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, DUAL>(p, A_rows, kernel_id, s);
+  if (big >= 2 * (int64_t)cus) return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   // row tiles that hold rows, about: every expert's last one is half full
   const int64_t row_tiles = A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2;
   const int64_t tiles = row_tiles * pk_ceil_div(p.N, 64), k_tiles = pk_ceil_div(p.K, kBK<T>) * p.nseg;
   // an fp32 tile is 1,024 cycles of the matrix cores per k-tile, whoever shares it: 64 x 32 tiles while
   // even those do not outnumber the CUs (200 to 512 rows, 256 x 512: -20 %)
   if (sizeof(T) == 4 && 2 * tiles <= cus) {
-    if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, DUAL>(p, A_rows, kernel_id, s);
-    return launch_tiles<T, 2, 1, 1, 1, 2, 1, B_KC, DUAL>(p, A_rows, kernel_id, s);
+    if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+    return launch_tiles<T, 2, 1, 1, 1, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   const int ks = reduction_groups(tiles, k_tiles, cus);
-  if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, DUAL ? 2 : 4, B_KC, DUAL>(p, A_rows, kernel_id, s);
-  if (ks == 2) return launch_tiles<T, 2, 2, 1, 1, 2, 2, B_KC, DUAL>(p, A_rows, kernel_id, s);
-  return launch_tiles<T, 2, 2, 1, 1, 3, 1, B_KC, DUAL>(p, A_rows, kernel_id, s);
+  if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, EPI == GATE_UP ? 2 : 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  if (ks == 2) return launch_tiles<T, 2, 2, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  return launch_tiles<T, 2, 2, 1, 1, 3, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
 }
 
 // ---------------------------------------------------------------------------------- ragged K

@@ -586,3 +586,63 @@ def test_experts_with_few_rows(dev, counts, H, I):
         for name, got, ref in (("g", g, ge), ("u", u, ue), ("h", h, he), ("y", y, he @ w2[e].double().t())):
             assert rel_err(got[s:s + c], ref) <= BF16_TOL, (name, e, c)
         s += c
+
+
+REGION_BACKWARD_CASES = [
+    # (counts, H, I): split reductions with every row and column remainder, unsplit 64-row tiles, 128-row
+    # tiles (parts of 64 columns), the persistent kernels at widths of 256 and 128 columns, a single row
+    ([0, 1, 63, 64, 65, 200, 0, 33], 72, 40),
+    ([1], 256, 256),
+    ([130, 0, 64, 300] * 8, 256, 512),
+    ([1000, 999, 0, 1025, 800, 1100, 900, 1300, 1000], 72, 1000),
+    ([2900, 2800, 3000], 128, 1024),
+    ([5000, 6000, 5003], 128, 384),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts,H,I", REGION_BACKWARD_CASES)
+def test_region_input_gradient_by_size(dev, dtype, counts, H, I):
+    """pk_region_dgrad_dh (whichever tiles it picks, the score gradient in parts or whole) and
+    pk_region_dgrad_dx against float64 matmuls of the same inputs."""
+    from piper_amd import _lib
+    from piper_amd._lib import call, current_stream, dtype_code, ptr
+    import ctypes
+    print(f"[case] region input gradient {dtype} counts={counts[:9]} H={H} I={I}", flush=True)
+    tol = BF16_TOL if dtype == torch.bfloat16 else F32_TOL
+    counts = list(counts) + ([1] if sum(counts) % 2 else [])
+    A, E, K = sum(counts), len(counts), 2
+    _, w1, w2, w3, _, cnt = (t.to(dev) for t in _make(41, counts, H, I, dtype))
+    gen = torch.Generator().manual_seed(5)
+    perm = torch.randperm(A, generator=gen).to(torch.int32).to(dev)
+    scores = (torch.rand(A // K, K, generator=gen) + 0.1).to(dev)
+    d_out = torch.randn(A // K, H, generator=gen).to(dtype).to(dev)
+    g, u = (torch.randn(A, I, generator=gen).to(dtype).to(dev) for _ in range(2))
+    starts = ops.counts_to_starts(cnt)
+    dg, du, hs = (torch.full_like(g, float("nan")) for _ in range(3))
+    ds = torch.zeros(A, device=dev)
+    ws = torch.full((int(_lib.load().pk_region_dgrad_dh_workspace_bytes(A, I)) // 4,), float("nan"), device=dev)
+    n_part = ctypes.c_int64(-1)
+    call("pk_region_dgrad_dh", ptr(d_out), ptr(perm), K, ptr(scores), ptr(w2), ptr(g), ptr(u), ptr(starts), ptr(dg), ptr(du), ptr(hs), ptr(ds),
+         ctypes.addressof(n_part), ptr(ws), ws.numel() * 4, A, H, I, E, dtype_code(dtype), current_stream(dev))
+    n = n_part.value
+    assert n in (0, (I + 31) // 32, (I + 63) // 64)
+    if n > 0:
+        ds = torch.zeros_like(ds).index_copy(0, perm.long(), ws[:n * A].view(n, A).sum(0))
+    dx = torch.full((A, H), float("nan"), dtype=dtype, device=dev)
+    call("pk_region_dgrad_dx", ptr(dg), ptr(du), ptr(w1), ptr(w3), ptr(starts), ptr(dx), A, H, I, E, dtype_code(dtype), current_stream(dev))
+    dg0, du0 = ops.grouped_swiglu_dgrad_dh(d_out[perm.long() // K].contiguous(), w2, g, u, starts)      # without the scores
+    sc = scores.reshape(-1)[perm.long()].double().unsqueeze(1)
+    go = g.double().requires_grad_(True)
+    uo = u.double().requires_grad_(True)
+    h = torch.nn.functional.silu(go) * uo
+    dh, dx_ref, s = torch.empty(A, I, dtype=torch.float64, device=dev), torch.empty(A, H, dtype=torch.float64, device=dev), 0
+    for e, c in enumerate(counts):
+        dh[s:s + c] = d_out[perm[s:s + c].long() // K].double() @ w2[e].double()
+        dx_ref[s:s + c] = dg[s:s + c].double() @ w1[e].double() + du[s:s + c].double() @ w3[e].double()
+        s += c
+    dg_ref, du_ref = torch.autograd.grad(h, (go, uo), dh)
+    ds_ref = torch.zeros(A, dtype=torch.float64, device=dev).index_copy(0, perm.long(), (dh * h).sum(1).detach())
+    for name, got, ref in (("d_g", dg, dg_ref * sc), ("d_u", du, du_ref * sc), ("score * h", hs, h.detach() * sc), ("d_score", ds, ds_ref),
+                           ("d_x", dx, dx_ref), ("d_g unscaled", dg0, dg_ref), ("d_u unscaled", du0, du_ref)):
+        assert rel_err(got, ref) <= tol, (name, rel_err(got, ref))
