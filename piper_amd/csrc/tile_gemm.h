@@ -99,32 +99,47 @@ __device__ __forceinline__ void mma_tiles(floatx16_t (&acc)[TM][TN], const Frag<
       for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j].v[q], a[i].v[q], acc[i][j], 0, 0, 0);
 }
 
+// a 16-byte piece of a row, as floats
 template <typename T>
-__device__ __forceinline__ void store4(T* p, const float (&f)[4]);
-template <>
-__device__ __forceinline__ void store4<float>(float* p, const float (&f)[4]) {
-  *reinterpret_cast<floatx4_t*>(p) = floatx4_t{f[0], f[1], f[2], f[3]};
-}
-template <>
-__device__ __forceinline__ void store4<bf16_t>(bf16_t* p, const float (&f)[4]) {
-  bf16x4_t v;
+__device__ __forceinline__ void load_piece(const T* p, float (&f)[kPiece<T>]) {
+  if constexpr (sizeof(T) == 4) {
+    const floatx4_t v = *reinterpret_cast<const floatx4_t*>(p);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = (bf16_t)f[i];
-  *reinterpret_cast<bf16x4_t*>(p) = v;
+    for (int i = 0; i < 4; ++i) f[i] = v[i];
+  } else {
+    const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(p);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = (float)v[i];
+  }
 }
 template <typename T>
-__device__ __forceinline__ void load4(const T* p, float (&f)[4]);
-template <>
-__device__ __forceinline__ void load4<float>(const float* p, float (&f)[4]) {
-  const floatx4_t v = *reinterpret_cast<const floatx4_t*>(p);
+__device__ __forceinline__ void store_piece(T* p, const float (&f)[kPiece<T>]) {
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<floatx4_t*>(p) = floatx4_t{f[0], f[1], f[2], f[3]};
+  } else {
+    bf16x8_t v;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) f[i] = v[i];
+    for (int i = 0; i < 8; ++i) v[i] = (bf16_t)f[i];
+    *reinterpret_cast<bf16x8_t*>(p) = v;
+  }
 }
-template <>
-__device__ __forceinline__ void load4<bf16_t>(const bf16_t* p, float (&f)[4]) {
-  const bf16x4_t v = *reinterpret_cast<const bf16x4_t*>(p);
+
+// The way of a product from the accumulators to memory: the waves put 32 rows each into LDS as fp32 [rows][X],
+// then every thread of the workgroup takes 16-byte pieces of T of it, neighbours along a row.  Straight from
+// the accumulators a store covers 16 bytes in each of 32 rows, and every 128-byte line is opened eight times.
+// 16-byte units of a row are XOR-ed with the row against bank conflicts.
+template <int X>
+__device__ __forceinline__ void stage_acc(float* lds, int row, int col, const float* four) {
+  *reinterpret_cast<floatx4_t*>(lds + row * X + (((col >> 2) ^ (row & (X / 4 - 1))) << 2)) = floatx4_t{four[0], four[1], four[2], four[3]};
+}
+template <int X, int N>
+__device__ __forceinline__ void staged(const float* lds, int row, int col, float (&f)[N]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) f[i] = (float)v[i];
+  for (int h = 0; h < N / 4; ++h) {
+    const floatx4_t v = *reinterpret_cast<const floatx4_t*>(lds + row * X + ((((col >> 2) + h) ^ (row & (X / 4 - 1))) << 2));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[4 * h + i] = v[i];
+  }
 }
 
 // f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
@@ -184,7 +199,7 @@ struct RaggedM {
   const void* Gin;          // BWD, BWD_SCALED: g and u of the forward [rows, ldc]
   const void* Uin;
   const float* scores;      // BWD_SCALED: score of every routed slot (row_map names the slot of a sorted row)
-  float* ds_part;           // BWD_SCALED: [ceil(N / columns of a wave)][total_rows]: the score gradient in parts
+  float* ds_part;           // BWD_SCALED: [column tiles][total_rows]: the score gradient in parts
   int64_t total_rows;
 };
 
@@ -202,7 +217,7 @@ __device__ __forceinline__ int unit_of_block(int b) {
 // BWD: the product is d_h; d_g = d_h * u * silu'(g), d_u = d_h * silu(g).
 // BWD_SCALED: the A rows are rows of d_out (gathered), the product is d_h before the routed row's score:
 // d_g and d_u from score * d_h, score * h for the weight gradient, and the row sums of d_h * h over a
-// wave's columns, whose total is the score's gradient.  d_h never leaves the registers.
+// tile's columns, whose total is the score's gradient.  d_h never leaves the workgroup.
 enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
 template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, int EPI>
 __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const RaggedM p) {
@@ -355,100 +370,89 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
     static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
   if constexpr (KS > 1) {
     add_groups<KS, NB * TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
-    if (group > 0) return;
   }
 
-  if constexpr (EPI == BWD || EPI == BWD_SCALED) {
-    constexpr int PART = 32 * TN;
-    const int col0 = n0 + wn * PART;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int r = (wm * TM + i) * 32 + (lane & 31);
-      const bool live = r < rows;
-      const int64_t o0 = (int64_t)(row0 + r) * p.ldc + col0 + 4 * (lane >> 5);
-      float g[TN][4][4], u[TN][4][4];       // all loads of a 32-row group are in flight together
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) g[j][q][t] = u[j][q][t] = 0.f;
-          if (live && col0 + 32 * j + 8 * q + 4 * (lane >> 5) < p.N) {
-            load4<T>(reinterpret_cast<const T*>(p.Gin) + o0 + 32 * j + 8 * q, g[j][q]);
-            load4<T>(reinterpret_cast<const T*>(p.Uin) + o0 + 32 * j + 8 * q, u[j][q]);
-          }
-        }
-      float sc = 1.f, ds = 0.f;
-      if (EPI == BWD_SCALED && live) sc = p.scores[p.row_map[row0 + r]];
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float og[4], ou[4], oh[4];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const float a = acc[0][i][j][4 * q + t], gv = g[j][q][t], uv = u[j][q][t];
-            const float sg = 1.f / (1.f + expf(-gv));
-            const float d = pk_to_float<T>(pk_from_float<T>(sc * a));      // d_h is a tensor of T
-            og[t] = d * uv * (sg * (1.f + gv * (1.f - sg)));
-            ou[t] = d * (gv * sg);
-            const float hv = (gv * sg) * uv;
-            ds += a * hv;
-            oh[t] = sc * hv;
-          }
-          if (live && col0 + 32 * j + 8 * q + 4 * (lane >> 5) < p.N) {
-            store4<T>(reinterpret_cast<T*>(p.O0) + o0 + 32 * j + 8 * q, og);
-            store4<T>(reinterpret_cast<T*>(p.O1) + o0 + 32 * j + 8 * q, ou);
-            if (EPI == BWD_SCALED) store4<T>(reinterpret_cast<T*>(p.O2) + o0 + 32 * j + 8 * q, oh);
-          }
-        }
-      if constexpr (EPI == BWD_SCALED) {
-        ds += __shfl_xor(ds, 32);             // lanes l and l + 32 hold the two column halves of a row
-        if (live && lane < 32 && col0 < p.N) p.ds_part[(int64_t)(col0 / PART) * p.total_rows + row0 + r] = ds;
-      }
-    }
-    return;
-  }
+  constexpr int CHUNK_ROWS = 32 * WM, ROW_PIECES = BN / PIECE, ALL = THREADS * KS;
+  static_assert(NB * CHUNK_ROWS * BN * 4 <= KS * 2 * STAGE, "the staged rows reuse the k-tiles' LDS");
+  static_assert(CHUNK_ROWS * ROW_PIECES % 64 == 0 && 64 % ROW_PIECES == 0, "whole waves, a row in one wave");
+  float* const lds = reinterpret_cast<float*>(smem_);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int r = (wm * TM + i) * 32 + (lane & 31);
-    if (r >= rows) continue;
+    __syncthreads();                         // the LDS has been read for the last time
+    if (group == 0) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+      for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + (wn * TN + j) * 32 + 8 * q + 4 * (lane >> 5);
-        if (n >= p.N) continue;
-        const int64_t o = (int64_t)(row0 + r) * p.ldc + n;
-        float f[4];
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) f[t] = acc[0][i][j][4 * q + t];
-        if constexpr (DUAL) {
-          float u[4], h[4];
+          for (int q = 0; q < 4; ++q)
+            stage_acc<BN>(lds + b * CHUNK_ROWS * BN, 32 * wm + (lane & 31), 32 * (wn * TN + j) + 8 * q + 4 * (lane >> 5),
+                          reinterpret_cast<const float*>(&acc[b][i][j]) + 4 * q);
+    }
+    __syncthreads();
+    for (int s = threadIdx.x; s < CHUNK_ROWS * ROW_PIECES; s += ALL) {
+      const int lr = s / ROW_PIECES, c = (s % ROW_PIECES) * PIECE, n = n0 + c;
+      const int r = (lr >> 5) * 32 * TM + 32 * i + (lr & 31);
+      const bool live = r < rows && n < p.N;
+      const int64_t o = (int64_t)(row0 + r) * p.ldc + n;
+      float a[PIECE];
+      staged<BN>(lds, lr, c, a);
+      if constexpr (EPI == PLAIN) {
+        if (live) store_piece<T>(reinterpret_cast<T*>(p.O0) + o, a);
+      } else if constexpr (EPI == GATE_UP) {
+        float u[PIECE], h[PIECE];
+        staged<BN>(lds + CHUNK_ROWS * BN, lr, c, u);
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            f[t] = pk_to_float<T>(pk_from_float<T>(f[t]));     // g and u are tensors of T
-            u[t] = pk_to_float<T>(pk_from_float<T>(acc[NB - 1][i][j][4 * q + t]));
-            h[t] = (f[t] / (1.f + expf(-f[t]))) * u[t];
+        for (int t = 0; t < PIECE; ++t) {
+          a[t] = pk_to_float<T>(pk_from_float<T>(a[t]));     // g and u are tensors of T
+          u[t] = pk_to_float<T>(pk_from_float<T>(u[t]));
+          h[t] = (a[t] / (1.f + expf(-a[t]))) * u[t];
+        }
+        if (live) {
+          if (p.O0) store_piece<T>(reinterpret_cast<T*>(p.O0) + o, a);
+          if (p.O1) store_piece<T>(reinterpret_cast<T*>(p.O1) + o, u);
+          store_piece<T>(reinterpret_cast<T*>(p.O2) + o, h);
+        }
+      } else {
+        float ds = 0.f;
+        if (live) {
+          float g[PIECE], u[PIECE], hs[PIECE];
+          load_piece<T>(reinterpret_cast<const T*>(p.Gin) + o, g);
+          load_piece<T>(reinterpret_cast<const T*>(p.Uin) + o, u);
+          const float sc = EPI == BWD_SCALED ? p.scores[p.row_map[row0 + r]] : 1.f;
+#pragma unroll
+          for (int t = 0; t < PIECE; ++t) {
+            const float sg = 1.f / (1.f + expf(-g[t]));
+            const float d = pk_to_float<T>(pk_from_float<T>(sc * a[t]));      // d_h is a tensor of T
+            const float hv = (g[t] * sg) * u[t];
+            ds += a[t] * hv;
+            hs[t] = sc * hv;
+            const float d_u = d * (g[t] * sg);
+            g[t] = d * u[t] * (sg * (1.f + g[t] * (1.f - sg)));
+            u[t] = d_u;
           }
-          if (p.O0) store4<T>(reinterpret_cast<T*>(p.O0) + o, f);
-          if (p.O1) store4<T>(reinterpret_cast<T*>(p.O1) + o, u);
-          store4<T>(reinterpret_cast<T*>(p.O2) + o, h);
-        } else {
-          store4<T>(reinterpret_cast<T*>(p.O0) + o, f);
+          store_piece<T>(reinterpret_cast<T*>(p.O0) + o, g);
+          store_piece<T>(reinterpret_cast<T*>(p.O1) + o, u);
+          if (EPI == BWD_SCALED) store_piece<T>(reinterpret_cast<T*>(p.O2) + o, hs);
+        }
+        if constexpr (EPI == BWD_SCALED) {
+#pragma unroll
+          for (int off = 1; off < ROW_PIECES; off <<= 1) ds += __shfl_xor(ds, off);
+          if (live && c == 0) p.ds_part[(int64_t)nt * p.total_rows + row0 + r] = ds;
         }
       }
+    }
   }
 }
 
-// *part_cols: columns per part of the score gradient
+// *part_cols: columns per part of the score gradient (those of a tile)
 template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, int EPI>
 inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id, hipStream_t s) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   p.n_tiles = (int32_t)pk_ceil_div(p.N, BN);
   const int64_t units = (pk_ceil_div(A_rows, BM) + p.E) * p.n_tiles;
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
-  if (part_cols) *part_cols = 32 * TN;
+  if (part_cols) *part_cols = BN;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(64 * WM * WN * KS);
   PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, DEPTH, KS, B_KC, EPI>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
@@ -617,35 +621,40 @@ __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
       static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
     if constexpr (KS > 1) {
       add_groups<KS, TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
-      if (group > 0) return;
     }
-  } else if (p.accumulate || group > 0) {
+  } else if (p.accumulate) {
     return;                       // an expert without rows adds nothing
   }
 
+  static_assert(BM * BN * 4 <= KS * 2 * STAGE, "the staged tile reuses the k-tiles' LDS");
+  float* const lds = reinterpret_cast<float*>(smem_);
+  __syncthreads();                           // the LDS has been read for the last time
+  if (group == 0) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          stage_acc<BN>(lds, (wm * TM + i) * 32 + (lane & 31), (wn * TN + j) * 32 + 8 * v + 4 * (lane >> 5),
+                        reinterpret_cast<const float*>(&acc[i][j]) + 4 * v);
+  }
+  __syncthreads();
   T* const C = reinterpret_cast<T*>(q.C) + (int64_t)e * q.M * q.N;
+  constexpr int ROW_PIECES = BN / PIECE;
+  for (int s = threadIdx.x; s < BM * ROW_PIECES; s += THREADS * KS) {
+    const int r = s / ROW_PIECES, c = (s % ROW_PIECES) * PIECE;
+    if (m0 + r >= q.M || n0 + c >= q.N) continue;
+    T* const out = C + (int64_t)(m0 + r) * q.N + n0 + c;
+    float f[PIECE];
+    staged<BN>(lds, r, c, f);
+    if (p.accumulate) {
+      float old[PIECE];
+      load_piece<T>(out, old);
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + (wm * TM + i) * 32 + (lane & 31);
-    if (m >= q.M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int n = n0 + (wn * TN + j) * 32 + 8 * v + 4 * (lane >> 5);
-        if (n >= q.N) continue;
-        T* const c = C + (int64_t)m * q.N + n;
-        float f[4];
-#pragma unroll
-        for (int x = 0; x < 4; ++x) f[x] = acc[i][j][4 * v + x];
-        if (p.accumulate) {
-          float old[4];
-          load4<T>(c, old);
-#pragma unroll
-          for (int x = 0; x < 4; ++x) f[x] += old[x];
-        }
-        store4<T>(c, f);
-      }
+      for (int x = 0; x < PIECE; ++x) f[x] += old[x];
+    }
+    store_piece<T>(out, f);
   }
 }
 
