@@ -408,32 +408,9 @@ __host__ __device__ __forceinline__ int padded_start(int start, int e) {
   return (start & ~(kTransposedAlign - 1)) + kTransposedAlign * e;
 }
 
-// Division of a non-negative int32 by a divisor fixed per launch without the ~25 instructions of
-// the general integer division: multiply-high by 2^(32-s) for d = 2^s, otherwise by
-// floor(2^(31+s)/d)+1 followed by a shift by s-1 with s = ceil(log2 d) (exact for 0 <= n < 2^31).
-struct FastDiv {
-  uint32_t mul;    // 0: divisor is 1
-  int32_t shift;
-  int64_t d;       // the divisor itself (host side checks)
-};
-inline FastDiv make_fastdiv(int64_t d) {
-  FastDiv f = {0u, 0, d < 1 ? 1 : d};
-  if (d <= 1) return f;
-  int s = 0;
-  while (((int64_t)1 << s) < d) ++s;
-  if (((int64_t)1 << s) == d) { f.mul = 1u << (32 - s); return f; }   // mulhi by 2^(32-s) is the shift by s
-  f.mul = (uint32_t)((((uint64_t)1 << (31 + s)) / (uint64_t)d) + 1u);
-  f.shift = s - 1;
-  return f;
-}
-// No branch on the divisor's kind (it would sit between the MFMAs of the loops that divide per lane):
-// the product is always formed and a mask picks n itself for a divisor of 1.
-__device__ __forceinline__ int fastdiv(int n, const FastDiv f) {
-  const uint32_t u = (uint32_t)n;
-  const uint32_t q = __umulhi(u, f.mul) >> f.shift;
-  const uint32_t keep = f.mul == 0u ? 0xffffffffu : 0u;
-  return (int)((u & keep) | (q & ~keep));
-}
+using pk_units::FastDiv;
+using pk_units::fastdiv;
+using pk_units::make_fastdiv;
 
 struct RaggedMParams {
   const bf16_t* A0;      // A operand of k-segment 0, row-major [rows, lda]
@@ -2270,7 +2247,7 @@ template <typename T>
 int gate_up_tile(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w3, const int32_t* starts,
                  void* g, void* u, void* h, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedM p = {};
-  p.A0 = p.A1 = x; p.lda = H; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.A0 = p.A1 = x; p.lda = H; p.row_map = row_map; p.map_div = pk_units::make_fastdiv(div);
   p.B0 = w1; p.B1 = w3; p.ldb = H; p.strideB = I * H;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
   p.O0 = g; p.O1 = u; p.O2 = h; p.ldc = I;
@@ -2279,7 +2256,7 @@ int gate_up_tile(const void* x, const int32_t* row_map, int64_t div, const void*
 template <typename T>
 int down_tile(const void* h, const void* w2, const int32_t* starts, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedM q = {};
-  q.A0 = q.A1 = h; q.lda = I; q.map_div = 1;
+  q.A0 = q.A1 = h; q.lda = I; q.map_div = pk_units::make_fastdiv(1);
   q.B0 = q.B1 = w2; q.ldb = I; q.strideB = H * I;
   q.starts = starts; q.E = (int32_t)E; q.K = (int32_t)I; q.nseg = 1; q.N = (int32_t)H;
   q.O0 = y; q.ldc = H;
@@ -2290,7 +2267,7 @@ template <typename T>
 int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map, int64_t div, const void* B0, const void* B1,
                void* C, int64_t N, int nseg, const int32_t* starts, int64_t A, int64_t E, int kernel_id, hipStream_t s) {
   pk_tile::RaggedM p = {};
-  p.A0 = A0; p.A1 = nseg > 1 ? A1 : A0; p.lda = K; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.A0 = A0; p.A1 = nseg > 1 ? A1 : A0; p.lda = K; p.row_map = row_map; p.map_div = pk_units::make_fastdiv(div);
   p.B0 = B0; p.B1 = nseg > 1 ? B1 : B0; p.ldb = N; p.strideB = K * N;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)K; p.nseg = nseg; p.N = (int32_t)N;
   p.O0 = C; p.ldc = N;
@@ -2303,7 +2280,7 @@ int dh_tile(const void* dy, const int32_t* row_map, int64_t div, const float* sc
             const int32_t* starts, void* d_g, void* d_u, void* hs, float* parts, int* part_cols, int64_t A, int64_t H,
             int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedM p = {};
-  p.A0 = p.A1 = dy; p.lda = H; p.row_map = row_map; p.map_div = (int32_t)div;
+  p.A0 = p.A1 = dy; p.lda = H; p.row_map = row_map; p.map_div = pk_units::make_fastdiv(div);
   p.B0 = p.B1 = w2; p.ldb = I; p.strideB = H * I;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
   p.O0 = d_g; p.O1 = d_u; p.O2 = hs; p.ldc = I;
@@ -2317,7 +2294,7 @@ int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void*
                const int32_t* row_map, int64_t div, const int32_t* starts, void* dw1, void* dw2, void* dw3, int acc,
                int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedK p = {};
-  p.starts = starts; p.E = (int32_t)E; p.map_div = (int32_t)div; p.accumulate = acc ? 1 : 0;
+  p.starts = starts; p.E = (int32_t)E; p.map_div = pk_units::make_fastdiv(div); p.accumulate = acc ? 1 : 0;
   if (dw2) p.prob[p.nprob++] = {dy, H, dy_map, h, I, nullptr, dw2, (int32_t)H, (int32_t)I};
   if (dw1) p.prob[p.nprob++] = {dg, I, nullptr, x, H, row_map, dw1, (int32_t)I, (int32_t)H};
   if (dw3) p.prob[p.nprob++] = {du, I, nullptr, x, H, row_map, dw3, (int32_t)I, (int32_t)H};

@@ -185,7 +185,7 @@ struct RaggedM {
   const void* A1;           // k-segment 1 (nseg == 2)
   int64_t lda;
   const int32_t* row_map;   // optional gather: A row = row_map[sorted row] / map_div
-  int32_t map_div;
+  pk_units::FastDiv map_div;
   const void* B0;           // weights of k-segment 0 (DUAL: gate)
   const void* B1;           // weights of k-segment 1 (DUAL: up)
   int64_t ldb, strideB;     // row stride, elements between experts
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
     const int r = (tid + i * THREADS) >> 3;
     a_ok[i] = r < rows;
     int64_t src = row0 + (a_ok[i] ? r : 0);
-    if (p.row_map) src = p.row_map[src] / p.map_div;
+    if (p.row_map) src = pk_units::fastdiv(p.row_map[src], p.map_div);
     a_ptr[i] = reinterpret_cast<const T*>(p.A0) + src * p.lda + a_kofs;
   }
   const T* const B = reinterpret_cast<const T*>(p.B0) + (int64_t)e * p.strideB;
@@ -491,7 +491,8 @@ struct RaggedK {
   int32_t first[4];         // first tile of problem q within an expert's tiles; first[nprob] = all of them
   int32_t nprob;
   const int32_t* starts;
-  int32_t E, map_div, accumulate;
+  pk_units::FastDiv map_div;
+  int32_t E, accumulate;
 };
 
 template <typename T, int TM, int TN, int DEPTH, int KS>
@@ -543,13 +544,13 @@ __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
     for (int i = 0; i < LA; ++i) {
       const int k = kt * BK + a_k[i];
       a_row[i] = -1;
-      if (k < rows && a_col[i] < q.M) a_row[i] = q.a_map ? q.a_map[row0 + k] / p.map_div : row0 + k;
+      if (k < rows && a_col[i] < q.M) a_row[i] = q.a_map ? pk_units::fastdiv(q.a_map[row0 + k], p.map_div) : row0 + k;
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
       const int k = kt * BK + b_k[i];
       b_row[i] = -1;
-      if (k < rows && b_col[i] < q.N) b_row[i] = q.b_map ? q.b_map[row0 + k] / p.map_div : row0 + k;
+      if (k < rows && b_col[i] < q.N) b_row[i] = q.b_map ? pk_units::fastdiv(q.b_map[row0 + k], p.map_div) : row0 + k;
     }
   };
   u32x4_t ra_[DEPTH][LA], rb_[DEPTH][LB];
@@ -676,7 +677,7 @@ inline int launch_ragged_k(RaggedK p, int64_t A_rows, int cus, int kernel_id, hi
   if (units == 0) return PK_OK;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(256);
   const int ks = large ? 1 : reduction_groups(units, pk_ceil_div(pk_ceil_div(A_rows, p.E), kBK<T>), cus);
-  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 2, 2, 1, 1>), grid, block, 0, s, p);
+  if (large) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 2, 2, 2, 1>), grid, block, 0, s, p);
   else if (ks == 4) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 4>), grid, dim3(256 * 4), 0, s, p);
   else if (ks == 2) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 2, 2>), grid, dim3(256 * 2), 0, s, p);
   else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, 1, 1, 3, 1>), grid, block, 0, s, p);

@@ -6,6 +6,33 @@
 
 namespace pk_units {
 
+// Division of a non-negative int32 by a divisor fixed per launch without the ~25 instructions of
+// the general integer division: multiply-high by 2^(32-s) for d = 2^s, otherwise by
+// floor(2^(31+s)/d)+1 followed by a shift by s-1 with s = ceil(log2 d) (exact for 0 <= n < 2^31).
+struct FastDiv {
+  uint32_t mul;    // 0: divisor is 1
+  int32_t shift;
+  int64_t d;       // the divisor itself (host side checks)
+};
+inline FastDiv make_fastdiv(int64_t d) {
+  FastDiv f = {0u, 0, d < 1 ? 1 : d};
+  if (d <= 1) return f;
+  int s = 0;
+  while (((int64_t)1 << s) < d) ++s;
+  if (((int64_t)1 << s) == d) { f.mul = 1u << (32 - s); return f; }   // mulhi by 2^(32-s) is the shift by s
+  f.mul = (uint32_t)((((uint64_t)1 << (31 + s)) / (uint64_t)d) + 1u);
+  f.shift = s - 1;
+  return f;
+}
+// No branch on the divisor's kind (it would sit between the MFMAs of the loops that divide per lane):
+// the product is always formed and a mask picks n itself for a divisor of 1.
+__device__ __forceinline__ int fastdiv(int n, const FastDiv f) {
+  const uint32_t u = (uint32_t)n;
+  const uint32_t q = __umulhi(u, f.mul) >> f.shift;
+  const uint32_t keep = f.mul == 0u ? 0xffffffffu : 0u;
+  return (int)((u & keep) | (q & ~keep));
+}
+
 // Read-only tables (row offsets, row maps) addressed wave-uniformly: going through the constant
 // address space makes these scalar loads (lgkmcnt), which leaves vmcnt to the LDS ring.
 typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
