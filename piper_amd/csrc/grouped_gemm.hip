@@ -2135,10 +2135,9 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 
 bool mfma_shape_ok(int64_t H, int64_t I) { return H % 128 == 0 && I % 128 == 0; }
 
-// SwiGLU backward of intermediate sizes that are a multiple of 128 but not of 256.  The other products of
-// such widths run on the tiles of tile_gemm.h (24,000 rows of 24 experts, 640 x 896, us, these tiles -> those:
-// down 63 -> 55, weight gradients 375 -> 197, d_x equal, but d_h 97 -> 107: its epilogue moves six arrays in rows of a
-// tile, which this kernel stages through LDS).
+// SwiGLU backward of intermediate sizes that are a multiple of 128 but not of 256 (wide_dh says when).  The other
+// products of such widths run on the tiles of tile_gemm.h (24,000 rows of 24 experts, 640 x 896, us, these tiles ->
+// those: down 63 -> 55, weight gradients 375 -> 176, d_x 94 -> 92).
 #define PK_RM_ALT 128, 128, 64, 2, 2, 4
 
 // 256 output columns per unit (for the gate/up kernel 128 gate and 128 up columns).
@@ -2179,7 +2178,10 @@ bool wide_fills(int64_t A, int64_t N, int64_t E, int quarters) {
   return (A / 128 + (A < E ? A : E) / 2) * pk_ceil_div(N, 256) * 4 > quarters * (int64_t)mf::persistent_grid();
 }
 bool wide_gate_up(int64_t A, int64_t I, int64_t E) { return wide_fills(A, 2 * I, E, 5); }
-bool wide_dh(int64_t A, int64_t I, int64_t E) { return wide_fills(A, I, E, 4); }
+// At widths that are not multiples of 256 the persistent kernel has 128 x 128 units, and only a long reduction makes up for
+// them (us, those units -> tiles: 384 x 640, 64 experts, 1,536 rows 267 -> 239; 512 x 128, 8 experts, 6,000 rows 47 -> 33;
+// 1024 x 384, 128 experts, 156 rows 82 -> 75; 1024 x 640, 16 experts, 1,024 rows 80 -> 82; 2048 x 896, 32 experts, 375 rows 107 -> 125).
+bool wide_dh(int64_t A, int64_t H, int64_t I, int64_t E) { return (I % 256 == 0 || H > 1024) && wide_fills(A, I, E, 4); }
 // With few rows an expert the last 128-row unit of an expert is mostly padding as often as not, and 64-row tiles
 // are the faster ones at several units per CU: up to 512 rows with a short reduction (512 rows, 1024 x 512,
 // 32 experts: 53 -> 49; 256 rows, 512 x 256, 128 experts: 46 -> 36; 1,024 rows: 70 -> 77), up to 64 with any
@@ -2406,7 +2408,7 @@ int pk_grouped_swiglu_dgrad_dh(const void* d_y, const void* w2, const void* g, c
   if (!d_y || !w2 || !g || !u || !starts || !d_g || !d_u) return PK_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_y, w2, g, u, d_g, d_u});
-  if (!(mfma && wide_dh(A, I, E)) && tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u}))
+  if (!(mfma && wide_dh(A, H, I, E)) && tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u}))
     return dtype == PK_F32 ? dh_tile<float>(d_y, nullptr, 1, nullptr, w2, g, u, starts, d_g, d_u, nullptr, nullptr, nullptr, A, H, I, E, s)
                            : dh_tile<bf16_t>(d_y, nullptr, 1, nullptr, w2, g, u, starts, d_g, d_u, nullptr, nullptr, nullptr, A, H, I, E, s);
   if (!mfma) {
@@ -2476,7 +2478,7 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
   }
   hipStream_t s = (hipStream_t)stream;
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_out, w2, g, u, d_g, d_u, hs});
-  if (n_partial && !(mfma && wide_dh(A, I, E)) && tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs})) {
+  if (n_partial && !(mfma && wide_dh(A, H, I, E)) && tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs})) {
     if (!workspace || workspace_bytes < pk_region_dgrad_dh_workspace_bytes(A, I)) return PK_ERR_WORKSPACE;
     int part_cols = 0;
     rc = dtype == PK_F32 ? dh_tile<float>(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, hs, (float*)workspace, &part_cols,
