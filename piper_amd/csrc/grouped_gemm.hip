@@ -2171,9 +2171,9 @@ int launch_rm(mf::RaggedMParams& p, int64_t A, int64_t N, int kernel_id, hipStre
 // has one unit and its whole reduction to itself and the tiles of tile_gemm.h, four to eight times as
 // many and with a split reduction, are done first.  Forward and backward of a region, all its grouped products,
 // us, these kernels -> those (rows an expert, widths, experts; units of d_h against 256 CUs):
-//     32 rows, 1024 x 512, 32 experts ( 48 units)  161 ->  94      128 rows (96 units)   204 -> 147
-//    256 rows                         (160 units)  256 -> 223      512 rows (288 units)  both at 353
-//   1024 rows, 1024 x 512,  8 experts (136 units)  315 -> 218     2048 rows, 2048 x 1024, 4 experts (264 units): d_h 86 -> 107
+//     32 rows, 1024 x 512, 32 experts ( 48 units)  161 ->  91      128 rows (96 units)   204 -> 143
+//    256 rows                         (160 units)  256 -> 208      512 rows (288 units)  both at 353
+//   1024 rows, 1024 x 512,  8 experts (136 units)  315 -> 203     2048 rows, 2048 x 1024, 4 experts (264 units): d_h 86 -> 107
 bool wide_fills(int64_t A, int64_t N, int64_t E, int quarters) {
   return (A / 128 + (A < E ? A : E) / 2) * pk_ceil_div(N, 256) * 4 > quarters * (int64_t)mf::persistent_grid();
 }
@@ -2681,8 +2681,8 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   hipStream_t s = (hipStream_t)stream;
   // wgrad_kernel's 256 x 256 tiles where they give at least half of the CUs work and every XCD an expert; otherwise
   // the 64- or 128-wide tiles of tile_gemm.h (us, 256 x 256 or, at widths that are not multiples of 256, its former
-  // 128 x 128 tiles -> those: 4 experts 2048 x 1024, 2,048 rows 260 -> 219; 24 experts 640 x 896, 1,000 rows 379 -> 196;
-  // 64 experts 384 x 640, 1,536 rows 614 -> 338; but 8 experts 1024 x 512, 1,024 rows, 192 tiles 50 against 79)
+  // 128 x 128 tiles -> those: 4 experts 2048 x 1024, 2,048 rows 260 -> 219; 24 experts 640 x 896, 1,000 rows 379 -> 176;
+  // 64 experts 384 x 640, 1,536 rows 614 -> 287; but 8 experts 1024 x 512, 1,024 rows, 192 tiles 50 against 79)
   const int n_weights = (d_w1 ? 1 : 0) + (d_w2 ? 1 : 0) + (d_w3 ? 1 : 0);
   const bool mfma = dtype == PK_BF16 && H % 256 == 0 && I % 256 == 0 && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}) &&
                     E >= mf::NXCD && E * (H / 256) * (I / 256) * n_weights >= mf::persistent_grid() / 2;
