@@ -124,10 +124,22 @@ void push_deferred(std::function<void()> fn) {
   py::gil_scoped_acquire gil;
   py::handle(g_queue).attr("push")(py::cpp_function(std::move(fn)));
 }
-bool leaf(const Tensor& p) { return p.is_leaf() && p.requires_grad(); }
+bool leaf(const Tensor& p) { return p.defined() && p.is_leaf() && p.requires_grad(); }
+// The parameters of a node, kept beside its saved variables: those that are leaves, undefined in the other
+// places.  What get_saved_variables() returns is for reading values only -- under saved-tensor hooks
+// (checkpointing, offload) it is a new leaf without a .grad -- while postponed and accumulated weight
+// gradients belong to the tensors that the caller handed in.
+void keep_parameters(AutogradContext* ctx, std::initializer_list<const Tensor*> ps) {
+  std::vector<Tensor> kept;
+  kept.reserve(ps.size());
+  for (const Tensor* p : ps) kept.push_back(leaf(*p) ? *p : Tensor());
+  ctx->saved_data["parameters"] = std::move(kept);
+}
+variable_list parameters_of(AutogradContext* ctx) { return ctx->saved_data["parameters"].toTensorVector(); }
+
 // A leaf whose existing .grad the kernels can add to directly.
 bool accumulates_in_place(const Tensor& p) {
-  if (!p.defined() || !leaf(p)) return false;
+  if (!leaf(p)) return false;
   const Tensor& g = p.grad();
   return g.defined() && g.scalar_type() == p.scalar_type() && g.sizes() == p.sizes() && g.is_contiguous() && g.device() == p.device();
 }
@@ -367,6 +379,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     Tensor out = region_forward(s, route, sv, true, true, xc, contig(w_gate), contig(bias), contig(w1), contig(w2), contig(w3),
                                 norm ? xc : contig(residual), contig(norm_w));
     ctx->save_for_backward({x, w_gate, bias, w1, w2, w3, norm_w, sv.mem.memory()});
+    keep_parameters(ctx, {&w_gate, &bias, &w1, &w2, &w3});
     ctx->saved_data["k"] = top_k;
     ctx->saved_data["norm"] = route_norm;
     ctx->saved_data["scale"] = route_scale;
@@ -377,20 +390,20 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &p_gate = saved[1], &p_bias = saved[2], &p1 = saved[3], &p2 = saved[4], &p3 = saved[5], &norm_w = saved[6];
+    const Tensor &x = saved[0], &bias = saved[2], &norm_w = saved[6];
     const bool norm = norm_w.defined();
-    const Shape s = region_shape(x, p_gate, p_bias, p1, p2, p3, ctx->saved_data["k"].toInt(), ctx->saved_data["norm"].toBool(),
+    const Shape s = region_shape(x, saved[1], bias, saved[3], saved[4], saved[5], ctx->saved_data["k"].toInt(), ctx->saved_data["norm"].toBool(),
                                  ctx->saved_data["scale"].toDouble(), ctx->saved_data["eps"].toDouble(), Tensor(), norm_w);
     Saved sv(s, true, norm);
     sv.mem.adopt(saved[7]);
     const Block& m = sv.mem;
     bool need[N_TENSORS];
-    const bool present[N_TENSORS] = {true, true, p_bias.defined(), true, true, true, ctx->saved_data["residual"].toBool(), norm};
+    const bool present[N_TENSORS] = {true, true, bias.defined(), true, true, true, ctx->saved_data["residual"].toBool(), norm};
     for (int i = 0, edge = 0; i < N_TENSORS; ++i) need[i] = present[i] && ctx->needs_input_grad(edge++);
     const bool need_xn = need[X] || (norm && need[NORM_W]);      // the gradient of what the router and the experts read
     const Tensor d_out = contig(grads[0]);
-    const Tensor xc = contig(x), w1 = contig(p1), w2 = contig(p2), w3 = contig(p3);
-    Tensor w_gate = contig(p_gate);
+    const Tensor xc = contig(x), w1 = contig(saved[3]), w2 = contig(saved[4]), w3 = contig(saved[5]);
+    Tensor w_gate = contig(saved[1]);
     if (!aligned16(w_gate)) w_gate = w_gate.clone();
     const void* x_rows = norm ? m.at_(sv.xn) : xc.data_ptr();
     const int32_t *perm = m.i32(sv.perm), *starts = m.i32(sv.starts);
@@ -451,10 +464,13 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
               ptr(ws), ws.defined() ? ws.numel() : 0, st);
       if (!need[X]) d_x = Tensor();
     };
+    // what the gradients are put into where this node does it itself (undefined: not a leaf)
+    const variable_list params = parameters_of(ctx);
+    const Tensor &p_gate = params[0], &p_bias = params[1], &p1 = params[2], &p2 = params[3], &p3 = params[4];
     Tensor d_w1, d_w2, d_w3, d_wg, d_b;
     const Tensor d_res = !norm && need[RESIDUAL] ? d_out : Tensor();
 
-    if (g_deferring.load() && all_w && need[W_GATE] && leaf(p_gate) && (!p_bias.defined() || leaf(p_bias)) && leaf(p1) && leaf(p2) && leaf(p3)) {
+    if (g_deferring.load() && all_w && need[W_GATE] && leaf(p_gate) && (!bias.defined() || leaf(p_bias)) && leaf(p1) && leaf(p2) && leaf(p3)) {
       // backward-input pass: the weight gradients of the experts and of the router gate are queued with
       // the tensors they need and computed by the weight pass
       push_deferred([wgrad, p1, p2, p3] { weight_grads_into_params(p1, p2, p3, wgrad); });
@@ -469,7 +485,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     // weight-gradient kernels add to them in their epilogues and autograd gets nothing to add
     const bool acc = g_accumulate.load();
     const bool experts_in_place = acc && all_w && accumulates_in_place(p1) && accumulates_in_place(p2) && accumulates_in_place(p3);
-    const bool gate_in_place = acc && need[W_GATE] && accumulates_in_place(p_gate) && (!p_bias.defined() || (need[BIAS] && leaf(p_bias)));
+    const bool gate_in_place = acc && need[W_GATE] && accumulates_in_place(p_gate) && (!bias.defined() || (need[BIAS] && leaf(p_bias)));
     const bool overlap = any_w && g_overlap.load() && !experts_in_place;
     const auto cur = c10::hip::getCurrentHIPStream(x.get_device());
     if (experts_in_place) {
@@ -493,7 +509,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     input_grad();
     if (!gate_in_place) {
       if (need[W_GATE]) d_wg = at::empty({s.E, s.H}, w_gate.options());
-      if (p_bias.defined() && need[BIAS]) d_b = at::empty({s.E}, w_gate.options());
+      if (bias.defined() && need[BIAS]) d_b = at::empty({s.E}, w_gate.options());
     }
     router_and_input(d_wg, d_b);
     if (gate_in_place) router_weight_grads(p_gate, p_bias, t.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
@@ -723,12 +739,14 @@ struct ExpertsFn : public torch::autograd::Function<ExpertsFn> {
     Tensor starts = counts_to_starts(counts), guh;
     Tensor y = run(w1, w2, w3, x, starts, guh);
     ctx->save_for_backward({w1, w2, w3, x, starts, guh});
+    keep_parameters(ctx, {&w1, &w2, &w3});
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list sv = ctx->get_saved_variables();
-    const Tensor &p1 = sv[0], &p2 = sv[1], &p3 = sv[2], starts = sv[4], guh = sv[5];
-    const Tensor w1 = contig(p1), w2 = contig(p2), w3 = contig(p3), x = contig(sv[3]), d_y = contig(grads[0]);
+    const variable_list params = parameters_of(ctx);
+    const Tensor &p1 = params[0], &p2 = params[1], &p3 = params[2], starts = sv[4], guh = sv[5];
+    const Tensor w1 = contig(sv[0]), w2 = contig(sv[1]), w3 = contig(sv[2]), x = contig(sv[3]), d_y = contig(grads[0]);
     const int64_t E = w1.size(0), I = w1.size(1), H = w1.size(2), A = x.size(0);
     const int code = dtype_code(x);
     const pk_stream_t st = stream_of(x);

@@ -1,0 +1,84 @@
+"""The native host path of the operators where autograd, the split backward and the bucket path meet
+tensors and callers other than the ordinary ones: saved-tensor hooks, forward-mode tangents, strided
+gradients, what a postponed weight pass keeps alive, and inputs past one launch's grid."""
+
+import pytest
+import torch
+from torch.utils.checkpoint import checkpoint
+
+from piper_amd import functional as F_
+
+pytestmark = pytest.mark.gpu
+
+T, H, E, K, I = 96, 256, 8, 2, 128
+
+
+def _params(dev, dtype=torch.bfloat16, seed=0, hidden=H, experts=E, inter=I):
+    g = torch.Generator().manual_seed(seed)
+
+    def rnd(*shape, scale, dt=dtype):
+        return (torch.randn(*shape, generator=g) * scale).to(dt).to(dev).requires_grad_(True)
+
+    return dict(norm=(1 + 0.1 * torch.randn(hidden, generator=g)).to(dtype).to(dev).requires_grad_(True),
+                w_gate=rnd(experts, hidden, scale=0.05, dt=torch.float32), bias=rnd(experts, scale=0.1, dt=torch.float32),
+                w1=rnd(experts, inter, hidden, scale=0.05), w2=rnd(experts, hidden, inter, scale=0.05),
+                w3=rnd(experts, inter, hidden, scale=0.05))
+
+
+def _activations(dev, tokens, dtype=torch.bfloat16, seed=1, hidden=H):
+    g = torch.Generator().manual_seed(seed)
+    return tuple(torch.randn(tokens, hidden, generator=g).to(dtype).to(dev) for _ in range(2))
+
+
+def _region(x, p):
+    return F_.expert_region(x, p["w_gate"], p["bias"], p["w1"], p["w2"], p["w3"], top_k=K, route_norm=True)
+
+
+def _block(x, p):
+    return F_.moe_block(x, p["norm"], p["w_gate"], p["bias"], p["w1"], p["w2"], p["w3"], top_k=K, route_norm=True)
+
+
+def _experts(x, p):
+    n = x.shape[0]
+    counts = torch.full((p["w1"].shape[0],), n // p["w1"].shape[0], dtype=torch.int32, device=x.device)
+    return F_.bmm_experts(p["w1"], p["w2"], p["w3"], x, counts)
+
+
+FLOWS = {"region": (_region, ("w_gate", "bias", "w1", "w2", "w3")),
+         "block": (_block, ("norm", "w_gate", "bias", "w1", "w2", "w3")),
+         "experts": (_experts, ("w1", "w2", "w3"))}
+
+
+def _under(hooks, fn, x):
+    if hooks == "none":
+        return fn(x)
+    if hooks == "checkpoint":
+        return checkpoint(fn, x, use_reentrant=False)
+    ctx = torch.autograd.graph.save_on_cpu() if hooks == "save_on_cpu" else \
+        torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t)
+    with ctx:
+        return fn(x)
+
+
+@pytest.mark.parametrize("hooks", ["identity", "save_on_cpu", "checkpoint"])
+@pytest.mark.parametrize("flow", FLOWS)
+def test_postponed_weight_gradients_reach_the_parameters_under_saved_tensor_hooks(dev, flow, hooks):
+    """A hook's unpacked tensor is a copy: the gradients belong to the parameters themselves, and are
+    those of the same pass without hooks, bit for bit."""
+    print(f"[case] postponed weight gradients, {flow}, {hooks}", flush=True)
+    fn, names = FLOWS[flow]
+    x0, d = _activations(dev, T)
+
+    def run(how):
+        p = _params(dev)
+        x = x0.clone().requires_grad_(True)
+        out = _under(how, lambda t: fn(t, p), x)
+        with F_.defer_weight_grads() as queue:
+            out.backward(d)
+        queue.run()
+        return {"x": x.grad, **{n: p[n].grad for n in names}}
+
+    want, got = run("none"), run(hooks)
+    for n in want:
+        assert got[n] is not None, f"{n} has no gradient"
+        assert torch.equal(got[n], want[n]), n
