@@ -165,24 +165,20 @@ void gate_bwd(const float* d_logits, const void* x, int x_dtype, const Tensor& w
   PK_CALL(pk_gate_logits_bwd, d_logits, x, x_dtype, fptr(w_gate), d_x32, static_cast<float*>(ptr(d_w)),
           static_cast<float*>(ptr(d_b)), accumulate ? 1 : 0, T, H, E, ptr(ws), ws.defined() ? ws.numel() : 0, stream_of(w_gate));
 }
-// d_w_gate (and d_gate_bias) added to / stored as the parameters' .grad.  The two may be at different
-// points of their accumulation (one of them cleared); the kernel has one flag for both.
+// d_w_gate (and d_gate_bias) added to / stored as the parameters' .grad: inside the kernel, which writes
+// contiguous fp32 and has one flag for both, where every .grad is such a buffer; a gradient that is
+// strided, or missing for one of the two only, is added to (or set) here.
 void router_weight_grads(const Tensor& p_gate, const Tensor& p_bias, const float* d_logits, const void* x, int x_dtype, const Tensor& w_gate,
                          int64_t T, int64_t H, int64_t E) {
-  const bool have_w = p_gate.grad().defined(), have_b = p_bias.defined() && p_bias.grad().defined();
-  const auto f32 = w_gate.options();
-  if (!p_bias.defined() || have_w == have_b) {
-    Tensor gw = have_w ? p_gate.grad() : at::empty_like(p_gate);
-    Tensor gb = !p_bias.defined() ? Tensor() : have_b ? p_bias.grad() : at::empty({E}, f32);
-    gate_bwd(d_logits, x, x_dtype, w_gate, nullptr, gw, gb, have_w, T, H, E);
-    const_cast<Tensor&>(p_gate).mutable_grad() = gw;
-    if (p_bias.defined()) const_cast<Tensor&>(p_bias).mutable_grad() = gb;
+  if (accumulates_in_place(p_gate) && (!p_bias.defined() || accumulates_in_place(p_bias))) {
+    gate_bwd(d_logits, x, x_dtype, w_gate, nullptr, p_gate.grad(), p_bias.defined() ? p_bias.grad() : Tensor(), true, T, H, E);
     return;
   }
-  Tensor gw = at::empty_like(p_gate), gb = at::empty({E}, f32);
+  const auto f32 = w_gate.options();
+  Tensor gw = at::empty({E, H}, f32), gb = p_bias.defined() ? at::empty({E}, f32) : Tensor();
   gate_bwd(d_logits, x, x_dtype, w_gate, nullptr, gw, gb, false, T, H, E);
   add_or_set_grad(p_gate, gw);
-  add_or_set_grad(p_bias, gb);
+  if (gb.defined()) add_or_set_grad(p_bias, gb);
 }
 
 // ------------------------------------------------------------------------------ the fused region
@@ -304,10 +300,11 @@ struct RegionWgrad {
               accumulate, s.A, s.H, s.I, s.E, s.dtype, st);
   }
 };
-// `wgrad` into the three parameters' .grad: inside the kernels where all three exist
+// `wgrad` into the three parameters' .grad: inside the kernels where all three are buffers that they can
+// write (contiguous, of the parameter's type), added or set here otherwise
 template <typename F>
 void weight_grads_into_params(const Tensor& p1, const Tensor& p2, const Tensor& p3, const F& wgrad) {
-  if (p1.grad().defined() && p2.grad().defined() && p3.grad().defined()) {
+  if (accumulates_in_place(p1) && accumulates_in_place(p2) && accumulates_in_place(p3)) {
     wgrad(p1.grad(), p2.grad(), p3.grad(), true);
     return;
   }

@@ -6,6 +6,7 @@ import pytest
 import torch
 from torch.utils.checkpoint import checkpoint
 
+from conftest import rel_err
 from piper_amd import functional as F_
 
 pytestmark = pytest.mark.gpu
@@ -82,3 +83,83 @@ def test_postponed_weight_gradients_reach_the_parameters_under_saved_tensor_hook
     for n in want:
         assert got[n] is not None, f"{n} has no gradient"
         assert torch.equal(got[n], want[n]), n
+
+
+def test_gate_weight_that_is_a_transposed_view(dev):
+    """The postponed gate gradient of a non-contiguous gate weight has the weight's elements in their places."""
+    x, d = _activations(dev, T)
+
+    def run(postponed):
+        p = _params(dev)
+        p["w_gate"] = torch.nn.Parameter(p["w_gate"].detach().t().contiguous().t())
+        assert not p["w_gate"].is_contiguous()
+        out = _region(x, p)
+        if postponed:
+            with F_.defer_weight_grads() as queue:
+                out.backward(d)
+            queue.run()
+        else:
+            out.backward(d)
+        return p["w_gate"].grad
+
+    assert torch.equal(run(True), run(False))
+
+
+def _strided(values):
+    """`values` in a tensor whose last two dimensions (or whose only one) are not laid out contiguously."""
+    if values.dim() == 1:
+        t = torch.zeros(2 * values.numel(), dtype=values.dtype, device=values.device)[::2]
+    else:
+        t = torch.zeros(values.transpose(-1, -2).shape, dtype=values.dtype, device=values.device).transpose(-1, -2)
+    t.copy_(values)
+    assert not t.is_contiguous()
+    return t
+
+
+@pytest.mark.parametrize("mode", ["postponed", "accumulate"])
+@pytest.mark.parametrize("flow,strided", [("region", ("w1",)), ("region", ("w1", "w2", "w3")), ("region", ("w_gate",)), ("region", ("bias",)),
+                                          ("region", ("w_gate", "bias", "w2")), ("experts", ("w1",)), ("experts", ("w1", "w2", "w3"))],
+                         ids=lambda v: v if isinstance(v, str) else "-".join(v))
+def test_gradients_are_added_to_strided_grad_buffers(dev, flow, strided, mode):
+    """A `.grad` that is not contiguous receives the sum autograd would leave in it: the kernels, which
+    write contiguous tensors, are not pointed at it."""
+    fn, names = FLOWS[flow]
+    print(f"[case] strided .grad, {flow}, {mode}, {strided}", flush=True)
+    x, d = _activations(dev, T)
+    p0 = _params(dev)
+    fn(x, p0).backward(d)
+    fresh = {n: p0[n].grad for n in names}
+
+    p = _params(dev)
+    before = {n: torch.randn_like(p[n]) for n in names}
+    for n in names:
+        p[n].grad = _strided(before[n]) if n in strided else before[n].clone()
+    held = {n: p[n].grad for n in strided}
+    out = fn(x, p)
+    if mode == "postponed":
+        with F_.defer_weight_grads() as queue:
+            out.backward(d)
+        queue.run()
+    else:
+        with F_.accumulate_weight_grads():
+            out.backward(d)
+    for n in names:
+        want = before[n].float() + fresh[n].float()
+        # one rounding to the buffer's type, of the sum or of the gradient and then the sum
+        tol = 2.0 ** -7 if p[n].dtype == torch.bfloat16 else 1e-6
+        assert rel_err(p[n].grad, want) <= tol, (n, rel_err(p[n].grad, want))
+    for n in strided:
+        assert rel_err(held[n], p[n].grad) == 0.0 and held[n].stride() == _strided(before[n]).stride(), n
+
+
+def test_expanded_grad_is_refused(dev):
+    """Several elements of an expanded `.grad` share one place in memory: an error, and nothing written past it."""
+    x, d = _activations(dev, T)
+    p = _params(dev)
+    for n in ("w1", "w2", "w3"):
+        p[n].grad = torch.zeros(1, 1, 1, dtype=p[n].dtype, device=dev).expand_as(p[n])
+    out = _region(x, p)
+    with F_.defer_weight_grads() as queue:
+        out.backward(d)
+    with pytest.raises(RuntimeError):
+        queue.run()
