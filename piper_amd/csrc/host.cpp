@@ -79,6 +79,17 @@ bool plain(std::initializer_list<const Tensor*> ts) {
   }
   return true;
 }
+// The operators have a backward and no rule for other transforms: a tensor that carries a forward-mode
+// tangent (it would be dropped on the way, whether or not a backward is wanted) or that is a functorch
+// wrapper (it has no memory of its own) is refused.
+void refuse_transforms(std::initializer_list<const Tensor*> ts, const char* what) {
+  for (const Tensor* t : ts) {
+    if (!t->defined()) continue;
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(/*level=*/0).defined(), what, " has no forward-mode derivative");
+    TORCH_CHECK(!t->key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper})), what,
+                " does not support functorch transforms");
+  }
+}
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
   if (!at::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
@@ -527,6 +538,7 @@ std::optional<Tensor> expert_region(const Tensor& x, const Tensor& w_gate, const
   PyObject* const route = route_.ptr() == Py_None ? nullptr : route_.ptr();
   const Tensor bias = opt(bias_), residual = opt(residual_), norm_w = opt(norm_w_);
   if (direct && !plain({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w})) return std::nullopt;
+  refuse_transforms({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w}, "expert_region");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   if (wants_grad({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w}))
@@ -575,6 +587,7 @@ struct NormFn : public torch::autograd::Function<NormFn> {
 };
 std::optional<Tensor> rmsnorm(const Tensor& x, const Tensor& w, double eps, bool direct) {
   if (direct && !plain({&x, &w})) return std::nullopt;
+  refuse_transforms({&x, &w}, "rmsnorm");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   return wants_grad({&x, &w}) ? NormFn::apply(x, w, eps) : NormFn::run(x, w, eps, Tensor());
@@ -647,6 +660,8 @@ struct RouterFn : public torch::autograd::Function<RouterFn> {
 };
 std::pair<Tensor, Tensor> router(const Tensor& x, const Tensor& w_gate, const OptTensor& bias, int64_t top_k, bool route_norm, double route_scale,
                                  const py::object& route) {
+  const Tensor b = opt(bias);
+  refuse_transforms({&x, &w_gate, &b}, "router");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   auto r = RouterFn::apply(x, w_gate, bias, top_k, route_norm, route_scale, route.ptr() == Py_None ? nullptr : route.ptr());
@@ -672,6 +687,7 @@ struct PermuteFn : public torch::autograd::Function<PermuteFn> {
   }
 };
 Tensor permute(const Tensor& x, const Tensor& perm, const Tensor& inv, int64_t top_k) {
+  refuse_transforms({&x, &perm, &inv}, "permute");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   return PermuteFn::apply(x, perm, inv, top_k);
@@ -697,6 +713,7 @@ struct CombineFn : public torch::autograd::Function<CombineFn> {
   }
 };
 Tensor combine(const Tensor& y, const Tensor& perm, const Tensor& inv, const Tensor& scores) {
+  refuse_transforms({&y, &perm, &inv, &scores}, "combine");
   require_gpu(y);
   c10::hip::HIPGuard device(y.device().index());
   return CombineFn::apply(y, perm, inv, scores);
@@ -775,8 +792,9 @@ struct ExpertsFn : public torch::autograd::Function<ExpertsFn> {
   }
 };
 std::optional<Tensor> bmm_experts(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& counts, bool direct) {
-  require_gpu(x);
   if (direct && !plain({&w1, &w2, &w3, &x, &counts})) return std::nullopt;
+  refuse_transforms({&w1, &w2, &w3, &x, &counts}, "bmm_experts");
+  require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   if (wants_grad({&w1, &w2, &w3, &x})) return ExpertsFn::apply(w1, w2, w3, x, counts);
   Tensor guh;

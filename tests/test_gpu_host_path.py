@@ -4,6 +4,7 @@ gradients, what a postponed weight pass keeps alive, and inputs past one launch'
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 from torch.utils.checkpoint import checkpoint
 
 from conftest import rel_err
@@ -163,3 +164,48 @@ def test_expanded_grad_is_refused(dev):
         out.backward(d)
     with pytest.raises(RuntimeError):
         queue.run()
+
+
+def test_forward_mode_tangents_are_refused(dev):
+    """None of the operators has a forward-mode rule: a dual tensor raises, also where no gradient is asked
+    for, and its tangent is not dropped."""
+    p = {n: t.detach() for n, t in _params(dev).items()}
+    x, v = _activations(dev, T)
+    calls = {
+        "region": lambda t: _region(t, p),
+        "region operator": lambda t: torch.ops.piper_amd.expert_region(t, p["w_gate"], p["bias"], p["w1"], p["w2"], p["w3"], K, True, 1.0, None),
+        "block": lambda t: _block(t, p),
+        "rmsnorm": lambda t: F_.rmsnorm(t, p["norm"]),
+        "rmsnorm operator": lambda t: torch.ops.piper_amd.rmsnorm(t, p["norm"], 1e-6),
+        "experts": lambda t: _experts(t, p),
+        "router": lambda t: F_.router(t, p["w_gate"], p["bias"], top_k=K, route_norm=True),
+        "permute": lambda t: F_.permute(t, torch.arange(T, dtype=torch.int32, device=dev), 1),
+        "combine": lambda t: F_.combine(t, torch.arange(T, dtype=torch.int32, device=dev), torch.ones(T, 1, device=dev)),
+    }
+    for name, call in calls.items():
+        for grad_mode in (True, False):
+            print(f"[case] forward mode, {name}, grad mode {grad_mode}", flush=True)
+            call(x)
+            with fwAD.dual_level(), torch.set_grad_enabled(grad_mode):
+                with pytest.raises(NotImplementedError):
+                    call(fwAD.make_dual(x, v))
+    # a tangent of a weight counts as much as one of the input
+    with fwAD.dual_level(), pytest.raises(NotImplementedError):
+        _region(x, dict(p, w2=fwAD.make_dual(p["w2"], torch.ones_like(p["w2"]))))
+
+
+def test_functorch_transforms(dev):
+    """A transform's wrapper tensors have no memory: the kernels refuse them.  (vmap over the operators that
+    go through the dispatcher runs them slice by slice.)"""
+    p = {n: t.detach() for n, t in _params(dev).items()}
+    x, _ = _activations(dev, T)
+    perm, one = torch.arange(T, dtype=torch.int32, device=dev), torch.ones(T, 1, device=dev)
+    for name, call in {"region": lambda t: _region(t, p), "rmsnorm": lambda t: F_.rmsnorm(t, p["norm"]), "experts": lambda t: _experts(t, p),
+                       "permute": lambda t: F_.permute(t, perm, 1), "combine": lambda t: F_.combine(t, perm, one)}.items():
+        print(f"[case] functorch grad, {name}", flush=True)
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda t: call(t).float().sum())(x)
+    xs = torch.stack([x, 2 * x])
+    assert torch.equal(torch.func.vmap(lambda t: F_.rmsnorm(t, p["norm"]))(xs), torch.stack([F_.rmsnorm(t, p["norm"]) for t in xs]))
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda t: F_.permute(t, perm, 1))(xs)
