@@ -153,21 +153,35 @@ class MoEFeedForwardBlock(nn.Module):
         self.moe = AnnotatedMoE(moe_args, dim, hidden_dim, dtype=dtype, fused=True)
 
     def _one_node(self) -> bool:
-        """Whether nobody can tell the submodules' own calls from one fused call: no hooks on them, no
-        replaced or subclassed parts."""
-        norm, moe = self.ffn_norm, self.moe
-        return (type(norm) is RMSNorm and type(moe) is AnnotatedMoE and moe.fused and not torch.compiler.is_compiling()
-                and not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                            for m in (norm, moe)))
+        """Whether nobody can tell the submodules' own calls from one fused call: both are called as this
+        module defines them (_called_as_defined) and so are the two operators they consist of."""
+        return (self.moe.fused and not torch.compiler.is_compiling() and _called_as_defined(self.ffn_norm, RMSNorm)
+                and _called_as_defined(self.moe, AnnotatedMoE) and (F_.rmsnorm, F_.expert_region) == _OPERATORS)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self._one_node():
             return self.moe(self.ffn_norm(x), residual=x)
+        bs, slen, dim = x.shape
         norm, moe = self.ffn_norm, self.moe
         router, experts = moe.router, moe.experts
-        shape = x.shape
         with annotate(EP_TAG):
-            out = F_.moe_block(x.reshape(-1, shape[-1]), norm.weight, router.gate.weight, router.gate.bias, experts.w1, experts.w2,
+            out = F_.moe_block(x.reshape(-1, dim), norm.weight, router.gate.weight, router.gate.bias, experts.w1, experts.w2,
                                experts.w3, top_k=router.top_k, route_norm=router.route_norm, route_scale=router.route_scale,
                                norm_eps=norm.eps)
-        return out.reshape(shape)
+        return out.reshape(bs, slen, dim)
+
+
+# What a call of the two submodules runs unless somebody has put something else in its place: hooks on the
+# instance or on all modules, a `forward` (or `_call_impl`) of its own on the instance, a patched class, a
+# patched nn.Module call (tracers, profilers), `module.compile()`, a subclass.
+_DEFINED = {cls: (cls.forward, nn.Module.__call__, nn.Module._call_impl) for cls in (RMSNorm, AnnotatedMoE)}
+_OPERATORS = (F_.rmsnorm, F_.expert_region)
+_GLOBAL_HOOKS = tuple(getattr(nn.modules.module, n) for n in ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
+                                                               "_global_backward_pre_hooks"))
+
+
+def _called_as_defined(m: nn.Module, cls: type) -> bool:
+    own = m.__dict__
+    return (type(m) is cls and (cls.forward, cls.__call__, cls._call_impl) == _DEFINED[cls] and "forward" not in own and "_call_impl" not in own
+            and m._compiled_call_impl is None
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or any(_GLOBAL_HOOKS)))
