@@ -110,6 +110,15 @@ class Block {
     mem_ = at::empty({(int64_t)(size_ ? size_ : 256)}, like.options().dtype(at::kByte));
     base_ = static_cast<char*>(mem_.data_ptr());
   }
+  // this block and another one in a single allocation: where both live equally long
+  void allocate_with(Block& other, const Tensor& like) {
+    const size_t mine = size_;
+    size_ += other.size_;
+    allocate(like);
+    size_ = mine;
+    other.mem_ = mem_;
+    other.base_ = base_ + mine;
+  }
   void adopt(Tensor mem) {
     mem_ = std::move(mem);
     base_ = static_cast<char*>(mem_.data_ptr());
@@ -227,21 +236,23 @@ Shape region_shape(const Tensor& x, const Tensor& w_gate, const Tensor& bias, co
   return s;
 }
 
-// What a forward leaves for its backward, in one allocation.
+// What a forward leaves for its backward: `rows` is read by the weight gradients as well, which may be
+// postponed past the rest of the backward, `mem` by the input pass only.
 struct Saved {
-  Block mem;
-  size_t logits, scores, idx, starts, perm, inv, order, g, u, xn, rstd;
+  Block rows, mem;
+  size_t starts, perm, order, xn;                     // in rows
+  size_t logits, scores, idx, inv, rstd, g, u;        // in mem
   // grads: g and u are kept, and with a norm its output and 1/rms
   Saved(const Shape& s, bool grads, bool norm) {
     const int64_t es = s.es;
+    starts = rows.add((s.E + 1) * 4);
+    perm = rows.add(s.A * 4);
+    order = rows.add(s.E * 4);
+    xn = rows.add(norm ? s.T * s.H * es : 0);
     logits = mem.add(s.T * s.E * 4);
     scores = mem.add(s.A * 4);
     idx = mem.add(s.A * 4);
-    starts = mem.add((s.E + 1) * 4);
-    perm = mem.add(s.A * 4);
     inv = mem.add(s.A * 4);
-    order = mem.add(s.E * 4);
-    xn = mem.add(norm ? s.T * s.H * es : 0);
     rstd = mem.add(norm ? s.T * 4 : 0);
     g = mem.add(grads ? s.A * s.I * es : 0);
     u = mem.add(grads ? s.A * s.I * es : 0);
@@ -261,10 +272,16 @@ void route_in_python(PyObject* route, const Shape& s, const Saved& sv, const Ten
 }
 
 // out = [residual +] region([norm](x)); every input contiguous
-Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, bool keep_order, const Tensor& x, const Tensor& w_gate, const Tensor& bias, const Tensor& w1,
+// for_backward: what is in sv outlives the call
+Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, bool for_backward, const Tensor& x, const Tensor& w_gate, const Tensor& bias, const Tensor& w1,
                       const Tensor& w2, const Tensor& w3, const Tensor& residual, const Tensor& norm_w) {
   Tensor out = at::empty({s.T, s.H}, x.options());
-  sv.mem.allocate(x);
+  if (for_backward) {
+    sv.rows.allocate(x);
+    sv.mem.allocate(x);
+  } else {
+    sv.rows.allocate_with(sv.mem, x);
+  }
   Block tmp;
   const int64_t ws_bytes = pk_gate_route_sort_workspace_bytes(s.T, s.H, s.E, s.K);
   TORCH_CHECK(ws_bytes >= 0, "pk_gate_route_sort_workspace_bytes failed: ", pk_status_string((int)ws_bytes));
@@ -272,22 +289,23 @@ Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, 
   const size_t h = tmp.add(s.A * s.I * s.es), y = tmp.add(s.A * s.H * s.es);
   tmp.allocate(x);
   const pk_stream_t st = stream_of(x);
-  const Block& m = sv.mem;
-  int32_t* const order = keep_order ? m.i32(sv.order) : nullptr;      // only the weight gradient asks for it
+  const Block &m = sv.mem, &r = sv.rows;
+  int32_t *const starts = r.i32(sv.starts), *const perm = r.i32(sv.perm);
+  int32_t* const order = for_backward ? r.i32(sv.order) : nullptr;      // only the weight gradient asks for it
   const void* xin = x.data_ptr();
   if (norm_w.defined()) {
-    PK_CALL(pk_rmsnorm_fwd, xin, s.dtype, ptr(norm_w), (float)s.eps, m.at_(sv.xn), m.f32(sv.rstd), s.T, s.H, st);
-    xin = m.at_(sv.xn);
+    PK_CALL(pk_rmsnorm_fwd, xin, s.dtype, ptr(norm_w), (float)s.eps, r.at_(sv.xn), m.f32(sv.rstd), s.T, s.H, st);
+    xin = r.at_(sv.xn);
   }
   if (route) {
     PK_CALL(pk_gate_logits, xin, s.dtype, fptr(w_gate), fptr(bias), m.f32(sv.logits), s.T, s.H, s.E, tmp.at_(ws), ws_bytes, st);
     route_in_python(route, s, sv, x);
-    PK_CALL(pk_sort_by_expert, m.i32(sv.idx), s.A, s.E, nullptr, m.i32(sv.starts), m.i32(sv.perm), m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
+    PK_CALL(pk_sort_by_expert, m.i32(sv.idx), s.A, s.E, nullptr, starts, perm, m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
   } else {
     PK_CALL(pk_gate_route_sort, xin, s.dtype, fptr(w_gate), fptr(bias), s.T, s.H, s.E, s.K, s.route_norm, (float)s.route_scale, m.f32(sv.logits),
-            m.f32(sv.scores), m.i32(sv.idx), nullptr, m.i32(sv.starts), m.i32(sv.perm), m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
+            m.f32(sv.scores), m.i32(sv.idx), nullptr, starts, perm, m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
   }
-  PK_CALL(pk_grouped_swiglu_fwd, xin, m.i32(sv.perm), s.K, ptr(w1), ptr(w2), ptr(w3), m.i32(sv.starts), keep_gu ? m.at_(sv.g) : nullptr,
+  PK_CALL(pk_grouped_swiglu_fwd, xin, perm, s.K, ptr(w1), ptr(w2), ptr(w3), starts, keep_gu ? m.at_(sv.g) : nullptr,
           keep_gu ? m.at_(sv.u) : nullptr, tmp.at_(h), tmp.at_(y), s.A, s.H, s.I, s.E, s.dtype, st);
   PK_CALL(pk_combine_fwd, tmp.at_(y), s.dtype, m.i32(sv.inv), m.f32(sv.scores), ptr(residual), ptr(out), s.T, s.H, s.K, st);
   return out;
@@ -296,7 +314,7 @@ Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, 
 // Weight-gradient kernels of the fused region with everything they read.
 struct RegionWgrad {
   Shape s;
-  Tensor d_out, x, saved, tmp;            // owners of the memory below
+  Tensor d_out, x, rows, grads;           // owners of the memory below (x: undefined where the rows are a norm's output)
   const void *x_rows, *d_g, *d_u, *hs;    // row-major, or
   const void *d_gT, *d_uT, *hsT;          // the transposed copies
   int64_t ldt;
@@ -386,7 +404,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const Tensor xc = contig(x);
     Tensor out = region_forward(s, route, sv, true, true, xc, contig(w_gate), contig(bias), contig(w1), contig(w2), contig(w3),
                                 norm ? xc : contig(residual), contig(norm_w));
-    ctx->save_for_backward({x, w_gate, bias, w1, w2, w3, norm_w, sv.mem.memory()});
+    ctx->save_for_backward({x, w_gate, bias, w1, w2, w3, norm_w, sv.rows.memory(), sv.mem.memory()});
     keep_parameters(ctx, {&w_gate, &bias, &w1, &w2, &w3});
     ctx->saved_data["k"] = top_k;
     ctx->saved_data["norm"] = route_norm;
@@ -403,8 +421,9 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const Shape s = region_shape(x, saved[1], bias, saved[3], saved[4], saved[5], ctx->saved_data["k"].toInt(), ctx->saved_data["norm"].toBool(),
                                  ctx->saved_data["scale"].toDouble(), ctx->saved_data["eps"].toDouble(), Tensor(), norm_w);
     Saved sv(s, true, norm);
-    sv.mem.adopt(saved[7]);
-    const Block& m = sv.mem;
+    sv.rows.adopt(saved[7]);
+    sv.mem.adopt(saved[8]);
+    const Block &m = sv.mem, &r = sv.rows;
     bool need[N_TENSORS];
     const bool present[N_TENSORS] = {true, true, bias.defined(), true, true, true, ctx->saved_data["residual"].toBool(), norm};
     for (int i = 0, edge = 0; i < N_TENSORS; ++i) need[i] = present[i] && ctx->needs_input_grad(edge++);
@@ -413,43 +432,57 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const Tensor xc = contig(x), w1 = contig(saved[3]), w2 = contig(saved[4]), w3 = contig(saved[5]);
     Tensor w_gate = contig(saved[1]);
     if (!aligned16(w_gate)) w_gate = w_gate.clone();
-    const void* x_rows = norm ? m.at_(sv.xn) : xc.data_ptr();
-    const int32_t *perm = m.i32(sv.perm), *starts = m.i32(sv.starts);
+    const void* x_rows = norm ? r.at_(sv.xn) : xc.data_ptr();
+    const int32_t *perm = r.i32(sv.perm), *starts = r.i32(sv.starts);
+    // what the gradients are put into where this node does it itself (undefined: not a leaf)
+    const variable_list params = parameters_of(ctx);
+    const Tensor &p_gate = params[0], &p_bias = params[1], &p1 = params[2], &p2 = params[3], &p3 = params[4];
+    const bool any_w = need[W1] || need[W2] || need[W3], all_w = need[W1] && need[W2] && need[W3];
+    // backward-input pass: the weight gradients of the experts and of the router gate are queued with the
+    // tensors they need and computed by the weight pass
+    const bool postpone = g_deferring.load() && all_w && need[W_GATE] && leaf(p_gate) && (!bias.defined() || leaf(p_bias)) && leaf(p1) && leaf(p2) &&
+                          leaf(p3);
 
     // Shapes where the K-contiguous weight-gradient path pays get d_g, d_u and score*h transposed; with long
     // experts the d_x GEMM reads its A operand from the same blocks and the row-major pair is left out.
     const int64_t ldt = pk_region_transposed_pays(s.A, s.H, s.I, s.E, s.dtype) ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
     const bool blocks_only = ldt > 0 && pk_grouped_swiglu_dx_from_transposed_pays(s.A, s.H, s.I, s.E, s.dtype);
-    Block t;
+    // w: what the weight gradients read, t: the rest
+    Block w, t;
     const int64_t ai = s.A * s.I * s.es, ait = ldt * s.I * s.es;
     const int64_t ds_ws = std::max<int64_t>(pk_region_dgrad_dh_workspace_bytes(s.A, s.I), 4);
     int64_t n_part = (s.I + 63) / 64;      // rows of partial score gradients; 0: d_scores is written
-    const size_t d_g = t.add(blocks_only ? 0 : ai), d_u = t.add(blocks_only ? 0 : ai), hs = t.add(ldt > 0 ? 0 : ai);
-    const size_t d_gT = t.add(ait), d_uT = t.add(ait), hsT = t.add(ait);
-    const size_t d_scores = t.add(ldt > 0 ? 0 : s.A * 4), part = t.add(ds_ws), d_logits = t.add(s.T * s.E * 4);
+    Block& gu = ldt > 0 ? t : w;           // the row-major pair: beside transposed copies only the d_x GEMM reads it
+    const size_t d_g = gu.add(blocks_only ? 0 : ai), d_u = gu.add(blocks_only ? 0 : ai), hs = w.add(ldt > 0 ? 0 : ai);
+    const size_t d_gT = w.add(ait), d_uT = w.add(ait), hsT = w.add(ait), d_logits = w.add(s.T * s.E * 4);
+    const size_t d_scores = t.add(ldt > 0 ? 0 : s.A * 4), part = t.add(ds_ws);
     const size_t d_xs = t.add(need_xn ? s.A * s.H * s.es : 0);
     const int64_t router_ws_bytes = pk_region_router_bwd_workspace_bytes(s.T, s.H, s.E, s.dtype);
     const size_t router_ws = t.add(router_ws_bytes);
     const size_t d_xn = t.add(norm && need_xn ? s.T * s.H * s.es : 0);
-    t.allocate(x);
+    if (postpone) {
+      w.allocate(x);
+      t.allocate(x);
+    } else {
+      w.allocate_with(t, x);
+    }
     const pk_stream_t st = stream_of(x);
-    void *dg = blocks_only ? nullptr : t.at_(d_g), *du = blocks_only ? nullptr : t.at_(d_u);
+    void *dg = blocks_only ? nullptr : gu.at_(d_g), *du = blocks_only ? nullptr : gu.at_(d_u);
     // the combine backward is folded into the d_h GEMM: d_out rows are gathered per routed row, the score
     // is applied in the epilogue
     if (ldt > 0)
       PK_CALL(pk_grouped_swiglu_dgrad_dh_scaled_t, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
-              t.at_(d_gT), t.at_(d_uT), t.at_(hsT), ldt, nullptr, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
+              w.at_(d_gT), w.at_(d_uT), w.at_(hsT), ldt, nullptr, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
     else
       PK_CALL(pk_region_dgrad_dh, ptr(d_out), perm, s.K, m.f32(sv.scores), ptr(w2), m.at_(sv.g), m.at_(sv.u), starts, dg, du,
-              t.at_(hs), t.f32(d_scores), &n_part, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
+              w.at_(hs), t.f32(d_scores), &n_part, t.at_(part), ds_ws, s.A, s.H, s.I, s.E, s.dtype, st);
 
-    const RegionWgrad wgrad{s, d_out, xc, sv.mem.memory(), t.memory(), x_rows, dg, du, t.at_(hs), t.at_(d_gT), t.at_(d_uT), t.at_(hsT),
-                            ldt, perm, starts, m.i32(sv.order)};
-    const bool any_w = need[W1] || need[W2] || need[W3], all_w = need[W1] && need[W2] && need[W3];
+    const RegionWgrad wgrad{s, d_out, norm ? Tensor() : xc, r.memory(), w.memory(), x_rows, ldt > 0 ? nullptr : dg, ldt > 0 ? nullptr : du,
+                            w.at_(hs), w.at_(d_gT), w.at_(d_uT), w.at_(hsT), ldt, perm, starts, r.i32(sv.order)};
     const auto input_grad = [&] {
       if (!need_xn) return;
       if (blocks_only)
-        PK_CALL(pk_grouped_swiglu_dgrad_dx_t, t.at_(d_gT), t.at_(d_uT), ldt, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
+        PK_CALL(pk_grouped_swiglu_dgrad_dx_t, w.at_(d_gT), w.at_(d_uT), ldt, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
       else
         PK_CALL(pk_region_dgrad_dx, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
     };
@@ -460,7 +493,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       if (need_xn) d_x = at::empty({s.T, s.H}, x.options());
       PK_CALL(pk_region_router_bwd, m.f32(sv.logits), m.i32(sv.idx), n_part > 0 ? nullptr : t.f32(d_scores), t.f32(part), n_part, m.i32(sv.inv),
               s.route_norm, (float)s.route_scale, x_rows, s.dtype, fptr(w_gate), t.at_(d_xs), !need_xn ? nullptr : norm ? t.at_(d_xn) : ptr(d_x),
-              static_cast<float*>(ptr(d_wg)), static_cast<float*>(ptr(d_b)), 0, t.f32(d_logits), s.T, s.H, s.E, s.K, t.at_(router_ws),
+              static_cast<float*>(ptr(d_wg)), static_cast<float*>(ptr(d_b)), 0, w.f32(d_logits), s.T, s.H, s.E, s.K, t.at_(router_ws),
               router_ws_bytes, st);
       if (!norm || !need_xn) return;
       Tensor ws;
@@ -472,19 +505,14 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
               ptr(ws), ws.defined() ? ws.numel() : 0, st);
       if (!need[X]) d_x = Tensor();
     };
-    // what the gradients are put into where this node does it itself (undefined: not a leaf)
-    const variable_list params = parameters_of(ctx);
-    const Tensor &p_gate = params[0], &p_bias = params[1], &p1 = params[2], &p2 = params[3], &p3 = params[4];
     Tensor d_w1, d_w2, d_w3, d_wg, d_b;
     const Tensor d_res = !norm && need[RESIDUAL] ? d_out : Tensor();
 
-    if (g_deferring.load() && all_w && need[W_GATE] && leaf(p_gate) && (!bias.defined() || leaf(p_bias)) && leaf(p1) && leaf(p2) && leaf(p3)) {
-      // backward-input pass: the weight gradients of the experts and of the router gate are queued with
-      // the tensors they need and computed by the weight pass
+    if (postpone) {
       push_deferred([wgrad, p1, p2, p3] { weight_grads_into_params(p1, p2, p3, wgrad); });
       input_grad();
       router_and_input(Tensor(), Tensor());
-      push_deferred([s, p_gate, p_bias, w_gate, x_rows, dl = t.f32(d_logits), keep = std::array<Tensor, 3>{t.memory(), sv.mem.memory(), xc}] {
+      push_deferred([s, p_gate, p_bias, w_gate, x_rows, dl = w.f32(d_logits), keep = std::array<Tensor, 3>{wgrad.x, wgrad.rows, wgrad.grads}] {
         router_weight_grads(p_gate, p_bias, dl, x_rows, s.dtype, w_gate, s.T, s.H, s.E);
       });
       return {d_x, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), d_res, d_norm_w, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
@@ -520,11 +548,11 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       if (bias.defined() && need[BIAS]) d_b = at::empty({s.E}, w_gate.options());
     }
     router_and_input(d_wg, d_b);
-    if (gate_in_place) router_weight_grads(p_gate, p_bias, t.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
+    if (gate_in_place) router_weight_grads(p_gate, p_bias, w.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
     if (overlap) {
       const auto side = side_stream(x.get_device());
       wait_stream(cur.stream(), side.stream());
-      for (const Tensor* b : {&d_out, &xc, &sv.mem.memory(), &t.memory()}) b->record_stream(as_cuda(side));
+      for (const Tensor* b : {&d_out, &xc, &r.memory(), &w.memory()}) b->record_stream(as_cuda(side));
       for (const Tensor* b : {&d_w1, &d_w2, &d_w3}) b->record_stream(as_cuda(cur));
     }
     return {d_x, d_wg, d_b, d_w1, d_w2, d_w3, d_res, d_norm_w, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
@@ -732,48 +760,54 @@ struct ExpertsFn : public torch::autograd::Function<ExpertsFn> {
   static void zero_tail(const Tensor& buf, const Tensor& starts) {
     PK_CALL(pk_zero_rows_from, ptr(buf), dtype_code(buf), starts.data_ptr<int32_t>() + starts.numel() - 1, buf.size(0), buf.size(1), stream_of(buf));
   }
-  // y [A,H]; the pre-activations and h are left in one tensor [3,A,I]
-  static Tensor run(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& starts, Tensor& guh) {
+  // y [A,H]; the pre-activations are left in gu [2,A,I], and h [A,I], which the weight gradients read as well.
+  // Without a backward (gu and h null) they share one allocation.
+  static Tensor run(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& starts, Tensor* gu, Tensor* h) {
     TORCH_CHECK_VALUE(w1.dim() == 3 && w2.dim() == 3 && w3.dim() == 3, "expert weights must be [E,I,H], [E,H,I], [E,I,H]");
     const int64_t E = w1.size(0), I = w1.size(1), H = w1.size(2), A = x.size(0);
     TORCH_CHECK_VALUE(w3.sizes() == w1.sizes() && w2.size(0) == E && w2.size(1) == H && w2.size(2) == I, "expert weight shapes disagree");
     TORCH_CHECK_VALUE(w1.scalar_type() == x.scalar_type() && w2.scalar_type() == x.scalar_type() && w3.scalar_type() == x.scalar_type(),
                       "expert weights and activations must share a dtype");
-    guh = at::empty({3, A, I}, x.options());
+    const Tensor guh = at::empty({gu ? 2 : 3, A, I}, x.options());
     Tensor y = at::empty({A, H}, x.options());
     char* const g = static_cast<char*>(guh.data_ptr());
     const int64_t step = A * I * x.element_size();
+    void* hp = g + 2 * step;
+    if (gu) {
+      *gu = guh;
+      *h = at::empty({A, I}, x.options());
+      hp = h->data_ptr();
+    }
     PK_CALL(pk_grouped_swiglu_fwd, ptr(contig(x)), nullptr, 1, ptr(contig(w1)), ptr(contig(w2)), ptr(contig(w3)), starts.data_ptr<int32_t>(), g,
-            g + step, g + 2 * step, ptr(y), A, H, I, E, dtype_code(x), stream_of(x));
+            g + step, hp, ptr(y), A, H, I, E, dtype_code(x), stream_of(x));
     zero_tail(y, starts);
     return y;
   }
   static Tensor forward(AutogradContext* ctx, const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& counts) {
     require_gpu(x);
-    Tensor starts = counts_to_starts(counts), guh;
-    Tensor y = run(w1, w2, w3, x, starts, guh);
-    ctx->save_for_backward({w1, w2, w3, x, starts, guh});
+    Tensor starts = counts_to_starts(counts), gu, h;
+    Tensor y = run(w1, w2, w3, x, starts, &gu, &h);
+    ctx->save_for_backward({w1, w2, w3, x, starts, gu, h});
     keep_parameters(ctx, {&w1, &w2, &w3});
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list sv = ctx->get_saved_variables();
     const variable_list params = parameters_of(ctx);
-    const Tensor &p1 = params[0], &p2 = params[1], &p3 = params[2], starts = sv[4], guh = sv[5];
+    const Tensor &p1 = params[0], &p2 = params[1], &p3 = params[2], starts = sv[4], gu = sv[5], h = sv[6];
     const Tensor w1 = contig(sv[0]), w2 = contig(sv[1]), w3 = contig(sv[2]), x = contig(sv[3]), d_y = contig(grads[0]);
     const int64_t E = w1.size(0), I = w1.size(1), H = w1.size(2), A = x.size(0);
     const int code = dtype_code(x);
     const pk_stream_t st = stream_of(x);
     const int64_t step = A * I * x.element_size();
-    char* const g = static_cast<char*>(guh.data_ptr());
+    char* const g = static_cast<char*>(gu.data_ptr());
     Tensor dgu = at::empty({2, A, I}, x.options()), d_x = at::empty({A, H}, x.options());
     char* const dg = static_cast<char*>(dgu.data_ptr());
     PK_CALL(pk_grouped_swiglu_dgrad, ptr(d_y), ptr(w1), ptr(w2), ptr(w3), g, g + step, starts.data_ptr<int32_t>(), dg, dg + step, ptr(d_x), A, H, I, E, code, st);
     zero_tail(d_x, starts);
-    const auto wgrad = [=](const Tensor& d1, const Tensor& d2, const Tensor& d3, bool accumulate) {
-      char* const gs = static_cast<char*>(guh.data_ptr());
+    const auto wgrad = [d_y, h, dgu, x, starts, A, H, I, E, code, step](const Tensor& d1, const Tensor& d2, const Tensor& d3, bool accumulate) {
       char* const ds = static_cast<char*>(dgu.data_ptr());
-      PK_CALL(pk_grouped_swiglu_wgrad, ptr(d_y), gs + 2 * step, ds, ds + step, ptr(x), nullptr, 1, starts.data_ptr<int32_t>(), nullptr, ptr(d1),
+      PK_CALL(pk_grouped_swiglu_wgrad, ptr(d_y), ptr(h), ds, ds + step, ptr(x), nullptr, 1, starts.data_ptr<int32_t>(), nullptr, ptr(d1),
               ptr(d2), ptr(d3), accumulate, A, H, I, E, code, stream_of(x));
     };
     Tensor d1, d2, d3;
@@ -797,8 +831,7 @@ std::optional<Tensor> bmm_experts(const Tensor& w1, const Tensor& w2, const Tens
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   if (wants_grad({&w1, &w2, &w3, &x})) return ExpertsFn::apply(w1, w2, w3, x, counts);
-  Tensor guh;
-  return ExpertsFn::run(w1, w2, w3, x, ExpertsFn::counts_to_starts(counts), guh);
+  return ExpertsFn::run(w1, w2, w3, x, ExpertsFn::counts_to_starts(counts), nullptr, nullptr);
 }
 
 // ------------------------------------------------------------------------------ bucket path

@@ -1,6 +1,7 @@
 """The native host path of the operators where autograd, the split backward and the bucket path meet
 tensors and callers other than the ordinary ones: saved-tensor hooks, forward-mode tangents, strided
 gradients, what a postponed weight pass keeps alive, and inputs past one launch's grid."""
+import gc
 
 import pytest
 import torch
@@ -9,6 +10,7 @@ from torch.utils.checkpoint import checkpoint
 
 from conftest import rel_err
 from piper_amd import functional as F_
+from piper_amd import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -209,3 +211,46 @@ def test_functorch_transforms(dev):
     assert torch.equal(torch.func.vmap(lambda t: F_.rmsnorm(t, p["norm"]))(xs), torch.stack([F_.rmsnorm(t, p["norm"]) for t in xs]))
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda t: F_.permute(t, perm, 1))(xs)
+
+
+# (flow, tokens, hidden, experts, top_k, inter, row layout of the copies the weight gradient reads)
+HELD = [("region", 4096, 512, 16, 2, 256), ("block", 4096, 512, 16, 2, 256), ("experts", 8192, 512, 16, 1, 256),
+        ("region", 4096, 2048, 128, 8, 768), ("block", 4096, 2048, 128, 8, 768)]
+
+
+@pytest.mark.parametrize("flow,tokens,hidden,experts,top_k,inter", HELD, ids=lambda v: str(v))
+def test_a_postponed_weight_pass_keeps_only_what_it_reads(dev, flow, tokens, hidden, experts, top_k, inter):
+    """Between the input pass and the weight pass of a microbatch: d_g, d_u and (score *) h, the operands' row
+    tables, the gate's d_logits and, with a norm in front, its output; no routed-row gradients and no
+    pre-activations."""
+    print(f"[case] memory between the passes, {flow} {tokens} x {hidden}", flush=True)
+    p = _params(dev, hidden=hidden, experts=experts, inter=inter)
+    x, d = _activations(dev, tokens, hidden=hidden)
+    x.requires_grad_(True)
+    kw = dict(top_k=top_k, route_norm=True)
+
+    def forward():
+        if flow == "experts":
+            return _experts(x, p)
+        if flow == "block":
+            return F_.moe_block(x, p["norm"], p["w_gate"], p["bias"], p["w1"], p["w2"], p["w3"], **kw)
+        return F_.expert_region(x, p["w_gate"], p["bias"], p["w1"], p["w2"], p["w3"], **kw)
+
+    gc.collect()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = forward()
+    with F_.defer_weight_grads() as queue:
+        out.backward(d)
+    del out
+    x.grad = p["norm"].grad = None
+    held = torch.cuda.memory_allocated() - before
+    rows = tokens * top_k
+    padded = max(rows, ops.transposed_ld(rows, hidden, inter, experts, torch.bfloat16)) if flow != "experts" else rows
+    reads = 3 * padded * inter * 2
+    if flow != "experts":
+        reads += rows * 4 + (2 * experts + 1) * 4 + tokens * experts * 4 + (tokens * hidden * 2 if flow == "block" else 0)
+    # the caching allocator rounds a block up by as much as 1 MiB
+    assert held <= reads + 4 * 2 ** 20, (held, reads)
+    queue.run()
+    assert p["w1"].grad is not None
