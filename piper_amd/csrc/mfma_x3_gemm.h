@@ -351,8 +351,8 @@ inline int launch(const Params& p, int kernel_id, hipStream_t s) {
   return PK_OK;
 }
 
-// d_logits: p.A [T, E], w_gate: p.B [E, H] (p.M = T, p.N = H, p.K = E).  PK_ERR_ALIGN: the operands cannot
-// be read in 16-byte pieces; the caller takes the two kernels instead.
+// d_logits: p.A [T, E], w_gate: p.B [E, H] (p.M = T, p.N = H, p.K = E).  PK_ERR_ALIGN: a base is not 16-byte
+// aligned, which the caller's contract asks for (widths without whole pieces go to the two kernels).
 template <typename TG>
 inline int launch_gather(const Params& p, const GatherAdd& ga, int kernel_id, hipStream_t s) {
   // 32 tokens x 128 columns (16,384 tokens, the router backward as a whole: 212 us; 64 x 128: 214, 64 x 64: 222;
@@ -360,12 +360,22 @@ inline int launch_gather(const Params& p, const GatherAdd& ga, int kernel_id, hi
   constexpr int WM = 1, WN = 4;
   if (!usable<WM, WN, true, false, float, float>(p) || p.N % PkVec16<TG>::N != 0 || !pk_aligned16(ga.rows) || !pk_aligned16(ga.out))
     return PK_ERR_ALIGN;
-  dim3 grid((unsigned)pk_ceil_div(p.N, 32 * WN), (unsigned)pk_ceil_div(p.M, 32 * WM));
-  if (grid.y > 65535u) return PK_ERR_SHAPE;
   const bool stream_rows = p.M * ga.K * p.N * (int64_t)sizeof(TG) > (int64_t)192 * 1024 * 1024;
-  if (stream_rows) PK_LAUNCH_NOCHECK(kernel_id, s, (gather_kernel<WM, WN, TG, true>), grid, dim3(64 * WM * WN), 0, s, p, ga);
-  else PK_LAUNCH_NOCHECK(kernel_id, s, (gather_kernel<WM, WN, TG, false>), grid, dim3(64 * WM * WN), 0, s, p, ga);
-  PK_RETURN_IF_LAUNCH_FAILED();
+  // one launch per 65,535 row blocks, what grid.y holds: the GEMM with 64-row blocks in front of a separate
+  // gather takes twice that many tokens, and so does the forward
+  constexpr int64_t SLICE = (int64_t)65535 * 32 * WM;
+  for (int64_t t0 = 0; t0 < p.M; t0 += SLICE) {
+    Params q = p;
+    GatherAdd gq = ga;
+    q.M = p.M - t0 < SLICE ? p.M - t0 : SLICE;
+    q.A = static_cast<const float*>(p.A) + t0 * p.sam;
+    gq.inv_perm = ga.inv_perm + t0 * ga.K;
+    gq.out = static_cast<TG*>(ga.out) + t0 * p.N;
+    const dim3 grid((unsigned)pk_ceil_div(p.N, 32 * WN), (unsigned)pk_ceil_div(q.M, 32 * WM));
+    if (stream_rows) PK_LAUNCH_NOCHECK(kernel_id, s, (gather_kernel<WM, WN, TG, true>), grid, dim3(64 * WM * WN), 0, s, q, gq);
+    else PK_LAUNCH_NOCHECK(kernel_id, s, (gather_kernel<WM, WN, TG, false>), grid, dim3(64 * WM * WN), 0, s, q, gq);
+    PK_RETURN_IF_LAUNCH_FAILED();
+  }
   return PK_OK;
 }
 

@@ -8,7 +8,7 @@ import torch
 import torch.autograd.forward_ad as fwAD
 from torch.utils.checkpoint import checkpoint
 
-from conftest import rel_err
+from conftest import BF16_TOL, rel_err
 from piper_amd import functional as F_
 from piper_amd import ops
 
@@ -254,3 +254,23 @@ def test_a_postponed_weight_pass_keeps_only_what_it_reads(dev, flow, tokens, hid
     assert held <= reads + 4 * 2 ** 20, (held, reads)
     queue.run()
     assert p["w1"].grad is not None
+
+
+def test_backward_of_more_tokens_than_one_launch_has_row_blocks(dev):
+    """The gather of the input gradient has 32-token row blocks on a grid dimension of at most 65,535."""
+    tokens, hidden, experts, top_k, inter = 65535 * 32 + 77, 32, 4, 2, 32
+    print(f"[case] {tokens} tokens", flush=True)
+    p = _params(dev, hidden=hidden, experts=experts, inter=inter)
+    g = torch.Generator(device=dev).manual_seed(2)
+    x0, d = (torch.randn(tokens, hidden, generator=g, device=dev).bfloat16() for _ in range(2))
+
+    def run(rows):
+        x = x0[rows].clone().requires_grad_(True)
+        out = F_.expert_region(x, p["w_gate"], p["bias"], p["w1"], p["w2"], p["w3"], top_k=top_k, route_norm=True)
+        (dx,) = torch.autograd.grad(out, x, d[rows])
+        return dx
+
+    whole = run(slice(None))
+    # a token's input gradient does not depend on the tokens beside it
+    for rows in (slice(0, 4096), slice(65535 * 32 - 64, 65535 * 32), slice(65535 * 32, tokens), slice(65535 * 32 - 33, 65535 * 32 + 33)):
+        assert rel_err(whole[rows], run(rows)) <= BF16_TOL, rows
