@@ -425,12 +425,80 @@ __global__ __launch_bounds__(64 * kSmallSortWaves) void route_sort_small_kernel(
   sort_small(chosen, T * K, E, out, l);
 }
 
-// Longer inputs: after sort_hist_kernel one workgroup per chunk works out for itself where every expert
-// starts and how many of its rows come from earlier chunks -- all of them read all the chunk
-// histograms, a few tens of kB out of the L2, which is quicker than a launch of one workgroup in
-// between that everybody waits for (10 us at 64 chunks, 16 us at 256) -- and then places its chunk with
-// four waves.  Workgroup 0 also writes counts, starts and order.
+// Inputs of more chunks than self_scan_chunks: one workgroup turns the chunk histograms into first positions.
+// The 1024 threads form G = 1024 / cols groups of cols columns (E rounded up to a power of two); group g of
+// expert e walks chunks [g * cpg, (g + 1) * cpg) twice, eight values at a time (one round trip per eight
+// chunks): once for the group's sum, once to replace chunk_hist[c][e] by the first output position of
+// expert e's rows of chunk c.
+__global__ __launch_bounds__(1024) void sort_scan_kernel(int32_t* __restrict__ chunk_hist, int nchunks, int E, int32_t* __restrict__ counts,
+                                                         int32_t* __restrict__ starts, int32_t* __restrict__ order) {
+  __shared__ int32_t part[1024];       // [g][e]: rows of expert e in the chunks of group g
+  __shared__ int32_t cnt[PK_MAX_EXPERTS], first[PK_MAX_EXPERTS], wave_sums[16];
+  int cols = 1;
+  while (cols < E) cols <<= 1;
+  const int G = 1024 / cols;
+  const int e = threadIdx.x % cols, g = threadIdx.x / cols;
+  const int cpg = (nchunks + G - 1) / G;
+  const int c0 = g * cpg, c1 = min(nchunks, c0 + cpg);
+  constexpr int WALK = 8;
+  int mine = 0;
+  if (e < E)
+    for (int c = c0; c < c1; c += WALK) {
+      int v[WALK];
+#pragma unroll
+      for (int i = 0; i < WALK; ++i) v[i] = c + i < c1 ? chunk_hist[(int64_t)(c + i) * E + e] : 0;
+#pragma unroll
+      for (int i = 0; i < WALK; ++i) mine += v[i];
+    }
+  part[threadIdx.x] = mine;
+  __syncthreads();
+  int total = 0, before = 0;           // rows of expert e in all chunks / in the chunks of earlier groups
+  for (int k = 0; k < G; ++k) {
+    const int v = part[k * cols + e];
+    total += v;
+    before += k < g ? v : 0;
+  }
+  const int start = block_exclusive_scan(g == 0 ? total : 0, wave_sums);      // (columns past E hold zeros)
+  if (g == 0 && e < E) {
+    cnt[e] = total;
+    first[e] = start;
+    if (counts) counts[e] = total;
+    starts[e] = start;
+    if (e == E - 1) starts[E] = start + total;
+  }
+  __syncthreads();
+  if (e < E) {
+    int run = first[e] + before;
+    for (int c = c0; c < c1; c += WALK) {
+      int v[WALK];
+#pragma unroll
+      for (int i = 0; i < WALK; ++i) v[i] = c + i < c1 ? chunk_hist[(int64_t)(c + i) * E + e] : 0;
+#pragma unroll
+      for (int i = 0; i < WALK; ++i)
+        if (c + i < c1) {
+          chunk_hist[(int64_t)(c + i) * E + e] = run;
+          run += v[i];
+        }
+    }
+  }
+  __syncthreads();
+  if (order) write_order(cnt, first, E, order);
+}
+
+// After sort_hist_kernel one workgroup per chunk works out for itself where every expert starts and how
+// many of its rows come from earlier chunks -- all of them read all the chunk histograms, a few tens of kB
+// out of the L2, which is quicker than sort_scan_kernel in between that everybody waits for -- and then
+// places its chunk with four waves.  Workgroup 0 also writes counts, starts and order.  What is read grows
+// with the square of the chunks, so SCANNED leaves it to sort_scan_kernel beyond self_scan_chunks.
 constexpr int kScatterThreads = 1024, kScatterWaves = kSortChunk / 128;
+// Where the two ways meet.  The whole sort, us, without -> with the scan kernel:
+//   experts      513 chunks       1,024 chunks     2,048 chunks      8,192 chunks
+//        8      12.2 -> 16.4      15.6 -> 19.5     30.0 -> 25.7       191 -> 65
+//       32      15.5 -> 16.7      24.3 -> 21.5     59.5 -> 31.8       593 -> 96
+//      128      29.3 -> 26.0      57.8 -> 39.7      171 -> 68        2910 -> 236
+//    1,024       159 -> 171        410 -> 269      1537 -> 472
+inline int self_scan_chunks(int64_t E) { return E <= 16 ? 1024 : 512; }
+template <bool SCANNED>
 __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int32_t* __restrict__ idx, int A, int E,
                                                                        const int32_t* __restrict__ chunk_hist, int nchunks,
                                                                        int32_t* __restrict__ counts, int32_t* __restrict__ starts,
@@ -445,7 +513,7 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
   const int chunk = blockIdx.x;
   for (int i = threadIdx.x; i < (2 + kScatterWaves) * E; i += blockDim.x) lds[i] = 0;
   __syncthreads();
-  {
+  if constexpr (!SCANNED) {
     // 1024 threads = G groups of E columns; group g adds up chunks g, g + G, ..., eight loads at a time
     int cols = 1;
     while (cols < E) cols <<= 1;
@@ -480,17 +548,17 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
     }
   __syncthreads();
   const int e = threadIdx.x;
-  const int total = e < E ? cnt[e] : 0;
-  const int start = block_exclusive_scan(total, wave_sums);
+  const int total = !SCANNED && e < E ? cnt[e] : 0;
+  const int start = SCANNED ? 0 : block_exclusive_scan(total, wave_sums);
   if (e < E) {
-    int run = start + before[e];
+    int run = SCANNED ? chunk_hist[(int64_t)chunk * E + e] : start + before[e];
 #pragma unroll
     for (int w = 0; w < kScatterWaves; ++w) {
       const int n = cursor[w * E + e];
       cursor[w * E + e] = run;
       run += n;
     }
-    if (chunk == 0) {
+    if (!SCANNED && chunk == 0) {
       if (counts) counts[e] = total;
       starts[e] = start;
       if (e == E - 1) starts[E] = start + total;
@@ -498,7 +566,7 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
   }
   __syncthreads();
   if (wave < kScatterWaves) place_slots(idx, s0, 128, A, E, id_bits_for(E), cursor + wave * E, perm, inv_perm);
-  if (chunk == 0 && order) write_order(cnt, before, E, order);
+  if (!SCANNED && chunk == 0 && order) write_order(cnt, before, E, order);
 }
 
 __global__ __launch_bounds__(1024) void counts_to_starts_kernel(const void* __restrict__ counts,
@@ -1040,8 +1108,17 @@ int pk_sort_by_expert(const int32_t* top_idx, int64_t A, int64_t E, int32_t* cou
   PK_LAUNCH_NOCHECK(pk_timing::K_SORT_HIST, s, sort_hist_kernel, dim3(nchunks), dim3(64), (size_t)E * sizeof(int32_t), s, top_idx, (int)A, (int)E,
                      chunk_hist);
   PK_RETURN_IF_LAUNCH_FAILED();
-  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel, dim3(nchunks), dim3(kScatterThreads),
-                    (size_t)(2 + kScatterWaves) * E * sizeof(int32_t), s, top_idx, (int)A, (int)E, chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
+  const size_t lds = (size_t)(2 + kScatterWaves) * E * sizeof(int32_t);
+  if (nchunks <= self_scan_chunks(E)) {
+    PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel<false>, dim3(nchunks), dim3(kScatterThreads), lds, s, top_idx, (int)A, (int)E,
+                      chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
+    PK_RETURN_IF_LAUNCH_FAILED();
+    return PK_OK;
+  }
+  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCAN, s, sort_scan_kernel, dim3(1), dim3(1024), 0, s, chunk_hist, nchunks, (int)E, counts, starts, order);
+  PK_RETURN_IF_LAUNCH_FAILED();
+  PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel<true>, dim3(nchunks), dim3(kScatterThreads), lds, s, top_idx, (int)A, (int)E,
+                    chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }

@@ -203,6 +203,45 @@ def test_counting_sort_on_both_sides_of_its_dispatch(dev, A, E):
     assert torch.equal(order.cpu().long(), torch.argsort(-ref_counts, stable=True))
 
 
+@pytest.mark.parametrize("A,E", [(262144, 128), (262145, 17), (524288, 16), (524289, 5), (300001, 1000), (1 << 20, 32)])
+def test_counting_sort_of_many_chunks(dev, A, E):
+    """512 chunks of slots (1,024 with few experts), whose workgroups add up the chunk histograms themselves,
+    and more, where one workgroup does it for all: every table bit for bit, with an expert that gets nothing."""
+    print(f"[case] sort A={A} E={E}", flush=True)
+    g = torch.Generator().manual_seed(A + E)
+    ids = torch.randint(0, E, (A, 1), generator=g, dtype=torch.int32)
+    ids[ids == E // 2] = 0
+    counts, starts, perm, inv, order = ops.sort_by_expert(ids.to(dev), E, with_order=True)
+    flat = ids.reshape(-1).long()
+    want = torch.argsort(flat, stable=True)
+    ref_counts = torch.bincount(flat, minlength=E)
+    assert torch.equal(perm.cpu().long(), want)
+    assert torch.equal(inv.cpu().long()[want], torch.arange(A))
+    assert torch.equal(counts.cpu().long(), ref_counts)
+    assert torch.equal(starts.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), ref_counts.cumsum(0)]))
+    assert torch.equal(order.cpu().long(), torch.argsort(-ref_counts, stable=True))
+
+
+def test_sort_time_grows_with_the_slots(dev):
+    """Four times the slots take about four times as long (sixteen where every chunk reads all others)."""
+    def us(A, E=1024):
+        idx = torch.randint(0, E, (A, 1), device=dev, dtype=torch.int32)
+        ops.sort_by_expert(idx, E)
+        best = float("inf")
+        for _ in range(3):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ops.sort_by_expert(idx, E)
+            b.record()
+            b.synchronize()
+            best = min(best, 1e3 * a.elapsed_time(b))
+        return best
+
+    short, long = us(1 << 20), us(1 << 22)
+    print(f"[case] sort of 1 M and 4 M slots, 1,024 experts: {short:.0f} and {long:.0f} us", flush=True)
+    assert long <= 8 * short
+
+
 @pytest.mark.parametrize("T,H,E,K,bias", [(1, 256, 8, 2, True), (65, 2048, 128, 8, False), (70, 520, 130, 5, True), (5000, 2048, 128, 8, True)])
 def test_gate_and_topk_in_one_call_match_the_two_calls(dev, T, H, E, K, bias):
     """pk_gate_route sums the gate GEMM's split-K partial results inside the top-k kernel: logits,
