@@ -226,7 +226,17 @@ _NO_STREAM = contextlib.nullcontext()
 def on_stream(stream):
     """Context manager: `stream` is the current one inside (None: nothing changes), as
     `torch.cuda.stream(stream)` without the Python in it."""
-    return _NO_STREAM if stream is None else host().StreamScope(stream.stream_id, stream.device_index, stream.device_type)
+    return _NO_STREAM if stream is None else host().StreamScope(*stream_key(stream))
+
+
+def stream_key(stream):
+    """A torch stream as the native host path takes it (None: the caller's current stream)."""
+    return None if stream is None else (stream.stream_id, stream.device_index, stream.device_type)
+
+
+def wait_stream(waiter, other) -> None:
+    """`waiter.wait_stream(other)` without its Python; either may be a stream of any device."""
+    host().wait_stream(stream_key(waiter), stream_key(other))
 
 
 def require_gpu(t: torch.Tensor) -> None:

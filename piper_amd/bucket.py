@@ -19,7 +19,7 @@ import logging
 import torch
 
 from . import ops
-from ._lib import host, on_stream
+from ._lib import host, on_stream, stream_key
 from .optim import FusedAdamW
 
 BUCKET_ALIGN_BYTES = 256
@@ -115,11 +115,6 @@ def flatten_params(bucket: BucketState, params: Sequence[torch.nn.Parameter], *,
     bucket.full_params_fresh = True
     bucket.optimizer = None
     return bucket
-
-
-def _stream_key(stream):
-    """A torch stream as the native host path takes it (None: the caller's current stream)."""
-    return None if stream is None else (stream.stream_id, stream.device_index, stream.device_type)
 
 
 @dataclass
@@ -264,7 +259,7 @@ class ParamStorage:
                 bucket.flat_grads = torch.zeros(bucket.param_shard_info[1], dtype=self.grad_buffer_dtype,
                                                 device=bucket.flat_params.device)
                 bucket.reduce_scatter_grads = bucket.flat_grads
-            host().pack_param_grads(specs, bucket.flat_grads, _stream_key(stream))
+            host().pack_param_grads(specs, bucket.flat_grads, stream_key(stream))
 
     def hold_param_grads(self, ubid, stream: torch.cuda.Stream | None = None) -> None:
         """In place of the LAST accumulate_zero_param_grads_to_flat of an iteration: keep the
@@ -275,7 +270,7 @@ class ParamStorage:
         if ubid is None or ubid not in self.stages.zero_managed_ubids:
             return
         for bucket in self.stages.bucket(ubid).with_companions():
-            bucket.pending_grads = host().hold_param_grads(bucket.param_view_specs, _stream_key(stream))
+            bucket.pending_grads = host().hold_param_grads(bucket.param_view_specs, stream_key(stream))
 
     def alloc_full_params(self, ubid) -> None:
         """Unflatten (src/runtime.py:312-352): make every parameter a view of the flat bucket."""

@@ -62,6 +62,7 @@ pk_stream_t stream_of(const Tensor& t) {
   const int dev = t.get_device();
   const uint64_t bit = 1ull << (dev & 63);
   if (!(ready.load(std::memory_order_acquire) & bit)) {
+    c10::hip::HIPGuard device((c10::DeviceIndex)dev);      // it prepares the current one
     PK_CALL(pk_init);
     ready.fetch_or(bit, std::memory_order_release);
   }
@@ -356,16 +357,22 @@ c10::hip::HIPStream side_stream(int dev) {
 c10::Stream as_cuda(const c10::hip::HIPStream& s) {
   return c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::CUDA, s.device_index()), s.id());
 }
+// A stream as Python hands it over: (stream_id, device_index, device_type)
+typedef std::tuple<int64_t, int64_t, int64_t> StreamKey;
+c10::hip::HIPStream hip_stream(const StreamKey& k) {
+  return c10::hip::HIPStream(
+      c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::HIP, (c10::DeviceIndex)std::get<1>(k)), std::get<0>(k)));
+}
 // `with torch.cuda.stream(s)` without its Python (about ten calls on the way in and out): makes a stream,
 // and its device, the current one.
 class StreamScope {
  public:
-  StreamScope(int64_t id, int64_t device, int64_t) : stream_(c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::HIP, (c10::DeviceIndex)device), id)) {}
+  StreamScope(int64_t id, int64_t device, int64_t type) : stream_(hip_stream({id, device, type})) {}
   void enter() {
     device_ = c10::hip::current_device();
     if (device_ != stream_.device_index()) c10::hip::set_device(stream_.device_index());
     before_ = c10::hip::getCurrentHIPStream(stream_.device_index());
-    c10::hip::setCurrentHIPStream(c10::hip::HIPStream(stream_));
+    c10::hip::setCurrentHIPStream(stream_);
   }
   void exit() {
     c10::hip::setCurrentHIPStream(*before_);
@@ -373,16 +380,20 @@ class StreamScope {
   }
 
  private:
-  c10::Stream stream_;
+  c10::hip::HIPStream stream_;
   std::optional<c10::hip::HIPStream> before_;
   c10::DeviceIndex device_ = 0;
 };
 
-// `waiter` waits for everything queued on `other` so far
-void wait_stream(hipStream_t waiter, hipStream_t other) {
+// `waiter` waits for everything queued on `other` so far.  An event belongs to the device that is current
+// when it is created, and only a stream of that device can record it.
+void wait_stream(const c10::hip::HIPStream& waiter, const c10::hip::HIPStream& other) {
   hipEvent_t e;
+  c10::hip::HIPGuard device(other.device_index());
   TORCH_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
-  const bool fine = hipEventRecord(e, other) == hipSuccess && hipStreamWaitEvent(waiter, e, 0) == hipSuccess;
+  bool fine = hipEventRecord(e, other.stream()) == hipSuccess;
+  device.set_index(waiter.device_index());
+  fine = fine && hipStreamWaitEvent(waiter.stream(), e, 0) == hipSuccess;
   (void)hipEventDestroy(e);
   TORCH_CHECK(fine, "event between two streams failed");
 }
@@ -535,7 +546,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       };
       if (overlap) {
         const auto side = side_stream(x.get_device());
-        wait_stream(side.stream(), cur.stream());
+        wait_stream(side, cur);
         c10::hip::HIPStreamGuard guard(side);
         fresh();
       } else {
@@ -551,7 +562,7 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     if (gate_in_place) router_weight_grads(p_gate, p_bias, w.f32(d_logits), x_rows, s.dtype, w_gate, s.T, s.H, s.E);
     if (overlap) {
       const auto side = side_stream(x.get_device());
-      wait_stream(cur.stream(), side.stream());
+      wait_stream(cur, side);
       for (const Tensor* b : {&d_out, &xc, &r.memory(), &w.memory()}) b->record_stream(as_cuda(side));
       for (const Tensor* b : {&d_w1, &d_w2, &d_w3}) b->record_stream(as_cuda(cur));
     }
@@ -626,6 +637,7 @@ std::optional<Tensor> rmsnorm(const Tensor& x, const Tensor& w, double eps, bool
 std::vector<Tensor> sort_by_expert(const Tensor& top_idx, int64_t E) {
   require_gpu(top_idx);
   TORCH_CHECK_VALUE(top_idx.scalar_type() == at::kInt, "sort_by_expert: top_idx must be int32");
+  c10::hip::HIPGuard device(top_idx.device().index());
   const Tensor flat = contig(top_idx);
   const int64_t A = flat.numel(), ws_bytes = pk_sort_workspace_bytes(A, E);
   TORCH_CHECK(ws_bytes >= 0, "pk_sort_workspace_bytes failed: ", pk_status_string((int)ws_bytes));
@@ -848,7 +860,7 @@ Tensor spec_param(PyObject* spec) {
 }
 int64_t spec_int(PyObject* spec, int i) { return PyLong_AsLongLong(spec_item(spec, i)); }
 
-std::optional<c10::Stream> unpack_stream(const std::optional<std::tuple<int64_t, int64_t, int64_t>>& s) {
+std::optional<c10::Stream> unpack_stream(const std::optional<StreamKey>& s) {
   if (!s) return std::nullopt;
   return c10::Stream::unpack3(std::get<0>(*s), (c10::DeviceIndex)std::get<1>(*s), (c10::DeviceType)std::get<2>(*s));
 }
@@ -872,8 +884,9 @@ std::vector<Tensor> take_grads(const py::list& specs, const std::optional<c10::S
 }
 // flat[off : off + n] += grad.to(flat.dtype) for the bucket's gradients, one launch per gradient dtype;
 // the parameters end without gradients.
-void pack_param_grads(const py::list& specs, const Tensor& flat, const std::optional<std::tuple<int64_t, int64_t, int64_t>>& stream) {
+void pack_param_grads(const py::list& specs, const Tensor& flat, const std::optional<StreamKey>& stream) {
   require_gpu(flat);
+  c10::hip::HIPGuard device(flat.device().index());
   const std::vector<Tensor> grads = take_grads(specs, unpack_stream(stream));
   const size_t n = grads.size();
   std::vector<const void*> ptrs(n);
@@ -899,7 +912,7 @@ void pack_param_grads(const py::list& specs, const Tensor& flat, const std::opti
               dtype_code(flat), 1, stream_of(flat));
   }
 }
-std::vector<Tensor> hold_param_grads(const py::list& specs, const std::optional<std::tuple<int64_t, int64_t, int64_t>>& stream) {
+std::vector<Tensor> hold_param_grads(const py::list& specs, const std::optional<StreamKey>& stream) {
   return take_grads(specs, unpack_stream(stream));
 }
 void clear_param_grads(const py::list& specs) {
@@ -913,6 +926,7 @@ void adamw_packed(const Tensor& master, const Tensor& exp_avg, const Tensor& exp
                   const std::vector<int64_t>& offsets, const std::vector<int64_t>& numels, int64_t step, double lr, double beta1, double beta2,
                   double eps, double weight_decay, const Tensor& shadow, double grad_scale, bool zero_grad) {
   require_gpu(master);
+  c10::hip::HIPGuard device(master.device().index());
   const size_t n = grads.size();
   TORCH_CHECK_VALUE(offsets.size() == n && numels.size() == n, "adamw_fused_packed: one offset and element count per tensor");
   const int64_t total = master.numel();
@@ -971,8 +985,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def(py::init<int64_t, int64_t, int64_t>())
       .def("__enter__", &StreamScope::enter)
       .def("__exit__", [](StreamScope& s, const py::args&) { s.exit(); });
-  // everything queued on `other` (a hipStream_t) so far happens before what `waiter` gets from now on
-  m.def("wait_stream", [](uintptr_t waiter, uintptr_t other) { wait_stream(reinterpret_cast<hipStream_t>(waiter), reinterpret_cast<hipStream_t>(other)); }, nogil);
+  // everything queued on `other` so far happens before what `waiter` gets from now on
+  m.def("wait_stream", [](const StreamKey& waiter, const StreamKey& other) { wait_stream(hip_stream(waiter), hip_stream(other)); }, nogil);
   m.def("set_accumulate", [](bool on) { return g_accumulate.exchange(on); });
   m.def("set_overlap", [](bool on) { return g_overlap.exchange(on); });
   // the WeightGradQueue that backward passes hand their weight gradients to (None: they run them)

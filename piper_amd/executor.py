@@ -16,7 +16,7 @@ from typing import Any, Sequence
 import torch
 
 from . import functional as F_
-from ._lib import host, on_stream
+from ._lib import on_stream, wait_stream
 from .bucket import ParamStorage, StageStore
 from .planner import plan_zero_lifetimes
 from .tasks import COMM_TASKS, TaskType
@@ -152,9 +152,9 @@ class StageExecutor:
         ps = self.pack_stream or cs
         # the microbatches (and whatever else the caller queued) were produced on the caller's stream
         if cs != caller:
-            host().wait_stream(cs.cuda_stream, caller.cuda_stream)
+            wait_stream(cs, caller)
         if ps != caller and ps is not cs:
-            host().wait_stream(ps.cuda_stream, caller.cuda_stream)
+            wait_stream(ps, caller)
         self.params.drain_pending_frees()        # src/executors.py:584
         self._fwd.clear()
         self._inp_grads.clear()
@@ -164,7 +164,7 @@ class StageExecutor:
         self.params.clear_param_grads()
         self.params.zero_grad_buffers(ps)
         if ps is not cs:
-            host().wait_stream(cs.cuda_stream, ps.cuda_stream)
+            wait_stream(cs, ps)
         ubids = list(self.stages.buckets.keys())
         # which task gathers / frees a bucket's parameters and which one packs its gradients
         lifetimes = plan_zero_lifetimes(tasks)
@@ -261,7 +261,7 @@ class StageExecutor:
             self.params.hold_param_grads(ubid, cs)
             return
         if ps is not cs:
-            host().wait_stream(ps.cuda_stream, cs.cuda_stream)
+            wait_stream(ps, cs)
         self.params.accumulate_zero_param_grads_to_flat(ubid, ps)
         if ps is not cs:
             done = torch.cuda.Event()

@@ -11,6 +11,7 @@ from torch.utils.checkpoint import checkpoint
 from conftest import BF16_TOL, rel_err
 from piper_amd import functional as F_
 from piper_amd import ops
+from piper_amd._lib import host, on_stream, wait_stream
 
 pytestmark = pytest.mark.gpu
 
@@ -274,3 +275,37 @@ def test_backward_of_more_tokens_than_one_launch_has_row_blocks(dev):
     # a token's input gradient does not depend on the tokens beside it
     for rows in (slice(0, 4096), slice(65535 * 32 - 64, 65535 * 32), slice(65535 * 32, tokens), slice(65535 * 32 - 33, 65535 * 32 + 33)):
         assert rel_err(whole[rows], run(rows)) <= BF16_TOL, rows
+
+
+def test_streams_wait_for_each_other(dev):
+    """Events between side streams and the default stream, whose handle is null."""
+    a, b, main = torch.cuda.Stream(dev), torch.cuda.Stream(dev), torch.cuda.current_stream(dev)
+    src = torch.arange(1 << 24, device=dev, dtype=torch.float32)
+    wait_stream(a, main)
+    with on_stream(a):
+        mid = src + 1
+    wait_stream(b, a)
+    with on_stream(b):
+        out = mid * 2
+    wait_stream(main, b)
+    assert torch.equal(out, (src + 1) * 2)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two GPUs")
+def test_operators_and_streams_of_a_device_that_is_not_current(dev):
+    one = torch.device("cuda:1")
+    with torch.cuda.device(0):
+        a, b = torch.cuda.Stream(one), torch.cuda.default_stream(one)
+        wait_stream(a, b)
+        with on_stream(a):
+            idx = torch.randint(0, 16, (9000, 1), device=one, dtype=torch.int32)
+        wait_stream(b, a)
+        perm = ops.sort_by_expert(idx, 16)[2]
+        assert torch.equal(perm.long(), torch.argsort(idx.reshape(-1).long(), stable=True))
+        p = torch.nn.Parameter(torch.zeros(16, device=one))
+        p.grad = torch.ones_like(p)
+        flat = torch.zeros(16, device=one)
+        host().pack_param_grads([(p, 0, 16, (16,))], flat, None)
+        assert p.grad is None and torch.equal(flat, torch.ones_like(flat))
+        assert torch.cuda.current_device() == 0

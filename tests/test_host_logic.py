@@ -115,3 +115,15 @@ def test_annotate_is_traceable_by_dynamo_fullgraph():
     out = torch.compile(fn, fullgraph=True, backend="eager")(torch.ones(3))
     assert torch.equal(out, torch.full((3,), 4.0))
     assert current_annotations() == ()
+
+
+def test_waiting_streams_are_named_with_their_devices(monkeypatch):
+    """A raw stream handle does not say whose device it is (every device's default stream is 0): the native
+    wait gets id, device and type of both streams."""
+    from types import SimpleNamespace as NS
+
+    from piper_amd import _lib
+    seen = []
+    monkeypatch.setattr(_lib, "host", lambda: NS(wait_stream=lambda *keys: seen.append(keys)))
+    _lib.wait_stream(NS(stream_id=0, device_index=1, device_type=1, cuda_stream=0), NS(stream_id=35, device_index=0, device_type=1, cuda_stream=7))
+    assert seen == [((0, 1, 1), (35, 0, 1))]
