@@ -853,7 +853,7 @@ PyObject* spec_item(PyObject* spec, int i) {
   TORCH_CHECK_TYPE(PyTuple_Check(spec) && PyTuple_GET_SIZE(spec) > i, "param_view_specs: tuples (param, offset, numel, shape)");
   return PyTuple_GET_ITEM(spec, i);
 }
-Tensor spec_param(PyObject* spec) {
+const Tensor& spec_param(PyObject* spec) {
   PyObject* const p = spec_item(spec, 0);
   TORCH_CHECK_TYPE(THPVariable_Check(p), "param_view_specs: tuples (param, offset, numel, shape)");
   return THPVariable_Unpack(p);
@@ -865,60 +865,67 @@ std::optional<c10::Stream> unpack_stream(const std::optional<StreamKey>& s) {
   return c10::Stream::unpack3(std::get<0>(*s), (c10::DeviceIndex)std::get<1>(*s), (c10::DeviceType)std::get<2>(*s));
 }
 
-// Takes the gradients off the parameters (p.grad = None); undefined where there was none.  With a
-// stream the memory is marked as used on it.
-std::vector<Tensor> take_grads(const py::list& specs, const std::optional<c10::Stream>& stream) {
+// The gradients of a bucket's parameters (undefined where there is none), which still have them.
+struct ParamGrads {
+  std::vector<const Tensor*> params;      // (the list owns them)
   std::vector<Tensor> grads;
-  grads.reserve(specs.size());
-  for (const py::handle spec : specs) {
-    Tensor p = spec_param(spec.ptr());
-    Tensor g = p.grad();
-    if (g.defined()) {
-      if (g.requires_grad()) g = g.detach();
-      if (stream) g.record_stream(*stream);
-      p.mutable_grad().reset();
+  explicit ParamGrads(const py::list& specs) {
+    params.reserve(specs.size());
+    grads.reserve(specs.size());
+    for (const py::handle spec : specs) {
+      params.push_back(&spec_param(spec.ptr()));
+      const Tensor& g = params.back()->grad();
+      grads.push_back(g.defined() && g.requires_grad() ? g.detach() : g);
     }
-    grads.push_back(std::move(g));
   }
-  return grads;
-}
+  // p.grad = None.  With a stream the memory is marked as used on it.
+  void drop(const std::optional<c10::Stream>& stream) {
+    for (size_t i = 0; i < grads.size(); ++i) {
+      if (!grads[i].defined()) continue;
+      if (stream) grads[i].record_stream(*stream);
+      params[i]->mutable_grad().reset();
+    }
+  }
+};
 // flat[off : off + n] += grad.to(flat.dtype) for the bucket's gradients, one launch per gradient dtype;
-// the parameters end without gradients.
+// the parameters end without gradients.  Where one of them cannot be packed none is, and all are kept.
 void pack_param_grads(const py::list& specs, const Tensor& flat, const std::optional<StreamKey>& stream) {
   require_gpu(flat);
+  TORCH_CHECK_VALUE(flat.is_contiguous(), "bucket_pack: the flat bucket must be contiguous");
   c10::hip::HIPGuard device(flat.device().index());
-  const std::vector<Tensor> grads = take_grads(specs, unpack_stream(stream));
-  const size_t n = grads.size();
-  std::vector<const void*> ptrs(n);
-  std::vector<int64_t> offs(n), nums(n);
+  ParamGrads pg(specs);
+  struct Launch {
+    std::vector<const void*> ptrs;
+    std::vector<int64_t> offs, nums;
+  } launches[2];
   std::vector<Tensor> keep;
-  for (const at::ScalarType want : {at::kBFloat16, at::kFloat}) {
-    size_t m = 0;
-    for (size_t i = 0; i < n; ++i) {
-      if (!grads[i].defined()) continue;
-      dtype_code(grads[i]);
-      if (grads[i].scalar_type() != want) continue;
-      Tensor g = contig(grads[i]);
-      ptrs[m] = g.data_ptr();
-      if (!g.is_same(grads[i])) keep.push_back(g);
-      PyObject* const spec = PyList_GET_ITEM(specs.ptr(), i);
-      offs[m] = spec_int(spec, 1);
-      nums[m] = g.numel();
-      TORCH_CHECK_VALUE(offs[m] >= 0 && offs[m] + nums[m] <= flat.numel(), "bucket_pack: tensor outside the bucket");
-      ++m;
-    }
-    if (m)
-      PK_CALL(pk_bucket_pack, ptrs.data(), offs.data(), nums.data(), (int64_t)m, want == at::kBFloat16 ? PK_BF16 : PK_F32, flat.data_ptr(),
+  for (size_t i = 0; i < pg.grads.size(); ++i) {
+    if (!pg.grads[i].defined()) continue;
+    Launch& l = launches[dtype_code(pg.grads[i]) == PK_F32];
+    Tensor g = contig(pg.grads[i]);
+    const int64_t off = spec_int(PyList_GET_ITEM(specs.ptr(), i), 1);
+    TORCH_CHECK_VALUE(off >= 0 && off + g.numel() <= flat.numel(), "bucket_pack: tensor outside the bucket");
+    l.ptrs.push_back(g.data_ptr());
+    l.offs.push_back(off);
+    l.nums.push_back(g.numel());
+    if (!g.is_same(pg.grads[i])) keep.push_back(std::move(g));
+  }
+  for (int f32 = 0; f32 < 2; ++f32) {
+    const Launch& l = launches[f32];
+    if (!l.ptrs.empty())
+      PK_CALL(pk_bucket_pack, l.ptrs.data(), l.offs.data(), l.nums.data(), (int64_t)l.ptrs.size(), f32 ? PK_F32 : PK_BF16, flat.data_ptr(),
               dtype_code(flat), 1, stream_of(flat));
   }
+  pg.drop(unpack_stream(stream));
 }
 std::vector<Tensor> hold_param_grads(const py::list& specs, const std::optional<StreamKey>& stream) {
-  return take_grads(specs, unpack_stream(stream));
+  ParamGrads pg(specs);
+  pg.drop(unpack_stream(stream));
+  return std::move(pg.grads);
 }
 void clear_param_grads(const py::list& specs) {
   for (const py::handle spec : specs) {
-    Tensor p = spec_param(spec.ptr());
-    p.mutable_grad().reset();
+    spec_param(spec.ptr()).mutable_grad().reset();
   }
 }
 

@@ -277,6 +277,19 @@ def test_backward_of_more_tokens_than_one_launch_has_row_blocks(dev):
         assert rel_err(whole[rows], run(rows)) <= BF16_TOL, rows
 
 
+def test_gradients_survive_a_pack_that_is_refused(dev):
+    """Nothing is packed and no gradient is dropped where one of them cannot be packed."""
+    flat = torch.zeros(64, device=dev)
+    good = torch.nn.Parameter(torch.zeros(16, device=dev))
+    bad = torch.nn.Parameter(torch.zeros(16, device=dev, dtype=torch.float64))
+    for second, specs in ((bad, [(good, 0, 16, (16,)), (bad, 16, 16, (16,))]), (good, [(good, 60, 16, (16,))])):
+        good.grad, bad.grad = torch.ones_like(good), torch.ones_like(bad)
+        with pytest.raises((TypeError, ValueError)):
+            host().pack_param_grads(specs, flat, None)
+        assert all(s[0].grad is not None for s in specs)
+        assert float(flat.abs().max()) == 0.0
+
+
 def test_streams_wait_for_each_other(dev):
     """Events between side streams and the default stream, whose handle is null."""
     a, b, main = torch.cuda.Stream(dev), torch.cuda.Stream(dev), torch.cuda.current_stream(dev)
