@@ -69,11 +69,11 @@ pk_stream_t stream_of(const Tensor& t) {
   return reinterpret_cast<pk_stream_t>(c10::hip::getCurrentHIPStream(dev).stream());
 }
 
-// Ordinary tensors outside every tracing or dispatch mode: the kernels may be launched directly.
+// Ordinary tensors outside every tracing or dispatch mode: the kernels may be launched directly.  (In a
+// call that torch.jit.trace records only the dispatcher leaves a node behind.)
 bool plain(std::initializer_list<const Tensor*> ts) {
-  if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python) ||
-      c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
-    return false;
+  for (const c10::DispatchKey mode : {c10::DispatchKey::Python, c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::Tracer})
+    if (c10::impl::tls_is_dispatch_key_included(mode)) return false;
   for (const Tensor* t : ts) {
     if (!t->defined()) continue;
     if (!t->is_cuda() || t->key_set().has(c10::DispatchKey::Python)) return false;

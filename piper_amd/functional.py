@@ -14,6 +14,7 @@ Two ways in:
 from __future__ import annotations
 
 import torch
+from torch.overrides import has_torch_function_variadic
 
 from . import ops
 from ._lib import host
@@ -58,11 +59,16 @@ def _inverse_of(perm: torch.Tensor) -> torch.Tensor:
     return cached[1]
 
 
+def _router(x, w_gate, gate_bias, top_k, route_norm, route_scale):
+    return host().router(x, w_gate, gate_bias, top_k, route_norm, route_scale, _replaced_route())
+
+
 def router(x, w_gate, gate_bias=None, *, top_k: int, route_norm: bool, route_scale: float = 1.0):
     """(top_scores [T,K] f32, selected_experts_indices [T,K] i32, num_tokens_per_expert [E] i32).
     The call `self.router(x, self.expert_bias)` of qwen3.py:237-241.  The histogram is the one the
     counting sort produces (no host sync, no second pass over the indices)."""
-    top_scores, top_idx = host().router(x, w_gate, gate_bias, int(top_k), bool(route_norm), float(route_scale), _replaced_route())
+    call = torch.ops.piper_amd.router if torch.jit.is_tracing() else _router
+    top_scores, top_idx = call(x, w_gate, gate_bias, int(top_k), bool(route_norm), float(route_scale))
     counts = _sorted_tables(top_idx, w_gate.shape[0])[0]
     return top_scores, top_idx, counts
 
@@ -75,10 +81,14 @@ def reorder(top_scores: torch.Tensor, top_idx: torch.Tensor, num_experts: int):
     return scores_sorted, perm, counts
 
 
+def _permute(x, perm, top_k):
+    return host().permute(x, perm, _inverse_of(perm), top_k)
+
+
 def permute(x: torch.Tensor, token_indices_experts_sorted: torch.Tensor, top_k: int) -> torch.Tensor:
     """routed_input = x[token_indices_experts_sorted // top_k]  (qwen3.py:250)."""
-    perm = token_indices_experts_sorted
-    return host().permute(x, perm, _inverse_of(perm), int(top_k))
+    call = torch.ops.piper_amd.permute if torch.jit.is_tracing() else _permute
+    return call(x, token_indices_experts_sorted, int(top_k))
 
 
 def _traced_without_data(*tensors) -> bool:
@@ -141,20 +151,31 @@ def register_reference_op() -> bool:
     return True
 
 
+def _direct(*tensors) -> bool:
+    """Whether a call may go to the kernels without the operator in between (the native side looks at the
+    tensors themselves and at dispatch modes): nothing is being compiled, and no tensor subclass, FX proxy
+    or torch-function mode waits for the operator's name."""
+    return not torch.compiler.is_compiling() and not has_torch_function_variadic(*tensors)
+
+
 def bmm_experts(w1, w2, w3, x, num_tokens_per_expert):
     """Same call as the reference's ``bmm_experts`` (qwen3_bmm_experts_patch.py:78-87)."""
     register_reference_op()
-    if not torch.compiler.is_compiling():     # ordinary tensors: the operator's kernel without the dispatcher
+    if _direct(w1, w2, w3, x, num_tokens_per_expert):     # ordinary tensors: the operator's kernel without the dispatcher
         out = host().bmm_experts(w1, w2, w3, x, num_tokens_per_expert, True) if x.is_cuda else None
         if out is not None:
             return out
     return torch.ops.piper_artifact.bmm_experts(w1, w2, w3, x, num_tokens_per_expert)
 
 
+def _combine(y, perm, top_scores):
+    return host().combine(y, perm, _inverse_of(perm), top_scores)
+
+
 def combine(gathered_output, token_indices_experts_sorted, top_scores):
     """Unpermute scatter + fp32 weighted sum over k (qwen3.py:265-283), fused."""
-    perm = token_indices_experts_sorted
-    return host().combine(gathered_output, perm, _inverse_of(perm), top_scores)
+    call = torch.ops.piper_amd.combine if torch.jit.is_tracing() else _combine
+    return call(gathered_output, token_indices_experts_sorted, top_scores)
 
 
 # --------------------------------------------------------------------------- split backward
@@ -280,6 +301,13 @@ def register_region_ops() -> bool:
         # CPU tensors reach the kernels' own check and are refused there; fake CPU tensors get a shape
         lib.impl(name, fwd, "CPU")
         lib.impl(name, auto, "AutogradCPU")
+    # what torch.jit.trace records of the piecewise operators that otherwise go to the kernels directly
+    lib.define("router(Tensor x, Tensor w_gate, Tensor? gate_bias, int top_k, bool route_norm, float route_scale) -> (Tensor, Tensor)")
+    lib.define("permute(Tensor x, Tensor perm, int top_k) -> Tensor")
+    lib.define("combine(Tensor y, Tensor perm, Tensor top_scores) -> Tensor")
+    for name, fn in (("router", _router), ("permute", _permute), ("combine", _combine)):
+        for key in ("CUDA", "AutogradCUDA", "CPU", "AutogradCPU"):
+            lib.impl(name, fn, key)
     _REGION_LIBS.append(lib)
     return True
 
@@ -288,7 +316,7 @@ def expert_region(x, w_gate, gate_bias, w1, w2, w3, *, top_k: int, route_norm: b
                   residual=None):
     """The whole MoE expert region of AnnotatedMoE.forward (qwen3.py:233-289) on x [T,H].
     `residual` [T,H] is added to the result in the combine kernel."""
-    if not torch.compiler.is_compiling():     # ordinary tensors: the operator's kernel without the dispatcher
+    if _direct(x, w_gate, gate_bias, w1, w2, w3, residual):     # ordinary tensors: the operator's kernel without the dispatcher
         out = host().expert_region(x, w_gate, gate_bias, w1, w2, w3, int(top_k), bool(route_norm), float(route_scale),
                                    residual, None, 0.0, _replaced_route(), True)
         if out is not None:
@@ -300,7 +328,7 @@ def expert_region(x, w_gate, gate_bias, w1, w2, w3, *, top_k: int, route_norm: b
 def rmsnorm(x, weight, eps: float = 1e-6):
     """RMSNorm over the last dimension (the block's ffn_norm, qwen3.py:313-314)."""
     shape = x.shape
-    if not torch.compiler.is_compiling():
+    if _direct(x, weight):
         out = host().rmsnorm(x.reshape(-1, shape[-1]), weight, float(eps), True)
         if out is not None:
             return out.reshape(shape)
@@ -312,7 +340,7 @@ def moe_block(h, norm_weight, w_gate, gate_bias, w1, w2, w3, *, top_k: int, rout
     """h + moe(ffn_norm(h)) on h [T,H] (qwen3.py:313-314): RMSNorm kernel, expert region, residual
     added in the combine kernel.  One autograd node: its backward adds the residual branch's gradient
     inside the norm's backward kernel."""
-    if not torch.compiler.is_compiling():
+    if _direct(h, norm_weight, w_gate, gate_bias, w1, w2, w3):
         out = host().expert_region(h, w_gate, gate_bias, w1, w2, w3, int(top_k), bool(route_norm), float(route_scale), None,
                                    norm_weight, float(norm_eps), _replaced_route(), True)
         if out is not None:

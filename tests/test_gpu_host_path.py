@@ -1,17 +1,21 @@
 """The native host path of the operators where autograd, the split backward and the bucket path meet
 tensors and callers other than the ordinary ones: saved-tensor hooks, forward-mode tangents, strided
-gradients, what a postponed weight pass keeps alive, and inputs past one launch's grid."""
+gradients, what a postponed weight pass keeps alive, inputs past one launch's grid, and whoever looks for
+the operators by name (tracers, torch-function modes and subclasses, the profiler)."""
 import gc
+import warnings
 
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
+from torch.overrides import TorchFunctionMode
 from torch.utils.checkpoint import checkpoint
 
 from conftest import BF16_TOL, rel_err
 from piper_amd import functional as F_
 from piper_amd import ops
 from piper_amd._lib import host, on_stream, wait_stream
+from piper_amd.moe import AnnotatedMoE, MoEArgs, MoEFeedForwardBlock, RMSNorm
 
 pytestmark = pytest.mark.gpu
 
@@ -322,3 +326,76 @@ def test_operators_and_streams_of_a_device_that_is_not_current(dev):
         host().pack_param_grads([(p, 0, 16, (16,))], flat, None)
         assert p.grad is None and torch.equal(flat, torch.ones_like(flat))
         assert torch.cuda.current_device() == 0
+
+
+def _modules(dev):
+    torch.manual_seed(0)
+    args = MoEArgs(num_experts=E, top_k=K, route_norm=True)
+    norm, moe, block = RMSNorm(H).to(dev), AnnotatedMoE(args, H, I).to(dev), MoEFeedForwardBlock(args, H, I).to(dev)
+    moe.init_weights()
+    block.moe.init_weights()
+    return {"norm": norm, "moe": moe, "block": block}
+
+
+class _Call(torch.nn.Module):
+    """One piecewise operator as a module, for torch.jit.trace."""
+
+    def __init__(self, name, dev):
+        super().__init__()
+        self.name = name
+        self.gate = torch.nn.Parameter(_params(dev)["w_gate"].detach())
+        self.w = torch.nn.ParameterList([t.detach() for n, t in _params(dev, torch.float32).items() if n in ("w1", "w2", "w3")])
+        self.register_buffer("perm", torch.randperm(T, generator=torch.Generator().manual_seed(0)).int().to(dev))
+        self.register_buffer("counts", torch.full((E,), T // E, dtype=torch.int32, device=dev))
+        self.register_buffer("one", torch.ones(T, 1, device=dev))
+
+    def forward(self, x):
+        if self.name == "router":
+            return F_.router(x, self.gate, None, top_k=K, route_norm=True)[0]
+        if self.name == "permute":
+            return F_.permute(x, self.perm, 1)
+        if self.name == "combine":
+            return F_.combine(x, self.perm, self.one)
+        return F_.bmm_experts(*self.w, x, self.counts)
+
+
+@pytest.mark.parametrize("name", ["norm", "moe", "block", "router", "permute", "combine", "experts"])
+def test_jit_trace_records_the_operators(dev, name):
+    """A traced module computes its output from its input: the kernels' results are no constants of the trace."""
+    print(f"[case] jit.trace, {name}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    x, other = (torch.randn(T, H, generator=g).to(dev) for _ in range(2))
+    mod = _modules(dev)[name] if name in ("norm", "moe", "block") else _Call(name, dev)
+    if name in ("norm", "moe", "block"):
+        x, other = x.view(2, T // 2, H), other.view(2, T // 2, H)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        traced = torch.jit.trace(mod, x, check_trace=False)
+    assert torch.equal(traced(other), mod(other))
+
+
+class _Names(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(getattr(func, "__name__", ""))
+        return func(*args, **(kwargs or {}))
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("name,operators", [("norm", ["rmsnorm"]), ("moe", ["expert_region"]), ("block", ["rmsnorm", "expert_region"]),
+                                            ("experts", ["bmm_experts"])])
+def test_torch_function_sees_the_operators(dev, name, operators):
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(3)).to(dev)
+    mod = _Call(name, dev) if name == "experts" else _modules(dev)[name]
+    x = x if name == "experts" else x.view(2, T // 2, H)
+    with _Names() as names:
+        out = mod(x)
+    assert [n for n in names.seen if n in ("rmsnorm", "expert_region", "bmm_experts")] == operators
+    sub = mod(x.as_subclass(_Subclass))
+    assert type(sub) is _Subclass and torch.equal(sub.as_subclass(torch.Tensor), out)

@@ -112,3 +112,8 @@ def test_replaced_operators(monkeypatch, name):
 def test_inputs_without_three_dimensions_are_refused(shape):
     with pytest.raises(ValueError):
         _block()(torch.zeros(shape))
+
+
+def test_fx_records_the_operator_of_the_norm():
+    graph = torch.fx.symbolic_trace(M.RMSNorm(16)).graph
+    assert torch.ops.piper_amd.rmsnorm in [n.target for n in graph.nodes]
