@@ -9,6 +9,7 @@
 // modules, and every decision that depends on Python state.  Functions that may meet something else
 // than ordinary GPU tensors (fake tensors, tracing modes) return None and leave the call to the
 // dispatcher.
+#include <ATen/record_function.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
 #include <hip/hip_runtime.h>
@@ -91,6 +92,15 @@ void refuse_transforms(std::initializer_list<const Tensor*> ts, const char* what
                 " does not support functorch transforms");
   }
 }
+// A direct call under its operator's name in the profiler (the dispatcher records its own calls)
+struct RecordDirect {
+  std::optional<at::RecordFunction> record;
+  RecordDirect(bool direct, const char* name) {
+    if (!direct) return;
+    record.emplace(at::RecordScope::FUNCTION);
+    if (record->isActive()) record->before(name);
+  }
+};
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
   if (!at::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
@@ -578,6 +588,7 @@ std::optional<Tensor> expert_region(const Tensor& x, const Tensor& w_gate, const
   const Tensor bias = opt(bias_), residual = opt(residual_), norm_w = opt(norm_w_);
   if (direct && !plain({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w})) return std::nullopt;
   refuse_transforms({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w}, "expert_region");
+  const RecordDirect record(direct, "piper_amd::expert_region");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   if (wants_grad({&x, &w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w}))
@@ -627,6 +638,7 @@ struct NormFn : public torch::autograd::Function<NormFn> {
 std::optional<Tensor> rmsnorm(const Tensor& x, const Tensor& w, double eps, bool direct) {
   if (direct && !plain({&x, &w})) return std::nullopt;
   refuse_transforms({&x, &w}, "rmsnorm");
+  const RecordDirect record(direct, "piper_amd::rmsnorm");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   return wants_grad({&x, &w}) ? NormFn::apply(x, w, eps) : NormFn::run(x, w, eps, Tensor());
@@ -840,6 +852,7 @@ struct ExpertsFn : public torch::autograd::Function<ExpertsFn> {
 std::optional<Tensor> bmm_experts(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& counts, bool direct) {
   if (direct && !plain({&w1, &w2, &w3, &x, &counts})) return std::nullopt;
   refuse_transforms({&w1, &w2, &w3, &x, &counts}, "bmm_experts");
+  const RecordDirect record(direct, "piper_artifact::bmm_experts");
   require_gpu(x);
   c10::hip::HIPGuard device(x.device().index());
   if (wants_grad({&w1, &w2, &w3, &x})) return ExpertsFn::apply(w1, w2, w3, x, counts);

@@ -399,3 +399,14 @@ def test_torch_function_sees_the_operators(dev, name, operators):
     assert [n for n in names.seen if n in ("rmsnorm", "expert_region", "bmm_experts")] == operators
     sub = mod(x.as_subclass(_Subclass))
     assert type(sub) is _Subclass and torch.equal(sub.as_subclass(torch.Tensor), out)
+
+
+@pytest.mark.parametrize("name,operators", [("norm", {"piper_amd::rmsnorm"}), ("moe", {"piper_amd::expert_region"}),
+                                            ("block", {"piper_amd::expert_region"}), ("experts", {"piper_artifact::bmm_experts"})])
+def test_the_profiler_names_the_operators(dev, name, operators):
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(3)).to(dev)
+    mod = _Call(name, dev) if name == "experts" else _modules(dev)[name]
+    x = x if name == "experts" else x.view(2, T // 2, H)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        mod(x)
+    assert operators <= {e.key for e in prof.key_averages()}
