@@ -20,6 +20,7 @@ from . import ops
 from ._lib import host
 
 _ROUTE_TOPK = ops.route_topk
+_is_tracing = torch._C._is_tracing          # torch.jit.is_tracing() without its check for scripted code
 
 
 def _replaced_route():
@@ -67,7 +68,7 @@ def router(x, w_gate, gate_bias=None, *, top_k: int, route_norm: bool, route_sca
     """(top_scores [T,K] f32, selected_experts_indices [T,K] i32, num_tokens_per_expert [E] i32).
     The call `self.router(x, self.expert_bias)` of qwen3.py:237-241.  The histogram is the one the
     counting sort produces (no host sync, no second pass over the indices)."""
-    call = torch.ops.piper_amd.router if torch.jit.is_tracing() else _router
+    call = torch.ops.piper_amd.router if _is_tracing() else _router
     top_scores, top_idx = call(x, w_gate, gate_bias, int(top_k), bool(route_norm), float(route_scale))
     counts = _sorted_tables(top_idx, w_gate.shape[0])[0]
     return top_scores, top_idx, counts
@@ -87,7 +88,7 @@ def _permute(x, perm, top_k):
 
 def permute(x: torch.Tensor, token_indices_experts_sorted: torch.Tensor, top_k: int) -> torch.Tensor:
     """routed_input = x[token_indices_experts_sorted // top_k]  (qwen3.py:250)."""
-    call = torch.ops.piper_amd.permute if torch.jit.is_tracing() else _permute
+    call = torch.ops.piper_amd.permute if _is_tracing() else _permute
     return call(x, token_indices_experts_sorted, int(top_k))
 
 
@@ -174,7 +175,7 @@ def _combine(y, perm, top_scores):
 
 def combine(gathered_output, token_indices_experts_sorted, top_scores):
     """Unpermute scatter + fp32 weighted sum over k (qwen3.py:265-283), fused."""
-    call = torch.ops.piper_amd.combine if torch.jit.is_tracing() else _combine
+    call = torch.ops.piper_amd.combine if _is_tracing() else _combine
     return call(gathered_output, token_indices_experts_sorted, top_scores)
 
 
