@@ -2221,12 +2221,22 @@ bool tile_gemm_ok(int dtype, int64_t H, int64_t I, std::initializer_list<const v
 //   128 experts 2048 x 768:  1 token 62 -> 20, 24 tokens 211 -> 172, 8 rows each 262 -> 257, 12 rows 266 -> 281
 //   32 experts 1024 x 512 (tiles of tile_gemm.h -> streaming): 32 rows 30 -> 52;  64 experts 1536 x 384, 48 rows 79 -> 117
 //   24 experts 1000 x 360 (against the tiles of tile_gemm.h): 21 rows each 29 -> 21, 32 rows 29 -> 31
-// Where the wide tiles have a unit for every CU they hold their own from about 8 rows per expert on, the
-// smaller tiles of tile_gemm.h elsewhere from about 24.
+// Where the wide tiles have a unit for every CU they hold their own from about 8 rows per expert on, with three
+// units for every CU from 5 (their last round is full then), the smaller tiles of tile_gemm.h elsewhere from about 24.
+// The rule knows the mean only; an expert with many rows is walked in 16- or 32-row units that each read its weights
+// again (from the L2).  gate/up + down, caches cold, us, other kernel -> streaming, for even counts / counts ~ 1 / rank / one
+// expert in every token / the same experts in every token:
+//   128 experts 2048 x 768, 4 rows: 270 -> 268 / 243 -> 228 / 289 -> 273 / 76 -> 71
+//                           6 rows: 271 -> 278 / 273 -> 288 / 292 -> 282 / 81 -> 95
+//                           8 rows: 273 -> 287 / 272 -> 305 / 290 -> 295 / 86 -> 119
+//   128 experts 1024 x 512, 8 rows: 122 -> 120 / 123 -> 130 / 129 -> 121 / 34 -> 50
+//    64 experts 2048 x 768, 8 rows: 177 -> 167 / 179 -> 175 / 182 -> 168 / 54 -> 66
+//    64 experts 1536 x 384, 8 rows: 87 -> 84 / 86 -> 90 / 87 -> 86 / 29 -> 34;  16 rows: 86 -> 89 / 86 -> 97 / 86 -> 98 / 34 -> 40
+//    32 experts 1024 x 512, 24 rows: 46 -> 48 / 53 -> 51 / 51 -> 49 / 24 -> 28
 int64_t skinny_rows(int64_t A, int64_t I, int64_t E) {
   const int64_t touched = A < E ? A : E, rows = pk_ceil_div(A, touched);
-  const bool fills = touched * pk_ceil_div(I, 128) >= mf::persistent_grid();
-  return rows <= (fills ? 8 : 24) ? rows : 0;
+  const int64_t wide_units = touched * pk_ceil_div(I, 128), cus = mf::persistent_grid();
+  return rows <= (wide_units >= 3 * cus ? 4 : wide_units >= cus ? 8 : 24) ? rows : 0;
 }
 int fwd_skinny(const void* x, const int32_t* row_map, int64_t div, const void* w1, const void* w2, const void* w3, const int32_t* starts,
                void* g, void* u, void* h, void* y, int64_t A, int64_t H, int64_t I, int64_t E, int64_t rows, hipStream_t s) {

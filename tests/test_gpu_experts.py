@@ -588,6 +588,18 @@ def test_experts_with_few_rows(dev, counts, H, I):
         s += c
 
 
+@pytest.mark.parametrize("experts,A", [(128, 512), (128, 513), (64, 512), (64, 513)])
+def test_experts_with_few_rows_and_popular_experts(dev, experts, A):
+    """Both sides of the lines between the weight-streaming forward and the wide tiles (4 rows an expert at
+    three wide units per CU, 8 below), with counts that fall as 1 / rank down to none."""
+    weights = 1.0 / torch.arange(1, experts + 1).double()
+    counts = (weights / weights.sum() * A).long()
+    counts[0] += A - int(counts.sum())
+    counts[experts // 2] += int(counts[-1])
+    counts[-1] = 0
+    test_experts_with_few_rows(dev, counts.tolist(), 256, 768)
+
+
 REGION_BACKWARD_CASES = [
     # (counts, H, I): split reductions with every row and column remainder, unsplit 64-row tiles, 128-row
     # tiles, the persistent kernels at widths of 256 and 128 columns, a single row
