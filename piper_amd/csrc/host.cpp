@@ -85,11 +85,11 @@ bool plain(std::initializer_list<const Tensor*> ts) {
 // tangent (it would be dropped on the way, whether or not a backward is wanted) or that is a functorch
 // wrapper (it has no memory of its own) is refused.
 void refuse_transforms(std::initializer_list<const Tensor*> ts, const char* what) {
+  constexpr c10::DispatchKeySet wrappers({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper});
   for (const Tensor* t : ts) {
     if (!t->defined()) continue;
     TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(/*level=*/0).defined(), what, " has no forward-mode derivative");
-    TORCH_CHECK(!t->key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper})), what,
-                " does not support functorch transforms");
+    TORCH_CHECK(!t->key_set().has_any(wrappers), what, " does not support functorch transforms");
   }
 }
 // A direct call under its operator's name in the profiler (the dispatcher records its own calls)

@@ -155,8 +155,12 @@ class MoEFeedForwardBlock(nn.Module):
     def _one_node(self) -> bool:
         """Whether nobody can tell the submodules' own calls from one fused call: both are called as this
         module defines them (_called_as_defined) and so are the two operators they consist of."""
-        return (self.moe.fused and not torch.compiler.is_compiling() and _called_as_defined(self.ffn_norm, RMSNorm)
-                and _called_as_defined(self.moe, AnnotatedMoE) and (F_.rmsnorm, F_.expert_region) == _OPERATORS)
+        if torch.compiler.is_compiling():
+            return False
+        norm, moe = self._modules["ffn_norm"], self._modules["moe"]
+        return (moe.fused and _called_as_defined(norm, RMSNorm) and _called_as_defined(moe, AnnotatedMoE)
+                and not (_FORWARD_HOOKS or _FORWARD_PRE_HOOKS or _BACKWARD_HOOKS or _BACKWARD_PRE_HOOKS)
+                and F_.rmsnorm is _OPERATORS[0] and F_.expert_region is _OPERATORS[1])
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self._one_node():
@@ -174,14 +178,15 @@ class MoEFeedForwardBlock(nn.Module):
 # What a call of the two submodules runs unless somebody has put something else in its place: hooks on the
 # instance or on all modules, a `forward` (or `_call_impl`) of its own on the instance, a patched class, a
 # patched nn.Module call (tracers, profilers), `module.compile()`, a subclass.
-_DEFINED = {cls: (cls.forward, nn.Module.__call__, nn.Module._call_impl) for cls in (RMSNorm, AnnotatedMoE)}
+_FORWARDS = {cls: cls.forward for cls in (RMSNorm, AnnotatedMoE)}
+_CALL, _CALL_IMPL = nn.Module.__call__, nn.Module._call_impl
 _OPERATORS = (F_.rmsnorm, F_.expert_region)
-_GLOBAL_HOOKS = tuple(getattr(nn.modules.module, n) for n in ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
-                                                               "_global_backward_pre_hooks"))
+_FORWARD_HOOKS, _FORWARD_PRE_HOOKS = nn.modules.module._global_forward_hooks, nn.modules.module._global_forward_pre_hooks
+_BACKWARD_HOOKS, _BACKWARD_PRE_HOOKS = nn.modules.module._global_backward_hooks, nn.modules.module._global_backward_pre_hooks
 
 
 def _called_as_defined(m: nn.Module, cls: type) -> bool:
     own = m.__dict__
-    return (type(m) is cls and (cls.forward, cls.__call__, cls._call_impl) == _DEFINED[cls] and "forward" not in own and "_call_impl" not in own
-            and m._compiled_call_impl is None
-            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or any(_GLOBAL_HOOKS)))
+    return (type(m) is cls and cls.forward is _FORWARDS[cls] and cls.__call__ is _CALL and cls._call_impl is _CALL_IMPL
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"])
+            and "forward" not in own and "_call_impl" not in own and own.get("_compiled_call_impl") is None)
