@@ -588,6 +588,16 @@ int pk_rmsnorm_fwd(const void* x, int dtype, const void* weight, float eps, void
   return PK_OK;
 }
 
+static int rmsnorm_dw_reduce(int dtype, const float* partial, int nb, void* d_weight, int64_t H, int accumulate, hipStream_t s) {
+  const dim3 grid((unsigned)pk_ceil_div(H, kDwCols));
+  if (dtype == PK_BF16)
+    PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<bf16_t>), grid, dim3(kDwCols * kDwGroups), 0, s, partial, nb, (bf16_t*)d_weight, H, accumulate ? 1 : 0);
+  else
+    PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<float>), grid, dim3(kDwCols * kDwGroups), 0, s, partial, nb, (float*)d_weight, H, accumulate ? 1 : 0);
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+
 int64_t pk_rmsnorm_bwd_workspace_bytes(int64_t T, int64_t H) {
   if (T < 0 || H <= 0) return PK_ERR_ARG;
   const int64_t nb = T < kNormBwdBlocks ? (T > 0 ? T : 1) : kNormBwdBlocks;
@@ -598,7 +608,8 @@ int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight
                    const void* d_x_addend, void* d_x, void* d_weight, int accumulate, int64_t T,
                    int64_t H, void* workspace, int64_t workspace_bytes, pk_stream_t stream) {
   if (T < 0 || H <= 0 || !pk_dtype_ok(dtype)) return PK_ERR_ARG;
-  if (T == 0) return PK_OK;
+  // no rows: their sum is zero
+  if (T == 0) return d_weight ? rmsnorm_dw_reduce(dtype, nullptr, 0, d_weight, H, accumulate, (hipStream_t)stream) : PK_OK;
   if (!d_y || !x || !weight || !rstd || !d_x) return PK_ERR_ARG;
   if (T > 0x7fffffffll) return PK_ERR_SHAPE;
   const bool vec = vec_ok(dtype, H, {d_y, x, weight, d_x, d_x_addend});
@@ -632,15 +643,7 @@ int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight
     return PK_OK;
   }
   if (rc != PK_OK) return rc;
-  if (d_weight) {
-    const dim3 grid((unsigned)pk_ceil_div(H, kDwCols));
-    if (dtype == PK_BF16)
-      PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<bf16_t>), grid, dim3(kDwCols * kDwGroups), 0, s, partial, nb, (bf16_t*)d_weight, H, accumulate ? 1 : 0);
-    else
-      PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_dw_reduce_kernel<float>), grid, dim3(kDwCols * kDwGroups), 0, s, partial, nb, (float*)d_weight, H, accumulate ? 1 : 0);
-    PK_RETURN_IF_LAUNCH_FAILED();
-  }
-  return PK_OK;
+  return d_weight ? rmsnorm_dw_reduce(dtype, partial, nb, d_weight, H, accumulate, s) : PK_OK;
 }
 
 }  // extern "C"

@@ -115,3 +115,13 @@ def test_rmsnorm_bwd_on_both_sides_of_the_wave_kernel(dev, dtype, T, H):
     _, rstd = ops.rmsnorm_fwd(x.to(dev), w.to(dev), 1e-6)
     dx, dw = ops.rmsnorm_bwd(dy.to(dev), x.to(dev), w.to(dev), rstd, d_x_addend=add.to(dev))
     assert rel_err(dx, xr.grad + add.double()) <= tol and rel_err(dw, wr.grad) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_rmsnorm_weight_gradient_of_no_rows(dev, dtype, accumulate):
+    """The sum over no rows is zero: written, or added to what is there."""
+    x = torch.empty(0, 264, dtype=dtype, device=dev)
+    before = torch.full((264,), 2.5 if accumulate else float("nan"), dtype=dtype, device=dev)
+    _, dw = ops.rmsnorm_bwd(x, x, torch.ones(264, dtype=dtype, device=dev), torch.empty(0, device=dev), d_weight=before, accumulate=accumulate)
+    assert torch.equal(dw, torch.full_like(dw, 2.5 if accumulate else 0.0))
