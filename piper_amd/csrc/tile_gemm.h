@@ -1,17 +1,19 @@
 // Grouped GEMMs on the matrix cores for what the 256-wide bf16 kernels of grouped_gemm.hip do not
 // take or are too coarse for: fp32 operands (v_mfma_f32_32x32x2_f32: exact fp32 products and sums), bf16
-// widths that are no multiple of 128 (256 for weight gradients), and products with few tiles.  Every row only has to be a whole number of 16-byte pieces (4 fp32 or 8 bf16
-// elements); row, column and reduction remainders are fetched as zeros and masked on store.
+// widths that are no multiple of 128 (256 for weight gradients), and products with few tiles.  Every row
+// only has to be a whole number of 16-byte pieces (4 fp32 or 8 bf16 elements); row, column and reduction
+// remainders are fetched as zeros and masked on store.
 //
 //   ragged M: C[rows_e, N] = sum_seg A_seg[rows_e, K] . B_seg[e]     (forward, input gradient)
 //   ragged K: C[e][M, N] (+)= A[rows_e, M]^T . B[rows_e, N]           (weight gradient)
 //
-// One workgroup of four waves (2 x 2) per output tile of 64 x 64 or 128 x 128.  A k-tile is 128 bytes
+// One workgroup per output tile: four waves (2 x 2) for tiles of 64 x 64 or 128 x 128, two (2 x 1) for the
+// 64 x 32 tiles that fp32 ragged-M products take where 64 x 64 ones leave CUs idle.  A k-tile is 128 bytes
 // of the reduction index of every operand row (32 fp32 or 64 bf16); two or three k-tiles are in flight in
 // registers (against one: -7 %) while another is multiplied out of LDS; two LDS buffers, one barrier per
 // k-tile.  The operands pass through registers rather than straight into LDS because the masking then
 // costs one select per piece and nothing has to be counted by hand.  Where the tiles are too few for
-// the chip, several groups of four waves share a tile's reduction.
+// the chip, several groups of waves share a tile's reduction.
 // Against one 64 x 64 FMA tile per workgroup (simt_gemm.h, which keeps the widths that are no multiple
 // of 16 bytes): see the figures at tile_gemm_ok in grouped_gemm.hip.
 #pragma once
