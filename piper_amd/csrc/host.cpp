@@ -2,8 +2,8 @@
 // the C ABI and the autograd nodes.  One forward and backward of the expert region is about thirty
 // launches of 2 us each on the host; with a Python call, a ctypes call and one to three tensor
 // allocations in front of every one of them it was 370 us, more than the GPU needs below about a
-// thousand tokens.  Here a node allocates one block of memory for what it saves and one for what it
-// does not, and issues its launches back to back.
+// thousand tokens.  Here a node allocates one block of memory for what the weight gradients read, one
+// for what else it saves and one for what it does not, and issues its launches back to back.
 //
 // Python keeps what it is the better place for: the torch.library definitions (functional.py), the
 // modules, and every decision that depends on Python state.  Functions that may meet something else

@@ -147,3 +147,34 @@ def test_static_sort_recorded_into_a_hip_graph(dev):
             torch.cuda.synchronize()
             for name in ref:
                 assert torch.equal(ref[name], o[name]), f"replay {rep}: {name} (A={A}, E={E})"
+
+
+def test_static_sort_in_three_launches(dev):
+    """More than 512 chunks (histograms, scan, scatter), eager and replayed out of a HIP graph, against torch's
+    stable sort."""
+    lib = _lib.load()
+    _lib.init_device()
+    A, E = 300_001, 100
+    buf, o = torch.zeros(A, dtype=torch.int32, device=dev), _outputs(A, E, dev)
+
+    def sort():
+        assert lib.pk_sort_by_expert_static(_p(buf), A, E, _p(o["counts"]), _p(o["starts"]), _p(o["perm"]), _p(o["inv_perm"]), _p(o["order"]),
+                                            C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)) == 0
+
+    sort()
+    torch.cuda.synchronize()
+    print("[case] static sort in three launches under graph capture", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        sort()
+    for rep in range(3):
+        buf.copy_(torch.randint(0, E, (A,), generator=torch.Generator().manual_seed(rep), dtype=torch.int32))
+        for run in (graph.replay, sort):
+            for t in o.values():
+                t.fill_(-7)
+            run()
+            torch.cuda.synchronize()
+            want, counts = torch.argsort(buf.long(), stable=True), torch.bincount(buf.long(), minlength=E)
+            assert torch.equal(o["perm"].long(), want) and torch.equal(o["inv_perm"].long()[want], torch.arange(A, device=dev))
+            assert torch.equal(o["counts"].long(), counts) and torch.equal(o["starts"][1:].long(), counts.cumsum(0)) and int(o["starts"][0]) == 0
+            assert torch.equal(o["order"].long(), torch.argsort(-counts, stable=True))
