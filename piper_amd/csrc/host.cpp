@@ -50,6 +50,11 @@ void require_gpu(const Tensor& t) {
   TORCH_CHECK(t.is_cuda(), "piper_amd kernels run on the GPU only; got a tensor on ", t.device(), " (there is no CPU fallback)");
 }
 
+void same_device(const Tensor& first, std::initializer_list<const Tensor*> others) {
+  for (const Tensor* t : others)
+    TORCH_CHECK_VALUE(!t->defined() || t->device() == first.device(), "all tensors of a call must be on one device");
+}
+
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 const float* fptr(const Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
 Tensor contig(const Tensor& t) { return t.defined() && !t.is_contiguous() ? t.contiguous() : t; }
@@ -239,8 +244,7 @@ Shape region_shape(const Tensor& x, const Tensor& w_gate, const Tensor& bias, co
                     "combine_fwd: residual must be [T,H] in the dtype of y");
   TORCH_CHECK_VALUE(!norm_w.defined() || (norm_w.dim() == 1 && norm_w.size(0) == s.H && norm_w.scalar_type() == x.scalar_type()),
                     "rmsnorm_fwd: x [T,H], weight [H] in the dtype of x");
-  for (const Tensor* t : {&w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w})
-    TORCH_CHECK_VALUE(!t->defined() || t->device() == x.device(), "all tensors of a call must be on one device");
+  same_device(x, {&w_gate, &bias, &w1, &w2, &w3, &residual, &norm_w});
   s.dtype = dtype_code(x);
   s.es = s.dtype == PK_BF16 ? 2 : 4;
   s.route_norm = route_norm; s.route_scale = route_scale; s.eps = eps;
@@ -640,6 +644,7 @@ std::optional<Tensor> rmsnorm(const Tensor& x, const Tensor& w, double eps, bool
   refuse_transforms({&x, &w}, "rmsnorm");
   const RecordDirect record(direct, "piper_amd::rmsnorm");
   require_gpu(x);
+  same_device(x, {&w});
   c10::hip::HIPGuard device(x.device().index());
   return wants_grad({&x, &w}) ? NormFn::apply(x, w, eps) : NormFn::run(x, w, eps, Tensor());
 }
@@ -715,6 +720,7 @@ std::pair<Tensor, Tensor> router(const Tensor& x, const Tensor& w_gate, const Op
   const Tensor b = opt(bias);
   refuse_transforms({&x, &w_gate, &b}, "router");
   require_gpu(x);
+  same_device(x, {&w_gate, &b});
   c10::hip::HIPGuard device(x.device().index());
   auto r = RouterFn::apply(x, w_gate, bias, top_k, route_norm, route_scale, route.ptr() == Py_None ? nullptr : route.ptr());
   return {r[0], r[1]};
@@ -741,6 +747,8 @@ struct PermuteFn : public torch::autograd::Function<PermuteFn> {
 Tensor permute(const Tensor& x, const Tensor& perm, const Tensor& inv, int64_t top_k) {
   refuse_transforms({&x, &perm, &inv}, "permute");
   require_gpu(x);
+  same_device(x, {&perm, &inv});
+  TORCH_CHECK_VALUE(x.dim() == 2, "permute: x [T,H]");
   c10::hip::HIPGuard device(x.device().index());
   return PermuteFn::apply(x, perm, inv, top_k);
 }
@@ -767,6 +775,9 @@ struct CombineFn : public torch::autograd::Function<CombineFn> {
 Tensor combine(const Tensor& y, const Tensor& perm, const Tensor& inv, const Tensor& scores) {
   refuse_transforms({&y, &perm, &inv, &scores}, "combine");
   require_gpu(y);
+  same_device(y, {&perm, &inv, &scores});
+  TORCH_CHECK_VALUE(y.dim() == 2 && scores.dim() == 2 && perm.numel() >= y.size(0) && inv.numel() >= y.size(0),
+                    "combine_fwd: y_sorted [A,H], scores [T,K] and a permutation of A slots");
   c10::hip::HIPGuard device(y.device().index());
   return CombineFn::apply(y, perm, inv, scores);
 }
@@ -787,6 +798,8 @@ struct ExpertsFn : public torch::autograd::Function<ExpertsFn> {
   // y [A,H]; the pre-activations are left in gu [2,A,I], and h [A,I], which the weight gradients read as well.
   // Without a backward (gu and h null) they share one allocation.
   static Tensor run(const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor& x, const Tensor& starts, Tensor* gu, Tensor* h) {
+    TORCH_CHECK_VALUE(x.dim() == 2 && w1.dim() == 3 && x.size(1) == w1.size(2) && starts.numel() > w1.size(0),
+                      "bmm_experts: x [A,H] and a row count for every expert");
     TORCH_CHECK_VALUE(w1.dim() == 3 && w2.dim() == 3 && w3.dim() == 3, "expert weights must be [E,I,H], [E,H,I], [E,I,H]");
     const int64_t E = w1.size(0), I = w1.size(1), H = w1.size(2), A = x.size(0);
     TORCH_CHECK_VALUE(w3.sizes() == w1.sizes() && w2.size(0) == E && w2.size(1) == H && w2.size(2) == I, "expert weight shapes disagree");
@@ -854,6 +867,8 @@ std::optional<Tensor> bmm_experts(const Tensor& w1, const Tensor& w2, const Tens
   refuse_transforms({&w1, &w2, &w3, &x, &counts}, "bmm_experts");
   const RecordDirect record(direct, "piper_artifact::bmm_experts");
   require_gpu(x);
+  require_gpu(counts);
+  same_device(x, {&w1, &w2, &w3, &counts});
   c10::hip::HIPGuard device(x.device().index());
   if (wants_grad({&w1, &w2, &w3, &x})) return ExpertsFn::apply(w1, w2, w3, x, counts);
   return ExpertsFn::run(w1, w2, w3, x, ExpertsFn::counts_to_starts(counts), nullptr, nullptr);
@@ -918,6 +933,7 @@ void pack_param_grads(const py::list& specs, const Tensor& flat, const std::opti
     Tensor g = contig(pg.grads[i]);
     const int64_t off = spec_int(PyList_GET_ITEM(specs.ptr(), i), 1);
     TORCH_CHECK_VALUE(off >= 0 && off + g.numel() <= flat.numel(), "bucket_pack: tensor outside the bucket");
+    same_device(flat, {&g});
     l.ptrs.push_back(g.data_ptr());
     l.offs.push_back(off);
     l.nums.push_back(g.numel());
@@ -956,6 +972,7 @@ void adamw_packed(const Tensor& master, const Tensor& exp_avg, const Tensor& exp
                     "adamw_fused_packed: flat_grad must match the bucket");
   TORCH_CHECK_VALUE(!shadow.defined() || (shadow.scalar_type() == at::kBFloat16 && shadow.numel() == total && shadow.is_contiguous()),
                     "adamw_fused_packed: bf16 shadow of the bucket's size");
+  same_device(master, {&exp_avg, &exp_avg_sq, &flat_grad, &shadow});
   std::vector<const void*> ptrs(std::max<size_t>(n, 1), nullptr);
   std::vector<Tensor> keep;
   std::optional<at::ScalarType> dtype;
@@ -964,6 +981,7 @@ void adamw_packed(const Tensor& master, const Tensor& exp_avg, const Tensor& exp
     if (!grads[i].has_value() || !grads[i]->defined()) continue;
     const Tensor& g = *grads[i];
     TORCH_CHECK_VALUE(g.numel() == numels[i], "adamw_fused_packed: gradient size differs from the tensor's");
+    same_device(master, {&g});
     TORCH_CHECK_VALUE(!dtype || *dtype == g.scalar_type(), "adamw_fused_packed: gradients of one call must share a dtype");
     dtype = g.scalar_type();
     if (g.is_contiguous()) {

@@ -410,3 +410,38 @@ def test_the_profiler_names_the_operators(dev, name, operators):
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
         mod(x)
     assert operators <= {e.key for e in prof.key_averages()}
+
+
+def test_tensors_of_another_device_are_refused(dev):
+    """A kernel cannot read host memory: an operand on the CPU, the row counts among them, is an error on the
+    host, and so are operands too short for what the kernels read."""
+    p = {n: t.detach() for n, t in _params(dev).items()}
+    x, _ = _activations(dev, T)
+    counts = torch.full((E,), T // E, dtype=torch.int32, device=dev)
+    perm, one = torch.arange(T, dtype=torch.int32, device=dev), torch.ones(T, 1, device=dev)
+    w = (p["w1"], p["w2"], p["w3"])
+    flat, grad = torch.zeros(16, device=dev), torch.nn.Parameter(torch.zeros(16))
+    grad.grad = torch.ones(16)
+    st = [torch.zeros(16, device=dev) for _ in range(3)]
+    calls = {
+        "counts": lambda: F_.bmm_experts(*w, x, counts.cpu()),
+        "counts, operator": lambda: torch.ops.piper_artifact.bmm_experts(*w, x, counts.cpu()),
+        "short counts": lambda: F_.bmm_experts(*w, x, counts[:-1]),
+        "other width": lambda: F_.bmm_experts(*w, x[:, :128].contiguous(), counts),
+        "expert weight": lambda: F_.bmm_experts(p["w1"].cpu(), p["w2"], p["w3"], x, counts),
+        "region weight": lambda: _region(x, dict(p, w2=p["w2"].cpu())),
+        "norm weight": lambda: F_.rmsnorm(x, p["norm"].cpu()),
+        "gate weight": lambda: F_.router(x, p["w_gate"].cpu(), None, top_k=K, route_norm=True),
+        "permutation": lambda: F_.permute(x, perm.cpu(), 1),
+        "combine permutation": lambda: F_.combine(x, perm.cpu(), one),
+        "short permutation": lambda: F_.combine(x, perm[:-1], one),
+        "packed gradient": lambda: host().pack_param_grads([(grad, 0, 16, (16,))], flat, None),
+        "AdamW gradient": lambda: ops.adamw_fused_packed(*st, None, [torch.ones(16)], [0], [16], step=1, lr=1e-3, beta1=0.9, beta2=0.95,
+                                                         eps=1e-8, weight_decay=0.1),
+    }
+    for name, call in calls.items():
+        print(f"[case] refused operand: {name}", flush=True)
+        with pytest.raises((RuntimeError, ValueError)):
+            call()
+    assert grad.grad is not None
+    torch.cuda.synchronize()
