@@ -138,6 +138,17 @@ PK_API int pk_region_router_bwd(const float* logits, const int32_t* top_idx, con
                          int64_t T, int64_t H, int64_t E, int64_t K, void* workspace, int64_t workspace_bytes,
                          pk_stream_t stream);
 
+/* pk_region_router_bwd (xn, d_xn: its x and d_x) followed by pk_rmsnorm_bwd of the norm whose output the region read
+ * (d_y: d_xn), with the same results: the two share launches.  d_norm_weight may be NULL.  xn and d_xn have x's dtype. */
+PK_API int64_t pk_region_router_norm_bwd_workspace_bytes(int64_t T, int64_t H, int64_t E, int x_dtype);
+PK_API int pk_region_router_norm_bwd(const float* logits, const int32_t* top_idx, const float* d_top_scores,
+                              const float* ds_partial, int64_t n_partial, const int32_t* inv_perm, int route_norm,
+                              float route_scale, const void* xn, int x_dtype, const float* w_gate, const void* d_rows,
+                              void* d_xn, float* d_w_gate, float* d_gate_bias, int accumulate, float* d_logits,
+                              const void* x, const void* norm_weight, const float* rstd, const void* d_x_addend,
+                              void* d_x, void* d_norm_weight, int64_t T, int64_t H, int64_t E, int64_t K,
+                              void* workspace, int64_t workspace_bytes, pk_stream_t stream);
+
 /* pk_gate_route and pk_sort_by_expert in one call (same results): for a decode step the top-k and the
  * sort share one launch.  counts, inv_perm and order may be NULL.  workspace:
  * pk_gate_route_sort_workspace_bytes. */

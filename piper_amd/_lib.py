@@ -38,6 +38,10 @@ SIGNATURES = {
     # logits idx d_scores part n_part inv_perm norm scale x x_dtype w_gate d_rows d_x d_w d_b accumulate d_logits T H E K ws ws_bytes stream
     "pk_region_router_bwd": (_c_int, [_p, _p, _p, _p, _c_i64, _p, _c_int, _c_f32, _p, _c_int, _p, _p, _p, _p, _p, _c_int, _p,
                                       _c_i64, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),
+    "pk_region_router_norm_bwd_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int]),
+    # ... w_gate d_rows d_xn d_w d_b accumulate d_logits x norm_weight rstd addend d_x d_norm_w T H E K ws ws_bytes stream
+    "pk_region_router_norm_bwd": (_c_int, [_p, _p, _p, _p, _c_i64, _p, _c_int, _c_f32, _p, _c_int, _p, _p, _p, _p, _p, _c_int, _p,
+                                           _p, _p, _p, _p, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),
     "pk_gate_route_sort_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "pk_gate_route_sort": (_c_int, [_p, _c_int, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p, _p, _p, _p, _p, _p,
                                     _p, _c_i64, _p]),

@@ -482,7 +482,8 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     const size_t d_gT = w.add(ait), d_uT = w.add(ait), hsT = w.add(ait), d_logits = w.add(s.T * s.E * 4);
     const size_t d_scores = t.add(ldt > 0 ? 0 : s.A * 4), part = t.add(ds_ws);
     const size_t d_xs = t.add(need_xn ? s.A * s.H * s.es : 0);
-    const int64_t router_ws_bytes = pk_region_router_bwd_workspace_bytes(s.T, s.H, s.E, s.dtype);
+    const int64_t router_ws_bytes = norm ? pk_region_router_norm_bwd_workspace_bytes(s.T, s.H, s.E, s.dtype)
+                                         : pk_region_router_bwd_workspace_bytes(s.T, s.H, s.E, s.dtype);
     const size_t router_ws = t.add(router_ws_bytes);
     const size_t d_xn = t.add(norm && need_xn ? s.T * s.H * s.es : 0);
     if (postpone) {
@@ -516,18 +517,18 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
     Tensor d_x, d_norm_w;
     const auto router_and_input = [&](const Tensor& d_wg, const Tensor& d_b) {
       if (need_xn) d_x = at::empty({s.T, s.H}, x.options());
-      PK_CALL(pk_region_router_bwd, m.f32(sv.logits), m.i32(sv.idx), n_part > 0 ? nullptr : t.f32(d_scores), t.f32(part), n_part, m.i32(sv.inv),
-              s.route_norm, (float)s.route_scale, x_rows, s.dtype, fptr(w_gate), t.at_(d_xs), !need_xn ? nullptr : norm ? t.at_(d_xn) : ptr(d_x),
-              static_cast<float*>(ptr(d_wg)), static_cast<float*>(ptr(d_b)), 0, w.f32(d_logits), s.T, s.H, s.E, s.K, t.at_(router_ws),
-              router_ws_bytes, st);
-      if (!norm || !need_xn) return;
-      Tensor ws;
-      if (need[NORM_W]) {
-        d_norm_w = at::empty({s.H}, norm_w.options());
-        ws = at::empty({pk_rmsnorm_bwd_workspace_bytes(s.T, s.H)}, x.options().dtype(at::kByte));
+      const float *const d_s = n_part > 0 ? nullptr : t.f32(d_scores), *const parts = t.f32(part);
+      float *const dwg = static_cast<float*>(ptr(d_wg)), *const db = static_cast<float*>(ptr(d_b));
+      if (!norm || !need_xn) {
+        PK_CALL(pk_region_router_bwd, m.f32(sv.logits), m.i32(sv.idx), d_s, parts, n_part, m.i32(sv.inv), s.route_norm, (float)s.route_scale,
+                x_rows, s.dtype, fptr(w_gate), t.at_(d_xs), need_xn ? ptr(d_x) : nullptr, dwg, db, 0, w.f32(d_logits), s.T, s.H, s.E, s.K,
+                t.at_(router_ws), router_ws_bytes, st);
+        return;
       }
-      PK_CALL(pk_rmsnorm_bwd, t.at_(d_xn), ptr(xc), s.dtype, ptr(contig(norm_w)), m.f32(sv.rstd), ptr(d_out), ptr(d_x), ptr(d_norm_w), 0, s.T, s.H,
-              ptr(ws), ws.defined() ? ws.numel() : 0, st);
+      if (need[NORM_W]) d_norm_w = at::empty({s.H}, norm_w.options());
+      PK_CALL(pk_region_router_norm_bwd, m.f32(sv.logits), m.i32(sv.idx), d_s, parts, n_part, m.i32(sv.inv), s.route_norm, (float)s.route_scale,
+              x_rows, s.dtype, fptr(w_gate), t.at_(d_xs), t.at_(d_xn), dwg, db, 0, w.f32(d_logits), ptr(xc), ptr(contig(norm_w)), m.f32(sv.rstd),
+              ptr(d_out), ptr(d_x), ptr(d_norm_w), s.T, s.H, s.E, s.K, t.at_(router_ws), router_ws_bytes, st);
       if (!need[X]) d_x = Tensor();
     };
     Tensor d_w1, d_w2, d_w3, d_wg, d_b;

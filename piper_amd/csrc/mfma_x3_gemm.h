@@ -233,20 +233,20 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 
 }
 
+// output tile (bx, by) of split bz
 template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
-__global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
+__device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int bx, int by, int bz) {
   constexpr int BM = 32 * WM, BN = 32 * WN;
-  __shared__ Lds<WM, WN, A_KC, B_KC, TA, TB> lds;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave / WN, wn = wave % WN;
-  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+  const int64_t m0 = (int64_t)by * BM, n0 = (int64_t)bx * BN;
   const int64_t kchunk = ((p.K + p.splits - 1) / p.splits + BK - 1) / BK * BK;
-  const int64_t kbeg = (int64_t)blockIdx.z * kchunk;
+  const int64_t kbeg = (int64_t)bz * kchunk;
   const int64_t kend = kbeg + kchunk < p.K ? kbeg + kchunk : p.K;
   floatx16_t acc;
   product<WM, WN, A_KC, B_KC, TA, TB>(p, lds, m0, n0, kbeg, kend, acc);
 
-  float* C = p.C + (p.splits > 1 ? (int64_t)blockIdx.z * p.M * p.N : 0);
+  float* C = p.C + (p.splits > 1 ? (int64_t)bz * p.M * p.N : 0);
   const int64_t n = n0 + wn * 32 + (lane & 31);
   if (n < p.N) {
     const float bias = (p.bias && p.splits == 1) ? p.bias[n] : 0.f;
@@ -261,6 +261,11 @@ __global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
     }
   }
 }
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+__global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
+  __shared__ Lds<WM, WN, A_KC, B_KC, TA, TB> lds;
+  gemm_tile<WM, WN, A_KC, B_KC, TA, TB>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
+}
 
 // The gradient of the region's input in one pass: out[t] = sum_k rows[inv_perm[t*K + k]] + d_logits[t] .
 // w_gate, the second term being this GEMM.  Its tile goes through LDS, and every thread then adds the K
@@ -273,16 +278,20 @@ struct GatherAdd {
   void* out;                  // [T, H]
   int32_t K;
 };
-template <int WM, int WN, typename TG, bool STREAM>
-__global__ __launch_bounds__(64 * WM * WN) void gather_kernel(const Params p, const GatherAdd ga) {
-  constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
+template <int WM, int WN>
+struct GatherLds {
   typedef Lds<WM, WN, true, false, float, float> Tiles;
-  constexpr int LDO = BN + 4;
-  constexpr int BYTES = sizeof(Tiles) > BM * LDO * 4 ? (int)sizeof(Tiles) : BM * LDO * 4;
-  __shared__ __attribute__((aligned(16))) char smem[BYTES];
+  static constexpr int LDO = 32 * WN + 4;
+  static constexpr int BYTES = sizeof(Tiles) > 32 * WM * LDO * 4 ? (int)sizeof(Tiles) : 32 * WM * LDO * 4;
+};
+template <int WM, int WN, typename TG, bool STREAM>
+__device__ __forceinline__ void gather_tile(const Params& p, const GatherAdd& ga, char* smem, int bx, int by) {
+  constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
+  typedef typename GatherLds<WM, WN>::Tiles Tiles;
+  constexpr int LDO = GatherLds<WM, WN>::LDO;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;
-  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+  const int64_t m0 = (int64_t)by * BM, n0 = (int64_t)bx * BN;
   floatx16_t acc;
   product<WM, WN, true, false, float, float>(p, *reinterpret_cast<Tiles*>(smem), m0, n0, 0, p.K, acc);
   float* const tile = reinterpret_cast<float*>(smem);       // (product ends with a barrier)
@@ -323,6 +332,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gather_kernel(const Params p, co
     *reinterpret_cast<decltype(o.v)*>(reinterpret_cast<TG*>(ga.out) + t * H + n0 + c) = o.v;
   }
 }
+template <int WM, int WN, typename TG, bool STREAM>
+__global__ __launch_bounds__(64 * WM * WN) void gather_kernel(const Params p, const GatherAdd ga) {
+  __shared__ __attribute__((aligned(16))) char smem[GatherLds<WM, WN>::BYTES];
+  gather_tile<WM, WN, TG, STREAM>(p, ga, smem, blockIdx.x, blockIdx.y);
+}
 
 // The operands must allow 4-element loads (pk_f32mm::vec4_ok); the caller falls back to
 // pk_f32mm::launch otherwise.
@@ -353,17 +367,26 @@ inline int launch(const Params& p, int kernel_id, hipStream_t s) {
 
 // d_logits: p.A [T, E], w_gate: p.B [E, H] (p.M = T, p.N = H, p.K = E).  PK_ERR_ALIGN: a base is not 16-byte
 // aligned, which the caller's contract asks for (widths without whole pieces go to the two kernels).
+// 32 tokens x 128 columns (16,384 tokens, the router backward as a whole: 212 us; 64 x 128: 214, 64 x 64: 222;
+// with the GEMM and the gather apart 270)
+constexpr int kGatherWM = 1, kGatherWN = 4;
+// one launch per 65,535 row blocks, what grid.y holds: the GEMM with 64-row blocks in front of a separate
+// gather takes twice that many tokens, and so does the forward
+constexpr int64_t kGatherSlice = (int64_t)65535 * 32 * kGatherWM;
+template <typename TG>
+inline bool gather_usable(const Params& p, const GatherAdd& ga) {
+  return usable<kGatherWM, kGatherWN, true, false, float, float>(p) && p.N % PkVec16<TG>::N == 0 && pk_aligned16(ga.rows) && pk_aligned16(ga.out);
+}
+template <typename TG>
+inline bool gather_streams(const Params& p, const GatherAdd& ga) {
+  return p.M * ga.K * p.N * (int64_t)sizeof(TG) > (int64_t)192 * 1024 * 1024;
+}
 template <typename TG>
 inline int launch_gather(const Params& p, const GatherAdd& ga, int kernel_id, hipStream_t s) {
-  // 32 tokens x 128 columns (16,384 tokens, the router backward as a whole: 212 us; 64 x 128: 214, 64 x 64: 222;
-  // with the GEMM and the gather apart 270)
-  constexpr int WM = 1, WN = 4;
-  if (!usable<WM, WN, true, false, float, float>(p) || p.N % PkVec16<TG>::N != 0 || !pk_aligned16(ga.rows) || !pk_aligned16(ga.out))
-    return PK_ERR_ALIGN;
-  const bool stream_rows = p.M * ga.K * p.N * (int64_t)sizeof(TG) > (int64_t)192 * 1024 * 1024;
-  // one launch per 65,535 row blocks, what grid.y holds: the GEMM with 64-row blocks in front of a separate
-  // gather takes twice that many tokens, and so does the forward
-  constexpr int64_t SLICE = (int64_t)65535 * 32 * WM;
+  constexpr int WM = kGatherWM, WN = kGatherWN;
+  if (!gather_usable<TG>(p, ga)) return PK_ERR_ALIGN;
+  const bool stream_rows = gather_streams<TG>(p, ga);
+  constexpr int64_t SLICE = kGatherSlice;
   for (int64_t t0 = 0; t0 < p.M; t0 += SLICE) {
     Params q = p;
     GatherAdd gq = ga;

@@ -2,6 +2,7 @@
 // (K-way gather-reduce), the fused unpermute+combine and its backward.  One block per row;
 // 16 bytes per lane per access, rows are contiguous so every access is fully coalesced.
 #include "pk_common.h"
+#include "gate_tail.h"
 #include <initializer_list>
 
 namespace {
@@ -264,12 +265,16 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_bwd_kernel(
 // needs no barrier (the block kernel above spends two per row, with every wave of the block waiting
 // on the slowest load).  Wave w of the grid walks rows w, w + waves, ...; its d_w sums stay in
 // registers, the four waves of a block add theirs in wave order through LDS and one partial row per
-// block goes to memory.  Bound by HBM (d_y and x in, d_x out).
+// block goes to memory.  Bound by HBM (d_y and x in, d_x out).  Blocks from nb on carry the gate's tail.
 template <typename T, int V>
 __global__ __launch_bounds__(kRowThreads) void rmsnorm_bwd_wave_kernel(
     const T* __restrict__ d_y, const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ rstd, const T* __restrict__ addend, T* __restrict__ d_x,
-    float* __restrict__ partial, int64_t rows, int64_t H) {
+    float* __restrict__ partial, int64_t rows, int64_t H, int nb, const GateTail tail) {
+  if ((int)blockIdx.x >= nb) {
+    gate_tail(tail, (int)blockIdx.x - nb);
+    return;
+  }
   using IO = RowIO<T, true>;
   constexpr int N = PkVec16<T>::N, WAVES = kRowThreads / 64;
   __shared__ float sums[64 * V * N];
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_bwd_wave_kernel(
     for (int i = 0; i < N; ++i) { dw[c][i] = 0.f; wv[c][i] = 0.f; }
     if (lane + 64 * c < nv) IO::load(w, lane + 64 * c, wv[c]);
   }
-  for (int64_t t = (int64_t)blockIdx.x * WAVES + wave; t < rows; t += (int64_t)gridDim.x * WAVES) {
+  for (int64_t t = (int64_t)blockIdx.x * WAVES + wave; t < rows; t += (int64_t)nb * WAVES) {
     const float rs = rstd[t];
     PkVec16<T> vy[V], vx[V], va[V];
 #pragma unroll
@@ -424,14 +429,14 @@ bool vec_ok(int dtype, int64_t H, std::initializer_list<const void*> ptrs) {
 template <typename T, bool VEC>
 int rmsnorm_bwd_launch(const void* d_y, const void* x, const void* weight, const float* rstd,
                        const void* addend, void* d_x, float* partial, int64_t rows, int64_t H,
-                       int nb, hipStream_t s) {
+                       int nb, GateTail tail, hipStream_t s) {
   const int64_t nv = H / (VEC ? PkVec16<T>::N : 1);
   const int64_t cpt = pk_ceil_div(nv, kRowThreads);
   const dim3 grid((unsigned)nb);
   if constexpr (VEC) {
 #define PK_NORM_BWD_WAVE(V)                                                                                       \
-  PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_bwd_wave_kernel<T, V>), grid, dim3(kRowThreads), 0, s, \
-                    (const T*)d_y, (const T*)x, (const T*)weight, rstd, (const T*)addend, (T*)d_x, partial, rows, H)
+  PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_bwd_wave_kernel<T, V>), dim3((unsigned)(nb + tail.blocks())), dim3(kRowThreads), 0, s, \
+                    (const T*)d_y, (const T*)x, (const T*)weight, rstd, (const T*)addend, (T*)d_x, partial, rows, H, nb, tail)
     if (nv <= 64 * kNormWaveVecs) {
       if (nv <= 64) { PK_NORM_BWD_WAVE(1); }
       else if (nv <= 128) { PK_NORM_BWD_WAVE(2); }
@@ -442,6 +447,8 @@ int rmsnorm_bwd_launch(const void* d_y, const void* x, const void* weight, const
     }
 #undef PK_NORM_BWD_WAVE
   }
+  const int rc = launch_gate_tail(tail, s);
+  if (rc != PK_OK) return rc;
 #define PK_NORM_BWD(C)                                                                                       \
   PK_LAUNCH_NOCHECK(pk_timing::K_RMSNORM_BWD, s, (rmsnorm_bwd_kernel<T, VEC, C>), grid, dim3(kRowThreads), 0, s, \
                     (const T*)d_y, (const T*)x, (const T*)weight, rstd, (const T*)addend, (T*)d_x, partial, rows, H)
@@ -607,9 +614,21 @@ int64_t pk_rmsnorm_bwd_workspace_bytes(int64_t T, int64_t H) {
 int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight, const float* rstd,
                    const void* d_x_addend, void* d_x, void* d_weight, int accumulate, int64_t T,
                    int64_t H, void* workspace, int64_t workspace_bytes, pk_stream_t stream) {
+  return pk_rmsnorm_bwd_with_tail(d_y, x, dtype, weight, rstd, d_x_addend, d_x, d_weight, accumulate, T, H, workspace, workspace_bytes,
+                                  GateTail{}, (hipStream_t)stream);
+}
+
+}  // extern "C"
+
+int pk_rmsnorm_bwd_with_tail(const void* d_y, const void* x, int dtype, const void* weight, const float* rstd, const void* d_x_addend,
+                             void* d_x, void* d_weight, int accumulate, int64_t T, int64_t H, void* workspace, int64_t workspace_bytes,
+                             const GateTail& tail, hipStream_t s) {
   if (T < 0 || H <= 0 || !pk_dtype_ok(dtype)) return PK_ERR_ARG;
   // no rows: their sum is zero
-  if (T == 0) return d_weight ? rmsnorm_dw_reduce(dtype, nullptr, 0, d_weight, H, accumulate, (hipStream_t)stream) : PK_OK;
+  if (T == 0) {
+    const int rc = launch_gate_tail(tail, s);
+    return rc == PK_OK && d_weight ? rmsnorm_dw_reduce(dtype, nullptr, 0, d_weight, H, accumulate, s) : rc;
+  }
   if (!d_y || !x || !weight || !rstd || !d_x) return PK_ERR_ARG;
   if (T > 0x7fffffffll) return PK_ERR_SHAPE;
   const bool vec = vec_ok(dtype, H, {d_y, x, weight, d_x, d_x_addend});
@@ -622,14 +641,13 @@ int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight
     if (!workspace || workspace_bytes < pk_rmsnorm_bwd_workspace_bytes(T, H)) return PK_ERR_WORKSPACE;
     partial = reinterpret_cast<float*>(workspace);
   }
-  hipStream_t s = (hipStream_t)stream;
   int rc;
   if (dtype == PK_BF16)
-    rc = vec ? rmsnorm_bwd_launch<bf16_t, true>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, s)
-             : rmsnorm_bwd_launch<bf16_t, false>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, s);
+    rc = vec ? rmsnorm_bwd_launch<bf16_t, true>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, tail, s)
+             : rmsnorm_bwd_launch<bf16_t, false>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, tail, s);
   else
-    rc = vec ? rmsnorm_bwd_launch<float, true>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, s)
-             : rmsnorm_bwd_launch<float, false>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, s);
+    rc = vec ? rmsnorm_bwd_launch<float, true>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, tail, s)
+             : rmsnorm_bwd_launch<float, false>(d_y, x, weight, rstd, d_x_addend, d_x, partial, T, H, nb, tail, s);
   if (rc == PK_ERR_UNSUPPORTED) {
     const dim3 rows_grid((unsigned)T), cols_grid((unsigned)pk_ceil_div(H, 256));
     if (dtype == PK_BF16) {
@@ -645,5 +663,3 @@ int pk_rmsnorm_bwd(const void* d_y, const void* x, int dtype, const void* weight
   if (rc != PK_OK) return rc;
   return d_weight ? rmsnorm_dw_reduce(dtype, partial, nb, d_weight, H, accumulate, s) : PK_OK;
 }
-
-}  // extern "C"

@@ -285,3 +285,41 @@ def test_router_backward_in_one_call_matches_the_three_calls(dev, dtype, T, H, E
              dtype_code(dtype), ptr(w), ptr(rows), ptr(got_x), ptr(got_w), ptr(got_b), 0, ptr(got_l), T, H, E, K, ptr(ws), ws.numel(),
              current_stream(dev))
         assert torch.equal(got_l, d_logits) and torch.equal(got_x, want_x) and torch.equal(got_w, want_w) and torch.equal(got_b, want_b)
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("dtype,T,H,E,K", [(torch.bfloat16, 1, 8, 4, 2), (torch.float32, 33, 136, 8, 3), (torch.bfloat16, 2100, 256, 132, 4),
+                                           (torch.float32, 2048, 2052, 4, 1), (torch.bfloat16, 300, 70, 12, 9), (torch.bfloat16, 40, 8200, 8, 2)])
+def test_router_and_norm_backward_share_launches(dev, dtype, T, H, E, K, accumulate):
+    """pk_region_router_norm_bwd: everything that pk_region_router_bwd and pk_rmsnorm_bwd give one after the other, bit for
+    bit, with the gate's gradients split or not, the bias in one or two steps, and rows that fit a wave or do not."""
+    from piper_amd import _lib
+    from piper_amd._lib import call, current_stream, dtype_code, ptr
+    g = torch.Generator().manual_seed(T + H)
+    x, rows, addend = (torch.randn(n, H, generator=g).to(dtype).to(dev) for n in (T, T * K, T))
+    w = (torch.randn(E, H, generator=g) * 0.02).to(dev)
+    norm_w = torch.randn(H, generator=g).to(dtype).to(dev)
+    xn, rstd = ops.rmsnorm_fwd(x, norm_w, 1e-6)
+    logits, d_s = torch.randn(T, E, generator=g).to(dev), torch.randn(T, K, generator=g).to(dev)
+    _, idx = ops.route_topk(logits, K, True)
+    inv = ops.sort_by_expert(idx, E)[3]
+    old_w, old_b, old_n = torch.randn(E, H, generator=g).to(dev), torch.randn(E, generator=g).to(dev), torch.randn(H, generator=g).to(dtype).to(dev)
+    lib, code, stream = _lib.load(), dtype_code(dtype), current_stream(dev)
+
+    def run(entry, ws_bytes, middle, norm):
+        out = [torch.empty_like(logits), torch.empty_like(x), old_w.clone(), old_b.clone(), torch.empty_like(x), old_n.clone()]
+        d_l, d_xn, d_w, d_b, d_x, d_n = out
+        ws = torch.empty(int(ws_bytes), dtype=torch.uint8, device=dev)
+        call(entry, ptr(logits), ptr(idx), ptr(d_s), None, 0, ptr(inv), 1, 1.5, ptr(xn), code, ptr(w), ptr(rows), ptr(d_xn), ptr(d_w),
+             ptr(d_b), int(accumulate), ptr(d_l), *([ptr(t) for t in (x, norm_w, rstd, addend, d_x, d_n)] if middle else []), T, H, E, K,
+             ptr(ws), ws.numel(), stream)
+        if norm:
+            nws = torch.empty(int(lib.pk_rmsnorm_bwd_workspace_bytes(T, H)), dtype=torch.uint8, device=dev)
+            call("pk_rmsnorm_bwd", ptr(d_xn), ptr(x), code, ptr(norm_w), ptr(rstd), ptr(addend), ptr(d_x), ptr(d_n), int(accumulate), T, H,
+                 ptr(nws), nws.numel(), stream)
+        return out
+
+    want = run("pk_region_router_bwd", lib.pk_region_router_bwd_workspace_bytes(T, H, E, code), False, True)
+    got = run("pk_region_router_norm_bwd", lib.pk_region_router_norm_bwd_workspace_bytes(T, H, E, code), True, False)
+    for name, a, b in zip(("d_logits", "d_xn", "d_w_gate", "d_gate_bias", "d_x", "d_norm_weight"), got, want):
+        assert torch.equal(a, b), name
