@@ -159,6 +159,14 @@ PK_API int pk_gate_route_sort(const void* x, int x_dtype, const float* w_gate, c
                        int32_t* inv_perm, int32_t* order, void* workspace, int64_t workspace_bytes,
                        pk_stream_t stream);
 
+/* pk_rmsnorm_fwd (x, norm_weight, eps -> xn, rstd; rstd may be NULL) and pk_gate_route_sort of xn, with the same results:
+ * up to a few thousand tokens the norm shares the gate's launch.  workspace as for pk_gate_route_sort. */
+PK_API int pk_norm_gate_route_sort(const void* x, int x_dtype, const void* norm_weight, float eps, void* xn, float* rstd,
+                            const float* w_gate, const float* gate_bias, int64_t T, int64_t H, int64_t E, int64_t K,
+                            int route_norm, float route_scale, float* logits, float* top_scores, int32_t* top_idx,
+                            int32_t* counts, int32_t* starts, int32_t* perm, int32_t* inv_perm, int32_t* order,
+                            void* workspace, int64_t workspace_bytes, pk_stream_t stream);
+
 /* pk_sort_by_expert for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same
  * inputs, outputs and result as pk_sort_by_expert; the per-chunk histograms live in a fixed array

@@ -45,6 +45,9 @@ SIGNATURES = {
     "pk_gate_route_sort_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "pk_gate_route_sort": (_c_int, [_p, _c_int, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p, _p, _p, _p, _p, _p,
                                     _p, _c_i64, _p]),
+    # x dtype norm_w eps xn rstd w_gate bias T H E K norm scale logits scores idx counts starts perm inv order ws ws_bytes stream
+    "pk_norm_gate_route_sort": (_c_int, [_p, _c_int, _p, _c_f32, _p, _p, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p,
+                                         _p, _p, _p, _p, _p, _p, _c_i64, _p]),
     "pk_route_topk_bwd": (_c_int, [_p, _p, _p, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p]),
     "pk_gate_bwd_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "pk_gate_logits_bwd": (_c_int, [_p, _p, _c_int, _p, _p, _p, _p, _c_int, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),

@@ -308,14 +308,19 @@ Tensor region_forward(const Shape& s, PyObject* route, Saved& sv, bool keep_gu, 
   int32_t *const starts = r.i32(sv.starts), *const perm = r.i32(sv.perm);
   int32_t* const order = for_backward ? r.i32(sv.order) : nullptr;      // only the weight gradient asks for it
   const void* xin = x.data_ptr();
-  if (norm_w.defined()) {
-    PK_CALL(pk_rmsnorm_fwd, xin, s.dtype, ptr(norm_w), (float)s.eps, r.at_(sv.xn), m.f32(sv.rstd), s.T, s.H, st);
-    xin = r.at_(sv.xn);
-  }
   if (route) {
+    if (norm_w.defined()) {
+      PK_CALL(pk_rmsnorm_fwd, xin, s.dtype, ptr(norm_w), (float)s.eps, r.at_(sv.xn), m.f32(sv.rstd), s.T, s.H, st);
+      xin = r.at_(sv.xn);
+    }
     PK_CALL(pk_gate_logits, xin, s.dtype, fptr(w_gate), fptr(bias), m.f32(sv.logits), s.T, s.H, s.E, tmp.at_(ws), ws_bytes, st);
     route_in_python(route, s, sv, x);
     PK_CALL(pk_sort_by_expert, m.i32(sv.idx), s.A, s.E, nullptr, starts, perm, m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
+  } else if (norm_w.defined()) {
+    PK_CALL(pk_norm_gate_route_sort, xin, s.dtype, ptr(norm_w), (float)s.eps, r.at_(sv.xn), m.f32(sv.rstd), fptr(w_gate), fptr(bias), s.T, s.H,
+            s.E, s.K, s.route_norm, (float)s.route_scale, m.f32(sv.logits), m.f32(sv.scores), m.i32(sv.idx), nullptr, starts, perm,
+            m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);
+    xin = r.at_(sv.xn);
   } else {
     PK_CALL(pk_gate_route_sort, xin, s.dtype, fptr(w_gate), fptr(bias), s.T, s.H, s.E, s.K, s.route_norm, (float)s.route_scale, m.f32(sv.logits),
             m.f32(sv.scores), m.i32(sv.idx), nullptr, starts, perm, m.i32(sv.inv), order, tmp.at_(ws), ws_bytes, st);

@@ -73,9 +73,19 @@ template <>
 __device__ __forceinline__ bf16_t pk_from_float<bf16_t>(float v) { return (bf16_t)v; }  // RNE
 
 // Wave-wide (64 lanes) butterfly reductions; every lane ends with the result.
+// The sum stays on the vector ALU: lanes 32 and 16 apart meet by swapping halves of two copies, lanes 8 to 1 apart by
+// rotating rows of 16 and permuting quads (after the steps before, lane i + 4 of a row holds what lane i ^ 4 does).  The
+// additions are those of a shuffle by 32, 16, .. 1; each shuffle is a round trip through the LDS.
 __device__ __forceinline__ float pk_wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, PK_WAVE);
+  const auto add = [](auto r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+  v = add(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+  v = add(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+#define PK_STEP(CTRL) v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true))
+  PK_STEP(0x128);   // row_ror 8
+  PK_STEP(0x124);   // row_ror 4
+  PK_STEP(0x4e);    // quad_perm 2 3 0 1
+  PK_STEP(0xb1);    // quad_perm 1 0 3 2
+#undef PK_STEP
   return v;
 }
 __device__ __forceinline__ float pk_wave_max(float v) {

@@ -59,7 +59,69 @@ struct GatePartials {
   int splits;
 };
 
-// One wave per token.  Lane l owns experts l, l+64, ... (EPL of them).
+// Top-k of NT tokens by one wave (two at a time hide each other's latency).  Lane l owns experts l, l+64, ... (EPL of
+// them): `val` their logits (0 past the last expert).  Lanes below K get the score and the expert of the k-th choice.
+template <int EPL, int NT>
+__device__ __forceinline__ void topk_of(const float (&val)[NT][EPL], int lane, int E, int K, int route_norm, float route_scale,
+                                        float (&out_s)[NT], int (&out_e)[NT]) {
+  uint32_t key[NT][EPL];
+  float vmax[NT], my_v[NT];
+  int my_e[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    vmax[n] = my_v[n] = 0.f;
+    my_e[n] = 0;
+#pragma unroll
+    for (int j = 0; j < EPL; ++j)
+      key[n][j] = lane + 64 * j < E ? orderable(val[n][j]) : 0u;  // 0 never wins: no value maps to it (the smallest, -inf, maps to 0x007fffff)
+  }
+  for (int k = 0; k < K; ++k) {
+    uint32_t best[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      best[n] = 0u;
+#pragma unroll
+      for (int j = 0; j < EPL; ++j) best[n] = key[n][j] > best[n] ? key[n][j] : best[n];
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) best[n] = wave_max_u32(best[n]);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      // the lowest expert id among those that hold the maximum: ids are lane + 64 j
+      int e_win = 0;
+      bool found = false;
+#pragma unroll
+      for (int j = 0; j < EPL; ++j) {
+        const unsigned long long at = __ballot(key[n][j] == best[n]);
+        if (!found && at != 0ull) {
+          found = true;
+          const int l = (int)__ffsll((long long)at) - 1;
+          e_win = l + 64 * j;
+          if (lane == l) key[n][j] = 0u;
+        }
+      }
+      const float v_win = from_orderable(best[n]);
+      if (k == 0) vmax[n] = v_win;
+      if (lane == k) { my_v[n] = v_win; my_e[n] = e_win; }
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    float part = 0.f;
+#pragma unroll
+    for (int j = 0; j < EPL; ++j)
+      if (lane + 64 * j < E) part += expf(val[n][j] - vmax[n]);
+    const float denom = wave_sum_f32(part);
+    float s = (lane < K) ? expf(my_v[n] - vmax[n]) / denom : 0.f;
+    if (route_norm) {
+      const float S = wave_sum_f32(s);
+      s = s / (S + 1e-20f);
+    }
+    out_s[n] = s * route_scale;
+    out_e[n] = my_e[n];
+  }
+}
+
 // PARTIALS: the logits are still split-K partial results; they are summed here (in split order, then
 // the bias: what reduce_partials_kernel would store) and written out on the way, which saves a launch
 // and a pass over [T, E].
@@ -67,8 +129,8 @@ template <int EPL, bool PARTIALS>
 __device__ __forceinline__ void route_topk_token(int t, int lane, const GatePartials gp, float* __restrict__ logits, int T, int E, int K,
                                                  int route_norm, float route_scale, float& out_s, int& out_e) {
   float* row = logits + (int64_t)t * E;
-  float val[EPL];
-  uint32_t key[EPL];
+  float val[1][EPL], score[1];
+  int expert[1];
   if (PARTIALS) {
     const int64_t n = (int64_t)T * E;
 #pragma unroll
@@ -86,60 +148,16 @@ __device__ __forceinline__ void route_topk_token(int t, int lane, const GatePart
         if (gp.bias) s += gp.bias[e];
         row[e] = s;
       }
-      val[j] = s;
+      val[0][j] = s;
     }
   }
+  if (!PARTIALS) {
 #pragma unroll
-  for (int j = 0; j < EPL; ++j) {
-    const int e = lane + 64 * j;
-    if (e < E) {
-      if (!PARTIALS) val[j] = row[e];
-      key[j] = orderable(val[j]);
-    } else {
-      val[j] = 0.f;
-      key[j] = 0u;  // never wins: no value maps to 0 (the smallest, -inf, maps to 0x007fffff)
-    }
+    for (int j = 0; j < EPL; ++j) val[0][j] = lane + 64 * j < E ? row[lane + 64 * j] : 0.f;
   }
-
-  float vmax = 0.f;
-  float my_v = 0.f;
-  int my_e = 0;
-  for (int k = 0; k < K; ++k) {
-    uint32_t best = 0u;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) best = key[j] > best ? key[j] : best;
-    best = wave_max_u32(best);
-    // the lowest expert id among those that hold the maximum: ids are lane + 64 j
-    int e_win = 0;
-    bool found = false;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-      const unsigned long long at = __ballot(key[j] == best);
-      if (!found && at != 0ull) {
-        found = true;
-        const int l = (int)__ffsll((long long)at) - 1;
-        e_win = l + 64 * j;
-        if (lane == l) key[j] = 0u;
-      }
-    }
-    const float v_win = from_orderable(best);
-    if (k == 0) vmax = v_win;
-    if (lane == k) { my_v = v_win; my_e = e_win; }
-  }
-
-  float part = 0.f;
-#pragma unroll
-  for (int j = 0; j < EPL; ++j)
-    if (lane + 64 * j < E) part += expf(val[j] - vmax);
-  const float denom = wave_sum_f32(part);
-
-  float s = (lane < K) ? expf(my_v - vmax) / denom : 0.f;
-  if (route_norm) {
-    const float S = wave_sum_f32(s);
-    s = s / (S + 1e-20f);
-  }
-  out_s = s * route_scale;
-  out_e = my_e;
+  topk_of<EPL, 1>(val, lane, E, K, route_norm, route_scale, score, expert);
+  out_s = score[0];
+  out_e = expert[0];
 }
 
 template <int EPL, bool PARTIALS>
@@ -256,7 +274,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_bwd_kernel(
 }
 
 // ------------------------------------------------------------------ counting sort
-constexpr int kSortChunk = 512;  // flat slots per chunk; one wave walks a chunk in order
+constexpr int kSortChunk = 512;  // flat slots per chunk
 
 __global__ __launch_bounds__(64) void sort_hist_kernel(const int32_t* __restrict__ idx, int A,
                                                        int E, int32_t* __restrict__ chunk_hist) {
@@ -357,15 +375,17 @@ constexpr int kSmallSortWaves = 16, kSmallSortSlots = 4096, kSmallSortExperts = 
 struct SortOut {
   int32_t *counts, *starts, *perm, *inv_perm, *order;     // counts, inv_perm, order may be null
 };
+template <int WAVES, int EXPERTS>
 struct SmallSortLds {
-  int32_t hist[kSmallSortWaves * kSmallSortExperts];      // [wave][E]
-  int32_t cnt[kSmallSortExperts], rank[kSmallSortExperts], wave_sums[kSmallSortWaves];
+  int32_t hist[WAVES * EXPERTS];      // [wave][E]
+  int32_t cnt[EXPERTS], rank[EXPERTS], wave_sums[WAVES];
 };
-__device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, const SortOut& out, SmallSortLds& l) {
+template <int WAVES, int EXPERTS>
+__device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, const SortOut& out, SmallSortLds<WAVES, EXPERTS>& l) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int per = ((A + kSmallSortWaves - 1) / kSmallSortWaves + 63) & ~63;      // slots per wave
+  const int per = ((A + WAVES - 1) / WAVES + 63) & ~63;      // slots per wave
   const int s0 = wave * per;
-  for (int i = threadIdx.x; i < kSmallSortWaves * E; i += blockDim.x) l.hist[i] = 0;
+  for (int i = threadIdx.x; i < WAVES * E; i += blockDim.x) l.hist[i] = 0;
   __syncthreads();
   for (int i = lane; i < per; i += 64) {
     const int s = s0 + i;
@@ -379,12 +399,12 @@ __device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, con
   int total = 0;
   if (e < E) {
 #pragma unroll
-    for (int w = 0; w < kSmallSortWaves; ++w) total += l.hist[w * E + e];
+    for (int w = 0; w < WAVES; ++w) total += l.hist[w * E + e];
   }
   const int start = block_exclusive_scan(total, l.wave_sums);
   if (e < E) {
     int run = start;
-    for (int w = 0; w < kSmallSortWaves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const int n = l.hist[w * E + e];
       l.hist[w * E + e] = run;
       run += n;
@@ -399,7 +419,7 @@ __device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, con
   if (out.order) write_order(l.cnt, l.rank, E, out.order);
 }
 __global__ __launch_bounds__(64 * kSmallSortWaves) void sort_small_kernel(const int32_t* __restrict__ idx, int A, int E, const SortOut out) {
-  __shared__ SmallSortLds l;
+  __shared__ SmallSortLds<kSmallSortWaves, kSmallSortExperts> l;
   sort_small(idx, A, E, out, l);
 }
 // Top-k and sort in one launch for a decode step: the 16 waves take the tokens in turn and hand the
@@ -409,7 +429,7 @@ template <int EPL, bool PARTIALS>
 __global__ __launch_bounds__(64 * kSmallSortWaves) void route_sort_small_kernel(const GatePartials gp, float* __restrict__ logits, int T, int E, int K,
                                                                                 int route_norm, float route_scale, float* __restrict__ top_scores,
                                                                                 int32_t* __restrict__ top_idx, const SortOut out) {
-  __shared__ SmallSortLds l;
+  __shared__ SmallSortLds<kSmallSortWaves, kSmallSortExperts> l;
   __shared__ int32_t chosen[kRouteSortSlots];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int t = wave; t < T; t += kSmallSortWaves) {
@@ -491,7 +511,7 @@ __global__ __launch_bounds__(1024) void sort_scan_kernel(int32_t* __restrict__ c
 // out of the L2, which is quicker than sort_scan_kernel in between that everybody waits for -- and then
 // places its chunk with four waves.  Workgroup 0 also writes counts, starts and order.  What is read grows
 // with the square of the chunks, so SCANNED leaves it to sort_scan_kernel beyond self_scan_chunks.
-constexpr int kScatterThreads = 1024, kScatterWaves = kSortChunk / 128;
+constexpr int kScatterThreads = 1024, kScatterWaves = 4;
 // Where the two ways meet.  The whole sort, us, without -> with the scan kernel:
 //   experts      513 chunks       1,024 chunks     2,048 chunks      8,192 chunks
 //        8      12.2 -> 16.4      15.6 -> 19.5     30.0 -> 25.7       191 -> 65
@@ -500,7 +520,7 @@ constexpr int kScatterThreads = 1024, kScatterWaves = kSortChunk / 128;
 //    1,024       159 -> 171        410 -> 269      1537 -> 472
 inline int self_scan_chunks(int64_t E) { return E <= 16 ? 1024 : 512; }
 template <bool SCANNED>
-__global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int32_t* __restrict__ idx, int A, int E,
+__global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int32_t* __restrict__ idx, int A, int E, int chunk_slots,
                                                                        const int32_t* __restrict__ chunk_hist, int nchunks,
                                                                        int32_t* __restrict__ counts, int32_t* __restrict__ starts,
                                                                        int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm,
@@ -538,9 +558,10 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
     }
   }
   // the wave's own share of the chunk, counted before anything is placed
-  const int s0 = chunk * kSortChunk + wave * 128;
+  const int per = ((chunk_slots + kScatterWaves - 1) / kScatterWaves + 63) & ~63;      // slots of a wave
+  const int s0 = chunk * chunk_slots + wave * per, n = min(per, chunk_slots - wave * per);
   if (wave < kScatterWaves)
-    for (int i = lane; i < 128; i += 64) {
+    for (int i = lane; i < n; i += 64) {
       const int s = s0 + i;
       if (s < A) {
         const int e = idx[s];
@@ -555,9 +576,9 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
     int run = SCANNED ? chunk_hist[(int64_t)chunk * E + e] : start + before[e];
 #pragma unroll
     for (int w = 0; w < kScatterWaves; ++w) {
-      const int n = cursor[w * E + e];
+      const int placed = cursor[w * E + e];
       cursor[w * E + e] = run;
-      run += n;
+      run += placed;
     }
     if (!SCANNED && chunk == 0) {
       if (counts) counts[e] = total;
@@ -566,8 +587,255 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
     }
   }
   __syncthreads();
-  if (wave < kScatterWaves) place_slots(idx, s0, 128, A, E, id_bits_for(E), cursor + wave * E, perm, inv_perm);
+  if (wave < kScatterWaves) place_slots(idx, s0, n, A, E, id_bits_for(E), cursor + wave * E, perm, inv_perm);
   if (!SCANNED && chunk == 0 && order) write_order(cnt, before, E, order);
+}
+
+// ------------------------------------------------------------------ norm, gate and top-k in one launch
+// A workgroup takes 16 tokens through the whole front of the region: the norm (its rows stay in LDS), the gate's
+// products, softmax and top-k, and the histogram of the chosen experts that sort_scatter_kernel wants.  With 16 tokens or
+// fewer it sorts as well.  What it replaces is four or five launches of 3 to 14 us each that are mostly latency: see
+// front_ok for where it pays.
+// The products are those of pk_x3mm::kernel, plane by plane and split by split, so that the logits are the same bit for
+// bit: a wave takes one split of the reduction for 32 experts, splits the weights into their three planes on the way
+// through LDS that only it uses (no barriers), and the waves' sums are added in the order of the splits.  Half of a
+// 32 x 32 MFMA tile has no tokens; with 32 a workgroup there are half as many workgroups, and the matrix cores are not
+// what is waited for: splitting the weights, once per 16 tokens, is.
+constexpr int kFrontTokens = 16, kFrontWaves = 8, kFrontExperts = 128, kFrontMaxVecs = 4;
+constexpr int64_t kFrontRowBytes = 64 * kFrontMaxVecs * 16;      // a row of x: 4 KB, 64 KB of LDS for 16 of them
+struct Front {
+  const void* x;              // [T, H]
+  const void* norm_w;         // [H], or nullptr: no norm
+  void* xn;                   // the norm's outputs
+  float* rstd;                //   (optional)
+  const float* w;
+  const float* bias;          // optional
+  float* logits;
+  float* top_scores;          // nullptr: logits only
+  int32_t* top_idx;
+  int32_t* chunk_hist;        // [workgroups][E], optional
+  int32_t T, H, E, K, route_norm, sort;
+  int32_t splits, kchunk;     // of the reduction: as many, and as deep, as pk_x3mm::kernel has them
+  float eps, route_scale;
+  SortOut out;                // sort: one workgroup has all tokens
+};
+__host__ __device__ inline int front_row_stride(int H, int es) { return (H + 31) / 32 * 32 * es + 16; }
+inline size_t front_lds_bytes(int64_t H, int es, int experts_padded) {
+  const size_t rows = (size_t)kFrontTokens * front_row_stride((int)H, es);
+  const size_t sums = (size_t)(kFrontWaves + 1) * kFrontTokens * experts_padded * sizeof(float);
+  return rows > sums ? rows : sums;
+}
+template <typename TX, int ET, int VECS>      // tiles of 32 experts; 16-byte vectors of a row that a lane holds
+__global__ __launch_bounds__(64 * kFrontWaves) void gate_front_kernel(const Front p) {
+  constexpr int N = PkVec16<TX>::N, ES = (int)sizeof(TX), EP = 32 * ET, EPL = (EP + 63) / 64;
+  constexpr int PA = pk_x3mm::Planes<TX>::N, PB = 3, LDK = pk_x3mm::LDK;
+  extern __shared__ __attribute__((aligned(16))) char front_lds[];
+  __shared__ int32_t hist[kFrontExperts];
+  __shared__ int32_t chosen[kRouteSortSlots];
+  __shared__ SmallSortLds<kFrontWaves, kFrontExperts> sort_lds;
+  __shared__ __attribute__((aligned(16))) bf16_t planes_lds[kFrontWaves][PB][32 * LDK];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = p.H, nv = H / N, ld = front_row_stride(H, ES);
+  const int t0 = blockIdx.x * kFrontTokens;
+
+  // ---- everything that does not depend on anything is requested first: the rows, the norm's weight, the first piece of the
+  // gate's (no branch in between, or the compiler waits for all of it at the first use).  Past an end: the last one again.
+  constexpr int ROWS = kFrontTokens / kFrontWaves;
+  typedef decltype(PkVec16<TX>::v) vec_t;
+  PkVec16<TX> v[ROWS][VECS], nw[VECS];
+#pragma unroll
+  for (int h = 0; h < ROWS; ++h) {
+    const vec_t* src = reinterpret_cast<const vec_t*>(reinterpret_cast<const TX*>(p.x) + (int64_t)min(t0 + wave + h * kFrontWaves, p.T - 1) * H);
+#pragma unroll
+    for (int m = 0; m < VECS; ++m) v[h][m].v = src[min(lane + 64 * m, nv - 1)];
+  }
+  {
+    const vec_t* src = reinterpret_cast<const vec_t*>(p.norm_w ? p.norm_w : p.x);
+#pragma unroll
+    for (int m = 0; m < VECS; ++m) nw[m].v = src[min(lane + 64 * m, nv - 1)];
+  }
+  // the wave's q-th share: split z of the reduction for 32 experts from 32 tile on (pieces: 32-deep steps; 0: no share)
+  const int tiles = (p.E + 31) / 32;
+  auto share = [&](int q, int& z, int& tile, int& k0, int& pieces) {
+    const int i = wave + q * kFrontWaves;
+    z = i % p.splits;
+    tile = i / p.splits;
+    k0 = z * p.kchunk;
+    pieces = tile < tiles ? (min(p.kchunk, H - k0) + 31) >> 5 : 0;
+  };
+  struct Regs { floatx4_t w[4]; };      // 32 rows of w, 32 deep: eight lanes to a row
+  auto request = [&](Regs& q, int tile, int k0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = min(32 * tile + 8 * i + (lane >> 3), p.E - 1), k = k0 + 4 * (lane & 7);      // (a column that is not stored)
+      q.w[i] = *reinterpret_cast<const floatx4_t*>(p.w + (int64_t)e * H + (k < H ? k : 0));      // (set to zero below)
+    }
+  };
+  int z, tile, k0, pieces;
+  share(0, z, tile, k0, pieces);
+  Regs cur;
+  request(cur, min(tile, tiles - 1), k0 < H ? k0 : 0);
+
+  // ---- rows into LDS, normalised on the way: y = x * rstd * w as rmsnorm_fwd_kernel computes it, with the sums of its four
+  // waves kept apart and added in its order, so that the result is the same bit for bit
+#pragma unroll
+  for (int h = 0; h < ROWS; ++h)
+#pragma unroll
+    for (int m = 0; m < VECS; ++m)
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (lane + 64 * m >= nv) v[h][m].set(i, 0.f);
+  if (p.norm_w) {
+    float rs[ROWS];
+#pragma unroll
+    for (int h = 0; h < ROWS; ++h) {
+      float ss[4] = {0.f, 0.f, 0.f, 0.f}, sum = 0.f;
+#pragma unroll
+      for (int m = 0; m < VECS; ++m)
+#pragma unroll
+        for (int i = 0; i < N; ++i) ss[m & 3] = fmaf(v[h][m].get(i), v[h][m].get(i), ss[m & 3]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sum += c < VECS ? pk_wave_sum(ss[c]) : 0.f;
+      rs[h] = rsqrtf(sum / (float)H + p.eps);
+    }
+#pragma unroll
+    for (int h = 0; h < ROWS; ++h)
+#pragma unroll
+      for (int m = 0; m < VECS; ++m)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[h][m].set(i, (v[h][m].get(i) * rs[h]) * nw[m].get(i));
+#pragma unroll
+    for (int h = 0; h < ROWS; ++h) {
+      const int t = t0 + wave + h * kFrontWaves;
+      if (t >= p.T) continue;
+      if (lane == 0 && p.rstd) p.rstd[t] = rs[h];
+      vec_t* const dst = reinterpret_cast<vec_t*>(reinterpret_cast<TX*>(p.xn) + (int64_t)t * H);
+#pragma unroll
+      for (int m = 0; m < VECS; ++m)
+        if (lane + 64 * m < nv) dst[lane + 64 * m] = v[h][m].v;
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < ROWS; ++h) {
+    char* const row = front_lds + (wave + h * kFrontWaves) * ld;
+#pragma unroll
+    for (int m = 0; m < VECS; ++m)
+      if (lane + 64 * m < nv) reinterpret_cast<vec_t*>(row)[lane + 64 * m] = v[h][m].v;
+    if (H + lane < (H + 31) / 32 * 32) reinterpret_cast<TX*>(row)[H + lane] = pk_from_float<TX>(0.f);
+  }
+  if (tid < kFrontExperts) hist[tid] = 0;
+  __syncthreads();
+
+  // ---- products
+  auto& planes = planes_lds[wave];
+  float keep[ET][8];
+#pragma unroll
+  for (int q = 0; q < ET; ++q) {
+    floatx16_t acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    int z2, tile2, k2, pieces2;
+    share(q + 1, z2, tile2, k2, pieces2);
+    if (pieces <= 0 && q + 1 < ET && pieces2 > 0) request(cur, tile2, k2);      // (a split past the end)
+    for (int n = 0; n < pieces; ++n, k0 += 32) {
+      const Regs now = cur;
+      if (n + 1 < pieces) request(cur, tile, k0 + 32);
+      else if (q + 1 < ET && pieces2 > 0) request(cur, tile2, k2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pk_x3mm::Raw<float> raw;
+        raw.v = now.w[i];
+        if (k0 + 4 * (lane & 7) >= H) pk_x3mm::zero_raw<float>(raw);
+        bf16x4_t pl[PB];
+        pk_x3mm::to_planes<float>(raw, pl);
+#pragma unroll
+        for (int b = 0; b < PB; ++b) *reinterpret_cast<bf16x4_t*>(&planes[b][(8 * i + (lane >> 3)) * LDK + 4 * (lane & 7)]) = pl[b];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int kk = 0; kk < 32; kk += 16) {
+        bf16x8_t a[PA], b[PB];
+        const TX* src = reinterpret_cast<const TX*>(front_lds + (lane & 15) * ld) + k0 + kk + 8 * (lane >> 5);      // rows 16..31: again
+        if constexpr (PA == 1) {
+          a[0] = *reinterpret_cast<const bf16x8_t*>(src);
+        } else {
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            pk_x3mm::Raw<float> raw;
+            raw.v = *reinterpret_cast<const floatx4_t*>(src + 4 * half);
+            bf16x4_t pl[PB];
+            pk_x3mm::to_planes<float>(raw, pl);
+#pragma unroll
+            for (int c = 0; c < PA; ++c)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) a[c][4 * half + i] = pl[c][i];
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < PB; ++c) b[c] = pk_x3mm::frag_kc(planes[c], 0, kk, lane);
+#pragma unroll
+        for (int s = PA + PB - 2; s >= 0; --s)      // small terms first
+#pragma unroll
+          for (int pa = 0; pa < PA; ++pa) {
+            const int pb = s - pa;
+            if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa], b[pb], acc, 0, 0, 0);
+          }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) keep[q][i] = acc[i];
+    z = z2; tile = tile2; k0 = k2; pieces = pieces2;
+  }
+  __syncthreads();                         // the rows have been read for the last time
+  // keep[q][i]: token 8 (i / 4) + 4 (l / 32) + i % 4, expert l % 32 of the q-th share
+  float* const part = reinterpret_cast<float*>(front_lds);                       // [split][token][EP]
+  float* const sums = part + kFrontWaves * kFrontTokens * EP;                    // [token][EP]
+#pragma unroll
+  for (int q = 0; q < ET; ++q) {
+    share(q, z, tile, k0, pieces);
+    if (tile < tiles) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        part[(z * kFrontTokens + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * EP + 32 * tile + (lane & 31)] = keep[q][i];
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < kFrontTokens * EP; i += 64 * kFrontWaves) {
+    const int r = i / EP, e = i % EP;
+    float s = 0.f;
+    for (int w = 0; w < p.splits; ++w) s += part[w * kFrontTokens * EP + i];
+    if (e < p.E) {
+      if (p.bias) s += p.bias[e];
+      if (t0 + r < p.T) p.logits[(int64_t)(t0 + r) * p.E + e] = s;
+    }
+    sums[i] = s;
+  }
+  if (!p.top_scores) return;
+  __syncthreads();
+  float val[ROWS][EPL], score[ROWS];
+  int expert[ROWS];
+#pragma unroll
+  for (int h = 0; h < ROWS; ++h)
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) val[h][j] = lane + 64 * j < p.E ? sums[(wave + h * kFrontWaves) * EP + lane + 64 * j] : 0.f;
+  topk_of<EPL, ROWS>(val, lane, p.E, p.K, p.route_norm, p.route_scale, score, expert);
+#pragma unroll
+  for (int h = 0; h < ROWS; ++h) {
+    const int64_t t = t0 + wave + h * kFrontWaves;
+    if (t < p.T && lane < p.K) {
+      p.top_scores[t * p.K + lane] = score[h];
+      p.top_idx[t * p.K + lane] = expert[h];
+      if (p.sort) chosen[t * p.K + lane] = expert[h];
+      else atomicAdd(&hist[expert[h]], 1);
+    }
+  }
+  if (!p.sort && !p.chunk_hist) return;
+  __syncthreads();
+  if (p.sort) sort_small(chosen, p.T * p.K, p.E, p.out, sort_lds);
+  else if (tid < p.E) p.chunk_hist[(int64_t)blockIdx.x * p.E + tid] = hist[tid];
 }
 
 __global__ __launch_bounds__(1024) void counts_to_starts_kernel(const void* __restrict__ counts,
@@ -739,6 +1007,14 @@ static int gate_fwd_splits(int64_t H) {
   return (int)(sp < 1 ? 1 : (sp > 8 ? 8 : sp));
 }
 
+// The reduction is split only as far as it takes to give every CU two workgroups: each split
+// writes and re-reads a [T, E] fp32 partial result, which soon outweighs reading x.
+static int gate_splits(int64_t T, int64_t H) {
+  int sp = gate_fwd_splits(H);
+  while (sp > 1 && pk_ceil_div(T, 64) * (sp / 2) >= 512) sp /= 2;
+  return sp;
+}
+
 static int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
 // bytes of the three bf16 planes of an fp32 array of n elements (0: cannot be pre-split)
 static int64_t plane_bytes(int64_t n) { return n % 4 == 0 ? align256(3 * n * (int64_t)sizeof(bf16_t)) : 0; }
@@ -807,6 +1083,60 @@ __global__ __launch_bounds__(256) void gate_small_kernel(const T* __restrict__ x
   }
 }
 
+// Whether gate_front_kernel takes a gate of these sizes: a rule on (T, H, E) and the gate's operands alone, so that every
+// entry point with a gate in it gives the same logits.  Every workgroup reads all of w_gate and splits it, 0.14 us for
+// 1,024 elements, beside some 8 us that do not depend on it; the launches it replaces take 10 us at a few tokens (and twice
+// the time on the host) and 17 to 30 at hundreds, whatever the weight's size.  Norm, gate, top-k and, beyond 16 tokens,
+// the sort's histogram, us, those -> this one:
+//     4 tokens,  808 x   8 experts 10.7 -> 11.2      1,030 tokens, 1000 x 24 experts 21.9 -> 12.0
+//   129 tokens,  408 x  16 (fp32)  16.5 -> 11.2      3,655 tokens,  768 x 64         25.8 -> 15.1
+// 2,048 tokens, 2048 x  16         23.2 -> 17.2        509 tokens, 2048 x 128        24.2 -> 43.5
+constexpr int64_t kFrontMaxTokens = 8192;
+static bool front_ok(const void* x, int x_dtype, const void* w_gate, int64_t T, int64_t H, int64_t E) {
+  const int64_t es = (int64_t)pk_dtype_size(x_dtype);
+  if (T <= 0 || T > kFrontMaxTokens || E > kFrontExperts || H % (16 / es) != 0 || H * es > kFrontRowBytes || !pk_aligned16(x) ||
+      !pk_aligned16(w_gate))
+    return false;
+  return E * H <= (T <= kGateSmallMax ? 32 * 1024 : 96 * 1024);
+}
+// Whether the sort goes by its histograms of 16 tokens each: every workgroup of sort_scatter_kernel reads all of them
+// (229 of 64 experts: 8.2 us against 5.3 + 6.0 with histograms of 512 slots in a launch of their own).
+static bool front_sorts(int64_t T, int64_t E) { return pk_ceil_div(T, kFrontTokens) * E <= 16 * 1024; }
+static int launch_front(const Front& p, int x_dtype, hipStream_t s) {
+  const dim3 grid((unsigned)pk_ceil_div(p.T, kFrontTokens)), block(64 * kFrontWaves);
+  const int vecs = (int)pk_ceil_div(p.H * (int64_t)pk_dtype_size(x_dtype), 64 * 16);
+#define PK_FRONT(TYPE, ET, VECS)                                                                                        \
+  PK_LAUNCH_NOCHECK(pk_timing::K_GATE_LOGITS, s, (gate_front_kernel<TYPE, ET, VECS>), grid, block,                      \
+                    front_lds_bytes(p.H, (int)sizeof(TYPE), 32 * ET), s, p)
+#define PK_FRONT_VECS(TYPE, ET)                   \
+  do {                                            \
+    if (vecs <= 1) PK_FRONT(TYPE, ET, 1);         \
+    else if (vecs <= 2) PK_FRONT(TYPE, ET, 2);    \
+    else PK_FRONT(TYPE, ET, 4);                   \
+  } while (0)
+#define PK_FRONT_TYPE(TYPE)                       \
+  do {                                            \
+    if (p.E <= 32) PK_FRONT_VECS(TYPE, 1);        \
+    else if (p.E <= 64) PK_FRONT_VECS(TYPE, 2);   \
+    else PK_FRONT_VECS(TYPE, 4);                  \
+  } while (0)
+  if (x_dtype == PK_BF16) PK_FRONT_TYPE(bf16_t);
+  else PK_FRONT_TYPE(float);
+#undef PK_FRONT_TYPE
+#undef PK_FRONT_VECS
+#undef PK_FRONT
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+static Front front_params(const void* x, const float* w_gate, const float* gate_bias, float* logits, int64_t T, int64_t H, int64_t E) {
+  Front p = {};
+  p.x = x; p.w = w_gate; p.bias = gate_bias; p.logits = logits;
+  p.T = (int32_t)T; p.H = (int32_t)H; p.E = (int32_t)E;
+  p.splits = gate_splits(T, H);
+  p.kchunk = (int32_t)pk_ceil_div(pk_ceil_div(H, p.splits), pk_x3mm::BK) * pk_x3mm::BK;
+  return p;
+}
+
 // The gate GEMM.  *splits > 1: `workspace` holds that many partial results [T, E] and logits is not
 // written yet (no bias either); otherwise the logits are complete.
 static int gate_gemm(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, float* logits, int64_t T, int64_t H,
@@ -815,6 +1145,7 @@ static int gate_gemm(const void* x, int x_dtype, const float* w_gate, const floa
   *splits = 1;
   if (T == 0) return PK_OK;
   if (!x || !w_gate || !logits) return PK_ERR_ARG;
+  if (front_ok(x, x_dtype, w_gate, T, H, E)) return launch_front(front_params(x, w_gate, gate_bias, logits, T, H, E), x_dtype, s);
   if (T <= kGateSmallMax && H % 4 == 0 && pk_aligned16(x) && pk_aligned16(w_gate)) {
     const dim3 grid((unsigned)pk_ceil_div(E, 4), (unsigned)pk_ceil_div(T, T == 1 ? 1 : kGateTokens)), block(256);
 #define PK_GATE_SMALL(TYPE, N)                                                                                                  \
@@ -826,11 +1157,7 @@ static int gate_gemm(const void* x, int x_dtype, const float* w_gate, const floa
     PK_RETURN_IF_LAUNCH_FAILED();
     return PK_OK;
   }
-  int sp = gate_fwd_splits(H);
-  // the reduction is split only as far as it takes to give every CU two workgroups: each split
-  // writes and re-reads a [T, E] fp32 partial result, which soon outweighs reading x
-  const int64_t row_tiles = pk_ceil_div(T, 64);
-  while (sp > 1 && row_tiles * (sp / 2) >= 512) sp /= 2;
+  int sp = gate_splits(T, H);
   if (sp > 1 && (!workspace || workspace_bytes < gate_fwd_partial_bytes(T, H, E))) sp = 1;
   // (Handing this GEMM the weight already split into bf16 planes does not shorten it: the kernel
   // waits on its loads and barriers, not on the instructions of the split.)
@@ -1070,6 +1397,12 @@ int pk_gate_route(const void* x, int x_dtype, const float* w_gate, const float* 
   if (K <= 0) return PK_ERR_ARG;
   if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E) return PK_ERR_SHAPE;
   if (T > 0 && (!top_scores || !top_idx)) return PK_ERR_ARG;
+  if (H > 0 && E > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits && front_ok(x, x_dtype, w_gate, T, H, E)) {
+    Front p = front_params(x, w_gate, gate_bias, logits, T, H, E);
+    p.top_scores = top_scores; p.top_idx = top_idx;
+    p.K = (int32_t)K; p.route_norm = route_norm; p.route_scale = route_scale;
+    return launch_front(p, x_dtype, (hipStream_t)stream);
+  }
   int splits = 1;
   const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, (hipStream_t)stream, &splits);
   if (rc != PK_OK || T == 0) return rc;
@@ -1239,14 +1572,14 @@ int pk_sort_by_expert(const int32_t* top_idx, int64_t A, int64_t E, int32_t* cou
   const size_t lds = (size_t)(2 + kScatterWaves) * E * sizeof(int32_t);
   if (nchunks <= self_scan_chunks(E)) {
     PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel<false>, dim3(nchunks), dim3(kScatterThreads), lds, s, top_idx, (int)A, (int)E,
-                      chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
+                      kSortChunk, chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
     PK_RETURN_IF_LAUNCH_FAILED();
     return PK_OK;
   }
   PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCAN, s, sort_scan_kernel, dim3(1), dim3(1024), 0, s, chunk_hist, nchunks, (int)E, counts, starts, order);
   PK_RETURN_IF_LAUNCH_FAILED();
   PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel<true>, dim3(nchunks), dim3(kScatterThreads), lds, s, top_idx, (int)A, (int)E,
-                    chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
+                    kSortChunk, chunk_hist, nchunks, counts, starts, perm, inv_perm, order);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
@@ -1254,24 +1587,53 @@ int pk_sort_by_expert(const int32_t* top_idx, int64_t A, int64_t E, int32_t* cou
 int64_t pk_gate_route_sort_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K) {
   if (T < 0 || H <= 0 || E <= 0 || K <= 0) return PK_ERR_ARG;
   const int64_t gate = pk_gate_workspace_bytes(T, H, E), sort = pk_sort_workspace_bytes(T * K, E);
-  return gate > sort ? gate : sort;
+  const int64_t front = pk_ceil_div(T, kFrontTokens) * E * (int64_t)sizeof(int32_t);      // histograms of gate_front_kernel
+  const int64_t most = gate > sort ? gate : sort;
+  return T <= kFrontMaxTokens && E <= kFrontExperts && front > most ? front : most;
 }
 
-int pk_gate_route_sort(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, int64_t T, int64_t H, int64_t E,
-                       int64_t K, int route_norm, float route_scale, float* logits, float* top_scores, int32_t* top_idx,
-                       int32_t* counts, int32_t* starts, int32_t* perm, int32_t* inv_perm, int32_t* order, void* workspace,
-                       int64_t workspace_bytes, pk_stream_t stream) {
+}  // extern "C"
+
+// norm_w: the norm whose output (xn, written) the gate reads; nullptr: it reads x
+static int norm_gate_route_sort(const void* x, int x_dtype, const void* norm_w, float eps, void* xn, float* rstd, const float* w_gate,
+                                const float* gate_bias, int64_t T, int64_t H, int64_t E, int64_t K, int route_norm, float route_scale,
+                                float* logits, float* top_scores, int32_t* top_idx, int32_t* counts, int32_t* starts, int32_t* perm,
+                                int32_t* inv_perm, int32_t* order, void* workspace, int64_t workspace_bytes, pk_stream_t stream) {
   if (T < 0 || K <= 0 || E <= 0) return PK_ERR_ARG;
   if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E || T > 0x7fffffffll / K) return PK_ERR_SHAPE;
   if (!starts || !workspace || (T > 0 && (!top_scores || !top_idx || !perm))) return PK_ERR_ARG;
   if (workspace_bytes < pk_gate_route_sort_workspace_bytes(T, H, E, K)) return PK_ERR_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  if (H > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits && front_ok(x, x_dtype, w_gate, T, H, E) &&
+      (!norm_w || (xn && pk_aligned16(norm_w) && pk_aligned16(xn)))) {
+    Front p = front_params(x, w_gate, gate_bias, logits, T, H, E);
+    p.norm_w = norm_w; p.eps = eps; p.xn = xn; p.rstd = rstd;
+    p.top_scores = top_scores; p.top_idx = top_idx;
+    p.K = (int32_t)K; p.route_norm = route_norm; p.route_scale = route_scale;
+    p.out = SortOut{counts, starts, perm, inv_perm, order};
+    p.sort = T <= kFrontTokens ? 1 : 0;
+    p.chunk_hist = p.sort || !front_sorts(T, E) ? nullptr : reinterpret_cast<int32_t*>(workspace);
+    const int rc = launch_front(p, x_dtype, s);
+    if (rc != PK_OK || p.sort) return rc;
+    if (!p.chunk_hist) return pk_sort_by_expert(top_idx, T * K, E, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
+    const int nchunks = (int)pk_ceil_div(T, kFrontTokens);
+    PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel<false>, dim3(nchunks), dim3(kScatterThreads),
+                      (size_t)(2 + kScatterWaves) * E * sizeof(int32_t), s, top_idx, (int)(T * K), (int)E, (int)(kFrontTokens * K), p.chunk_hist,
+                      nchunks, counts, starts, perm, inv_perm, order);
+    PK_RETURN_IF_LAUNCH_FAILED();
+    return PK_OK;
+  }
+  if (norm_w) {
+    const int rc = pk_rmsnorm_fwd(x, x_dtype, norm_w, eps, xn, rstd, T, H, stream);
+    if (rc != PK_OK) return rc;
+    x = xn;
+  }
   if (T == 0 || T > kRouteSortTokens || T * K > kRouteSortSlots || E > kSmallSortExperts) {
     const int rc = pk_gate_route(x, x_dtype, w_gate, gate_bias, T, H, E, K, route_norm, route_scale, logits, top_scores, top_idx, workspace,
                                  workspace_bytes, stream);
     if (rc != PK_OK) return rc;
     return pk_sort_by_expert(top_idx, T * K, E, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
   }
-  hipStream_t s = (hipStream_t)stream;
   int splits = 1;
   const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, s, &splits);
   if (rc != PK_OK) return rc;
@@ -1291,6 +1653,25 @@ int pk_gate_route_sort(const void* x, int x_dtype, const float* w_gate, const fl
 #undef PK_LAUNCH_ROUTE_SORT
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
+}
+
+extern "C" {
+
+int pk_gate_route_sort(const void* x, int x_dtype, const float* w_gate, const float* gate_bias, int64_t T, int64_t H, int64_t E,
+                       int64_t K, int route_norm, float route_scale, float* logits, float* top_scores, int32_t* top_idx,
+                       int32_t* counts, int32_t* starts, int32_t* perm, int32_t* inv_perm, int32_t* order, void* workspace,
+                       int64_t workspace_bytes, pk_stream_t stream) {
+  return norm_gate_route_sort(x, x_dtype, nullptr, 0.f, nullptr, nullptr, w_gate, gate_bias, T, H, E, K, route_norm, route_scale, logits,
+                              top_scores, top_idx, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
+}
+
+int pk_norm_gate_route_sort(const void* x, int x_dtype, const void* norm_weight, float eps, void* xn, float* rstd, const float* w_gate,
+                            const float* gate_bias, int64_t T, int64_t H, int64_t E, int64_t K, int route_norm, float route_scale,
+                            float* logits, float* top_scores, int32_t* top_idx, int32_t* counts, int32_t* starts, int32_t* perm,
+                            int32_t* inv_perm, int32_t* order, void* workspace, int64_t workspace_bytes, pk_stream_t stream) {
+  if (T < 0 || H <= 0 || !pk_dtype_ok(x_dtype) || !(eps >= 0.f) || (T > 0 && (!x || !norm_weight || !xn))) return PK_ERR_ARG;
+  return norm_gate_route_sort(x, x_dtype, norm_weight, eps, xn, rstd, w_gate, gate_bias, T, H, E, K, route_norm, route_scale, logits,
+                              top_scores, top_idx, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
 }
 
 int pk_sort_by_expert_static(const int32_t* top_idx, int64_t A, int64_t E, int32_t* counts,

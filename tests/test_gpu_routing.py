@@ -323,3 +323,42 @@ def test_router_and_norm_backward_share_launches(dev, dtype, T, H, E, K, accumul
     got = run("pk_region_router_norm_bwd", lib.pk_region_router_norm_bwd_workspace_bytes(T, H, E, code), True, False)
     for name, a, b in zip(("d_logits", "d_xn", "d_w_gate", "d_gate_bias", "d_x", "d_norm_weight"), got, want):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype,T,H,E,K,bias", [
+    (torch.bfloat16, 1, 8, 1, 1, False), (torch.float32, 15, 36, 5, 5, True), (torch.bfloat16, 16, 1000, 24, 4, False),
+    (torch.float32, 17, 2048, 16, 2, True), (torch.bfloat16, 33, 392, 17, 17, True), (torch.bfloat16, 1030, 1000, 64, 64, False),
+    (torch.bfloat16, 65, 768, 128, 8, True), (torch.float32, 500, 1028, 65, 3, False), (torch.bfloat16, 8192, 256, 32, 6, False),
+    (torch.bfloat16, 100, 2048, 24, 3, True), (torch.float32, 40, 1024, 16, 2, False), (torch.bfloat16, 4100, 256, 72, 2, False),
+    (torch.bfloat16, 70, 1032, 40, 2, True),
+    (torch.bfloat16, 64, 1032, 32, 8, True), (torch.bfloat16, 8193, 64, 8, 2, False), (torch.bfloat16, 40, 4104, 8, 2, False)])
+def test_norm_gate_topk_and_sort_in_one_call(dev, dtype, T, H, E, K, bias):
+    """pk_norm_gate_route_sort on either side of every limit of its one-launch path: bit for bit what the norm, the gate,
+    the top-k and the sort give one by one, the logits within 1e-5 of float64 on the norm's output."""
+    from piper_amd import _lib
+    from piper_amd._lib import call, current_stream, dtype_code, ptr
+    g = torch.Generator().manual_seed(T + H + E)
+    x, norm_w = torch.randn(T, H, generator=g).to(dtype).to(dev), torch.randn(H, generator=g).to(dtype).to(dev)
+    w = (torch.randn(E, H, generator=g) * 0.02).to(dev)
+    b = torch.randn(E, generator=g).to(dev) if bias else None
+    want_xn, want_rstd = ops.rmsnorm_fwd(x, norm_w, 1e-6)
+    want_l = ops.gate_logits(want_xn, w, b)
+    want_s, want_i = ops.route_topk(want_l, K, True, 1.5)
+    want_sort = ops.sort_by_expert(want_i, E, with_order=True)
+    ws = torch.empty(int(_lib.load().pk_gate_route_sort_workspace_bytes(T, H, E, K)), dtype=torch.uint8, device=dev)
+    i32 = dict(dtype=torch.int32, device=dev)
+    for norm in (True, False):
+        xn, rstd, logits, scores = torch.empty_like(x), torch.empty_like(want_rstd), torch.empty_like(want_l), torch.empty_like(want_s)
+        idx, got_sort = torch.empty_like(want_i), [torch.empty(n, **i32) for n in (E, E + 1, T * K, T * K, E)]
+        tail = [ptr(w), ptr(b), T, H, E, K, 1, 1.5, ptr(logits), ptr(scores), ptr(idx), *[ptr(t) for t in got_sort], ptr(ws), ws.numel(),
+                current_stream(dev)]
+        if norm:
+            call("pk_norm_gate_route_sort", ptr(x), dtype_code(dtype), ptr(norm_w), 1e-6, ptr(xn), ptr(rstd), *tail)
+            assert torch.equal(xn, want_xn) and torch.equal(rstd, want_rstd)
+        else:
+            call("pk_gate_route_sort", ptr(want_xn), dtype_code(dtype), *tail)
+        assert torch.equal(logits, want_l) and torch.equal(scores, want_s) and torch.equal(idx, want_i)
+        for name, a, c in zip(("counts", "starts", "perm", "inv_perm", "order"), got_sort, want_sort):
+            assert torch.equal(a, c), name
+    exact = want_xn.double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0.0)
+    assert rel_err(want_l.double().cpu(), exact) <= F32_TOL
