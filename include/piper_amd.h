@@ -186,6 +186,17 @@ PK_API int pk_sort_by_expert_static(const int32_t* top_idx, int64_t A, int64_t E
 PK_API int pk_counts_to_starts(const void* counts, int counts_is_i64, int64_t E, int32_t* starts,
                         pk_stream_t stream);
 
+/* The expert region without a backward for a few routed rows, in three launches:
+ *   out = [residual +] combine(experts(route([norm](x))))
+ * i.e. pk_norm_gate_route_sort (norm_weight NULL: pk_gate_route_sort), pk_grouped_swiglu_fwd and pk_combine_fwd up to the
+ * summation order of the products.  pk_region_decode_workspace_bytes returns 0 where it does not apply: bf16, T*K <= 16,
+ * widths in multiples of 8 (H up to 8,192).  Every operand must be 16-byte aligned; gate_bias and residual may be NULL. */
+PK_API int64_t pk_region_decode_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t I, int64_t K, int dtype);
+PK_API int pk_region_decode(const void* x, int dtype, const void* norm_weight, float eps, const float* w_gate,
+                     const float* gate_bias, const void* w1, const void* w2, const void* w3, int route_norm,
+                     float route_scale, const void* residual, void* out, int64_t T, int64_t H, int64_t E, int64_t I,
+                     int64_t K, void* workspace, int64_t workspace_bytes, pk_stream_t stream);
+
 /* ------------------------------------------------- permute / unpermute+combine */
 
 /* routed[p,:] = x[perm[p] / K, :] for p in [0,A).   (qwen3.py:250) */

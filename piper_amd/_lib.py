@@ -42,6 +42,10 @@ SIGNATURES = {
     # ... w_gate d_rows d_xn d_w d_b accumulate d_logits x norm_weight rstd addend d_x d_norm_w T H E K ws ws_bytes stream
     "pk_region_router_norm_bwd": (_c_int, [_p, _p, _p, _p, _c_i64, _p, _c_int, _c_f32, _p, _c_int, _p, _p, _p, _p, _p, _c_int, _p,
                                            _p, _p, _p, _p, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),
+    "pk_region_decode_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int]),
+    # x dtype norm_w eps w_gate bias w1 w2 w3 norm scale residual out T H E I K ws ws_bytes stream
+    "pk_region_decode": (_c_int, [_p, _c_int, _p, _c_f32, _p, _p, _p, _p, _p, _c_int, _c_f32, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                  _p, _c_i64, _p]),
     "pk_gate_route_sort_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "pk_gate_route_sort": (_c_int, [_p, _c_int, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _p, _p, _p, _p, _p, _p, _p, _p,
                                     _p, _c_i64, _p]),

@@ -18,7 +18,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libpiper_amd.so"
 HOST_PATH = PKG_DIR / "_pk_host.so"
-SOURCES = ["bucket.hip", "route.hip", "permute.hip", "grouped_gemm.hip", "timing.hip"]
+SOURCES = ["bucket.hip", "route.hip", "permute.hip", "grouped_gemm.hip", "decode.hip", "timing.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -60,6 +60,11 @@ const float* fptr(const Tensor& t) { return t.defined() ? t.data_ptr<float>() : 
 Tensor contig(const Tensor& t) { return t.defined() && !t.is_contiguous() ? t.contiguous() : t; }
 Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0; }
+bool aligned16_all(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t->defined() && !aligned16(*t)) return false;
+  return true;
+}
 
 // The stream of the current context on t's device; pk_init runs once per device before its first
 // launch, so that the launch may already sit inside a HIP graph capture.
@@ -605,11 +610,21 @@ std::optional<Tensor> expert_region(const Tensor& x, const Tensor& w_gate, const
     return RegionFn::apply(x, w_gate, bias_, w1, w2, w3, residual_, norm_w_, top_k, route_norm, route_scale, eps, route);
   const Shape s = region_shape(x, w_gate, bias, w1, w2, w3, top_k, route_norm, route_scale, eps, residual, norm_w);
   const Tensor xc = contig(x), w1c = contig(w1), w2c = contig(w2), w3c = contig(w3);
+  const Tensor gc = contig(w_gate), bc = contig(bias), rc = norm_w.defined() ? xc : contig(residual), nc = contig(norm_w);
+  // a decode step: three launches of its own, nothing sorted
+  const int64_t decode_ws = route ? 0 : pk_region_decode_workspace_bytes(s.T, s.H, s.E, s.I, s.K, s.dtype);
+  if (decode_ws > 0 && aligned16_all({&xc, &gc, &bc, &w1c, &w2c, &w3c, &rc, &nc})) {
+    Tensor out = at::empty({s.T, s.H}, x.options());
+    const Tensor ws = at::empty({decode_ws}, x.options().dtype(at::kByte));
+    PK_CALL(pk_region_decode, ptr(xc), s.dtype, ptr(nc), (float)s.eps, fptr(gc), fptr(bc), ptr(w1c), ptr(w2c), ptr(w3c), s.route_norm,
+            (float)s.route_scale, ptr(rc), ptr(out), s.T, s.H, s.E, s.I, s.K, ptr(ws), decode_ws, stream_of(x));
+    return out;
+  }
   // without a backward the pre-activations need not be written, except by the any-width kernels
   const int64_t piece = 16 / s.es;
   const bool keep_gu = s.H % piece != 0 || s.I % piece != 0 || !aligned16(xc) || !aligned16(w1c) || !aligned16(w2c) || !aligned16(w3c);
   Saved sv(s, keep_gu, norm_w.defined());
-  return region_forward(s, route, sv, keep_gu, false, xc, contig(w_gate), contig(bias), w1c, w2c, w3c, norm_w.defined() ? xc : contig(residual), contig(norm_w));
+  return region_forward(s, route, sv, keep_gu, false, xc, gc, bc, w1c, w2c, w3c, rc, nc);
 }
 
 // ------------------------------------------------------------------------------ RMSNorm

@@ -1,56 +1,14 @@
 // Routing: gate logits, wavefront softmax/top-k (+ backward), stable counting sort by expert.
 #include "pk_common.h"
 #include "gate_tail.h"
+#include "topk.h"
 #include "mfma_x3_gemm.h"
 #include <mutex>
 
 namespace {
 
 // ------------------------------------------------------------------ top-k
-// Order-preserving map float -> uint32 (larger float -> larger uint).  -0.0 is folded into
-// +0.0 and every NaN into the positive quiet NaN so that ties and NaNs behave like
-// torch.sort(descending=True, stable=True).
-__device__ __forceinline__ uint32_t orderable(float v) {
-  v = v + 0.0f;
-  uint32_t u = __float_as_uint(v);
-  if (v != v) u = 0x7fc00000u;
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float from_orderable(uint32_t o) {
-  const uint32_t u = (o & 0x80000000u) ? (o ^ 0x80000000u) : ~o;
-  return __uint_as_float(u);
-}
-
 constexpr int kRouteThreads = 256;  // 4 waves, one token per wave
-
-// Wave-wide reductions on the vector ALU: lanes are combined within rows of 16 and then across rows with
-// data-parallel-primitive operands, and lane 63 ends with the result, read back into a scalar.  Six
-// dependent instructions, where a butterfly of LDS-permute shuffles waits for the LDS six times (twelve
-// for a 64-bit value): top-8 of 128 spent most of its time in them.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
-}
-#define PK_DPP_STEPS(OP)                    \
-  OP(0x111, 0xf) /* row_shr 1 */            \
-  OP(0x112, 0xf) /* row_shr 2 */            \
-  OP(0x114, 0xf) /* row_shr 4 */            \
-  OP(0x118, 0xf) /* row_shr 8 */            \
-  OP(0x142, 0xa) /* row_bcast 15 */         \
-  OP(0x143, 0xc) /* row_bcast 31 */
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {      // identity 0
-#define PK_STEP(C, R) { const uint32_t o = dpp_or_zero<C, R>(v); v = o > v ? o : v; }
-  PK_DPP_STEPS(PK_STEP)
-#undef PK_STEP
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-__device__ __forceinline__ float wave_sum_f32(float f) {
-#define PK_STEP(C, R) f += __uint_as_float(dpp_or_zero<C, R>(__float_as_uint(f)));
-  PK_DPP_STEPS(PK_STEP)
-#undef PK_STEP
-  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(f), 63));
-}
-#undef PK_DPP_STEPS
 
 // Split-K partial results of the gate GEMM, summed by whoever reads the logits first.
 struct GatePartials {
@@ -58,69 +16,6 @@ struct GatePartials {
   const float* bias;    // [E] or nullptr
   int splits;
 };
-
-// Top-k of NT tokens by one wave (two at a time hide each other's latency).  Lane l owns experts l, l+64, ... (EPL of
-// them): `val` their logits (0 past the last expert).  Lanes below K get the score and the expert of the k-th choice.
-template <int EPL, int NT>
-__device__ __forceinline__ void topk_of(const float (&val)[NT][EPL], int lane, int E, int K, int route_norm, float route_scale,
-                                        float (&out_s)[NT], int (&out_e)[NT]) {
-  uint32_t key[NT][EPL];
-  float vmax[NT], my_v[NT];
-  int my_e[NT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    vmax[n] = my_v[n] = 0.f;
-    my_e[n] = 0;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j)
-      key[n][j] = lane + 64 * j < E ? orderable(val[n][j]) : 0u;  // 0 never wins: no value maps to it (the smallest, -inf, maps to 0x007fffff)
-  }
-  for (int k = 0; k < K; ++k) {
-    uint32_t best[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      best[n] = 0u;
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) best[n] = key[n][j] > best[n] ? key[n][j] : best[n];
-    }
-#pragma unroll
-    for (int n = 0; n < NT; ++n) best[n] = wave_max_u32(best[n]);
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      // the lowest expert id among those that hold the maximum: ids are lane + 64 j
-      int e_win = 0;
-      bool found = false;
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) {
-        const unsigned long long at = __ballot(key[n][j] == best[n]);
-        if (!found && at != 0ull) {
-          found = true;
-          const int l = (int)__ffsll((long long)at) - 1;
-          e_win = l + 64 * j;
-          if (lane == l) key[n][j] = 0u;
-        }
-      }
-      const float v_win = from_orderable(best[n]);
-      if (k == 0) vmax[n] = v_win;
-      if (lane == k) { my_v[n] = v_win; my_e[n] = e_win; }
-    }
-  }
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    float part = 0.f;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j)
-      if (lane + 64 * j < E) part += expf(val[n][j] - vmax[n]);
-    const float denom = wave_sum_f32(part);
-    float s = (lane < K) ? expf(my_v[n] - vmax[n]) / denom : 0.f;
-    if (route_norm) {
-      const float S = wave_sum_f32(s);
-      s = s / (S + 1e-20f);
-    }
-    out_s[n] = s * route_scale;
-    out_e[n] = my_e[n];
-  }
-}
 
 // PARTIALS: the logits are still split-K partial results; they are summed here (in split order, then
 // the bias: what reduce_partials_kernel would store) and written out on the way, which saves a launch
@@ -375,17 +270,15 @@ constexpr int kSmallSortWaves = 16, kSmallSortSlots = 4096, kSmallSortExperts = 
 struct SortOut {
   int32_t *counts, *starts, *perm, *inv_perm, *order;     // counts, inv_perm, order may be null
 };
-template <int WAVES, int EXPERTS>
 struct SmallSortLds {
-  int32_t hist[WAVES * EXPERTS];      // [wave][E]
-  int32_t cnt[EXPERTS], rank[EXPERTS], wave_sums[WAVES];
+  int32_t hist[kSmallSortWaves * kSmallSortExperts];      // [wave][E]
+  int32_t cnt[kSmallSortExperts], rank[kSmallSortExperts], wave_sums[kSmallSortWaves];
 };
-template <int WAVES, int EXPERTS>
-__device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, const SortOut& out, SmallSortLds<WAVES, EXPERTS>& l) {
+__device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, const SortOut& out, SmallSortLds& l) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int per = ((A + WAVES - 1) / WAVES + 63) & ~63;      // slots per wave
+  const int per = ((A + kSmallSortWaves - 1) / kSmallSortWaves + 63) & ~63;      // slots per wave
   const int s0 = wave * per;
-  for (int i = threadIdx.x; i < WAVES * E; i += blockDim.x) l.hist[i] = 0;
+  for (int i = threadIdx.x; i < kSmallSortWaves * E; i += blockDim.x) l.hist[i] = 0;
   __syncthreads();
   for (int i = lane; i < per; i += 64) {
     const int s = s0 + i;
@@ -399,12 +292,12 @@ __device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, con
   int total = 0;
   if (e < E) {
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) total += l.hist[w * E + e];
+    for (int w = 0; w < kSmallSortWaves; ++w) total += l.hist[w * E + e];
   }
   const int start = block_exclusive_scan(total, l.wave_sums);
   if (e < E) {
     int run = start;
-    for (int w = 0; w < WAVES; ++w) {
+    for (int w = 0; w < kSmallSortWaves; ++w) {
       const int n = l.hist[w * E + e];
       l.hist[w * E + e] = run;
       run += n;
@@ -419,7 +312,7 @@ __device__ __forceinline__ void sort_small(const int32_t* idx, int A, int E, con
   if (out.order) write_order(l.cnt, l.rank, E, out.order);
 }
 __global__ __launch_bounds__(64 * kSmallSortWaves) void sort_small_kernel(const int32_t* __restrict__ idx, int A, int E, const SortOut out) {
-  __shared__ SmallSortLds<kSmallSortWaves, kSmallSortExperts> l;
+  __shared__ SmallSortLds l;
   sort_small(idx, A, E, out, l);
 }
 // Top-k and sort in one launch for a decode step: the 16 waves take the tokens in turn and hand the
@@ -429,7 +322,7 @@ template <int EPL, bool PARTIALS>
 __global__ __launch_bounds__(64 * kSmallSortWaves) void route_sort_small_kernel(const GatePartials gp, float* __restrict__ logits, int T, int E, int K,
                                                                                 int route_norm, float route_scale, float* __restrict__ top_scores,
                                                                                 int32_t* __restrict__ top_idx, const SortOut out) {
-  __shared__ SmallSortLds<kSmallSortWaves, kSmallSortExperts> l;
+  __shared__ SmallSortLds l;
   __shared__ int32_t chosen[kRouteSortSlots];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int t = wave; t < T; t += kSmallSortWaves) {
@@ -593,9 +486,8 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
 
 // ------------------------------------------------------------------ norm, gate and top-k in one launch
 // A workgroup takes 16 tokens through the whole front of the region: the norm (its rows stay in LDS), the gate's
-// products, softmax and top-k, and the histogram of the chosen experts that sort_scatter_kernel wants.  With 16 tokens or
-// fewer it sorts as well.  What it replaces is four or five launches of 3 to 14 us each that are mostly latency: see
-// front_ok for where it pays.
+// products, softmax and top-k, and the histogram of the chosen experts that sort_scatter_kernel wants.  What it replaces is
+// four or five launches of 3 to 14 us each that are mostly latency: see front_ok for where it pays.
 // The products are those of pk_x3mm::kernel, plane by plane and split by split, so that the logits are the same bit for
 // bit: a wave takes one split of the reduction for 32 experts, splits the weights into their three planes on the way
 // through LDS that only it uses (no barriers), and the waves' sums are added in the order of the splits.  Half of a
@@ -614,10 +506,9 @@ struct Front {
   float* top_scores;          // nullptr: logits only
   int32_t* top_idx;
   int32_t* chunk_hist;        // [workgroups][E], optional
-  int32_t T, H, E, K, route_norm, sort;
+  int32_t T, H, E, K, route_norm;
   int32_t splits, kchunk;     // of the reduction: as many, and as deep, as pk_x3mm::kernel has them
   float eps, route_scale;
-  SortOut out;                // sort: one workgroup has all tokens
 };
 __host__ __device__ inline int front_row_stride(int H, int es) { return (H + 31) / 32 * 32 * es + 16; }
 inline size_t front_lds_bytes(int64_t H, int es, int experts_padded) {
@@ -631,8 +522,6 @@ __global__ __launch_bounds__(64 * kFrontWaves) void gate_front_kernel(const Fron
   constexpr int PA = pk_x3mm::Planes<TX>::N, PB = 3, LDK = pk_x3mm::LDK;
   extern __shared__ __attribute__((aligned(16))) char front_lds[];
   __shared__ int32_t hist[kFrontExperts];
-  __shared__ int32_t chosen[kRouteSortSlots];
-  __shared__ SmallSortLds<kFrontWaves, kFrontExperts> sort_lds;
   __shared__ __attribute__((aligned(16))) bf16_t planes_lds[kFrontWaves][PB][32 * LDK];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -828,14 +717,12 @@ __global__ __launch_bounds__(64 * kFrontWaves) void gate_front_kernel(const Fron
     if (t < p.T && lane < p.K) {
       p.top_scores[t * p.K + lane] = score[h];
       p.top_idx[t * p.K + lane] = expert[h];
-      if (p.sort) chosen[t * p.K + lane] = expert[h];
-      else atomicAdd(&hist[expert[h]], 1);
+      atomicAdd(&hist[expert[h]], 1);
     }
   }
-  if (!p.sort && !p.chunk_hist) return;
+  if (!p.chunk_hist) return;
   __syncthreads();
-  if (p.sort) sort_small(chosen, p.T * p.K, p.E, p.out, sort_lds);
-  else if (tid < p.E) p.chunk_hist[(int64_t)blockIdx.x * p.E + tid] = hist[tid];
+  if (tid < p.E) p.chunk_hist[(int64_t)blockIdx.x * p.E + tid] = hist[tid];
 }
 
 __global__ __launch_bounds__(1024) void counts_to_starts_kernel(const void* __restrict__ counts,
@@ -1083,21 +970,103 @@ __global__ __launch_bounds__(256) void gate_small_kernel(const T* __restrict__ x
   }
 }
 
+// The norm and the gate for a few tokens in one launch: a workgroup takes four experts of one token and computes the token's
+// norm for itself, as rmsnorm_fwd_kernel does (256 threads, the same sums); the products are those of gate_small_kernel,
+// so that both results are the same bit for bit.  One token, 2048 x 128 experts: 2.4 + 3.0 us in two launches, 4.5 in one.
+template <typename TX, bool NORM>
+__global__ __launch_bounds__(256) void norm_gate_small_kernel(const TX* __restrict__ x, const TX* __restrict__ norm_w, float eps, TX* __restrict__ xn,
+                                                              float* __restrict__ rstd, const float* __restrict__ w, const float* __restrict__ bias,
+                                                              float* __restrict__ logits, int H, int E) {
+  constexpr int N = PkVec16<TX>::N;
+  typedef decltype(PkVec16<TX>::v) vec_t;
+  extern __shared__ __attribute__((aligned(16))) char gate_row[];
+  __shared__ float red[16];
+  TX* const row = reinterpret_cast<TX*>(gate_row);
+  const int lane = threadIdx.x & 63, t = blockIdx.y, nv = H / N;
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
+  // the first 2,048 columns of the weight and the bias: requested in front of the norm
+  constexpr int STEPS = 8;
+  const float* const wr = w + (int64_t)min(e, E - 1) * H;
+  floatx4_t wv[STEPS];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) wv[s] = *reinterpret_cast<const floatx4_t*>(wr + min(4 * lane + 256 * s, H - 4));
+  const float b = bias ? bias[min(e, E - 1)] : 0.f;
+  const TX* const src = x + (int64_t)t * H;
+  float ss = 0.f;
+  for (int v = threadIdx.x; v < nv; v += 256) {
+    PkVec16<TX> f;
+    f.v = reinterpret_cast<const vec_t*>(src)[v];
+    reinterpret_cast<vec_t*>(row)[v] = f.v;
+    if (NORM) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) ss = fmaf(f.get(i), f.get(i), ss);
+    }
+  }
+  if (NORM) {
+    const float rs = rsqrtf(pk_block_sum(ss, red) / (float)H + eps);
+    if (rstd && blockIdx.x == 0 && threadIdx.x == 0) rstd[t] = rs;
+    for (int v = threadIdx.x; v < nv; v += 256) {
+      PkVec16<TX> f, g;
+      f.v = reinterpret_cast<vec_t*>(row)[v];
+      g.v = reinterpret_cast<const vec_t*>(norm_w)[v];
+#pragma unroll
+      for (int i = 0; i < N; ++i) f.set(i, (f.get(i) * rs) * g.get(i));
+      reinterpret_cast<vec_t*>(row)[v] = f.v;
+      if (blockIdx.x == 0) reinterpret_cast<vec_t*>(xn + (int64_t)t * H)[v] = f.v;
+    }
+  }
+  __syncthreads();
+  if (e >= E) return;
+  float acc = 0.f;
+  for (int k0 = 4 * lane; k0 < H; k0 += 256 * STEPS) {
+    float xv[STEPS][4];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) pk_f32mm::load4<TX>(row + min(k0 + 256 * s, H - 4), xv[s]);
+    if (k0 != 4 * lane) {
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) wv[s] = *reinterpret_cast<const floatx4_t*>(wr + min(k0 + 256 * s, H - 4));
+    }
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+      if (k0 + 256 * s < H) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = fmaf(xv[s][i], wv[s][i], acc);
+      }
+  }
+  acc = wave_sum_f32(acc);
+  if (lane == 0) logits[(int64_t)t * E + e] = acc + b;
+}
+
+constexpr int64_t kNormGateMaxWidth = 8192;      // columns of a row in LDS
+// (declared where it is used as well: decode.hip)
+int pk_norm_gate_small(const void* x, int dtype, const void* norm_w, float eps, void* xn, float* rstd, const float* w_gate, const float* gate_bias,
+                       float* logits, int64_t T, int64_t H, int64_t E, hipStream_t s) {
+  const dim3 grid((unsigned)pk_ceil_div(E, 4), (unsigned)T), block(256);
+#define PK_NORM_GATE(TYPE, NORM)                                                                                                  \
+  PK_LAUNCH_NOCHECK(pk_timing::K_GATE_LOGITS, s, (norm_gate_small_kernel<TYPE, NORM>), grid, block, (size_t)H * sizeof(TYPE), s, (const TYPE*)x, \
+                    (const TYPE*)norm_w, eps, (TYPE*)xn, rstd, w_gate, gate_bias, logits, (int)H, (int)E)
+  if (dtype == PK_BF16) { if (norm_w) PK_NORM_GATE(bf16_t, true); else PK_NORM_GATE(bf16_t, false); }
+  else { if (norm_w) PK_NORM_GATE(float, true); else PK_NORM_GATE(float, false); }
+#undef PK_NORM_GATE
+  PK_RETURN_IF_LAUNCH_FAILED();
+  return PK_OK;
+}
+
 // Whether gate_front_kernel takes a gate of these sizes: a rule on (T, H, E) and the gate's operands alone, so that every
 // entry point with a gate in it gives the same logits.  Every workgroup reads all of w_gate and splits it, 0.14 us for
-// 1,024 elements, beside some 8 us that do not depend on it; the launches it replaces take 10 us at a few tokens (and twice
-// the time on the host) and 17 to 30 at hundreds, whatever the weight's size.  Norm, gate, top-k and, beyond 16 tokens,
-// the sort's histogram, us, those -> this one:
-//     4 tokens,  808 x   8 experts 10.7 -> 11.2      1,030 tokens, 1000 x 24 experts 21.9 -> 12.0
-//   129 tokens,  408 x  16 (fp32)  16.5 -> 11.2      3,655 tokens,  768 x 64         25.8 -> 15.1
-// 2,048 tokens, 2048 x  16         23.2 -> 17.2        509 tokens, 2048 x 128        24.2 -> 43.5
+// 1,024 elements, beside some 8 us that do not depend on it; the launches it replaces take 17 to 30 us whatever the
+// weight's size, 8 to 13 up to 64 tokens (norm_gate_small_kernel).  Norm, gate, top-k and the sort's histogram, us,
+// those -> this one:
+//   129 tokens,  408 x  16 (fp32)  16.5 -> 11.2      1,030 tokens, 1000 x  24 experts 21.9 -> 12.0
+// 2,048 tokens, 2048 x  16         23.2 -> 17.2      3,655 tokens,  768 x  64         25.8 -> 15.1
+//   509 tokens, 2048 x 128         24.2 -> 43.5
 constexpr int64_t kFrontMaxTokens = 8192;
 static bool front_ok(const void* x, int x_dtype, const void* w_gate, int64_t T, int64_t H, int64_t E) {
   const int64_t es = (int64_t)pk_dtype_size(x_dtype);
-  if (T <= 0 || T > kFrontMaxTokens || E > kFrontExperts || H % (16 / es) != 0 || H * es > kFrontRowBytes || !pk_aligned16(x) ||
+  if (T <= kGateSmallMax || T > kFrontMaxTokens || E > kFrontExperts || H % (16 / es) != 0 || H * es > kFrontRowBytes || !pk_aligned16(x) ||
       !pk_aligned16(w_gate))
     return false;
-  return E * H <= (T <= kGateSmallMax ? 32 * 1024 : 96 * 1024);
+  return E * H <= 96 * 1024;
 }
 // Whether the sort goes by its histograms of 16 tokens each: every workgroup of sort_scatter_kernel reads all of them
 // (229 of 64 experts: 8.2 us against 5.3 + 6.0 with histograms of 512 slots in a launch of their own).
@@ -1610,11 +1579,9 @@ static int norm_gate_route_sort(const void* x, int x_dtype, const void* norm_w, 
     p.norm_w = norm_w; p.eps = eps; p.xn = xn; p.rstd = rstd;
     p.top_scores = top_scores; p.top_idx = top_idx;
     p.K = (int32_t)K; p.route_norm = route_norm; p.route_scale = route_scale;
-    p.out = SortOut{counts, starts, perm, inv_perm, order};
-    p.sort = T <= kFrontTokens ? 1 : 0;
-    p.chunk_hist = p.sort || !front_sorts(T, E) ? nullptr : reinterpret_cast<int32_t*>(workspace);
+    p.chunk_hist = front_sorts(T, E) ? reinterpret_cast<int32_t*>(workspace) : nullptr;
     const int rc = launch_front(p, x_dtype, s);
-    if (rc != PK_OK || p.sort) return rc;
+    if (rc != PK_OK) return rc;
     if (!p.chunk_hist) return pk_sort_by_expert(top_idx, T * K, E, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
     const int nchunks = (int)pk_ceil_div(T, kFrontTokens);
     PK_LAUNCH_NOCHECK(pk_timing::K_SORT_SCATTER, s, sort_scatter_kernel<false>, dim3(nchunks), dim3(kScatterThreads),
@@ -1623,20 +1590,27 @@ static int norm_gate_route_sort(const void* x, int x_dtype, const void* norm_w, 
     PK_RETURN_IF_LAUNCH_FAILED();
     return PK_OK;
   }
+  bool have_logits = false;
   if (norm_w) {
-    const int rc = pk_rmsnorm_fwd(x, x_dtype, norm_w, eps, xn, rstd, T, H, stream);
+    have_logits = T > 0 && T <= kGateSmallMax && H <= kNormGateMaxWidth && H % (16 / (int64_t)pk_dtype_size(x_dtype)) == 0 && w_gate && logits &&
+                  pk_aligned16(x) && pk_aligned16(norm_w) && pk_aligned16(xn) && pk_aligned16(w_gate);
+    const int rc = have_logits ? pk_norm_gate_small(x, x_dtype, norm_w, eps, xn, rstd, w_gate, gate_bias, logits, T, H, E, s)
+                               : pk_rmsnorm_fwd(x, x_dtype, norm_w, eps, xn, rstd, T, H, stream);
     if (rc != PK_OK) return rc;
     x = xn;
   }
   if (T == 0 || T > kRouteSortTokens || T * K > kRouteSortSlots || E > kSmallSortExperts) {
-    const int rc = pk_gate_route(x, x_dtype, w_gate, gate_bias, T, H, E, K, route_norm, route_scale, logits, top_scores, top_idx, workspace,
-                                 workspace_bytes, stream);
+    const int rc = have_logits ? pk_route_topk(logits, T, E, K, route_norm, route_scale, top_scores, top_idx, stream)
+                               : pk_gate_route(x, x_dtype, w_gate, gate_bias, T, H, E, K, route_norm, route_scale, logits, top_scores, top_idx,
+                                               workspace, workspace_bytes, stream);
     if (rc != PK_OK) return rc;
     return pk_sort_by_expert(top_idx, T * K, E, counts, starts, perm, inv_perm, order, workspace, workspace_bytes, stream);
   }
   int splits = 1;
-  const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, s, &splits);
-  if (rc != PK_OK) return rc;
+  if (!have_logits) {
+    const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, s, &splits);
+    if (rc != PK_OK) return rc;
+  }
   const GatePartials gp{splits > 1 ? reinterpret_cast<const float*>(workspace) : nullptr, gate_bias, splits};
   const SortOut out{counts, starts, perm, inv_perm, order};
   const dim3 grid(1), block(64 * kSmallSortWaves);

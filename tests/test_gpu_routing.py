@@ -330,7 +330,9 @@ def test_router_and_norm_backward_share_launches(dev, dtype, T, H, E, K, accumul
     (torch.float32, 17, 2048, 16, 2, True), (torch.bfloat16, 33, 392, 17, 17, True), (torch.bfloat16, 1030, 1000, 64, 64, False),
     (torch.bfloat16, 65, 768, 128, 8, True), (torch.float32, 500, 1028, 65, 3, False), (torch.bfloat16, 8192, 256, 32, 6, False),
     (torch.bfloat16, 100, 2048, 24, 3, True), (torch.float32, 40, 1024, 16, 2, False), (torch.bfloat16, 4100, 256, 72, 2, False),
-    (torch.bfloat16, 70, 1032, 40, 2, True),
+    (torch.bfloat16, 70, 1032, 40, 2, True), (torch.bfloat16, 24, 2048, 128, 8, True), (torch.float32, 64, 8188, 20, 3, False),
+    (torch.bfloat16, 33, 8200, 130, 2, False), (torch.float32, 65, 36, 5, 5, True), (torch.bfloat16, 81, 8, 1, 1, False),
+    (torch.bfloat16, 66, 1000, 33, 33, True),
     (torch.bfloat16, 64, 1032, 32, 8, True), (torch.bfloat16, 8193, 64, 8, 2, False), (torch.bfloat16, 40, 4104, 8, 2, False)])
 def test_norm_gate_topk_and_sort_in_one_call(dev, dtype, T, H, E, K, bias):
     """pk_norm_gate_route_sort on either side of every limit of its one-launch path: bit for bit what the norm, the gate,
