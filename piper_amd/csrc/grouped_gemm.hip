@@ -16,6 +16,7 @@
 #include "tile_gemm.h"
 #include "skinny_gemm.h"
 #include "unit_index.h"
+#include <algorithm>
 #include <functional>
 #include <initializer_list>
 #include <map>
@@ -2132,6 +2133,8 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_WG_BIG_THREADS 512
 #define PK_WG_BIG_SHORTK 256, 256, 32, 2, 4, 4
 #define PK_WG_SHORTK_ROWS 512
+// rows an expert up to which d_h is formed on the tiles of tile_gemm.h, and without transposed copies
+#define PK_DH_TILE_ROWS 40
 
 bool mfma_shape_ok(int64_t H, int64_t I) { return H % 128 == 0 && I % 128 == 0; }
 
@@ -2167,31 +2170,53 @@ int launch_rm(mf::RaggedMParams& p, int64_t A, int64_t N, int kernel_id, hipStre
 }
 
 // Whether a bf16 product with N output columns (gate and up: 2 I) goes to the persistent kernels: their
-// 128 x 256 units have to outnumber the CUs, by a quarter where the epilogue is short.  Below, a CU
-// has one unit and its whole reduction to itself and the tiles of tile_gemm.h, four to eight times as
-// many and with a split reduction, are done first.  Forward and backward of a region, all its grouped products,
-// us, these kernels -> those (rows an expert, widths, experts; units of d_h against 256 CUs):
-//     32 rows, 1024 x 512, 32 experts ( 48 units)  161 ->  91      128 rows (96 units)   204 -> 143
-//    256 rows                         (160 units)  256 -> 208      512 rows (288 units)  both at 353
-//   1024 rows, 1024 x 512,  8 experts (136 units)  315 -> 203     2048 rows, 2048 x 1024, 4 experts (264 units): d_h 86 -> 107
+// 128 x 256 units have to outnumber the CUs by so many quarters.  Below, a CU has one unit and its whole reduction to
+// itself and the tiles of tile_gemm.h, four to eight times as many, are done first; with few rows an expert most of a unit
+// is padding and the tiles, several to a CU, have more loads of the weights in flight.  All figures: us, weights from HBM,
+// persistent kernel / 128 x 128 tiles / 64 x 64 tiles (the latter two also split into what launch_ragged_m takes).
 bool wide_fills(int64_t A, int64_t N, int64_t E, int quarters) {
   return (A / 128 + (A < E ? A : E) / 2) * pk_ceil_div(N, 256) * 4 > quarters * (int64_t)mf::persistent_grid();
 }
-bool wide_gate_up(int64_t A, int64_t I, int64_t E) { return wide_fills(A, 2 * I, E, 5); }
+// Gate and up, units in rounds of the CUs, persistent / 64 x 64: few rows: 2048 x 768, 128 experts: 4 rows, 1.6 rounds
+// 169 / 145, 32 rows, 2.2 rounds 172 / 155, 64 rows, 3 rounds 183 / 185 (counts ~ 1 / sqrt(rank) 219 / 197), 96 rows,
+// 3.75 rounds 200 / 204 (216 / 215); 2048 x 1024, 64 experts, 96 rows, 2.5 rounds
+// 162 / 141.  More rows, long reduction: 2048 x 1024, 16 experts, 256 rows, 1.25 rounds 90 / 74, 384 rows, 1.75 rounds
+// 87 / 103; shorter: 1024 x 512, 64 experts, 192 rows, 2 rounds 65 / 66, 8 experts, 2,048 rows, 2.06 rounds 68 / 73,
+// 1024 x 256, 64 experts, 384 rows, 1.75 rounds 67 / 63; 512 x 256, 128 experts, 256 rows, 2.5 rounds 63 / 50, 32 experts,
+// 2,048 rows, 4.1 rounds 82 / 92.
+bool wide_gate_up(int64_t A, int64_t H, int64_t I, int64_t E) {
+  return wide_fills(A, 2 * I, E, A <= 128 * E ? 13 : H <= 512 ? 11 : H <= 1024 ? 8 : 5);
+}
+// From this size on h is formed with the hardware's exponential and reciprocal, on the persistent kernels and on the
+// tiles alike: the line between the two kernels then moves no value.
+bool hw_sigmoid(int64_t A, int64_t I, int64_t E) { return wide_fills(A, 2 * I, E, 5); }
 // At widths that are not multiples of 256 the persistent kernel has 128 x 128 units, and only a long reduction makes up for
 // them (us, those units -> tiles: 384 x 640, 64 experts, 1,536 rows 267 -> 239; 512 x 128, 8 experts, 6,000 rows 47 -> 33;
 // 1024 x 384, 128 experts, 156 rows 82 -> 75; 1024 x 640, 16 experts, 1,024 rows 80 -> 82; 2048 x 896, 32 experts, 375 rows 107 -> 125).
-bool wide_dh(int64_t A, int64_t H, int64_t I, int64_t E) { return (I % 256 == 0 || H > 1024) && wide_fills(A, I, E, 4); }
-// With few rows an expert the last 128-row unit of an expert is mostly padding as often as not, and 64-row tiles
-// are the faster ones at several units per CU: up to 512 rows with a short reduction (512 rows, 1024 x 512,
-// 32 experts: 53 -> 49; 256 rows, 512 x 256, 128 experts: 46 -> 36; 1,024 rows: 70 -> 77), up to 64 with any
-// (128 experts, 2048 x 768: 19 rows 101 -> 86, 32 rows 105 -> 90, 64 rows 111 -> 102, 111 rows 122 -> 122).
-bool wide_down(int64_t A, int64_t H, int64_t I, int64_t E) {
-  const bool short_rows = A <= (I <= 512 ? 512 : 64) * E;
-  return H % 256 == 0 && wide_fills(A, H, E, short_rows ? 16 : 5);
+// With few rows an expert the tiles are ahead at any width (2048 x 768, 128 experts: 32 rows 108 / 100 / 92, 96 rows
+// 136 / 129 / 141, 128 rows 166 / 164 / 167).
+bool wide_dh(int64_t A, int64_t H, int64_t I, int64_t E) {
+  return A > PK_DH_TILE_ROWS * E && (I % 256 == 0 || H > 1024) && wide_fills(A, I, E, 4);
 }
-// the same for a reduction of a few k-tiles (256 rows, 512 x 256, 128 experts: 58 -> 50)
-bool wide_dx(int64_t A, int64_t H, int64_t I, int64_t E) { return H % 256 == 0 && wide_fills(A, H, E, I < 512 ? 12 : 4); }
+// Down: the last 128-row unit of an expert is mostly padding as often as not, and 64- or 128-row tiles are ahead up to
+// 96 rows whatever the number of units (2048 x 768, 128 experts: 32 rows 104 / 92 / 84, 96 rows, 5 rounds 117 / 104 / 131,
+// 128 rows, 6 rounds 131 / 130 / 157, 192 rows, 8 rounds 147 / 167 / 218).  Above, the more rounds the shorter the
+// reduction: 2048 x 768, 32 experts, 192 rows, 2 rounds 61 / 46 / 58, 384 rows, 3.5 rounds 76 / 78 / 94; 2048 x 1024,
+// 4 experts, 2,048 rows, 2.06 rounds 63 / 70 / 80; 1024 x 512, 64 experts, 256 rows, 2.5 rounds 54 / 46 / 52, 512 rows, 4.5
+// rounds 71 / 73 / 93; 1024 x 256, 128 experts, 256 rows, 5 rounds 59 / 53 / 64, 512 rows, 9 rounds 88 / 91 / 115;
+// 2048 x 128, 64 experts, 384 rows, 7 rounds 67 / 55 / 60, 768 rows, 13 rounds 88 / 97 / 112.
+bool wide_down(int64_t A, int64_t H, int64_t I, int64_t E) {
+  return H % 256 == 0 && A > 96 * E && wide_fills(A, H, E, (int)std::max<int64_t>(8, 6144 / I));
+}
+// d_x, the same (2048 x 768, 128 experts: 32 rows, 3 rounds 162 / 158 / 164, 64 rows, 4 rounds 173 / 168 / 200 (counts ~ 1 /
+// sqrt(rank) 176 / 187 / 198), 128 rows 203 / 229 / 284; 2048 x 1024, 64 experts, 96 rows, 2.5 rounds 135 / 125 / 157;
+// 2048 x 1024, 16 experts, 256 rows, 1.25 rounds 80 / 85 / 84; 2048 x 768, 8 experts, 768 rows, 1.6 rounds 66 / 68 / 81;
+// 1024 x 512, 32 experts, 384 rows, 1.75 rounds 57 / 51 / 63, 64 experts, 256 rows, 2.5 rounds 76 / 75 / 89, 768 rows, 6.5
+// rounds 136 / 170 / 239; 1024 x 256, 64 experts, 384 rows, 3.5 rounds 66 / 61 / 71, 512 rows, 4.5 rounds 71 / 73 / 93;
+// 2048 x 128, 64 experts, 384 rows, 7 rounds 77 / 72 / 85, 512 rows, 9 rounds 88 / 89 / 115).
+bool wide_dx(int64_t A, int64_t H, int64_t I, int64_t E) {
+  return H % 256 == 0 && wide_fills(A, H, E, A <= 112 * E ? 15 : I >= 768 ? 4 : (int)std::max<int64_t>(8, 4096 / I));
+}
 
 bool all_aligned16(std::initializer_list<const void*> ptrs) {
   for (const void* p : ptrs)
@@ -2217,22 +2242,18 @@ bool tile_gemm_ok(int dtype, int64_t H, int64_t I, std::initializer_list<const v
 }
 
 // Expected rows of an expert that has any, if they are few enough for the weight-streaming forward
-// kernels of skinny_gemm.h; 0 otherwise.  Measured (gate/up + down, us, wide tiles -> streaming):
-//   128 experts 2048 x 768:  1 token 62 -> 20, 24 tokens 211 -> 172, 8 rows each 262 -> 257, 12 rows 266 -> 281
-//   32 experts 1024 x 512 (tiles of tile_gemm.h -> streaming): 32 rows 30 -> 52;  64 experts 1536 x 384, 48 rows 79 -> 117
-//   24 experts 1000 x 360 (against the tiles of tile_gemm.h): 21 rows each 29 -> 21, 32 rows 29 -> 31
-// Where the wide tiles have a unit for every CU they hold their own from about 8 rows per expert on, with three
-// units for every CU from 5 (their last round is full then), the smaller tiles of tile_gemm.h elsewhere from about 24.
+// kernels of skinny_gemm.h; 0 otherwise.  gate/up + down, caches cold, us, 64 x 64 tiles of tile_gemm.h -> streaming:
+//   128 experts 2048 x 768: 1 row 165 -> 157, 2 rows 204 -> 198, 3 rows 217 -> 218, 4 rows 228 -> 234, 6 rows 232 -> 249
+//   128 experts 1024 x 512: 1 row 62 -> 64, 4 rows 86 -> 91, 8 rows 88 -> 99
+//    64 experts 2048 x 768: 2 rows 120 -> 102, 8 rows 140 -> 138, 12 rows 139 -> 152
+//    64 experts 1536 x 384: 4 rows 64 -> 60, 8 rows 65 -> 65, 12 rows 57 -> 69, 24 rows 60 -> 85
+//    32 experts 1024 x 512: 2 rows 30 -> 28, 8 rows 32 -> 31, 12 rows 32 -> 34, 24 rows 33 -> 38
+//    16 experts 2048 x 1024: 8 rows 57 -> 52, 12 rows 57 -> 55, 16 rows 57 -> 59, 24 rows 58 -> 64
+//    24 experts 1000 x 360: 8 rows 28 -> 26, 12 rows 28 -> 28, 24 rows 29 -> 31
+// The streaming kernels add a product's terms in another order than the tiles, and a last bit of a forward's result decides
+// between near-tied experts in the layers behind it: the line lies where runs have had it, not at the 8 rows of the table.
 // The rule knows the mean only; an expert with many rows is walked in 16- or 32-row units that each read its weights
-// again (from the L2).  gate/up + down, caches cold, us, other kernel -> streaming, for even counts / counts ~ 1 / rank / one
-// expert in every token / the same experts in every token:
-//   128 experts 2048 x 768, 4 rows: 270 -> 268 / 243 -> 228 / 289 -> 273 / 76 -> 71
-//                           6 rows: 271 -> 278 / 273 -> 288 / 292 -> 282 / 81 -> 95
-//                           8 rows: 273 -> 287 / 272 -> 305 / 290 -> 295 / 86 -> 119
-//   128 experts 1024 x 512, 8 rows: 122 -> 120 / 123 -> 130 / 129 -> 121 / 34 -> 50
-//    64 experts 2048 x 768, 8 rows: 177 -> 167 / 179 -> 175 / 182 -> 168 / 54 -> 66
-//    64 experts 1536 x 384, 8 rows: 87 -> 84 / 86 -> 90 / 87 -> 86 / 29 -> 34;  16 rows: 86 -> 89 / 86 -> 97 / 86 -> 98 / 34 -> 40
-//    32 experts 1024 x 512, 24 rows: 46 -> 48 / 53 -> 51 / 51 -> 49 / 24 -> 28
+// again (from the L2).
 int64_t skinny_rows(int64_t A, int64_t I, int64_t E) {
   const int64_t touched = A < E ? A : E, rows = pk_ceil_div(A, touched);
   const int64_t wide_units = touched * pk_ceil_div(I, 128), cus = mf::persistent_grid();
@@ -2262,8 +2283,8 @@ int gate_up_tile(const void* x, const int32_t* row_map, int64_t div, const void*
   p.A0 = p.A1 = x; p.lda = H; p.row_map = row_map; p.map_div = pk_units::make_fastdiv(div);
   p.B0 = w1; p.B1 = w3; p.ldb = H; p.strideB = I * H;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
-  p.O0 = g; p.O1 = u; p.O2 = h; p.ldc = I;
-  return pk_tile::launch_ragged_m<T, true, pk_tile::GATE_UP>(p, A, mf::persistent_grid(), nullptr, pk_timing::K_SWIGLU_GATE_UP, s);
+  p.O0 = g; p.O1 = u; p.O2 = h; p.ldc = I; p.hw_sigmoid = mfma_shape_ok(H, I) && hw_sigmoid(A, I, E);
+  return pk_tile::launch_ragged_m<T, true, pk_tile::GATE_UP>(p, A, mf::persistent_grid(), 0, nullptr, pk_timing::K_SWIGLU_GATE_UP, s);
 }
 template <typename T>
 int down_tile(const void* h, const void* w2, const int32_t* starts, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
@@ -2272,7 +2293,8 @@ int down_tile(const void* h, const void* w2, const int32_t* starts, void* y, int
   q.B0 = q.B1 = w2; q.ldb = I; q.strideB = H * I;
   q.starts = starts; q.E = (int32_t)E; q.K = (int32_t)I; q.nseg = 1; q.N = (int32_t)H;
   q.O0 = y; q.ldc = H;
-  return pk_tile::launch_ragged_m<T, true, pk_tile::PLAIN>(q, A, mf::persistent_grid(), nullptr, pk_timing::K_SWIGLU_DOWN, s);
+  // (2048 x 768, 128 experts, 128 x 128 -> 64 x 64: 32 rows 92 -> 84, 48 rows 95 -> 93, 64 rows 97 -> 107)
+  return pk_tile::launch_ragged_m<T, true, pk_tile::PLAIN>(q, A, mf::persistent_grid(), 40, nullptr, pk_timing::K_SWIGLU_DOWN, s);
 }
 // C [A, N] = sum over nseg weight matrices [K, N] (row-major) of A_seg . B_seg
 template <typename T>
@@ -2283,7 +2305,9 @@ int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map
   p.B0 = B0; p.B1 = nseg > 1 ? B1 : B0; p.ldb = N; p.strideB = K * N;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)K; p.nseg = nseg; p.N = (int32_t)N;
   p.O0 = C; p.ldc = N;
-  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), nullptr, kernel_id, s);
+  // (1536 x 384, 64 experts, d_x, 128 x 128 -> 64 x 64: 32 rows 37 -> 31, 64 rows 41 -> 40, 96 rows 44 -> 53; with the longer
+  // reduction of 2048 x 768, 128 experts: 16 rows 153 -> 155, 32 rows 158 -> 164)
+  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), K < 512 ? 48 : 0, nullptr, kernel_id, s);
 }
 // d_h = d_y . w2[e] with the SwiGLU backward in the epilogue.  With scores: d_y is d_out, gathered through
 // row_map, and the score gradient is left as partial sums over *part_cols columns each.
@@ -2298,8 +2322,9 @@ int dh_tile(const void* dy, const int32_t* row_map, int64_t div, const float* sc
   p.O0 = d_g; p.O1 = d_u; p.O2 = hs; p.ldc = I;
   p.Gin = g; p.Uin = u; p.scores = scores; p.ds_part = parts; p.total_rows = A;
   const int id = pk_timing::K_SWIGLU_DGRAD_DH;
-  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), nullptr, id, s);
-  return pk_tile::launch_ragged_m<T, false, pk_tile::BWD_SCALED>(p, A, mf::persistent_grid(), part_cols, id, s);
+  // (2048 x 768, 128 experts, 128 x 128 -> 64 x 64: 32 rows 100 -> 92, 48 rows 107 -> 104, 64 rows 114 -> 117)
+  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), PK_DH_TILE_ROWS, nullptr, id, s);
+  return pk_tile::launch_ragged_m<T, false, pk_tile::BWD_SCALED>(p, A, mf::persistent_grid(), PK_DH_TILE_ROWS, part_cols, id, s);
 }
 template <typename T>
 int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void* dg, const void* du, const void* x,
@@ -2387,7 +2412,7 @@ int pk_grouped_swiglu_fwd(const void* x_rows, const int32_t* row_map, int64_t ro
   if (!pieces)
     return fwd_simt<bf16_t>(x_rows, row_map, row_map_div, w1, w2, w3, starts, g, u, h, y, A, H, I, E, s);
 
-  if (mfma && wide_gate_up(A, I, E)) {
+  if (mfma && wide_gate_up(A, H, I, E)) {
     mf::RaggedMParams p = {};
     p.A0 = (const bf16_t*)x_rows; p.A1 = nullptr; p.lda = H;
     p.row_map = row_map; p.map_div = mf::make_fastdiv(row_map_div);
@@ -2638,8 +2663,10 @@ int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dt
   // d_h fills the chip (32 experts 1024 x 512: 128 rows 100 -> 66, 512 rows 168 -> 158, 1,024 rows 246 -> 241).  Above,
   // the transposed pair is ahead (16 experts 2048 x 1024, 1,024 rows 369 -> 410); wgrad_kernel deals experts out
   // over the XCDs and leaves some idle below eight (4 experts 2048 x 1024, 2,048 rows 275 -> 349).
+  // With few rows an expert the copies are mostly padding, and d_h without them runs on smaller tiles (128 experts 2048 x 768,
+  // forward and backward, us, transposed -> plain: 4 rows 761 -> 715, 12 rows 814 -> 772, 62 rows 895 -> 927).
   const int64_t w2_units = E * (H / 256) * (I / 256);
-  if (w2_units < mf::persistent_grid() / 2) return 0;
+  if (w2_units < mf::persistent_grid() / 2 || A <= PK_DH_TILE_ROWS * E) return 0;
   return E < mf::NXCD || w2_units > mf::persistent_grid() || wide_fills(A, I, E, 8);
 }
 

@@ -201,6 +201,7 @@ struct RaggedM {
   int64_t ldc;
   const void* Gin;          // BWD, BWD_SCALED: g and u of the forward [rows, ldc]
   const void* Uin;
+  int32_t hw_sigmoid;       // GATE_UP, bf16: hardware exponential and reciprocal, as the persistent kernels form h
   const float* scores;      // BWD_SCALED: score of every routed slot (row_map names the slot of a sorted row)
   float* ds_part;           // BWD_SCALED: [column tiles][total_rows]: the score gradient in parts
   int64_t total_rows;
@@ -409,7 +410,13 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
         for (int t = 0; t < PIECE; ++t) {
           a[t] = pk_to_float<T>(pk_from_float<T>(a[t]));     // g and u are tensors of T
           u[t] = pk_to_float<T>(pk_from_float<T>(u[t]));
-          h[t] = (a[t] / (1.f + expf(-a[t]))) * u[t];
+        }
+        if (sizeof(T) == 2 && p.hw_sigmoid) {
+#pragma unroll
+          for (int t = 0; t < PIECE; ++t) h[t] = (a[t] * __builtin_amdgcn_rcpf(1.f + __expf(-a[t]))) * u[t];
+        } else {
+#pragma unroll
+          for (int t = 0; t < PIECE; ++t) h[t] = (a[t] / (1.f + expf(-a[t]))) * u[t];
         }
         if (live) {
           if (p.O0) store_piece<T>(reinterpret_cast<T*>(p.O0) + o, a);
@@ -461,12 +468,24 @@ inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
+// few_rows: rows an expert up to which the 64 x 64 tiles are the faster ones however many tiles there are (each
+// product's own; the caller says with what it measured).
 template <typename T, bool B_KC, int EPI>
-inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int* part_cols, int kernel_id, hipStream_t s) {
-  // 128 x 128 tiles once they give every CU work for two rounds; below that the chip is filled by
-  // four times as many 64 x 64 tiles
-  const int64_t big = (A_rows / 128 + (p.E + 1) / 2) * pk_ceil_div(p.N, 128);
-  if (big >= 2 * (int64_t)cus) return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int64_t few_rows, int* part_cols, int kernel_id, hipStream_t s) {
+  // 128 x 128 tiles halve what a product reads from LDS per multiplication, and fit a CU once or twice: they need a
+  // tile for every CU and some more (bf16, us, 64 x 64 -> 128 x 128: down, 2048 x 1024, 8 experts, 256 rows, 320 tiles
+  // 31.3 -> 28.9; 384 rows, 448 tiles 36.1 -> 28.8; 8 experts 2048 x 768, 192 rows, 256 tiles 20.6 -> 20.0;
+  // 24 experts 768 x 256, 192 rows, 288 tiles 11.2 -> 12.8), those with the SwiGLU backward half a round more
+  // (1536 x 384, 64 experts: 128 rows, 288 tiles 35.8 -> 46.0, 192 rows, 384 tiles 53.4 -> 48.4).
+  // Not for the pair of products with the SwiGLU behind it: 128 accumulator registers a wave leave one
+  // workgroup to a CU (128 experts 2048 x 768, 32 rows 155 -> 185, 256 rows 402 -> 433), and not in fp32, where the matrix
+  // cores are the bound and the finer tiles fill the last round better (16 experts 1024 x 512, 16,384 rows:
+  // gate/up 335 -> 435, down 176 -> 215, d_h 197 -> 251, d_x 340 -> 414).
+  if constexpr (sizeof(T) == 2 && EPI != GATE_UP) {
+    const int64_t big = (A_rows / 128 + (p.E + 1) / 2) * pk_ceil_div(p.N, 128);
+    if (A_rows > few_rows * p.E && 4 * big >= (EPI == PLAIN ? 5 : 6) * (int64_t)cus)
+      return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  }
   // row tiles that hold rows, about: every expert's last one is half full
   const int64_t row_tiles = A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2;
   const int64_t tiles = row_tiles * pk_ceil_div(p.N, 64), k_tiles = pk_ceil_div(p.K, kBK<T>) * p.nseg;

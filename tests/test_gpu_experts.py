@@ -600,6 +600,34 @@ def test_experts_with_few_rows_and_popular_experts(dev, experts, A):
     test_experts_with_few_rows(dev, counts.tolist(), 256, 768)
 
 
+@pytest.mark.parametrize("A", [9599, 14336, 24703])
+def test_one_more_row_takes_other_kernels_to_the_same_bits(dev, A):
+    """128 experts of 512 x 768: from these sizes on one more row takes gate/up (9,600 rows), d_x (14,337) and down (24,704)
+    from the tiles to the persistent kernels.  Both add a product's terms in the same order and form h with the
+    same sigmoid, so what the other rows get does not change; values against float64 for a few experts."""
+    H, I, E = 512, 768, 128
+    print(f"[case] one more row after {A}", flush=True)
+    x, w1, w2, w3, dy, cnt = (t.to(dev) for t in _make(43, [A // E] * (E - 1) + [A + 1 - A // E * (E - 1)], H, I, torch.bfloat16))
+    got = []
+    for n in (A, A + 1):
+        c = cnt.clone()
+        c[-1] -= A + 1 - n
+        starts = ops.counts_to_starts(c)
+        y, g, u, h = ops.grouped_swiglu_fwd(x[:n], w1, w2, w3, starts)
+        got.append((y, g, u, h) + tuple(ops.grouped_swiglu_dgrad(dy[:n], w1, w2, w3, g, u, starts)))
+    for few, more in zip(*got):
+        assert torch.equal(few, more[:A])
+    y, g, u, h = got[0][:4]
+    s = 0
+    for e in range(3):
+        r = slice(s, s + A // E)
+        ge, ue = x[r].double() @ w1[e].double().t(), x[r].double() @ w3[e].double().t()
+        he = torch.nn.functional.silu(ge) * ue
+        for name, out, ref in (("g", g, ge), ("u", u, ue), ("h", h, he), ("y", y, he @ w2[e].double().t())):
+            assert rel_err(out[r], ref) <= BF16_TOL, (name, e)
+        s += A // E
+
+
 REGION_BACKWARD_CASES = [
     # (counts, H, I): split reductions with every row and column remainder, unsplit 64-row tiles, 128-row
     # tiles, the persistent kernels at widths of 256 and 128 columns, a single row
