@@ -172,12 +172,12 @@ struct Frags {
   bf16x8_t a[TM];
   bf16x8_t b[TN];
 };
-template <int BK, int TM, int TN, bool A_KC, bool B_KC, int ACOLS, int BCOLS>
+template <int BK, int TM, int TN, bool A_KC, bool B_KC, int ACOLS, int BCOLS, int ASTEP = 32>
 __device__ __forceinline__ void load_frags(Frags<TM, TN>& f, const char* At, const char* Bt,
                                            int wrow0, int wcol0, int ks, int lane) {
 #pragma unroll
   for (int i = 0; i < TM; ++i)
-    f.a[i] = A_KC ? frag_kc<BK>(At, wrow0 + 32 * i, ks, lane) : frag_mn<ACOLS>(At, wrow0 + 32 * i, ks, lane);
+    f.a[i] = A_KC ? frag_kc<BK>(At, wrow0 + ASTEP * i, ks, lane) : frag_mn<ACOLS>(At, wrow0 + ASTEP * i, ks, lane);
 #pragma unroll
   for (int j = 0; j < TN; ++j)
     f.b[j] = B_KC ? frag_kc<BK>(Bt, wcol0 + 32 * j, ks, lane) : frag_mn<BCOLS>(Bt, wcol0 + 32 * j, ks, lane);
@@ -628,6 +628,12 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
   constexpr bool BWD = EPI == EPI_SWIGLU_BWD || EPI == EPI_SWIGLU_BWD_SCALED;
   constexpr bool SCALED = EPI == EPI_SWIGLU_BWD_SCALED;
   constexpr bool PP = NW == 8;    // two waves per SIMD: the groups of the ping-pong k-loop
+  // A wave's 32-row chunks.  d_x in 256-row units: every WMW-th chunk, so that a unit with few rows is shared by both groups,
+  // and only the chunks that hold rows are multiplied (16,384 tokens, 128 experts 2048 x 768: 759 -> 721 us; 1,024 rows
+  // each 780 -> 752, 513 rows 504 -> 463).  Elsewhere neighbours, multiplied all or not at all: spread, gate/up of 1,024 rows
+  // each goes from 808 to 822 us, d_h from 559 to 575, 128-row units by up to 2 %.
+  constexpr bool SPREAD = PP && TM == 4 && EPI == EPI_PLAIN && !B_KC;
+  constexpr int RS = SPREAD ? 32 * WMW : 32;
   constexpr int OUT_COLS = (EPI == EPI_SWIGLU) ? WTN / 2 : WTN;   // columns a wave writes per output tensor
   constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;       // output columns per tile
   constexpr int RING = NS * STAGE;
@@ -656,6 +662,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WNW, wn = wave % WNW;
+  const int wrow = SPREAD ? 32 * wm : WTM * wm;            // first row of the wave's first chunk
   // staging area while `cur_stage` is the stage of the coming unit's k-tile 0
   auto staging_area = [&](int cur_stage) -> char* {
     return ALIAS ? smem + (cur_stage == 0 ? NS - 1 : cur_stage - 1) * STAGE : smem + RING;
@@ -856,7 +863,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
     int unit_next = -1;
     next_known = false;
     ld_on_next = false;
-    const bool wave_has_rows = wm * WTM < cur_u.rows;   // waves whose row slice is empty skip the math
+    const bool wave_has_rows = wrow < cur_u.rows;   // waves whose row slice is empty skip the math
 
     floatx16_t acc[TM][TN];
 #pragma unroll
@@ -899,54 +906,102 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
       // own loads of tile t+1 have landed when the phase before 2t+2 ends: group 0 waits for them
       // at the end of C_t, group 1 at the end of M_t.
       constexpr int KS = BK / 16;
-      Frags<TM, TN> fr[KS];
       const int grp = wave / (NW / 2);
       if (grp == 1) block_barrier();
-      for (int kt = 0; kt < nkt; ++kt) {
-        // ---- memory phase
-        ld_target(cur + NS - 1 >= NS ? cur - 1 : cur + NS - 1);   // the stage of k-tile kt-1 takes k-tile kt+NS-1
-        const char* st = smem + cur * STAGE;
-        if (wave_has_rows) {
+      // a wave's own part of tile kt+1 must have landed when the phase before its first read
+      // ends: younger than it are the NS-2 tiles after it and, while tile kt+1 is one of those
+      // requested before the previous epilogue's stores, these stores
+      auto wait_next_tile = [&](int kt) {
+        if (kt <= NS - 3) wait_vm_le((NS - 2) * L + st_after);
+        else wait_dma<(NS - 2) * L>();
+      };
+      if constexpr (SPREAD) {
+        // One loop for every number of chunks with rows, all with the same barriers: a branch inside the loop costs
+        // registers (a copy of the accumulators across it), and as a version of this one the loop below does.
+        auto k_loop = [&](auto live_c) __attribute__((always_inline)) {
+          constexpr int LIVE = decltype(live_c)::value;
+          Frags<(LIVE > 0 ? LIVE : 1), TN> fr[KS];
+          for (int kt = 0; kt < nkt; ++kt) {
+            // ---- memory phase
+            ld_target(cur + NS - 1 >= NS ? cur - 1 : cur + NS - 1);   // the stage of k-tile kt-1 takes k-tile kt+NS-1
+            const char* st = smem + cur * STAGE;
+            if constexpr (LIVE > 0) {
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks)
-            load_frags<BK, TM, TN, !A_T, B_KC, BM, BN>(fr[ks], st, st + A_BYTES, wm * WTM, wn * WTN, ks, lane);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        static_for<L>([&](auto pc) { issue_piece(pc); });
-        ld_advance();
-        cur = cur + 1 == NS ? 0 : cur + 1;
-        // a wave's own part of tile kt+1 must have landed when the phase before its first read
-        // ends: younger than it are the NS-2 tiles after it and, while tile kt+1 is one of those
-        // requested before the previous epilogue's stores, these stores
-        auto wait_next_tile = [&]() {
-          if (kt <= NS - 3) wait_vm_le((NS - 2) * L + st_after);
-          else wait_dma<(NS - 2) * L>();
+              for (int ks = 0; ks < KS; ++ks)
+                load_frags<BK, LIVE, TN, !A_T, B_KC, BM, BN, RS>(fr[ks], st, st + A_BYTES, wrow, wn * WTN, ks, lane);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<L>([&](auto pc) { issue_piece(pc); });
+            ld_advance();
+            cur = cur + 1 == NS ? 0 : cur + 1;
+            if (grp == 1) wait_next_tile(kt);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            block_barrier();
+            // ---- compute phase
+            if constexpr (LIVE > 0) {
+              __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+              for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int i = 0; i < LIVE; ++i)
+#pragma unroll
+                  for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[ks].b[j], fr[ks].a[i], acc[i][j], 0, 0, 0);
+              __builtin_amdgcn_s_setprio(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (grp == 0) wait_next_tile(kt);
+            block_barrier();
+          }
         };
-        if (grp == 1) wait_next_tile();
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        block_barrier();
-        // ---- compute phase
-        if (wave_has_rows) {
-          __builtin_amdgcn_s_setprio(1);
+        const int live = min(TM, max(0, (cur_u.rows - wrow + RS - 1) / RS));
+        if (live == TM) k_loop(std::integral_constant<int, TM>{});
+        else if (live == 3) k_loop(std::integral_constant<int, 3>{});
+        else if (live == 2) k_loop(std::integral_constant<int, 2>{});
+        else if (live == 1) k_loop(std::integral_constant<int, 1>{});
+        else k_loop(std::integral_constant<int, 0>{});
+      } else {
+        Frags<TM, TN> fr[KS];
+        for (int kt = 0; kt < nkt; ++kt) {
+          // ---- memory phase
+          ld_target(cur + NS - 1 >= NS ? cur - 1 : cur + NS - 1);   // the stage of k-tile kt-1 takes k-tile kt+NS-1
+          const char* st = smem + cur * STAGE;
+          if (wave_has_rows) {
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks)
+            for (int ks = 0; ks < KS; ++ks)
+              load_frags<BK, TM, TN, !A_T, B_KC, BM, BN>(fr[ks], st, st + A_BYTES, wrow, wn * WTN, ks, lane);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          static_for<L>([&](auto pc) { issue_piece(pc); });
+          ld_advance();
+          cur = cur + 1 == NS ? 0 : cur + 1;
+          if (grp == 1) wait_next_tile(kt);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+          block_barrier();
+          // ---- compute phase
+          if (wave_has_rows) {
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+            for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-              for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[ks].b[j], fr[ks].a[i], acc[i][j], 0, 0, 0);
-          __builtin_amdgcn_s_setprio(0);
+              for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                  acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[ks].b[j], fr[ks].a[i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_s_setprio(0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if (grp == 0) wait_next_tile(kt);
+          block_barrier();
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (grp == 0) wait_next_tile();
-        block_barrier();
       }
       if (grp == 0) block_barrier();   // the whole ring is free: every fragment is in registers or used
     } else {
       Frags<TM, TN> f0;     // fragments of the first k-step of the coming k-tile, read one tile ahead
       if (wave_has_rows)
-        load_frags<BK, TM, TN, !A_T, B_KC, BM, BN>(f0, smem + cur * STAGE, smem + cur * STAGE + A_BYTES, wm * WTM, wn * WTN, 0, lane);
+        load_frags<BK, TM, TN, !A_T, B_KC, BM, BN>(f0, smem + cur * STAGE, smem + cur * STAGE + A_BYTES, wrow, wn * WTN, 0, lane);
 
       // k-tile kt+1 has to be in LDS before the MFMAs of k-tile kt: its first fragments are read
       // while they run, so that no wave waits for LDS behind the barrier of the next tile
@@ -958,7 +1013,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
         const char* st = smem + cur * STAGE;
         const char* stn = smem + (cur + 1 == NS ? 0 : cur + 1) * STAGE;
         if (wave_has_rows) {
-          mma_ktile<BK, TM, TN, !A_T, B_KC, BM, BN, L>(st, st + A_BYTES, stn, stn + A_BYTES, wm * WTM, wn * WTN, f0, acc,
+          mma_ktile<BK, TM, TN, !A_T, B_KC, BM, BN, L>(st, st + A_BYTES, stn, stn + A_BYTES, wrow, wn * WTN, f0, acc,
                                                        [&](auto pc) {
                                                          issue_piece(pc);
                                                          if constexpr (decltype(pc)::value == L - 1) ld_advance();
@@ -1000,7 +1055,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
     int lane_e = lane;      // opaque: the epilogue's per-lane addresses are formed per unit (see Stage32::flush)
     asm volatile("" : "+v"(lane_e));
     const int lrow = lane_e & 31, lq = 4 * (lane_e >> 5);
-    const int64_t grow0 = (int64_t)(cur_u.row0 + wm * WTM) * p.ldc;
+    const int64_t grow0 = (int64_t)(cur_u.row0 + wrow) * p.ldc;
     const int64_t gcol0 = (int64_t)cur_u.nt * BN_OUT + wn * OUT_COLS;
     // SwiGLU backward: the epilogue reads g and u (and, scaled, the row's combine score through the
     // row map).  Each of these is a round trip to HBM, so they are requested in batches: all scores
@@ -1013,10 +1068,10 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
     u32x2_t graw[JB][4], uraw[JB][4];
     float sc_chunk[BWD ? TM : 1];
     auto load_gu = [&](int i, int j0) {
-      const int crows = min(32, cur_u.rows - wm * WTM - 32 * i);
+      const int crows = min(32, cur_u.rows - wrow - RS * i);
       if (crows <= 0) return;
       const int rr = lrow < crows ? lrow : crows - 1;
-      const int64_t goff = grow0 + (int64_t)(32 * i) * p.ldc + gcol0 + (int64_t)rr * p.ldc + lq;
+      const int64_t goff = grow0 + (int64_t)(RS * i) * p.ldc + gcol0 + (int64_t)rr * p.ldc + lq;
 #pragma unroll
       for (int j = 0; j < JB; ++j)
 #pragma unroll
@@ -1030,9 +1085,9 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
         int slot[TM];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-          const int crows = min(32, cur_u.rows - wm * WTM - 32 * i);
+          const int crows = min(32, cur_u.rows - wrow - RS * i);
           const int rr = lrow < crows ? lrow : (crows > 0 ? crows - 1 : 0);
-          slot[i] = crows > 0 ? p.row_map[cur_u.row0 + wm * WTM + 32 * i + rr] : 0;
+          slot[i] = crows > 0 ? p.row_map[cur_u.row0 + wrow + RS * i + rr] : 0;
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i) sc_chunk[i] = p.scores[slot[i]];
@@ -1049,8 +1104,8 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int crows = min(32, cur_u.rows - wm * WTM - 32 * i);   // valid rows of this chunk
-      const int64_t goff = grow0 + (int64_t)(32 * i) * p.ldc + gcol0;
+      const int crows = min(32, cur_u.rows - wrow - RS * i);   // valid rows of this chunk
+      const int64_t goff = grow0 + (int64_t)(RS * i) * p.ldc + gcol0;
       if (EPI == EPI_SWIGLU) {
 #pragma unroll
         for (int which = 0; which < 3; ++which) {
@@ -1140,7 +1195,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
               __builtin_amdgcn_sched_barrier(0);
               prefetch_next();
             }
-            const int64_t tofs = ((int64_t)((cur_u.tcol + wm * WTM + 32 * i) >> 5) * p.ldc + gcol0 + 32 * j) * 32;
+            const int64_t tofs = ((int64_t)((cur_u.tcol + wrow + RS * i) >> 5) * p.ldc + gcol0 + 32 * j) * 32;
             wave_lds_fence();
             st_after += S2::template flush<false>(sb0, p.O0 + goff + 32 * j, p.ldc, crows, lane_e);
             st_after += S2::template flush<false>(sb1, p.O1 + goff + 32 * j, p.ldc, crows, lane_e);
@@ -1166,7 +1221,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
             // lanes l and l+32 hold the two column halves of row l % 32
             ds += __shfl_xor(ds, 32);
             if (lane_e < 32 && lrow < crows)
-              p.ds_partial[(int64_t)((cur_u.nt * BN + wn * WTN) >> 6) * p.total_rows + cur_u.row0 + wm * WTM + 32 * i + lrow] = ds;
+              p.ds_partial[(int64_t)((cur_u.nt * BN + wn * WTN) >> 6) * p.total_rows + cur_u.row0 + wrow + RS * i + lrow] = ds;
             st_after += 1;
           }
         } else if (i == TM - 1) {
@@ -1215,7 +1270,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
             // lanes l and l+32 hold the two column halves of row l % 32
             ds += __shfl_xor(ds, 32);
             if (lane < 32 && lrow < crows)
-              p.ds_partial[(int64_t)((cur_u.nt * BN + wn * WTN) >> 6) * p.total_rows + cur_u.row0 + wm * WTM + 32 * i + lrow] = ds;
+              p.ds_partial[(int64_t)((cur_u.nt * BN + wn * WTN) >> 6) * p.total_rows + cur_u.row0 + wrow + RS * i + lrow] = ds;
             st_after += 1;
           }
           const bool transposed = SCALED && p.T0 != nullptr;
@@ -1237,7 +1292,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
             if constexpr (SCALED) {
               if (transposed)
                 st_after += St::flush_t(sbuf, (which == 0 ? p.T0 : which == 1 ? p.T1 : p.T2) +
-                                                  ((int64_t)((cur_u.tcol + wm * WTM + 32 * i) >> 5) * p.ldc + gcol0) * 32,
+                                                  ((int64_t)((cur_u.tcol + wrow + RS * i) >> 5) * p.ldc + gcol0) * 32,
                                         32, crows);
             }
             wave_lds_fence();
@@ -2125,6 +2180,13 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_RM_SHORT 128, 256, 64, 2, 4, 3
 #define PK_RM_LOWM_UNITS 3
 #define PK_RM_SHORT_ROWS 512
+// d_x already with fewer rows and units: of the three products it reads most of its weights through the transposing LDS
+// read, which the taller unit halves (128 -> 256 rows, us, even / skewed counts: 128 experts 2048 x 768, 320 rows
+// 333 -> 317 / 333 -> 312, 448 rows 424 -> 376 / 422 -> 394; 272 rows 303 -> 311 / 297 -> 279; 1024 x 512, 320 rows 139 -> 142 /
+// 142 -> 142, 384 rows 165 -> 151 / 152 -> 155; 64 experts 2048 x 1024, 352 rows 245 -> 222 / 242 -> 237; 32 experts 2048 x 768,
+// 384 rows, 2.25 units per CU 117 -> 103).  gate/up and down gain as much with even counts between 128 and 200 rows, and
+// lose more with skewed ones (128 experts 2048 x 768, 144 rows: 243 -> 233 / 231 -> 247, 143 -> 133 / 133 -> 140).
+#define PK_RM_DX_ROWS 320
 // Weight gradient of the piecewise entry points (wgrad_kernel; the fused region runs
 // wgrad_pp_kernel, whose tile is fixed): 256x256x64 in a 2-stage ring; with fewer than
 // PK_WG_SHORTK_ROWS rows per expert on average 32-deep tiles in a 4-stage ring with the loads spread
@@ -2158,12 +2220,14 @@ int launch_rm(mf::RaggedMParams& p, int64_t A, int64_t N, int kernel_id, hipStre
   // 256-row tiles unless they would leave the persistent grid with only a few units per
   // workgroup (then the last round of units runs on a half-empty chip)
   const int64_t big_units = (A / 256 + p.E / 2) * p.n_tiles;
-  const bool lowm = big_units < (int64_t)PK_RM_LOWM_UNITS * mf::persistent_grid();
+  // (d_x, row-major operands: see PK_RM_DX_ROWS)
+  constexpr bool DX = EPI == mf::EPI_PLAIN && !B_KC && !A_T;
+  const bool lowm = big_units < (int64_t)(DX ? 2 : PK_RM_LOWM_UNITS) * mf::persistent_grid();
   // the scaled SwiGLU backward stays on 128-row units: its time goes into the epilogue (loads of g
   // and u, the arithmetic, six stores per value), which 256-row units do not shorten, and with
   // 128 accumulator registers that epilogue spills (measured 14 % slower at 16,384 tokens even
   // with the packed outputs staged 32 columns at a time)
-  if (EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)PK_RM_SHORT_ROWS * p.E)
+  if (EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)(DX ? PK_RM_DX_ROWS : PK_RM_SHORT_ROWS) * p.E)
     return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
   if constexpr (EPI != mf::EPI_SWIGLU_BWD_SCALED) return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
   return PK_ERR_SHAPE;
