@@ -2195,7 +2195,7 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_WG_BIG_THREADS 512
 #define PK_WG_BIG_SHORTK 256, 256, 32, 2, 4, 4
 #define PK_WG_SHORTK_ROWS 512
-// rows an expert up to which d_h is formed on the tiles of tile_gemm.h, and without transposed copies
+// rows an expert up to which d_h is formed on the tiles of tile_gemm.h
 #define PK_DH_TILE_ROWS 40
 
 bool mfma_shape_ok(int64_t H, int64_t I) { return H % 128 == 0 && I % 128 == 0; }
@@ -2258,9 +2258,9 @@ bool hw_sigmoid(int64_t A, int64_t I, int64_t E) { return wide_fills(A, 2 * I, E
 // them (us, those units -> tiles: 384 x 640, 64 experts, 1,536 rows 267 -> 239; 512 x 128, 8 experts, 6,000 rows 47 -> 33;
 // 1024 x 384, 128 experts, 156 rows 82 -> 75; 1024 x 640, 16 experts, 1,024 rows 80 -> 82; 2048 x 896, 32 experts, 375 rows 107 -> 125).
 // With few rows an expert the tiles are ahead at any width (2048 x 768, 128 experts: 32 rows 108 / 100 / 92, 96 rows
-// 136 / 129 / 141, 128 rows 166 / 164 / 167).
-bool wide_dh(int64_t A, int64_t H, int64_t I, int64_t E) {
-  return A > PK_DH_TILE_ROWS * E && (I % 256 == 0 || H > 1024) && wide_fills(A, I, E, 4);
+// 136 / 129 / 141, 128 rows 166 / 164 / 167); a call with one expert per token keeps the order of its sums (see launch_ragged_m).
+bool wide_dh(bool any_order, int64_t A, int64_t H, int64_t I, int64_t E) {
+  return (!any_order || A > PK_DH_TILE_ROWS * E) && (I % 256 == 0 || H > 1024) && wide_fills(A, I, E, 4);
 }
 // Down: the last 128-row unit of an expert is mostly padding as often as not, and 64- or 128-row tiles are ahead up to
 // 96 rows whatever the number of units (2048 x 768, 128 experts: 32 rows 104 / 92 / 84, 96 rows, 5 rounds 117 / 104 / 131,
@@ -2348,7 +2348,7 @@ int gate_up_tile(const void* x, const int32_t* row_map, int64_t div, const void*
   p.B0 = w1; p.B1 = w3; p.ldb = H; p.strideB = I * H;
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)H; p.nseg = 1; p.N = (int32_t)I;
   p.O0 = g; p.O1 = u; p.O2 = h; p.ldc = I; p.hw_sigmoid = mfma_shape_ok(H, I) && hw_sigmoid(A, I, E);
-  return pk_tile::launch_ragged_m<T, true, pk_tile::GATE_UP>(p, A, mf::persistent_grid(), 0, nullptr, pk_timing::K_SWIGLU_GATE_UP, s);
+  return pk_tile::launch_ragged_m<T, true, pk_tile::GATE_UP>(p, A, mf::persistent_grid(), false, 0, nullptr, pk_timing::K_SWIGLU_GATE_UP, s);
 }
 template <typename T>
 int down_tile(const void* h, const void* w2, const int32_t* starts, void* y, int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
@@ -2358,12 +2358,12 @@ int down_tile(const void* h, const void* w2, const int32_t* starts, void* y, int
   q.starts = starts; q.E = (int32_t)E; q.K = (int32_t)I; q.nseg = 1; q.N = (int32_t)H;
   q.O0 = y; q.ldc = H;
   // (2048 x 768, 128 experts, 128 x 128 -> 64 x 64: 32 rows 92 -> 84, 48 rows 95 -> 93, 64 rows 97 -> 107)
-  return pk_tile::launch_ragged_m<T, true, pk_tile::PLAIN>(q, A, mf::persistent_grid(), 40, nullptr, pk_timing::K_SWIGLU_DOWN, s);
+  return pk_tile::launch_ragged_m<T, true, pk_tile::PLAIN>(q, A, mf::persistent_grid(), false, 40, nullptr, pk_timing::K_SWIGLU_DOWN, s);
 }
 // C [A, N] = sum over nseg weight matrices [K, N] (row-major) of A_seg . B_seg
 template <typename T>
 int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map, int64_t div, const void* B0, const void* B1,
-               void* C, int64_t N, int nseg, const int32_t* starts, int64_t A, int64_t E, int kernel_id, hipStream_t s) {
+               void* C, int64_t N, int nseg, const int32_t* starts, bool any_order, int64_t A, int64_t E, int kernel_id, hipStream_t s) {
   pk_tile::RaggedM p = {};
   p.A0 = A0; p.A1 = nseg > 1 ? A1 : A0; p.lda = K; p.row_map = row_map; p.map_div = pk_units::make_fastdiv(div);
   p.B0 = B0; p.B1 = nseg > 1 ? B1 : B0; p.ldb = N; p.strideB = K * N;
@@ -2371,7 +2371,7 @@ int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map
   p.O0 = C; p.ldc = N;
   // (1536 x 384, 64 experts, d_x, 128 x 128 -> 64 x 64: 32 rows 37 -> 31, 64 rows 41 -> 40, 96 rows 44 -> 53; with the longer
   // reduction of 2048 x 768, 128 experts: 16 rows 153 -> 155, 32 rows 158 -> 164)
-  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), K < 512 ? 48 : 0, nullptr, kernel_id, s);
+  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), any_order, K < 512 ? 48 : 0, nullptr, kernel_id, s);
 }
 // d_h = d_y . w2[e] with the SwiGLU backward in the epilogue.  With scores: d_y is d_out, gathered through
 // row_map, and the score gradient is left as partial sums over *part_cols columns each.
@@ -2387,8 +2387,8 @@ int dh_tile(const void* dy, const int32_t* row_map, int64_t div, const float* sc
   p.Gin = g; p.Uin = u; p.scores = scores; p.ds_part = parts; p.total_rows = A;
   const int id = pk_timing::K_SWIGLU_DGRAD_DH;
   // (2048 x 768, 128 experts, 128 x 128 -> 64 x 64: 32 rows 100 -> 92, 48 rows 107 -> 104, 64 rows 114 -> 117)
-  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), PK_DH_TILE_ROWS, nullptr, id, s);
-  return pk_tile::launch_ragged_m<T, false, pk_tile::BWD_SCALED>(p, A, mf::persistent_grid(), PK_DH_TILE_ROWS, part_cols, id, s);
+  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), true, PK_DH_TILE_ROWS, nullptr, id, s);
+  return pk_tile::launch_ragged_m<T, false, pk_tile::BWD_SCALED>(p, A, mf::persistent_grid(), div > 1, PK_DH_TILE_ROWS, part_cols, id, s);
 }
 template <typename T>
 int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void* dg, const void* du, const void* x,
@@ -2507,7 +2507,7 @@ int pk_grouped_swiglu_dgrad_dh(const void* d_y, const void* w2, const void* g, c
   if (!d_y || !w2 || !g || !u || !starts || !d_g || !d_u) return PK_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_y, w2, g, u, d_g, d_u});
-  if (!(mfma && wide_dh(A, H, I, E)) && tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u}))
+  if (!(mfma && wide_dh(true, A, H, I, E)) && tile_gemm_ok(dtype, H, I, {d_y, w2, g, u, d_g, d_u}))
     return dtype == PK_F32 ? dh_tile<float>(d_y, nullptr, 1, nullptr, w2, g, u, starts, d_g, d_u, nullptr, nullptr, nullptr, A, H, I, E, s)
                            : dh_tile<bf16_t>(d_y, nullptr, 1, nullptr, w2, g, u, starts, d_g, d_u, nullptr, nullptr, nullptr, A, H, I, E, s);
   if (!mfma) {
@@ -2577,7 +2577,7 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
   }
   hipStream_t s = (hipStream_t)stream;
   const bool mfma = dtype == PK_BF16 && mfma_shape_ok(H, I) && all_aligned16({d_out, w2, g, u, d_g, d_u, hs});
-  if (n_partial && !(mfma && wide_dh(A, H, I, E)) && tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs})) {
+  if (n_partial && !(mfma && wide_dh(row_map_div > 1, A, H, I, E)) && tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs})) {
     if (!workspace || workspace_bytes < pk_region_dgrad_dh_workspace_bytes(A, I)) return PK_ERR_WORKSPACE;
     int part_cols = 0;
     rc = dtype == PK_F32 ? dh_tile<float>(d_out, row_map, row_map_div, scores, w2, g, u, starts, d_g, d_u, hs, (float*)workspace, &part_cols,
@@ -2591,9 +2591,9 @@ static int dgrad_dh_scaled_impl(const void* d_out, const int32_t* row_map, int64
     // unscaled d_h = d_out[token] . w2[e], staged in d_u's buffer; then one wave per row
     const bool tile = tile_gemm_ok(dtype, H, I, {d_out, w2, g, u, d_g, d_u, hs});
     if (tile && dtype == PK_F32)
-      rc = dgrad_tile<float>(d_out, nullptr, H, row_map, row_map_div, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s);
+      rc = dgrad_tile<float>(d_out, nullptr, H, row_map, row_map_div, w2, nullptr, d_u, I, 1, starts, row_map_div > 1, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s);
     else if (tile)
-      rc = dgrad_tile<bf16_t>(d_out, nullptr, H, row_map, row_map_div, w2, nullptr, d_u, I, 1, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s);
+      rc = dgrad_tile<bf16_t>(d_out, nullptr, H, row_map, row_map_div, w2, nullptr, d_u, I, 1, starts, row_map_div > 1, A, E, pk_timing::K_SWIGLU_DGRAD_DH, s);
     else if (dtype == PK_F32) rc = simt_ragged_m<float>(d_out, H, row_map, row_map_div, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
     else rc = simt_ragged_m<bf16_t>(d_out, H, row_map, row_map_div, w2, I, 1, H * I, d_u, I, starts, A, I, H, E, 0, s);
     if (rc) return rc;
@@ -2680,8 +2680,8 @@ static int dgrad_dx_impl(const void* d_g, const void* d_u, const void* w1, const
     // d_x = d_g . w1[e] + d_u . w3[e]   (w[e] is [I, H]: B(k=i, n=h) = w[i*H + h])
     if (tile_gemm_ok(dtype, H, I, {d_g, d_u, w1, w3, d_x_sorted}))
       return dtype == PK_F32
-                 ? dgrad_tile<float>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s)
-                 : dgrad_tile<bf16_t>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s);
+                 ? dgrad_tile<float>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, true, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s)
+                 : dgrad_tile<bf16_t>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, true, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s);
     if (dtype == PK_F32) {
       rc = simt_ragged_m<float>(d_g, I, nullptr, 1, w1, H, 1, I * H, d_x_sorted, H, starts, A, H, I, E, 0, s);
       if (rc) return rc;
@@ -2727,10 +2727,8 @@ int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dt
   // d_h fills the chip (32 experts 1024 x 512: 128 rows 100 -> 66, 512 rows 168 -> 158, 1,024 rows 246 -> 241).  Above,
   // the transposed pair is ahead (16 experts 2048 x 1024, 1,024 rows 369 -> 410); wgrad_kernel deals experts out
   // over the XCDs and leaves some idle below eight (4 experts 2048 x 1024, 2,048 rows 275 -> 349).
-  // With few rows an expert the copies are mostly padding, and d_h without them runs on smaller tiles (128 experts 2048 x 768,
-  // forward and backward, us, transposed -> plain: 4 rows 761 -> 715, 12 rows 814 -> 772, 62 rows 895 -> 927).
   const int64_t w2_units = E * (H / 256) * (I / 256);
-  if (w2_units < mf::persistent_grid() / 2 || A <= PK_DH_TILE_ROWS * E) return 0;
+  if (w2_units < mf::persistent_grid() / 2) return 0;
   return E < mf::NXCD || w2_units > mf::persistent_grid() || wide_fills(A, I, E, 8);
 }
 

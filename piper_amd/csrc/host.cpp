@@ -480,7 +480,11 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
 
     // Shapes where the K-contiguous weight-gradient path pays get d_g, d_u and score*h transposed; with long
     // experts the d_x GEMM reads its A operand from the same blocks and the row-major pair is left out.
-    const int64_t ldt = pk_region_transposed_pays(s.A, s.H, s.I, s.E, s.dtype) ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
+    // With few rows an expert the transposed copies are mostly padding, and d_h without them runs on smaller tiles (128 experts
+    // 2048 x 768, forward and backward, us, with -> without: 4 rows 761 -> 715, 12 rows 814 -> 772, 62 rows 895 -> 927).  (One
+    // expert per token: the order of the sums behind the score's gradient stays, see pk_tile::launch_ragged_m.)
+    const bool few_rows = s.K > 1 && s.A <= 40 * s.E;
+    const int64_t ldt = !few_rows && pk_region_transposed_pays(s.A, s.H, s.I, s.E, s.dtype) ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
     const bool blocks_only = ldt > 0 && pk_grouped_swiglu_dx_from_transposed_pays(s.A, s.H, s.I, s.E, s.dtype);
     // w: what the weight gradients read, t: the rest
     Block w, t;

@@ -468,10 +468,15 @@ inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
+// any_order: the sums over k (and the parts of a score gradient) may be ordered otherwise than they are with the tiles that
+// the number of 64 x 64 tiles alone selects.  A token with one expert and a normalised score has a gate gradient of zero, and what
+// is left of it in floating point is the rounding of that order: the callers keep it for the forward, which knows nothing of
+// the router, and for the score's gradient of such tokens.
 // few_rows: rows an expert up to which the 64 x 64 tiles are the faster ones however many tiles there are (each
 // product's own; the caller says with what it measured).
 template <typename T, bool B_KC, int EPI>
-inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int64_t few_rows, int* part_cols, int kernel_id, hipStream_t s) {
+inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_order, int64_t few_rows, int* part_cols, int kernel_id,
+                           hipStream_t s) {
   // 128 x 128 tiles halve what a product reads from LDS per multiplication, and fit a CU once or twice: they need a
   // tile for every CU and some more (bf16, us, 64 x 64 -> 128 x 128: down, 2048 x 1024, 8 experts, 256 rows, 320 tiles
   // 31.3 -> 28.9; 384 rows, 448 tiles 36.1 -> 28.8; 8 experts 2048 x 768, 192 rows, 256 tiles 20.6 -> 20.0;
@@ -483,17 +488,38 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, int64_t fe
   // gate/up 335 -> 435, down 176 -> 215, d_h 197 -> 251, d_x 340 -> 414).
   if constexpr (sizeof(T) == 2 && EPI != GATE_UP) {
     const int64_t big = (A_rows / 128 + (p.E + 1) / 2) * pk_ceil_div(p.N, 128);
-    if (A_rows > few_rows * p.E && 4 * big >= (EPI == PLAIN ? 5 : 6) * (int64_t)cus)
+    if (EPI == BWD_SCALED && !any_order ? big >= 2 * (int64_t)cus
+                                        : A_rows > few_rows * p.E && 4 * big >= (EPI == PLAIN ? 5 : 6) * (int64_t)cus)
       return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   // row tiles that hold rows, about: every expert's last one is half full
   const int64_t row_tiles = A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2;
   const int64_t tiles = row_tiles * pk_ceil_div(p.N, 64), k_tiles = pk_ceil_div(p.K, kBK<T>) * p.nseg;
-  // an fp32 tile is 1,024 cycles of the matrix cores per k-tile, whoever shares it: 64 x 32 tiles while
-  // even those do not outnumber the CUs (200 to 512 rows, 256 x 512: -20 %)
-  if (sizeof(T) == 4 && 2 * tiles <= cus) {
-    if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
-    return launch_tiles<T, 2, 1, 1, 1, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  // An fp32 tile of 64 x 64 is 1,024 cycles of the matrix cores per k-tile, whoever shares it, so the finer tiles win wherever
+  // the coarse ones leave CUs without one or a last round nearly empty (us, 64 x 64 with a split reduction where there
+  // are CUs for it -> the tile chosen; tiles of 64 x 64 against 256 CUs):
+  if constexpr (sizeof(T) == 4) {
+    const int64_t rows = A_rows / (A_rows < p.E ? A_rows : p.E);
+    //  32 x 32, four groups: 70 tiles, 408 x 472, d_x 23 -> 14; 96 tiles, 1024 x 512, d_h 26 -> 15; 96 tiles,
+    //  512 x 256, d_x 16 -> 10; 126 tiles, 704 x 408, d_h 22 -> 18 (64 x 32: 18)
+    if (any_order && 8 * tiles <= 3 * (int64_t)cus) return launch_tiles<T, 1, 1, 1, 1, 2, 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+    //  half as wide: 128 tiles, 1024 x 512, gate/up 44 -> 30, d_h 27 -> 22
+    if (2 * tiles <= cus) {
+      if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+      return launch_tiles<T, 2, 1, 1, 1, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+    }
+    //  half as high, where most of a tile would be padding: 64 experts 896 x 384, 8 rows, 240 tiles, gate/up 73 -> 45, 16 rows, 288
+    //  tiles 68 -> 47, d_h 43 -> 28; 64 experts 512 x 256, 8 rows, 320 tiles, down 16 -> 13, d_x 27 -> 19; 128 experts
+    //  1024 x 256, 31 rows, 504 tiles, d_h 52 -> 42, but gate/up 83 -> 97; 64 experts 896 x 384, 2 rows, 476 tiles, down 26 -> 31
+    //  (the same order as long as the 64 x 64 tiles would take two groups)
+    const bool flat = 2 * tiles <= 3 * (int64_t)cus ? rows <= 16 : (EPI == BWD || EPI == BWD_SCALED) && rows <= 32 && tiles <= 2 * (int64_t)cus;
+    if (flat && (any_order || reduction_groups(tiles, k_tiles, cus) == 2))
+      return launch_tiles<T, 1, 2, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+    //  half as wide again, where the CUs would have one or two tiles: 280 tiles, 408 x 472, d_x 47 -> 29, down 26 -> 18;
+    //  320 tiles, 1024 x 512, d_h 52 -> 40; 384 tiles, d_x 49 -> 39; but 490 tiles, 408 x 472, down 27 -> 34; gate/up, which
+    //  reads twice the weights for its rows, 320 tiles, 1024 x 512 78 -> 83
+    if (any_order && EPI != GATE_UP && tiles > cus && 2 * tiles <= 3 * (int64_t)cus && k_tiles >= 4)
+      return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   const int ks = reduction_groups(tiles, k_tiles, cus);
   if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, EPI == GATE_UP ? 2 : 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
@@ -702,8 +728,15 @@ inline int launch_ragged_k(RaggedK p, int64_t A_rows, int cus, int kernel_id, hi
     p.first[p.nprob] = (int32_t)tiles;
     return tiles * p.E;
   };
-  int64_t units = plan(128);
-  const bool large = units >= 2 * (int64_t)cus;      // as for the ragged-M tiles
+  // 128 x 128 tiles with two of them for every CU, unless they are that much more padding: in fp32 the two are within
+  // 5 % of each other (us, 64 x 64 -> 128 x 128: 16 experts 1024 x 512, 250 rows 161 -> 152; 408 x 472, 14 % more
+  // padding, 82 -> 101), in bf16 the larger are a quarter faster (24 experts 1000 x 360, 172 rows 54 -> 41)
+  int64_t units = plan(128), area_128 = 0, area_64 = 0;
+  for (int q = 0; q < p.nprob; ++q) {
+    area_128 += pk_ceil_div(p.prob[q].M, 128) * pk_ceil_div(p.prob[q].N, 128) * 4;
+    area_64 += pk_ceil_div(p.prob[q].M, 64) * pk_ceil_div(p.prob[q].N, 64);
+  }
+  const bool large = units >= 2 * (int64_t)cus && 100 * area_128 <= (sizeof(T) == 4 ? 105 : 125) * area_64;
   if (!large) units = plan(64);
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
   if (units == 0) return PK_OK;

@@ -547,6 +547,70 @@ def test_widths_without_a_multiple_of_the_wide_tiles(dev, dtype, counts, H, I):
         s += c
 
 
+FP32_TILE_CASES = [
+    # (counts, H, I), with the 64 x 64 tiles that gate/up and d_h | down and d_x would have:
+    # 84 | 96: 32 x 32 tiles
+    ([0, 1, 31, 32, 33, 63, 64, 65, 100, 131], 456, 424),
+    # 112 | 128: 64 x 32
+    ([0, 1, 31, 32, 33, 63, 64, 65, 101, 200], 504, 424),
+    # few rows an expert: 290 | 348, 32 x 64 tiles, experts with more than one of them
+    ([0, 1, 16, 15, 3, 7, 8, 9] * 5 + [0, 1, 2, 33, 3, 7, 60, 1], 712, 584),
+    # 31 rows: 527, 32 x 64 in d_h only
+    ([31] * 32, 392, 1032),
+    # 343, 64 x 32 with a split reduction in all but gate/up
+    ([100, 99, 101, 64, 136, 100] * 4, 392, 392),
+]
+
+
+@pytest.mark.parametrize("K", [1, 2])
+@pytest.mark.parametrize("counts,H,I", FP32_TILE_CASES)
+def test_fp32_tiles_by_their_number(dev, counts, H, I, K):
+    """The tiles that launch_ragged_m picks in fp32 by their number and the rows an expert, forward and region backward, for
+    calls that keep the order of their sums (one expert per token) and others, against float64 matmuls: sums of
+    n products are within n * 2^-24 of the sum of magnitudes in any order, far below F32_TOL."""
+    from piper_amd._lib import call, current_stream, dtype_code, ptr
+    from piper_amd import _lib
+    import ctypes
+    counts = list(counts)
+    counts[-1] += sum(counts) % 2
+    print(f"[case] fp32 tiles A={sum(counts)} E={len(counts)} H={H} I={I} K={K}", flush=True)
+    A, E = sum(counts), len(counts)
+    x, w1, w2, w3, d_out, cnt = (t.to(dev) for t in _make(47, counts, H, I, torch.float32))
+    x, d_out = x[:A // K], d_out[:A // K]
+    gen = torch.Generator().manual_seed(6)
+    perm = torch.randperm(A, generator=gen).to(torch.int32).to(dev)
+    scores = (torch.rand(A, generator=gen) + 0.1).to(dev)
+    starts = ops.counts_to_starts(cnt)
+    y, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts, row_map=perm, row_map_div=K)
+    dg, du, hs = (torch.full_like(g, float("nan")) for _ in range(3))
+    ds = torch.zeros(A, device=dev)
+    ws = torch.full((int(_lib.load().pk_region_dgrad_dh_workspace_bytes(A, I)) // 4,), float("nan"), device=dev)
+    n_part = ctypes.c_int64(-1)
+    call("pk_region_dgrad_dh", ptr(d_out), ptr(perm), K, ptr(scores), ptr(w2), ptr(g), ptr(u), ptr(starts), ptr(dg), ptr(du), ptr(hs), ptr(ds),
+         ctypes.addressof(n_part), ptr(ws), ws.numel() * 4, A, H, I, E, dtype_code(torch.float32), current_stream(dev))
+    ds = ws[:n_part.value * A].view(n_part.value, A).double().sum(0)
+    dx = torch.full((A, H), float("nan"), device=dev)
+    call("pk_region_dgrad_dx", ptr(dg), ptr(du), ptr(w1), ptr(w3), ptr(starts), ptr(dx), A, H, I, E, dtype_code(torch.float32), current_stream(dev))
+    rows = (perm.long() // K)
+    s = 0
+    for e, c in enumerate(counts):
+        if c == 0:
+            continue
+        r = slice(s, s + c)
+        s += c
+        xe, de, sc = x[rows[r]].double(), d_out[rows[r]].double(), scores[perm.long()[r]].double()[:, None]
+        ge, ue = xe @ w1[e].double().t(), xe @ w3[e].double().t()
+        sg = torch.sigmoid(ge)
+        he, dh = ge * sg * ue, de @ w2[e].double()
+        dge, due = sc * dh * ue * (sg * (1 + ge * (1 - sg))), sc * dh * (ge * sg)
+        for name, got, ref in (("g", g[r], ge), ("u", u[r], ue), ("h", h[r], he), ("y", y[r], he @ w2[e].double().t()), ("dg", dg[r], dge),
+                               ("du", du[r], due), ("hs", hs[r], sc * he),
+                               ("dx", dx[r], dge @ w1[e].double() + due @ w3[e].double())):
+            assert rel_err(got, ref) <= F32_TOL, (name, e, c, rel_err(got, ref))
+        # a sum of I products that cancel: judged, as the bound is, by the sum of their magnitudes
+        assert ((ds[r] - (dh * he).sum(1)).abs() <= F32_TOL * (dh * he).abs().sum(1)).all(), ("ds", e, c)
+
+
 SKINNY_CASES = [
     # (counts, H, I): below, at and above the 16- and 32-row units, reductions of less than one step (64)
     # per wave and with a remainder, widths with a partly filled column tile, empty experts
