@@ -139,8 +139,9 @@ struct Lds {
   __attribute__((aligned(16))) bf16_t Bs[Planes<TB>::N][B_KC ? BN * LDK : BK * LDB];
 };
 
-// acc of one wave: rows m0 + 32 wm .., columns n0 + 32 wn .. of the product over k in [kbeg, kend)
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+// acc of one wave: rows m0 + 32 wm .., columns n0 + 32 wn .. of the product over k in [kbeg, kend).
+// AHEAD > 0: the reduction has at most that many k-tiles, and all of them are requested at once.
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0>
 __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
                                         int64_t kend, floatx16_t& acc) {
   constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
@@ -163,26 +164,44 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
   // (two, four and eight tiles in flight: no gain at 509 tokens, 2 to 20 % slower at 16,384)
   constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
   static_assert(NA >= 1 && NB >= 1, "tile too small for the thread count");
-  Raw<TA> ra[NA];
-  Raw<TB> rb[NB];
+  struct Tile { Raw<TA> a[NA]; Raw<TB> b[NB]; };
   auto slot = [](int idx, bool kc, int R, int& row, int& k) {
     if (kc) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); }
     else { row = (idx % (R / 4)) * 4; k = idx / (R / 4); }
   };
-  auto load_tile = [&](int64_t k0) {
+  // (AHEAD: every load is made, past the ends from the last elements, as a branch would hold up the loads behind it;
+  // what lies past kend is cleared when it goes to LDS)
+  auto load_tile = [&](Tile& t, int64_t k0) {
+    if constexpr (AHEAD > 0) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        int m, k;
+        slot(tid + i * THREADS, A_KC, BM, m, k);
+        const int64_t mm = min(m0 + m, p.M - (A_KC ? 1 : 4)), kk = min(k0 + k, kend - (A_KC ? 4 : 1));
+        fetch4<TA>(A + mm * p.sam + kk * p.sak, p.plane_a, t.a[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        int n, k;
+        slot(tid + i * THREADS, B_KC, BN, n, k);
+        const int64_t nn = min(n0 + n, p.N - (B_KC ? 1 : 4)), kk = min(k0 + k, kend - (B_KC ? 4 : 1));
+        fetch4<TB>(B + kk * p.sbk + nn * p.sbn, p.plane_b, t.b[i]);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       int m, k;
       slot(tid + i * THREADS, A_KC, BM, m, k);
-      zero_raw<TA>(ra[i]);
-      if (m0 + m < p.M && k0 + k < kend) fetch4<TA>(A + (m0 + m) * p.sam + (k0 + k) * p.sak, p.plane_a, ra[i]);
+      zero_raw<TA>(t.a[i]);
+      if (m0 + m < p.M && k0 + k < kend) fetch4<TA>(A + (m0 + m) * p.sam + (k0 + k) * p.sak, p.plane_a, t.a[i]);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       int n, k;
       slot(tid + i * THREADS, B_KC, BN, n, k);
-      zero_raw<TB>(rb[i]);
-      if (n0 + n < p.N && k0 + k < kend) fetch4<TB>(B + (k0 + k) * p.sbk + (n0 + n) * p.sbn, p.plane_b, rb[i]);
+      zero_raw<TB>(t.b[i]);
+      if (n0 + n < p.N && k0 + k < kend) fetch4<TB>(B + (k0 + k) * p.sbk + (n0 + n) * p.sbn, p.plane_b, t.b[i]);
     }
   };
   // one 8-byte store per plane: along k of a [row][k] tile for a K-contiguous operand, along the
@@ -192,26 +211,27 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 #pragma unroll
     for (int q = 0; q < P; ++q) *reinterpret_cast<bf16x4_t*>(&tiles[q][kc ? row * LDK + k : k * ld_mn + row]) = v[q];
   };
-  if (kbeg < kend) load_tile(kbeg);
-  for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
+  auto store_tile = [&](Tile& t, int64_t k0) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       int m, k;
       slot(tid + i * THREADS, A_KC, BM, m, k);
+      if (AHEAD > 0 && k0 + k >= kend) zero_raw<TA>(t.a[i]);
       bf16x4_t v[PA];
-      to_planes<TA>(ra[i], v);
+      to_planes<TA>(t.a[i], v);
       store4(As, std::integral_constant<int, PA>{}, A_KC, LDA, m, k, v);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       int n, k;
       slot(tid + i * THREADS, B_KC, BN, n, k);
+      if (AHEAD > 0 && k0 + k >= kend) zero_raw<TB>(t.b[i]);
       bf16x4_t v[PB];
-      to_planes<TB>(rb[i], v);
+      to_planes<TB>(t.b[i], v);
       store4(Bs, std::integral_constant<int, PB>{}, B_KC, LDB, n, k, v);
     }
-    __syncthreads();
-    if (k0 + BK < kend) load_tile(k0 + BK);
+  };
+  auto multiply = [&]() {
 #pragma unroll
     for (int kk = 0; kk < BK; kk += 16) {
       bf16x8_t a[PA], b[PB];
@@ -228,13 +248,35 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
           if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa], b[pb], acc, 0, 0, 0);
         }
     }
-    __syncthreads();
+  };
+  if constexpr (AHEAD > 0) {
+    Tile t[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) load_tile(t[i], kbeg + i * BK);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (kbeg + i * BK < kend) {
+        store_tile(t[i], kbeg + i * BK);
+        __syncthreads();
+        multiply();
+        __syncthreads();
+      }
+  } else {
+    Tile t;
+    if (kbeg < kend) load_tile(t, kbeg);
+    for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
+      store_tile(t, k0);
+      __syncthreads();
+      if (k0 + BK < kend) load_tile(t, k0 + BK);
+      multiply();
+      __syncthreads();
+    }
   }
-
 }
 
 // output tile (bx, by) of split bz
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0>
 __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int bx, int by, int bz) {
   constexpr int BM = 32 * WM, BN = 32 * WN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -244,7 +286,7 @@ __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_K
   const int64_t kbeg = (int64_t)bz * kchunk;
   const int64_t kend = kbeg + kchunk < p.K ? kbeg + kchunk : p.K;
   floatx16_t acc;
-  product<WM, WN, A_KC, B_KC, TA, TB>(p, lds, m0, n0, kbeg, kend, acc);
+  product<WM, WN, A_KC, B_KC, TA, TB, AHEAD>(p, lds, m0, n0, kbeg, kend, acc);
 
   float* C = p.C + (p.splits > 1 ? (int64_t)bz * p.M * p.N : 0);
   const int64_t n = n0 + wn * 32 + (lane & 31);
@@ -261,10 +303,10 @@ __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_K
     }
   }
 }
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0>
 __global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
   __shared__ Lds<WM, WN, A_KC, B_KC, TA, TB> lds;
-  gemm_tile<WM, WN, A_KC, B_KC, TA, TB>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
+  gemm_tile<WM, WN, A_KC, B_KC, TA, TB, AHEAD>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // The gradient of the region's input in one pass: out[t] = sum_k rows[inv_perm[t*K + k]] + d_logits[t] .
@@ -360,6 +402,19 @@ inline int launch(const Params& p, int kernel_id, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return PK_OK;
   dim3 grid((unsigned)pk_ceil_div(p.N, 32 * WN), (unsigned)pk_ceil_div(p.M, 32 * WM), (unsigned)p.splits);
   if (grid.y > 65535u || grid.z > 65535u) return PK_ERR_SHAPE;
+  // A workgroup that has a CU to itself waits for every k-tile's loads in turn: a reduction of up to 256, which is what the gate's
+  // splits leave, is requested as a whole.  Where workgroups share a CU the registers for it cost more (gate, us, 128
+  // experts 2048 wide: 300 tokens 13.7 -> 11.8, 1,777 tokens, 224 workgroups 14.1 -> 12.6, 3,000 tokens, 376 16.7 -> 18.9;
+  // 64 experts, 1,500 tokens 12.1 -> 8.8; fp32, 128 experts 1024 wide, 1,000 tokens 10.8 -> 9.9, 4,000 14.7 -> 16.2).
+  if constexpr (A_KC && B_KC) {
+    const int64_t k_tiles = pk_ceil_div(pk_ceil_div(p.K, p.splits), BK);
+    if ((int64_t)grid.x * grid.y * grid.z <= 256 && k_tiles <= 8) {
+      if (k_tiles <= 4) PK_LAUNCH_NOCHECK(kernel_id, s, (kernel<WM, WN, A_KC, B_KC, TA, TB, 4>), grid, dim3(64 * WM * WN), 0, s, p);
+      else PK_LAUNCH_NOCHECK(kernel_id, s, (kernel<WM, WN, A_KC, B_KC, TA, TB, 8>), grid, dim3(64 * WM * WN), 0, s, p);
+      PK_RETURN_IF_LAUNCH_FAILED();
+      return PK_OK;
+    }
+  }
   PK_LAUNCH_NOCHECK(kernel_id, s, (kernel<WM, WN, A_KC, B_KC, TA, TB>), grid, dim3(64 * WM * WN), 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;

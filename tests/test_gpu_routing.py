@@ -242,6 +242,23 @@ def test_sort_time_grows_with_the_slots(dev):
     assert long <= 8 * short
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,E", [(2048, 128), (1000, 120), (1800, 96), (2040, 64)])
+def test_gate_with_its_reduction_requested_at_once(dev, dtype, H, E):
+    """Up to 256 workgroups the gate requests a workgroup's whole reduction at once (four or eight k-tiles, the last ones
+    partly or wholly past the end); one row of tokens more and it goes k-tile by k-tile.  The same products in the same
+    order: the tokens of both calls get the same logits bit for bit, and those of the oracle."""
+    _note(f"gate ahead {dtype} H={H} E={E}")
+    splits = max(1, min(8, H // 128))
+    T = 64 * (256 // splits)
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(T + 1, H, generator=g).to(dtype)
+    w = torch.randn(E, H, generator=g) * 0.05
+    few, more = ops.gate_logits(x[:T].to(dev), w.to(dev)), ops.gate_logits(x.to(dev), w.to(dev))
+    assert torch.equal(few, more[:T])
+    assert rel_err(few, O.gate_logits(x[:T], w, None)) <= F32_TOL
+
+
 @pytest.mark.parametrize("T,H,E,K,bias", [(1, 256, 8, 2, True), (65, 2048, 128, 8, False), (70, 520, 130, 5, True), (5000, 2048, 128, 8, True)])
 def test_gate_and_topk_in_one_call_match_the_two_calls(dev, T, H, E, K, bias):
     """pk_gate_route sums the gate GEMM's split-K partial results inside the top-k kernel: logits,
@@ -364,3 +381,12 @@ def test_norm_gate_topk_and_sort_in_one_call(dev, dtype, T, H, E, K, bias):
             assert torch.equal(a, c), name
     exact = want_xn.double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0.0)
     assert rel_err(want_l.double().cpu(), exact) <= F32_TOL
+
+
+@pytest.mark.parametrize("T,H,E,K,bias", [(129, 2048, 128, 8, True), (1033, 1600, 61, 1, False), (2048, 1024, 128, 3, True), (2049, 1024, 128, 1, True),
+                                          (205, 1024, 97, 5, False)])
+def test_topk_with_the_sorts_histogram(dev, T, H, E, K, bias):
+    """Above the gates that gate_front_kernel takes and up to 16 K chunk counts (2,048 tokens of 128 experts, 2,049 are too
+    many): the top-k writes the histograms of 16 tokens each that the sort places the slots by.  Partly filled last
+    chunks, one and two experts a lane, more than 1,024 slots: bit for bit the separate calls."""
+    test_norm_gate_topk_and_sort_in_one_call(dev, torch.bfloat16, T, H, E, K, bias)
