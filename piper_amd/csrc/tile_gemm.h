@@ -522,7 +522,9 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_o
       return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   const int ks = reduction_groups(tiles, k_tiles, cus);
-  if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, EPI == GATE_UP ? 2 : 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  // (fp32 products with so few tiles are on the finer ones above)
+  if constexpr (sizeof(T) == 2)
+    if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, EPI == GATE_UP ? 2 : 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   if (ks == 2) return launch_tiles<T, 2, 2, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   return launch_tiles<T, 2, 2, 1, 1, 3, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
 }
