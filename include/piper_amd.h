@@ -388,6 +388,12 @@ PK_API int pk_region_dgrad_dh(const void* d_out, const int32_t* row_map, int64_t
 PK_API int pk_region_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3,
                        const int32_t* starts, void* d_x_sorted, int64_t A, int64_t H, int64_t I, int64_t E,
                        int dtype, pk_stream_t stream);
+/* The same with the sums over I ordered by size as well: faster in fp32, for callers that do not mind which rounding the
+ * gradient carries into the layer in front (one expert per token with normalised scores does: its gate gradient is
+ * nothing but rounding). */
+PK_API int pk_region_dgrad_dx_any_order(const void* d_g, const void* d_u, const void* w1, const void* w3,
+                                 const int32_t* starts, void* d_x_sorted, int64_t A, int64_t H, int64_t I, int64_t E,
+                                 int dtype, pk_stream_t stream);
 /* HOST, tuning hint: 1 when the backward of a region is faster through the transposed copies (0 also where
  * pk_grouped_swiglu_transposed_ld says there are none). */
 PK_API int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dtype);

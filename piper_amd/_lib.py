@@ -87,6 +87,7 @@ SIGNATURES = {
     "pk_region_dgrad_dh_workspace_bytes": (_c_i64, [_c_i64, _c_i64]),
     "pk_region_dgrad_dh": (_c_int, [_p, _p, _c_i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _c_i64,
                                     _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _p]),
+    "pk_region_dgrad_dx_any_order": (_c_int, [_p, _p, _p, _p, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _p]),
     "pk_region_dgrad_dx": (_c_int, [_p, _p, _p, _p, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _p]),
     "pk_region_transposed_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int]),
     "pk_grouped_swiglu_dx_from_transposed_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int]),

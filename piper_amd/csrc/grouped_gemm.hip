@@ -2387,7 +2387,7 @@ int dh_tile(const void* dy, const int32_t* row_map, int64_t div, const float* sc
   p.Gin = g; p.Uin = u; p.scores = scores; p.ds_part = parts; p.total_rows = A;
   const int id = pk_timing::K_SWIGLU_DGRAD_DH;
   // (2048 x 768, 128 experts, 128 x 128 -> 64 x 64: 32 rows 100 -> 92, 48 rows 107 -> 104, 64 rows 114 -> 117)
-  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), true, PK_DH_TILE_ROWS, nullptr, id, s);
+  if (!scores) return pk_tile::launch_ragged_m<T, false, pk_tile::BWD>(p, A, mf::persistent_grid(), false, PK_DH_TILE_ROWS, nullptr, id, s);
   return pk_tile::launch_ragged_m<T, false, pk_tile::BWD_SCALED>(p, A, mf::persistent_grid(), div > 1, PK_DH_TILE_ROWS, part_cols, id, s);
 }
 template <typename T>
@@ -2668,7 +2668,7 @@ int pk_grouped_swiglu_dgrad_dh_scaled_t(const void* d_out, const int32_t* row_ma
 // by_size: small products may go to the tiles of tile_gemm.h.  Without it a shape that has a transposed path
 // stays on the kernels of that path, whose result is then the same bit for bit.
 static int dgrad_dx_impl(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
-                         bool by_size, int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
+                         bool by_size, bool any_order, int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
   int rc = check_common(A, H, I, E, dtype);
   if (rc) return rc;
   if (A == 0) return PK_OK;
@@ -2680,8 +2680,8 @@ static int dgrad_dx_impl(const void* d_g, const void* d_u, const void* w1, const
     // d_x = d_g . w1[e] + d_u . w3[e]   (w[e] is [I, H]: B(k=i, n=h) = w[i*H + h])
     if (tile_gemm_ok(dtype, H, I, {d_g, d_u, w1, w3, d_x_sorted}))
       return dtype == PK_F32
-                 ? dgrad_tile<float>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, true, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s)
-                 : dgrad_tile<bf16_t>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, true, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s);
+                 ? dgrad_tile<float>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, any_order, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s)
+                 : dgrad_tile<bf16_t>(d_g, d_u, I, nullptr, 1, w1, w3, d_x_sorted, H, 2, starts, any_order, A, E, pk_timing::K_SWIGLU_DGRAD_DX, s);
     if (dtype == PK_F32) {
       rc = simt_ragged_m<float>(d_g, I, nullptr, 1, w1, H, 1, I * H, d_x_sorted, H, starts, A, H, I, E, 0, s);
       if (rc) return rc;
@@ -2702,11 +2702,15 @@ static int dgrad_dx_impl(const void* d_g, const void* d_u, const void* w1, const
 
 int pk_grouped_swiglu_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
                                int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
-  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, false, A, H, I, E, dtype, stream);
+  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, false, false, A, H, I, E, dtype, stream);
 }
 int pk_region_dgrad_dx(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
                        int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
-  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, true, A, H, I, E, dtype, stream);
+  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, true, false, A, H, I, E, dtype, stream);
+}
+int pk_region_dgrad_dx_any_order(const void* d_g, const void* d_u, const void* w1, const void* w3, const int32_t* starts, void* d_x_sorted,
+                                 int64_t A, int64_t H, int64_t I, int64_t E, int dtype, pk_stream_t stream) {
+  return dgrad_dx_impl(d_g, d_u, w1, w3, starts, d_x_sorted, true, true, A, H, I, E, dtype, stream);
 }
 
 int pk_grouped_swiglu_dx_from_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dtype) {

@@ -523,6 +523,8 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
       if (!need_xn) return;
       if (blocks_only)
         PK_CALL(pk_grouped_swiglu_dgrad_dx_t, w.at_(d_gT), w.at_(d_uT), ldt, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
+      else if (s.K > 1)
+        PK_CALL(pk_region_dgrad_dx_any_order, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
       else
         PK_CALL(pk_region_dgrad_dx, dg, du, ptr(w1), ptr(w3), starts, t.at_(d_xs), s.A, s.H, s.I, s.E, s.dtype, st);
     };

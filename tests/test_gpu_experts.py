@@ -590,7 +590,8 @@ def test_fp32_tiles_by_their_number(dev, counts, H, I, K):
          ctypes.addressof(n_part), ptr(ws), ws.numel() * 4, A, H, I, E, dtype_code(torch.float32), current_stream(dev))
     ds = ws[:n_part.value * A].view(n_part.value, A).double().sum(0)
     dx = torch.full((A, H), float("nan"), device=dev)
-    call("pk_region_dgrad_dx", ptr(dg), ptr(du), ptr(w1), ptr(w3), ptr(starts), ptr(dx), A, H, I, E, dtype_code(torch.float32), current_stream(dev))
+    call("pk_region_dgrad_dx_any_order" if K > 1 else "pk_region_dgrad_dx", ptr(dg), ptr(du), ptr(w1), ptr(w3), ptr(starts), ptr(dx), A, H, I, E,
+         dtype_code(torch.float32), current_stream(dev))
     rows = (perm.long() // K)
     s = 0
     for e, c in enumerate(counts):
