@@ -176,7 +176,7 @@ int pk_region_decode(const void* x, int dtype, const void* norm_weight, float ep
   const int64_t need = pk_region_decode_workspace_bytes(T, H, E, I, K, dtype);
   if (need < 0) return PK_ERR_ARG;
   if (need == 0) return PK_ERR_UNSUPPORTED;
-  if (!x || !w_gate || !w1 || !w2 || !w3 || !out) return PK_ERR_ARG;
+  if (!x || !w_gate || !w1 || !w2 || !w3 || !out || (norm_weight && !(eps >= 0.f))) return PK_ERR_ARG;
   if (!workspace || workspace_bytes < need) return PK_ERR_WORKSPACE;
   for (const void* p : {x, norm_weight, (const void*)w_gate, w1, w2, w3, residual, (const void*)out, (const void*)workspace})
     if (!pk_aligned16(p)) return PK_ERR_ALIGN;

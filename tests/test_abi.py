@@ -42,6 +42,27 @@ def test_host_only_calls():
     assert lib.pk_sort_workspace_bytes(-1, 128) < 0
 
 
+def test_decode_step_refuses_what_the_norm_refuses():
+    """A negative or undefined eps is an argument error in pk_rmsnorm_fwd, and in the calls that have the norm in them (the
+    check comes before any launch; without a norm eps is not looked at, and the workspace check is next)."""
+    lib = _lib.load()
+    buf = ctypes.create_string_buffer(1 << 16)
+    p = (ctypes.addressof(buf) + 15) // 16 * 16
+    T, H, E, I, K = 1, 64, 4, 64, 2
+
+    def decode(norm_w, eps):
+        return lib.pk_region_decode(p, _lib.PK_BF16, norm_w, eps, p, None, p, p, p, 1, 1.0, None, p, T, H, E, I, K, None, 0, None)
+
+    workspace = decode(p, 1e-6)
+    assert "workspace" in _lib.status_string(workspace) and decode(None, -1.0) == workspace
+    for eps in (-1e-6, float("nan"), float("-inf")):
+        norm = lib.pk_rmsnorm_fwd(p, _lib.PK_BF16, p, eps, p, None, T, H, None)
+        assert "invalid argument" in _lib.status_string(norm)
+        assert decode(p, eps) == norm
+        assert lib.pk_norm_gate_route_sort(p, _lib.PK_BF16, p, eps, p, None, p, None, T, H, E, K, 1, 1.0, p, p, p, None, p, p, None, None, p, 0,
+                                           None) == norm
+
+
 def test_counter_sets_are_handed_out_per_stream_and_capture():
     """Launches that can overlap must not share scheduling counters: every (stream, capture
     sequence) pair keeps a set of its own; the same pair always gets the same set."""

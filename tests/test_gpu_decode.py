@@ -65,6 +65,15 @@ def test_decode_step_is_what_the_region_runs(dev):
         assert few == 3 and many > 3 and rel_err(got, want) <= BF16_TOL
 
 
+@pytest.mark.parametrize("tokens", [1, 100])
+def test_eps_that_the_norm_refuses(dev, tokens):
+    """moe_block with an eps below zero raises whichever path its tokens take."""
+    from piper_amd import functional as F_
+    t = _inputs(dev, tokens, 256, 16, 128, False, False, 6)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="invalid argument"):
+        F_.moe_block(t["x"], t["norm_w"], t["w_gate"], None, t["w1"], t["w2"], t["w3"], top_k=4, route_norm=True, norm_eps=-1.0)
+
+
 def test_decode_step_applies_to_few_rows_only():
     """Where it does not apply the workspace query says so (CPU side of the rule; the call itself refuses)."""
     q = _lib.load().pk_region_decode_workspace_bytes
