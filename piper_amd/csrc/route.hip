@@ -700,6 +700,10 @@ __global__ __launch_bounds__(64 * kFrontWaves) void gate_front_kernel(const Fron
             if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa], b[pb], acc, 0, 0, 0);
           }
       }
+      // the next piece's planes go to where other lanes have just read
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) keep[q][i] = acc[i];
