@@ -259,6 +259,38 @@ def test_gate_with_its_reduction_requested_at_once(dev, dtype, H, E):
     assert rel_err(few, O.gate_logits(x[:T], w, None)) <= F32_TOL
 
 
+def _launches(fn):
+    """what fn returns, and the names of the kernels it launched"""
+    from piper_amd import _lib
+    _lib.timing_enable(True)
+    _lib.timing_collect()
+    out = fn()
+    names = [n for n, _ in _lib.timing_collect()]
+    _lib.timing_enable(False)
+    return out, names
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("dtype,T,H,E", [
+    (torch.bfloat16, 65, 1024, 32), (torch.bfloat16, 200, 264, 17), (torch.bfloat16, 500, 1000, 33), (torch.bfloat16, 600, 488, 65),
+    (torch.bfloat16, 1000, 512, 128), (torch.bfloat16, 4096, 256, 100), (torch.bfloat16, 2000, 1992, 24), (torch.float32, 65, 512, 20),
+    (torch.float32, 130, 260, 31), (torch.float32, 1030, 1000, 24), (torch.float32, 600, 300, 97), (torch.float32, 4095, 1020, 32)])
+def test_gate_in_the_front_kernel_gives_the_bits_of_the_gate_gemm(dev, dtype, T, H, E, bias):
+    """gate_front_kernel against pk_x3mm::kernel: the same tokens and experts with more experts behind them than the front
+    kernel takes (129), which leaves the reduction's splits as they are.  Every pair of logits is equal bit for bit, with
+    two to eight splits, one to four tiles of experts, widths that end inside a step and operands of three planes."""
+    _note(f"front against gemm {dtype} T={T} H={H} E={E}")
+    g = torch.Generator().manual_seed(T + H + E)
+    x = torch.randn(T, H, generator=g).to(dtype).to(dev)
+    w = (torch.randn(129, H, generator=g) * 0.05).to(dev)
+    b = torch.randn(129, generator=g).to(dev) if bias else None
+    front, few = _launches(lambda: ops.gate_logits(x, w[:E].contiguous(), b[:E].contiguous() if bias else None))
+    gemm, many = _launches(lambda: ops.gate_logits(x, w, b))
+    assert len(few) == 1 and len(many) == 2      # (the GEMM's partial results are added up by a second launch)
+    assert torch.equal(front, gemm[:, :E])
+    assert rel_err(gemm.double().cpu(), x.double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0.0)) <= F32_TOL
+
+
 @pytest.mark.parametrize("T,H,E,K,bias", [(1, 256, 8, 2, True), (65, 2048, 128, 8, False), (70, 520, 130, 5, True), (5000, 2048, 128, 8, True)])
 def test_gate_and_topk_in_one_call_match_the_two_calls(dev, T, H, E, K, bias):
     """pk_gate_route sums the gate GEMM's split-K partial results inside the top-k kernel: logits,
