@@ -514,7 +514,7 @@ __global__ __launch_bounds__(kScatterThreads) void sort_scatter_kernel(const int
 // ------------------------------------------------------------------ norm, gate and top-k in one launch
 // A workgroup takes 16 tokens through the whole front of the region: the norm (its rows stay in LDS), the gate's
 // products, softmax and top-k, and the histogram of the chosen experts that sort_scatter_kernel wants.  What it replaces is
-// four or five launches of 3 to 14 us each that are mostly latency: see front_ok for where it pays.
+// four or five launches of 3 to 14 us each that are mostly latency: see front_pays for where it pays.
 // The products are those of pk_x3mm::kernel, plane by plane and split by split, so that the logits are the same bit for
 // bit: a wave takes one split of the reduction for 32 experts, splits the weights into their three planes on the way
 // through LDS that only it uses (no barriers), and the waves' sums are added in the order of the splits.  Half of a
@@ -1083,21 +1083,46 @@ int pk_norm_gate_small(const void* x, int dtype, const void* norm_w, float eps, 
   return PK_OK;
 }
 
-// Whether gate_front_kernel takes a gate of these sizes: a rule on (T, H, E) and the gate's operands alone, so that every
-// entry point with a gate in it gives the same logits.  Every workgroup reads all of w_gate and splits it, 0.14 us for
-// 1,024 elements, beside some 8 us that do not depend on it; the launches it replaces take 17 to 30 us whatever the
-// weight's size, 8 to 13 up to 64 tokens (norm_gate_small_kernel).  Norm, gate, top-k and the sort's histogram, us,
-// those -> this one:
-//   129 tokens,  408 x  16 (fp32)  16.5 -> 11.2      1,030 tokens, 1000 x  24 experts 21.9 -> 12.0
-// 2,048 tokens, 2048 x  16         23.2 -> 17.2      3,655 tokens,  768 x  64         25.8 -> 15.1
-//   509 tokens, 2048 x 128         24.2 -> 43.5
+// Whether gate_front_kernel takes a gate of these sizes.  It gives the bits of the launches that it replaces, so each entry point
+// has its own answer: how many launches those are.  Every workgroup reads all of w_gate and splits it, for whole tiles of 32
+// experts: some 5 us in bf16, with top-k, sort and norm 12, and 0.12 us for 1,024 elements of that; in fp32 half as much again
+// (x is split as well).  The launches it replaces hardly depend on the weight's size, but on the tokens.  Us, those -> this one
+// (launched back to back, graph; top 4):
+//                             65 tokens      1,024        2,048        4,096        4,097        8,192
+//   norm .. sort, 1024 x  24  16.5 -> 13.6   21 -> 14     25 -> 15     30 -> 17     30 -> 24     36 -> 29
+//                 1024 x  64  17.0 -> 18.1   23 -> 19     27 -> 20     33 -> 23     34 -> 35     38 -> 38
+//                  768 x 128  19.3 -> 24.3   25 -> 26     30 -> 28     40 -> 32     40 -> 47     44 -> 49
+//           fp32, 1000 x  64  18.0 -> 24.6   25 -> 26     30 -> 28     35 -> 31     35 -> 50     44 -> 56
+//   gate .. sort,  768 x  64                              21 -> 17
+//                 2048 x  24  16.1 -> 17.2                                          24 -> 29     31 -> 38
+//   gate alone,    512 x  64   8.9 ->  6.9   10 ->  7     10 ->  7     11 ->  7     11 -> 12     15 -> 13
+//                 2048 x  32  12.0 -> 11.0   13 -> 11     13 -> 11     14 -> 12     16 -> 20     20 -> 27
+//                  768 x 128   9.8 -> 14.7   11 -> 16     13 -> 16     18 -> 16     19 -> 29     24 -> 30
+// Once the CUs have taken a workgroup or two each (front_lds_bytes says which), the next ones wait a whole round for them.
+enum FrontCall { FRONT_LOGITS, FRONT_TOPK, FRONT_SORT, FRONT_NORM };
 constexpr int64_t kFrontMaxTokens = 8192;
-static bool front_ok(const void* x, int x_dtype, const void* w_gate, int64_t T, int64_t H, int64_t E) {
-  const int64_t es = (int64_t)pk_dtype_size(x_dtype);
+static bool front_pays(FrontCall call, int es, int64_t T, int64_t H, int64_t E) {
+  if (E * H > 96 * 1024) return false;
+  const int experts = E <= 32 ? 32 : E <= 64 ? 64 : kFrontExperts;
+  const bool narrow = E <= 32, long_rows = H * es > 3072;
+  const int64_t work = pk_ceil_div(E, 32) * 32 * H * (es == 2 ? 2 : 3) / 2 / 1024;
+  constexpr int64_t LDS = 160 * 1024, PLANES = (int64_t)kFrontWaves * 3 * 32 * pk_x3mm::LDK * 2 + kFrontExperts * 4;
+  const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(2, LDS / ((int64_t)front_lds_bytes(H, es, experts) + PLANES)));
+  if (pk_ceil_div(T, kFrontTokens) > 256 * per_cu) {      // a second round
+    if (call == FRONT_NORM) return narrow || (E <= 64 && work <= 32);
+    return call != FRONT_TOPK && narrow && H * es <= 2048 && (work <= 16 || T > 6000);
+  }
+  if (call == FRONT_NORM) return work <= (T < 2048 ? 64 : 128);
+  if (long_rows && (call == FRONT_SORT ? T <= 512 : call == FRONT_TOPK && T <= 2048)) return false;
+  if (narrow) return work <= 64;
+  return work <= (T < 1024 || (T <= 2048 && call != FRONT_SORT) ? 32 : T < 4096 ? 64 : 80);
+}
+static bool front_ok(FrontCall call, const void* x, int x_dtype, const void* w_gate, int64_t T, int64_t H, int64_t E) {
+  const int es = (int)pk_dtype_size(x_dtype);
   if (T <= kGateSmallMax || T > kFrontMaxTokens || E > kFrontExperts || H % (16 / es) != 0 || H * es > kFrontRowBytes || !pk_aligned16(x) ||
       !pk_aligned16(w_gate))
     return false;
-  return E * H <= 96 * 1024;
+  return front_pays(call, es, T, H, E);
 }
 // Whether the sort goes by its histograms of 16 tokens each: every workgroup of sort_scatter_kernel reads all of them
 // (229 of 64 experts: 8.2 us against 5.3 + 6.0 with histograms of 512 slots in a launch of their own).
@@ -1145,7 +1170,6 @@ static int gate_gemm(const void* x, int x_dtype, const float* w_gate, const floa
   *splits = 1;
   if (T == 0) return PK_OK;
   if (!x || !w_gate || !logits) return PK_ERR_ARG;
-  if (front_ok(x, x_dtype, w_gate, T, H, E)) return launch_front(front_params(x, w_gate, gate_bias, logits, T, H, E), x_dtype, s);
   if (T <= kGateSmallMax && H % 4 == 0 && pk_aligned16(x) && pk_aligned16(w_gate)) {
     const dim3 grid((unsigned)pk_ceil_div(E, 4), (unsigned)pk_ceil_div(T, T == 1 ? 1 : kGateTokens)), block(256);
 #define PK_GATE_SMALL(TYPE, N)                                                                                                  \
@@ -1184,6 +1208,8 @@ int pk_gate_logits(const void* x, int x_dtype, const float* w_gate, const float*
                    float* logits, int64_t T, int64_t H, int64_t E, void* workspace,
                    int64_t workspace_bytes, pk_stream_t stream) {
   hipStream_t s = (hipStream_t)stream;
+  if (H > 0 && E > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits && front_ok(FRONT_LOGITS, x, x_dtype, w_gate, T, H, E))
+    return launch_front(front_params(x, w_gate, gate_bias, logits, T, H, E), x_dtype, s);
   int splits = 1;
   const int rc = gate_gemm(x, x_dtype, w_gate, gate_bias, logits, T, H, E, workspace, workspace_bytes, s, &splits);
   if (rc != PK_OK || splits == 1) return rc;
@@ -1397,7 +1423,7 @@ int pk_gate_route(const void* x, int x_dtype, const float* w_gate, const float* 
   if (K <= 0) return PK_ERR_ARG;
   if (E > PK_MAX_EXPERTS || K > PK_MAX_TOPK || K > E) return PK_ERR_SHAPE;
   if (T > 0 && (!top_scores || !top_idx)) return PK_ERR_ARG;
-  if (H > 0 && E > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits && front_ok(x, x_dtype, w_gate, T, H, E)) {
+  if (H > 0 && E > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits && front_ok(FRONT_TOPK, x, x_dtype, w_gate, T, H, E)) {
     Front p = front_params(x, w_gate, gate_bias, logits, T, H, E);
     p.top_scores = top_scores; p.top_idx = top_idx;
     p.K = (int32_t)K; p.route_norm = route_norm; p.route_scale = route_scale;
@@ -1607,7 +1633,8 @@ static int norm_gate_route_sort(const void* x, int x_dtype, const void* norm_w, 
   if (!starts || !workspace || (T > 0 && (!top_scores || !top_idx || !perm))) return PK_ERR_ARG;
   if (workspace_bytes < pk_gate_route_sort_workspace_bytes(T, H, E, K)) return PK_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
-  if (H > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits && front_ok(x, x_dtype, w_gate, T, H, E) &&
+  if (H > 0 && pk_dtype_ok(x_dtype) && x && w_gate && logits &&
+      front_ok(norm_w ? FRONT_NORM : FRONT_SORT, x, x_dtype, w_gate, T, H, E) &&
       (!norm_w || (xn && pk_aligned16(norm_w) && pk_aligned16(xn)))) {
     Front p = front_params(x, w_gate, gate_bias, logits, T, H, E);
     p.norm_w = norm_w; p.eps = eps; p.xn = xn; p.rstd = rstd;

@@ -272,9 +272,9 @@ def _launches(fn):
 
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("dtype,T,H,E", [
-    (torch.bfloat16, 65, 1024, 32), (torch.bfloat16, 200, 264, 17), (torch.bfloat16, 500, 1000, 33), (torch.bfloat16, 600, 488, 65),
-    (torch.bfloat16, 1000, 512, 128), (torch.bfloat16, 4096, 256, 100), (torch.bfloat16, 2000, 1992, 24), (torch.float32, 65, 512, 20),
-    (torch.float32, 130, 260, 31), (torch.float32, 1030, 1000, 24), (torch.float32, 600, 300, 97), (torch.float32, 4095, 1020, 32)])
+    (torch.bfloat16, 65, 1024, 32), (torch.bfloat16, 200, 264, 17), (torch.bfloat16, 3000, 1000, 33), (torch.bfloat16, 2500, 488, 65),
+    (torch.bfloat16, 4096, 512, 128), (torch.bfloat16, 4096, 256, 100), (torch.bfloat16, 2000, 1992, 24), (torch.float32, 65, 512, 20),
+    (torch.float32, 130, 260, 31), (torch.float32, 1030, 1000, 24), (torch.float32, 4096, 300, 97), (torch.float32, 4095, 1020, 32)])
 def test_gate_in_the_front_kernel_gives_the_bits_of_the_gate_gemm(dev, dtype, T, H, E, bias):
     """gate_front_kernel against pk_x3mm::kernel: the same tokens and experts with more experts behind them than the front
     kernel takes (129), which leaves the reduction's splits as they are.  Every pair of logits is equal bit for bit, with
@@ -289,6 +289,40 @@ def test_gate_in_the_front_kernel_gives_the_bits_of_the_gate_gemm(dev, dtype, T,
     assert len(few) == 1 and len(many) == 2      # (the GEMM's partial results are added up by a second launch)
     assert torch.equal(front, gemm[:, :E])
     assert rel_err(gemm.double().cpu(), x.double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0.0)) <= F32_TOL
+
+
+@pytest.mark.parametrize("dtype,T,H,E,alone,with_norm", [
+    (torch.bfloat16, 65, 768, 32, True, True), (torch.bfloat16, 4096, 768, 32, True, True), (torch.bfloat16, 4097, 256, 32, True, True),
+    (torch.bfloat16, 2048, 512, 64, True, True), (torch.bfloat16, 4096, 768, 96, True, True), (torch.float32, 1024, 512, 16, True, True),
+    # more weight than the launches it stands for are worth, a few tokens
+    (torch.bfloat16, 65, 1024, 96, False, False), (torch.bfloat16, 500, 768, 128, False, False), (torch.float32, 100, 1000, 96, False, False),
+    (torch.float32, 1030, 1000, 48, False, False), (torch.bfloat16, 300, 1024, 64, False, True), (torch.bfloat16, 2048, 768, 128, False, True),
+    # one token more than the CUs take at once
+    (torch.bfloat16, 4097, 768, 128, False, False), (torch.bfloat16, 4097, 2048, 48, False, False), (torch.float32, 4097, 1000, 96, False, False),
+    (torch.bfloat16, 4097, 768, 32, False, True), (torch.bfloat16, 8192, 1536, 64, False, False)])
+def test_the_front_kernel_is_taken_where_it_pays(dev, dtype, T, H, E, alone, with_norm):
+    """gate_front_kernel on either side of front_pays, for the gate alone and with norm, top-k and sort: where it was taken and
+    took up to twice as long as the launches it stands for, those are back.  The same bits from every one of them."""
+    from piper_amd import _lib
+    from piper_amd._lib import call, current_stream, dtype_code, ptr
+    _note(f"front kernel {dtype} T={T} H={H} E={E}")
+    K = min(E, 4)
+    g = torch.Generator().manual_seed(T + H + E)
+    x, norm_w = torch.randn(T, H, generator=g).to(dtype).to(dev), torch.ones(H, dtype=dtype, device=dev)
+    w = (torch.randn(E, H, generator=g) * 0.02).to(dev)
+    xn = ops.rmsnorm_fwd(x, norm_w, 1e-6)[0]
+    gate, names = _launches(lambda: ops.gate_logits(xn, w, None))
+    assert len(names) == (1 if alone else 2), names
+    ws = torch.empty(int(_lib.load().pk_gate_route_sort_workspace_bytes(T, H, E, K)), dtype=torch.uint8, device=dev)
+    got = [torch.empty_like(x), torch.empty(T, device=dev), torch.empty_like(gate), torch.empty(T, K, device=dev)]
+    ints = [torch.empty(n, dtype=torch.int32, device=dev) for n in (T * K, E + 1, T * K)]
+    _, names = _launches(lambda: call("pk_norm_gate_route_sort", ptr(x), dtype_code(dtype), ptr(norm_w), 1e-6, ptr(got[0]), ptr(got[1]), ptr(w), None,
+                                      T, H, E, K, 1, 1.0, ptr(got[2]), ptr(got[3]), ptr(ints[0]), None, ptr(ints[1]), ptr(ints[2]), None, None,
+                                      ptr(ws), ws.numel(), current_stream(dev)))
+    assert ("rmsnorm_fwd" not in names) == with_norm, names
+    scores, idx = ops.route_topk(gate, K, True)
+    assert torch.equal(got[0], xn) and torch.equal(got[2], gate) and torch.equal(got[3], scores) and torch.equal(ints[0].view(T, K), idx)
+    assert torch.equal(ints[2], ops.sort_by_expert(idx, E)[2])
 
 
 @pytest.mark.parametrize("T,H,E,K,bias", [(1, 256, 8, 2, True), (65, 2048, 128, 8, False), (70, 520, 130, 5, True), (5000, 2048, 128, 8, True)])
