@@ -2268,9 +2268,13 @@ bool wide_dh(bool any_order, int64_t A, int64_t H, int64_t I, int64_t E) {
 // reduction: 2048 x 768, 32 experts, 192 rows, 2 rounds 61 / 46 / 58, 384 rows, 3.5 rounds 76 / 78 / 94; 2048 x 1024,
 // 4 experts, 2,048 rows, 2.06 rounds 63 / 70 / 80; 1024 x 512, 64 experts, 256 rows, 2.5 rounds 54 / 46 / 52, 512 rows, 4.5
 // rounds 71 / 73 / 93; 1024 x 256, 128 experts, 256 rows, 5 rounds 59 / 53 / 64, 512 rows, 9 rounds 88 / 91 / 115;
-// 2048 x 128, 64 experts, 384 rows, 7 rounds 67 / 55 / 60, 768 rows, 13 rounds 88 / 97 / 112.
+// 2048 x 128, 64 experts, 384 rows, 7 rounds 67 / 55 / 60, 512 rows, 9 rounds 74 / 75 (counts ~ 1 / sqrt(rank) 67 / 76), 768
+// rows, 13 rounds 88 / 97 / 112; 1024 x 512, 128 experts, 144 rows, 3.25 rounds 72 / 62 (71 / 64), 192 rows, 4 rounds
+// 68 / 66 (80 / 76); 64 experts, 384 rows, 3.5 rounds 66 / 63 (71 / 63).  Hence at least four rounds at these widths while
+// experts have up to 512 rows, and eight at most.
 bool wide_down(int64_t A, int64_t H, int64_t I, int64_t E) {
-  return H % 256 == 0 && A > 96 * E && wide_fills(A, H, E, (int)std::max<int64_t>(8, 6144 / I));
+  const int64_t least = I <= 512 && A <= 512 * E ? 16 : 8;
+  return H % 256 == 0 && A > 96 * E && wide_fills(A, H, E, (int)std::min<int64_t>(32, std::max(least, 6144 / I)));
 }
 // d_x, the same (2048 x 768, 128 experts: 32 rows, 3 rounds 162 / 158 / 164, 64 rows, 4 rounds 173 / 168 / 200 (counts ~ 1 /
 // sqrt(rank) 176 / 187 / 198), 128 rows 203 / 229 / 284; 2048 x 1024, 64 experts, 96 rows, 2.5 rounds 135 / 125 / 157;
