@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <array>
 #include <atomic>
 #include <functional>
@@ -480,10 +481,16 @@ struct RegionFn : public torch::autograd::Function<RegionFn> {
 
     // Shapes where the K-contiguous weight-gradient path pays get d_g, d_u and score*h transposed; with long
     // experts the d_x GEMM reads its A operand from the same blocks and the row-major pair is left out.
-    // With few rows an expert the transposed copies are mostly padding, and d_h without them runs on smaller tiles (128 experts
-    // 2048 x 768, forward and backward, us, with -> without: 4 rows 761 -> 715, 12 rows 814 -> 772, 62 rows 895 -> 927).  (One
-    // expert per token: the order of the sums behind the score's gradient stays, see pk_tile::launch_ragged_m.)
-    const bool few_rows = s.K > 1 && s.A <= 40 * s.E;
+    // With few rows an expert the transposed copies are mostly padding, and d_h without them runs on smaller tiles.  d_h and the
+    // weight gradients, us, with -> without, even / counts ~ 1 / sqrt(rank):
+    //   128 experts 2048 x  768, 8 rows 328 -> 296 / 328 -> 290, 32 rows 340 -> 326 / 335 -> 344, 36 rows 329 -> 334 / 338 -> 359
+    //   128 experts 2048 x  512, 32 rows 225 -> 228 / 256 -> 227      64 experts 1024 x 512, 32 rows 98 -> 67 / 89 -> 68
+    //    64 experts 2048 x 1024, 16 rows 207 -> 209 / 216 -> 212, 32 rows 217 -> 229 / 246 -> 232, 40 rows 214 -> 239 / 251 -> 232
+    //    16 experts 2048 x 1024, 40 rows  86 ->  80 /  90 ->  81       4 experts 2048 x 1024, 32 and 40 rows 59 -> 39
+    // Where d_h's persistent units (128 x 256) outnumber the 256 CUs they lose less, hence the lower line.  (One expert per
+    // token: the order of the sums behind the score's gradient stays, see pk_tile::launch_ragged_m.)
+    const int64_t dh_units = (s.A / 128 + std::min(s.A, s.E) / 2) * ((s.I + 255) / 256);
+    const bool few_rows = s.K > 1 && s.A <= (dh_units > 256 ? 32 : 40) * s.E;
     const int64_t ldt = !few_rows && pk_region_transposed_pays(s.A, s.H, s.I, s.E, s.dtype) ? pk_grouped_swiglu_transposed_ld(s.A, s.H, s.I, s.E, s.dtype) : 0;
     const bool blocks_only = ldt > 0 && pk_grouped_swiglu_dx_from_transposed_pays(s.A, s.H, s.I, s.E, s.dtype);
     // w: what the weight gradients read, t: the rest

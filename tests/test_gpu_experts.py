@@ -695,6 +695,42 @@ def test_one_more_row_takes_other_kernels_to_the_same_bits(dev, H, I, E, A):
         s += A // E
 
 
+@pytest.mark.parametrize("H,I,E,K,T", [(256, 768, 128, 8, 512), (2048, 1024, 4, 2, 80)])
+def test_few_rows_an_expert_leave_out_the_transposed_copies(dev, H, I, E, K, T):
+    """Up to 32 rows an expert (128 experts, more units of d_h than CUs) or 40 (4 experts) the region's backward runs without the
+    transposed copies, with one more token through them: the weight-gradient kernels that were launched say so.  Every
+    gradient against float64 on the same experts, on both sides."""
+    from piper_amd import _lib
+    gen = torch.Generator(device=dev).manual_seed(H + E)
+    rand = lambda *shape, scale=1.0: torch.randn(shape, generator=gen, device=dev) * scale
+    w1, w3 = (rand(E, I, H, scale=0.05).bfloat16().requires_grad_(True) for _ in range(2))
+    w2, w_gate = rand(E, H, I, scale=0.05).bfloat16().requires_grad_(True), rand(E, H, scale=0.05).requires_grad_(True)
+    x_all, d_all = rand(T + 1, H).bfloat16(), rand(T + 1, H).bfloat16()
+    for tokens in (T, T + 1):
+        print(f"[case] {tokens} tokens, {E} experts {H} x {I}", flush=True)
+        x, d_out = x_all[:tokens].clone().requires_grad_(True), d_all[:tokens]
+        out = F_.expert_region(x, w_gate, None, w1, w2, w3, top_k=K, route_norm=True)
+        _lib.timing_enable(True)
+        _lib.timing_collect()
+        got = torch.autograd.grad(out, (x, w_gate, w1, w2, w3), d_out)
+        names = [n for n, _ in _lib.timing_collect()]
+        _lib.timing_enable(False)
+        assert ("swiglu_wgrad" in names) == (tokens == T) and ("swiglu_wgrad_w13" in names) == (tokens > T), names
+        idx = ops.route_topk(ops.gate_logits(x.detach(), w_gate.detach()), K, True)[1].long()
+        ref = [t.detach().double().requires_grad_(True) for t in (x, w_gate, w1, w2, w3)]
+        xd, gd, w1d, w2d, w3d = ref
+        scores = torch.gather(torch.softmax(xd @ gd.t(), 1), 1, idx)
+        scores = scores / scores.sum(1, keepdim=True)
+        y = torch.zeros_like(xd)
+        for e in range(E):
+            t, k = (idx == e).nonzero(as_tuple=True)
+            h = torch.nn.functional.silu(xd[t] @ w1d[e].t()) * (xd[t] @ w3d[e].t())
+            y = y.index_add(0, t, (h @ w2d[e].t()) * scores[t, k][:, None])
+        want = torch.autograd.grad(y, ref, d_out.double())
+        for name, a, b in zip(("x", "w_gate", "w1", "w2", "w3"), got, want):
+            assert rel_err(a, b) <= BF16_TOL, name
+
+
 REGION_BACKWARD_CASES = [
     # (counts, H, I): split reductions with every row and column remainder, unsplit 64-row tiles, 128-row
     # tiles, the persistent kernels at widths of 256 and 128 columns, a single row
