@@ -24,14 +24,26 @@ def _inputs(dev, T, H, E, I, bias, residual, seed):
     (16, 264, 5, 40, 1, True, True, False), (4, 1000, 4, 360, 4, False, False, True), (3, 520, 70, 1024, 5, True, False, True),
     (1, 2056, 300, 776, 16, False, True, False), (2, 72, 1024, 2056, 7, True, False, True)])
 def test_decode_step(dev, T, H, E, I, K, norm, bias, residual):
-    """Same experts as the general path's router (its logits bit for bit), output within bf16 of float64 on the same experts:
-    tokens that share experts, one expert for all, widths around the 64-deep steps and beyond a wave's share in flight."""
+    """Same logits, scores and experts as the general path's router, bit for bit (read back from the workspace), output within bf16
+    of float64 on the same experts: tokens that share experts, one expert for all, widths around the 64-deep steps and
+    beyond a wave's share in flight."""
     t = _inputs(dev, T, H, E, I, bias, residual, T * H + E)
     need = int(_lib.load().pk_region_decode_workspace_bytes(T, H, E, I, K, _lib.PK_BF16))
     ws, out = torch.empty(need, dtype=torch.uint8, device=dev), torch.empty_like(t["x"])
     call("pk_region_decode", ptr(t["x"]), _lib.PK_BF16, ptr(t["norm_w"] if norm else None), 1e-6, ptr(t["w_gate"]), ptr(t["bias"]), ptr(t["w1"]),
          ptr(t["w2"]), ptr(t["w3"]), 1, 1.5, ptr(t["residual"]), ptr(out), T, H, E, I, K, ptr(ws), need, current_stream(dev))
     x = ops.rmsnorm_fwd(t["x"], t["norm_w"], 1e-6)[0] if norm else t["x"]
+    # the workspace: the norm's output, logits, scores, experts and h, each from a multiple of 256 bytes on
+    at, took = 0, []
+    for n, dtype in ((T * H, torch.bfloat16), (T * E, torch.float32), (T * K, torch.float32), (T * K, torch.int32), (T * K * I, torch.bfloat16)):
+        took.append(ws[at:at + n * dtype.itemsize].view(dtype))
+        at += (n * dtype.itemsize + 255) // 256 * 256
+    assert at == need
+    router = ops.gate_logits(x, t["w_gate"], t["bias"])
+    scores, experts = ops.route_topk(router, K, True, 1.5)
+    if norm:
+        assert torch.equal(took[0].view(T, H), x)
+    assert torch.equal(took[1].view(T, E), router) and torch.equal(took[2].view(T, K), scores) and torch.equal(took[3].view(T, K), experts)
     d = {k: None if v is None else v.double().cpu() for k, v in t.items()}
     xd = x.double().cpu()
     logits = xd @ d["w_gate"].t() + (d["bias"] if bias else 0.0)

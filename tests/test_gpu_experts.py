@@ -731,6 +731,61 @@ def test_few_rows_an_expert_leave_out_the_transposed_copies(dev, H, I, E, K, T):
             assert rel_err(a, b) <= BF16_TOL, name
 
 
+def _dx_of_random_gradients(dev, seed, counts, H, I):
+    """d_g, d_u, w1, w3 and d_x(n): pk_region_dgrad_dx of the first n rows"""
+    from piper_amd import _lib
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    E, A = len(counts), sum(counts)
+    d_g, d_u = (torch.randn((A, I), generator=gen, device=dev).bfloat16() for _ in range(2))
+    w1, w3 = ((torch.randn((E, I, H), generator=gen, device=dev) * 0.05).bfloat16() for _ in range(2))
+    cnt = torch.tensor(counts, dtype=torch.long, device=dev)
+
+    def d_x(n):
+        c = cnt.clone()
+        c[-1] -= A - n
+        starts = ops.counts_to_starts(c)
+        out = torch.empty((n, H), dtype=torch.bfloat16, device=dev)
+        _lib.call("pk_region_dgrad_dx", d_g.data_ptr(), d_u.data_ptr(), w1.data_ptr(), w3.data_ptr(), starts.data_ptr(), out.data_ptr(), n, H, I, E,
+                  _lib.PK_BF16, _lib.current_stream(dev))
+        return out
+    return d_g, d_u, w1, w3, d_x
+
+
+def test_input_gradient_of_every_last_unit(dev):
+    """d_x in 256-row units (1,000 rows an expert and more, 8 column tiles: over 512 units) whose last unit holds one to eight
+    32-row chunks, full or with a single row: a wave has none to four of them with rows.  Against float64."""
+    H, I = 2048, 256
+    last = [129, 160, 161, 192, 193, 224, 225, 255, 1, 32, 33, 64, 65, 96, 97, 128]
+    counts = [1024 + n for n in last]
+    print(f"[case] d_x last units {last}", flush=True)
+    d_g, d_u, w1, w3, d_x = _dx_of_random_gradients(dev, 51, counts, H, I)
+    got, s = d_x(sum(counts)), 0
+    for e, c in enumerate(counts):
+        want = d_g[s:s + c].double() @ w1[e].double() + d_u[s:s + c].double() @ w3[e].double()
+        assert rel_err(got[s:s + c], want) <= BF16_TOL, (e, c)
+        assert rel_err(got[s + 1024:s + c], want[1024:]) <= BF16_TOL, (e, c)      # the last unit by itself
+        s += c
+
+
+def test_input_gradient_on_both_sides_of_the_taller_units(dev):
+    """320 rows an expert (64 experts, 2048 x 256) take d_x to 256-row units, one row fewer to 128-row ones: the same sums in the
+    same order, so the rows that both calls have get the same bits; values against float64."""
+    H, I, E = 2048, 256, 64
+    counts = [320 + (-1) ** e * (37 * (e // 2) % 150) for e in range(E)]
+    A = sum(counts)
+    assert A == 320 * E
+    print("[case] d_x at 320 rows an expert", flush=True)
+    d_g, d_u, w1, w3, d_x = _dx_of_random_gradients(dev, 53, counts, H, I)
+    tall = d_x(A)
+    assert torch.equal(d_x(A - 1), tall[:A - 1])
+    s = 0
+    for e in range(E):
+        c = counts[e]
+        want = d_g[s:s + c].double() @ w1[e].double() + d_u[s:s + c].double() @ w3[e].double()
+        assert rel_err(tall[s:s + c], want) <= BF16_TOL, (e, c)
+        s += c
+
+
 REGION_BACKWARD_CASES = [
     # (counts, H, I): split reductions with every row and column remainder, unsplit 64-row tiles, 128-row
     # tiles, the persistent kernels at widths of 256 and 128 columns, a single row
