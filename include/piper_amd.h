@@ -192,6 +192,8 @@ PK_API int pk_counts_to_starts(const void* counts, int counts_is_i64, int64_t E,
  * summation order of the products.  pk_region_decode_workspace_bytes returns 0 where it does not apply: bf16, T*K <= 16,
  * widths in multiples of 8 (H up to 8,192).  Every operand must be 16-byte aligned; gate_bias and residual may be NULL. */
 PK_API int64_t pk_region_decode_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t I, int64_t K, int dtype);
+/* HOST, tuning hint: 1 when these three launches are faster than the general path. */
+PK_API int pk_region_decode_pays(int64_t T, int64_t H, int64_t E, int64_t I, int64_t K);
 PK_API int pk_region_decode(const void* x, int dtype, const void* norm_weight, float eps, const float* w_gate,
                      const float* gate_bias, const void* w1, const void* w2, const void* w3, int route_norm,
                      float route_scale, const void* residual, void* out, int64_t T, int64_t H, int64_t E, int64_t I,

@@ -43,6 +43,7 @@ SIGNATURES = {
     "pk_region_router_norm_bwd": (_c_int, [_p, _p, _p, _p, _c_i64, _p, _c_int, _c_f32, _p, _c_int, _p, _p, _p, _p, _p, _c_int, _p,
                                            _p, _p, _p, _p, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _p, _c_i64, _p]),
     "pk_region_decode_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int]),
+    "pk_region_decode_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
     # x dtype norm_w eps w_gate bias w1 w2 w3 norm scale residual out T H E I K ws ws_bytes stream
     "pk_region_decode": (_c_int, [_p, _c_int, _p, _c_f32, _p, _p, _p, _p, _p, _c_int, _c_f32, _p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                   _p, _c_i64, _p]),

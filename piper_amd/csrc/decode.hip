@@ -170,6 +170,35 @@ int64_t pk_region_decode_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_
   return DecodeWorkspace(T, H, E, I, K).bytes;
 }
 
+// Against the general path its time grows with the tokens (every workgroup chooses the experts of all of them), with rounds of
+// experts (down: two for each of four waves) and with I (down: chunks of 768), and falls with H (down: a workgroup per eight
+// columns).  us, general -> here, tokens x experts a token:
+//   128 experts 2048 x  768   1x8 53 -> 44   2x8 81 -> 74   8x2 76 -> 73   10x1 59 -> 57   14x1 73 -> 76
+//    24         1000 x  360   1x8 31 -> 25   2x8 37 -> 33   8x2 32 -> 29   16x1 35 -> 33
+//    64          512 x  512   1x8 29 -> 25   9x1 28 -> 29   2x8 32 -> 39   16x1 31 -> 45
+//   128         1024 x  384   1x8 32 -> 27   5x2 33 -> 31   2x6 35 -> 35    2x8 37 -> 39   16x1 37 -> 43
+//    64         1536 x  768   1x8 46 -> 39   9x1 46 -> 41   2x8 66 -> 63   14x1 59 -> 58   16x1 61 -> 67
+//    16         2048 x 1024   1x8 60 -> 55   5x2 67 -> 64   4x4 70 -> 67    8x2 73 -> 77
+//    32         1024 x 1024   1x6 37 -> 35   1x8 41 -> 42   2x6 50 -> 56   16x1 46 -> 63
+//     8          512 x  256   2x8 26 -> 23   8x2 26 -> 26  16x1 26 -> 29
+//     8         1024 x 4096   1x2 48 -> 40   1x4 61 -> 63   2x8 97 -> 115
+//    16         4096 x 4096   1x4 145 -> 138  4x2 202 -> 201  2x8 252 -> 269  16x1 240 -> 300
+//    16         8192 x 1024   1x6 137 -> 133  2x4 144 -> 152  2x8 187 -> 215
+// Widths that are no multiple of 128 leave the general path smaller steps, and it loses everywhere.
+int pk_region_decode_pays(int64_t T, int64_t H, int64_t E, int64_t I, int64_t K) {
+  if (T <= 0 || K <= 0 || T > kDecodeRows || K > kDecodeRows || T * K > kDecodeRows) return 0;
+  const int64_t n = T * K;
+  const bool deep = I > 768 && H < 2 * I;
+  if (I > H) return n <= 2 || (n <= 8 && I <= 768);
+  if (H > 4096) return n <= 6;
+  if (n <= 8) return !deep || n <= 6 || (H > I && T <= 4);
+  if (H % 128 != 0 || I % 128 != 0) return I <= 1024;
+  if (deep) return 0;
+  if (E <= 8) return H <= 2048 && T <= (E <= 4 && I <= 768 ? 16 : H == 2048 ? 12 : 10);
+  if (H >= 1536) return T <= (I > 768 ? 5 : H >= 2048 ? 12 : 10);
+  return H >= 1000 && n <= (I <= 256 ? 12 : 10);
+}
+
 int pk_region_decode(const void* x, int dtype, const void* norm_weight, float eps, const float* w_gate, const float* gate_bias, const void* w1,
                      const void* w2, const void* w3, int route_norm, float route_scale, const void* residual, void* out, int64_t T, int64_t H,
                      int64_t E, int64_t I, int64_t K, void* workspace, int64_t workspace_bytes, pk_stream_t stream) {

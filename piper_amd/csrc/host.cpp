@@ -625,7 +625,7 @@ std::optional<Tensor> expert_region(const Tensor& x, const Tensor& w_gate, const
   const Tensor xc = contig(x), w1c = contig(w1), w2c = contig(w2), w3c = contig(w3);
   const Tensor gc = contig(w_gate), bc = contig(bias), rc = norm_w.defined() ? xc : contig(residual), nc = contig(norm_w);
   // a decode step: three launches of its own, nothing sorted
-  const int64_t decode_ws = route ? 0 : pk_region_decode_workspace_bytes(s.T, s.H, s.E, s.I, s.K, s.dtype);
+  const int64_t decode_ws = route || !pk_region_decode_pays(s.T, s.H, s.E, s.I, s.K) ? 0 : pk_region_decode_workspace_bytes(s.T, s.H, s.E, s.I, s.K, s.dtype);
   if (decode_ws > 0 && aligned16_all({&xc, &gc, &bc, &w1c, &w2c, &w3c, &rc, &nc})) {
     Tensor out = at::empty({s.T, s.H}, x.options());
     const Tensor ws = at::empty({decode_ws}, x.options().dtype(at::kByte));

@@ -63,6 +63,16 @@ def test_decode_step_refuses_what_the_norm_refuses():
                                            None) == norm
 
 
+def test_decode_step_pays_only_where_it_applies():
+    lib = _lib.load()
+    for T in (-1, 0, 1, 2, 5, 16, 17, 2**62):
+        for K in (0, 1, 4, 16, 17, 2**62):
+            for H, E, I in ((256, 16, 128), (2048, 128, 768), (8192, 64, 1024), (1000, 24, 360)):
+                if lib.pk_region_decode_pays(T, H, E, I, K):
+                    assert T > 0 and 0 < T * K <= 16
+                    assert K > E or lib.pk_region_decode_workspace_bytes(T, H, E, I, K, _lib.PK_BF16) > 0
+
+
 def test_counter_sets_are_handed_out_per_stream_and_capture():
     """Launches that can overlap must not share scheduling counters: every (stream, capture
     sequence) pair keeps a set of its own; the same pair always gets the same set."""

@@ -77,6 +77,30 @@ def test_decode_step_is_what_the_region_runs(dev):
         assert few == 3 and many > 3 and rel_err(got, want) <= BF16_TOL
 
 
+@pytest.mark.parametrize("T,H,E,I,K,pays", [
+    (1, 2048, 128, 768, 8, True), (2, 2048, 128, 768, 8, True), (14, 2048, 128, 768, 1, False), (12, 2048, 64, 768, 1, True), (16, 1024, 8, 512, 1, False),
+    (10, 1024, 8, 512, 1, True), (16, 1000, 24, 360, 1, True), (2, 512, 64, 512, 8, False), (1, 512, 64, 512, 8, True), (5, 1024, 128, 384, 2, True),
+    (2, 1024, 128, 384, 8, False), (1, 1024, 8, 4096, 4, False), (1, 1024, 8, 4096, 2, True), (16, 1024, 4, 512, 1, True), (2, 8192, 4, 1024, 4, False)])
+def test_decode_step_where_it_pays(dev, T, H, E, I, K, pays):
+    """On either side of pk_region_decode_pays the region takes the path that is the faster one there: three launches or the general
+    path's.  Where it does not pay the three launches still give the same result when they are called."""
+    from piper_amd import functional as F_
+    lib = _lib.load()
+    assert bool(lib.pk_region_decode_pays(T, H, E, I, K)) == pays
+    t = _inputs(dev, T, H, E, I, False, False, T + H + E + I)
+    _lib.timing_enable(True)
+    _lib.timing_collect()
+    got = F_.expert_region(t["x"], t["w_gate"], None, t["w1"], t["w2"], t["w3"], top_k=K, route_norm=True)
+    names = [n for n, _ in _lib.timing_collect()]
+    _lib.timing_enable(False)
+    assert (names == ["gate_logits", "swiglu_gate_up", "swiglu_down"]) == pays, names
+    need = int(lib.pk_region_decode_workspace_bytes(T, H, E, I, K, _lib.PK_BF16))
+    ws, out = torch.empty(need, dtype=torch.uint8, device=dev), torch.empty_like(t["x"])
+    call("pk_region_decode", ptr(t["x"]), _lib.PK_BF16, None, 0.0, ptr(t["w_gate"]), None, ptr(t["w1"]), ptr(t["w2"]), ptr(t["w3"]), 1, 1.0, None,
+         ptr(out), T, H, E, I, K, ptr(ws), need, current_stream(dev))
+    assert torch.equal(got, out) if pays else rel_err(got, out) <= BF16_TOL
+
+
 @pytest.mark.parametrize("tokens", [1, 100])
 def test_eps_that_the_norm_refuses(dev, tokens):
     """moe_block with an eps below zero raises whichever path its tokens take."""
