@@ -2375,12 +2375,8 @@ int dgrad_tile(const void* A0, const void* A1, int64_t K, const int32_t* row_map
   p.starts = starts; p.E = (int32_t)E; p.K = (int32_t)K; p.nseg = nseg; p.N = (int32_t)N;
   p.O0 = C; p.ldc = N;
   // (1536 x 384, 64 experts, d_x, 128 x 128 -> 64 x 64: 32 rows 37 -> 31, 64 rows 41 -> 40, 96 rows 44 -> 53; with the longer
-  // reduction of 2048 x 768, 128 experts: 16 rows 153 -> 155, 32 rows 158 -> 164).  In between, 1024 x 512, it is the number of
-  // 128 x 128 tiles that counts, two for every CU (64 experts, even / counts ~ 1 / sqrt(rank): 16 rows 24 -> 27 / 24 -> 26,
-  // 32 rows 25 -> 28 / 38 -> 29, 48 rows 26 -> 31 / 41 -> 31).
-  const bool few_tiles = (A / 128 + (E + 1) / 2) * pk_ceil_div(N, 128) < 2 * (int64_t)mf::persistent_grid();
-  const int64_t few_rows = K < 512 || (K == 512 && few_tiles && A > 16 * E) ? 48 : 0;
-  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), any_order, few_rows, nullptr, kernel_id, s);
+  // reduction of 2048 x 768, 128 experts: 16 rows 153 -> 155, 32 rows 158 -> 164)
+  return pk_tile::launch_ragged_m<T, false, pk_tile::PLAIN>(p, A, mf::persistent_grid(), any_order, K < 512 ? 48 : 0, nullptr, kernel_id, s);
 }
 // d_h = d_y . w2[e] with the SwiGLU backward in the epilogue.  With scores: d_y is d_out, gathered through
 // row_map, and the score gradient is left as partial sums over *part_cols columns each.

@@ -486,10 +486,17 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_o
   // workgroup to a CU (128 experts 2048 x 768, 32 rows 155 -> 185, 256 rows 402 -> 433), and not in fp32, where the matrix
   // cores are the bound and the finer tiles fill the last round better (16 experts 1024 x 512, 16,384 rows:
   // gate/up 335 -> 435, down 176 -> 215, d_h 197 -> 251, d_x 340 -> 414).
+  // Below two tiles for every CU all of them have to fit at once, also where every expert's last one is nearly empty: with
+  // uneven counts some CUs are left with a third (64 x 64 -> 128 x 128, even / counts ~ 1 / sqrt(rank): d_x, 32 experts
+  // 2048 x 768, 24 rows, 608 tiles at most 45 -> 39 / 47 -> 40, 32 rows, 640 tiles 47 -> 40 / 46 -> 63; 64 experts
+  // 1024 x 512, 16 rows 29 -> 26 / 27 -> 26, 32 rows, 640 tiles 28 -> 25 / 29 -> 38; 896 x 384, 64 rows, 672 tiles
+  // 31 -> 27 / 32 -> 38; down, 32 experts 2048 x 512, 48 rows, 704 tiles 31 -> 33 / 32 -> 39).
   if constexpr (sizeof(T) == 2 && EPI != GATE_UP) {
-    const int64_t big = (A_rows / 128 + (p.E + 1) / 2) * pk_ceil_div(p.N, 128);
-    if (EPI == BWD_SCALED && !any_order ? big >= 2 * (int64_t)cus
-                                        : A_rows > few_rows * p.E && 4 * big >= (EPI == PLAIN ? 5 : 6) * (int64_t)cus)
+    const int64_t cols = pk_ceil_div(p.N, 128), big = (A_rows / 128 + (p.E + 1) / 2) * cols;
+    const int64_t most = (A_rows / 128 + (A_rows < p.E ? A_rows : p.E)) * cols;
+    const bool fill = EPI == PLAIN ? 4 * big >= 5 * (int64_t)cus && (big >= 2 * (int64_t)cus || 5 * most <= 12 * (int64_t)cus)
+                                   : 4 * big >= 6 * (int64_t)cus;
+    if (EPI == BWD_SCALED && !any_order ? big >= 2 * (int64_t)cus : A_rows > few_rows * p.E && fill)
       return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   // row tiles that hold rows, about: every expert's last one is half full

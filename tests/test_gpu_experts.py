@@ -666,10 +666,11 @@ def test_experts_with_few_rows_and_popular_experts(dev, experts, A):
 
 
 @pytest.mark.parametrize("H,I,E,A", [(512, 768, 128, 9599), (512, 768, 128, 14336), (512, 768, 128, 24703), (2048, 128, 128, 5247),
-                                     (1024, 512, 64, 28799)])
+                                     (1024, 512, 64, 28799), (1024, 640, 64, 1663)])
 def test_one_more_row_takes_other_kernels_to_the_same_bits(dev, H, I, E, A):
     """128 experts of 512 x 768: from these sizes on one more row takes gate/up (9,600 rows), d_x (14,337) and down (24,704)
-    from the tiles to the persistent kernels, with 2048 x 128 d_x (5,248), with 64 of 1024 x 512 down (28,800).  Tiles that do not
+    from the tiles to the persistent kernels, with 2048 x 128 d_x (5,248), with 64 of 1024 x 512 down (28,800); with 64 of
+    1024 x 640 d_x goes from 128 x 128 to 64 x 64 tiles (1,664).  Tiles that do not
     split the reduction add a product's terms in the persistent kernels' order and, from a quarter above one round of gate/up
     units on, form h with their sigmoid, so at these crossings what the other rows get does not change; values against
     float64 for a few experts."""
