@@ -490,11 +490,12 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_o
   // uneven counts some CUs are left with a third (64 x 64 -> 128 x 128, even / counts ~ 1 / sqrt(rank): d_x, 32 experts
   // 2048 x 768, 24 rows, 608 tiles at most 45 -> 39 / 47 -> 40, 32 rows, 640 tiles 47 -> 40 / 46 -> 63; 64 experts
   // 1024 x 512, 16 rows 29 -> 26 / 27 -> 26, 32 rows, 640 tiles 28 -> 25 / 29 -> 38; 896 x 384, 64 rows, 672 tiles
-  // 31 -> 27 / 32 -> 38; down, 32 experts 2048 x 512, 48 rows, 704 tiles 31 -> 33 / 32 -> 39).
+  // 31 -> 27 / 32 -> 38; down, 32 experts 2048 x 512, 48 rows, 704 tiles 31 -> 33 / 32 -> 39).  From 128 rows an expert on that
+  // last tile weighs less (16 experts 2048 x 1024, 188 rows, 624 tiles: down 49 -> 37, d_x 68 -> 52, skewed).
   if constexpr (sizeof(T) == 2 && EPI != GATE_UP) {
     const int64_t cols = pk_ceil_div(p.N, 128), big = (A_rows / 128 + (p.E + 1) / 2) * cols;
     const int64_t most = (A_rows / 128 + (A_rows < p.E ? A_rows : p.E)) * cols;
-    const bool fill = EPI == PLAIN ? 4 * big >= 5 * (int64_t)cus && (big >= 2 * (int64_t)cus || 5 * most <= 12 * (int64_t)cus)
+    const bool fill = EPI == PLAIN ? 4 * big >= 5 * (int64_t)cus && (big >= 2 * (int64_t)cus || A_rows >= 128 * p.E || 5 * most <= 12 * (int64_t)cus)
                                    : 4 * big >= 6 * (int64_t)cus;
     if (EPI == BWD_SCALED && !any_order ? big >= 2 * (int64_t)cus : A_rows > few_rows * p.E && fill)
       return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
