@@ -184,7 +184,9 @@ int64_t pk_region_decode_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_
 //     8         1024 x 4096   1x2 48 -> 40   1x4 61 -> 63   2x8 97 -> 115
 //    16         4096 x 4096   1x4 145 -> 138  4x2 202 -> 201  2x8 252 -> 269  16x1 240 -> 300
 //    16         8192 x 1024   1x6 137 -> 133  2x4 144 -> 152  2x8 187 -> 215
-// Widths that are no multiple of 128 leave the general path smaller steps, and it loses everywhere.
+// Widths that are no multiple of 128 leave the general path smaller steps, and it loses everywhere.  Popular experts (counts ~ 1 /
+// sqrt(rank)) leave fewer to read and move the line up: 16 experts 640 x 128, 7x2 26 -> 23; 64 experts 512 x 256, 12x1
+// 26 -> 23 (even 27 -> 30), 16x1 26 -> 24 (27 -> 35); 128 experts 1280 x 384, 12x1 32 -> 29 (1024 x 384, even 34 -> 37).
 int pk_region_decode_pays(int64_t T, int64_t H, int64_t E, int64_t I, int64_t K) {
   if (T <= 0 || K <= 0 || T > kDecodeRows || K > kDecodeRows || T * K > kDecodeRows) return 0;
   const int64_t n = T * K;
@@ -194,9 +196,9 @@ int pk_region_decode_pays(int64_t T, int64_t H, int64_t E, int64_t I, int64_t K)
   if (n <= 8) return !deep || n <= 6 || (H > I && T <= 4);
   if (H % 128 != 0 || I % 128 != 0) return I <= 1024;
   if (deep) return 0;
-  if (E <= 8) return H <= 2048 && T <= (E <= 4 && I <= 768 ? 16 : H == 2048 ? 12 : 10);
-  if (H >= 1536) return T <= (I > 768 ? 5 : H >= 2048 ? 12 : 10);
-  return H >= 1000 && n <= (I <= 256 ? 12 : 10);
+  if (E <= 8) return H <= 2048 && T <= (E <= 4 && I <= 768 ? 16 : 12);
+  if (H >= 1536) return T <= (I > 768 ? 5 : 12);
+  return n <= (I <= 128 ? 16 : I <= 256 ? 14 : 12);
 }
 
 int pk_region_decode(const void* x, int dtype, const void* norm_weight, float eps, const float* w_gate, const float* gate_bias, const void* w1,
