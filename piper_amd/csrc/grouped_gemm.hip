@@ -629,7 +629,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
   constexpr bool SCALED = EPI == EPI_SWIGLU_BWD_SCALED;
   constexpr bool PP = NW == 8;    // two waves per SIMD: the groups of the ping-pong k-loop
   // A wave's 32-row chunks.  d_x in 256-row units: every WMW-th chunk, so that a unit with few rows is shared by both groups,
-  // and only the chunks that hold rows are multiplied (16,384 tokens, 128 experts 2048 x 768: 759 -> 721 us; 1,024 rows
+  // and only the chunks that hold rows are multiplied (16,384 tokens, 128 experts 2048 x 768: 759 -> 741 to 756 us; 1,024 rows
   // each 780 -> 752, 513 rows 504 -> 463).  Elsewhere neighbours, multiplied all or not at all: spread, gate/up of 1,024 rows
   // each goes from 808 to 822 us, d_h from 559 to 575, 128-row units by up to 2 %.
   constexpr bool SPREAD = PP && TM == 4 && EPI == EPI_PLAIN && !B_KC;
@@ -2251,14 +2251,15 @@ bool wide_fills(int64_t A, int64_t N, int64_t E, int quarters) {
 bool wide_gate_up(int64_t A, int64_t H, int64_t I, int64_t E) {
   return wide_fills(A, 2 * I, E, A <= 128 * E ? 13 : H <= 512 ? 11 : H <= 1024 ? 8 : 5);
 }
-// From this size on h is formed with the hardware's exponential and reciprocal, on the persistent kernels and on the
-// tiles alike: the line between the two kernels then moves no value.
+// From this size on h is formed with the hardware's exponential and reciprocal, on the persistent kernels and on the tiles alike:
+// the line between the two kernels then moves no value (below it the tiles take expf and a division).
 bool hw_sigmoid(int64_t A, int64_t I, int64_t E) { return wide_fills(A, 2 * I, E, 5); }
 // At widths that are not multiples of 256 the persistent kernel has 128 x 128 units, and only a long reduction makes up for
 // them (us, those units -> tiles: 384 x 640, 64 experts, 1,536 rows 267 -> 239; 512 x 128, 8 experts, 6,000 rows 47 -> 33;
 // 1024 x 384, 128 experts, 156 rows 82 -> 75; 1024 x 640, 16 experts, 1,024 rows 80 -> 82; 2048 x 896, 32 experts, 375 rows 107 -> 125).
 // With few rows an expert the tiles are ahead at any width (2048 x 768, 128 experts: 32 rows 108 / 100 / 92, 96 rows
-// 136 / 129 / 141, 128 rows 166 / 164 / 167); a call with one expert per token keeps the order of its sums (see launch_ragged_m).
+// 136 / 129 / 141, 128 rows 166 / 164 / 167); a call with one expert per token keeps the order of its sums (see launch_ragged_m), the
+// operator by itself, which has no score gradient, goes by the rows like the others.
 bool wide_dh(bool any_order, int64_t A, int64_t H, int64_t I, int64_t E) {
   return (!any_order || A > PK_DH_TILE_ROWS * E) && (I % 256 == 0 || H > 1024) && wide_fills(A, I, E, 4);
 }

@@ -471,7 +471,8 @@ inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id
 // any_order: the sums over k (and the parts of a score gradient) may be ordered otherwise than they are with the tiles that
 // the number of 64 x 64 tiles alone selects.  A token with one expert and a normalised score has a gate gradient of zero, and what
 // is left of it in floating point is the rounding of that order, in its own layer and in those in front of it: the callers
-// keep it for such tokens and for products that know nothing of the router (the forward, the operators one by one).
+// keep it for such tokens and for products that know nothing of the router (the forward, the operators one by one).  Without a
+// split all of these tiles, and the persistent kernels, add along k in the same order; a split (reduction_groups) moves it.
 // few_rows: rows an expert up to which the 64 x 64 tiles are the faster ones however many tiles there are (each
 // product's own; the caller says with what it measured).
 template <typename T, bool B_KC, int EPI>
