@@ -2402,9 +2402,10 @@ int wgrad_tile(const void* dy, const int32_t* dy_map, const void* h, const void*
                int64_t A, int64_t H, int64_t I, int64_t E, hipStream_t s) {
   pk_tile::RaggedK p = {};
   p.starts = starts; p.E = (int32_t)E; p.map_div = pk_units::make_fastdiv(div); p.accumulate = acc ? 1 : 0;
-  if (dw2) p.prob[p.nprob++] = {dy, H, dy_map, h, I, nullptr, dw2, (int32_t)H, (int32_t)I};
-  if (dw1) p.prob[p.nprob++] = {dg, I, nullptr, x, H, row_map, dw1, (int32_t)I, (int32_t)H};
-  if (dw3) p.prob[p.nprob++] = {du, I, nullptr, x, H, row_map, dw3, (int32_t)I, (int32_t)H};
+  const int32_t h32 = (int32_t)H, i32 = (int32_t)I;
+  if (dw2) p.prob[p.nprob++] = {dy, h32, h, i32, dy_map, dy_map != nullptr, 0, dw2, h32, i32};
+  if (dw1) p.prob[p.nprob++] = {dg, i32, x, h32, row_map, 0, row_map != nullptr, dw1, i32, h32};
+  if (dw3) p.prob[p.nprob++] = {du, i32, x, h32, row_map, 0, row_map != nullptr, dw3, i32, h32};
   return pk_tile::launch_ragged_k<T>(p, A, mf::persistent_grid(), pk_timing::K_SWIGLU_WGRAD, s);
 }
 

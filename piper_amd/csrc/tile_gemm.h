@@ -9,11 +9,24 @@
 //
 // One workgroup per output tile: four waves (2 x 2) for tiles of 64 x 64 or 128 x 128, two (2 x 1) for the
 // 64 x 32 tiles that fp32 ragged-M products take where 64 x 64 ones leave CUs idle.  A k-tile is 128 bytes
-// of the reduction index of every operand row (32 fp32 or 64 bf16); two or three k-tiles are in flight in
-// registers (against one: -7 %) while another is multiplied out of LDS; two LDS buffers, one barrier per
+// of the reduction index of every operand row (32 fp32 or 64 bf16); two k-tiles are in flight in
+// registers while another is multiplied out of LDS; two LDS buffers, one barrier per
 // k-tile.  The operands pass through registers rather than straight into LDS because the masking then
 // costs one select per piece and nothing has to be counted by hand.  Where the tiles are too few for
 // the chip, several groups of waves share a tile's reduction.
+//
+// What the k-loops wait for.  No load stands behind a branch (addresses are clamped, the last k-tile is masked on its way into
+// LDS), the loop has one way out, and the k-tiles past the last whole round have code of their own: then the compiler knows how
+// many loads are younger than the ones it needs.  With the loads behind masks it waited for all of them (vmcnt(0)) in every
+// second or third k-tile, so that nothing was in flight across it; three workgroups on a CU hid most of that in the ragged-M
+// products, but not in the weight gradients, whose reductions are short.  Measured, caches cold, us, before -> now:
+//   weight gradients, bf16: 24 experts 1000 x 360, 172 rows 44.1 -> 32.5; 32 experts 1024 x 512, 128 rows 56.6 -> 42.8 (64-wide
+//   tiles 70.0 -> 52); fp32: 16 experts 512 x 256, 250 rows 53.8 -> 42.4; 32 experts 1024 x 512, 128 rows 182 -> 154
+//   down 32 experts 512 -> 1024, 128 rows 17.4 -> 15.0; d_x 24 experts 1000 x 360, 172 rows 26.6 -> 24.7; gate/up 128 experts
+//   2048 x 768, 32 rows 184 -> 170, 24 experts 1000 x 360 27.3 -> 26.0, fp32 32 experts 1024 x 512 119 -> 113
+// Three k-tiles in flight, or the fragments of all four steps at once, cost a workgroup per CU (188 registers instead of
+// 144 in gate/up): 24 experts 1000 x 360, down 14.5 -> 16.0, 32 experts 1024 x 512, weight gradients in 64-wide tiles 52 -> 62.
+// What is left in a k-tile of the 64 x 64 kernels: without their loads 0.6 us, without their LDS reads 0.7, together 0.85.
 // Against one 64 x 64 FMA tile per workgroup (simt_gemm.h, which keeps the widths that are no multiple
 // of 16 bytes): see the figures at tile_gemm_ok in grouped_gemm.hip.
 #pragma once
@@ -30,6 +43,8 @@ typedef short shortx8_t __attribute__((ext_vector_type(8)));
 
 template <typename T> constexpr int kBK = 128 / (int)sizeof(T);      // reduction depth of a k-tile
 template <typename T> constexpr int kPiece = 16 / (int)sizeof(T);    // elements of a 16-byte piece
+constexpr int DEPTH = 2;      // k-tiles in flight in registers
+constexpr int AHEAD = 2;      // steps of a k-tile whose fragments are in registers or on their way there
 
 // ---- LDS tiles, in 16-byte pieces, XOR-swizzled against bank conflicts (both are X * 128 bytes):
 // KC: [X rows of the M or N index][8 pieces along k];  piece c of row r sits at c ^ ((r >> 1) & 7)
@@ -223,7 +238,7 @@ __device__ __forceinline__ int unit_of_block(int b) {
 // d_g and d_u from score * d_h, score * h for the weight gradient, and the row sums of d_h * h over a
 // tile's columns, whose total is the score's gradient.  d_h never leaves the workgroup.
 enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
-template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, int EPI>
+template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI>
 __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const RaggedM p) {
   constexpr int THREADS = 64 * WM * WN;       // of a group: WM x WN waves of TM x TN MFMA tiles
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, BK = kBK<T>, PIECE = kPiece<T>;
@@ -250,17 +265,18 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
   const int rows = min(BM, p.starts[e + 1] - row0);
   const int n0 = nt * BN;
 
-  // the thread's A rows (fixed over the reduction) and B rows or columns
+  // The thread's A rows (fixed over the reduction) and B rows or columns.  Rows past the expert's end and columns
+  // past N read the tile's first ones instead: what comes of them is stored nowhere.  Only the reduction index
+  // is masked, on the way into LDS, so that no load stands behind a branch: the compiler then counts the loads in
+  // flight, where a branch around one makes it wait for all of them.
   const T* a_ptr[LA];
   const T* b_ptr[LB];
   int b_k[LB];                       // MN weights: k-row of the piece inside a k-tile
   const int a_kofs = (tid & 7) * PIECE;
-  bool a_ok[LA], b_ok[LB];
 #pragma unroll
   for (int i = 0; i < LA; ++i) {
     const int r = (tid + i * THREADS) >> 3;
-    a_ok[i] = r < rows;
-    int64_t src = row0 + (a_ok[i] ? r : 0);
+    int64_t src = row0 + (r < rows ? r : 0);
     if (p.row_map) src = pk_units::fastdiv(p.row_map[src], p.map_div);
     a_ptr[i] = reinterpret_cast<const T*>(p.A0) + src * p.lda + a_kofs;
   }
@@ -270,45 +286,53 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
     const int s = tid + i * THREADS;
     if (B_KC) {
       const int n = n0 + (s >> 3);
-      b_ok[i] = n < p.N;
       b_k[i] = a_kofs;
-      b_ptr[i] = B + (int64_t)(b_ok[i] ? n : 0) * p.ldb + a_kofs;
+      b_ptr[i] = B + (int64_t)(n < p.N ? n : n0) * p.ldb + a_kofs;
     } else {
       b_k[i] = s / Mn<T, BN>::CPR;
       const int n = n0 + (s % Mn<T, BN>::CPR) * PIECE;
-      b_ok[i] = n < p.N;
-      b_ptr[i] = B + (int64_t)b_k[i] * p.ldb + (b_ok[i] ? n : 0);
+      b_ptr[i] = B + (int64_t)b_k[i] * p.ldb + (n < p.N ? n : n0);
     }
   }
   const int64_t seg_a = reinterpret_cast<const T*>(p.A1) - reinterpret_cast<const T*>(p.A0);
   const int64_t seg_b = reinterpret_cast<const T*>(p.B1) - reinterpret_cast<const T*>(p.B0);
   const int kt_per_seg = (p.K + BK - 1) / BK, nkt = kt_per_seg * p.nseg;
 
+  // k-tile kt into register set d: what lies past K, or past the last tile, is read from the start of the
+  // reduction and masked by deposit()
   u32x4_t ra_[DEPTH][LA], rb_[DEPTH][NB][LB];
   auto fetch = [&](auto d_c, int kt) {
     auto& ra = ra_[decltype(d_c)::value];
     auto& rb = rb_[decltype(d_c)::value];
+    kt = kt < nkt ? kt : 0;
     const bool second = kt >= kt_per_seg;
     const int k0 = (second ? kt - kt_per_seg : kt) * BK;
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    const int64_t sa = second ? seg_a : 0, sb = second ? seg_b : 0;
+    const int ka = k0 + a_kofs < p.K ? k0 : -a_kofs;
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      ra[i] = zero;
-      if (a_ok[i] && kt < nkt && k0 + a_kofs < p.K) ra[i] = *reinterpret_cast<const u32x4_t*>(a_ptr[i] + k0 + (second ? seg_a : 0));
-    }
+    for (int i = 0; i < LA; ++i) ra[i] = *reinterpret_cast<const u32x4_t*>(a_ptr[i] + (sa + ka));
 #pragma unroll
     for (int q = 0; q < NB; ++q)
 #pragma unroll
       for (int i = 0; i < LB; ++i) {
-        rb[q][i] = zero;
-        const int64_t k_at = B_KC ? (int64_t)k0 : (int64_t)k0 * p.ldb;
-        if (b_ok[i] && kt < nkt && k0 + b_k[i] < p.K)
-          rb[q][i] = *reinterpret_cast<const u32x4_t*>(b_ptr[i] + k_at + (DUAL ? (q ? seg_b : 0) : (second ? seg_b : 0)));
+        const int64_t kb = B_KC ? (int64_t)ka : (int64_t)(k0 + b_k[i] < p.K ? k0 : -b_k[i]) * p.ldb;
+        rb[q][i] = *reinterpret_cast<const u32x4_t*>(b_ptr[i] + (DUAL ? (q ? seg_b : 0) : sb) + kb);
       }
   };
-  auto deposit = [&](auto d_c, char* st) {
+  auto deposit = [&](auto d_c, int kt, char* st) {
     auto& ra = ra_[decltype(d_c)::value];
     auto& rb = rb_[decltype(d_c)::value];
+    // reduction elements left from this tile on (both operands are masked: zero times infinity is not zero)
+    const int left = kt >= nkt ? 0 : p.K - (kt >= kt_per_seg ? kt - kt_per_seg : kt) * BK;
+    if (left < BK) {
+      const u32x4_t zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int i = 0; i < LA; ++i) ra[i] = a_kofs < left ? ra[i] : zero;
+#pragma unroll
+      for (int q = 0; q < NB; ++q)
+#pragma unroll
+        for (int i = 0; i < LB; ++i) rb[q][i] = b_k[i] < left ? rb[q][i] : zero;
+    }
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
       const int s = tid + i * THREADS, r = s >> 3, c = s & 7;
@@ -344,34 +368,47 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
   const bool wave_has_rows = wm * 32 * TM < rows;
   const int mine = (nkt + KS - 1) / KS;      // k-tiles of a group (past the last one: zeros)
   // DEPTH of the group's k-tiles are in flight, each in a register set of its own
-  auto step = [&](auto d_c, int kt) {
-    constexpr int d = decltype(d_c)::value;
+  auto step = [&](auto d_c, int kt, bool more) {
     char* const st = smem + (kt & 1) * STAGE;
-    deposit(d_c, st);
+    deposit(d_c, kt * KS + group, st);
     __syncthreads();
-    if (kt + DEPTH < mine) fetch(std::integral_constant<int, d>{}, (kt + DEPTH) * KS + group);
+    if (more) fetch(d_c, (kt + DEPTH) * KS + group);
     if (wave_has_rows) {
+      Frag<T> a[AHEAD][TM], b[AHEAD][NB][TN];
+      auto read = [&](int step) {
 #pragma unroll
-      for (int step = 0; step < 4; ++step) {
-        Frag<T> a[TM], b[NB][TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = frag_kc<T>(st, (wm * TM + i) * 32, step, lane);
+        for (int i = 0; i < TM; ++i) a[step % AHEAD][i] = frag_kc<T>(st, (wm * TM + i) * 32, step, lane);
 #pragma unroll
         for (int q = 0; q < NB; ++q)
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
             const char* const t = st + A_BYTES + q * B_BYTES;
-            if constexpr (B_KC) b[q][j] = frag_kc<T>(t, (wn * TN + j) * 32, step, lane);
-            else b[q][j] = frag_mn<T, BN>(t, (wn * TN + j) * 32, step, lane);
+            if constexpr (B_KC) b[step % AHEAD][q][j] = frag_kc<T>(t, (wn * TN + j) * 32, step, lane);
+            else b[step % AHEAD][q][j] = frag_mn<T, BN>(t, (wn * TN + j) * 32, step, lane);
           }
+      };
 #pragma unroll
-        for (int q = 0; q < NB; ++q) mma_tiles<TM, TN>(acc[q], a, b[q]);
+      for (int step = 0; step < AHEAD - 1; ++step) read(step);
+#pragma unroll
+      for (int step = 0; step < 4; ++step) {
+        if (step + AHEAD - 1 < 4) read(step + AHEAD - 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < NB; ++q) mma_tiles<TM, TN>(acc[q], a[step % AHEAD], b[step % AHEAD][q]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  static_for<DEPTH>([&](auto d) { if (d < mine) fetch(d, d * KS + group); });
-  for (int kt = 0; kt < mine; kt += DEPTH)
-    static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
+  if (mine > 0) {
+    static_for<DEPTH>([&](auto d) {
+      fetch(d, d * KS + group);
+      __builtin_amdgcn_sched_barrier(0);       // in this order: the counts of loads in flight depend on it
+    });
+    int kt = 0;
+    for (; kt + DEPTH <= mine; kt += DEPTH)    // nothing to skip and one way out, for the counts' sake too
+      static_for<DEPTH>([&](auto d) { step(d, kt + d, true); });
+    static_for<DEPTH - 1>([&](auto d) { if (kt + d < mine) step(d, kt + d, false); });
+  }
   if constexpr (KS > 1) {
     add_groups<KS, NB * TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
   }
@@ -456,7 +493,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
 }
 
 // *part_cols: columns per part of the score gradient (those of a tile)
-template <typename T, int WM, int WN, int TM, int TN, int DEPTH, int KS, bool B_KC, int EPI>
+template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI>
 inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id, hipStream_t s) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   p.n_tiles = (int32_t)pk_ceil_div(p.N, BN);
@@ -464,7 +501,7 @@ inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
   if (part_cols) *part_cols = BN;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(64 * WM * WN * KS);
-  PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, DEPTH, KS, B_KC, EPI>), grid, block, 0, s, p);
+  PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, KS, B_KC, EPI>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
@@ -499,7 +536,7 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_o
     const bool fill = EPI == PLAIN ? 4 * big >= 5 * (int64_t)cus && (big >= 2 * (int64_t)cus || A_rows >= 128 * p.E || 5 * most <= 12 * (int64_t)cus)
                                    : 4 * big >= 6 * (int64_t)cus;
     if (EPI == BWD_SCALED && !any_order ? big >= 2 * (int64_t)cus : A_rows > few_rows * p.E && fill)
-      return launch_tiles<T, 2, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+      return launch_tiles<T, 2, 2, 2, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   // row tiles that hold rows, about: every expert's last one is half full
   const int64_t row_tiles = A_rows / 64 + (A_rows < p.E ? A_rows : p.E) / 2;
@@ -511,11 +548,11 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_o
     const int64_t rows = A_rows / (A_rows < p.E ? A_rows : p.E);
     //  32 x 32, four groups: 70 tiles, 408 x 472, d_x 23 -> 14; 96 tiles, 1024 x 512, d_h 26 -> 15; 96 tiles,
     //  512 x 256, d_x 16 -> 10; 126 tiles, 704 x 408, d_h 22 -> 18 (64 x 32: 18)
-    if (any_order && 8 * tiles <= 3 * (int64_t)cus) return launch_tiles<T, 1, 1, 1, 1, 2, 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+    if (any_order && 8 * tiles <= 3 * (int64_t)cus) return launch_tiles<T, 1, 1, 1, 1, 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
     //  half as wide: 128 tiles, 1024 x 512, gate/up 44 -> 30, d_h 27 -> 22
     if (2 * tiles <= cus) {
-      if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
-      return launch_tiles<T, 2, 1, 1, 1, 2, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+      if (reduction_groups(2 * tiles, k_tiles, cus) > 1) return launch_tiles<T, 2, 1, 1, 1, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+      return launch_tiles<T, 2, 1, 1, 1, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
     }
     //  half as high, where most of a tile would be padding: 64 experts 896 x 384, 8 rows, 240 tiles, gate/up 73 -> 45, 16 rows, 288
     //  tiles 68 -> 47, d_h 43 -> 28; 64 experts 512 x 256, 8 rows, 320 tiles, down 16 -> 13, d_x 27 -> 19; 128 experts
@@ -523,25 +560,27 @@ inline int launch_ragged_m(const RaggedM& p, int64_t A_rows, int cus, bool any_o
     //  (the same order as long as the 64 x 64 tiles would take two groups)
     const bool flat = 2 * tiles <= 3 * (int64_t)cus ? rows <= 16 : (EPI == BWD || EPI == BWD_SCALED) && rows <= 32 && tiles <= 2 * (int64_t)cus;
     if (flat && (any_order || reduction_groups(tiles, k_tiles, cus) == 2))
-      return launch_tiles<T, 1, 2, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+      return launch_tiles<T, 1, 2, 1, 1, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
     //  half as wide again, where the CUs would have one or two tiles: 280 tiles, 408 x 472, d_x 47 -> 29, down 26 -> 18;
     //  320 tiles, 1024 x 512, d_h 52 -> 40; 384 tiles, d_x 49 -> 39; but 490 tiles, 408 x 472, down 27 -> 34; gate/up, which
     //  reads twice the weights for its rows, 320 tiles, 1024 x 512 78 -> 83
     if (any_order && EPI != GATE_UP && tiles > cus && 2 * tiles <= 3 * (int64_t)cus && k_tiles >= 4)
-      return launch_tiles<T, 2, 1, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+      return launch_tiles<T, 2, 1, 1, 1, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
   }
   const int ks = reduction_groups(tiles, k_tiles, cus);
   // (fp32 products with so few tiles are on the finer ones above)
   if constexpr (sizeof(T) == 2)
-    if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, 2, EPI == GATE_UP ? 2 : 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
-  if (ks == 2) return launch_tiles<T, 2, 2, 1, 1, 2, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
-  return launch_tiles<T, 2, 2, 1, 1, 3, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+    if (ks == 4) return launch_tiles<T, 2, 2, 1, 1, EPI == GATE_UP ? 2 : 4, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  if (ks == 2) return launch_tiles<T, 2, 2, 1, 1, 2, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
+  return launch_tiles<T, 2, 2, 1, 1, 1, B_KC, EPI>(p, A_rows, part_cols, kernel_id, s);
 }
 
 // ---------------------------------------------------------------------------------- ragged K
 struct RaggedKProblem {
-  const void* A; int64_t lda; const int32_t* a_map;
-  const void* B; int64_t ldb; const int32_t* b_map;
+  const void* A; int32_t lda;
+  const void* B; int32_t ldb;
+  const int32_t* map;       // row map of one operand (neither: some map of as many rows all the same, if the launch has one)
+  int32_t map_a, map_b;     // which operand's rows are map[row] / map_div
   void* C;                  // [E][M][N]
   int32_t M, N;
 };
@@ -554,15 +593,14 @@ struct RaggedK {
   int32_t E, accumulate;
 };
 
-// MAPPED: some operand's rows are gathered.
-template <typename T, int TM, int TN, int DEPTH, int KS, bool MAPPED>
+// TILE: 64-wide (1) or 128-wide (2) tiles.  MAPPED: some operand's rows are gathered.
+template <typename T, int TILE, int KS, bool MAPPED>
 __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
   constexpr int THREADS = 256;
-  constexpr int BM = 64 * TM, BN = 64 * TN, BK = kBK<T>, PIECE = kPiece<T>;
-  constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
-  constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
-  using MA = Mn<T, BM>;
-  using MB = Mn<T, BN>;
+  constexpr int TM = TILE, TN = TILE, BM = 64 * TILE, BN = BM, BK = kBK<T>, PIECE = kPiece<T>;
+  constexpr int L = BM * 8 / THREADS;
+  constexpr int A_BYTES = BM * 128, STAGE = 2 * A_BYTES;
+  using M = Mn<T, BM>;
   __shared__ __attribute__((aligned(16))) char smem_[KS * 2 * STAGE];
 
   const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / THREADS);      // as in ragged_m_kernel
@@ -583,77 +621,67 @@ __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
   const int row0 = p.starts[e], rows = p.starts[e + 1] - row0;
   const int nkt = (rows + BK - 1) / BK, mine = (nkt + KS - 1) / KS;
 
-  int a_k[LA], b_k[LB], a_col[LA], b_col[LB];
+  // The thread's pieces sit at the same k-rows of both operands.  Columns past M or N read the tile's first piece instead
+  // and k-rows past the expert's end its first row: no load stands behind a branch (see ragged_m_kernel).
+  int k_row[L], a_col[L], b_col[L];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int s = tid + i * THREADS;
-    a_k[i] = s / MA::CPR;
-    a_col[i] = m0 + (s % MA::CPR) * PIECE;
+  for (int i = 0; i < L; ++i) {
+    const int s = tid + i * THREADS, c = (s % M::CPR) * PIECE;
+    k_row[i] = s / M::CPR;
+    a_col[i] = m0 + (m0 + c < q.M ? c : 0);
+    b_col[i] = n0 + (n0 + c < q.N ? c : 0);
   }
-#pragma unroll
-  for (int i = 0; i < LB; ++i) {
-    const int s = tid + i * THREADS;
-    b_k[i] = s / MB::CPR;
-    b_col[i] = n0 + (s % MB::CPR) * PIECE;
-  }
-  // Row map entries (or rows) of a k-tile, -1 past the expert's rows or the operand's columns.  MAPPED: they are
-  // requested one tile before the tile's pieces and in front of the pieces of the tile before, and divided only
-  // when their own tile is fetched: memory answers in order, so a wait for an entry never waits for pieces in
-  // flight (weight gradients of 16,384 tokens, 384 x 640, 64 experts 428 -> 353 us).
-  int a_entry[LA], b_entry[LB];
-  auto lookup = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const int k = kt * BK + a_k[i];
-      a_entry[i] = -1;
-      if (k < rows && a_col[i] < q.M) a_entry[i] = MAPPED && q.a_map ? q.a_map[row0 + k] : row0 + k;
-    }
-#pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int k = kt * BK + b_k[i];
-      b_entry[i] = -1;
-      if (k < rows && b_col[i] < q.N) b_entry[i] = MAPPED && q.b_map ? q.b_map[row0 + k] : row0 + k;
-    }
+  auto source_row = [&](int kt, int i) {
+    const int k = kt * BK + k_row[i];
+    return row0 + (k < rows ? k : 0);
   };
-  pk_units::FastDiv a_div = p.map_div, b_div = p.map_div;      // mul 0: the entries are rows already
-  if (!q.a_map) a_div.mul = 0u;
-  if (!q.b_map) b_div.mul = 0u;
-  u32x4_t ra_[DEPTH][LA], rb_[DEPTH][LB];
-  // k-tile kt into register set d; the entries of kt + KS are requested on the way if `more`
-  auto fetch = [&](auto d_c, int kt, bool more) {
+  // Row map entries of a k-tile.  MAPPED: they are requested one round of the register sets before the tile's pieces, and
+  // divided when these are fetched: memory answers in order, so a wait for them waits for nothing still needed in flight.
+  int entry_[DEPTH][L];
+  auto lookup = [&](auto d_c, int kt) {
+#pragma unroll
+    for (int i = 0; i < L; ++i) entry_[decltype(d_c)::value][i] = q.map[source_row(kt, i)];
+  };
+  u32x4_t ra_[DEPTH][L], rb_[DEPTH][L];
+  // k-tile kt into register set d; the entries of the tile after it there are requested on the way
+  auto fetch = [&](auto d_c, int kt) {
     auto& ra = ra_[decltype(d_c)::value];
     auto& rb = rb_[decltype(d_c)::value];
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
-    if constexpr (!MAPPED) lookup(kt);
-    int a_row[LA], b_row[LB];
+    int a_row[L], b_row[L];
 #pragma unroll
-    for (int i = 0; i < LA; ++i) a_row[i] = MAPPED && a_entry[i] >= 0 ? pk_units::fastdiv(a_entry[i], a_div) : a_entry[i];
-#pragma unroll
-    for (int i = 0; i < LB; ++i) b_row[i] = MAPPED && b_entry[i] >= 0 ? pk_units::fastdiv(b_entry[i], b_div) : b_entry[i];
-    if (MAPPED && more) lookup(kt + KS);
-#pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      ra[i] = zero;
-      if (a_row[i] >= 0) ra[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const T*>(q.A) + (int64_t)a_row[i] * q.lda + a_col[i]);
+    for (int i = 0; i < L; ++i) {
+      a_row[i] = b_row[i] = source_row(kt, i);
+      if constexpr (MAPPED) {
+        const int r = pk_units::fastdiv(entry_[decltype(d_c)::value][i], p.map_div);
+        a_row[i] = q.map_a ? r : a_row[i];
+        b_row[i] = q.map_b ? r : b_row[i];
+      }
     }
+    if constexpr (MAPPED) lookup(d_c, kt + DEPTH * KS);
 #pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      rb[i] = zero;
-      if (b_row[i] >= 0) rb[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const T*>(q.B) + (int64_t)b_row[i] * q.ldb + b_col[i]);
-    }
+    for (int i = 0; i < L; ++i)
+      ra[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const T*>(q.A) + (int64_t)a_row[i] * q.lda + a_col[i]);
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+      rb[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const T*>(q.B) + (int64_t)b_row[i] * q.ldb + b_col[i]);
   };
-  auto deposit = [&](auto d_c, char* st) {
+  auto deposit = [&](auto d_c, int kt, char* st) {
     auto& ra = ra_[decltype(d_c)::value];
     auto& rb = rb_[decltype(d_c)::value];
+    const int left = rows - kt * BK;
+    if (left < BK) {                           // both: zero times infinity is not zero
+      const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const int s = tid + i * THREADS, c = s % MA::CPR;
-      *reinterpret_cast<u32x4_t*>(st + a_k[i] * (MA::CPR * 16) + ((c ^ MA::swz(a_k[i])) << 4)) = ra[i];
+      for (int i = 0; i < L; ++i) ra[i] = k_row[i] < left ? ra[i] : zero;
+#pragma unroll
+      for (int i = 0; i < L; ++i) rb[i] = k_row[i] < left ? rb[i] : zero;
     }
 #pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int s = tid + i * THREADS, c = s % MB::CPR;
-      *reinterpret_cast<u32x4_t*>(st + A_BYTES + b_k[i] * (MB::CPR * 16) + ((c ^ MB::swz(b_k[i])) << 4)) = rb[i];
+    for (int i = 0; i < L; ++i) {
+      const int c = (tid + i * THREADS) % M::CPR;
+      char* const t = st + k_row[i] * (M::CPR * 16) + ((c ^ M::swz(k_row[i])) << 4);
+      *reinterpret_cast<u32x4_t*>(t) = ra[i];
+      *reinterpret_cast<u32x4_t*>(t + A_BYTES) = rb[i];
     }
   };
 
@@ -666,29 +694,38 @@ __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
   if (nkt > 0) {
-    if constexpr (MAPPED) lookup(group);
-    // (the look at `more` shortens the one k-tile of a short expert: 81 -> 77 us at 48 rows; with 64-wide tiles, whose
-    // k-tiles come three at a time, it costs more than it saves: 20 -> 25 us at 256 rows)
+    if constexpr (MAPPED) static_for<DEPTH>([&](auto d) { lookup(d, d * KS + group); });
+    __builtin_amdgcn_sched_barrier(0);
     static_for<DEPTH>([&](auto d) {
-      if (d < mine) fetch(d, d * KS + group, TM == 1 || d + 1 < mine);
+      fetch(d, d * KS + group);
+      __builtin_amdgcn_sched_barrier(0);       // in this order, as in ragged_m_kernel
     });
-    auto step = [&](auto d_c, int kt) {
+    auto step = [&](auto d_c, int kt, bool more) {
       char* const st = smem + (kt & 1) * STAGE;
-      deposit(d_c, st);
+      deposit(d_c, kt * KS + group, st);
       __syncthreads();
-      if (kt + DEPTH < mine) fetch(d_c, (kt + DEPTH) * KS + group, true);
+      if (more) fetch(d_c, (kt + DEPTH) * KS + group);
+      Frag<T> a[AHEAD][TM], b[AHEAD][TN];
+      auto read = [&](int step) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[step % AHEAD][i] = frag_mn<T, BM>(st, (wm * TM + i) * 32, step, lane);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[step % AHEAD][j] = frag_mn<T, BN>(st + A_BYTES, (wn * TN + j) * 32, step, lane);
+      };
+#pragma unroll
+      for (int step = 0; step < AHEAD - 1; ++step) read(step);
 #pragma unroll
       for (int step = 0; step < 4; ++step) {
-        Frag<T> a[TM], b[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = frag_mn<T, BM>(st, (wm * TM + i) * 32, step, lane);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) b[j] = frag_mn<T, BN>(st + A_BYTES, (wn * TN + j) * 32, step, lane);
-        mma_tiles<TM, TN>(acc, a, b);
+        if (step + AHEAD - 1 < 4) read(step + AHEAD - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_tiles<TM, TN>(acc, a[step % AHEAD], b[step % AHEAD]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     };
-    for (int kt = 0; kt < mine; kt += DEPTH)
-      static_for<DEPTH>([&](auto d) { if (kt + d < mine) step(d, kt + d); });
+    int kt = 0;
+    for (; kt + DEPTH <= mine; kt += DEPTH)
+      static_for<DEPTH>([&](auto d) { step(d, kt + d, true); });
+    static_for<DEPTH - 1>([&](auto d) { if (kt + d < mine) step(d, kt + d, false); });
     if constexpr (KS > 1) {
       add_groups<KS, TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
     }
@@ -740,8 +777,9 @@ inline int launch_ragged_k(RaggedK p, int64_t A_rows, int cus, int kernel_id, hi
     return tiles * p.E;
   };
   // 128 x 128 tiles with two of them for every CU, unless they are that much more padding: in fp32 the two are within
-  // 5 % of each other (us, 64 x 64 -> 128 x 128: 16 experts 1024 x 512, 250 rows 161 -> 152; 408 x 472, 14 % more
-  // padding, 82 -> 101), in bf16 the larger are a quarter faster (24 experts 1000 x 360, 172 rows 54 -> 41)
+  // 7 % of each other (us, 64 x 64 -> 128 x 128: 16 experts 1024 x 512, 250 rows 159 -> 148, 32 experts, 60 rows 109 -> 109;
+  // 408 x 472, 14 % more padding, 71 -> 95), in bf16 the larger are a tenth faster (24 experts 1000 x 360, 172 rows 38 -> 33,
+  // 16 experts 1024 x 512, 250 rows 39 -> 34; 408 x 472 22 -> 22)
   int64_t units = plan(128), area_128 = 0, area_64 = 0;
   for (int q = 0; q < p.nprob; ++q) {
     area_128 += pk_ceil_div(p.prob[q].M, 128) * pk_ceil_div(p.prob[q].N, 128) * 4;
@@ -753,17 +791,20 @@ inline int launch_ragged_k(RaggedK p, int64_t A_rows, int cus, int kernel_id, hi
   if (units == 0) return PK_OK;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD));
   const int ks = large ? 1 : reduction_groups(units, pk_ceil_div(pk_ceil_div(A_rows, p.E), kBK<T>), cus);
-  bool mapped = false;
-  for (int q = 0; q < p.nprob; ++q) mapped = mapped || p.prob[q].a_map || p.prob[q].b_map;
-#define PK_RAGGED_K(TILE, DEPTH, KS)                                                                                                   \
+  const int32_t* map = nullptr;
+  for (int q = 0; q < p.nprob; ++q)
+    if (p.prob[q].map) map = p.prob[q].map;
+  for (int q = 0; q < p.nprob; ++q)
+    if (!p.prob[q].map) p.prob[q].map = map;
+#define PK_RAGGED_K(TILE, KS)                                                                                                          \
   do {                                                                                                                                 \
-    if (mapped) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, TILE, TILE, DEPTH, KS, true>), grid, dim3(256 * KS), 0, s, p);      \
-    else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, TILE, TILE, DEPTH, KS, false>), grid, dim3(256 * KS), 0, s, p);            \
+    if (map) PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, TILE, KS, true>), grid, dim3(256 * KS), 0, s, p);      \
+    else PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_k_kernel<T, TILE, KS, false>), grid, dim3(256 * KS), 0, s, p);            \
   } while (0)
-  if (large) PK_RAGGED_K(2, 2, 1);
-  else if (ks == 4) PK_RAGGED_K(1, 2, 4);
-  else if (ks == 2) PK_RAGGED_K(1, 2, 2);
-  else PK_RAGGED_K(1, 3, 1);
+  if (large) PK_RAGGED_K(2, 1);
+  else if (ks == 4) PK_RAGGED_K(1, 4);
+  else if (ks == 2) PK_RAGGED_K(1, 2);
+  else PK_RAGGED_K(1, 1);
 #undef PK_RAGGED_K
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;

@@ -845,3 +845,44 @@ def test_region_input_gradient_by_size(dev, dtype, counts, H, I):
     for name, got, ref in (("d_g", dg, dg_ref * sc), ("d_u", du, du_ref * sc), ("score * h", hs, h.detach() * sc), ("d_score", ds, ds_ref),
                            ("d_x", dx, dx_ref), ("d_g unscaled", dg0, dg_ref), ("d_u unscaled", du0, du_ref)):
         assert rel_err(got, ref) <= tol, (name, rel_err(got, ref))
+
+
+# widths and row counts that leave a remainder in the last k-tile of every product
+REMAINDER_CASES = [
+    ([3, 70, 0, 129], 200, 104),        # 64-wide tiles, reductions split over groups of waves
+    ([65] * 64, 328, 136),              # 64-wide tiles, one group
+    ([190] * 24, 1000, 360),            # 128-wide tiles
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts,H,I", REMAINDER_CASES)
+def test_infinities_stay_in_the_rows_and_columns_that_hold_them(dev, dtype, counts, H, I):
+    """The tile kernels read an expert's first row, and a row's first elements, where a tile's remainder has none of its own, and mask
+    both operands: an infinity in these places is neither multiplied by zero nor seen by anybody else (bit for bit)."""
+    print(f"[case] infinities {dtype} counts={counts[:4]}x{len(counts)} H={H} I={I}", flush=True)
+    x, w1, w2, w3, dy, cnt = _make(23, counts, H, I, dtype)
+    X, W1, W2, W3, DY = (t.to(dev) for t in (x, w1, w2, w3, dy))
+    starts = ops.counts_to_starts(cnt.to(dev))
+    E, e = len(counts), 1
+    row = counts[0]                      # first row of expert 1
+    y, g, u, h = ops.grouped_swiglu_fwd(X, W1, W2, W3, starts)
+    dw1, dw2, dw3 = ops.grouped_swiglu_wgrad(DY, h, g, u, X, starts, E)      # g and u stand for any d_g and d_u
+
+    X2, DY2 = X.clone(), DY.clone()
+    X2[row, 0] = float("inf")
+    DY2[row, 5] = float("inf")
+    y2, g2, u2, h2 = ops.grouped_swiglu_fwd(X2, W1, W2, W3, starts)
+    assert torch.isinf(g2[row]).all() and torch.isinf(u2[row]).all()
+    others = torch.arange(sum(counts), device=dev) != row
+    for got, want in ((y2, y), (g2, g), (u2, u), (h2, h)):
+        assert torch.equal(got[others], want[others])
+    e1, e2, e3 = ops.grouped_swiglu_wgrad(DY2, h, g, u, X2, starts, E)
+    assert torch.isinf(e2[e, 5]).all() and torch.isinf(e1[e, :, 0]).all() and torch.isinf(e3[e, :, 0]).all()
+    keep = torch.ones(E, H, dtype=torch.bool, device=dev)
+    keep[e, 5] = False
+    assert torch.equal(e2[keep], dw2[keep])
+    keep = torch.ones(E, H, dtype=torch.bool, device=dev)
+    keep[e, 0] = False
+    keep = keep[:, None, :].expand(E, I, H)
+    assert torch.equal(e1[keep], dw1[keep]) and torch.equal(e3[keep], dw3[keep])
