@@ -1321,11 +1321,31 @@ struct WgradParams {
   const int32_t* starts;
   const int32_t* order;      // optional [E]: experts by descending row count
   int32_t E;
+  const int32_t* row_map;    // the map that some problem's a_map or b_map is; null: none has one
   FastDiv map_div;
   int32_t accumulate;
-  int32_t tiles_per_expert;  // (M/BM)*(N/BN), identical for the three problems
+  int32_t tiles_per_problem; // (M/BM)*(N/BN), identical for the three problems
   int32_t nprob;
+  int32_t run;               // wgrad_runs_kernel: neighbouring tiles of one workgroup, a divisor of tiles_per_problem
+  int32_t chunk;             // workgroups of one chunk (see dealt_unit)
 };
+
+// Workgroup b runs on XCD b % 8.  Units, sorted by expert, come in chunks of neighbours, and chunk c goes to XCD c % 8 in
+// "snake" order (0..7, 7..0, 0..7, ...): the tiles of a chunk read the same rows through one L2.  Chunks used to be whole
+// experts, which leaves XCDs idle where experts are few or uneven; now an XCD has at least 16 (deal_chunk).  us, whole experts
+// -> chunks, even counts / ~ 1 / sqrt(rank): 8 experts 2048 x 1024, 256 rows 58 -> 57 / 81 -> 58, 1,024 rows 143 -> 140 /
+// 222 -> 147; 32 experts 1024 x 512, 256 rows 59 -> 59 / 73 -> 61; 128 experts 2048 x 768, 64 rows 323 -> 323 / 337 -> 335.
+__device__ __forceinline__ int dealt_unit(int chunk) {
+  const int xcd = blockIdx.x % NXCD, pos = blockIdx.x / NXCD;
+  const int turn = pos / chunk;
+  return ((turn & 1) ? turn * NXCD + (NXCD - 1 - xcd) : turn * NXCD + xcd) * chunk + pos % chunk;
+}
+// host: the chunk for `units` units, `per_expert` of them an expert's
+int32_t deal_chunk(int64_t units, int64_t per_expert) {
+  int64_t chunk = per_expert;
+  while (chunk % 2 == 0 && units < 16 * NXCD * chunk) chunk /= 2;
+  return (int32_t)chunk;
+}
 
 template <int BM, int BN, int BK, int WMW, int WNW, int NS>
 __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams p) {
@@ -1340,20 +1360,15 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];
 
   const int nprob = p.nprob;
-  // Workgroup b runs on XCD b % 8.  All tiles of one expert stay on one XCD, back to back, so its
-  // rows are read from HBM once.  Experts are dealt to the XCDs in "snake" order (0..7, 7..0,
-  // 0..7, ...) of p.order, the experts sorted by descending row count (pk_sort_by_expert), which
-  // balances skewed routing; without an order they are dealt by index.
+  // p.order: the experts by descending row count (pk_sort_by_expert), so that the long ones start first
   const const_i32_ptr starts = as_const(p.starts);
-  const int xcd = blockIdx.x % NXCD, pos = blockIdx.x / NXCD;
-  // the problems of one expert follow each other on its XCD: d_w1 and d_w3 read the same x rows
-  const int per_expert = p.tiles_per_expert * nprob;
-  const int jq = pos / per_expert;                               // position in this XCD's queue
-  const int rem = pos % per_expert;
-  const WgradProblem& q = p.prob[rem / p.tiles_per_expert];
-  const int t = rem % p.tiles_per_expert;
-  const int want = (jq & 1) ? jq * NXCD + (NXCD - 1 - xcd) : jq * NXCD + xcd;   // rank to serve
-  if (want >= p.E) return;
+  // the problems of one expert follow each other: d_w1 and d_w3 read the same x rows
+  const int per_expert = p.tiles_per_problem * nprob;
+  const int unit = dealt_unit(p.chunk);
+  if (unit >= p.E * per_expert) return;
+  const int want = unit / per_expert, rem = unit % per_expert;
+  const WgradProblem& q = p.prob[rem / p.tiles_per_problem];
+  const int t = rem % p.tiles_per_problem;
   const int e = p.order ? as_const(p.order)[want] : want;
   const int n_tiles = q.N / BN;
   const int mt = t / n_tiles, nt = t % n_tiles;
@@ -1398,7 +1413,6 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
     }
   };
   uint32_t is_a = 0, is_b = 0;     // LDS destinations of this wave's pieces in the stage being filled
-  bool is_real = true;             // false: no tile left, the pieces read zeros (rows are not looked up)
   auto issue_setup = [&](int stage) {
     char* st = smem + stage * STAGE;
     is_a = lds_addr(st) + (wave * LA) * 1024;
@@ -1414,7 +1428,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 #pragma unroll
       for (int r = 0; r < A_RPI; ++r) {
         const int v = arow[i * A_RPI + r];
-        if (is_real && v >= 0) {
+        if (v >= 0) {
           const bf16_t* cand = Abase + (int64_t)v * lda;
           if (lane / A_CPR == r) src = cand + cofs;
         }
@@ -1428,7 +1442,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 #pragma unroll
       for (int r = 0; r < B_RPI; ++r) {
         const int v = brow[i * B_RPI + r];
-        if (is_real && v >= 0) {
+        if (v >= 0) {
           const bf16_t* cand = Bbase + (int64_t)v * ldb;
           if (lane / B_CPR == r) src = cand + cofs;
         }
@@ -1450,60 +1464,23 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  if constexpr (NS >= 3) {
-    // every slot issues its loads (rows past the expert's end read a block of zeros), so the
-    // number of loads in flight is the same at every k-tile
 #pragma unroll
-    for (int s = 0; s < NS - 1; ++s) {
-      is_real = s < nkt;
-      if (is_real) fetch_rows(s);
+  for (int s = 0; s < NS - 1; ++s)
+    if (s < nkt) {
+      fetch_rows(s);
       issue(s);
     }
-    if (NS - 1 < nkt) fetch_rows(NS - 1);
-  } else {
-#pragma unroll
-    for (int s = 0; s < NS - 1; ++s)
-      if (s < nkt) {
-        fetch_rows(s);
-        issue(s);
-      }
-    if (NS - 1 < nkt) fetch_rows(NS - 1);
-  }
+  if (NS - 1 < nkt) fetch_rows(NS - 1);
   int cur = 0, nxt = NS - 1;
-  if constexpr (NS >= 3) {
-    // Rings of three or more stages: the loads of tile kt+NS-1 and the fragment reads of the
-    // next k-step are spread between the MFMAs, and the first fragments of tile kt+1 are read
-    // during tile kt (the barrier at the top of tile kt waits for tile kt+1).
-    constexpr int L = LA + LB;
-    wait_dma<(NS - 2) * L>();
+  for (int kt = 0; kt < nkt; ++kt) {
+    if (kt + NS - 2 < nkt) wait_dma<(NS - 2) * (LA + LB)>(); else wait_dma<0>();
     block_barrier();
-    Frags<TM, TN> f0;
-    load_frags<BK, TM, TN, false, false, BM, BN>(f0, smem, smem + A_BYTES, wm * WTM, wn * WTN, 0, lane);
-    for (int kt = 0; kt < nkt; ++kt) {
-      wait_dma<(NS - 3) * L>();
-      block_barrier();
-      issue_setup(nxt);
-      is_real = kt + NS - 1 < nkt;
-      const char* st = smem + cur * STAGE;
-      const char* stn = smem + (cur + 1 == NS ? 0 : cur + 1) * STAGE;
-      mma_ktile<BK, TM, TN, false, false, BM, BN, L>(st, st + A_BYTES, stn, stn + A_BYTES, wm * WTM, wn * WTN,
-                                                     f0, acc, [&](int piece) { issue_piece(piece); });
-      if (kt + NS < nkt) fetch_rows(kt + NS);
-      cur = cur + 1 == NS ? 0 : cur + 1;
-      nxt = nxt + 1 == NS ? 0 : nxt + 1;
-    }
-    wait_dma<0>();   // zero loads of the last k-tiles: the staging below reuses the ring
-  } else {
-    for (int kt = 0; kt < nkt; ++kt) {
-      if (kt + NS - 2 < nkt) wait_dma<(NS - 2) * (LA + LB)>(); else wait_dma<0>();
-      block_barrier();
-      if (kt + NS - 1 < nkt) issue(nxt);
-      if (kt + NS < nkt) fetch_rows(kt + NS);
-      const char* st = smem + cur * STAGE;
-      mma_tile<BK, TM, TN, false, false, BM, BN, (TM * TN >= 16)>(st, st + A_BYTES, wm * WTM, wn * WTN, acc);
-      cur = cur + 1 == NS ? 0 : cur + 1;
-      nxt = nxt + 1 == NS ? 0 : nxt + 1;
-    }
+    if (kt + NS - 1 < nkt) issue(nxt);
+    if (kt + NS < nkt) fetch_rows(kt + NS);
+    const char* st = smem + cur * STAGE;
+    mma_tile<BK, TM, TN, false, false, BM, BN, (TM * TN >= 16)>(st, st + A_BYTES, wm * WTM, wn * WTN, acc);
+    cur = cur + 1 == NS ? 0 : cur + 1;
+    nxt = nxt + 1 == NS ? 0 : nxt + 1;
   }
 
   block_barrier();
@@ -1521,6 +1498,154 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
   wave_lds_fence();
   if (p.accumulate) St::template flush<WTM, true>(sbuf, C, q.N, WTM);
   else St::template flush<WTM, false>(sbuf, C, q.N, WTM);
+}
+
+// The same products for experts with few rows, where an output tile takes a handful of k-tiles: the kernel is bound by the
+// gradients that it writes, and wgrad_kernel, with one workgroup to a CU and its loads, MFMAs and stores one after the other,
+// leaves the memory idle while it waits for rows (128 experts 2048 x 768, 32 rows, us: without its loads 228, without its stores
+// 180, together 286; 1.2 GB of stores alone take 195).  Here a workgroup forms p.run neighbouring tiles of one expert and
+// problem, and the k-tiles of all of them are one sequence in a ring of three stages: the next tile's rows are on their way
+// while a tile is multiplied and stored.  The wait in front of a k-tile counts the operations behind its loads, stores among
+// them.  Every wave stages 32 rows of its output at a time in the stage that has just been multiplied, so the ring is all the LDS.
+// Tiles stay 256 wide: 512 bytes of a gradient's row leave together (128 x 128 tiles, four workgroups to a CU: 255 us; 128-wide
+// runs: 230 us for the stores alone).  us, even counts / ~ 1 / sqrt(rank), wgrad_kernel -> this: 128 experts 2048 x 768: 4 rows
+// 237 -> 211 / 237 -> 212, 32 rows 281 -> 240 / 286 -> 237, 64 rows 325 -> 258 / 342 -> 266, 128 rows 411 -> 366 / 446 -> 399;
+// 64 experts 1536 x 768, 24 rows 111 -> 90 / 109 -> 93; 32 experts 1024 x 512: 32 rows 33 -> 28 / 32 -> 28, 128 rows 45 -> 44 /
+// 54 -> 46; 16 experts 2048 x 1024, 64 rows 66 -> 54 / 71 -> 56; 24 experts 1024 x 768, 20 rows 36 -> 30 / 36 -> 30.
+// With 512 rows wgrad_kernel's deeper k-tiles are ahead (16 experts 2048 x 1024 160 / 165, 32 experts 1024 x 512, 1,024 rows
+// 145 / 152).  The order of the sums is wgrad_kernel's.
+// MAPPED: some problem's rows are gathered (p.row_map).
+template <bool ACC, bool MAPPED>
+__global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p) {
+  constexpr int WMW = 2, WNW = 4, TM = 4, TN = 2, NS = 3, NTHREADS = 64 * WMW * WNW;
+  constexpr int WTM = 32 * TM, WTN = 32 * TN, BM = WMW * WTM, BN = WNW * WTN, BK = 32;
+  constexpr int A_BYTES = BM * BK * 2, STAGE = (BM + BN) * BK * 2;
+  constexpr int L = A_BYTES / (NTHREADS * 16);        // loads of a wave for a k-tile, per operand
+  constexpr int STORES = 4 * TM;                      // stores of a wave for a tile
+  using St = Stage32<WTN>;
+  static_assert(BM == BN, "both operands' pieces lie alike");
+  static_assert(WMW * WNW * St::BYTES <= STAGE, "the output is staged in one stage");
+  __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
+
+  const const_i32_ptr starts = as_const(p.starts);
+  const int unit = dealt_unit(p.chunk);
+  const int per_problem = p.tiles_per_problem / p.run, per_expert = per_problem * p.nprob;
+  if (unit >= p.E * per_expert) return;
+  const int rank = unit / per_expert, rem = unit - rank * per_expert;
+  const int which = rem / per_problem;
+  const WgradProblem& q = p.prob[which];
+  const int e = p.order ? as_const(p.order)[rank] : rank;
+  const int n_tiles = q.N / BN;
+  const int row_begin = starts[e], rows = starts[e + 1] - row_begin;
+  const int nkt = (rows + BK - 1) / BK;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wm = wave / WNW, wn = wave % WNW;
+  const int lrow = lane & 31, lq = 4 * (lane >> 5);
+  int tile = (rem - which * per_problem) * p.run, left = p.run;
+
+  floatx16_t acc[TM][TN];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  };
+  auto store_tile = [&](char* stage) {
+    bf16_t* const C = q.C + (int64_t)e * q.M * q.N + ((int64_t)(tile / n_tiles) * BM + wm * WTM) * q.N + (tile % n_tiles) * BN + wn * WTN;
+    char* const sbuf = stage + wave * St::BYTES;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd)
+          St::put(sbuf, lrow, 32 * j + 8 * qd + lq,
+                  pack4(acc[i][j][4 * qd], acc[i][j][4 * qd + 1], acc[i][j][4 * qd + 2], acc[i][j][4 * qd + 3]));
+      wave_lds_fence();
+      St::template flush<ACC, true>(sbuf, C + (int64_t)(32 * i) * q.N, q.N, 32, lane);
+      wave_lds_fence();
+    }
+  };
+  clear();
+  if (nkt == 0) {                 // no rows: zeros, or nothing to add
+    if (!ACC)
+      for (; left > 0; --left, ++tile) store_tile(smem);
+    return;
+  }
+
+  // The lanes' pieces of a k-tile, in both operands alike, and the row map entries of the k-tile that is fetched next: they are
+  // requested one fetch ahead, in front of the loads of that fetch, so the wait for these covers them.
+  int krow[L], col[L], entry[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) mn_slot<BM>(wave * L + i, lane, krow[i], col[i]);
+  auto lookup = [&](int kt) {
+    if constexpr (MAPPED) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) {
+        const int k = kt * BK + krow[i];
+        entry[i] = p.row_map[row_begin + (k < rows ? k : rows - 1)];
+      }
+    }
+  };
+  const bool map_a = MAPPED && q.a_map, map_b = MAPPED && q.b_map;
+  const uint32_t lds = lds_addr(smem) + wave * L * 1024;
+  int f_tile = tile, f_kt = 0, f_left = left, f_stage = 0;       // what is fetched next
+  // returns the number of loads issued
+  auto fetch = [&]() -> int {
+    if (f_left == 0) return 0;
+    const bf16_t* const A = q.A + (int64_t)(f_tile / n_tiles) * BM;
+    const bf16_t* const B = q.B + (int64_t)(f_tile % n_tiles) * BN;
+    const void *a[L], *b[L];
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      const int k = f_kt * BK + krow[i], direct = row_begin + k;
+      int mapped = direct;
+      if constexpr (MAPPED) mapped = fastdiv(entry[i], p.map_div);
+      a[i] = k < rows ? (const void*)(A + (int64_t)(map_a ? mapped : direct) * q.lda + col[i]) : g_zero16;
+      b[i] = k < rows ? (const void*)(B + (int64_t)(map_b ? mapped : direct) * q.ldb + col[i]) : g_zero16;
+    }
+    f_kt = f_kt + 1 < nkt ? f_kt + 1 : 0;
+    lookup(f_kt);
+    const uint32_t to = lds + f_stage * STAGE;
+#pragma unroll
+    for (int i = 0; i < L; ++i) dma16(a[i], to + i * 1024);
+#pragma unroll
+    for (int i = 0; i < L; ++i) dma16(b[i], to + A_BYTES + i * 1024);
+    if (f_kt == 0) {
+      ++f_tile;
+      --f_left;
+    }
+    f_stage = f_stage + 1 == NS ? 0 : f_stage + 1;
+    return 2 * L;
+  };
+  lookup(0);
+  fetch();
+  // operations behind the loads of the k-tile that comes next (at least: row map entries come on top): the stores of the step
+  // that issued those, the loads and the stores of the step after it
+  int stores_before = 0, loads_behind = fetch(), stores_behind = 0;
+  for (int kt = 0, stage = 0;; stage = stage + 1 == NS ? 0 : stage + 1) {
+    wait_vm_le(stores_before + loads_behind + stores_behind);
+    // everybody's loads of this k-tile have landed, and nobody reads the stage of the last one any more, as operands or as
+    // staged output: the next fetch may overwrite it
+    block_barrier();
+    loads_behind = fetch();
+    char* const st = smem + stage * STAGE;
+    mma_tile<BK, TM, TN, false, false, BM, BN, false>(st, st + A_BYTES, wm * WTM, wn * WTN, acc);
+    stores_before = stores_behind;
+    stores_behind = 0;
+    if (++kt == nkt) {
+      block_barrier();            // every wave has read its fragments
+      store_tile(st);
+      if (--left == 0) break;
+      ++tile;
+      clear();
+      stores_behind = STORES;
+      kt = 0;
+    }
+  }
 }
 
 // ---- weight gradient with one K-contiguous operand, persistent workgroups.
@@ -2187,14 +2312,12 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 // 384 rows, 2.25 units per CU 117 -> 103).  gate/up and down gain as much with even counts between 128 and 200 rows, and
 // lose more with skewed ones (128 experts 2048 x 768, 144 rows: 243 -> 233 / 231 -> 247, 143 -> 133 / 133 -> 140).
 #define PK_RM_DX_ROWS 320
-// Weight gradient of the piecewise entry points (wgrad_kernel; the fused region runs
-// wgrad_pp_kernel, whose tile is fixed): 256x256x64 in a 2-stage ring; with fewer than
-// PK_WG_SHORTK_ROWS rows per expert on average 32-deep tiles in a 4-stage ring with the loads spread
-// between the MFMAs (measured against the 64-deep ring: -1.8 % at 256 rows per expert, +7 % at 1,024).
+// Weight gradients from row-major operands (with the transposed copies wgrad_pp_kernel, whose tile is fixed): 256 x 256
+// tiles with 64-deep k-tiles in a 2-stage ring; below PK_WG_RUNS_ROWS rows an expert wgrad_runs_kernel.
 #define PK_WG_BIG 256, 256, 64, 2, 4, 2
-#define PK_WG_BIG_THREADS 512
-#define PK_WG_BIG_SHORTK 256, 256, 32, 2, 4, 4
-#define PK_WG_SHORTK_ROWS 512
+#define PK_WG_THREADS 512
+#define PK_WG_RUNS_ROWS 512
+#define PK_WG_DYNAMIC_ROWS 512
 // rows an expert up to which d_h is formed on the tiles of tile_gemm.h
 #define PK_DH_TILE_ROWS 40
 
@@ -2827,16 +2950,37 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   }
   if (n == 0) return PK_OK;
   p.starts = starts; p.order = expert_order; p.E = (int32_t)E; p.map_div = mf::make_fastdiv(row_map_div);
+  for (int q = 0; q < n; ++q)
+    if (p.prob[q].a_map || p.prob[q].b_map) p.row_map = row_map;
   p.accumulate = accumulate ? 1 : 0;
-  p.tiles_per_expert = (int32_t)((H / 256) * (I / 256));
+  p.tiles_per_problem = (int32_t)((H / 256) * (I / 256));
   p.nprob = n;
-  const int64_t blocks = (int64_t)p.tiles_per_expert * n * pk_ceil_div(E, mf::NXCD) * mf::NXCD;
-  const int gy = 1;
+  // Few rows an expert: wgrad_runs_kernel.  Longer runs hide more of a tile's start, as long as there are several of them for
+  // every CU and none is long (us, runs of 1 / 2 / 4 tiles, even counts: 128 experts 2048 x 768, 36 tiles a CU: 16 rows 225 / 222 /
+  // 230, 32 rows 252 / 240 / 240, 48 rows 290 / 256 / 243, 96 rows 368 / 321 / 310; 64 experts 1536 x 768, 13 tiles: 24 rows
+  // 90 / 96, 48 rows 118 / 111 / 118, 128 rows 161 / 148 / 165; 16 experts 2048 x 1024, 6 tiles, 64 rows 61 / 54 / 58, 512 rows,
+  // ~ 1 / sqrt(rank) 172 / 181; 32 experts 1024 x 512, 3 tiles: 32 rows 30 / 28, 128 rows 44 / 45 (46 / 55); 64 experts
+  // 512 x 256, 1.5 tiles, 100 rows 26 / 23 (32 / 54)).
+  const bool few_rows = A < (int64_t)PK_WG_RUNS_ROWS * E;
+  const int64_t tiles = (int64_t)p.tiles_per_problem * n * E, per_cu = tiles / mf::persistent_grid();
+  p.run = 1;
+  if (few_rows) {
+    if (per_cu >= 24 && A > 32 * E && A <= 192 * E && p.tiles_per_problem % 4 == 0) p.run = 4;
+    else if (p.tiles_per_problem % 2 == 0 && per_cu >= 3 && A <= (per_cu >= 6 ? 192 : 64) * E && (per_cu < 12 || per_cu >= 24 || A > 32 * E)) p.run = 2;
+  }
+  p.chunk = mf::deal_chunk(tiles / p.run, (int64_t)p.tiles_per_problem * n / p.run);
+  const int64_t blocks = pk_ceil_div(tiles / p.run, p.chunk * (int64_t)mf::NXCD) * p.chunk * mf::NXCD;
   if (blocks > 0x7ffffff0ll) return PK_ERR_SHAPE;
-  if (A < (int64_t)PK_WG_SHORTK_ROWS * E)
-    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG_SHORTK>), dim3((unsigned)blocks, gy), dim3(PK_WG_BIG_THREADS), 0, s, p);
-  else
-    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), dim3((unsigned)blocks, gy), dim3(PK_WG_BIG_THREADS), 0, s, p);
+  const dim3 grid((unsigned)blocks), block(PK_WG_THREADS);
+#define PK_WG_RUNS(ACC)                                                                                                          \
+  do {                                                                                                                           \
+    if (p.row_map) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_runs_kernel<ACC, true>), grid, block, 0, s, p);    \
+    else PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_runs_kernel<ACC, false>), grid, block, 0, s, p);             \
+  } while (0)
+  if (!few_rows) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), grid, block, 0, s, p);
+  else if (p.accumulate) PK_WG_RUNS(true);
+  else PK_WG_RUNS(false);
+#undef PK_WG_RUNS
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }
@@ -2886,7 +3030,7 @@ int pk_grouped_swiglu_wgrad_scaled_t(const void* d_out, const void* hsT, const v
   base.accumulate = accumulate ? 1 : 0;
   // skewed routing (experts of very different size) needs the dynamic hand-out of units; with a few
   // hundred rows per expert the static one is a few per cent faster
-  const bool dynamic = A >= (int64_t)PK_WG_SHORTK_ROWS * E;
+  const bool dynamic = A >= (int64_t)PK_WG_DYNAMIC_ROWS * E;
   // the kernels address the gathered operand with 32-bit byte offsets from its base
   if (((A + row_map_div - 1) / row_map_div) * H * 2 > 0xffffffffll) return PK_ERR_SHAPE;
   auto launch = [&](mf::WgradKcParams& p, bool a_kc) -> int {

@@ -886,3 +886,51 @@ def test_infinities_stay_in_the_rows_and_columns_that_hold_them(dev, dtype, coun
     keep[e, 0] = False
     keep = keep[:, None, :].expand(E, I, H)
     assert torch.equal(e1[keep], dw1[keep]) and torch.equal(e3[keep], dw3[keep])
+
+
+# Weight gradients of 256-wide tiles: rows of one expert around the k-tile's 32, and shapes whose workgroups form one tile, two
+# neighbouring ones or four; with 512 rows an expert the 64-deep k-tiles.  Experts come in chunks that are dealt to the XCDs:
+# fewer experts than XCDs do not get here, nine leave chunks over.
+RUN_CASES = [
+    ([0, 1, 31, 32, 33, 64, 65, 100, 300], 512, 768),                # one tile at a time
+    ([31, 0, 65, 32] * 8, 1024, 512),                                # two
+    ([0, 33, 64, 1, 97, 32, 45, 90] * 16, 1024, 1024),               # four
+    ([900, 0, 31, 2, 1500, 65, 1000, 700], 1024, 512),               # 64-deep k-tiles
+]
+
+
+@pytest.mark.parametrize("counts,H,I", RUN_CASES)
+@pytest.mark.parametrize("mapped", [True, False])
+def test_weight_gradients_in_runs_of_tiles(dev, counts, H, I, mapped):
+    """Every gradient against float64, stored over NaNs and added to old values, with gathered rows and without."""
+    print(f"[case] runs of tiles counts={counts[:8]}x{len(counts)} H={H} I={I} mapped={mapped}", flush=True)
+    E, A, K = len(counts), sum(counts), 2 if mapped else 1
+    gen = torch.Generator(device=dev).manual_seed(H + I + E)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device=dev).bfloat16()
+    T = -(-A // K)
+    perm = torch.randperm(T * K, generator=gen, device=dev)[:A].int()
+    x, dy, hs, dg, du = rand(T, H), rand(T, H), rand(A, I), rand(A, I), rand(A, I)
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    order = torch.argsort(torch.tensor(counts, device=dev), descending=True, stable=True).int()
+    old = [rand(*s) for s in ((E, I, H), (E, H, I), (E, I, H))]
+    kw = dict(row_map=perm, row_map_div=K, scaled=True) if mapped else {}
+    fresh = [torch.full_like(o, float("nan")) for o in old]
+    ops.grouped_swiglu_wgrad(dy, hs, dg, du, x, starts, E, d_w1=fresh[0], d_w2=fresh[1], d_w3=fresh[2], expert_order=order, **kw)
+    added = [o.clone() for o in old]
+    ops.grouped_swiglu_wgrad(dy, hs, dg, du, x, starts, E, d_w1=added[0], d_w2=added[1], d_w3=added[2], accumulate=True, **kw)
+    rows = (perm // K).long() if mapped else torch.arange(A, device=dev)
+    first = 0
+    for e, n in enumerate(counts):
+        r = slice(first, first + n)
+        first += n
+        if e >= 16 and e + 8 < E:          # the pattern repeats
+            continue
+        xe, dye = x[rows[r]].double(), dy[rows[r]].double()
+        for got, acc, o, a, b in zip(fresh, added, old, (dg[r].double(), dye, du[r].double()), (xe, hs[r].double(), xe)):
+            want, size = a.T @ b, a.abs().T @ b.abs()
+            # fp32 sums of n products, then one rounding to bf16 (and one more of the sum with the old value)
+            bound = want.abs() * 2**-8 + size * (n + 1) * 2**-23
+            assert ((got[e].double() - want).abs() <= bound).all(), (e, n)
+            total = want + o[e].double()
+            bound = total.abs() * 2**-8 + bound + (size + total.abs()) * (n + 2) * 2**-23
+            assert ((acc[e].double() - total).abs() <= bound).all(), (e, n)
