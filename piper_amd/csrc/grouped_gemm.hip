@@ -618,10 +618,13 @@ __device__ __forceinline__ void mma_ktile(const char* At, const char* Bt, const 
 template <int BM, int BN, int BK, int WMW, int WNW, int NS, bool B_KC, int EPI, bool A_T = false>
 __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMParams p) {
   constexpr int NW = WMW * WNW, NTHREADS = 64 * NW;
-  constexpr int WTM = BM / WMW, WTN = BN / WNW;          // wave tile
-  constexpr int TM = WTM / 32, TN = WTN / 32;
+  constexpr int WTN = BN / WNW;                           // wave tile: TM chunks of 32 rows (some waves one less), WTN columns
+  constexpr int TM = (BM / 32 + WMW - 1) / WMW, TN = WTN / 32;
   constexpr int A_BYTES = BM * BK * 2, STAGE = (BM + BN) * BK * 2;
-  constexpr int LA = A_BYTES / (NTHREADS * 16), LB = (STAGE - A_BYTES) / (NTHREADS * 16), L = LA + LB;
+  // A loads of a wave for a k-tile: LAF of 64 lanes and, where these do not come out even (160 rows), one of LAP lanes
+  constexpr int LAF = A_BYTES / (NTHREADS * 16), LAP = A_BYTES % (NTHREADS * 16) / (NW * 16);
+  constexpr int LA = LAF + (LAP ? 1 : 0), LB = (STAGE - A_BYTES) / (NTHREADS * 16), L = LA + LB;
+  static_assert(BM % 32 == 0 && !(A_T && LAP), "whole chunks");
   static_assert(LA >= 1 && LB >= 1 && TM >= 1 && TN >= 1, "tile too small for the wave grid");
   static_assert(EPI != EPI_SWIGLU || (WTN % 64 == 0), "gate/up pairs must stay inside a wave");
   static_assert(EPI != EPI_SWIGLU_BWD_SCALED || WTN == 64, "one score-gradient partial per 64 columns");
@@ -632,7 +635,8 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
   // and only the chunks that hold rows are multiplied (16,384 tokens, 128 experts 2048 x 768: 759 -> 741 to 756 us; 1,024 rows
   // each 780 -> 752, 513 rows 504 -> 463).  Elsewhere neighbours, multiplied all or not at all: spread, gate/up of 1,024 rows
   // each goes from 808 to 822 us, d_h from 559 to 575, 128-row units by up to 2 %.
-  constexpr bool SPREAD = PP && TM == 4 && EPI == EPI_PLAIN && !B_KC;
+  // 160-row units too: five chunks, of which the first group has three.
+  constexpr bool SPREAD = PP && ((TM == 4 && EPI == EPI_PLAIN && !B_KC) || LAP);
   constexpr int RS = SPREAD ? 32 * WMW : 32;
   constexpr int OUT_COLS = (EPI == EPI_SWIGLU) ? WTN / 2 : WTN;   // columns a wave writes per output tensor
   constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;       // output columns per tile
@@ -656,13 +660,15 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
   static_assert(SMEM_BYTES + RM_BYTES + BOX_BYTES <= 160 * 1024, "LDS budget");
   __shared__ __attribute__((aligned(1024))) char smem[SMEM_BYTES + RM_BYTES + BOX_BYTES];
   constexpr int CPR = BK / 8, RPI = 64 / CPR;            // 16-byte chunks per A row, A rows per dma16
-  static_assert(LA * RPI <= 64, "a wave's A rows of a tile: one entry per lane");
+  constexpr int RPP = LAP / CPR;                         // A rows of the short load
+  static_assert(LAF * RPI + RPP <= 64, "a wave's A rows of a tile: one entry per lane");
+  static_assert(LAP % CPR == 0, "whole rows");
   static_assert(!A_T || BM % 32 == 0, "whole 32-row blocks of the transposed copy");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WNW, wn = wave % WNW;
-  const int wrow = SPREAD ? 32 * wm : WTM * wm;            // first row of the wave's first chunk
+  const int wrow = SPREAD ? 32 * wm : BM / WMW * wm;            // first row of the wave's first chunk
   // staging area while `cur_stage` is the stage of the coming unit's k-tile 0
   auto staging_area = [&](int cur_stage) -> char* {
     return ALIAS ? smem + (cur_stage == 0 ? NS - 1 : cur_stage - 1) * STAGE : smem + RING;
@@ -689,7 +695,11 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
   // ---- lane constants of the loaders: byte offsets of a lane's 16 bytes from a wave-uniform base
   uint32_t a_kofs[LA];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) { int r, k; kc_slot<BK>(wave * LA + i, lane, r, k); a_kofs[i] = (uint32_t)k * 2u; }
+  for (int i = 0; i < LAF; ++i) { int r, k; kc_slot<BK>(wave * LAF + i, lane, r, k); a_kofs[i] = (uint32_t)k * 2u; }
+  // tile row of lane `lane` in load i, and its place among the wave's rows; the short load's rows lie behind all others
+  auto a_place = [&](int i) { return i < LAF ? i * RPI + lane / CPR : LAF * RPI + lane / CPR % (RPP ? RPP : 1); };
+  auto a_row = [&](int i) { return i < LAF ? wave * LAF * RPI + a_place(i) : NW * LAF * RPI + wave * RPP + a_place(i) - LAF * RPI; };
+  if constexpr (LAP) a_kofs[LAF] = (uint32_t)(((lane % CPR) ^ kc_swz<BK>(a_row(LAF))) * 8) * 2u;
   // EPI_SWIGLU: the rows of a wave's B pieces are 32 consecutive tile rows, i.e. 32 gate rows
   // (even waves) or 32 up rows (odd waves): a wave reads one of the two matrices only
   static_assert(EPI != EPI_SWIGLU || (B_KC && LB * RPI == 32), "a wave's B pieces are one 32-row group");
@@ -749,20 +759,21 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
       if (!p.row_map) {
 #pragma unroll
         for (int i = 0; i < LA; ++i) {
-          const int rbase = (wave * LA + i) * RPI;     // first tile row of this dma16 (wave-uniform)
-          t.voff_a[i] = (uint32_t)min(rbase + lane / CPR, t.rows - 1) * row_bytes + a_kofs[i];   // rows past the range are never stored
+          t.voff_a[i] = (uint32_t)min(a_row(i), t.rows - 1) * row_bytes + a_kofs[i];   // rows past the range are never stored
         }
       }
     }
   };
-  // With a row map the A rows are gathered: the entries of the wave's LA * RPI tile rows of unit t
+  // With a row map the A rows are gathered: the entries of the wave's tile rows of unit t
   // go straight into LDS (one 4-byte load per lane, nothing waits for it), and the loader turns
   // them into lane offsets when it enters the unit, by which time they have landed: every
   // vector-memory operation of a wave retires in issue order, and the k-loop has by then waited
   // for tiles requested after them (rows_landed below).
   int* const rm_area = reinterpret_cast<int*>(smem + SMEM_BYTES) + wave * 64;
   auto request_rows = [&](const Unit& t) {
-    const int r = wave * (LA * RPI) + lane % (LA * RPI);
+    int r = wave * (LAF * RPI) + lane % (LAF * RPI);
+    if constexpr (LAP)
+      if (lane >= LAF * RPI) r = NW * LAF * RPI + wave * RPP + (lane - LAF * RPI) % RPP;
     dma4_s((uint32_t)(t.row0 + min(r, t.rows - 1)) * 4u, p.row_map, lds_addr(rm_area));
   };
 
@@ -791,7 +802,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
     if (p.row_map) {
 #pragma unroll
       for (int i = 0; i < LA; ++i)
-        ld_voff_a[i] = (uint32_t)fastdiv(rm_area[i * RPI + lane / CPR], p.map_div) * row_bytes + a_kofs[i];
+        ld_voff_a[i] = (uint32_t)fastdiv(rm_area[a_place(i)], p.map_div) * row_bytes + a_kofs[i];
     } else {
 #pragma unroll
       for (int i = 0; i < LA; ++i) ld_voff_a[i] = t.voff_a[i];
@@ -799,14 +810,16 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
     ld_idle = false;
     ld_point(0);
   };
-  uint32_t ld_lds_a = 0, ld_lds_b = 0;     // LDS destinations of this wave's pieces in the stage being filled
+  uint32_t ld_lds_a = 0, ld_lds_ap = 0, ld_lds_b = 0;     // LDS destinations of this wave's pieces in the stage being filled
   auto ld_target = [&](int stage) {
-    ld_lds_a = lds_addr(smem) + stage * STAGE + wave * (LA * 1024);
+    ld_lds_a = lds_addr(smem) + stage * STAGE + wave * (LAF * 1024);
+    if constexpr (LAP) ld_lds_ap = lds_addr(smem) + stage * STAGE + NW * LAF * 1024 + wave * (LAP * 16);
     ld_lds_b = lds_addr(smem) + stage * STAGE + A_BYTES + wave * (LB * 1024);
   };
   auto issue_piece = [&](auto piece_c) {
     constexpr int P = decltype(piece_c)::value;
-    if constexpr (P < LA) dma16_s<P * 1024>(ld_voff_a[P], ld_a, ld_lds_a);
+    if constexpr (P < LAF) dma16_s<P * 1024>(ld_voff_a[P], ld_a, ld_lds_a);
+    else if constexpr (P < LA) { if (lane < LAP) dma16_s<0>(ld_voff_a[P], ld_a, ld_lds_ap); }
     else dma16_s<(P - LA) * 1024>(voffB[P - LA], ld_b, ld_lds_b);
   };
   Unit cur_u, nxt_u;
@@ -957,7 +970,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
         };
         const int live = min(TM, max(0, (cur_u.rows - wrow + RS - 1) / RS));
         if (live == TM) k_loop(std::integral_constant<int, TM>{});
-        else if (live == 3) k_loop(std::integral_constant<int, 3>{});
+        else if (TM > 3 && live == 3) k_loop(std::integral_constant<int, (TM > 3 ? 3 : 0)>{});
         else if (live == 2) k_loop(std::integral_constant<int, 2>{});
         else if (live == 1) k_loop(std::integral_constant<int, 1>{});
         else k_loop(std::integral_constant<int, 0>{});
@@ -2312,6 +2325,22 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 // 384 rows, 2.25 units per CU 117 -> 103).  gate/up and down gain as much with even counts between 128 and 200 rows, and
 // lose more with skewed ones (128 experts 2048 x 768, 144 rows: 243 -> 233 / 231 -> 247, 143 -> 133 / 133 -> 140).
 #define PK_RM_DX_ROWS 320
+// 160 rows, otherwise like the 128-row ones: what fits the LDS (3 x 52 KB).  A unit costs about a fifth more time than one of
+// 128 rows and there are fewer of them, above all fewer with a handful of rows (256 rows an expert: two units where half of
+// the experts had three).  tall_units_pay says when; 128 (or where named 256) rows -> 160, us, even counts / ~ 1 / sqrt(rank):
+// 128 experts 2048 x 768: 256 rows: gate/up 285 -> 260 / 281 -> 273, down 174 -> 164 / 177 -> 170, d_x 280 -> 259 / 280 -> 270; 480
+// rows: gate/up 449 -> 418 / 449 -> 426, down 270 -> 253 / 274 -> 247; 224 rows: 266 -> 271 / 260 -> 257, 162 -> 165 / 165 -> 161,
+// 253 -> 262 / 264 -> 255; 111 rows 199 -> 197 / 194 -> 198.  64 experts 1536 x 768, 450 rows: 198 -> 178 / 200 -> 179, 115 -> 105 /
+// 114 -> 110.  Few rounds of units, where the last one counts: 16 experts 2048 x 1024, 512 rows 114 -> 97 / 109 -> 94, 70 -> 63 / 66 -> 60,
+// 108 -> 95 / 104 -> 98; 64 experts 2048 x 768, 256 rows (3.75 rounds -> 3.15) 157 -> 168 / 159 -> 167; 8 experts 1024 x 512, 4,000 rows
+// (3.97 -> 3.19) 94 -> 103 / 95 -> 100; 128 experts 1024 x 512, 300 rows (5.7 -> 4.75) 134 -> 140 / 136 -> 144.
+// Against 256 rows: gate/up at any size (128 experts 2048 x 768: 512 rows 463 -> 446 / 468 -> 434, 1,024 rows 833 -> 809 / 836 -> 810;
+// 16 experts 2048 x 1024, 2,048 rows 302 -> 279 / 310 -> 281), down with a long reduction (64 experts 2048 x 1024, 512 rows 191 -> 179 /
+// 191 -> 177; but 2048 x 768, 512 rows 267 -> 277 / 278 -> 263, 1,024 rows 490 -> 494 / 493 -> 493), d_x not (512 rows 423 -> 440 /
+// 429 -> 430, 1,024 rows 748 -> 804 / 763 -> 805).
+#define PK_RM_TALL 160, 256, 64, 2, 4, 3
+#define PK_RM_TALL_ROWS 248
+#define PK_RM_TALL_DOWN_K 1024
 // Weight gradients from row-major operands (with the transposed copies wgrad_pp_kernel, whose tile is fixed): 256 x 256
 // tiles with 64-deep k-tiles in a 2-stage ring; below PK_WG_RUNS_ROWS rows an expert wgrad_runs_kernel.
 #define PK_WG_BIG 256, 256, 64, 2, 4, 2
@@ -2327,6 +2356,16 @@ bool mfma_shape_ok(int64_t H, int64_t I) { return H % 128 == 0 && I % 128 == 0; 
 // products of such widths run on the tiles of tile_gemm.h (24,000 rows of 24 experts, 640 x 896, us, these tiles ->
 // those: down 63 -> 55, weight gradients 375 -> 176, d_x 94 -> 92).
 #define PK_RM_ALT 128, 128, 64, 2, 2, 4
+
+// Whether units of 160 rows are ahead of 128: with more than six rounds of the latter wherever there are fewer of the former, below
+// that by the number of rounds, a taller one at six fifths of the time (where that is a draw, from 352 rows an expert on).
+bool tall_units_pay(int64_t A, int64_t E, int64_t cols) {
+  if (A < (int64_t)PK_RM_TALL_ROWS * E) return false;
+  const int64_t grid = mf::persistent_grid(), u128 = (A / 128 + E / 2) * cols, u160 = (A / 160 + E / 2) * cols;
+  if (u128 >= 6 * grid) return true;
+  const int64_t c128 = 5 * pk_ceil_div(u128, grid), c160 = 6 * pk_ceil_div(u160, grid);
+  return c160 < c128 || (c160 == c128 && A >= 352 * E);
+}
 
 // 256 output columns per unit (for the gate/up kernel 128 gate and 128 up columns).
 template <bool B_KC, int EPI, bool A_T = false>
@@ -2350,9 +2389,14 @@ int launch_rm(mf::RaggedMParams& p, int64_t A, int64_t N, int kernel_id, hipStre
   // and u, the arithmetic, six stores per value), which 256-row units do not shorten, and with
   // 128 accumulator registers that epilogue spills (measured 14 % slower at 16,384 tokens even
   // with the packed outputs staged 32 columns at a time)
-  if (EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)(DX ? PK_RM_DX_ROWS : PK_RM_SHORT_ROWS) * p.E)
-    return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
-  if constexpr (EPI != mf::EPI_SWIGLU_BWD_SCALED) return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  const bool low = EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)(DX ? PK_RM_DX_ROWS : PK_RM_SHORT_ROWS) * p.E;
+  if constexpr ((EPI == mf::EPI_SWIGLU || EPI == mf::EPI_PLAIN) && !A_T) {
+    if ((low || EPI == mf::EPI_SWIGLU || (B_KC && p.Kseg >= PK_RM_TALL_DOWN_K)) && tall_units_pay(A, p.E, p.n_tiles))
+      return mf::launch_ragged_m<PK_RM_TALL, B_KC, EPI>(p, A, kernel_id, s);
+  }
+  if (low || EPI == mf::EPI_SWIGLU) return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  if constexpr (EPI != mf::EPI_SWIGLU_BWD_SCALED && EPI != mf::EPI_SWIGLU)
+    return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
   return PK_ERR_SHAPE;
 }
 

@@ -934,3 +934,44 @@ def test_weight_gradients_in_runs_of_tiles(dev, counts, H, I, mapped):
             total = want + o[e].double()
             bound = total.abs() * 2**-8 + bound + (size + total.abs()) * (n + 2) * 2**-23
             assert ((acc[e].double() - total).abs() <= bound).all(), (e, n)
+
+
+@pytest.mark.parametrize("mapped", [True, False])
+@pytest.mark.parametrize("skew", [True, False])
+def test_units_of_160_rows(dev, mapped, skew):
+    """Sizes that the persistent products take in units of 160 rows (gate/up, down and d_x alike): experts around one and two units, with
+    one row, a chunk and one, and none.  Every result against float64 of what the product read."""
+    H, I, E, A = 768, 1024, 8, 21504
+    counts = [0, 1, 159, 160, 161, 321, 33] if skew else [2560, 2720, 2687, 2689, 2700, 2721, 2710]
+    counts.append(A - sum(counts))
+    print(f"[case] units of 160 rows counts={counts} mapped={mapped}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(160 + skew)
+    rand = lambda *shape, scale=1.0: (torch.randn(shape, generator=gen, device=dev) * scale).bfloat16()
+    K = 2 if mapped else 1
+    x = rand(A // K, H)
+    w1, w3, w2 = rand(E, I, H, scale=0.05), rand(E, I, H, scale=0.05), rand(E, H, I, scale=0.05)
+    perm = torch.randperm(A, generator=gen, device=dev).int()
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    kw = dict(row_map=perm, row_map_div=K, num_rows=A) if mapped else {}
+    y, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts, **kw)
+    dx = ops.grouped_swiglu_dgrad_dx(g, u, w1, w3, starts)                 # g and u stand for any d_g and d_u
+    rows = (perm // K).long() if mapped else torch.arange(A, device=dev)
+
+    def check(got, pairs, what):
+        """got: the sum of the products of `pairs`, in fp32 and rounded once"""
+        want = sum(a @ b for a, b in pairs)
+        size, k = sum(a.abs() @ b.abs() for a, b in pairs), sum(a.shape[1] for a, _ in pairs)
+        assert ((got.double() - want).abs() <= want.abs() * 2**-8 + size * (k + 1) * 2**-23).all(), what
+
+    first = 0
+    for e, n in enumerate(counts):
+        r = slice(first, first + n)
+        first += n
+        xe, ge, ue, he = x[rows[r]].double(), g[r].double(), u[r].double(), h[r].double()
+        check(g[r], [(xe, w1[e].double().T)], ("g", e, n))
+        check(u[r], [(xe, w3[e].double().T)], ("u", e, n))
+        # silu with the hardware's exponential and reciprocal, one rounding to bf16
+        want = torch.nn.functional.silu(ge) * ue
+        assert ((he - want).abs() <= want.abs() * (2**-8 + 2**-18) + 1e-30).all(), ("h", e, n)
+        check(y[r], [(he, w2[e].double().T)], ("y", e, n))
+        check(dx[r], [(ge, w1[e].double()), (ue, w3[e].double())], ("d_x", e, n))
