@@ -118,13 +118,23 @@ template <typename T>
 __device__ __forceinline__ void to_planes(const Raw<T>& r, bf16x4_t (&out)[Planes<T>::N]) {
   constexpr int P = Planes<T>::N;
   if constexpr (std::is_same<T, float>::value) {
-    bf16_t pl[4][P];
+    // split(), two values to a conversion: the pair is also where the rounded values are taken from
+    typedef float floatx2_t __attribute__((ext_vector_type(2)));
+    typedef bf16_t bf16x2_t __attribute__((ext_vector_type(2)));
+    static_assert(P == 3, "three planes");
 #pragma unroll
-    for (int j = 0; j < 4; ++j) split<P>(r.v[j], pl[j]);
+    for (int j = 0; j < 4; j += 2) {
+      floatx2_t v = {r.v[j], r.v[j + 1]};
 #pragma unroll
-    for (int q = 0; q < P; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) out[q][j] = pl[j][q];
+      for (int q = 0; q < 3; ++q) {
+        const bf16x2_t b = __builtin_convertvector(v, bf16x2_t);
+        out[q][j] = b[0];
+        out[q][j + 1] = b[1];
+        const uint32_t u = __builtin_bit_cast(uint32_t, b);
+        v[0] -= __builtin_bit_cast(float, u << 16);
+        v[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+      }
+    }
   } else {
 #pragma unroll
     for (int q = 0; q < P; ++q) out[q] = r.v[q];
@@ -139,9 +149,26 @@ struct Lds {
   __attribute__((aligned(16))) bf16_t Bs[Planes<TB>::N][B_KC ? BN * LDK : BK * LDB];
 };
 
+// How k-tiles are requested ahead (see product).  2: two in flight, for the products whose reduction is long: the forward from bf16
+// and the weight gradients.  1: one, for the fp32 forward, whose split takes the registers of the second (64 experts 1024 wide,
+// 10,000 tokens 18.5 -> 17.6 us).  0: one, ordered by the compiler, for d_x: its reduction over the experts is one to four k-tiles.
+template <bool A_KC, bool B_KC, typename TA>
+constexpr int in_flight() { return A_KC && !B_KC ? 0 : A_KC && std::is_same<TA, float>::value ? 1 : 2; }
+
+// What bounds these products is the instructions and the waits around their matrix instructions, 6 or 12 a wave and k-tile.  The
+// addresses are worked out once and advance by a constant, and the fp32 values are split two to a conversion: 100 vector
+// instructions for two k-tiles of the bf16 forward, where forming the addresses of every load, masking it and splitting values one
+// by one took 260.  The older of two k-tiles in flight is waited for by count, as nothing in the loop is conditional; without the
+// scheduling barriers the compiler puts the requests behind the products and converts the younger tile first.  Four waves a
+// SIMD (128 registers) matter more than a second k-tile.  us, before -> now, 128 experts 2048 wide unless said: forward 16,384 tokens
+// 53 -> 47, 4,096 19.2 -> 18.6, 509 (all requested at once) 12.7 -> 12.0, 8 experts, 16,384 37 -> 25; weight gradient 16,384 60 -> 56,
+// fp32, 64 experts 1024 wide, 4,000 15.0 -> 11.4; d_x 16,384 96 -> 85; the router's backward in one launch (router_grads_kernel)
+// 16,384 202 -> 189, 4,096 62 -> 58, 3,000 36 -> 33.
+// (Its weight gradient's tiles dealt out among those of the gather instead of in front of them: 190 -> 195 to 262.)
+//
 // acc of one wave: rows m0 + 32 wm .., columns n0 + 32 wn .. of the product over k in [kbeg, kend).
 // AHEAD > 0: the reduction has at most that many k-tiles, and all of them are requested at once.
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0>
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0, int FLIGHT = 2>
 __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
                                         int64_t kend, floatx16_t& acc) {
   constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
@@ -159,9 +186,8 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
 
-  // every thread fetches 4 consecutive elements of the contiguous index per load (every plane of
-  // them for a pre-split operand); the loads of tile k+1 are in flight while tile k is multiplied
-  // (two, four and eight tiles in flight: no gain at 509 tokens, 2 to 20 % slower at 16,384)
+  // Every thread fetches 4 consecutive elements of the contiguous index per load (every plane of them for a pre-split operand).
+  // No load stands behind a branch: rows past the ends are read from the last ones, and their results are not stored.
   constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
   static_assert(NA >= 1 && NB >= 1, "tile too small for the thread count");
   struct Tile { Raw<TA> a[NA]; Raw<TB> b[NB]; };
@@ -169,39 +195,62 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
     if (kc) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); }
     else { row = (idx % (R / 4)) * 4; k = idx / (R / 4); }
   };
-  // (AHEAD: every load is made, past the ends from the last elements, as a branch would hold up the loads behind it;
-  // what lies past kend is cleared when it goes to LDS)
-  auto load_tile = [&](Tile& t, int64_t k0) {
-    if constexpr (AHEAD > 0) {
+  const MA* pa[NA];
+  const MB* pb[NB];
 #pragma unroll
-      for (int i = 0; i < NA; ++i) {
-        int m, k;
-        slot(tid + i * THREADS, A_KC, BM, m, k);
-        const int64_t mm = min(m0 + m, p.M - (A_KC ? 1 : 4)), kk = min(k0 + k, kend - (A_KC ? 4 : 1));
-        fetch4<TA>(A + mm * p.sam + kk * p.sak, p.plane_a, t.a[i]);
-      }
+  for (int i = 0; i < NA; ++i) {
+    int m, k;
+    slot(tid + i * THREADS, A_KC, BM, m, k);
+    pa[i] = A + min(m0 + m, p.M - (A_KC ? 1 : 4)) * p.sam + (A_KC ? kbeg + k : (kbeg + k) * p.sak);
+  }
 #pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        int n, k;
-        slot(tid + i * THREADS, B_KC, BN, n, k);
-        const int64_t nn = min(n0 + n, p.N - (B_KC ? 1 : 4)), kk = min(k0 + k, kend - (B_KC ? 4 : 1));
-        fetch4<TB>(B + kk * p.sbk + nn * p.sbn, p.plane_b, t.b[i]);
-      }
-      return;
-    }
+  for (int i = 0; i < NB; ++i) {
+    int n, k;
+    slot(tid + i * THREADS, B_KC, BN, n, k);
+    pb[i] = B + min(n0 + n, p.N - (B_KC ? 1 : 4)) * p.sbn + (B_KC ? kbeg + k : (kbeg + k) * p.sbk);
+  }
+  const int64_t step_a = A_KC ? BK : BK * p.sak, step_b = B_KC ? BK : BK * p.sbk;
+  const int64_t left = kend - kbeg;            // (nothing, or less, where the splits outnumber the k-tiles)
+  const int full = left > 0 ? (int)(left / BK) : 0, rest = left > 0 ? (int)(left % BK) : 0;
+  // the next k-tile, which is a whole one
+  auto request = [&](Tile& t) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) { fetch4<TA>(pa[i], p.plane_a, t.a[i]); pa[i] += step_a; }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) { fetch4<TB>(pb[i], p.plane_b, t.b[i]); pb[i] += step_b; }
+  };
+  // the next k-tile, of which only `have` (a multiple of 4 along a contiguous k) are there, the others from the last of them
+  auto request_rest = [&](Tile& t, int have) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       int m, k;
       slot(tid + i * THREADS, A_KC, BM, m, k);
-      zero_raw<TA>(t.a[i]);
-      if (m0 + m < p.M && k0 + k < kend) fetch4<TA>(A + (m0 + m) * p.sam + (k0 + k) * p.sak, p.plane_a, t.a[i]);
+      const int64_t back = max(0, k - (have - (A_KC ? 4 : 1)));
+      fetch4<TA>(pa[i] - (A_KC ? back : back * p.sak), p.plane_a, t.a[i]);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       int n, k;
       slot(tid + i * THREADS, B_KC, BN, n, k);
-      zero_raw<TB>(t.b[i]);
-      if (n0 + n < p.N && k0 + k < kend) fetch4<TB>(B + (k0 + k) * p.sbk + (n0 + n) * p.sbn, p.plane_b, t.b[i]);
+      const int64_t back = max(0, k - (have - (B_KC ? 4 : 1)));
+      fetch4<TB>(pb[i] - (B_KC ? back : back * p.sbk), p.plane_b, t.b[i]);
+    }
+  };
+  // k-tile i of a reduction that is requested as a whole: past its end from its last elements
+  auto request_clamped = [&](Tile& t, int i) {
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+      int m, k;
+      slot(tid + j * THREADS, A_KC, BM, m, k);
+      const int64_t go = min((int64_t)(k + i * BK), left - (A_KC ? 4 : 1)) - k;
+      fetch4<TA>(pa[j] + (A_KC ? go : go * p.sak), p.plane_a, t.a[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      int n, k;
+      slot(tid + j * THREADS, B_KC, BN, n, k);
+      const int64_t go = min((int64_t)(k + i * BK), left - (B_KC ? 4 : 1)) - k;
+      fetch4<TB>(pb[j] + (B_KC ? go : go * p.sbk), p.plane_b, t.b[j]);
     }
   };
   // one 8-byte store per plane: along k of a [row][k] tile for a K-contiguous operand, along the
@@ -211,12 +260,12 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 #pragma unroll
     for (int q = 0; q < P; ++q) *reinterpret_cast<bf16x4_t*>(&tiles[q][kc ? row * LDK + k : k * ld_mn + row]) = v[q];
   };
-  auto store_tile = [&](Tile& t, int64_t k0) {
+  auto store_tile = [&](Tile& t, int have) {     // (cleared from k-index `have` on)
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       int m, k;
       slot(tid + i * THREADS, A_KC, BM, m, k);
-      if (AHEAD > 0 && k0 + k >= kend) zero_raw<TA>(t.a[i]);
+      if (have < BK && k >= have) zero_raw<TA>(t.a[i]);
       bf16x4_t v[PA];
       to_planes<TA>(t.a[i], v);
       store4(As, std::integral_constant<int, PA>{}, A_KC, LDA, m, k, v);
@@ -225,7 +274,7 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
     for (int i = 0; i < NB; ++i) {
       int n, k;
       slot(tid + i * THREADS, B_KC, BN, n, k);
-      if (AHEAD > 0 && k0 + k >= kend) zero_raw<TB>(t.b[i]);
+      if (have < BK && k >= have) zero_raw<TB>(t.b[i]);
       bf16x4_t v[PB];
       to_planes<TB>(t.b[i], v);
       store4(Bs, std::integral_constant<int, PB>{}, B_KC, LDB, n, k, v);
@@ -249,34 +298,70 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
         }
     }
   };
+  auto use = [&](Tile& t, int have, auto next) {
+    store_tile(t, have);
+    __syncthreads();
+    next();
+    if constexpr (FLIGHT > 0) __builtin_amdgcn_sched_barrier(0);       // requested before the products, and the next tile not waited for before their end
+    multiply();
+    __syncthreads();
+    if constexpr (FLIGHT > 0) __builtin_amdgcn_sched_barrier(0);
+  };
+  auto nothing = [] {};
   if constexpr (AHEAD > 0) {
     Tile t[AHEAD];
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i) load_tile(t[i], kbeg + i * BK);
+    for (int i = 0; i < AHEAD; ++i)
+      request_clamped(t[i], i);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
-      if (kbeg + i * BK < kend) {
-        store_tile(t[i], kbeg + i * BK);
-        __syncthreads();
-        multiply();
-        __syncthreads();
-      }
-  } else {
+      if (i * BK < left) use(t[i], (int)left - i * BK, nothing);
+  } else if constexpr (FLIGHT <= 1) {
     Tile t;
-    if (kbeg < kend) load_tile(t, kbeg);
-    for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
-      store_tile(t, k0);
-      __syncthreads();
-      if (k0 + BK < kend) load_tile(t, k0 + BK);
-      multiply();
-      __syncthreads();
+    if (full > 0) {
+      request(t);
+      for (int j = 1; j < full; ++j) use(t, BK, [&] { request(t); });
+      use(t, BK, [&] { if (rest) request_rest(t, rest); });
+    } else if (rest) {
+      request_rest(t, rest);
+    }
+    if (rest) use(t, rest, nothing);
+  } else {
+    // two k-tiles in flight; the loop has one exit and nothing in it is conditional, so that it waits for the older tile's loads only
+    Tile t[2];
+    int j = 0;
+    if (full > 3) {
+      request(t[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      request(t[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      do {
+        use(t[0], BK, [&] { request(t[0]); });
+        use(t[1], BK, [&] { request(t[1]); });
+        j += 2;
+      } while (j + 3 < full);
+    } else {
+      if (full > 0) request(t[0]);
+      if (full > 1) request(t[1]);
+    }
+    if (full - j == 3) {
+      use(t[0], BK, [&] { request(t[0]); });
+      use(t[1], BK, nothing);
+      use(t[0], BK, nothing);
+    } else {
+      if (full - j >= 1) use(t[0], BK, nothing);
+      if (full - j >= 2) use(t[1], BK, nothing);
+    }
+    if (rest) {
+      request_rest(t[0], rest);
+      use(t[0], rest, nothing);
     }
   }
 }
 
 // output tile (bx, by) of split bz
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0>
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0, int FLIGHT = 2>
 __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int bx, int by, int bz) {
   constexpr int BM = 32 * WM, BN = 32 * WN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -286,7 +371,7 @@ __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_K
   const int64_t kbeg = (int64_t)bz * kchunk;
   const int64_t kend = kbeg + kchunk < p.K ? kbeg + kchunk : p.K;
   floatx16_t acc;
-  product<WM, WN, A_KC, B_KC, TA, TB, AHEAD>(p, lds, m0, n0, kbeg, kend, acc);
+  product<WM, WN, A_KC, B_KC, TA, TB, AHEAD, FLIGHT>(p, lds, m0, n0, kbeg, kend, acc);
 
   float* C = p.C + (p.splits > 1 ? (int64_t)bz * p.M * p.N : 0);
   const int64_t n = n0 + wn * 32 + (lane & 31);
@@ -303,10 +388,10 @@ __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_K
     }
   }
 }
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0>
-__global__ __launch_bounds__(64 * WM * WN) void kernel(const Params p) {
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0, int FLIGHT = in_flight<A_KC, B_KC, TA>()>
+__global__ __launch_bounds__(64 * WM * WN, 4) void kernel(const Params p) {
   __shared__ Lds<WM, WN, A_KC, B_KC, TA, TB> lds;
-  gemm_tile<WM, WN, A_KC, B_KC, TA, TB, AHEAD>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
+  gemm_tile<WM, WN, A_KC, B_KC, TA, TB, AHEAD, FLIGHT>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // The gradient of the region's input in one pass: out[t] = sum_k rows[inv_perm[t*K + k]] + d_logits[t] .
@@ -335,7 +420,7 @@ __device__ __forceinline__ void gather_tile(const Params& p, const GatherAdd& ga
   const int wm = wave / WN, wn = wave % WN;
   const int64_t m0 = (int64_t)by * BM, n0 = (int64_t)bx * BN;
   floatx16_t acc;
-  product<WM, WN, true, false, float, float>(p, *reinterpret_cast<Tiles*>(smem), m0, n0, 0, p.K, acc);
+  product<WM, WN, true, false, float, float, 0, 1>(p, *reinterpret_cast<Tiles*>(smem), m0, n0, 0, p.K, acc);
   float* const tile = reinterpret_cast<float*>(smem);       // (product ends with a barrier)
 #pragma unroll
   for (int v = 0; v < 16; ++v)
@@ -375,7 +460,7 @@ __device__ __forceinline__ void gather_tile(const Params& p, const GatherAdd& ga
   }
 }
 template <int WM, int WN, typename TG, bool STREAM>
-__global__ __launch_bounds__(64 * WM * WN) void gather_kernel(const Params p, const GatherAdd ga) {
+__global__ __launch_bounds__(64 * WM * WN, 4) void gather_kernel(const Params p, const GatherAdd ga) {
   __shared__ __attribute__((aligned(16))) char smem[GatherLds<WM, WN>::BYTES];
   gather_tile<WM, WN, TG, STREAM>(p, ga, smem, blockIdx.x, blockIdx.y);
 }

@@ -848,7 +848,7 @@ struct RouterGrads {
   int32_t accumulate;
 };
 template <typename TX, bool STREAM>
-__global__ __launch_bounds__(256) void router_grads_kernel(const RouterGrads p) {
+__global__ __launch_bounds__(256, 4) void router_grads_kernel(const RouterGrads p) {
   using namespace pk_x3mm;
   typedef Lds<2, 2, false, false, split3_t, TX> WLds;
   constexpr int GATHER = GatherLds<kGatherWM, kGatherWN>::BYTES, BYTES = (int)sizeof(WLds) > GATHER ? (int)sizeof(WLds) : GATHER;

@@ -456,3 +456,32 @@ def test_topk_with_the_sorts_histogram(dev, T, H, E, K, bias):
     many): the top-k writes the histograms of 16 tokens each that the sort places the slots by.  Partly filled last
     chunks, one and two experts a lane, more than 1,024 slots: bit for bit the separate calls."""
     test_norm_gate_topk_and_sort_in_one_call(dev, torch.bfloat16, T, H, E, K, bias)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("product", ["forward", "d_x", "weight gradient"])
+def test_router_products_at_every_end_of_their_k_loops(dev, dtype, product):
+    """No, one to seven whole k-tiles of 32 with and without a part of one behind them, two in flight at most; rows and
+    columns past the ends are read from the last ones.  A sum of n fp32-accurate products is within (n + 8) 2^-24 of the sum
+    of their magnitudes (every plane product left out is below 2^-24 of its product)."""
+    g = torch.Generator().manual_seed(31)
+    for n in (4, 28, 32, 36, 64, 68, 96, 100, 128, 132, 160, 164, 192, 196, 224, 228):
+        if product == "forward":             # more workgroups than are requested at once, one split
+            T, H, E = 64 * 260 + 1, n, 12
+        elif product == "d_x":
+            T, H, E = 129, 196, n
+        else:                                # 512 tiles: one split
+            T, H, E = n - n % 3, 2044, 1020
+        _note(f"{product} {dtype} T={T} H={H} E={E}")
+        x = torch.randn(T, H, generator=g).to(dtype)
+        w, d = torch.randn(E, H, generator=g) * 0.05, torch.randn(T, E, generator=g)
+        if product == "forward":
+            got, a, b = ops.gate_logits(x.to(dev), w.to(dev)), x.double(), w.double().t()
+        elif product == "d_x":
+            got, a, b = ops.gate_logits_bwd(d.to(dev), x.to(dev), w.to(dev)), d.double(), w.double()
+        else:
+            got = torch.empty(E, H, device=dev)
+            ops.gate_logits_bwd(d.to(dev), x.to(dev), w.to(dev), False, got)
+            a, b = d.double().t(), x.double()
+        bound = (a.shape[1] + 8) * 2.0**-24 * (a.abs() @ b.abs())
+        assert bool(((got.double().cpu() - a @ b).abs() <= bound).all()), (n, float(((got.double().cpu() - a @ b).abs() / bound).max()))
