@@ -124,6 +124,21 @@ def one_f_one_b(num_microbatches: int, ubids: Sequence[Any]) -> list[Task]:
     return tasks
 
 
+def plan_packs(tasks: Sequence[Task], lifetimes: dict, fuse_last_pack: bool) -> tuple[set, set]:
+    """Indices of the tasks whose gradients stay as they are for the optimizer step (with `fuse_last_pack` each bucket's last
+    ones), and of those whose pack an update has to wait for: the pack stream runs in order, so that is each bucket's last
+    pack in front of the update, and no other needs an event."""
+    reduces = [ti for ti, task in enumerate(tasks) if ti in lifetimes and lifetimes[ti].reduce_grads_after]
+    held = set({tasks[ti].ubid: ti for ti in reduces}.values()) if fuse_last_pack else set()
+    last, awaited = {}, set()
+    for ti, task in enumerate(tasks):
+        if task.type is TaskType.UPD:
+            awaited.update(last.values())
+        elif ti in lifetimes and lifetimes[ti].reduce_grads_after and ti not in held:
+            last[task.ubid] = ti
+    return held, awaited
+
+
 @dataclass
 class StageExecutor:
     stages: StageStore
@@ -150,11 +165,11 @@ class StageExecutor:
         caller = torch.cuda.current_stream()
         cs = self.compute_stream or caller
         ps = self.pack_stream or cs
-        # the microbatches (and whatever else the caller queued) were produced on the caller's stream
-        if cs != caller:
-            wait_stream(cs, caller)
-        if ps != caller and ps is not cs:
-            wait_stream(ps, caller)
+        # the microbatches (and whatever else the caller queued) were produced on the caller's stream.  The pack stream waits for
+        # it, and the compute stream, further down, for the pack stream: a wait is 10 to 17 us of host time.
+        first = cs if ps is cs else ps
+        if first != caller:
+            wait_stream(first, caller)
         self.params.drain_pending_frees()        # src/executors.py:584
         self._fwd.clear()
         self._inp_grads.clear()
@@ -168,11 +183,7 @@ class StageExecutor:
         ubids = list(self.stages.buckets.keys())
         # which task gathers / frees a bucket's parameters and which one packs its gradients
         lifetimes = plan_zero_lifetimes(tasks)
-        last_pack = {}          # bucket -> index of the task whose gradients are the last ones packed
-        if self.fuse_last_pack:
-            for ti, task in enumerate(tasks):
-                if ti in lifetimes and lifetimes[ti].reduce_grads_after:
-                    last_pack[task.ubid] = ti
+        held, awaited = plan_packs(tasks, lifetimes, self.fuse_last_pack)
         for ti, task in enumerate(tasks):
             tt = task.type
             life = lifetimes.get(ti)
@@ -227,7 +238,8 @@ class StageExecutor:
                 if split:
                     self._wgrad_queues[(task.ubid, task.mb)] = queue
                 if life.reduce_grads_after:
-                    self._pack_after_backward(task.ubid, cs, ps, pack_events, hold=last_pack.get(task.ubid) == ti)
+                    self._pack_after_backward(task.ubid, cs, ps, pack_events if ti in awaited else None,
+                                              hold=ti in held)
                 if life.free_params_after:
                     self._free_params_after(task.ubid, cs)
             elif tt is TaskType.BWD_W:
@@ -235,7 +247,8 @@ class StageExecutor:
                 with on_stream(cs):
                     queue.run()
                 if life.reduce_grads_after:
-                    self._pack_after_backward(task.ubid, cs, ps, pack_events, hold=last_pack.get(task.ubid) == ti)
+                    self._pack_after_backward(task.ubid, cs, ps, pack_events if ti in awaited else None,
+                                              hold=ti in held)
                 if life.free_params_after:
                     self._free_params_after(task.ubid, cs)
             elif tt is TaskType.UPD:
@@ -253,20 +266,21 @@ class StageExecutor:
         evt.record(cs)
         self.params.defer_free_full_params(ubid, evt)
 
-    def _pack_after_backward(self, ubid, cs, ps, pack_events: dict, hold: bool = False) -> None:
+    def _pack_after_backward(self, ubid, cs, ps, pack_events: dict | None, hold: bool = False) -> None:
         """Gradient pack on the second stream, ordered after the backward that produced the grads.
         hold: these are the bucket's last gradients of the iteration and the optimizer step, which
-        runs on the compute stream, takes them as they are."""
+        runs on the compute stream, takes them as they are.  pack_events: where the event of a pack that an update waits for goes."""
         if hold:
             self.params.hold_param_grads(ubid, cs)
             return
         if ps is not cs:
             wait_stream(ps, cs)
         self.params.accumulate_zero_param_grads_to_flat(ubid, ps)
-        if ps is not cs:
+        if ps is not cs and (pack_events is not None or ubid in self.stages.grad_sharded_ubids):
             done = torch.cuda.Event()
             done.record(ps)
-            pack_events[ubid] = done
+            if pack_events is not None:
+                pack_events[ubid] = done
             if ubid in self.stages.grad_sharded_ubids:
                 self.params.defer_free_full_grads(ubid, done)     # src/executors.py:719
 

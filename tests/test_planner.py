@@ -6,7 +6,7 @@ import random
 
 import pytest
 
-from piper_amd.executor import Task
+from piper_amd.executor import Task, plan_packs
 from piper_amd.planner import bucket_layers, plan_param_buckets, plan_zero_lifetimes
 from piper_amd.tasks import TaskType
 
@@ -229,3 +229,20 @@ def test_bucket_size_of_a_schedule_cuts_the_stage():
     for bad in (0, -3, "x"):
         with pytest.raises(ValueError):
             stage_bucket_bytes([sched[0], {"op": "replicate", "filter": {"PP": 0}, "devices": [0], "bucket_size": bad}])
+
+
+@pytest.mark.parametrize("fuse", [False, True])
+def test_an_update_waits_for_each_buckets_last_pack_in_front_of_it(fuse):
+    """Two buckets, five microbatches, an update after the third and one at the end.  With the last pack folded into the step
+    the one before it is the last that was packed (none here since the first update where the microbatch is the only one)."""
+    def iteration(mbs):
+        return [t for mb in mbs for t in (Task(TaskType.FWD, "a", mb), Task(TaskType.FWD, "b", mb), Task(TaskType.BWD, "b", mb),
+                                          Task(TaskType.BWD, "a", mb))]
+    for tail in ([3], [3, 4]):
+        tasks = iteration(range(3)) + [Task(TaskType.UPD)] + iteration(tail) + [Task(TaskType.UPD)]
+        held, awaited = plan_packs(tasks, plan_zero_lifetimes(tasks), fuse)
+        where = {(t.ubid, t.mb): i for i, t in enumerate(tasks) if t.type is TaskType.BWD}
+        packed = [mb for mb in [0, 1, 2] + tail if not (fuse and mb == tail[-1])]
+        assert held == ({where[u, tail[-1]] for u in "ab"} if fuse else set())
+        # each bucket's last pack in front of the first update, and its last pack of all
+        assert awaited == {where[u, mb] for u in "ab" for mb in (2, packed[-1])}
