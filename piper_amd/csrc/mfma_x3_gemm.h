@@ -114,10 +114,18 @@ __device__ __forceinline__ void fetch4(const typename Mem<T>::type* src, int64_t
     for (int q = 0; q < Planes<T>::N; ++q) out.v[q] = *reinterpret_cast<const bf16x4_t*>(src + q * plane_stride);
   }
 }
-template <typename T>
+template <typename T, bool PAIRS = true>
 __device__ __forceinline__ void to_planes(const Raw<T>& r, bf16x4_t (&out)[Planes<T>::N]) {
   constexpr int P = Planes<T>::N;
-  if constexpr (std::is_same<T, float>::value) {
+  if constexpr (std::is_same<T, float>::value && !PAIRS) {
+    bf16_t pl[4][P];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) split<P>(r.v[j], pl[j]);
+#pragma unroll
+    for (int q = 0; q < P; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) out[q][j] = pl[j][q];
+  } else if constexpr (std::is_same<T, float>::value) {
     // split(), two values to a conversion: the pair is also where the rounded values are taken from
     typedef float floatx2_t __attribute__((ext_vector_type(2)));
     typedef bf16_t bf16x2_t __attribute__((ext_vector_type(2)));
@@ -161,14 +169,13 @@ constexpr int in_flight() { return A_KC && !B_KC ? 0 : A_KC && std::is_same<TA, 
 // by one took 260.  The older of two k-tiles in flight is waited for by count, as nothing in the loop is conditional; without the
 // scheduling barriers the compiler puts the requests behind the products and converts the younger tile first.  Four waves a
 // SIMD (128 registers) matter more than a second k-tile.  us, before -> now, 128 experts 2048 wide unless said: forward 16,384 tokens
-// 53 -> 47, 4,096 19.2 -> 18.6, 509 (all requested at once) 12.7 -> 12.0, 8 experts, 16,384 37 -> 25; weight gradient 16,384 60 -> 56,
+// 53 -> 47, 4,096 19.2 -> 18.6, 8 experts, 16,384 37 -> 25; weight gradient 16,384 60 -> 56,
 // fp32, 64 experts 1024 wide, 4,000 15.0 -> 11.4; d_x 16,384 96 -> 85; the router's backward in one launch (router_grads_kernel)
 // 16,384 202 -> 189, 4,096 62 -> 58, 3,000 36 -> 33.
 // (Its weight gradient's tiles dealt out among those of the gather instead of in front of them: 190 -> 195 to 262.)
 //
 // acc of one wave: rows m0 + 32 wm .., columns n0 + 32 wn .. of the product over k in [kbeg, kend).
-// AHEAD > 0: the reduction has at most that many k-tiles, and all of them are requested at once.
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0, int FLIGHT = 2>
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int FLIGHT = 2>
 __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
                                         int64_t kend, floatx16_t& acc) {
   constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
@@ -236,23 +243,6 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
       fetch4<TB>(pb[i] - (B_KC ? back : back * p.sbk), p.plane_b, t.b[i]);
     }
   };
-  // k-tile i of a reduction that is requested as a whole: past its end from its last elements
-  auto request_clamped = [&](Tile& t, int i) {
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      int m, k;
-      slot(tid + j * THREADS, A_KC, BM, m, k);
-      const int64_t go = min((int64_t)(k + i * BK), left - (A_KC ? 4 : 1)) - k;
-      fetch4<TA>(pa[j] + (A_KC ? go : go * p.sak), p.plane_a, t.a[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      int n, k;
-      slot(tid + j * THREADS, B_KC, BN, n, k);
-      const int64_t go = min((int64_t)(k + i * BK), left - (B_KC ? 4 : 1)) - k;
-      fetch4<TB>(pb[j] + (B_KC ? go : go * p.sbk), p.plane_b, t.b[j]);
-    }
-  };
   // one 8-byte store per plane: along k of a [row][k] tile for a K-contiguous operand, along the
   // rows of a [k][row] tile otherwise
   auto store4 = [](auto& tiles, auto nplanes, bool kc, int ld_mn, int row, int k, const auto& v) {
@@ -308,16 +298,7 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
     if constexpr (FLIGHT > 0) __builtin_amdgcn_sched_barrier(0);
   };
   auto nothing = [] {};
-  if constexpr (AHEAD > 0) {
-    Tile t[AHEAD];
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i)
-      request_clamped(t[i], i);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i)
-      if (i * BK < left) use(t[i], (int)left - i * BK, nothing);
-  } else if constexpr (FLIGHT <= 1) {
+  if constexpr (FLIGHT <= 1) {
     Tile t;
     if (full > 0) {
       request(t);
@@ -360,6 +341,99 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
   }
 }
 
+// The same of a reduction of at most AHEAD k-tiles along both operands' contiguous index, all of them requested at once.  Its loads,
+// masks and splits are formed one by one: with those of product() it takes a microsecond more (us, 128 experts 2048 wide, 509
+// tokens 9.7 -> 10.7, 1,777 12.0 -> 13.1, fp32 1024 wide, 1,000 7.8 -> 9.1), as a workgroup alone on its CU has nothing to do meanwhile.
+template <int WM, int WN, typename TA, typename TB, int AHEAD>
+__device__ __forceinline__ void product_at_once(const Params& p, Lds<WM, WN, true, true, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
+                                                int64_t kend, floatx16_t& acc) {
+  constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
+  constexpr int PA = Planes<TA>::N, PB = Planes<TB>::N;
+  auto& As = lds.As;
+  auto& Bs = lds.Bs;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  typedef typename Mem<TA>::type MA;
+  typedef typename Mem<TB>::type MB;
+  const MA* A = reinterpret_cast<const MA*>(p.A);
+  const MB* B = reinterpret_cast<const MB*>(p.B);
+
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+
+  constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
+  struct Tile { Raw<TA> a[NA]; Raw<TB> b[NB]; };
+  auto slot = [](int idx, int& row, int& k) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); };
+  // (past the ends from the last elements, as a branch would hold up the loads behind it; what lies past kend is cleared when it
+  // goes to LDS)
+  auto load_tile = [&](Tile& t, int64_t k0) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      int m, k;
+      slot(tid + i * THREADS, m, k);
+      fetch4<TA>(A + min(m0 + m, p.M - 1) * p.sam + min(k0 + k, kend - 4) * p.sak, p.plane_a, t.a[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      int n, k;
+      slot(tid + i * THREADS, n, k);
+      fetch4<TB>(B + min(k0 + k, kend - 4) * p.sbk + min(n0 + n, p.N - 1) * p.sbn, p.plane_b, t.b[i]);
+    }
+  };
+  auto store_tile = [&](Tile& t, int64_t k0) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      int m, k;
+      slot(tid + i * THREADS, m, k);
+      if (k0 + k >= kend) zero_raw<TA>(t.a[i]);
+      bf16x4_t v[PA];
+      to_planes<TA, false>(t.a[i], v);
+#pragma unroll
+      for (int q = 0; q < PA; ++q) *reinterpret_cast<bf16x4_t*>(&As[q][m * LDK + k]) = v[q];
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      int n, k;
+      slot(tid + i * THREADS, n, k);
+      if (k0 + k >= kend) zero_raw<TB>(t.b[i]);
+      bf16x4_t v[PB];
+      to_planes<TB, false>(t.b[i], v);
+#pragma unroll
+      for (int q = 0; q < PB; ++q) *reinterpret_cast<bf16x4_t*>(&Bs[q][n * LDK + k]) = v[q];
+    }
+  };
+  auto multiply = [&]() {
+#pragma unroll
+    for (int kk = 0; kk < BK; kk += 16) {
+      bf16x8_t a[PA], b[PB];
+#pragma unroll
+      for (int pl = 0; pl < PA; ++pl) a[pl] = frag_kc(As[pl], wm * 32, kk, lane);
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl) b[pl] = frag_kc(Bs[pl], wn * 32, kk, lane);
+      // small terms first
+#pragma unroll
+      for (int s = PA + PB - 2; s >= 0; --s)
+#pragma unroll
+        for (int pa = 0; pa < PA; ++pa) {
+          const int pb = s - pa;
+          if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa], b[pb], acc, 0, 0, 0);
+        }
+    }
+  };
+  Tile t[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) load_tile(t[i], kbeg + i * BK);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    if (kbeg + i * BK < kend) {
+      store_tile(t[i], kbeg + i * BK);
+      __syncthreads();
+      multiply();
+      __syncthreads();
+    }
+}
+
 // output tile (bx, by) of split bz
 template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0, int FLIGHT = 2>
 __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int bx, int by, int bz) {
@@ -371,7 +445,8 @@ __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_K
   const int64_t kbeg = (int64_t)bz * kchunk;
   const int64_t kend = kbeg + kchunk < p.K ? kbeg + kchunk : p.K;
   floatx16_t acc;
-  product<WM, WN, A_KC, B_KC, TA, TB, AHEAD, FLIGHT>(p, lds, m0, n0, kbeg, kend, acc);
+  if constexpr (AHEAD > 0) product_at_once<WM, WN, TA, TB, AHEAD>(p, lds, m0, n0, kbeg, kend, acc);
+  else product<WM, WN, A_KC, B_KC, TA, TB, FLIGHT>(p, lds, m0, n0, kbeg, kend, acc);
 
   float* C = p.C + (p.splits > 1 ? (int64_t)bz * p.M * p.N : 0);
   const int64_t n = n0 + wn * 32 + (lane & 31);
@@ -388,10 +463,15 @@ __device__ __forceinline__ void gemm_tile(const Params& p, Lds<WM, WN, A_KC, B_K
     }
   }
 }
-template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int AHEAD = 0, int FLIGHT = in_flight<A_KC, B_KC, TA>()>
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
 __global__ __launch_bounds__(64 * WM * WN, 4) void kernel(const Params p) {
   __shared__ Lds<WM, WN, A_KC, B_KC, TA, TB> lds;
-  gemm_tile<WM, WN, A_KC, B_KC, TA, TB, AHEAD, FLIGHT>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
+  gemm_tile<WM, WN, A_KC, B_KC, TA, TB, 0, in_flight<A_KC, B_KC, TA>()>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+template <int WM, int WN, typename TA, typename TB, int AHEAD>
+__global__ __launch_bounds__(64 * WM * WN) void at_once_kernel(const Params p) {
+  __shared__ Lds<WM, WN, true, true, TA, TB> lds;
+  gemm_tile<WM, WN, true, true, TA, TB, AHEAD>(p, lds, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // The gradient of the region's input in one pass: out[t] = sum_k rows[inv_perm[t*K + k]] + d_logits[t] .
@@ -420,7 +500,7 @@ __device__ __forceinline__ void gather_tile(const Params& p, const GatherAdd& ga
   const int wm = wave / WN, wn = wave % WN;
   const int64_t m0 = (int64_t)by * BM, n0 = (int64_t)bx * BN;
   floatx16_t acc;
-  product<WM, WN, true, false, float, float, 0, 1>(p, *reinterpret_cast<Tiles*>(smem), m0, n0, 0, p.K, acc);
+  product<WM, WN, true, false, float, float, 1>(p, *reinterpret_cast<Tiles*>(smem), m0, n0, 0, p.K, acc);
   float* const tile = reinterpret_cast<float*>(smem);       // (product ends with a barrier)
 #pragma unroll
   for (int v = 0; v < 16; ++v)
@@ -494,8 +574,8 @@ inline int launch(const Params& p, int kernel_id, hipStream_t s) {
   if constexpr (A_KC && B_KC) {
     const int64_t k_tiles = pk_ceil_div(pk_ceil_div(p.K, p.splits), BK);
     if ((int64_t)grid.x * grid.y * grid.z <= 256 && k_tiles <= 8) {
-      if (k_tiles <= 4) PK_LAUNCH_NOCHECK(kernel_id, s, (kernel<WM, WN, A_KC, B_KC, TA, TB, 4>), grid, dim3(64 * WM * WN), 0, s, p);
-      else PK_LAUNCH_NOCHECK(kernel_id, s, (kernel<WM, WN, A_KC, B_KC, TA, TB, 8>), grid, dim3(64 * WM * WN), 0, s, p);
+      if (k_tiles <= 4) PK_LAUNCH_NOCHECK(kernel_id, s, (at_once_kernel<WM, WN, TA, TB, 4>), grid, dim3(64 * WM * WN), 0, s, p);
+      else PK_LAUNCH_NOCHECK(kernel_id, s, (at_once_kernel<WM, WN, TA, TB, 8>), grid, dim3(64 * WM * WN), 0, s, p);
       PK_RETURN_IF_LAUNCH_FAILED();
       return PK_OK;
     }
