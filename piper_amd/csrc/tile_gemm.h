@@ -1,8 +1,8 @@
 // Grouped GEMMs on the matrix cores for what the 256-wide bf16 kernels of grouped_gemm.hip do not
 // take or are too coarse for: fp32 operands (v_mfma_f32_32x32x2_f32: exact fp32 products and sums), bf16
 // widths that are no multiple of 128 (256 for weight gradients), and products with few tiles.  Every row
-// only has to be a whole number of 16-byte pieces (4 fp32 or 8 bf16 elements); row, column and reduction
-// remainders are fetched as zeros and masked on store.
+// only has to be a whole number of 16-byte pieces (4 fp32 or 8 bf16 elements); rows and columns past the ends are read from a
+// tile's first ones and never stored, reduction remainders are cleared on their way into LDS.
 //
 //   ragged M: C[rows_e, N] = sum_seg A_seg[rows_e, K] . B_seg[e]     (forward, input gradient)
 //   ragged K: C[e][M, N] (+)= A[rows_e, M]^T . B[rows_e, N]           (weight gradient)
@@ -16,7 +16,7 @@
 // the chip, several groups of waves share a tile's reduction.
 //
 // What the k-loops wait for.  No load stands behind a branch (addresses are clamped, the last k-tile is masked on its way into
-// LDS), the loop has one way out, and the k-tiles past the last whole round have code of their own: then the compiler knows how
+// LDS), the loop has one way out, and the k-tiles behind it have code of their own: then the compiler knows how
 // many loads are younger than the ones it needs.  With the loads behind masks it waited for all of them (vmcnt(0)) in every
 // second or third k-tile, so that nothing was in flight across it; three workgroups on a CU hid most of that in the ragged-M
 // products, but not in the weight gradients, whose reductions are short.  Measured, caches cold, us, before -> now:
@@ -169,6 +169,45 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
+// The k-loop of a tile: fetch(set) requests the k-tile of that number into the register set of that number, step(set, kt, more)
+// multiplies k-tile kt out of it and, with `more`, requests k-tile kt + DEPTH into it.  Exactly the k-tiles that are there are
+// requested: an expert with one or two of them is bound by the memory's answer to these.  The loop has nothing to skip and one way
+// out, and whatever leads to a step has requested the same number of tiles behind its own: the compiler's counts depend on both.
+// us, one loop that always requests DEPTH tiles more -> this, caches cold: weight gradients 24 experts 1000 x 360, 8 rows 28.4 ->
+// 26.1 (rows not gathered 26.5 -> 25.0), 32 rows 28.8 -> 27.1, 172 rows 42.2 -> 40.2; 32 experts 1000 x 512, uneven rows not gathered,
+// 8 38.7 -> 34.6, 64 49.1 -> 47.0; fp32 32 experts 1024 x 512, 16 rows 73.7 -> 70.2; 24 experts 1000 x 360, 96 rows 88.1 -> 84.7.  bf16 in
+// 64 x 64 tiles: d_x 24 experts 1000 x 360, 8 rows 19.8 -> 18.9, 96 rows 26.6 -> 25.6; gate/up 172 rows 37.6 -> 35.8; d_h 32 experts
+// 1000 x 512, 24 uneven rows 24.4 -> 23.4.  The launch bounds keep the waves on a SIMD: without them the 128 x 128 weight gradients
+// have one (36 us at the first of these sizes).
+template <typename Fetch, typename Step>
+__device__ __forceinline__ void run_k_tiles(int n, Fetch&& fetch, Step&& step) {
+  static_assert(DEPTH == 2, "the rounds below");
+  constexpr std::integral_constant<int, 0> s0{};
+  constexpr std::integral_constant<int, 1> s1{};
+  if (n > 1) {
+    fetch(s0);
+    __builtin_amdgcn_sched_barrier(0);         // in this order
+    fetch(s1);
+    __builtin_amdgcn_sched_barrier(0);
+    int kt = 0;
+    for (; kt + 3 < n; kt += 2) {
+      step(s0, kt, true);
+      step(s1, kt + 1, true);
+    }
+    if (kt + 3 == n) {
+      step(s0, kt, true);
+      step(s1, kt + 1, false);
+      step(s0, kt + 2, false);
+    } else {
+      step(s0, kt, false);
+      step(s1, kt + 1, false);
+    }
+  } else if (n == 1) {
+    fetch(s0);
+    step(s0, 0, false);
+  }
+}
+
 // acc of group 0 += acc of the other groups, in group order (every thread of the workgroup calls it).
 template <int KS, int TILES, int THREADS>
 __device__ __forceinline__ void add_groups(floatx16_t* acc, float* lds, int group, int tid) {
@@ -239,11 +278,13 @@ __device__ __forceinline__ int unit_of_block(int b) {
 // tile's columns, whose total is the score's gradient.  d_h never leaves the workgroup.
 enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
 template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI>
-__global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const RaggedM p) {
+__global__ __launch_bounds__(64 * WM * WN * KS, sizeof(T) == 4 || KS > 1 || TM * TN > 1 ? 1 : EPI == GATE_UP ? 3 : 4) void ragged_m_kernel(const RaggedM p) {
   constexpr int THREADS = 64 * WM * WN;       // of a group: WM x WN waves of TM x TN MFMA tiles
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr bool DUAL = EPI == GATE_UP;
   constexpr int NB = DUAL ? 2 : 1;
+  // run_k_tiles in bf16 with 64 x 64 tiles; the longer code costs the others registers, and with them a workgroup on a CU or spills
+  constexpr bool EXACT = sizeof(T) == 2 && TM * TN == 1;
   constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, STAGE = A_BYTES + NB * B_BYTES;
   static_assert(!DUAL || B_KC, "gate and up weights are K-contiguous");
@@ -369,7 +410,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
   const int mine = (nkt + KS - 1) / KS;      // k-tiles of a group (past the last one: zeros)
   // DEPTH of the group's k-tiles are in flight, each in a register set of its own
   auto step = [&](auto d_c, int kt, bool more) {
-    char* const st = smem + (kt & 1) * STAGE;
+    char* const st = smem + (EXACT ? decltype(d_c)::value : kt & 1) * STAGE;
     deposit(d_c, kt * KS + group, st);
     __syncthreads();
     if (more) fetch(d_c, (kt + DEPTH) * KS + group);
@@ -399,7 +440,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void ragged_m_kernel(const Ragge
       }
     }
   };
-  if (mine > 0) {
+  if constexpr (EXACT) {
+    run_k_tiles(mine, [&](auto d) { fetch(d, d * KS + group); }, step);
+  } else if (mine > 0) {
     static_for<DEPTH>([&](auto d) {
       fetch(d, d * KS + group);
       __builtin_amdgcn_sched_barrier(0);       // in this order: the counts of loads in flight depend on it
@@ -595,7 +638,7 @@ struct RaggedK {
 
 // TILE: 64-wide (1) or 128-wide (2) tiles.  MAPPED: some operand's rows are gathered.
 template <typename T, int TILE, int KS, bool MAPPED>
-__global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
+__global__ __launch_bounds__(256 * KS, TILE == 2 ? 2 : 4) void ragged_k_kernel(const RaggedK p) {
   constexpr int THREADS = 256;
   constexpr int TM = TILE, TN = TILE, BM = 64 * TILE, BN = BM, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr int L = BM * 8 / THREADS;
@@ -694,14 +737,8 @@ __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
   if (nkt > 0) {
-    if constexpr (MAPPED) static_for<DEPTH>([&](auto d) { lookup(d, d * KS + group); });
-    __builtin_amdgcn_sched_barrier(0);
-    static_for<DEPTH>([&](auto d) {
-      fetch(d, d * KS + group);
-      __builtin_amdgcn_sched_barrier(0);       // in this order, as in ragged_m_kernel
-    });
     auto step = [&](auto d_c, int kt, bool more) {
-      char* const st = smem + (kt & 1) * STAGE;
+      char* const st = smem + decltype(d_c)::value * STAGE;
       deposit(d_c, kt * KS + group, st);
       __syncthreads();
       if (more) fetch(d_c, (kt + DEPTH) * KS + group);
@@ -722,10 +759,9 @@ __global__ __launch_bounds__(256 * KS) void ragged_k_kernel(const RaggedK p) {
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    int kt = 0;
-    for (; kt + DEPTH <= mine; kt += DEPTH)
-      static_for<DEPTH>([&](auto d) { step(d, kt + d, true); });
-    static_for<DEPTH - 1>([&](auto d) { if (kt + d < mine) step(d, kt + d, false); });
+    if constexpr (MAPPED) static_for<DEPTH>([&](auto d) { lookup(d, d * KS + group); });
+    __builtin_amdgcn_sched_barrier(0);
+    run_k_tiles(mine, [&](auto d) { fetch(d, d * KS + group); }, step);
     if constexpr (KS > 1) {
       add_groups<KS, TM * TN, THREADS>(reinterpret_cast<floatx16_t*>(&acc), reinterpret_cast<float*>(smem_), group, tid);
     }

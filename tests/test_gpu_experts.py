@@ -975,3 +975,74 @@ def test_units_of_160_rows(dev, mapped, skew):
         assert ((he - want).abs() <= want.abs() * (2**-8 + 2**-18) + 1e-30).all(), ("h", e, n)
         check(y[r], [(he, w2[e].double().T)], ("y", e, n))
         check(dx[r], [(ge, w1[e].double()), (ue, w3[e].double())], ("d_x", e, n))
+
+
+# Tile kernels request the k-tiles that are there and no others: reductions of none, one to nine k-tiles for a group of waves, a part of
+# one at their ends.  Widths whose tiles are 64 wide with four, two and one such groups, and 128 wide.
+K_LOOP_CASES = [(104, 72, 4), (200, 104, 2), (584, 264, 1), (1000, 512, 1)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,I,groups", K_LOOP_CASES)
+@pytest.mark.parametrize("mapped", [True, False])
+def test_weight_gradients_at_every_end_of_their_k_loops(dev, dtype, H, I, groups, mapped):
+    print(f"[case] k-loop ends, weight gradients {dtype} H={H} I={I} groups={groups} mapped={mapped}", flush=True)
+    bk = (64 if dtype == torch.bfloat16 else 32) * groups
+    counts = [max(0, n * bk + off) for n, off in zip([0, 1, 1, 2, 2, 3, 4, 5, 6, 7, 8, 9, 9], [0, -bk + 1, 0, 0, -3, 0, 5, -1, 0, 1, 0, -7, 0])]
+    E, A, K = len(counts), sum(counts), 2 if mapped else 1
+    gen = torch.Generator(device=dev).manual_seed(H + I + bk)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device=dev).to(dtype)
+    T = -(-A // K)
+    perm = torch.randperm(T * K, generator=gen, device=dev)[:A].int()
+    x, dy, hs, dg, du = rand(T, H), rand(T, H), rand(A, I), rand(A, I), rand(A, I)
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    kw = dict(row_map=perm, row_map_div=K, scaled=True) if mapped else {}
+    got = [torch.full(s, float("nan"), dtype=dtype, device=dev) for s in ((E, I, H), (E, H, I), (E, I, H))]
+    ops.grouped_swiglu_wgrad(dy, hs, dg, du, x, starts, E, d_w1=got[0], d_w2=got[1], d_w3=got[2], **kw)
+    rows = (perm // K).long() if mapped else torch.arange(A, device=dev)
+    ulp = 2**-8 if dtype == torch.bfloat16 else 2**-24
+    first = 0
+    for e, n in enumerate(counts):
+        r = slice(first, first + n)
+        first += n
+        xe, dye = x[rows[r]].double(), dy[rows[r]].double()
+        for g, a, b in zip(got, (dg[r].double(), dye, du[r].double()), (xe, hs[r].double(), xe)):
+            want, size = a.T @ b, a.abs().T @ b.abs()
+            assert ((g[e].double() - want).abs() <= want.abs() * ulp + size * (n + 1) * 2**-23).all(), (e, n)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("many", [True, False])
+def test_tile_products_at_every_end_of_their_k_loops(dev, dtype, many):
+    """Gate/up over H, down and d_x over I (d_x twice as long).  many: enough tiles that nobody shares a reduction."""
+    bk = 64 if dtype == torch.bfloat16 else 32
+    counts = [0, 1, 63, 64, 65, 130] * (10 if many else 1)
+    E, A = len(counts), sum(counts)
+    gen = torch.Generator(device=dev).manual_seed(bk + many)
+    rand = lambda *shape, scale=1.0: (torch.randn(shape, generator=gen, device=dev) * scale).to(dtype)
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    ulp = 2**-8 if dtype == torch.bfloat16 else 2**-24
+
+    def check(got, pairs, what):
+        want = sum(a @ b for a, b in pairs)
+        size, k = sum(a.abs() @ b.abs() for a, b in pairs), sum(a.shape[1] for a, _ in pairs)
+        assert ((got.double() - want).abs() <= want.abs() * ulp + size * (k + 1) * 2**-23).all(), what
+
+    for n in range(1, 10):
+        for k in (n * bk - 24, n * bk):
+            for H, I in ((k, 392), (392, k)):
+                print(f"[case] k-loop ends {dtype} H={H} I={I} E={E}", flush=True)
+                x, w1, w3, w2 = rand(A, H), rand(E, I, H, scale=0.05), rand(E, I, H, scale=0.05), rand(E, H, I, scale=0.05)
+                y, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts)
+                dx = ops.grouped_swiglu_dgrad_dx(g, u, w1, w3, starts)
+                first = 0
+                for e in range(E):
+                    r = slice(first, first + counts[e])
+                    first += counts[e]
+                    if e >= 6 and e + 6 < E:           # the pattern repeats
+                        continue
+                    xe, ge, ue = x[r].double(), g[r].double(), u[r].double()
+                    check(g[r], [(xe, w1[e].double().T)], ("g", e))
+                    check(u[r], [(xe, w3[e].double().T)], ("u", e))
+                    check(y[r], [(h[r].double(), w2[e].double().T)], ("y", e))
+                    check(dx[r], [(ge, w1[e].double()), (ue, w3[e].double())], ("d_x", e))
