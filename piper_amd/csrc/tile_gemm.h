@@ -277,8 +277,17 @@ __device__ __forceinline__ int unit_of_block(int b) {
 // d_g and d_u from score * d_h, score * h for the weight gradient, and the row sums of d_h * h over a
 // tile's columns, whose total is the score's gradient.  d_h never leaves the workgroup.
 enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
-template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI>
-__global__ __launch_bounds__(64 * WM * WN * KS, sizeof(T) == 4 || KS > 1 || TM * TN > 1 ? 1 : EPI == GATE_UP ? 3 : 4) void ragged_m_kernel(const RaggedM p) {
+// SPARSE (fp32): at least half of a tile's rows are not there, about.  They are left out of the loads, which then stand behind
+// branches: the compiler still knows of the weights' loads behind them.  Read from the tile's first row instead, as everywhere else,
+// they take up the path to the registers and a long fp32 reduction with few rows is 5 to 17 % slower (us, all rows read -> this: 24
+// experts 1000 x 360, 8 rows: gate/up 49.0 -> 45.4, d_h 26.2 -> 25.1, d_x 34.2 -> 33.3; 32 experts 1024 x 512, 16 rows, d_x 59.8 -> 53.7; 64 experts
+// 896 x 384, 16 rows, gate/up 83.7 -> 81.3, d_x 81.3 -> 78.2).  With more rows the branches cost as much (24 experts 1000 x 360, 48 rows,
+// gate/up 51.4 -> 54.7; 128 experts 512 x 128, 48 uneven rows, d_x 41.9 -> 48.6), with fewer than twelve k-tiles there is little to
+// gain (128 experts 512 x 128, 32 rows, down 20.0 -> 21.1); the 32 x 32 tiles gain in d_h alone (24 experts 1000 x 360, 8 rows
+// 26.0 -> 25.1; 16 experts 408 x 472, 16 rows, d_x 19.8 -> 20.6).
+template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI, bool SPARSE>
+__global__ __launch_bounds__(64 * WM * WN * KS, (sizeof(T) == 4 && !SPARSE) || WM * WN < 4 || KS > 1 || TM * TN > 1 ? 1 : EPI == GATE_UP ? 3 : 4)
+void ragged_m_kernel(const RaggedM p) {
   constexpr int THREADS = 64 * WM * WN;       // of a group: WM x WN waves of TM x TN MFMA tiles
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, BK = kBK<T>, PIECE = kPiece<T>;
   constexpr bool DUAL = EPI == GATE_UP;
@@ -342,6 +351,12 @@ __global__ __launch_bounds__(64 * WM * WN * KS, sizeof(T) == 4 || KS > 1 || TM *
   // k-tile kt into register set d: what lies past K, or past the last tile, is read from the start of the
   // reduction and masked by deposit()
   u32x4_t ra_[DEPTH][LA], rb_[DEPTH][NB][LB];
+  if constexpr (SPARSE) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+#pragma unroll
+      for (int i = 0; i < LA; ++i) ra_[d][i] = u32x4_t{0u, 0u, 0u, 0u};
+  }
   auto fetch = [&](auto d_c, int kt) {
     auto& ra = ra_[decltype(d_c)::value];
     auto& rb = rb_[decltype(d_c)::value];
@@ -351,7 +366,8 @@ __global__ __launch_bounds__(64 * WM * WN * KS, sizeof(T) == 4 || KS > 1 || TM *
     const int64_t sa = second ? seg_a : 0, sb = second ? seg_b : 0;
     const int ka = k0 + a_kofs < p.K ? k0 : -a_kofs;
 #pragma unroll
-    for (int i = 0; i < LA; ++i) ra[i] = *reinterpret_cast<const u32x4_t*>(a_ptr[i] + (sa + ka));
+    for (int i = 0; i < LA; ++i)
+      if (!SPARSE || ((tid + i * THREADS) >> 3) < rows) ra[i] = *reinterpret_cast<const u32x4_t*>(a_ptr[i] + (sa + ka));
 #pragma unroll
     for (int q = 0; q < NB; ++q)
 #pragma unroll
@@ -544,7 +560,11 @@ inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id
   if (units > 0x7fffff00ll) return PK_ERR_SHAPE;
   if (part_cols) *part_cols = BN;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(64 * WM * WN * KS);
-  PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, KS, B_KC, EPI>), grid, block, 0, s, p);
+  constexpr bool MAY_BE_SPARSE = sizeof(T) == 4 && (WM * WN > 1 || EPI != PLAIN);
+  if (MAY_BE_SPARSE && 2 * A_rows <= BM * (A_rows < p.E ? A_rows : p.E) && pk_ceil_div(p.K, kBK<T>) * p.nseg >= 12)
+    PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, KS, B_KC, EPI, MAY_BE_SPARSE>), grid, block, 0, s, p);
+  else
+    PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, KS, B_KC, EPI, false>), grid, block, 0, s, p);
   PK_RETURN_IF_LAUNCH_FAILED();
   return PK_OK;
 }

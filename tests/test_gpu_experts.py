@@ -1046,3 +1046,60 @@ def test_tile_products_at_every_end_of_their_k_loops(dev, dtype, many):
                     check(u[r], [(xe, w3[e].double().T)], ("u", e))
                     check(y[r], [(h[r].double(), w2[e].double().T)], ("y", e))
                     check(dx[r], [(ge, w1[e].double()), (ue, w3[e].double())], ("d_x", e))
+
+
+# fp32 products whose tiles are mostly padding: their loads leave out the rows that are not there.  From one row an expert to half a
+# tile on average with some tiles full, in the tiles that few and many of them are cut into.
+SPARSE_CASES = [
+    ([1, 2, 0, 5], 456, 392),                        # 32 x 32, four groups
+    ([8] * 24, 1000, 392),                           # 64 x 32
+    ([16] * 16, 512, 400),                           # 32 x 64
+    ([0, 130, 1, 31, 2, 20, 33, 5] * 4, 1000, 520),  # 64 x 64
+    ([32, 64, 1, 7] * 16, 904, 424),
+]
+
+
+@pytest.mark.parametrize("counts,H,I", SPARSE_CASES)
+def test_fp32_products_with_mostly_empty_tiles(dev, counts, H, I):
+    print(f"[case] mostly empty tiles counts={counts[:8]}x{len(counts)} H={H} I={I}", flush=True)
+    E, A, K = len(counts), sum(counts) - sum(counts) % 2, 2
+    counts = counts[:-1] + [counts[-1] - (sum(counts) - A)]
+    gen = torch.Generator(device=dev).manual_seed(E + H)
+    rand = lambda *shape, scale=1.0: torch.randn(shape, generator=gen, device=dev) * scale
+    x, dy, w1, w3, w2 = rand(A // K, H), rand(A // K, H), rand(E, I, H, scale=0.05), rand(E, I, H, scale=0.05), rand(E, H, I, scale=0.05)
+    perm = torch.randperm(A, generator=gen, device=dev).int()
+    scores = torch.rand((A // K, K), generator=gen, device=dev) + 0.1
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    y, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts, row_map=perm, row_map_div=K, num_rows=A)
+    dg, du, hs, ds = ops.grouped_swiglu_dgrad_dh_scaled(dy, perm, scores, w2, g, u, starts)
+    dx = ops.grouped_swiglu_dgrad_dx(g, u, w1, w3, starts)
+    rows = (perm // K).long()
+
+    def check(got, pairs, what):
+        want = sum(a @ b for a, b in pairs)
+        size, k = sum(a.abs() @ b.abs() for a, b in pairs), sum(a.shape[1] for a, _ in pairs)
+        assert ((got.double() - want).abs() <= size * (k + 2) * 2**-23).all(), what
+
+    first = 0
+    for e, n in enumerate(counts):
+        r = slice(first, first + n)
+        first += n
+        xe, ge, ue, dye = x[rows[r]].double(), g[r].double(), u[r].double(), dy[rows[r]].double()
+        sc = scores.flatten()[perm[r].long()].double()
+        check(g[r], [(xe, w1[e].double().T)], ("g", e))
+        check(u[r], [(xe, w3[e].double().T)], ("u", e))
+        check(y[r], [(h[r].double(), w2[e].double().T)], ("y", e))
+        check(dx[r], [(ge, w1[e].double()), (ue, w3[e].double())], ("d_x", e))
+        # d_u = score * d_h * silu(g): the product's bound times the factor, and a few roundings of the factor itself
+        dh, size = dye @ w2[e].double(), dye.abs() @ w2[e].double().abs()
+        f = sc[:, None] * torch.nn.functional.silu(ge)
+        assert ((du[r].double() - dh * f).abs() <= (size * (H + 2) * 2**-23 + dh.abs() * 2**-20) * f.abs() + 1e-30).all(), ("d_u", e)
+        sg = torch.sigmoid(ge)
+        f = sc[:, None] * ue * (sg * (1 + ge * (1 - sg)))
+        # (1 + g (1 - sigmoid)) can cancel: its own rounding is relative to its terms
+        terms = sc[:, None] * ue.abs() * sg * (1 + ge.abs())
+        assert ((dg[r].double() - dh * f).abs() <= size * (H + 2) * 2**-23 * f.abs() + dh.abs() * terms * 2**-20 + 1e-30).all(), ("d_g", e)
+        hv = torch.nn.functional.silu(ge) * ue
+        assert ((hs[r].double() - sc[:, None] * hv).abs() <= sc[:, None] * hv.abs() * 2**-20 + 1e-30).all(), ("score * h", e)
+        bound = (size * hv.abs()).sum(1) * (H + I) * 2**-22
+        assert ((ds.flatten()[perm[r].long()].double() - (dh * hv).sum(1)).abs() <= bound + 1e-30).all(), ("d_score", e)
