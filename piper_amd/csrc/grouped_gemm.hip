@@ -1536,6 +1536,7 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
   constexpr int L = A_BYTES / (NTHREADS * 16);        // loads of a wave for a k-tile, per operand
   constexpr int STORES = 4 * TM;                      // stores of a wave for a tile
   using St = Stage32<WTN>;
+  static_assert(64 * 8 == 2 * BM, "a piece is two rows");
   static_assert(BM == BN, "both operands' pieces lie alike");
   static_assert(WMW * WNW * St::BYTES <= STAGE, "the output is staged in one stage");
   __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
@@ -1589,17 +1590,21 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
     return;
   }
 
-  // The lanes' pieces of a k-tile, in both operands alike, and the row map entries of the k-tile that is fetched next: they are
-  // requested one fetch ahead, in front of the loads of that fetch, so the wait for these covers them.
-  int krow[L], col[L], entry[L];
+  // The lanes' pieces of a k-tile, in both operands alike, and the row map entries of the wave's rows of the k-tile that is fetched
+  // next, requested one fetch ahead.  They take the scalar path: of vector loads the compiler waits for by its own count, in which the
+  // ring's loads do not appear, so every fetch began with a wait for the one before it and for a finished tile's stores (us, gathered
+  // rows: 128 experts 2048 x 768, 64 rows 253 -> 247, 64 uneven rows 288 -> 276, 128 uneven rows 401 -> 383; 64 experts 1536 x 768, 64 rows
+  // 111.7 -> 110.5; one k-tile an expert within noise).
+  constexpr int RPI = 64 * 8 / BM;                    // rows of a piece
+  int krow[L], col[L], entry[L * RPI];
 #pragma unroll
   for (int i = 0; i < L; ++i) mn_slot<BM>(wave * L + i, lane, krow[i], col[i]);
   auto lookup = [&](int kt) {
     if constexpr (MAPPED) {
 #pragma unroll
-      for (int i = 0; i < L; ++i) {
-        const int k = kt * BK + krow[i];
-        entry[i] = p.row_map[row_begin + (k < rows ? k : rows - 1)];
+      for (int i = 0; i < L * RPI; ++i) {
+        const int k = kt * BK + wave * (L * RPI) + i;
+        entry[i] = as_const(p.row_map)[row_begin + (k < rows ? k : rows - 1)];
       }
     }
   };
@@ -1616,12 +1621,15 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
     for (int i = 0; i < L; ++i) {
       const int k = f_kt * BK + krow[i], direct = row_begin + k;
       int mapped = direct;
-      if constexpr (MAPPED) mapped = fastdiv(entry[i], p.map_div);
+      if constexpr (MAPPED) {
+        const int first = fastdiv(entry[i * RPI], p.map_div), second = fastdiv(entry[i * RPI + 1], p.map_div);
+        mapped = lane < 64 / RPI ? first : second;
+      }
       a[i] = k < rows ? (const void*)(A + (int64_t)(map_a ? mapped : direct) * q.lda + col[i]) : g_zero16;
       b[i] = k < rows ? (const void*)(B + (int64_t)(map_b ? mapped : direct) * q.ldb + col[i]) : g_zero16;
     }
     f_kt = f_kt + 1 < nkt ? f_kt + 1 : 0;
-    lookup(f_kt);
+    if (nkt > 1) lookup(f_kt);      // (one k-tile: the same rows every time)
     const uint32_t to = lds + f_stage * STAGE;
 #pragma unroll
     for (int i = 0; i < L; ++i) dma16(a[i], to + i * 1024);
