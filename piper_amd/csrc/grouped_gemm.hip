@@ -464,7 +464,7 @@ struct Stage32 {
   // (lane: the caller's lane id; a caller that wants the per-lane addresses formed here, not hoisted
   // out of its loops into registers that stay live across them, passes a value the compiler cannot
   // see through)
-  template <bool ACC, bool STREAM = false>
+  template <bool STREAM = false>
   __device__ static __forceinline__ int flush(const char* buf, bf16_t* dst, int64_t ldc, int nrows, int lane = threadIdx.x & 63) {
     constexpr int RPP = 64 / CH, NP = 32 / RPP;
     const int lr = lane / CH, lc = lane % CH;
@@ -479,14 +479,6 @@ struct Stage32 {
       const int r = q * RPP + lr;
       if (r < nrows) {
         u32x4_t* g = reinterpret_cast<u32x4_t*>(dst + (int64_t)r * ldc + lc * 8);
-        if (ACC) {
-          const bf16x8_t a = __builtin_bit_cast(bf16x8_t, v[q]);
-          const bf16x8_t o = __builtin_bit_cast(bf16x8_t, *g);
-          bf16x8_t sum;
-#pragma unroll
-          for (int t = 0; t < 8; ++t) sum[t] = (bf16_t)((float)a[t] + (float)o[t]);
-          v[q] = __builtin_bit_cast(u32x4_t, sum);
-        }
         if (STREAM) __builtin_nontemporal_store(v[q], g);
         else *g = v[q];
       }
@@ -1142,7 +1134,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
                 St::put(sbuf, lrow, 16 * j + 8 * q + lq, v);
               }
             wave_lds_fence();
-            st_after += St::template flush<false>(sbuf, out + goff, p.ldc, crows);
+            st_after += St::template flush<>(sbuf, out + goff, p.ldc, crows);
             wave_lds_fence();
           }
         }
@@ -1158,7 +1150,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
                 St::put(sbuf, lrow, 32 * (j - j0) + 8 * q + lq,
                         pack4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]));
             wave_lds_fence();
-            st_after += St::template flush<false>(sbuf, p.O0 + goff + 32 * j0, p.ldc, crows);
+            st_after += St::template flush<>(sbuf, p.O0 + goff + 32 * j0, p.ldc, crows);
             wave_lds_fence();
           }
         }
@@ -1210,8 +1202,8 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
             }
             const int64_t tofs = ((int64_t)((cur_u.tcol + wrow + RS * i) >> 5) * p.ldc + gcol0 + 32 * j) * 32;
             wave_lds_fence();
-            st_after += S2::template flush<false>(sb0, p.O0 + goff + 32 * j, p.ldc, crows, lane_e);
-            st_after += S2::template flush<false>(sb1, p.O1 + goff + 32 * j, p.ldc, crows, lane_e);
+            st_after += S2::template flush<>(sb0, p.O0 + goff + 32 * j, p.ldc, crows, lane_e);
+            st_after += S2::template flush<>(sb1, p.O1 + goff + 32 * j, p.ldc, crows, lane_e);
             if constexpr (SCALED) {
               if (transposed) {
                 st_after += S2::flush_t(sb0, p.T0 + tofs, 32, crows, lane_e);
@@ -1224,7 +1216,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
 #pragma unroll
                 for (int q = 0; q < 4; ++q) S2::put(sb0, lrow, 8 * q + lq, hsv[q]);
                 wave_lds_fence();
-                if (p.O2) st_after += S2::template flush<false>(sb0, p.O2 + goff + 32 * j, p.ldc, crows, lane_e);
+                if (p.O2) st_after += S2::template flush<>(sb0, p.O2 + goff + 32 * j, p.ldc, crows, lane_e);
                 if (transposed) st_after += S2::flush_t(sb0, p.T2 + tofs, 32, crows, lane_e);
                 wave_lds_fence();
               }
@@ -1301,7 +1293,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
                 St::put(sbuf, lrow, 32 * j + 8 * q + lq, (transposed && !live) ? zero2 : v);
               }
             wave_lds_fence();
-            if (out) st_after += St::template flush<false>(sbuf, out + goff, p.ldc, crows);
+            if (out) st_after += St::template flush<>(sbuf, out + goff, p.ldc, crows);
             if constexpr (SCALED) {
               if (transposed)
                 st_after += St::flush_t(sbuf, (which == 0 ? p.T0 : which == 1 ? p.T1 : p.T2) +
@@ -1567,8 +1559,32 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
   };
+  auto tile_dst = [&] {
+    return q.C + (int64_t)e * q.M * q.N + ((int64_t)(tile / n_tiles) * BM + wm * WTM) * q.N + (tile % n_tiles) * BN + wn * WTN;
+  };
+  // ACC: the gradients that are there, requested 64 rows at a time: the first half of a tile in front of its last products, the
+  // second behind them (all of them at once are more registers than there are).  Read row by row where they are added they are
+  // 16 round trips a tile, each with the stores and the ring's loads in front of it (us, so -> this: 128 experts 2048 x 768, 32 rows
+  // 648 -> 418, 128 rows 744 -> 468, 400 rows 1127 -> 907; 32 experts 1024 x 512, 32 rows 79 -> 49; 16 experts 2048 x 1024, 128 uneven rows
+  // 158 -> 99; wgrad_kernel at the first three 691, 786, 1,080).
+  constexpr int HALF = TM / 2, OLD_NP = 32 * St::CH / 64, OLD = ACC ? HALF * OLD_NP : 0;     // OLD: loads of a half
+  u32x4_t old[ACC ? TM : 1][OLD_NP];
+  auto request_old = [&](auto half_c) {
+    if constexpr (ACC) {
+      constexpr int H0 = decltype(half_c)::value * HALF;
+      __builtin_amdgcn_sched_barrier(0);
+      const bf16_t* const C = tile_dst();
+#pragma unroll
+      for (int i = H0; i < H0 + HALF; ++i)
+#pragma unroll
+        for (int x = 0; x < OLD_NP; ++x)
+          old[i][x] = __builtin_nontemporal_load(
+              reinterpret_cast<const u32x4_t*>(C + (int64_t)(32 * i + x * (64 / St::CH) + lane / St::CH) * q.N + lane % St::CH * 8));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   auto store_tile = [&](char* stage) {
-    bf16_t* const C = q.C + (int64_t)e * q.M * q.N + ((int64_t)(tile / n_tiles) * BM + wm * WTM) * q.N + (tile % n_tiles) * BN + wn * WTN;
+    bf16_t* const C = tile_dst();
     char* const sbuf = stage + wave * St::BYTES;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -1579,7 +1595,8 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
           St::put(sbuf, lrow, 32 * j + 8 * qd + lq,
                   pack4(acc[i][j][4 * qd], acc[i][j][4 * qd + 1], acc[i][j][4 * qd + 2], acc[i][j][4 * qd + 3]));
       wave_lds_fence();
-      St::template flush<ACC, true>(sbuf, C + (int64_t)(32 * i) * q.N, q.N, 32, lane);
+      if constexpr (ACC) St::template flush_add<true>(sbuf, C + (int64_t)(32 * i) * q.N, q.N, old[i], lane);
+      else St::template flush<true>(sbuf, C + (int64_t)(32 * i) * q.N, q.N, 32, lane);
       wave_lds_fence();
     }
   };
@@ -1644,26 +1661,33 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
   };
   lookup(0);
   fetch();
-  // operations behind the loads of the k-tile that comes next (at least: row map entries come on top): the stores of the step
-  // that issued those, the loads and the stores of the step after it
-  int stores_before = 0, loads_behind = fetch(), stores_behind = 0;
+  // operations behind the loads of the k-tile that comes next: what followed these in their own step, the loads of the step after it
+  // (behind the old values' first half), and what followed them there
+  int after_before = 0, loads_behind = fetch(), after_behind = 0;
   for (int kt = 0, stage = 0;; stage = stage + 1 == NS ? 0 : stage + 1) {
-    wait_vm_le(stores_before + loads_behind + stores_behind);
+    wait_vm_le(after_before + loads_behind + after_behind);
     // everybody's loads of this k-tile have landed, and nobody reads the stage of the last one any more, as operands or as
     // staged output: the next fetch may overwrite it
     block_barrier();
-    loads_behind = fetch();
+    const bool last = ++kt == nkt;
+    loads_behind = 0;
+    if (ACC && last) {
+      request_old(std::integral_constant<int, 0>{});
+      loads_behind = OLD;
+    }
+    loads_behind += fetch();
     char* const st = smem + stage * STAGE;
     mma_tile<BK, TM, TN, false, false, BM, BN, false>(st, st + A_BYTES, wm * WTM, wn * WTN, acc);
-    stores_before = stores_behind;
-    stores_behind = 0;
-    if (++kt == nkt) {
+    after_before = after_behind;
+    after_behind = 0;
+    if (last) {
+      request_old(std::integral_constant<int, 1>{});
       block_barrier();            // every wave has read its fragments
       store_tile(st);
       if (--left == 0) break;
       ++tile;
       clear();
-      stores_behind = STORES;
+      after_behind = OLD + STORES;
       kt = 0;
     }
   }
@@ -2094,7 +2118,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_pp_kernel(const WgradKcP
                       pack4(acc[i][jh + jj][4 * qd], acc[i][jh + jj][4 * qd + 1], acc[i][jh + jj][4 * qd + 2], acc[i][jh + jj][4 * qd + 3]));
           wave_lds_fence();
           if constexpr (ACCUMULATE) st_after += St::template flush_add<true>(sbuf, chunk_dst(c), p.N, old[c - c0]);
-          else st_after += St::template flush<false, true>(sbuf, chunk_dst(c), p.N, 32);
+          else st_after += St::template flush<true>(sbuf, chunk_dst(c), p.N, 32);
           wave_lds_fence();
         }
       }
