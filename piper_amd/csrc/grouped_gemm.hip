@@ -1418,6 +1418,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
     }
   };
   uint32_t is_a = 0, is_b = 0;     // LDS destinations of this wave's pieces in the stage being filled
+  bool is_real = true;             // false: no tile left, the pieces read zeros (rows are not looked up)
   auto issue_setup = [&](int stage) {
     char* st = smem + stage * STAGE;
     is_a = lds_addr(st) + (wave * LA) * 1024;
@@ -1433,7 +1434,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 #pragma unroll
       for (int r = 0; r < A_RPI; ++r) {
         const int v = arow[i * A_RPI + r];
-        if (v >= 0) {
+        if (is_real && v >= 0) {
           const bf16_t* cand = Abase + (int64_t)v * lda;
           if (lane / A_CPR == r) src = cand + cofs;
         }
@@ -1447,7 +1448,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 #pragma unroll
       for (int r = 0; r < B_RPI; ++r) {
         const int v = brow[i * B_RPI + r];
-        if (v >= 0) {
+        if (is_real && v >= 0) {
           const bf16_t* cand = Bbase + (int64_t)v * ldb;
           if (lane / B_CPR == r) src = cand + cofs;
         }
@@ -1469,23 +1470,60 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
+  if constexpr (NS >= 3) {
+    // every slot issues its loads (rows past the expert's end read a block of zeros), so the
+    // number of loads in flight is the same at every k-tile
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < nkt) {
-      fetch_rows(s);
+    for (int s = 0; s < NS - 1; ++s) {
+      is_real = s < nkt;
+      if (is_real) fetch_rows(s);
       issue(s);
     }
-  if (NS - 1 < nkt) fetch_rows(NS - 1);
+    if (NS - 1 < nkt) fetch_rows(NS - 1);
+  } else {
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s)
+      if (s < nkt) {
+        fetch_rows(s);
+        issue(s);
+      }
+    if (NS - 1 < nkt) fetch_rows(NS - 1);
+  }
   int cur = 0, nxt = NS - 1;
-  for (int kt = 0; kt < nkt; ++kt) {
-    if (kt + NS - 2 < nkt) wait_dma<(NS - 2) * (LA + LB)>(); else wait_dma<0>();
+  if constexpr (NS >= 3) {
+    // Rings of three or more stages: the loads of tile kt+NS-1 and the fragment reads of the
+    // next k-step are spread between the MFMAs, and the first fragments of tile kt+1 are read
+    // during tile kt (the barrier at the top of tile kt waits for tile kt+1).
+    constexpr int L = LA + LB;
+    wait_dma<(NS - 2) * L>();
     block_barrier();
-    if (kt + NS - 1 < nkt) issue(nxt);
-    if (kt + NS < nkt) fetch_rows(kt + NS);
-    const char* st = smem + cur * STAGE;
-    mma_tile<BK, TM, TN, false, false, BM, BN, (TM * TN >= 16)>(st, st + A_BYTES, wm * WTM, wn * WTN, acc);
-    cur = cur + 1 == NS ? 0 : cur + 1;
-    nxt = nxt + 1 == NS ? 0 : nxt + 1;
+    Frags<TM, TN> f0;
+    load_frags<BK, TM, TN, false, false, BM, BN>(f0, smem, smem + A_BYTES, wm * WTM, wn * WTN, 0, lane);
+    for (int kt = 0; kt < nkt; ++kt) {
+      wait_dma<(NS - 3) * L>();
+      block_barrier();
+      issue_setup(nxt);
+      is_real = kt + NS - 1 < nkt;
+      const char* st = smem + cur * STAGE;
+      const char* stn = smem + (cur + 1 == NS ? 0 : cur + 1) * STAGE;
+      mma_ktile<BK, TM, TN, false, false, BM, BN, L>(st, st + A_BYTES, stn, stn + A_BYTES, wm * WTM, wn * WTN,
+                                                     f0, acc, [&](int piece) { issue_piece(piece); });
+      if (kt + NS < nkt) fetch_rows(kt + NS);
+      cur = cur + 1 == NS ? 0 : cur + 1;
+      nxt = nxt + 1 == NS ? 0 : nxt + 1;
+    }
+    wait_dma<0>();   // zero loads of the last k-tiles: the staging below reuses the ring
+  } else {
+    for (int kt = 0; kt < nkt; ++kt) {
+      if (kt + NS - 2 < nkt) wait_dma<(NS - 2) * (LA + LB)>(); else wait_dma<0>();
+      block_barrier();
+      if (kt + NS - 1 < nkt) issue(nxt);
+      if (kt + NS < nkt) fetch_rows(kt + NS);
+      const char* st = smem + cur * STAGE;
+      mma_tile<BK, TM, TN, false, false, BM, BN, (TM * TN >= 16)>(st, st + A_BYTES, wm * WTM, wn * WTN, acc);
+      cur = cur + 1 == NS ? 0 : cur + 1;
+      nxt = nxt + 1 == NS ? 0 : nxt + 1;
+    }
   }
 
   block_barrier();
@@ -1517,8 +1555,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 // 237 -> 211 / 237 -> 212, 32 rows 281 -> 240 / 286 -> 237, 64 rows 325 -> 258 / 342 -> 266, 128 rows 411 -> 366 / 446 -> 399;
 // 64 experts 1536 x 768, 24 rows 111 -> 90 / 109 -> 93; 32 experts 1024 x 512: 32 rows 33 -> 28 / 32 -> 28, 128 rows 45 -> 44 /
 // 54 -> 46; 16 experts 2048 x 1024, 64 rows 66 -> 54 / 71 -> 56; 24 experts 1024 x 768, 20 rows 36 -> 30 / 36 -> 30.
-// With 512 rows wgrad_kernel's deeper k-tiles are ahead (16 experts 2048 x 1024 160 / 165, 32 experts 1024 x 512, 1,024 rows
-// 145 / 152).  The order of the sums is wgrad_kernel's.
+// With more rows wgrad_kernel's k-loops are ahead (lines and figures at PK_WG_RUNS_ROWS).  The order of the sums is wgrad_kernel's.
 // MAPPED: some problem's rows are gathered (p.row_map).
 template <bool ACC, bool MAPPED>
 __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p) {
@@ -2373,11 +2410,19 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_RM_TALL 160, 256, 64, 2, 4, 3
 #define PK_RM_TALL_ROWS 248
 #define PK_RM_TALL_DOWN_K 1024
-// Weight gradients from row-major operands (with the transposed copies wgrad_pp_kernel, whose tile is fixed): 256 x 256
-// tiles with 64-deep k-tiles in a 2-stage ring; below PK_WG_RUNS_ROWS rows an expert wgrad_runs_kernel.
+// Weight gradients from row-major operands (with the transposed copies wgrad_pp_kernel, whose tile is fixed), 256 x 256 tiles by
+// rows an expert: few, wgrad_runs_kernel; from PK_WG_BIG_ROWS on 64-deep k-tiles in a 2-stage ring; between them 32-deep ones in a
+// 4-stage ring with the loads spread between the MFMAs.  us, runs -> 4-stage ring, gathered rows, even counts / ~ 1 / sqrt(rank): 128 experts
+// 2048 x 768: 192 rows 449 -> 476 / 516 -> 503, 256 rows 571 -> 556 / 658 -> 599, 400 rows 783 -> 734 / 876 -> 796; 64 experts 1536 x 768, 400
+// rows 299 -> 287 / 327 -> 312; 24 experts 1024 x 768, 400 rows, not gathered, 88 -> 81 / 82 -> 72.  With fewer than two tiles for every CU the
+// longest expert's k-loop counts sooner (64 experts 512 x 256, 192 rows, not gathered, 33.2 -> 34.0 / 48.0 -> 43.8).  Accumulating, the runs'
+// way to the old values is ahead at any size (128 experts 2048 x 768, 400 rows 907 against 1,080).
 #define PK_WG_BIG 256, 256, 64, 2, 4, 2
+#define PK_WG_BIG_ROWS 512
+#define PK_WG_RING 256, 256, 32, 2, 4, 4
 #define PK_WG_THREADS 512
-#define PK_WG_RUNS_ROWS 512
+#define PK_WG_RUNS_ROWS 224
+#define PK_WG_RUNS_ROWS_ONE 160
 #define PK_WG_DYNAMIC_ROWS 512
 // rows an expert up to which d_h is formed on the tiles of tile_gemm.h
 #define PK_DH_TILE_ROWS 40
@@ -3037,8 +3082,8 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   // 90 / 96, 48 rows 118 / 111 / 118, 128 rows 161 / 148 / 165; 16 experts 2048 x 1024, 6 tiles, 64 rows 61 / 54 / 58, 512 rows,
   // ~ 1 / sqrt(rank) 172 / 181; 32 experts 1024 x 512, 3 tiles: 32 rows 30 / 28, 128 rows 44 / 45 (46 / 55); 64 experts
   // 512 x 256, 1.5 tiles, 100 rows 26 / 23 (32 / 54)).
-  const bool few_rows = A < (int64_t)PK_WG_RUNS_ROWS * E;
   const int64_t tiles = (int64_t)p.tiles_per_problem * n * E, per_cu = tiles / mf::persistent_grid();
+  const bool few_rows = A < (int64_t)(p.accumulate ? PK_WG_BIG_ROWS : per_cu < 2 ? PK_WG_RUNS_ROWS_ONE : PK_WG_RUNS_ROWS) * E;
   p.run = 1;
   if (few_rows) {
     if (per_cu >= 24 && A > 32 * E && A <= 192 * E && p.tiles_per_problem % 4 == 0) p.run = 4;
@@ -3053,7 +3098,9 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
     if (p.row_map) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_runs_kernel<ACC, true>), grid, block, 0, s, p);    \
     else PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_runs_kernel<ACC, false>), grid, block, 0, s, p);             \
   } while (0)
-  if (!few_rows) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), grid, block, 0, s, p);
+  if (!few_rows && A < (int64_t)PK_WG_BIG_ROWS * E)
+    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_RING>), grid, block, 0, s, p);
+  else if (!few_rows) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), grid, block, 0, s, p);
   else if (p.accumulate) PK_WG_RUNS(true);
   else PK_WG_RUNS(false);
 #undef PK_WG_RUNS

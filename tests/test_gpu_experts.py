@@ -896,6 +896,8 @@ RUN_CASES = [
     ([31, 0, 65, 32] * 8, 1024, 512),                                # two
     ([0, 33, 64, 1, 97, 32, 45, 90] * 16, 1024, 1024),               # four
     ([900, 0, 31, 2, 1500, 65, 1000, 700], 1024, 512),               # 64-deep k-tiles
+    ([300, 0, 31, 2, 500, 65, 900, 97], 1024, 512),                  # 32-deep ones in a ring of four stages
+    ([224, 240, 0, 33, 500, 64, 700, 300] * 2, 1024, 768),           # (from two tiles for every CU on)
 ]
 
 
