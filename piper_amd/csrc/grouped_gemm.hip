@@ -1337,7 +1337,7 @@ struct WgradParams {
 
 // Workgroup b runs on XCD b % 8.  Units, sorted by expert, come in chunks of neighbours, and chunk c goes to XCD c % 8 in
 // "snake" order (0..7, 7..0, 0..7, ...): the tiles of a chunk read the same rows through one L2.  Chunks used to be whole
-// experts, which leaves XCDs idle where experts are few or uneven; now an XCD has at least 16 (deal_chunk).  us, whole experts
+// experts, which leaves XCDs idle where experts are few or uneven.  us, whole experts
 // -> chunks, even counts / ~ 1 / sqrt(rank): 8 experts 2048 x 1024, 256 rows 58 -> 57 / 81 -> 58, 1,024 rows 143 -> 140 /
 // 222 -> 147; 32 experts 1024 x 512, 256 rows 59 -> 59 / 73 -> 61; 128 experts 2048 x 768, 64 rows 323 -> 323 / 337 -> 335.
 __device__ __forceinline__ int dealt_unit(int chunk) {
@@ -1345,11 +1345,14 @@ __device__ __forceinline__ int dealt_unit(int chunk) {
   const int turn = pos / chunk;
   return ((turn & 1) ? turn * NXCD + (NXCD - 1 - xcd) : turn * NXCD + xcd) * chunk + pos % chunk;
 }
-// host: the chunk for `units` units, `per_expert` of them an expert's
+// host: the chunk for `units` units, `per_expert` of them an expert's: 16 or more for an XCD where there are as many units, at most an
+// expert.  It need not divide an expert's units: halved while it is even it stays whole experts where these have an odd number, or few
+// chunks (us, so -> this, even counts / ~ 1 / sqrt(rank): 8 experts 1280 x 768, 128 rows 26 -> 26 / 37 -> 24, 1,024 rows 88 -> 89 / 148 -> 83; 12
+// experts 1280 x 1280, 256 rows 83 -> 69 / 87 -> 67; 16 experts 768 x 768, 256 rows 38 -> 39 / 49 -> 38; 24 experts 1536 x 768, 1,024 rows
+// 251 -> 254 / 265 -> 245).
 int32_t deal_chunk(int64_t units, int64_t per_expert) {
-  int64_t chunk = per_expert;
-  while (chunk % 2 == 0 && units < 16 * NXCD * chunk) chunk /= 2;
-  return (int32_t)chunk;
+  const int64_t chunk = units / (16 * NXCD);
+  return (int32_t)(chunk < 1 ? 1 : chunk < per_expert ? chunk : per_expert);
 }
 
 template <int BM, int BN, int BK, int WMW, int WNW, int NS>

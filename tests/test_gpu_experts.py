@@ -898,6 +898,9 @@ RUN_CASES = [
     ([900, 0, 31, 2, 1500, 65, 1000, 700], 1024, 512),               # 64-deep k-tiles
     ([300, 0, 31, 2, 500, 65, 900, 97], 1024, 512),                  # 32-deep ones in a ring of four stages
     ([224, 240, 0, 33, 500, 64, 700, 300] * 2, 1024, 768),           # (from two tiles for every CU on)
+    ([0, 70, 33, 1, 130, 20, 64, 9] * 2, 768, 768),                  # an odd number of tiles an expert, dealt out in chunks of 3
+    ([40, 0, 90, 32] * 3, 1280, 1280),                               # of 7, which cross from one expert to the next
+    ([600, 0, 900, 1, 40, 1200, 700, 800], 1280, 768),               # one by one
 ]
 
 
