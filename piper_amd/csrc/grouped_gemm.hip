@@ -2983,8 +2983,12 @@ int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dt
   // (d_h + weight gradients, us, transposed -> plain: 8 experts 1024 x 512, 64 tiles each, 4,096 rows an expert
   // 440 -> 270; 16 experts 512 x 256, 32 tiles, 4,096 rows 419 -> 304), and with 256 tiles it depends on whether
   // d_h fills the chip (32 experts 1024 x 512: 128 rows 100 -> 66, 512 rows 168 -> 158, 1,024 rows 246 -> 241).  Above,
-  // the transposed pair is ahead (16 experts 2048 x 1024, 1,024 rows 369 -> 410); wgrad_kernel deals experts out
-  // over the XCDs and leaves some idle below eight (4 experts 2048 x 1024, 2,048 rows 275 -> 349).
+  // the transposed pair is ahead (16 experts 2048 x 1024, 1,024 rows 369 -> 410), and below eight experts, where the tiles of tile_gemm.h
+  // stood in for wgrad_kernel at any size (4 experts 2048 x 1024, 2,048 rows 275 -> 349).  Both lines are older than the dealing of tiles
+  // in chunks (dealt_unit), with which the plain pair is level or ahead from 128 to 256 tiles too but for long reductions
+  // (transposed -> plain, even counts / ~ 1 / sqrt(rank): 8 experts 2048 x 512, 600 rows 178 -> 155 / 203 -> 148; 4 experts 2048 x 1024, 64 rows
+  // 71 -> 65 / 74 -> 67, 2,048 rows 265 -> 235 / 351 -> 264; 24 experts 1024 x 512, 128 rows 114 -> 109 / 121 -> 101, 2,048 rows 398 -> 394 /
+  // 554 -> 404; 32 experts 1024 x 512, 1,024 rows 249 -> 254 / 354 -> 294, 2,048 rows 403 -> 438 / 589 -> 497).
   const int64_t w2_units = E * (H / 256) * (I / 256);
   if (w2_units < mf::persistent_grid() / 2) return 0;
   return E < mf::NXCD || w2_units > mf::persistent_grid() || wide_fills(A, I, E, 8);
@@ -3036,13 +3040,18 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   if (!row_map) row_map_div = 1;
   const int32_t* dy_map = dy_gathered ? row_map : nullptr;
   hipStream_t s = (hipStream_t)stream;
-  // wgrad_kernel's 256 x 256 tiles where they give at least half of the CUs work and every XCD an expert; otherwise
-  // the 64- or 128-wide tiles of tile_gemm.h (us, 256 x 256 or, at widths that are not multiples of 256, its former
-  // 128 x 128 tiles -> those: 4 experts 2048 x 1024, 2,048 rows 260 -> 219; 24 experts 640 x 896, 1,000 rows 379 -> 176;
-  // 64 experts 384 x 640, 1,536 rows 614 -> 287; but 8 experts 1024 x 512, 1,024 rows, 192 tiles 50 against 79)
+  // 256 x 256 tiles where they give at least half of the CUs work; otherwise the 64- or 128-wide tiles of tile_gemm.h (us, 256 x 256 or, at
+  // widths that are not multiples of 256, its former 128 x 128 tiles -> those: 24 experts 640 x 896, 1,000 rows 379 -> 176; 64 experts
+  // 384 x 640, 1,536 rows 614 -> 287; but 8 experts 1024 x 512, 1,024 rows, 192 tiles 50 against 79).  With fewer experts than XCDs and
+  // long reductions a last round of few tiles, or an expert longer than the others, costs more than the smaller tiles do: two tiles
+  // for every CU there (tile_gemm.h's / 256 x 256, even counts, ~ 1 / sqrt(rank): 4 experts 2048 x 1024, 24 rows 22 / 17, 21 / 17, 300 rows 42 /
+  // 42, 42 / 37, 2,048 rows 155 / 172, 154 / 152; 4 experts 1024 x 1024, 128 rows 18 / 16, 20 / 18, 600 rows 37 / 36, 40 / 44, 2,048 rows 96 / 90,
+  // 94 / 120; 6 experts 2048 x 768, 300 rows 47 / 43, 47 / 43, 2,048 rows 179 / 176, 189 / 206; 4 experts 2048 x 2048, 300 rows 73 / 62, 74 / 61,
+  // 2,048 rows 295 / 262, 311 / 269).
   const int n_weights = (d_w1 ? 1 : 0) + (d_w2 ? 1 : 0) + (d_w3 ? 1 : 0);
+  const int64_t tiles_256 = E * (H / 256) * (I / 256) * n_weights, cus = mf::persistent_grid();
   const bool mfma = dtype == PK_BF16 && H % 256 == 0 && I % 256 == 0 && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}) &&
-                    E >= mf::NXCD && E * (H / 256) * (I / 256) * n_weights >= mf::persistent_grid() / 2;
+                    tiles_256 >= cus / 2 && (E >= mf::NXCD || A < (int64_t)PK_WG_BIG_ROWS * E || tiles_256 >= 2 * cus);
   if (!mfma && tile_gemm_ok(dtype, H, I, {d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}))
     return dtype == PK_F32
                ? wgrad_tile<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, A, H, I, E, s)

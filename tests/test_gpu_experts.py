@@ -901,6 +901,9 @@ RUN_CASES = [
     ([0, 70, 33, 1, 130, 20, 64, 9] * 2, 768, 768),                  # an odd number of tiles an expert, dealt out in chunks of 3
     ([40, 0, 90, 32] * 3, 1280, 1280),                               # of 7, which cross from one expert to the next
     ([600, 0, 900, 1, 40, 1200, 700, 800], 1280, 768),               # one by one
+    ([40, 0, 65, 33], 1024, 1024),                                   # fewer experts than XCDs
+    ([300, 500, 1, 0, 460], 2048, 768),
+    ([1000, 700, 0, 900], 2048, 2048),
 ]
 
 
