@@ -3092,7 +3092,7 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   // every CU and none is long (us, runs of 1 / 2 / 4 tiles, even counts: 128 experts 2048 x 768, 36 tiles a CU: 16 rows 225 / 222 /
   // 230, 32 rows 252 / 240 / 240, 48 rows 290 / 256 / 243, 96 rows 368 / 321 / 310; 64 experts 1536 x 768, 13 tiles: 24 rows
   // 90 / 96, 48 rows 118 / 111, 128 rows 161 / 148; 16 experts 2048 x 1024, 6 tiles, 64 rows 61 / 54 / 58, 512 rows,
-  // ~ 1 / sqrt(rank) 172 / 181; 32 experts 1024 x 512, 3 tiles: 32 rows 30 / 28, 128 rows 44 / 45 (46 / 55); 64 experts
+  // ~ 1 / sqrt(rank) 172 / 181; 32 experts 1024 x 512, 3 tiles: 32 rows 30 / 28, 64 rows 31.3 / 32.7 (37 / 34), 128 rows 44 / 45 (46 / 55); 64 experts
   // 512 x 256, 1.5 tiles, 100 rows 26 / 23 (32 / 54)).  Two against one in per cent: 64 experts 1024 x 1024, 12 tiles a CU, 8 rows -7 / -1
   // uneven, 32 rows -9 / -5; 128 experts 1024 x 512, 12 tiles, 24 rows -4 / -3; 96 experts 1024 x 1024, 18 tiles, 24 rows -9 / -2; 24 experts
   // 2048 x 1024, 9 tiles, 24 rows -7 / -6; but 64 experts 1536 x 768, whose 18 tiles make an odd number of pairs, 24 rows +2 / +10; 64 experts
@@ -3102,9 +3102,10 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   const bool few_rows = A < (int64_t)(p.accumulate ? PK_WG_BIG_ROWS : per_cu < 2 ? PK_WG_RUNS_ROWS_ONE : PK_WG_RUNS_ROWS) * E;
   p.run = 1;
   if (few_rows) {
+    const int64_t two = (per_cu < 6 ? 64 : 192) / (p.tiles_per_problem >= 8 ? 1 : per_cu < 6 ? 2 : 3);
     if (per_cu >= 24 && A > 32 * E && A <= 192 * E && p.tiles_per_problem % 4 == 0)
       p.run = 4;
-    else if (p.tiles_per_problem % 2 == 0 && per_cu >= 3 && A <= (per_cu < 6 ? 32 : p.tiles_per_problem < 8 ? 64 : 192) * E &&
+    else if (p.tiles_per_problem % 2 == 0 && per_cu >= 3 && A <= two * E &&
              (per_cu < 12 || per_cu >= 24 || A > 32 * E || p.tiles_per_problem % 4 == 0))
       p.run = 2;
   }
