@@ -1155,29 +1155,25 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
           }
         }
       } else if constexpr (LEAN_BWD) {
-        // EPI_SWIGLU_BWD[_SCALED] with 128 accumulator registers: the packed outputs of 32 columns
-        // at a time, d_g and d_u side by side in the staging buffer, score * h after them
+        // EPI_SWIGLU_BWD with 128 accumulator registers: the packed outputs of 32 columns at a time, d_g and d_u side by side in
+        // the staging buffer.  Not the scaled form, whose third output, transposed copies and optional row-major ones (null where
+        // only the copies are read) are the other branch's.
+        static_assert(!SCALED, "units of more than 128 rows: the unscaled backward only");
         using S2 = Stage32<32>;
         static_assert(2 * S2::BYTES <= St::BYTES, "two 32-column areas in a wave's staging buffer");
         char* const sb0 = sbuf;
         char* const sb1 = sbuf + S2::BYTES;
-        float ds = 0.f;
         if (crows > 0) {
-          const float sc = sc_chunk[i];
           load_gu(i, 0);
           __builtin_amdgcn_sched_barrier(0);
           // the loads must have returned before the next unit's first tiles are requested: a load
           // behind those requests would wait for all of them
-          const bool transposed = SCALED && p.T0 != nullptr;
-          const bool live = lrow < crows;      // the transposed copies want zeros in the rows past the end
-          const u32x2_t zero2 = {0u, 0u};
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
-            u32x2_t hsv[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              float dh[4], g[4], u[4], og[4], ou[4], oh[4];
-              unpack4(pack4(sc * acc[i][j][4 * q], sc * acc[i][j][4 * q + 1], sc * acc[i][j][4 * q + 2], sc * acc[i][j][4 * q + 3]), dh);
+              float dh[4], g[4], u[4], og[4], ou[4];
+              unpack4(pack4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]), dh);
               unpack4(graw[j][q], g);
               unpack4(uraw[j][q], u);
 #pragma unroll
@@ -1185,49 +1181,18 @@ __global__ __launch_bounds__(64 * WMW * WNW) void ragged_m_kernel(const RaggedMP
                 const float sg = sigmoid_fast(g[t]);
                 og[t] = dh[t] * u[t] * (sg * (1.f + g[t] * (1.f - sg)));
                 ou[t] = dh[t] * (g[t] * sg);
-                if (SCALED) {
-                  const float hv = (g[t] * sg) * u[t];
-                  ds += acc[i][j][4 * q + t] * hv;
-                  oh[t] = sc * hv;
-                }
               }
-              const bool dead = transposed && !live;
-              S2::put(sb0, lrow, 8 * q + lq, dead ? zero2 : pack4(og[0], og[1], og[2], og[3]));
-              S2::put(sb1, lrow, 8 * q + lq, dead ? zero2 : pack4(ou[0], ou[1], ou[2], ou[3]));
-              if (SCALED) hsv[q] = dead ? zero2 : pack4(oh[0], oh[1], oh[2], oh[3]);
+              S2::put(sb0, lrow, 8 * q + lq, pack4(og[0], og[1], og[2], og[3]));
+              S2::put(sb1, lrow, 8 * q + lq, pack4(ou[0], ou[1], ou[2], ou[3]));
             }
             if (j == TN - 1 && i == TM - 1) {
               __builtin_amdgcn_sched_barrier(0);
               prefetch_next();
             }
-            const int64_t tofs = ((int64_t)((cur_u.tcol + wrow + RS * i) >> 5) * p.ldc + gcol0 + 32 * j) * 32;
             wave_lds_fence();
             st_after += S2::template flush<>(sb0, p.O0 + goff + 32 * j, p.ldc, crows, lane_e);
             st_after += S2::template flush<>(sb1, p.O1 + goff + 32 * j, p.ldc, crows, lane_e);
-            if constexpr (SCALED) {
-              if (transposed) {
-                st_after += S2::flush_t(sb0, p.T0 + tofs, 32, crows, lane_e);
-                st_after += S2::flush_t(sb1, p.T1 + tofs, 32, crows, lane_e);
-              }
-            }
             wave_lds_fence();
-            if constexpr (SCALED) {
-              if (p.O2 || transposed) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) S2::put(sb0, lrow, 8 * q + lq, hsv[q]);
-                wave_lds_fence();
-                if (p.O2) st_after += S2::template flush<>(sb0, p.O2 + goff + 32 * j, p.ldc, crows, lane_e);
-                if (transposed) st_after += S2::flush_t(sb0, p.T2 + tofs, 32, crows, lane_e);
-                wave_lds_fence();
-              }
-            }
-          }
-          if (SCALED) {
-            // lanes l and l+32 hold the two column halves of row l % 32
-            ds += __shfl_xor(ds, 32);
-            if (lane_e < 32 && lrow < crows)
-              p.ds_partial[(int64_t)((cur_u.nt * BN + wn * WTN) >> 6) * p.total_rows + cur_u.row0 + wrow + RS * i + lrow] = ds;
-            st_after += 1;
           }
         } else if (i == TM - 1) {
           prefetch_next();

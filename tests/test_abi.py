@@ -100,3 +100,21 @@ def test_counter_sets_are_handed_out_per_stream_and_capture():
     assert all(0 <= s < 1024 for s in seen) and len(seen) == 1024
     assert lib.pk_sched_slot_index(dev, stream_a, 0, 0) == a
     assert lib.pk_sched_slot_index(-1, 0, 0, 0) < 0 and lib.pk_sched_slot_index(64, 0, 0, 0) < 0
+
+
+def test_the_scaled_backward_in_units_of_more_than_128_rows_does_not_compile(tmp_path):
+    """Its epilogue would store through outputs that are null where only the transposed copies are read."""
+    import shutil
+    import subprocess
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("no hipcc")
+    src = Path(_lib.__file__).resolve().parent / "csrc" / "grouped_gemm.hip"
+    for epilogue, compiles in (("EPI_SWIGLU_BWD", True), ("EPI_SWIGLU_BWD_SCALED", False)):
+        unit = tmp_path / f"{epilogue}.hip"
+        unit.write_text(f'#include "{src}"\nnamespace {{ template __global__ void mf::ragged_m_kernel<256, 256, 32, 2, 4, 4, false, mf::{epilogue}>'
+                        "(const mf::RaggedMParams); }\n")
+        run = subprocess.run([hipcc, "--offload-arch=gfx950", "-std=c++17", "--cuda-device-only", "-fsyntax-only", str(unit)],
+                             capture_output=True, text=True, timeout=120)
+        assert (run.returncode == 0) == compiles, run.stderr
+        assert compiles or "the unscaled backward only" in run.stderr, run.stderr
