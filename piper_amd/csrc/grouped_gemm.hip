@@ -1,17 +1,18 @@
 // Grouped SwiGLU expert GEMMs (forward, input gradient, weight gradient).
 //   bf16: v_mfma_f32_32x32x16_bf16 tiles fed by a ring of direct-to-LDS loads.
 //         Forward and input gradient (ragged_m_kernel): persistent workgroups (one per CU) that
-//         take (expert, row tile, column tile) units from per-XCD counters, 256x256x32 or
-//         128x256x64 block tiles with 8 waves, fused SwiGLU / SwiGLU-backward epilogues, permute
+//         take (expert, row tile, column tile) units from per-XCD counters, 256x256x32, 160x256x64 or
+//         128x256x64 block tiles with 8 waves (unit_rows in launch_rules.h), fused SwiGLU / SwiGLU-backward epilogues, permute
 //         fused into the A-operand loader; ragged row tiles are located on the device from
 //         starts[] (no host sync).  Weight gradient: wgrad_pp_kernel (persistent, 256x256x32, one
-//         operand from the transposed copies the scaled SwiGLU backward writes) for the fused
-//         region; wgrad_kernel (one workgroup per (expert, output tile), both operands through the
-//         transposing LDS read) for the piecewise entry points.
+//         operand from the transposed copies the scaled SwiGLU backward writes) where the fused region keeps
+//         those; from row-major operands, both through the transposing LDS read, 256x256 tiles of wgrad_runs_kernel (few rows an
+//         expert) or wgrad_kernel.
 //   f32, and bf16 widths that are no multiple of 128: 64x64 / 128x128 matrix-core tiles
 //         (tile_gemm.h; fp32 products and sums are exact) + elementwise SwiGLU backward kernels.
 //   rows that are no whole number of 16-byte pieces: tiled FMA kernel (simt_gemm.h).
 #include "pk_common.h"
+#include "launch_rules.h"
 #include "simt_gemm.h"
 #include "tile_gemm.h"
 #include "skinny_gemm.h"
@@ -30,7 +31,7 @@ namespace {
 // ===================================================================== bf16 MFMA path
 namespace mf {
 
-constexpr int NXCD = 8;
+constexpr int NXCD = pk_rules::NXCD;
 
 
 // EPI_SWIGLU_BWD_SCALED: the A rows are rows of d_out gathered through the row map, the
@@ -1297,28 +1298,8 @@ struct WgradParams {
   int32_t tiles_per_problem; // (M/BM)*(N/BN), identical for the three problems
   int32_t nprob;
   int32_t run;               // wgrad_runs_kernel: neighbouring tiles of one workgroup, a divisor of tiles_per_problem
-  int32_t chunk;             // workgroups of one chunk (see dealt_unit)
+  int32_t chunk;             // workgroups of one chunk (see dealt_unit in launch_rules.h)
 };
-
-// Workgroup b runs on XCD b % 8.  Units, sorted by expert, come in chunks of neighbours, and chunk c goes to XCD c % 8 in
-// "snake" order (0..7, 7..0, 0..7, ...): the tiles of a chunk read the same rows through one L2.  Chunks used to be whole
-// experts, which leaves XCDs idle where experts are few or uneven.  us, whole experts
-// -> chunks, even counts / ~ 1 / sqrt(rank): 8 experts 2048 x 1024, 256 rows 58 -> 57 / 81 -> 58, 1,024 rows 143 -> 140 /
-// 222 -> 147; 32 experts 1024 x 512, 256 rows 59 -> 59 / 73 -> 61; 128 experts 2048 x 768, 64 rows 323 -> 323 / 337 -> 335.
-__device__ __forceinline__ int dealt_unit(int chunk) {
-  const int xcd = blockIdx.x % NXCD, pos = blockIdx.x / NXCD;
-  const int turn = pos / chunk;
-  return ((turn & 1) ? turn * NXCD + (NXCD - 1 - xcd) : turn * NXCD + xcd) * chunk + pos % chunk;
-}
-// host: the chunk for `units` units, `per_expert` of them an expert's: 16 or more for an XCD where there are as many units, at most an
-// expert.  It need not divide an expert's units: halved while it is even it stays whole experts where these have an odd number, or few
-// chunks (us, so -> this, even counts / ~ 1 / sqrt(rank): 8 experts 1280 x 768, 128 rows 26 -> 26 / 37 -> 24, 1,024 rows 88 -> 89 / 148 -> 83; 12
-// experts 1280 x 1280, 256 rows 83 -> 69 / 87 -> 67; 16 experts 768 x 768, 256 rows 38 -> 39 / 49 -> 38; 24 experts 1536 x 768, 1,024 rows
-// 251 -> 254 / 265 -> 245).
-int32_t deal_chunk(int64_t units, int64_t per_expert) {
-  const int64_t chunk = units / (16 * NXCD);
-  return (int32_t)(chunk < 1 ? 1 : chunk < per_expert ? chunk : per_expert);
-}
 
 template <int BM, int BN, int BK, int WMW, int WNW, int NS>
 __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams p) {
@@ -1337,7 +1318,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
   const const_i32_ptr starts = as_const(p.starts);
   // the problems of one expert follow each other: d_w1 and d_w3 read the same x rows
   const int per_expert = p.tiles_per_problem * nprob;
-  const int unit = dealt_unit(p.chunk);
+  const int unit = pk_rules::dealt_unit(blockIdx.x, p.chunk);
   if (unit >= p.E * per_expert) return;
   const int want = unit / per_expert, rem = unit % per_expert;
   const WgradProblem& q = p.prob[rem / p.tiles_per_problem];
@@ -1523,7 +1504,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void wgrad_kernel(const WgradParams
 // 237 -> 211 / 237 -> 212, 32 rows 281 -> 240 / 286 -> 237, 64 rows 325 -> 258 / 342 -> 266, 128 rows 411 -> 366 / 446 -> 399;
 // 64 experts 1536 x 768, 24 rows 111 -> 90 / 109 -> 93; 32 experts 1024 x 512: 32 rows 33 -> 28 / 32 -> 28, 128 rows 45 -> 44 /
 // 54 -> 46; 16 experts 2048 x 1024, 64 rows 66 -> 54 / 71 -> 56; 24 experts 1024 x 768, 20 rows 36 -> 30 / 36 -> 30.
-// With more rows wgrad_kernel's k-loops are ahead (lines and figures at PK_WG_RUNS_ROWS).  The order of the sums is wgrad_kernel's.
+// With more rows wgrad_kernel's k-loops are ahead (lines and figures at WG_RUNS_ROWS).  The order of the sums is wgrad_kernel's.
 // MAPPED: some problem's rows are gathered (p.row_map).
 template <bool ACC, bool MAPPED>
 __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p) {
@@ -1539,7 +1520,7 @@ __global__ __launch_bounds__(512, 2) void wgrad_runs_kernel(const WgradParams p)
   __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
 
   const const_i32_ptr starts = as_const(p.starts);
-  const int unit = dealt_unit(p.chunk);
+  const int unit = pk_rules::dealt_unit(blockIdx.x, p.chunk);
   const int per_problem = p.tiles_per_problem / p.run, per_expert = per_problem * p.nprob;
   if (unit >= p.E * per_expert) return;
   const int rank = unit / per_expert, rem = unit - rank * per_expert;
@@ -2345,52 +2326,19 @@ int simt_ragged_k(const void* A, int64_t lda, const int32_t* a_map, const void* 
 #define PK_RM_CFG 256, 256, 32, 2, 4, 4
 #define PK_RM_BN 256
 // Same width with 128 rows, 64-deep k-tiles in a 3-stage ring (a weight row contributes 128
-// contiguous bytes per k-tile).  For launches that would give a workgroup fewer than
-// PK_RM_LOWM_UNITS of the 256-row units (the last round of units would run on a half-empty chip);
-// for experts with fewer than PK_RM_SHORT_ROWS rows on average, where the weights dominate the
-// traffic and are read from HBM by one or two row tiles each (measured at 256 rows per expert
-// against the 256x256x32 tiles: gate/up -8 %, down -4 %, d_x -3 %; at 1,024 rows per expert +2 %
-// to +8 %); and for the scaled SwiGLU backward at any size (against 32-deep k-tiles in a 5-stage
+// contiguous bytes per k-tile).  For launches that would give a workgroup only a few of the 256-row units (the last round of
+// units would run on a half-empty chip); for experts with few rows, where the weights dominate the traffic and are read from
+// HBM by one or two row tiles each (measured at 256 rows per expert against the 256x256x32 tiles: down -4 %, d_x -3 %; at 1,024
+// rows per expert +2 % to +8 %); and for the scaled SwiGLU backward at any size (against 32-deep k-tiles in a 5-stage
 // ring: -9 % at 4,096 tokens, -8 % at 16,384).
 #define PK_RM_SHORT 128, 256, 64, 2, 4, 3
-#define PK_RM_LOWM_UNITS 3
-#define PK_RM_SHORT_ROWS 512
-// d_x already with fewer rows and units: of the three products it reads most of its weights through the transposing LDS
-// read, which the taller unit halves (128 -> 256 rows, us, even / skewed counts: 128 experts 2048 x 768, 320 rows
-// 333 -> 317 / 333 -> 312, 448 rows 424 -> 376 / 422 -> 394; 272 rows 303 -> 311 / 297 -> 279; 1024 x 512, 320 rows 139 -> 142 /
-// 142 -> 142, 384 rows 165 -> 151 / 152 -> 155; 64 experts 2048 x 1024, 352 rows 245 -> 222 / 242 -> 237; 32 experts 2048 x 768,
-// 384 rows, 2.25 units per CU 117 -> 103).  gate/up and down gain as much with even counts between 128 and 200 rows, and
-// lose more with skewed ones (128 experts 2048 x 768, 144 rows: 243 -> 233 / 231 -> 247, 143 -> 133 / 133 -> 140).
-#define PK_RM_DX_ROWS 320
-// 160 rows, otherwise like the 128-row ones: what fits the LDS (3 x 52 KB).  A unit costs about a fifth more time than one of
-// 128 rows and there are fewer of them, above all fewer with a handful of rows (256 rows an expert: two units where half of
-// the experts had three).  tall_units_pay says when; 128 (or where named 256) rows -> 160, us, even counts / ~ 1 / sqrt(rank):
-// 128 experts 2048 x 768: 256 rows: gate/up 285 -> 260 / 281 -> 273, down 174 -> 164 / 177 -> 170, d_x 280 -> 259 / 280 -> 270; 480
-// rows: gate/up 449 -> 418 / 449 -> 426, down 270 -> 253 / 274 -> 247; 224 rows: 266 -> 271 / 260 -> 257, 162 -> 165 / 165 -> 161,
-// 253 -> 262 / 264 -> 255; 111 rows 199 -> 197 / 194 -> 198.  64 experts 1536 x 768, 450 rows: 198 -> 178 / 200 -> 179, 115 -> 105 /
-// 114 -> 110.  Few rounds of units, where the last one counts: 16 experts 2048 x 1024, 512 rows 114 -> 97 / 109 -> 94, 70 -> 63 / 66 -> 60,
-// 108 -> 95 / 104 -> 98; 64 experts 2048 x 768, 256 rows (3.75 rounds -> 3.15) 157 -> 168 / 159 -> 167; 8 experts 1024 x 512, 4,000 rows
-// (3.97 -> 3.19) 94 -> 103 / 95 -> 100; 128 experts 1024 x 512, 300 rows (5.7 -> 4.75) 134 -> 140 / 136 -> 144.
-// Against 256 rows: gate/up at any size (128 experts 2048 x 768: 512 rows 463 -> 446 / 468 -> 434, 1,024 rows 833 -> 809 / 836 -> 810;
-// 16 experts 2048 x 1024, 2,048 rows 302 -> 279 / 310 -> 281), down with a long reduction (64 experts 2048 x 1024, 512 rows 191 -> 179 /
-// 191 -> 177; but 2048 x 768, 512 rows 267 -> 277 / 278 -> 263, 1,024 rows 490 -> 494 / 493 -> 493), d_x not (512 rows 423 -> 440 /
-// 429 -> 430, 1,024 rows 748 -> 804 / 763 -> 805).
+// 160 rows, otherwise the same: what fits the LDS (3 x 52 KB)
 #define PK_RM_TALL 160, 256, 64, 2, 4, 3
-#define PK_RM_TALL_ROWS 248
-#define PK_RM_TALL_DOWN_K 1024
-// Weight gradients from row-major operands (with the transposed copies wgrad_pp_kernel, whose tile is fixed), 256 x 256 tiles by
-// rows an expert: few, wgrad_runs_kernel; from PK_WG_BIG_ROWS on 64-deep k-tiles in a 2-stage ring; between them 32-deep ones in a
-// 4-stage ring with the loads spread between the MFMAs.  us, runs -> 4-stage ring, gathered rows, even counts / ~ 1 / sqrt(rank): 128 experts
-// 2048 x 768: 192 rows 449 -> 476 / 516 -> 503, 256 rows 571 -> 556 / 658 -> 599, 400 rows 783 -> 734 / 876 -> 796; 64 experts 1536 x 768, 400
-// rows 299 -> 287 / 327 -> 312; 24 experts 1024 x 768, 400 rows, not gathered, 88 -> 81 / 82 -> 72.  With fewer than two tiles for every CU the
-// longest expert's k-loop counts sooner (64 experts 512 x 256, 192 rows, not gathered, 33.2 -> 34.0 / 48.0 -> 43.8).  Accumulating, the runs'
-// way to the old values is ahead at any size (128 experts 2048 x 768, 400 rows 907 against 1,080).
+// (which of them: unit_rows in launch_rules.h)
+// Weight gradients from row-major operands (wgrad_kernel there), tiles of 256 x 256
 #define PK_WG_BIG 256, 256, 64, 2, 4, 2
-#define PK_WG_BIG_ROWS 512
 #define PK_WG_RING 256, 256, 32, 2, 4, 4
 #define PK_WG_THREADS 512
-#define PK_WG_RUNS_ROWS 224
-#define PK_WG_RUNS_ROWS_ONE 160
 #define PK_WG_DYNAMIC_ROWS 512
 // rows an expert up to which d_h is formed on the tiles of tile_gemm.h
 #define PK_DH_TILE_ROWS 40
@@ -2401,16 +2349,6 @@ bool mfma_shape_ok(int64_t H, int64_t I) { return H % 128 == 0 && I % 128 == 0; 
 // products of such widths run on the tiles of tile_gemm.h (24,000 rows of 24 experts, 640 x 896, us, these tiles ->
 // those: down 63 -> 55, weight gradients 375 -> 176, d_x 94 -> 92).
 #define PK_RM_ALT 128, 128, 64, 2, 2, 4
-
-// Whether units of 160 rows are ahead of 128: with more than six rounds of the latter wherever there are fewer of the former, below
-// that by the number of rounds, a taller one at six fifths of the time (where that is a draw, from 352 rows an expert on).
-bool tall_units_pay(int64_t A, int64_t E, int64_t cols) {
-  if (A < (int64_t)PK_RM_TALL_ROWS * E) return false;
-  const int64_t grid = mf::persistent_grid(), u128 = (A / 128 + E / 2) * cols, u160 = (A / 160 + E / 2) * cols;
-  if (u128 >= 6 * grid) return true;
-  const int64_t c128 = 5 * pk_ceil_div(u128, grid), c160 = 6 * pk_ceil_div(u160, grid);
-  return c160 < c128 || (c160 == c128 && A >= 352 * E);
-}
 
 // 256 output columns per unit (for the gate/up kernel 128 gate and 128 up columns).
 template <bool B_KC, int EPI, bool A_T = false>
@@ -2424,24 +2362,15 @@ int launch_rm(mf::RaggedMParams& p, int64_t A, int64_t N, int kernel_id, hipStre
   }
   if (N % per_tile != 0) return PK_ERR_SHAPE;
   p.n_tiles = (int32_t)(N / per_tile);
-  // 256-row tiles unless they would leave the persistent grid with only a few units per
-  // workgroup (then the last round of units runs on a half-empty chip)
-  const int64_t big_units = (A / 256 + p.E / 2) * p.n_tiles;
-  // (d_x, row-major operands: see PK_RM_DX_ROWS)
-  constexpr bool DX = EPI == mf::EPI_PLAIN && !B_KC && !A_T;
-  const bool lowm = big_units < (int64_t)(DX ? 2 : PK_RM_LOWM_UNITS) * mf::persistent_grid();
-  // the scaled SwiGLU backward stays on 128-row units: its time goes into the epilogue (loads of g
-  // and u, the arithmetic, six stores per value), which 256-row units do not shorten, and with
-  // 128 accumulator registers that epilogue spills (measured 14 % slower at 16,384 tokens even
-  // with the packed outputs staged 32 columns at a time)
-  const bool low = EPI == mf::EPI_SWIGLU_BWD_SCALED || lowm || A < (int64_t)(DX ? PK_RM_DX_ROWS : PK_RM_SHORT_ROWS) * p.E;
-  if constexpr ((EPI == mf::EPI_SWIGLU || EPI == mf::EPI_PLAIN) && !A_T) {
-    if ((low || EPI == mf::EPI_SWIGLU || (B_KC && p.Kseg >= PK_RM_TALL_DOWN_K)) && tall_units_pay(A, p.E, p.n_tiles))
-      return mf::launch_ragged_m<PK_RM_TALL, B_KC, EPI>(p, A, kernel_id, s);
-  }
-  if (low || EPI == mf::EPI_SWIGLU) return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  constexpr pk_rules::Product WHAT = EPI == mf::EPI_SWIGLU ? pk_rules::GATE_UP : EPI == mf::EPI_SWIGLU_BWD ? pk_rules::DH
+                                     : EPI == mf::EPI_SWIGLU_BWD_SCALED ? pk_rules::DH_SCALED
+                                     : B_KC ? pk_rules::DOWN : A_T ? pk_rules::DX_TRANSPOSED : pk_rules::DX;
+  const int rows = pk_rules::unit_rows(WHAT, A, p.E, p.n_tiles, p.Kseg, mf::persistent_grid());
+  if (rows == 128) return mf::launch_ragged_m<PK_RM_SHORT, B_KC, EPI, A_T>(p, A, kernel_id, s);
+  if constexpr ((EPI == mf::EPI_SWIGLU || EPI == mf::EPI_PLAIN) && !A_T)
+    if (rows == 160) return mf::launch_ragged_m<PK_RM_TALL, B_KC, EPI>(p, A, kernel_id, s);
   if constexpr (EPI != mf::EPI_SWIGLU_BWD_SCALED && EPI != mf::EPI_SWIGLU)
-    return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
+    if (rows == 256) return mf::launch_ragged_m<PK_RM_CFG, B_KC, EPI, A_T>(p, A, kernel_id, s);
   return PK_ERR_SHAPE;
 }
 
@@ -2938,7 +2867,7 @@ int pk_grouped_swiglu_dx_from_transposed_pays(int64_t A, int64_t H, int64_t I, i
   // 9 % and the d_x GEMM 4 % faster without the row-major copies (256-row units, the A tile arrives
   // as runs of 4 KB); with 256 rows per expert the d_x GEMM on 128-row units loses 6 %, more than
   // the SwiGLU backward gains
-  return A >= (int64_t)PK_RM_SHORT_ROWS * E ? 1 : 0;
+  return A >= pk_rules::SHORT_ROWS * E ? 1 : 0;
 }
 
 int pk_region_transposed_pays(int64_t A, int64_t H, int64_t I, int64_t E, int dtype) {
@@ -3005,18 +2934,9 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   if (!row_map) row_map_div = 1;
   const int32_t* dy_map = dy_gathered ? row_map : nullptr;
   hipStream_t s = (hipStream_t)stream;
-  // 256 x 256 tiles where they give at least half of the CUs work; otherwise the 64- or 128-wide tiles of tile_gemm.h (us, 256 x 256 or, at
-  // widths that are not multiples of 256, its former 128 x 128 tiles -> those: 24 experts 640 x 896, 1,000 rows 379 -> 176; 64 experts
-  // 384 x 640, 1,536 rows 614 -> 287; but 8 experts 1024 x 512, 1,024 rows, 192 tiles 50 against 79).  With fewer experts than XCDs and
-  // long reductions a last round of few tiles, or an expert longer than the others, costs more than the smaller tiles do: two tiles
-  // for every CU there (tile_gemm.h's / 256 x 256, even counts, ~ 1 / sqrt(rank): 4 experts 2048 x 1024, 24 rows 22 / 17, 21 / 17, 300 rows 42 /
-  // 42, 42 / 37, 2,048 rows 155 / 172, 154 / 152; 4 experts 1024 x 1024, 128 rows 18 / 16, 20 / 18, 600 rows 37 / 36, 40 / 44, 2,048 rows 96 / 90,
-  // 94 / 120; 6 experts 2048 x 768, 300 rows 47 / 43, 47 / 43, 2,048 rows 179 / 176, 189 / 206; 4 experts 2048 x 2048, 300 rows 73 / 62, 74 / 61,
-  // 2,048 rows 295 / 262, 311 / 269).
   const int n_weights = (d_w1 ? 1 : 0) + (d_w2 ? 1 : 0) + (d_w3 ? 1 : 0);
-  const int64_t tiles_256 = E * (H / 256) * (I / 256) * n_weights, cus = mf::persistent_grid();
-  const bool mfma = dtype == PK_BF16 && H % 256 == 0 && I % 256 == 0 && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}) &&
-                    tiles_256 >= cus / 2 && (E >= mf::NXCD || A < (int64_t)PK_WG_BIG_ROWS * E || tiles_256 >= 2 * cus);
+  const pk_rules::WgradKernel kernel = pk_rules::wgrad_kernel(A, H, I, E, n_weights, accumulate != 0, mf::persistent_grid());
+  const bool mfma = dtype == PK_BF16 && kernel != pk_rules::TILES && all_aligned16({d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3});
   if (!mfma && tile_gemm_ok(dtype, H, I, {d_y, h, d_g, d_u, x_rows, d_w1, d_w2, d_w3}))
     return dtype == PK_F32
                ? wgrad_tile<float>(d_y, dy_map, h, d_g, d_u, x_rows, row_map, row_map_div, starts, d_w1, d_w2, d_w3, accumulate, A, H, I, E, s)
@@ -3053,29 +2973,10 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
   p.accumulate = accumulate ? 1 : 0;
   p.tiles_per_problem = (int32_t)((H / 256) * (I / 256));
   p.nprob = n;
-  // Few rows an expert: wgrad_runs_kernel.  Longer runs hide more of a tile's start, as long as there are several of them for
-  // every CU and none is long (us, runs of 1 / 2 / 4 tiles, even counts: 128 experts 2048 x 768, 36 tiles a CU: 16 rows 225 / 222 /
-  // 230, 32 rows 252 / 240 / 240, 48 rows 290 / 256 / 243, 96 rows 368 / 321 / 310; 64 experts 1536 x 768, 13 tiles: 24 rows
-  // 90 / 96, 48 rows 118 / 111, 128 rows 161 / 148; 16 experts 2048 x 1024, 6 tiles, 64 rows 61 / 54 / 58, 512 rows,
-  // ~ 1 / sqrt(rank) 172 / 181; 32 experts 1024 x 512, 3 tiles: 32 rows 30 / 28, 64 rows 31.3 / 32.7 (37 / 34), 128 rows 44 / 45 (46 / 55); 64 experts
-  // 512 x 256, 1.5 tiles, 100 rows 26 / 23 (32 / 54)).  Two against one in per cent: 64 experts 1024 x 1024, 12 tiles a CU, 8 rows -7 / -1
-  // uneven, 32 rows -9 / -5; 128 experts 1024 x 512, 12 tiles, 24 rows -4 / -3; 96 experts 1024 x 1024, 18 tiles, 24 rows -9 / -2; 24 experts
-  // 2048 x 1024, 9 tiles, 24 rows -7 / -6; but 64 experts 1536 x 768, whose 18 tiles make an odd number of pairs, 24 rows +2 / +10; 64 experts
-  // 512 x 512, 3 tiles, 24 rows -2 / -9, 48 rows +4 / +13; 128 experts 512 x 512, 6 tiles, 64 rows -4 / -3, 128 rows -7 / +14: with
-  // four tiles a gradient the longest expert's few workgroups are what the launch waits for.
-  const int64_t tiles = (int64_t)p.tiles_per_problem * n * E, per_cu = tiles / mf::persistent_grid();
-  const bool few_rows = A < (int64_t)(p.accumulate ? PK_WG_BIG_ROWS : per_cu < 2 ? PK_WG_RUNS_ROWS_ONE : PK_WG_RUNS_ROWS) * E;
-  p.run = 1;
-  if (few_rows) {
-    const int64_t two = (per_cu < 6 ? 64 : 192) / (p.tiles_per_problem >= 8 ? 1 : per_cu < 6 ? 2 : 3);
-    if (per_cu >= 24 && A > 32 * E && A <= 192 * E && p.tiles_per_problem % 4 == 0)
-      p.run = 4;
-    else if (p.tiles_per_problem % 2 == 0 && per_cu >= 3 && A <= two * E &&
-             (per_cu < 12 || per_cu >= 24 || A > 32 * E || p.tiles_per_problem % 4 == 0))
-      p.run = 2;
-  }
-  p.chunk = mf::deal_chunk(tiles / p.run, (int64_t)p.tiles_per_problem * n / p.run);
-  const int64_t blocks = pk_ceil_div(tiles / p.run, p.chunk * (int64_t)mf::NXCD) * p.chunk * mf::NXCD;
+  const int64_t tiles = (int64_t)p.tiles_per_problem * n * E;
+  p.run = kernel == pk_rules::RUNS ? pk_rules::wgrad_run(A, E, p.tiles_per_problem, tiles / mf::persistent_grid()) : 1;
+  p.chunk = (int32_t)pk_rules::deal_chunk(tiles / p.run, (int64_t)p.tiles_per_problem * n / p.run);
+  const int64_t blocks = pk_rules::dealt_blocks(tiles / p.run, p.chunk);
   if (blocks > 0x7ffffff0ll) return PK_ERR_SHAPE;
   const dim3 grid((unsigned)blocks), block(PK_WG_THREADS);
 #define PK_WG_RUNS(ACC)                                                                                                          \
@@ -3083,9 +2984,8 @@ static int wgrad_impl(const void* d_y, int dy_gathered, const void* h, const voi
     if (p.row_map) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_runs_kernel<ACC, true>), grid, block, 0, s, p);    \
     else PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_runs_kernel<ACC, false>), grid, block, 0, s, p);             \
   } while (0)
-  if (!few_rows && A < (int64_t)PK_WG_BIG_ROWS * E)
-    PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_RING>), grid, block, 0, s, p);
-  else if (!few_rows) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), grid, block, 0, s, p);
+  if (kernel == pk_rules::RING) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_RING>), grid, block, 0, s, p);
+  else if (kernel == pk_rules::BIG) PK_LAUNCH_NOCHECK(pk_timing::K_SWIGLU_WGRAD, s, (mf::wgrad_kernel<PK_WG_BIG>), grid, block, 0, s, p);
   else if (p.accumulate) PK_WG_RUNS(true);
   else PK_WG_RUNS(false);
 #undef PK_WG_RUNS

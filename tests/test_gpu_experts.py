@@ -900,7 +900,7 @@ RUN_CASES = [
     ([224, 240, 0, 33, 500, 64, 700, 300] * 2, 1024, 768),           # (from two tiles for every CU on)
     ([0, 70, 33, 1, 130, 20, 64, 9] * 2, 768, 768),                  # an odd number of tiles an expert, dealt out in chunks of 3
     ([40, 0, 90, 32] * 3, 1280, 1280),                               # of 7, which cross from one expert to the next
-    ([600, 0, 900, 1, 40, 1200, 700, 800], 1280, 768),               # one by one
+    ([600, 0, 900, 1, 40, 1200, 700, 800], 1280, 768),               # of 2, which 45 is no multiple of
     ([40, 0, 65, 33], 1024, 1024),                                   # fewer experts than XCDs
     ([300, 500, 1, 0, 460], 2048, 768),
     ([1000, 700, 0, 900], 2048, 2048),
@@ -1111,3 +1111,48 @@ def test_fp32_products_with_mostly_empty_tiles(dev, counts, H, I):
         assert ((hs[r].double() - sc[:, None] * hv).abs() <= sc[:, None] * hv.abs() * 2**-20 + 1e-30).all(), ("score * h", e)
         bound = (size * hv.abs()).sum(1) * (H + I) * 2**-22
         assert ((ds.flatten()[perm[r].long()].double() - (dh * hv).sum(1)).abs() <= bound + 1e-30).all(), ("d_score", e)
+
+
+@pytest.mark.parametrize("H", [128, 256])
+def test_units_of_160_rows_with_short_reductions(dev, H):
+    """Gate/up with two or four k-tiles and gathered rows: the loader enters the next unit in the epilogue, not in the k-loop."""
+    I, E, K = 1280, 64, 2
+    counts = [159, 160, 161, 319, 320, 321, 1, 639] * 8
+    A = sum(counts)
+    print(f"[case] units of 160 rows, H={H}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(H)
+    rand = lambda *shape, scale=1.0: (torch.randn(shape, generator=gen, device=dev) * scale).bfloat16()
+    x = rand(A // K, H)
+    w1, w3, w2 = rand(E, I, H, scale=0.1), rand(E, I, H, scale=0.1), rand(E, H, I, scale=0.05)
+    perm = torch.randperm(A, generator=gen, device=dev).int()
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    y, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts, row_map=perm, row_map_div=K, num_rows=A)
+    rows = (perm // K).long()
+    first = 0
+    for e, n in enumerate(counts):
+        r = slice(first, first + n)
+        first += n
+        xe, ge, ue = x[rows[r]].double(), g[r].double(), u[r].double()
+        for got, w in ((g, w1), (u, w3)):
+            want, size = xe @ w[e].double().T, xe.abs() @ w[e].double().abs().T
+            assert ((got[r].double() - want).abs() <= want.abs() * 2**-8 + size * (H + 1) * 2**-23).all(), e
+        want = torch.nn.functional.silu(ge) * ue
+        assert ((h[r].double() - want).abs() <= want.abs() * (2**-8 + 2**-18) + 1e-30).all(), e
+
+
+def test_gate_and_up_do_not_depend_on_the_units_height(dev):
+    """The first 16 of 64 experts by themselves are on 128-row units, all of them on 160-row ones: the same sums in the same order."""
+    H, I, K = 2048, 1280, 2
+    counts = [159, 160, 161, 319, 320, 321, 1, 639] * 8
+    A, few = sum(counts), sum(counts[:16])
+    print("[case] 160- against 128-row units", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(160)
+    rand = lambda *shape, scale=1.0: (torch.randn(shape, generator=gen, device=dev) * scale).bfloat16()
+    x = rand(A // K, H)
+    w1, w3, w2 = rand(64, I, H, scale=0.05), rand(64, I, H, scale=0.05), rand(64, H, I, scale=0.05)
+    perm = torch.randperm(A, generator=gen, device=dev).int()
+    starts = ops.counts_to_starts(torch.tensor(counts, dtype=torch.int32, device=dev))
+    _, g, u, h = ops.grouped_swiglu_fwd(x, w1, w2, w3, starts, row_map=perm, row_map_div=K, num_rows=A)
+    _, g2, u2, h2 = ops.grouped_swiglu_fwd(x, w1[:16], w2[:16], w3[:16], starts[:17].contiguous(), row_map=perm[:few].contiguous(),
+                                           row_map_div=K, num_rows=few)
+    assert torch.equal(g[:few], g2) and torch.equal(u[:few], u2) and torch.equal(h[:few], h2)
