@@ -157,6 +157,70 @@ struct Lds {
   __attribute__((aligned(16))) bf16_t Bs[Planes<TB>::N][B_KC ? BN * LDK : BK * LDB];
 };
 
+// What the products below have in common: a thread's share of a k-tile in registers, its way into the LDS, and the matrix
+// instructions.  Every thread holds 4 consecutive elements of the contiguous index per load (every plane of them for a pre-split operand).
+template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB>
+struct KTile {
+  typedef Lds<WM, WN, A_KC, B_KC, TA, TB> Tiles;
+  static constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
+  static constexpr int PA = Planes<TA>::N, PB = Planes<TB>::N;
+  static constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
+  static_assert(NA >= 1 && NB >= 1, "tile too small for the thread count");
+  Raw<TA> a[NA];
+  Raw<TB> b[NB];
+
+  __device__ static __forceinline__ void slot(int idx, bool kc, int R, int& row, int& k) {
+    if (kc) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); }
+    else { row = (idx % (R / 4)) * 4; k = idx / (R / 4); }
+  }
+  // one 8-byte store per plane: along k of a [row][k] tile for a K-contiguous operand, along the
+  // rows of a [k][row] tile otherwise
+  template <int P, typename Operand>
+  __device__ static __forceinline__ void store4(Operand& tiles, bool kc, int ld_mn, int row, int k, const bf16x4_t (&v)[P]) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) *reinterpret_cast<bf16x4_t*>(&tiles[q][kc ? row * LDK + k : k * ld_mn + row]) = v[q];
+  }
+  // into the LDS, cleared from k-index `have` on
+  __device__ __forceinline__ void store(Tiles& lds, int tid, int have) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      int m, k;
+      slot(tid + i * THREADS, A_KC, BM, m, k);
+      if (have < BK && k >= have) zero_raw<TA>(a[i]);
+      bf16x4_t v[PA];
+      to_planes<TA>(a[i], v);
+      store4(lds.As, A_KC, Tiles::LDA, m, k, v);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      int n, k;
+      slot(tid + i * THREADS, B_KC, BN, n, k);
+      if (have < BK && k >= have) zero_raw<TB>(b[i]);
+      bf16x4_t v[PB];
+      to_planes<TB>(b[i], v);
+      store4(lds.Bs, B_KC, Tiles::LDB, n, k, v);
+    }
+  }
+  __device__ static __forceinline__ void multiply(const Tiles& lds, int wm, int wn, int lane, floatx16_t& acc) {
+#pragma unroll
+    for (int kk = 0; kk < BK; kk += 16) {
+      bf16x8_t fa[PA], fb[PB];
+#pragma unroll
+      for (int pl = 0; pl < PA; ++pl) fa[pl] = A_KC ? frag_kc(lds.As[pl], wm * 32, kk, lane) : frag_mn(lds.As[pl], Tiles::LDA, wm * 32, kk, lane);
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl) fb[pl] = B_KC ? frag_kc(lds.Bs[pl], wn * 32, kk, lane) : frag_mn(lds.Bs[pl], Tiles::LDB, wn * 32, kk, lane);
+      // small terms first
+#pragma unroll
+      for (int s = PA + PB - 2; s >= 0; --s)
+#pragma unroll
+        for (int pa = 0; pa < PA; ++pa) {
+          const int pb = s - pa;
+          if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa], fb[pb], acc, 0, 0, 0);
+        }
+    }
+  }
+};
+
 // How k-tiles are requested ahead (see product).  2: two in flight, for the products whose reduction is long: the forward from bf16
 // and the weight gradients.  1: one, for the fp32 forward, whose split takes the registers of the second (64 experts 1024 wide,
 // 10,000 tokens 18.5 -> 17.6 us).  0: one, ordered by the compiler, for d_x: its reduction over the experts is one to four k-tiles.
@@ -168,7 +232,8 @@ constexpr int in_flight() { return A_KC && !B_KC ? 0 : A_KC && std::is_same<TA, 
 // instructions for two k-tiles of the bf16 forward, where forming the addresses of every load, masking it and splitting values one
 // by one took 260.  The older of two k-tiles in flight is waited for by count, as nothing in the loop is conditional; without the
 // scheduling barriers the compiler puts the requests behind the products and converts the younger tile first.  Four waves a
-// SIMD (128 registers) matter more than a second k-tile.  us, before -> now, 128 experts 2048 wide unless said: forward 16,384 tokens
+// SIMD (128 registers) matter more than a second k-tile, and more than the two registers that the fp32 weight gradient spills for
+// them (three waves, nothing spilled: in one launch 2048 wide, 128 experts, 1,000 tokens 27.4 -> 30.2, 16,000 304 -> 309).  us, before -> now, 128 experts 2048 wide unless said: forward 16,384 tokens
 // 53 -> 47, 4,096 19.2 -> 18.6, 8 experts, 16,384 37 -> 25; weight gradient 16,384 60 -> 56,
 // fp32, 64 experts 1024 wide, 4,000 15.0 -> 11.4; d_x 16,384 96 -> 85; the router's backward in one launch (router_grads_kernel)
 // 16,384 202 -> 189, 4,096 62 -> 58, 3,000 36 -> 33.
@@ -179,10 +244,6 @@ template <int WM, int WN, bool A_KC, bool B_KC, typename TA, typename TB, int FL
 __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
                                         int64_t kend, floatx16_t& acc) {
   constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
-  constexpr int PA = Planes<TA>::N, PB = Planes<TB>::N;
-  constexpr int LDA = BM + MN_PAD, LDB = BN + MN_PAD;
-  auto& As = lds.As;
-  auto& Bs = lds.Bs;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;
   typedef typename Mem<TA>::type MA;
@@ -193,27 +254,21 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
 
-  // Every thread fetches 4 consecutive elements of the contiguous index per load (every plane of them for a pre-split operand).
   // No load stands behind a branch: rows past the ends are read from the last ones, and their results are not stored.
-  constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
-  static_assert(NA >= 1 && NB >= 1, "tile too small for the thread count");
-  struct Tile { Raw<TA> a[NA]; Raw<TB> b[NB]; };
-  auto slot = [](int idx, bool kc, int R, int& row, int& k) {
-    if (kc) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); }
-    else { row = (idx % (R / 4)) * 4; k = idx / (R / 4); }
-  };
+  typedef KTile<WM, WN, A_KC, B_KC, TA, TB> Tile;
+  constexpr int NA = Tile::NA, NB = Tile::NB;
   const MA* pa[NA];
   const MB* pb[NB];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
     int m, k;
-    slot(tid + i * THREADS, A_KC, BM, m, k);
+    Tile::slot(tid + i * THREADS, A_KC, BM, m, k);
     pa[i] = A + min(m0 + m, p.M - (A_KC ? 1 : 4)) * p.sam + (A_KC ? kbeg + k : (kbeg + k) * p.sak);
   }
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     int n, k;
-    slot(tid + i * THREADS, B_KC, BN, n, k);
+    Tile::slot(tid + i * THREADS, B_KC, BN, n, k);
     pb[i] = B + min(n0 + n, p.N - (B_KC ? 1 : 4)) * p.sbn + (B_KC ? kbeg + k : (kbeg + k) * p.sbk);
   }
   const int64_t step_a = A_KC ? BK : BK * p.sak, step_b = B_KC ? BK : BK * p.sbk;
@@ -231,69 +286,24 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       int m, k;
-      slot(tid + i * THREADS, A_KC, BM, m, k);
+      Tile::slot(tid + i * THREADS, A_KC, BM, m, k);
       const int64_t back = max(0, k - (have - (A_KC ? 4 : 1)));
       fetch4<TA>(pa[i] - (A_KC ? back : back * p.sak), p.plane_a, t.a[i]);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       int n, k;
-      slot(tid + i * THREADS, B_KC, BN, n, k);
+      Tile::slot(tid + i * THREADS, B_KC, BN, n, k);
       const int64_t back = max(0, k - (have - (B_KC ? 4 : 1)));
       fetch4<TB>(pb[i] - (B_KC ? back : back * p.sbk), p.plane_b, t.b[i]);
     }
   };
-  // one 8-byte store per plane: along k of a [row][k] tile for a K-contiguous operand, along the
-  // rows of a [k][row] tile otherwise
-  auto store4 = [](auto& tiles, auto nplanes, bool kc, int ld_mn, int row, int k, const auto& v) {
-    constexpr int P = decltype(nplanes)::value;
-#pragma unroll
-    for (int q = 0; q < P; ++q) *reinterpret_cast<bf16x4_t*>(&tiles[q][kc ? row * LDK + k : k * ld_mn + row]) = v[q];
-  };
-  auto store_tile = [&](Tile& t, int have) {     // (cleared from k-index `have` on)
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      int m, k;
-      slot(tid + i * THREADS, A_KC, BM, m, k);
-      if (have < BK && k >= have) zero_raw<TA>(t.a[i]);
-      bf16x4_t v[PA];
-      to_planes<TA>(t.a[i], v);
-      store4(As, std::integral_constant<int, PA>{}, A_KC, LDA, m, k, v);
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      int n, k;
-      slot(tid + i * THREADS, B_KC, BN, n, k);
-      if (have < BK && k >= have) zero_raw<TB>(t.b[i]);
-      bf16x4_t v[PB];
-      to_planes<TB>(t.b[i], v);
-      store4(Bs, std::integral_constant<int, PB>{}, B_KC, LDB, n, k, v);
-    }
-  };
-  auto multiply = [&]() {
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-      bf16x8_t a[PA], b[PB];
-#pragma unroll
-      for (int pl = 0; pl < PA; ++pl) a[pl] = A_KC ? frag_kc(As[pl], wm * 32, kk, lane) : frag_mn(As[pl], LDA, wm * 32, kk, lane);
-#pragma unroll
-      for (int pl = 0; pl < PB; ++pl) b[pl] = B_KC ? frag_kc(Bs[pl], wn * 32, kk, lane) : frag_mn(Bs[pl], LDB, wn * 32, kk, lane);
-      // small terms first
-#pragma unroll
-      for (int s = PA + PB - 2; s >= 0; --s)
-#pragma unroll
-        for (int pa = 0; pa < PA; ++pa) {
-          const int pb = s - pa;
-          if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa], b[pb], acc, 0, 0, 0);
-        }
-    }
-  };
   auto use = [&](Tile& t, int have, auto next) {
-    store_tile(t, have);
+    t.store(lds, tid, have);
     __syncthreads();
     next();
     if constexpr (FLIGHT > 0) __builtin_amdgcn_sched_barrier(0);       // requested before the products, and the next tile not waited for before their end
-    multiply();
+    Tile::multiply(lds, wm, wn, lane, acc);
     __syncthreads();
     if constexpr (FLIGHT > 0) __builtin_amdgcn_sched_barrier(0);
   };
@@ -347,10 +357,7 @@ __device__ __forceinline__ void product(const Params& p, Lds<WM, WN, A_KC, B_KC,
 template <int WM, int WN, typename TA, typename TB, int AHEAD>
 __device__ __forceinline__ void product_at_once(const Params& p, Lds<WM, WN, true, true, TA, TB>& lds, int64_t m0, int64_t n0, int64_t kbeg,
                                                 int64_t kend, floatx16_t& acc) {
-  constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN;
-  constexpr int PA = Planes<TA>::N, PB = Planes<TB>::N;
-  auto& As = lds.As;
-  auto& Bs = lds.Bs;
+  typedef KTile<WM, WN, true, true, TA, TB> Tile;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;
   typedef typename Mem<TA>::type MA;
@@ -361,63 +368,39 @@ __device__ __forceinline__ void product_at_once(const Params& p, Lds<WM, WN, tru
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
 
-  constexpr int NA = BM * BK / (THREADS * 4), NB = BN * BK / (THREADS * 4);
-  struct Tile { Raw<TA> a[NA]; Raw<TB> b[NB]; };
-  auto slot = [](int idx, int& row, int& k) { k = (idx % (BK / 4)) * 4; row = idx / (BK / 4); };
-  // (past the ends from the last elements, as a branch would hold up the loads behind it; what lies past kend is cleared when it
-  // goes to LDS)
+  // (past the ends from the last elements, as a branch would hold up the loads behind it)
   auto load_tile = [&](Tile& t, int64_t k0) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
+    for (int i = 0; i < Tile::NA; ++i) {
       int m, k;
-      slot(tid + i * THREADS, m, k);
+      Tile::slot(tid + i * Tile::THREADS, true, Tile::BM, m, k);
       fetch4<TA>(A + min(m0 + m, p.M - 1) * p.sam + min(k0 + k, kend - 4) * p.sak, p.plane_a, t.a[i]);
     }
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
+    for (int i = 0; i < Tile::NB; ++i) {
       int n, k;
-      slot(tid + i * THREADS, n, k);
+      Tile::slot(tid + i * Tile::THREADS, true, Tile::BN, n, k);
       fetch4<TB>(B + min(k0 + k, kend - 4) * p.sbk + min(n0 + n, p.N - 1) * p.sbn, p.plane_b, t.b[i]);
     }
   };
   auto store_tile = [&](Tile& t, int64_t k0) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
+    for (int i = 0; i < Tile::NA; ++i) {
       int m, k;
-      slot(tid + i * THREADS, m, k);
+      Tile::slot(tid + i * Tile::THREADS, true, Tile::BM, m, k);
       if (k0 + k >= kend) zero_raw<TA>(t.a[i]);
-      bf16x4_t v[PA];
+      bf16x4_t v[Tile::PA];
       to_planes<TA, false>(t.a[i], v);
-#pragma unroll
-      for (int q = 0; q < PA; ++q) *reinterpret_cast<bf16x4_t*>(&As[q][m * LDK + k]) = v[q];
+      Tile::store4(lds.As, true, 0, m, k, v);
     }
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
+    for (int i = 0; i < Tile::NB; ++i) {
       int n, k;
-      slot(tid + i * THREADS, n, k);
+      Tile::slot(tid + i * Tile::THREADS, true, Tile::BN, n, k);
       if (k0 + k >= kend) zero_raw<TB>(t.b[i]);
-      bf16x4_t v[PB];
+      bf16x4_t v[Tile::PB];
       to_planes<TB, false>(t.b[i], v);
-#pragma unroll
-      for (int q = 0; q < PB; ++q) *reinterpret_cast<bf16x4_t*>(&Bs[q][n * LDK + k]) = v[q];
-    }
-  };
-  auto multiply = [&]() {
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-      bf16x8_t a[PA], b[PB];
-#pragma unroll
-      for (int pl = 0; pl < PA; ++pl) a[pl] = frag_kc(As[pl], wm * 32, kk, lane);
-#pragma unroll
-      for (int pl = 0; pl < PB; ++pl) b[pl] = frag_kc(Bs[pl], wn * 32, kk, lane);
-      // small terms first
-#pragma unroll
-      for (int s = PA + PB - 2; s >= 0; --s)
-#pragma unroll
-        for (int pa = 0; pa < PA; ++pa) {
-          const int pb = s - pa;
-          if (pb >= 0 && pb < PB && s <= 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa], b[pb], acc, 0, 0, 0);
-        }
+      Tile::store4(lds.Bs, true, 0, n, k, v);
     }
   };
   Tile t[AHEAD];
@@ -429,7 +412,7 @@ __device__ __forceinline__ void product_at_once(const Params& p, Lds<WM, WN, tru
     if (kbeg + i * BK < kend) {
       store_tile(t[i], kbeg + i * BK);
       __syncthreads();
-      multiply();
+      Tile::multiply(lds, wm, wn, lane, acc);
       __syncthreads();
     }
 }
