@@ -173,7 +173,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // multiplies k-tile kt out of it and, with `more`, requests k-tile kt + DEPTH into it.  Exactly the k-tiles that are there are
 // requested: an expert with one or two of them is bound by the memory's answer to these.  The loop has nothing to skip and one way
 // out, and whatever leads to a step has requested the same number of tiles behind its own: the compiler's counts depend on both.
-// us, one loop that always requests DEPTH tiles more -> this, caches cold: weight gradients 24 experts 1000 x 360, 8 rows 28.4 ->
+// us, one loop that always requests DEPTH tiles more -> this, each launch behind a fill of 640 MB: weight gradients 24 experts 1000 x 360, 8 rows 28.4 ->
 // 26.1 (rows not gathered 26.5 -> 25.0), 32 rows 28.8 -> 27.1, 172 rows 42.2 -> 40.2; 32 experts 1000 x 512, uneven rows not gathered,
 // 8 38.7 -> 34.6, 64 49.1 -> 47.0; fp32 32 experts 1024 x 512, 16 rows 73.7 -> 70.2; 24 experts 1000 x 360, 96 rows 88.1 -> 84.7.  bf16 in
 // 64 x 64 tiles: d_x 24 experts 1000 x 360, 8 rows 19.8 -> 18.9, 96 rows 26.6 -> 25.6; gate/up 172 rows 37.6 -> 35.8; d_h 32 experts
