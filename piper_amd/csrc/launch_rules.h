@@ -1,5 +1,6 @@
-// Which kernel a grouped product of the 256-wide bf16 kernels takes, and how its work is cut up, by the sizes alone.  Plain functions of
-// numbers, without a GPU in them, so that a test can ask them too.  cus: workgroups of the persistent grid.
+// Which kernel a grouped product takes, and how its work is cut up, by the sizes alone (the 256-wide bf16 kernels, and what the fp32
+// tile products load).  Plain functions of numbers, without a GPU in them, so that a test can ask them too.  cus: CUs, which are
+// also the workgroups of the persistent grid.
 #pragma once
 #include <cstdint>
 
@@ -117,5 +118,18 @@ constexpr int64_t deal_chunk(int64_t units, int64_t per_expert) {
 }
 // workgroups that it takes: whole turns of eight chunks
 constexpr int64_t dealt_blocks(int64_t units, int64_t chunk) { return ceil_div(units, chunk * NXCD) * chunk * NXCD; }
+
+// ---- fp32 products in tiles of 64 x 64 and below
+// Whether they leave the rows that are not there out of the loads (the SPARSE kernels of tile_gemm.h, with what that gains): with up
+// to half a tile of rows an expert and at least twelve k-tiles, as long as the tiles fit the CUs at once, which hold three of
+// gate/up, four of the others.  Beyond that other tiles hide what it saves, and the branches are left (us, all rows read -> left out:
+// gate/up 128 experts 1024 x 512, 16 rows, 1,024 tiles 189 -> 224, 100 experts, 8 rows, 800 tiles 184 -> 202, 128 experts 2048 x 768, 8 rows
+// 407 -> 440; but 96 experts 1024 x 512, 768 tiles 147 -> 141; d_x 80 experts 1024 x 512, 20 uneven rows, 1,280 tiles 144 -> 158, 96 experts,
+// 8 rows 145 -> 161, but 64 experts 1024 x 768, 8 rows, 1,024 tiles 151 -> 143; d_h 128 experts 2048 x 768, 8 rows, 1,536 tiles 245 -> 251,
+// 1024 x 512, 16 rows, 1,024 tiles 113 -> 107).
+constexpr bool absent_rows_left_out(bool gate_up, int64_t A, int64_t E, int64_t tile_rows, int64_t col_tiles, int64_t k_tiles, int64_t cus) {
+  const int64_t experts = A < E ? A : E;
+  return 2 * A <= tile_rows * experts && k_tiles >= 12 && experts * col_tiles <= (gate_up ? 3 : 4) * cus;
+}
 
 }  // namespace pk_rules

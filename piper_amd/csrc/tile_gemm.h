@@ -31,12 +31,13 @@
 // of 16 bytes): see the figures at tile_gemm_ok in grouped_gemm.hip.
 #pragma once
 #include "pk_common.h"
+#include "launch_rules.h"
 #include "unit_index.h"
 #include <type_traits>
 
 namespace pk_tile {
 
-constexpr int NXCD = 8;
+constexpr int NXCD = pk_rules::NXCD, CUS = 256;
 
 typedef short shortx4_t __attribute__((ext_vector_type(4)));
 typedef short shortx8_t __attribute__((ext_vector_type(8)));
@@ -283,8 +284,9 @@ enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
 // experts 1000 x 360, 8 rows: gate/up 49.0 -> 45.4, d_h 26.2 -> 25.1, d_x 34.2 -> 33.3; 32 experts 1024 x 512, 16 rows, d_x 59.8 -> 53.7; 64 experts
 // 896 x 384, 16 rows, gate/up 83.7 -> 81.3, d_x 81.3 -> 78.2).  With more rows the branches cost as much (24 experts 1000 x 360, 48 rows,
 // gate/up 51.4 -> 54.7; 128 experts 512 x 128, 48 uneven rows, d_x 41.9 -> 48.6), with fewer than twelve k-tiles there is little to
-// gain (128 experts 512 x 128, 32 rows, down 20.0 -> 21.1); the 32 x 32 tiles gain in d_h alone (24 experts 1000 x 360, 8 rows
-// 26.0 -> 25.1; 16 experts 408 x 472, 16 rows, d_x 19.8 -> 20.6).
+// gain (128 experts 512 x 128, 32 rows, down 20.0 -> 21.1), and with more tiles than fit the CUs at once nothing (figures at
+// absent_rows_left_out); the 32 x 32 tiles gain in d_h alone (24 experts 1000 x 360, 8 rows 26.0 -> 25.1; 16 experts 408 x 472, 16 rows,
+// d_x 19.8 -> 20.6).
 template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI, bool SPARSE>
 __global__ __launch_bounds__(64 * WM * WN * KS, (sizeof(T) == 4 && !SPARSE) || WM * WN < 4 || KS > 1 || TM * TN > 1 ? 1 : EPI == GATE_UP ? 3 : 4)
 void ragged_m_kernel(const RaggedM p) {
@@ -561,7 +563,7 @@ inline int launch_tiles(RaggedM p, int64_t A_rows, int* part_cols, int kernel_id
   if (part_cols) *part_cols = BN;
   const dim3 grid((unsigned)(pk_ceil_div(units, CHUNK * NXCD) * CHUNK * NXCD)), block(64 * WM * WN * KS);
   constexpr bool MAY_BE_SPARSE = sizeof(T) == 4 && (WM * WN > 1 || EPI != PLAIN);
-  if (MAY_BE_SPARSE && 2 * A_rows <= BM * (A_rows < p.E ? A_rows : p.E) && pk_ceil_div(p.K, kBK<T>) * p.nseg >= 12)
+  if (MAY_BE_SPARSE && pk_rules::absent_rows_left_out(EPI == GATE_UP, A_rows, p.E, BM, p.n_tiles, pk_ceil_div(p.K, kBK<T>) * p.nseg, CUS))
     PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, KS, B_KC, EPI, MAY_BE_SPARSE>), grid, block, 0, s, p);
   else
     PK_LAUNCH_NOCHECK(kernel_id, s, (ragged_m_kernel<T, WM, WN, TM, TN, KS, B_KC, EPI, false>), grid, block, 0, s, p);

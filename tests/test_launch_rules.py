@@ -22,6 +22,7 @@ int wgrad(int64_t A, int64_t H, int64_t I, int64_t E, int64_t n, int acc, int64_
 int run(int64_t A, int64_t E, int64_t tiles, int64_t per_cu) { return wgrad_run(A, E, tiles, per_cu); }
 int64_t chunk(int64_t units, int64_t per_expert) { return deal_chunk(units, per_expert); }
 int64_t blocks(int64_t units, int64_t chunk) { return dealt_blocks(units, chunk); }
+int absent(int gate_up, int64_t A, int64_t E, int64_t rows, int64_t cols, int64_t k, int64_t cus) { return absent_rows_left_out(gate_up != 0, A, E, rows, cols, k, cus); }
 int unit(int block, int chunk) { return dealt_unit(block, chunk); }
 }
 """
@@ -42,6 +43,7 @@ def rules(tmp_path_factory):
     lib.rows.argtypes = [ctypes.c_int] + [i64] * 5
     lib.wgrad.argtypes = [i64] * 5 + [ctypes.c_int, i64]
     lib.run.argtypes = [i64] * 4
+    lib.absent.argtypes = [ctypes.c_int] + [i64] * 6
     lib.chunk.argtypes = lib.blocks.argtypes = [i64, i64]
     lib.chunk.restype = lib.blocks.restype = i64
     return lib
@@ -89,3 +91,15 @@ def test_every_unit_is_dealt_out_once(rules, units, per_expert):
     blocks = rules.blocks(units, chunk)
     dealt = sorted(rules.unit(b, chunk) for b in range(blocks))
     assert dealt == list(range(blocks)) and blocks >= units
+
+
+@pytest.mark.parametrize("gate_up,E,rows,col_tiles,k_tiles,want", [
+    (1, 24, 8, 6, 32, True), (1, 96, 8, 8, 32, True), (1, 100, 8, 8, 32, False), (1, 128, 16, 12, 64, False),
+    (0, 64, 8, 16, 48, True), (0, 80, 20, 16, 32, False), (0, 64, 32, 16, 48, True), (0, 64, 33, 16, 48, False),
+    (0, 64, 8, 16, 12, True), (0, 64, 8, 16, 11, False), (0, 128, 16, 8, 32, True), (0, 128, 8, 12, 64, False),
+])
+def test_which_fp32_products_leave_out_absent_rows(rules, gate_up, E, rows, col_tiles, k_tiles, want):
+    assert bool(rules.absent(gate_up, E * rows, E, 64, col_tiles, k_tiles, CUS)) == want
+    if rows == 8 and want:
+        assert rules.absent(gate_up, 3, E, 64, col_tiles, k_tiles, CUS) == 1      # fewer rows than experts
+        assert rules.absent(gate_up, E * 17, E, 32, col_tiles, k_tiles, CUS) == 0
