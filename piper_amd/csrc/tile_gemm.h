@@ -287,11 +287,12 @@ enum Epilogue { PLAIN = 0, GATE_UP = 1, BWD = 2, BWD_SCALED = 3 };
 // gain (128 experts 512 x 128, 32 rows, down 20.0 -> 21.1), and with more tiles than fit the CUs at once nothing (figures at
 // absent_rows_left_out); the 32 x 32 tiles gain in d_h alone (24 experts 1000 x 360, 8 rows 26.0 -> 25.1; 16 experts 408 x 472, 16 rows,
 // d_x 19.8 -> 20.6).
-// Gate and up of more tiles than CUs wait for all of a round's k-tiles before they ask for the next ones, but for 64 x 64 tiles in two
-// groups: what masked loads did by themselves.  Where some CUs have two tiles and others one, requests that run ahead make these wait (us, without
-// -> this, r rows an expert: 24 experts 2048 x 384, r 8, 83 -> 75, masked 71; 1024 x 384 46.5 -> 44, 42; 1000 x 360 45.3 -> 43.5, 42; 40 experts 1024 x 256, r 8, 43.8 -> 42.2; 64 experts 1536 x 384, r 24, 133.8 -> 129.8; 128 experts 512 x 256,
-// uneven r 24, 75.3 -> 73.2); with a tile for every CU at most it costs as much (24 experts 1000 x 256, r 8, 30.2 -> 32.1, 12 experts
-// 1000 x 360 29.0 -> 30.2), and 64 x 64 tiles in two groups lose (32 experts 1024 x 512, uneven r 24, 89.4 -> 96.8).
+// Gate and up of more tiles than CUs wait for all of a round's k-tiles before they ask for the next ones, which masked loads did by
+// themselves: where some CUs have two tiles and others one, requests that run ahead make these wait (us, without -> this, r rows an
+// expert: 24 experts 2048 x 384, r 8, 83 -> 75, masked 71; 1024 x 384 46.5 -> 44, 42; 1000 x 360 45.3 -> 43.5, 42; 40 experts 1024 x 256, r 8,
+// 43.8 -> 42.2; 64 experts 1536 x 384, r 24, 133.8 -> 129.8; 128 experts 512 x 256, uneven r 24, 75.3 -> 73.2).  With a tile for every CU
+// at most it costs as much (24 experts 1000 x 256, r 8, 30.2 -> 32.1; 12 experts 1000 x 360 29.0 -> 30.2), and 64 x 64 tiles in two groups
+// lose (32 experts 1024 x 512, uneven r 24, 89.4 -> 96.8).
 template <typename T, int WM, int WN, int TM, int TN, int KS, bool B_KC, int EPI, bool SPARSE>
 __global__ __launch_bounds__(64 * WM * WN * KS, (sizeof(T) == 4 && !SPARSE) || WM * WN < 4 || KS > 1 || TM * TN > 1 ? 1 : EPI == GATE_UP ? 3 : 4)
 void ragged_m_kernel(const RaggedM p) {
